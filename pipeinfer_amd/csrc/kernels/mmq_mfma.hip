@@ -1233,6 +1233,7 @@ extern "C" int pi_op_mul_mat_reserve(void) {
     mmvq_args g; memset(&g, 0, sizeof g);                      // g.frag == nullptr: the instances only set their attribute
     for (int type : { PI_Q3_K, PI_Q4_K, PI_Q5_K, PI_Q6_K }) for (int cfg : mmq_cfgs) for (int nt : { 8, 16, 32, 64 }) { g.nt = nt; mmq_dispatch(type, g, 0, cfg, nullptr, nullptr, nullptr); }
     for (int type_b : { PI_Q5_K, PI_Q6_K }) for (int r : { 1, 2, 3 }) for (int rb : { 1, r }) for (bool four : { false, true }) mmq_2t_dispatch(type_b, r, rb, four, g, 0, 0, nullptr, nullptr, nullptr);
+    if (pi_mmq_q0_reserve() != 0) return -1;
     done = true;
     PI_CHECK_LAUNCH();
     return 0;

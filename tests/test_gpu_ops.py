@@ -144,6 +144,23 @@ def test_mul_mat_vs_oracle(gpu, t, k, rows, n_tok):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("t", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("k,rows,n_tok", [(32, 1, 9), (96, 17, 16), (128, 64, 10), (160, 65, 17), (4544, 130, 32), (256, 63, 33), (4096, 129, 64), (1056, 68, 65), (2048, 1030, 130), (11008, 66, 47)])
+def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
+    """k_mmq_q0 (prompts of the 32-value block types on the matrix cores), one instance per 16 / 32 / more tokens: last groups of less than four blocks, rows and tokens that end inside a tile, row
+    counts that are no multiple of four (scalar stores) — the reference's bits, with and without a residual"""
+    lib, U = gpu
+    rng = np.random.default_rng(k + rows + n_tok)
+    blocks = synth.random_blocks(t, rows * k, rng, 0.05).reshape(rows, -1)
+    act = np.stack([signal(k, s + n_tok) for s in range(n_tok)])
+    res = rng.standard_normal((n_tok, rows)).astype(np.float32)
+    w = upload_weight(lib, t, rows, k, blocks)
+    want = O.Impl("oracle").mul_mat(t, blocks, k, rows, act)
+    assert np.array_equal(gpu_mul_mat(lib, U, t, w, k, rows, act).view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(gpu_mul_mat(lib, U, t, w, k, rows, act, residual=res).view(np.uint32), (res + want).view(np.uint32))
+    lib.pi_weight_free(w)
+
+
 @pytest.mark.parametrize("t", QTYPES)
 def test_mul_mat_integer_sums_exact(gpu, t):
     """Scales forced to powers of two and integer activations small enough that every partial sum is an integer < 2^24:
