@@ -5,19 +5,21 @@
 // `exact` selects what enters the product: 0 (serving precision) rounds the activations to bfloat16 (nearest even), so a product of two bfloat16 values is exact in fp32 and only the
 // order of the fp32 sum differs between the kernels below; 1 keeps the activations in fp32 (weights widen exactly), every multiply-add a true fp32 fma.
 //
-//   k_dense_rows   one wave per output row, K spread over the lanes with 16 / 8 / 2-byte weight loads, TT tokens held in registers: the mat-vec of decode (weights streamed
-//                  once from HBM whatever TT is) and every width of the fp32 mode
-//   k_dense_mfma_lds  serving precision, >= 96 tokens: 128 tokens x 128 rows per workgroup, both operands staged through LDS as bfloat16, double-buffered
-//   k_dense_mfma   serving precision, 16 .. 95 tokens: 64 tokens x 64 rows per workgroup on v_mfma_f32_16x16x32_bf16; a wave owns 16 tokens and four 16-row tiles, operands go
-//                  straight from global memory into the lane layout of the instruction (A: weight row l % 16, k block l / 16; B: token l % 16, k block l / 16)
+//   k_dense_rows   one wave per output row, K spread over the lanes with 16 / 8 / 2-byte weight loads, TT tokens held in registers: the mat-vec of single tokens (weights streamed once from HBM:
+//                  6.7 TB/s at 32000 x 4096, 4.3 at 4096 x 4096, 4 us of launch below 1024 x 1024) and every width of the fp32 mode
+//   k_dense_split  serving precision, 2 .. 32 tokens: 16 or 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (4.6 TB/s at 32000 x 4096 and up to
+//                  8 tokens).  On the mat-vec every row reads all tokens' activations again, 2 T times its own bytes: 28 us for 4096 x 4096 at 8 tokens, 11 here
+//   k_dense_tile   serving precision, more tokens: tiles of 64 .. 128 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory
+//                  (26 bytes a cycle of cold weights and activations), large ones by the shared levels of memory and the steps' latency: 730 TFLOP/s at 16384 x 4096 x 2048 tokens (the tiles without
+//                  deeper prefetch and in plain order: 472), 17 us for 2048 x 2048 x 512 (82 before)
 //   k_embed        rows of the table gathered, widened and scaled
 #include "ops_common.h"
+#include "dense_tile.h"
 #include "kernel_timing.h"
 
 #include <algorithm>
+#include <type_traits>
 
-typedef __bf16 dn_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float dn_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t dn_u16x8 __attribute__((ext_vector_type(8)));
 
 static __device__ __forceinline__ float dn_widen(uint16_t b) { return __uint_as_float((uint32_t) b << 16); }
@@ -86,122 +88,113 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
     }
 }
 
-// 64 tokens x 64 rows per workgroup; K % 8 == 0, 16-byte aligned rows of W and X
-__global__ void __launch_bounds__(256) k_dense_mfma(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
-                                                    int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 1)) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int li = lane & 15, kb = lane >> 4;
-    const int64_t n0 = (int64_t) blockIdx.x * 64;
-    const int tok = blockIdx.y * 64 + wave * 16 + li;                  // the token this lane feeds as operand B
-    const bool tok_ok = tok < T;
-    const float * xrow = X + (int64_t) (tok_ok ? tok : 0) * xs;
-    const uint16_t * wrow[4]; bool row_ok[4];
+// one float4 of results (four rows of one token): bias, activation, store
+static __device__ __forceinline__ void dn_store4(dt_f32x4 v4, int64_t row, int64_t N, int tok, float * __restrict__ Y, int64_t ys, int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias) {
+    float v[4] = { v4[0], v4[1], v4[2], v4[3] };
+    if (bias || act_a != PI_ACT_NONE || act_b != PI_ACT_NONE)
 #pragma unroll
-    for (int j = 0; j < 4; j++) { const int64_t r = n0 + j * 16 + li; row_ok[j] = r < N; wrow[j] = W + (row_ok[j] ? r : 0) * K; }
-    dn_f32x4 acc[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[j] = dn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t k0 = 0; k0 < K; k0 += 32) {
-        const int64_t k = k0 + kb * 8;
-        const bool k_ok = k < K;                                       // (K % 8 == 0: a block of 8 is inside or outside as a whole)
-        dn_u16x8 b = dn_u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (k_ok && tok_ok) {
-            const float4 v0 = *(const float4 *) (xrow + k), v1 = *(const float4 *) (xrow + k + 4);
-            b[0] = (uint16_t) dn_round_bits(v0.x); b[1] = (uint16_t) dn_round_bits(v0.y); b[2] = (uint16_t) dn_round_bits(v0.z); b[3] = (uint16_t) dn_round_bits(v0.w);
-            b[4] = (uint16_t) dn_round_bits(v1.x); b[5] = (uint16_t) dn_round_bits(v1.y); b[6] = (uint16_t) dn_round_bits(v1.z); b[7] = (uint16_t) dn_round_bits(v1.w);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            dn_u16x8 a = dn_u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (k_ok && row_ok[j]) a = *(const dn_u16x8 *) (wrow[j] + k);
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_bf16x8, a), __builtin_bit_cast(dn_bf16x8, b), acc[j], 0, 0, 0);
-        }
-    }
-    // D: lane holds token l % 16 and rows (l / 16) * 4 .. + 3 of each tile
-    if (!tok_ok) return;
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int64_t row = n0 + j * 16 + kb * 4 + r;
-            if (row < N) Y[(int64_t) tok * ys + row] = dn_act(bias ? acc[j][r] + bias[row] : acc[j][r], row < rows_a ? act_a : act_b);
-        }
+    for (int r = 0; r < 4; r++) v[r] = dn_act(bias ? v4[r] + bias[min(row + r, N - 1)] : v4[r], row + r < rows_a ? act_a : act_b);
+    float * dst = Y + (int64_t) tok * ys + row;
+    if (row + 3 < N && (ys & 3) == 0 && (((uintptr_t) Y) & 15) == 0) *(float4 *) dst = make_float4(v[0], v[1], v[2], v[3]);
+    else for (int r = 0; r < 4; r++) if (row + r < N) dst[r] = v[r];
 }
 
-// 128 tokens x 128 rows per workgroup, operands staged through LDS as bfloat16 (activations are rounded once, while they are staged): a wave owns 64 x 64 = sixteen 16 x 16
-// tiles, so one K step of 32 costs it eight 16-byte LDS reads for sixteen MFMAs; the next K step's global loads are in flight while the current one is multiplied.
-// K % 8 == 0, 16-byte aligned rows of W and X.
-__global__ void __launch_bounds__(256) k_dense_mfma_lds(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
-                                                        int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, const int32_t * __restrict__ abort_w) {
+// BN rows x BT tokens per workgroup (dense_tile.h).  Workgroup n runs on XCD n % 8: an XCD takes a contiguous run of tiles, eight blocks of rows wide and then along the tokens, so that the 64 tiles it
+// works on at a time are 8 x 8 and share the rows and tokens that pass through its L2
+template <int BN, int BT, int WN, int WT, int KG>
+__global__ void __launch_bounds__(256 * KG, 2) k_dense_tile(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
+                                                       int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int tok_blocks, int tiles, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 1)) return;
-    __shared__ __attribute__((aligned(16))) uint16_t sw[2][128 * 32], sx[2][128 * 32];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
-    const int wr = wave >> 1, wt = wave & 1;                           // the wave's 64 rows / 64 tokens inside the tile
-    const int64_t n0 = (int64_t) blockIdx.x * 128;
-    const int t0 = blockIdx.y * 128;
-    // staging: thread -> (row or token tid / 2, 16 k values of half tid % 2)
-    const int sr = tid >> 1, sh = tid & 1;
-    const bool w_ok = n0 + sr < N, x_ok = t0 + sr < T;
-    const uint16_t * wsrc = W + (w_ok ? n0 + sr : 0) * K + sh * 16;
-    const float * xsrc = X + (int64_t) (x_ok ? t0 + sr : 0) * xs + sh * 16;
-    uint4 wreg[2]; float4 xreg[4];
-    auto fetch = [&](int64_t k0) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES(BN, BT, KG)];
+    const int tile = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int row_blocks = tiles / tok_blocks, grp = tile / (8 * tok_blocks), in_grp = tile % (8 * tok_blocks), gsz = min(8, row_blocks - 8 * grp);
+    const int64_t n0 = (int64_t) (8 * grp + in_grp % gsz) * BN;
+    const int t0 = (in_grp / gsz) * BT, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    const int64_t nr = min(n0 + (tid >> 3), N - 1); const int tr = min(t0 + (tid >> 3), T - 1);
+    dt_offs wo, xo;                                                    // the rows this thread stages, from the first
 #pragma unroll
-        for (int i = 0; i < 2; i++) wreg[i] = (w_ok && k0 + sh * 16 + i * 8 < K) ? *(const uint4 *) (wsrc + k0 + i * 8) : make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < BN / 32; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, N - 1) - nr) * K);
 #pragma unroll
-        for (int i = 0; i < 4; i++) xreg[i] = (x_ok && k0 + sh * 16 + i * 4 < K) ? *(const float4 *) (xsrc + k0 + i * 4) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    };
-    auto stage = [&](int buf) {
-        *(uint4 *) (sw[buf] + sr * 32 + sh * 16) = wreg[0]; *(uint4 *) (sw[buf] + sr * 32 + sh * 16 + 8) = wreg[1];
-        uint32_t pk[8];
+    for (int i = 0; i < BT / 32; i++) xo[i] = (uint32_t) ((min(tr + 32 * i, T - 1) - tr) * xs);
+    dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
+    dt_tile<BN, BT, WN, WT, 2, KG, false>(W + nr * K, wo, X + (int64_t) tr * xs, xo, 0, [](float a, float) { return a; }, K, lds, acc);
+    if (KG > 1 && threadIdx.x >= 256) return;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            pk[2 * i]     = dn_round_bits(xreg[i].x) | dn_round_bits(xreg[i].y) << 16;
-            pk[2 * i + 1] = dn_round_bits(xreg[i].z) | dn_round_bits(xreg[i].w) << 16;
-        }
-        *(uint4 *) (sx[buf] + sr * 32 + sh * 16) = make_uint4(pk[0], pk[1], pk[2], pk[3]); *(uint4 *) (sx[buf] + sr * 32 + sh * 16 + 8) = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-    };
-    dn_f32x4 acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = dn_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    fetch(0);
-    stage(0);
-    __syncthreads();
-    int buf = 0;
-    for (int64_t k0 = 0; k0 < K; k0 += 32) {
-        const bool more = k0 + 32 < K;
-        if (more) fetch(k0 + 32);
-        dn_u16x8 af[4], bf[4];
-#pragma unroll
-        for (int a = 0; a < 4; a++) af[a] = *(const dn_u16x8 *) (sw[buf] + (wr * 64 + a * 16 + li) * 32 + kb * 8);
-#pragma unroll
-        for (int b = 0; b < 4; b++) bf[b] = *(const dn_u16x8 *) (sx[buf] + (wt * 64 + b * 16 + li) * 32 + kb * 8);
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dn_bf16x8, af[a]), __builtin_bit_cast(dn_bf16x8, bf[b]), acc[a][b], 0, 0, 0);
-        if (more) stage(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
-    }
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        const int tok = t0 + wt * 64 + b * 16 + li;
+    for (int b = 0; b < BT / WT / 16; b++) {
+        const int tok = t0 + (wave % WT) * (BT / WT) + b * 16 + (lane & 15);
         if (tok >= T) continue;
 #pragma unroll
-        for (int a = 0; a < 4; a++) {
-            const int64_t row = n0 + wr * 64 + a * 16 + kb * 4;
-            float v[4];
+        for (int a = 0; a < BN / WN / 16; a++) dn_store4(acc[a][b], n0 + (wave / WT) * (BN / WN) + a * 16 + (lane >> 4) * 4, N, tok, Y, ys, act_a, rows_a, act_b, bias);
+    }
+}
+
+// 2 .. 64 tokens: RT x 16 rows and TT x 16 tokens per workgroup, K split over its eight waves, which meet in LDS.  The weights are streamed once, straight from memory in the operand's lane layout: the
+// four lanes of a row take 64 consecutive bytes of it per product, the activations come from L2 once per workgroup.  Rows in segments: as k_dense_rows, whole tiles
+// inside a segment (the host checks).
+template <int RT, int TT>
+__global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
+                                                     int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int64_t seg_rows, int64_t seg_off, int seg_last, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 0)) return;
+    constexpr int KS = 8;
+    __shared__ dt_f32x4 red[KS][RT * TT][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
+    const int64_t n0 = (int64_t) blockIdx.x * (16 * RT);
+    const int t0 = blockIdx.y * (16 * TT);
+    if (seg_rows > 0) X += min(n0 / seg_rows, (int64_t) seg_last) * seg_off;
+    const int64_t per = (K + 64 * KS - 1) / (64 * KS) * 64, k_begin = wave * per, k_end = min(K, k_begin + per);
+    const uint16_t * wrow[RT]; const float * xrow[TT];
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = dn_act(bias ? acc[a][b][r] + bias[min(row + r, N - 1)] : acc[a][b][r], row + r < rows_a ? act_a : act_b);
-            float * dst = Y + (int64_t) tok * ys + row;
-            if (row + 3 < N && (ys & 3) == 0 && (((uintptr_t) Y) & 15) == 0) *(float4 *) dst = make_float4(v[0], v[1], v[2], v[3]);
-            else for (int r = 0; r < 4; r++) if (row + r < N) dst[r] = v[r];
+    for (int a = 0; a < RT; a++) wrow[a] = W + min(n0 + a * 16 + li, N - 1) * K + kb * 8;
+#pragma unroll
+    for (int b = 0; b < TT; b++) xrow[b] = X + (int64_t) min(t0 + b * 16 + li, T - 1) * xs + kb * 8;
+    dt_f32x4 acc[RT][TT];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < TT; b++) acc[a][b] = dt_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const dt_u32x4 zero4 = { 0, 0, 0, 0 }; const dt_f32x4 zerof = { 0.0f, 0.0f, 0.0f, 0.0f };
+    constexpr int U = RT * TT == 1 ? 4 : RT * TT == 2 ? 2 : 1;                   // steps of 64 whose loads go out together
+    auto steps = [&](auto n_steps, int64_t k, bool ok0, bool ok1) {
+        constexpr int NS = decltype(n_steps)::value;
+        dt_u32x4 af[NS][RT][2]; dt_f32x4 xf[NS][TT][4];
+#pragma unroll
+        for (int u = 0; u < NS; u++) {
+#pragma unroll
+            for (int a = 0; a < RT; a++) { af[u][a][0] = ok0 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u) : zero4; af[u][a][1] = ok1 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u + 32) : zero4; }
+#pragma unroll
+            for (int b = 0; b < TT; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) xf[u][b][i] = (i < 2 ? ok0 : ok1) ? *(const dt_f32x4 *) (xrow[b] + k + 64 * u + (i < 2 ? 0 : 24) + 4 * i) : zerof;
         }
+        __builtin_amdgcn_sched_barrier(0);                             // (all of them issued before the first product waits)
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+#pragma unroll
+            for (int b = 0; b < TT; b++) {
+                const dt_u32x4 b0 = dt_pack8(xf[u][b][0], xf[u][b][1]), b1 = dt_pack8(xf[u][b][2], xf[u][b][3]);
+#pragma unroll
+                for (int a = 0; a < RT; a++) { acc[a][b] = dt_mfma(af[u][a][0], b0, acc[a][b]); acc[a][b] = dt_mfma(af[u][a][1], b1, acc[a][b]); }
+            }
+    };
+    using one = std::integral_constant<int, 1>;
+    int64_t k = k_begin;
+    if constexpr (U > 1) for (; k + 64 * U <= k_end; k += 64 * U) steps(std::integral_constant<int, U>{}, k, true, true);
+    for (; k + 64 <= k_end; k += 64) steps(one{}, k, true, true);
+    if (k < k_end) steps(one{}, k, k + kb * 8 < K, k + kb * 8 + 32 < K);       // (K % 8 == 0)
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < TT; b++) red[wave][a * TT + b][lane] = acc[a][b];
+    __syncthreads();
+    for (int i = tid; i < RT * TT * 64; i += 512) {
+        const int tile = i >> 6, l = i & 63, tok = t0 + (tile % TT) * 16 + (l & 15);
+        if (tok >= T) continue;
+        dt_f32x4 v = red[0][tile][l];
+#pragma unroll
+        for (int w = 1; w < KS; w++) v += red[w][tile][l];
+        const int64_t row = n0 + (tile / TT) * 16 + (l >> 4) * 4;
+        if (row < N) dn_store4(v, row, N, tok, Y, ys, act_a, rows_a, act_b, bias);
     }
 }
 
@@ -212,8 +205,6 @@ extern "C" int pi_op_embed(const pi_weight * w, const int32_t * tokens, int n_to
     PI_CHECK_LAUNCH(); return 0;
 }
 
-static int dense_mfma_min_tokens() { static const int v = getenv("PI_DENSE_MFMA_MIN") ? atoi(getenv("PI_DENSE_MFMA_MIN")) : 16; return v; }
-
 template <int VW, bool EXACT>
 static void launch_rows(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias = nullptr, int64_t seg_rows = 0, int64_t seg_off = 0, int seg_last = 0) {
     const uint16_t * W = (const uint16_t *) w->p0;
@@ -222,6 +213,36 @@ static void launch_rows(const pi_weight * w, const float * x, int64_t xs, int n_
     if (n_tok == 1)      PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, nt_acct, bytes, (k_dense_rows<1, VW, EXACT>), dim3(gx, 1), dim3(256), 0, s, W, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word());
     else if (n_tok <= 4) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, nt_acct, bytes, (k_dense_rows<4, VW, EXACT>), dim3(gx, 1), dim3(256), 0, s, W, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word());
     else PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, nt_acct, bytes, (k_dense_rows<8, VW, EXACT>), dim3(gx, (unsigned) ((n_tok + 7) / 8)), dim3(256), 0, s, W, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word());
+}
+
+// Which kernel takes a pass of serving precision (aligned rows; measured against each other over 512 .. 32000 rows, K 1024 .. 4096, us):
+//   1 token                the mat-vec; 2 tokens of a matrix of at most 4 M values too (2048 x 2048: 5.5, k_dense_split 5.7: both at the floor of a launch)
+//   .. 32 tokens           k_dense_split (4096 x 4096 at 4 / 8 / 16 / 32 tokens: 9.7 / 11 / 14 / 21; the mat-vec 15 / 28 at 4 / 8, k_dense_tile 27 at 32); of 16384 rows and more only .. 8 tokens, where the tiles
+//                          fill the chip and read the activations less often (32000 x 2048 at 24: 41 against 26)
+//   more                   k_dense_tile
+static bool dense_takes_split(int64_t rows, int64_t k, int n_tok) { return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32) && !(n_tok == 2 && rows * k <= (4 << 20)); }
+// 32 rows per workgroup where that still leaves a workgroup per compute unit; at up to four tokens long rows rather take twice the workgroups (8192 x 4096 at 2 tokens: 14.7 against 16.7; 32000 x 2048: 31 against 24)
+static void launch_split(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias, int64_t seg_rows = 0,
+                         int64_t seg_off = 0, int seg_last = 0) {
+    const bool two = w->ne1 >= 8192 && (n_tok > 4 || w->ne0 < 4096);
+#define DN_SPLIT(RT, TT) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_split<RT, TT>), dim3((unsigned) ((w->ne1 + 16 * RT - 1) / (16 * RT)), (unsigned) ((n_tok + 16 * TT - 1) / (16 * TT))), \
+                                     dim3(512), 0, s, (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word())
+    if (n_tok <= 16) { if (two) DN_SPLIT(2, 1); else DN_SPLIT(1, 1); }
+    else { if (two) DN_SPLIT(2, 2); else DN_SPLIT(1, 2); }
+#undef DN_SPLIT
+}
+// The largest tile that gives the chip's 256 compute units one workgroup each; where the next larger one would not, two groups of waves share K (measured at 512 .. 32000 rows x 24 .. 2048 tokens; the crossings:
+// 2048 x 2048 at 512 tokens 64 x 64 in two groups 17.1, one 18.6, 128 x 64 21.1; at 1000 128 x 64 in two groups 24.3, one 25.9, 64 x 64 27.9, 128 x 128 34.6; 6144 x 2048 at 512 128 x 64 39.1, 128 x 128 41.9;
+// 8192 x 4096 at 1000 128 x 128 108, 128 x 64 129)
+static void launch_tile(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias) {
+    auto tiles = [&](int bn, int bt) { return (w->ne1 + bn - 1) / bn * ((n_tok + bt - 1) / bt); };
+#define DN_TILE(BN, BT, KG) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_tile<BN, BT, 2, 2, KG>), dim3((unsigned) ((tiles(BN, BT) + 7) / 8 * 8)), dim3(256 * KG), 0, s, \
+                     (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, (n_tok + BT - 1) / BT, (int) tiles(BN, BT), pi_abort_word())
+    if (tiles(64, 64) <= 256) DN_TILE(64, 64, 2);
+    else if (tiles(128, 64) <= 256) DN_TILE(128, 64, 2);
+    else if (tiles(128, 128) <= 256) DN_TILE(128, 64, 1);
+    else DN_TILE(128, 128, 1);
+#undef DN_TILE
 }
 
 extern "C" int pi_op_dense(const pi_weight * w, const float * x, int64_t x_stride, int n_tok, float * out, int64_t out_stride, int act_a, int64_t rows_a, int act_b, int exact, void * stream) {
@@ -236,15 +257,9 @@ extern "C" int pi_op_dense_bias(const pi_weight * w, const float * bias, const f
     const double bytes = 2.0 * K * w->ne1 + 4.0 * n_tok * (K + w->ne1);
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
     const bool al8  = K % 4 == 0 && ((uintptr_t) w->p0 % 8) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
-    static const int lds_min = getenv("PI_DENSE_LDS_MIN") ? atoi(getenv("PI_DENSE_LDS_MIN")) : 96;
-    if (!exact && al16 && n_tok >= lds_min) {
-        PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, k_dense_mfma_lds, dim3((unsigned) ((w->ne1 + 127) / 128), (unsigned) ((n_tok + 127) / 128)), dim3(256), 0, s,
-                     (const uint16_t *) w->p0, K, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, pi_abort_word());
-        PI_CHECK_LAUNCH(); return 0;
-    }
-    if (!exact && al16 && n_tok >= dense_mfma_min_tokens()) {
-        PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, k_dense_mfma, dim3((unsigned) ((w->ne1 + 63) / 64), (unsigned) ((n_tok + 63) / 64)), dim3(256), 0, s,
-                     (const uint16_t *) w->p0, K, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, pi_abort_word());
+    if (!exact && al16 && (n_tok > 2 || dense_takes_split(w->ne1, K, n_tok))) {
+        if (dense_takes_split(w->ne1, K, n_tok)) launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
+        else launch_tile(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
         PI_CHECK_LAUNCH(); return 0;
     }
     if (al16 && K >= 512) { if (exact) launch_rows<8, true>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); else launch_rows<8, false>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); }
@@ -263,7 +278,11 @@ extern "C" int pi_op_dense_segments(const pi_weight * w, const float * x, int64_
     const int64_t K = w->ne0;
     if (x_stride < (int64_t) (n_seg - 1) * seg_off + K || out_stride < w->ne1) { pi_set_error("pi_op_dense_segments: row strides below the sizes"); return -1; }
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0 && seg_off % 4 == 0;
-    if (exact || !al16 || n_tok < dense_mfma_min_tokens()) {
+    if (!exact && al16 && dense_takes_split(w->ne1, K, n_tok) && seg_rows % 32 == 0) {
+        launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, (hipStream_t) stream, 2.0 * K * w->ne1 + 4.0 * n_tok * (n_seg * K + w->ne1), nullptr, seg_rows, seg_off, n_seg - 1);
+        PI_CHECK_LAUNCH(); return 0;
+    }
+    if (exact || !al16 || n_tok < 16) {
         const bool al8 = K % 4 == 0 && ((uintptr_t) w->p0 % 8) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0 && seg_off % 4 == 0;
         const double bytes = 2.0 * K * w->ne1 + 4.0 * n_tok * (n_seg * K + w->ne1);
         hipStream_t s = (hipStream_t) stream;

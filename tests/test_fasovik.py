@@ -186,6 +186,45 @@ def test_dense_every_kernel_and_width(K, N, T, exact):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,N,T", [(8, 1, 2), (72, 33, 16), (1096, 130, 17), (520, 8193, 32), (4104, 8200, 3), (64, 16, 33), (1000, 70, 65), (2048, 16390, 9),
+                                   (200, 2100, 520), (136, 4100, 600), (72, 8200, 600)])
+def test_dense_on_the_matrix_cores(K, N, T):
+    """16-byte aligned rows: k_dense_split (one / two tiles of rows and of tokens; K that ends inside a step, or before some of the waves' shares begin) and k_dense_tile (64 x 64 and 128 x 64 with K over
+    two groups of waves, 128 x 64 and 128 x 128), rows and tokens that end inside a tile, padded strides, a bias and both activations.  Sums of K products of bfloat16 values in fp32: 2e-6 as above"""
+    U, lib = gpu()
+    rng = np.random.default_rng(K + N + T)
+    w, x, b = bf(rng, N, K, s=0.2), rng.standard_normal((T, K + 8)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    wd, xd, bd, od = upload_bf16(lib, w), U.Dev(x), U.Dev(b), U.Dev(nbytes=4 * T * (N + 5))
+    z = O.bf16_round(x[:, :K]).astype(np.float64) @ w.astype(np.float64).T
+    for os_, bias, act_a, rows_a, act_b in ((N, None, 0, N, 0), (N + 5, bd.ptr, 1, N // 2, 3)):
+        L.check(lib.pi_op_dense_bias(wd, bias, xd.ptr, K + 8, T, od.ptr, os_, act_a, rows_a, act_b, 0, None))
+        got, want = od.get(np.float32)[:T * os_].reshape(T, os_)[:, :N], z + b if bias else z
+        if act_a:
+            want = np.concatenate([O.silu(want[:, :rows_a]), np.maximum(want[:, rows_a:], 0) ** 2], axis=1)
+        assert rel_rms(got, want) < 2e-6, (os_, rel_rms(got, want))
+        assert np.abs(got - want).max() < 1e-4 * np.abs(want).max()                  # (no single tile, row or token left out)
+    lib.pi_weight_free(wd)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 9, 30, 70])
+def test_dense_segments_on_the_matrix_cores(T):
+    """segments of whole row tiles in one k_dense_split launch, more tokens a tile launch each"""
+    U, lib = gpu()
+    rng = np.random.default_rng(T)
+    K, seg, last, n_seg = 136, 64, 24, 4
+    rows = (n_seg - 1) * seg + last
+    w, x = bf(rng, rows, K, s=0.2), rng.standard_normal((T, n_seg * K)).astype(np.float32)
+    wd, xd, od = upload_bf16(lib, w), U.Dev(x), U.Dev(nbytes=4 * T * rows)
+    L.check(lib.pi_op_dense_segments(wd, xd.ptr, n_seg * K, seg, K, n_seg, T, od.ptr, rows, 0, rows - last, 4, 0, None))
+    xin = O.bf16_round(x).astype(np.float64)
+    want = np.concatenate([xin[:, g * K:(g + 1) * K] @ w[g * seg:min((g + 1) * seg, rows)].T.astype(np.float64) for g in range(n_seg)], axis=1)
+    want[:, rows - last:] = np.tanh(want[:, rows - last:])
+    assert rel_rms(od.get(np.float32, (T, rows)), want) < 2e-6
+    lib.pi_weight_free(wd)
+
+
+@pytest.mark.gpu
 def test_embedding_rows_are_scaled():
     U, lib = gpu()
     rng = np.random.default_rng(1)
