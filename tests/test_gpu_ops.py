@@ -412,6 +412,33 @@ def test_elementwise_exact(gpu):
     assert np.array_equal(od.get(np.float32).view(np.uint32), o.silu(allx).view(np.uint32))
 
 
+@pytest.mark.parametrize("n_vocab", [5, 40, 2049, 32000, 32769, 65537, 70001])
+def test_topk_edges(gpu, n_vocab):
+    """every instance (8, 16, 32 values per lane, re-read from memory), slices that end early or are empty; rows of equal values, of -inf, with values that are not numbers, with both zeros"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(n_vocab)
+    x = (rng.standard_normal((7, n_vocab)) * 3).astype(np.float32)
+    x[1] = 1.5
+    x[2] = -np.inf
+    x[3, ::2] = np.nan
+    x[4] = np.where(np.arange(n_vocab) % 3 == 0, np.float32(-0.0), np.float32(0.0))
+    x[5] = np.round(x[5])                                            # many ties
+    x[6] = -np.inf
+    x[6, n_vocab // 2] = -2.0
+    ld, ids, vals, se, scr = U.Dev(x), U.Dev(nbytes=4 * 7 * 8), U.Dev(nbytes=4 * 7 * 8), U.Dev(nbytes=4 * 7), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(7))
+    L.check(lib.pi_op_topk(ld.ptr, n_vocab, 7, 8, ids.ptr, vals.ptr, se.ptr, scr.ptr, None))
+    gi, gv, gs = ids.get(np.int32, (7, 8)), vals.get(np.float32, (7, 8)), se.get(np.float32)
+    for t in range(7):
+        num = np.flatnonzero(~np.isnan(x[t]))
+        order = num[np.lexsort((num, -x[t][num]))][:8]
+        assert list(gi[t][:len(order)]) == list(order) and np.array_equal(gv[t][:len(order)].view(np.uint32), x[t][order].view(np.uint32)), t
+        assert (gi[t][len(order):] == 0x7fffffff).all() and (gv[t][len(order):] == -np.inf).all()
+        if t in (0, 1, 4, 5, 6):                                     # (fp32 sum of up to 70001 terms in pairs per slice)
+            want = np.exp((x[t] - x[t].max()).astype(np.float64)).sum()
+            assert abs(gs[t] - want) / want < 1e-5
+
+
 @pytest.mark.parametrize("n_vocab", [512, 32000, 65024])
 def test_topk(gpu, n_vocab):
     lib, U = gpu
