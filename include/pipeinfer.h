@@ -65,7 +65,7 @@ struct pi_kt_row;
 LLAMA_API int pipeinfer_get_launch_rows(struct llama_context * ctx, struct pi_kt_row * out, int cap);
 /* Run tap (tests: per-run oracle comparison of whatever schedule the context runs — segments, feeder, coalesced passes).  Called on the CALLER's thread, twice per run:
  * from llama_start_async_decode with logits == NULL, and from llama_finish_async_decode with the run's rows [n_tokens][n_vocab] (NULL again when the run produced none:
- * cancelled before or after its start, or a failed launch).  meta = the run's own metadata block (tokens | pos | {kv_head, n_kv, n_tokens, 0} | mask rows), valid during the call. */
+ * cancelled before or after its start, or a failed launch; or when the tap was not set yet as the run was started: only the rows its caller asked for came back).  meta = the run's own metadata block (tokens | pos | {kv_head, n_kv, n_tokens, 0} | mask rows), valid during the call. */
 typedef void (*pipeinfer_run_tap_fn)(void * user, int32_t run_id, int32_t batch_id, int32_t n_tokens, const void * meta, size_t meta_bytes, const float * logits);
 LLAMA_API void pipeinfer_context_set_run_tap(struct llama_context * ctx, pipeinfer_run_tap_fn fn, void * user);
 

@@ -240,6 +240,7 @@ struct pi_run {                                // one llama_start_async_decode .
     hipEvent_t done = nullptr, begin = nullptr;
     float * logits_host = nullptr;            // pinned [n_tokens][n_vocab]
     size_t logits_cap = 0;
+    bool all_rows = false;                    // every row comes back to logits_host, not only the wanted ones (a run tap was set when the run was started)
     int32_t * topk_ids = nullptr; float * topk_vals = nullptr; float * topk_sum = nullptr;   // pinned [n_tokens][8], [n_tokens]
     uint8_t * meta_host = nullptr; size_t meta_cap = 0;                                       // pinned staging for tokens/pos/mask
     int64_t t_start_us = 0;

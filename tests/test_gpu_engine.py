@@ -861,3 +861,32 @@ def test_pipeinfer_driver_is_lossless_with_run_coalescing(LL, tgt, dft, n_draft,
         c.free()
     for m in (mt, md):
         m.free()
+
+
+@pytest.mark.parametrize("wanted", [[], [11], [0], [0, 1, 2, 11], [3, 5, 6, 9], list(range(0, 24, 2)), list(range(24))])
+def test_only_the_wanted_rows_come_back(LL, wanted):
+    """llama_batch.logits: the flagged rows are those of a pass that wants all of them (one range, several, more than eight: from the first to the last), the top-8 of every row comes back whatever was
+    flagged, and a run tap still gets every row"""
+    m = LL.Model(os.path.join(GOLD, "tiny_llama_q4_k_m.gguf"))
+    n = 24
+    toks = [int(t) for t in np.random.default_rng(5).integers(3, m.n_vocab, n)]
+    ctx = LL.Context(m, n_ctx=64, n_batch=32)
+    full = ctx.decode(toks, list(range(n)), [[0]] * n)
+    tops = [ctx.topk(i) for i in range(n)]
+
+    def again():
+        ctx.kv_clear()
+        b = LL.Batch(toks, list(range(n)), [[0]] * n)
+        b.lg[:] = 0
+        b.lg[wanted] = 1
+        assert ctx.lib.llama_decode(ctx.h, b.c) == 0
+        return ctx.logits(n)
+    got = again()
+    assert np.array_equal(got[wanted].view(np.uint32), full[wanted].view(np.uint32))
+    assert [ctx.topk(i) for i in range(n)] == tops
+    seen = []
+    ctx.set_run_tap(lambda run_id, batch_id, k, block, rows: seen.append(rows))
+    again()
+    ctx.set_run_tap(None)
+    assert len(seen) == 2 and seen[0] is None and np.array_equal(seen[1].view(np.uint32), full.view(np.uint32))
+    ctx.free(); m.free()
