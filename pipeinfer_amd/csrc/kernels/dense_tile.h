@@ -22,15 +22,18 @@ static __device__ __forceinline__ dt_u32x4 dt_pack8(dt_f32x4 a, dt_f32x4 b) { re
 static __device__ __forceinline__ dt_f32x4 dt_mfma(dt_u32x4 a, dt_u32x4 b, dt_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dt_bf16x8, a), __builtin_bit_cast(dt_bf16x8, b), c, 0, 0, 0); }
 
 #define DT_LDS_BYTES(BN, BT, KG) ((KG) * 2 * ((BN) + (BT)) * 128)
+#define DT_LDS_BYTES_PL(BN, BT, PL) (2 * ((BN) + (PL) * (BT)) * 128)
 
 // w + wo[i] / x + xo[i]: the rows this thread stages, numbers tid / 8 + 32 i of the tile (16-byte aligned; rows past the end repeat a valid one and are not stored); K % 8 == 0.
+// PL = 3: X is not rounded but taken apart into three bfloat16 values that add up to it, three products instead of one: the products are exact, as an fp32 one of the two factors is.
 // PAIR: an X value is join(x[k], x[k + pair_off]) of two fp32 values (the two halves of a gated hidden layer).  On return lane l of wave (wn, wt) holds in acc[a][b] the rows
 // wn BN / WN + 16 a + 4 (l / 16) .. + 3 of token wt BT / WT + 16 b + l % 16.
-template <int BN, int BT, int WN, int WT, int D, int KG, bool PAIR, class Join>
+template <int BN, int BT, int WN, int WT, int D, int KG, bool PAIR, int PL = 1, class Join>
 static __device__ __forceinline__ void dt_tile(const uint16_t * __restrict__ w, dt_offs wo, const float * __restrict__ x, dt_offs xo, int64_t pair_off, Join join, int64_t K, uint8_t * lds,
                                                dt_f32x4 (&acc)[BN / WN / 16][BT / WT / 16]) {
+    static_assert(PL == 1 || KG == 1, "one group of waves where X is in three parts");
     static_assert(D % 2 == 0, "an even number of register sets: a step's buffer is known when the code is compiled");
-    constexpr int NW = BN / 32, NX = BT / 32, RT = BN / WN / 16, TT = BT / WT / 16, BUF = (BN + BT) * 128;
+    constexpr int NW = BN / 32, NX = BT / 32, RT = BN / WN / 16, TT = BT / WT / 16, BUF = (BN + PL * BT) * 128;
     const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4, kg = KG > 1 ? threadIdx.x >> 8 : 0;
     uint8_t * const all = lds;
     lds += kg * (2 * BUF);
@@ -79,7 +82,12 @@ static __device__ __forceinline__ void dt_tile(const uint16_t * __restrict__ w, 
 #pragma unroll
                     for (int e = 0; e < 4; e++) a[e] = join(a[e], yreg[i][h][e]);
                 }
-                *(dt_u32x2 *) (base + BN * 128 + i * 4096 + (h ? place_x ^ 64 : place_x)) = dt_u32x2{ dt_pack(a[0], a[1]), dt_pack(a[2], a[3]) };
+#pragma unroll
+                for (int p = 0; p < PL; p++) {
+                    const dt_u32x2 b = { dt_pack(a[0], a[1]), dt_pack(a[2], a[3]) };
+                    *(dt_u32x2 *) (base + (BN + p * BT) * 128 + i * 4096 + (h ? place_x ^ 64 : place_x)) = b;
+                    if constexpr (PL > 1) a -= dt_f32x4{ __uint_as_float(b[0] << 16), __uint_as_float(b[0] & 0xffff0000u), __uint_as_float(b[1] << 16), __uint_as_float(b[1] & 0xffff0000u) };
+                }
             }
     };
 #pragma unroll
@@ -111,11 +119,14 @@ static __device__ __forceinline__ void dt_tile(const uint16_t * __restrict__ w, 
 #pragma unroll
                 for (int a = 0; a < RT; a++) af[a] = *(const dt_u32x4 *) (wb + a * 2048 + at);
 #pragma unroll
-                for (int b = 0; b < TT; b++) bf[b] = *(const dt_u32x4 *) (xb + b * 2048 + at);
+                for (int p = 0; p < PL; p++) {
 #pragma unroll
-                for (int a = 0; a < RT; a++)
+                    for (int b = 0; b < TT; b++) bf[b] = *(const dt_u32x4 *) (xb + p * BT * 128 + b * 2048 + at);
 #pragma unroll
-                    for (int b = 0; b < TT; b++) acc[a][b] = dt_mfma(af[a], bf[b], acc[a][b]);
+                    for (int a = 0; a < RT; a++)
+#pragma unroll
+                        for (int b = 0; b < TT; b++) acc[a][b] = dt_mfma(af[a], bf[b], acc[a][b]);
+                }
             }
             __syncthreads();
         }

@@ -13,6 +13,7 @@
 //   k_moe_up / _down     the chosen experts of every token (gathered mat-vecs), identity experts pass their input through
 #include "ops_common.h"
 #include "kernel_timing.h"
+#include "prompt_attention.h"
 
 #include <algorithm>
 #include <cmath>
@@ -718,7 +719,7 @@ extern "C" int pi_op_copy_f32(const float * src, float * dst, int64_t n, void * 
 // feeds M accumulators, the M queries come through wave-uniform (scalar) loads — and a slice of the latent's rank in the value phase, where the probabilities of a cell are
 // broadcast from LDS to M x RPT accumulators; every split leaves an un-normalised partial (max, sum, sum of p * c) in scratch.  (3) k_latent_combine merges the splits with
 // the sink term, normalises and applies the value up-projection.  K / V are never materialised; single tokens are spread over the chip by the splits (64 cells each),
-// prompts take splits only when a score row would not fit LDS.
+// longer passes take splits only when a score row would not fit LDS.  A pass of 9 tokens and more takes these kernels where sizes, alignment or scratch memory keep it off prompt_attention.hip.
 // A cached row is [latent (rank) | rotated key part (rot values, shared by the heads; none by default)]: the folded query carries its own rotated part behind the rank values, so a score is one
 // dot product over the row's width; only the latent is summed with the probabilities.  Which cells a token sees is the mask's alone (a window of positions: pi_op_window_mask).
 // scratch (floats): qa [n_tok][heads][rank + rot] | pol [n_tok][heads][S][rank] | pml [n_tok][heads][S][2]
@@ -1049,6 +1050,27 @@ extern "C" int pi_op_latent_attention_rot(const float * q, int64_t q_stride, con
     return pi_op_latent_attention_gated(q, q_stride, cache, mask, wuk, wuv, sink_dev, gate_dev, gate_stride, gate_act, 1, scale, heads, dim, rot, vdim, rank, rotary_table, PI_PAIR_NEIGHBOURS, pos_dev, n_tok, n_kv, scratch_dev,
                                         scratch_floats, out, out_stride, dyn_dev, stream);
 }
+// A prompt with its keys and values written out (prompt_attention.hip), in as few launches over the cells as the scratch memory allows; false: not for that kernel
+static bool latent_prompt(pa_args a, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, size_t scratch_floats, double bytes, hipStream_t s) {
+    if ((rank & 7) || (a.k2_row & 3) || ((uintptr_t) cache & 15) || ((uintptr_t) scratch & 15)) return false;
+    const size_t per_cell = (size_t) a.heads * (a.dim1 + a.vdim), state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3;
+    size_t cells = ((size_t) a.n_kv + 63) / 64 * 64;
+    if (cells * per_cell > scratch_floats) {
+        cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
+        if (cells < 1024) return false;
+        a.state = scratch + cells * per_cell;
+    }
+    a.k1 = scratch; a.k1_row = (int64_t) a.heads * a.dim1; a.k1_head = a.dim1;
+    a.v = scratch + cells * (size_t) a.k1_row; a.v_row = (int64_t) a.heads * a.vdim; a.v_head = a.vdim;
+    a.k2 = cache + rank;
+    if (!pa_takes(a, 1, PA_LATENT_TOKENS)) return false;
+    for (size_t c = 0; c < (size_t) a.n_kv; c += cells) {
+        a.cell0 = (int) c; a.cell1 = (int) std::min((size_t) a.n_kv, c + cells); a.first = c == 0; a.last = c + cells >= (size_t) a.n_kv;
+        pa_expand(cache, a.k2_row, rank, wuk, wuv, a.cell0, a.cell1, a.n_kv, a.dyn, scratch, scratch + cells * (size_t) a.k1_row, s);
+        pa_launch(a, 1, bytes, s);
+    }
+    return true;
+}
 extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev, const float * gate_dev,
                                             int64_t gate_stride, int gate_act, int gate_width, float scale, int heads, int dim, int rot, int vdim, int rank, const void * rotary_table, int pairing, const int32_t * pos_dev,
                                             int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride, const int32_t * dyn_dev, void * stream) {
@@ -1075,6 +1097,11 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     float * qa = scratch_dev, * pol = qa + (size_t) n_tok * heads * (rank + rot), * pml = pol + (size_t) n_tok * heads * p.S * rank;
     const int nta = std::min(n_tok, PI_KT_MAXNT - 1);
     const int acct = pi_account_n_kv() > 0 ? pi_account_n_kv() : n_kv;
+    pa_args a = {};
+    a.q = q; a.qs = q_stride; a.dim1 = dim; a.k2_row = rank + rot; a.dim2 = rot; a.vdim = vdim; a.heads = heads; a.per_kv = 1; a.n_tok = n_tok; a.n_kv = n_kv; a.dyn = dyn_dev; a.mask = mask; a.pos = rot > 0 ? pos_dev : nullptr;
+    a.cs = cs; a.n_pos = n_pos; a.pairing = pairing; a.scale = scale; a.weights = PI_WEIGHTS_SOFTMAX; a.sink = sink_dev; a.gate = gate_dev; a.gs = gate_stride; a.gate_act = gate_act; a.gate_width = gate_width; a.out_mult = 1.0f;
+    a.out = out; a.os = out_stride;
+    if (latent_prompt(a, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) { PI_CHECK_LAUNCH(); return 0; }
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * dim + 4.0 * n_tok * heads * (dim + rank + 2.0 * rot), k_latent_absorb, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((rank + 63) / 64 + (rot + 63) / 64)), dim3(256), (size_t) 16 * dim, s,
                  q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, pi_abort_word());
     PI_CHECK_LAUNCH();

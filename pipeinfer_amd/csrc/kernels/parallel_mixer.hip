@@ -12,6 +12,7 @@
 //   k_ssd_steps          dt = softplus(raw + bias), a = exp(-exp(A_log) * dt)
 //   k_gate_group_norm    u = y * silu(z); each of `groups` equal parts of u divided by its root mean square; * w * mult
 #include "ops_common.h"
+#include "prompt_attention.h"
 #include "kernel_timing.h"
 
 #include <algorithm>
@@ -561,6 +562,14 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
     if (maps * hpg * vdim > 256 * CA_MAXOUT || lds > 60 * 1024) { pi_set_error("pi_op_chunk_attention: %d query heads per key head of sizes %d / %d are beyond the kernel (LDS %zu bytes)", hpg, dim, vdim, lds); return -1; }
     const int acct = pi_account_n_kv() > 0 ? pi_account_n_kv() : n_kv;
     const double visible = chunk > 0 ? std::min(acct, chunk) + (pool > 0 ? std::max(acct - chunk, 0) / pool : std::min(std::max(acct - chunk, 0), keep_first)) : acct;
+    if (pool == 0 && !pool_here) {                                     // a prompt: 32 tokens of a head at a time
+        pa_args a = {};
+        a.q = q; a.qs = q_stride; a.k1 = k_cache; a.k1_row = (int64_t) kv_heads * maps * dim; a.k1_head = (int64_t) maps * dim; a.dim1 = dim; a.v = v_cache; a.v_row = (int64_t) kv_heads * vdim; a.v_head = vdim; a.vdim = vdim;
+        a.cell1 = n_kv; a.heads = heads; a.per_kv = heads / kv_heads; a.n_tok = n_tok; a.n_kv = n_kv; a.dyn = dyn_dev; a.mask = mask_dev; a.cell_pos = cell_pos_dev; a.pos = pos_dev; a.mask_kind = mask_kind; a.chunk = chunk;
+        a.keep_first = keep_first; a.scale = scale; a.hbias = head_bias_dev; a.softcap = softcap; a.weights = weights; a.sink = sink_dev; a.gate = gate_dev; a.gs = gate_stride; a.gate_act = gate_act; a.gate_width = 1;
+        a.out_mult = out_mult; a.lam = mp.lam; a.eps = mp.eps; a.out = out; a.os = out_stride; a.first = a.last = 1;
+        if (pa_takes(a, maps, PA_CACHE_TOKENS)) { pa_launch(a, maps, 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (hipStream_t) stream); PI_CHECK_LAUNCH(); return 0; }
+    }
 #define CA_GO(R, MP)     PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (k_chunk_attention<R, MP>), dim3((unsigned) n_tok, (unsigned) kv_heads, (unsigned) (n_z * n_cs + (pool_here ? 1 : 0))), dim3(256), lds, \
                  (hipStream_t) stream, q, q_stride, k_cache, v_cache, cell_pos_dev, mask_dev, pos_dev, head_bias_dev, gate_dev, gate_stride, gate_act, scale, out_mult, weights, softcap, chunk, heads, kv_heads, dim, vdim, n_kv, tile, hpg, out, out_stride, \
                  dyn_dev, sink_dev, mask_kind, pool, (int) pooled_row_offset, pool_here ? n_z * n_cs : 0, n_z, n_cs, split_cells, scratch, keep_first, mp, pi_abort_word());

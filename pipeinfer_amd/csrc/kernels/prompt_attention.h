@@ -1,0 +1,32 @@
+// Attention of a prompt's many tokens on the matrix cores (prompt_attention.hip): what the operators of hybrid.hip and parallel_mixer.hip hand over.  Internal to the kernels.
+#pragma once
+#include "ops_common.h"
+
+struct pa_args {
+    const float * q; int64_t qs;                                       // [token][qs]: heads of MAPS x (dim1 + dim2) values
+    const float * k1; int64_t k1_row, k1_head; int dim1;               // a cell's key: dim1 values of its head at k1 + cell * k1_row + (head / per_kv) * k1_head, ...
+    const float * k2; int64_t k2_row; int dim2;                        // ... then dim2 values that the heads share
+    const float * v; int64_t v_row, v_head; int vdim;
+    int cell0, cell1;                                                  // the cells of this launch; k1 and v begin at cell0, everything else at cell 0
+    int heads, per_kv, n_tok, n_kv; const int32_t * dyn;
+    const uint32_t * mask; const int32_t * cell_pos, * pos;            // cell_pos null: what a token sees is the mask's alone
+    int mask_kind, chunk, keep_first;
+    const float2 * cs; int n_pos, pairing;                             // dim2 > 0: the query's last dim2 values are turned by the token's position
+    float scale; const float * hbias; float softcap; int weights; const float * sink;
+    const float * gate; int64_t gs; int gate_act, gate_width;
+    float out_mult, lam, eps;
+    float * out; int64_t os;
+    float * state; int first, last;                                    // the cells in several launches: [token][head][vdim sums | maximum | denominator] between them
+};
+// a launch over the cells [cell0, cell1); maps = 2: see ca_join_maps.  false: sizes or alignment that the kernel does not take (pa_takes)
+bool pa_takes(const pa_args & a, int maps, int min_tokens);
+void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s);
+// Which passes take tiles of 32 tokens rather than a workgroup per token (measured against each other over 9 .. 128 tokens, 16 and 32 heads, contexts of the pass's own tokens, 512 .. 1000 and 4096 cells, us):
+//   keys in a cache     from 32 tokens on: 16 heads of 128 over 4: 32 tokens in a window of 256 of 1000 cells 84 -> 47, all of 4096 cells 1082 -> 359, but 18 -> 23 where they are alone in the cache; 128 tokens
+//                       alone 38 -> 24.  With 16 tokens the per-token kernel cuts the cells into splits: 32 against 41
+//   keys of a latent    from 9 tokens on (fewer: splits of 64 cells): 16 heads of 128, rank 512: 9 tokens alone 74 -> 27, of 512 cells 179 -> 65, of 4096 440 -> 379; 128 tokens 123 -> 38, 213 -> 69, 836 -> 374.
+//                       (32 heads of 192, 4096 cells: 9 .. 32 tokens 469 -> 515, from 48 on 898 -> 511)
+#define PA_CACHE_TOKENS 32
+#define PA_LATENT_TOKENS 9
+// keys [cell][heads * dim] and values [cell][heads * vdim] of the cells [cell0, cell1) from their latents (row stride `width` floats)
+void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, const int32_t * dyn, float * k, float * v, hipStream_t s);

@@ -1,0 +1,333 @@
+// Attention of a prompt: 32 tokens x one head per workgroup, scores and sums on the fp32 matrix cores.
+//
+// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; 62 reached at 2048 tokens x 32 heads of 128).  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
+// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  2048 tokens, 32 heads of 128, rank 512: 7.1 ms -> 0.63; 1000 tokens, 16 heads of 192: 2.4 ms -> 0.21;
+// 1000 tokens of 16 differential heads over a window of 256: 535 us -> 98; 333 tokens of 16 heads with capped scores: 139 us -> 42.
+//   k_latent_expand   the keys and values of the pass's cells written out once: an fp32 latent in three bfloat16 parts times the bfloat16 matrix on the matrix cores, exact products (dense_tile.h)
+//   k_prompt_attention  a wave owns 32 queries (two operand tiles, so a key is read for both) and every fourth run of 32 cells; no barrier until the four waves' sums meet at the end.  The scores are
+//                     computed transposed (rows = cells): what a lane then holds - four cells of one query - is already the operand of the product with the values, nothing crosses lanes but the maximum.
+#include "prompt_attention.h"
+#include "dense_tile.h"
+#include "kernel_timing.h"
+
+#include <algorithm>
+
+typedef float pa_f32x4 __attribute__((ext_vector_type(4)));
+typedef int pa_i32x4 __attribute__((ext_vector_type(4)));
+
+// tiles of 128 rows of the two matrices x 64 cells; an XCD takes a contiguous run of tiles, eight blocks of rows wide and then along the cells (k_dense_tile)
+__global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restrict__ cache, int64_t width, int64_t rank, const uint16_t * __restrict__ wuk, int64_t nk, const uint16_t * __restrict__ wuv, int64_t nv, int cell0, int cell1,
+                                                          const int32_t * __restrict__ dyn, float * __restrict__ ko, float * __restrict__ vo, int cell_blocks, int tiles, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 5)) return;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES_PL(128, 64, 3)];
+    const int tile = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int row_blocks = tiles / cell_blocks, grp = tile / (8 * cell_blocks), in_grp = tile % (8 * cell_blocks), gsz = min(8, row_blocks - 8 * grp);
+    const int k_blocks = (int) ((nk + 127) / 128), block = 8 * grp + in_grp % gsz;
+    const bool is_v = block >= k_blocks;
+    const uint16_t * W = is_v ? wuv : wuk;
+    const int64_t N = is_v ? nv : nk, n0 = (int64_t) (is_v ? block - k_blocks : block) * 128;
+    if (dyn) cell1 = min(cell1, dyn[1]);
+    const int t0 = cell0 + (in_grp / gsz) * 64, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (t0 >= cell1) return;                                          // (cells of the context that hold nothing yet)
+    const int64_t nr = min(n0 + (tid >> 3), N - 1); const int tr = min(t0 + (tid >> 3), cell1 - 1);
+    dt_offs wo, xo;
+#pragma unroll
+    for (int i = 0; i < 4; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, N - 1) - nr) * rank);
+#pragma unroll
+    for (int i = 0; i < 2; i++) xo[i] = (uint32_t) ((min(tr + 32 * i, cell1 - 1) - tr) * width);
+    dt_f32x4 acc[4][2];
+    dt_tile<128, 64, 2, 2, 2, 1, false, 3>(W + nr * rank, wo, cache + (int64_t) tr * width, xo, 0, [](float a, float) { return a; }, rank, lds, acc);
+    float * out = is_v ? vo : ko;
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const int cell = t0 + (wave & 1) * 32 + b * 16 + (lane & 15);
+        if (cell >= cell1) continue;
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const int64_t n = n0 + (wave >> 1) * 64 + a * 16 + (lane >> 4) * 4;
+            if (n < N) *(dt_f32x4 *) (out + (int64_t) (cell - cell0) * N + n) = acc[a][b];      // (N % 4 == 0)
+        }
+    }
+}
+
+static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
+// weights of the cells 4 g + c of a tile of 16, and of the sums the outputs 4 NV (4 g + c) + j
+template <int NK, int NV, int MAPS>
+__global__ void __launch_bounds__(256, NK + 4 * NV > 16 ? 1 : 2) k_prompt_attention(const pa_args A, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 5)) return;
+    constexpr int NJ = 4 * NV, VW = 64 * NV, PARTS = 4 / MAPS;
+    __shared__ __attribute__((aligned(16))) float meet[4][16][VW];
+    __shared__ float meet_m[4][32], meet_l[4][32];
+    __shared__ int meet_odd[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, map = wave % MAPS, part = wave / MAPS;
+    const int h = blockIdx.x, t0 = (int) (gridDim.y - 1 - blockIdx.y) * 32;       // (the last tokens, which see the most, first)
+    const int n_kv = min(A.dyn ? A.dyn[1] : A.n_kv, A.n_kv), c_end = min(n_kv, A.cell1), words = (A.n_kv + 31) / 32;
+    const int n1 = (A.dim1 + 15) / 16;
+    const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * A.dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
+    const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
+    pa_f32x4 q[2][NK], acc[2][NJ];
+    float m_run[2] = { -INFINITY, -INFINITY }, l_run[2] = { 0.0f, 0.0f };
+    int first_pos[2], odd = 0;
+    const uint32_t * mrow[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int t = min(t0 + 16 * u + n, A.n_tok - 1), p = A.pos ? A.pos[t] : 0;
+        mrow[u] = A.mask + (int64_t) t * words;
+        first_pos[u] = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
+        const float * qr = A.q + (int64_t) t * A.qs + (int64_t) (h * MAPS + map) * (A.dim1 + A.dim2);
+#pragma unroll
+        for (int i = 0; i < NK; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int d = (i < n1 ? i : i - n1) * 16 + 4 * g + c;
+                float x = 0.0f;                                       // (values past the end: the keys there repeat others)
+                if (i < n1) { if (d < A.dim1) x = qr[d]; }
+                else if (d < A.dim2) {
+                    const pi_turn r = pi_turn_of(d, A.dim2 / 2, A.pairing);
+                    const float2 t2 = A.cs[(int64_t) min(p, A.n_pos - 1) * (A.dim2 / 2) + r.angle];
+                    const float own = qr[A.dim1 + d], other = qr[A.dim1 + r.mate];
+                    x = r.lead ? own * t2.x - other * t2.y : own * t2.x + other * t2.y;
+                }
+                q[u][i][c] = x;
+                if (i >= n1) __builtin_amdgcn_sched_barrier(0);        // (one pair at a time)
+            }
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[u][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+    const float bias = A.hbias ? A.hbias[h] : 0.0f;
+    for (int c0 = (A.cell0 & ~31) + 32 * part; c0 < c_end; c0 += 32 * PARTS) {
+        uint32_t vis[2];
+        const uint32_t in = (c_end - c0 >= 32 ? 0xffffffffu : (1u << (c_end - c0)) - 1u) & (c0 < A.cell0 ? 0xffffffffu << (A.cell0 - c0) : 0xffffffffu);
+#pragma unroll
+        for (int u = 0; u < 2; u++) vis[u] = mrow[u][c0 >> 5] & in;
+        if (A.cell_pos) {                              // a lane looks at eight cells, the four of a query put them together
+            uint32_t near[2] = { 0u, 0u };
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const int cp = A.cell_pos[min(c0 + 8 * g + b, c_end - 1)];
+#pragma unroll
+                for (int u = 0; u < 2; u++) near[u] |= (cp >= first_pos[u] || cp < A.keep_first ? 1u : 0u) << (8 * g + b);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++) { near[u] |= __shfl_xor(near[u], 16, 64); near[u] |= __shfl_xor(near[u], 32, 64); vis[u] &= near[u]; }
+        }
+        uint32_t some = vis[0] | vis[1];                              // the cells that any of the tokens sees; what the others hold is not read
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
+        some = (uint32_t) __builtin_amdgcn_readfirstlane((int) some);
+#pragma unroll 1
+        for (int half = 0; half < 2; half++) {
+            const uint32_t here = (some >> (16 * half)) & 0xffffu;
+            if (!here) continue;
+            const int cb = c0 + 16 * half, spare = __ffs(here) - 1;
+            const int ck = cb + (here >> n & 1u ? n : spare);
+            const float * kr1 = k1 + (int64_t) (ck - A.cell0) * A.k1_row, * kr2 = A.k2 + (int64_t) ck * A.k2_row;
+            pa_f32x4 kf[NK], vf[4][NV];
+#pragma unroll
+            for (int i = 0; i < NK; i++) {
+                const int d = (i < n1 ? i : i - n1) * 16 + 4 * g;
+                kf[i] = i < n1 || A.dim2 == 0 ? *(const pa_f32x4 *) (kr1 + min(d, A.dim1 - 4)) : *(const pa_f32x4 *) (kr2 + min(d, A.dim2 - 4));
+            }
+            auto values = [&]() {
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const float * vr = vb + (int64_t) (cb + (here >> (4 * g + c) & 1u ? 4 * g + c : spare) - A.cell0) * A.v_row;
+#pragma unroll
+                    for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, A.vdim - 4));
+                }
+            };
+            constexpr bool LATE = NK + 4 * NV > 16;                   // (the registers do not hold the keys and the values of a tile at a time)
+            if constexpr (!LATE) values();
+            pa_f32x4 s[2] = { pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }, pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f } };
+#pragma unroll
+            for (int i = 0; i < NK; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) { s[0] = pa_mfma(kf[i][c], q[0][i][c], s[0]); s[1] = pa_mfma(kf[i][c], q[1][i][c], s[1]); }
+            if constexpr (LATE) { __builtin_amdgcn_sched_barrier(0); values(); }
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint32_t mine = vis[u] >> (16 * half + 4 * g);
+                float top = -INFINITY;
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    float x = s[u][c] * A.scale + bias;
+                    if (soft && A.softcap > 0.0f) x = A.softcap * tanhf(x / A.softcap);
+                    s[u][c] = x;
+                    if (mine >> c & 1u) top = fmaxf(top, x);
+                }
+                if (soft) {
+                    top = fmaxf(top, __shfl_xor(top, 16, 64)); top = fmaxf(top, __shfl_xor(top, 32, 64));
+                    const float m_new = fmaxf(m_run[u], top);
+                    const float f = m_run[u] == m_new ? 1.0f : expf(m_run[u] - m_new);            // (nothing seen yet: expf(-inf) = 0, or both -inf)
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) { const float e = mine >> c & 1u ? expf(s[u][c] - m_new) : 0.0f; s[u][c] = e; sum += e; }
+                    l_run[u] = fmaf(l_run[u], f, sum); m_run[u] = m_new;                          // (a lane's own cells; the four of a query meet at the end)
+                    if (__any(f != 1.0f))
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) acc[u][j] *= f;
+                } else
+#pragma unroll
+                    for (int c = 0; c < 4; c++) s[u][c] = mine >> c & 1u ? 1.0f / (1.0f + expf(-s[u][c])) : 0.0f;
+            }
+            uint32_t big = 0;                                         // an infinity or a NaN among the values must not meet the zero weight of a token that does not see it: it joins at the end
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) big = max(big, __float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu);
+            if (__any(big >= 0x7f800000u)) {
+                odd = 1;
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[c][j >> 2][j & 3] = 0.0f;
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) { acc[0][j] = pa_mfma(vf[c][j >> 2][j & 3], s[0][c], acc[0][j]); acc[1][j] = pa_mfma(vf[c][j >> 2][j & 3], s[1][c], acc[1][j]); }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        l_run[u] += __shfl_xor(l_run[u], 16, 64); l_run[u] += __shfl_xor(l_run[u], 32, 64);
+        if (lane == 0) meet_odd[wave] = odd;
+        if (g == 0) { meet_m[wave][16 * u + n] = m_run[u]; meet_l[wave][16 * u + n] = l_run[u]; }
+    }
+    // the waves meet, 16 tokens at a time: sixteen threads per token, four outputs of every 64 each
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        if (u) __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int j = 0; j < NV; j++) *(pa_f32x4 *) &meet[wave][n][NJ * (4 * g + c) + 4 * j] = pa_f32x4{ acc[u][4 * j][c], acc[u][4 * j + 1][c], acc[u][4 * j + 2][c], acc[u][4 * j + 3][c] };
+        __syncthreads();
+        const int r = tid >> 4, t = t0 + 16 * u + r, v0 = (tid & 15) * 4;
+        pa_f32x4 o[MAPS][NV]; float M[MAPS], L[MAPS];
+        float * st = A.state ? A.state + ((int64_t) min(t, A.n_tok - 1) * A.heads + h) * (A.vdim + 2) : nullptr;
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            M[mp] = st && !A.first ? st[A.vdim] : -INFINITY; L[mp] = 0.0f;
+            const float m_before = M[mp];
+            if (soft) {
+#pragma unroll
+                for (int w = 0; w < PARTS; w++) M[mp] = fmaxf(M[mp], meet_m[w * MAPS + mp][16 * u + r]);
+            }
+#pragma unroll
+            for (int j = 0; j < NV; j++) o[mp][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+            if (st && !A.first) {
+                const float f = !soft ? 1.0f : m_before == -INFINITY ? 0.0f : expf(m_before - M[mp]);
+                L[mp] = st[A.vdim + 1] * f;
+                if (f > 0.0f)
+#pragma unroll
+                    for (int j = 0; j < NV; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) o[mp][j][e] = st[v0 + 64 * j + e] * f;
+            }
+#pragma unroll
+            for (int w = 0; w < PARTS; w++) {
+                const int ww = w * MAPS + mp;
+                const float mw = meet_m[ww][16 * u + r], f = !soft ? 1.0f : mw == -INFINITY ? 0.0f : expf(mw - M[mp]);
+                L[mp] = fmaf(meet_l[ww][16 * u + r], f, L[mp]);
+                if (!soft || mw != -INFINITY)
+#pragma unroll
+                    for (int j = 0; j < NV; j++) o[mp][j] += *(const pa_f32x4 *) &meet[ww][r][v0 + 64 * j] * f;
+            }
+        }
+        if (t >= A.n_tok) continue;
+        if (meet_odd[0] | meet_odd[1] | meet_odd[2] | meet_odd[3]) {  // the infinities and NaNs of the cells that this token sees
+            const int p = A.pos ? A.pos[t] : 0, fp = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
+            for (int cell = A.cell0; cell < c_end; cell++) {
+                if (!(A.mask[(int64_t) t * words + (cell >> 5)] >> (cell & 31) & 1u)) continue;
+                if (A.cell_pos && A.cell_pos[cell] < fp && A.cell_pos[cell] >= A.keep_first) continue;
+#pragma unroll
+                for (int j = 0; j < NV; j++) {
+                    const pa_f32x4 x = *(const pa_f32x4 *) (vb + (int64_t) (cell - A.cell0) * A.v_row + min(v0 + 64 * j, A.vdim - 4));
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if ((__float_as_uint(x[e]) & 0x7fffffffu) >= 0x7f800000u)
+#pragma unroll
+                            for (int mp = 0; mp < MAPS; mp++) o[mp][j][e] += x[e];
+                }
+            }
+        }
+        if (!A.last) {
+#pragma unroll
+            for (int j = 0; j < NV; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) st[v0 + 64 * j + e] = o[0][j][e];
+            if (v0 == 0) { st[A.vdim] = M[0]; st[A.vdim + 1] = L[0]; }
+            continue;
+        }
+        if (soft) {
+            const bool has_sink = A.sink || A.weights == PI_WEIGHTS_SOFTMAX_SINK;
+            const float sk = A.sink ? A.sink[h] : 0.0f;
+#pragma unroll
+            for (int mp = 0; mp < MAPS; mp++) {
+                const float ms = has_sink ? fmaxf(M[mp], sk) : M[mp];
+                const float f = M[mp] == -INFINITY ? 0.0f : expf(M[mp] - ms), den = fmaf(L[mp], f, has_sink ? expf(sk - ms) : 0.0f);
+                const float inv = f / den;
+#pragma unroll
+                for (int j = 0; j < NV; j++) o[mp][j] = M[mp] == -INFINITY ? pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f } : o[mp][j] * inv;
+            }
+        }
+        float mult = A.out_mult;
+        if constexpr (MAPS == 2) {                                    // the difference of the two maps, normed
+            float ss = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NV; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) { const float x = o[0][j][e] - A.lam * o[1][j][e]; o[0][j][e] = x; ss = fmaf(x, x, ss); }
+#pragma unroll
+            for (int s = 1; s < 16; s <<= 1) ss += __shfl_xor(ss, s, 64);
+            mult = A.out_mult / sqrtf(ss / (float) A.vdim + A.eps);
+        } else if (A.gate && A.gate_width == 1) {
+            float gt = A.gate[(int64_t) t * A.gs + h];
+            if (A.gate_act == PI_ACT_SIGMOID) gt = 1.0f / (1.0f + expf(-gt));
+            mult *= gt;
+        }
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int v = v0 + 64 * j + e;
+                if (v >= A.vdim) continue;
+                float x = o[0][j][e] * mult;
+                if (MAPS == 1 && A.gate && A.gate_width > 1) {
+                    float gt = A.gate[(int64_t) t * A.gs + (int64_t) h * A.vdim + v];
+                    if (A.gate_act == PI_ACT_SIGMOID) gt = 1.0f / (1.0f + expf(-gt));
+                    x *= gt;
+                }
+                A.out[(int64_t) t * A.os + (int64_t) h * A.vdim + v] = x;
+            }
+    }
+}
+
+static int pa_steps(const pa_args & a) { return (a.dim1 + 15) / 16 + (a.dim2 + 15) / 16; }
+bool pa_takes(const pa_args & a, int maps, int min_tokens) {
+    auto four = [](int64_t n) { return (n & 3) == 0; };
+    return a.n_tok >= min_tokens && pa_steps(a) <= 12 && a.vdim <= 128 && a.dim1 >= 4 && a.vdim >= 4 && four(a.dim1) && four(a.dim2) && four(a.vdim) && four(a.k1_row) && four(a.k1_head) && four(a.k2_row) && four(a.v_row) &&
+           four(a.v_head) && ((uintptr_t) a.k1 & 15) == 0 && ((uintptr_t) a.k2 & 15) == 0 && ((uintptr_t) a.v & 15) == 0 && (maps == 1 || a.dim2 == 0);
+}
+template <int NK, int NV>
+static void pa_go(const pa_args & a, int maps, double bytes, hipStream_t s) {
+    const dim3 grid((unsigned) a.heads, (unsigned) ((a.n_tok + 31) / 32));
+    const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
+    if (maps == 2) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, NV, 2>), grid, dim3(256), 0, s, a, pi_abort_word());
+    else PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, NV, 1>), grid, dim3(256), 0, s, a, pi_abort_word());
+}
+void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s) {
+    const int nk = pa_steps(a);
+#define PA_NK(NV) do { if (nk <= 4) pa_go<4, NV>(a, maps, bytes, s); else if (nk <= 6) pa_go<6, NV>(a, maps, bytes, s); else if (nk <= 8) pa_go<8, NV>(a, maps, bytes, s); else pa_go<12, NV>(a, maps, bytes, s); } while (0)
+    if (a.vdim <= 64) PA_NK(1); else PA_NK(2);
+#undef PA_NK
+}
+void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, const int32_t * dyn, float * k, float * v, hipStream_t s) {
+    const int cell_blocks = (cell1 - cell0 + 63) / 64, tiles = cell_blocks * (int) ((wuk->ne1 + 127) / 128 + (wuv->ne1 + 127) / 128);
+    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, PI_KT_MAXNT - 1, 2.0 * rank * (wuk->ne1 + wuv->ne1) + 4.0 * std::min(cell1 - cell0, n_kv) * (double) (width + wuk->ne1 + wuv->ne1), k_latent_expand, dim3((unsigned) ((tiles + 7) / 8 * 8)), dim3(256), 0, s,
+                 cache, width, (int64_t) rank, (const uint16_t *) wuk->p0, wuk->ne1, (const uint16_t *) wuv->p0, wuv->ne1, cell0, cell1, dyn, k, v, cell_blocks, tiles, pi_abort_word());
+}

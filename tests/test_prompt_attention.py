@@ -1,0 +1,78 @@
+"""Passes of many tokens (prompt_attention.hip): 32 tokens of a head at a time, keys and values of a latent written out first.  Against the explicit fp64 sums that the per-token kernels are tested with."""
+import numpy as np
+import pytest
+
+from pipeinfer_amd import lib as L
+from tests.test_letevik import HALVES, NEIGHBOURS, SIGMOID, O, diff_attention_ref, gpu, latent_case, pack_mask, rel_rms, run_diff
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,R,V,rank,T,n_kv", [(3, 8, 4, 12, 24, 9, 33), (32, 8, 4, 12, 24, 33, 33), (32, 64, 0, 64, 72, 32, 300), (8, 128, 64, 128, 512, 130, 200), (11, 20, 36, 68, 136, 95, 161), (4, 64, 0, 64, 256, 300, 2500), (64, 4, 2, 4, 8, 70, 97)])
+def test_latent_prompt(H, D, R, V, rank, T, n_kv):
+    """tiles that are not full (tokens, cells, key and output values), both pairings, every kind of gate, with and without a sink; the long one takes two launches over the cells (its scratch memory holds the
+    keys and values of 1600)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H * 100 + T)
+    pos = np.arange(n_kv - T, n_kv)
+    for pairing, width, sink in ((HALVES, V, True), (NEIGHBOURS, 1, False)) if n_kv > 1000 else ((HALVES, V, True), (NEIGHBOURS, V, False), (HALVES, 1, True), (HALVES, 0, False)):
+        got, want = latent_case(U, lib, rng, H, D, R, V, rank, n_kv, pos, 500.0, pairing, width, rng.standard_normal(H) * 2 if sink else None, (D + R) ** -0.5)
+        assert rel_rms(got, want) < 1e-5, (pairing, width, sink)
+
+
+def scattered(rng, T, n_kv, n_ctx):
+    """positions of cells in any order, tokens' positions, what the mask shows (a token sees at least itself)"""
+    cpos = rng.permutation(n_ctx).astype(np.int32)
+    pos = np.sort(rng.integers(n_kv // 3, n_kv, T)).astype(np.int32)
+    near = [int(np.argmax(np.where(cpos[:n_kv] <= p, cpos[:n_kv], -1))) for p in pos]
+    pos = cpos[near]
+    vis = (cpos[None, :n_kv] <= pos[:, None]) & (rng.random((T, n_kv)) < 0.8)
+    vis[np.arange(T), near] = True
+    return cpos, pos, vis
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 4, 4, 3, 2, 40, 32), (8, 2, 64, 128, 256, 4, 700, 97), (3, 3, 36, 68, 0, 0, 130, 65), (4, 1, 128, 64, 9, 33, 333, 200), (4, 2, 192, 128, 50, 0, 161, 40)])
+@pytest.mark.parametrize("maps", [2, 1])
+def test_window_prompt(H, G, D, V, size, keep, n_kv, T, maps):
+    """plain and differential heads over windows with kept positions, cells in any order, garbage behind the live cells"""
+    U, lib = gpu()
+    rng = np.random.default_rng(D + T)
+    kc, vc = (rng.standard_normal((n_kv + 13, G, maps, D)) * 1.5).astype(np.float32), rng.standard_normal((n_kv + 13, G, V)).astype(np.float32)
+    kc[n_kv:], vc[n_kv:] = np.nan, np.nan
+    cpos, pos, vis = scattered(rng, T, n_kv, n_kv + 13)
+    q = (rng.standard_normal((T, H, maps, D)) * 2).astype(np.float32)
+    args = (q, kc, vc, cpos, vis, pos, 0.6 * D ** -0.25, size, keep, maps, 0.45, 0.7, 1e-3, H, G)
+    want = diff_attention_ref(*(a[:n_kv] if a is kc or a is vc or a is cpos else a for a in args))
+    assert rel_rms(run_diff(U, lib, *args, True), want) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V,chunk,n_kv,T", [(2, 1, 16, 8, 32, 90, 33), (8, 2, 128, 128, 256, 600, 150), (40, 1, 8, 128, 9, 290, 32)])
+@pytest.mark.parametrize("softcap", [0.0, 3.0])
+def test_weights_of_a_prompt(H, G, D, V, chunk, n_kv, T, softcap):
+    """sigmoid weights, a soft-max and one with a sink, a bias and a gate per head, capped scores (of a soft-max); a token that sees nothing; values that are no numbers reach the tokens that see them and no others"""
+    U, lib = gpu()
+    rng = np.random.default_rng(n_kv + T)
+    kc, vc = rng.standard_normal((n_kv, G, D)).astype(np.float32), rng.standard_normal((n_kv, G, V)).astype(np.float32)
+    cpos, pos, vis = scattered(rng, T, n_kv, n_kv)
+    vis[7] = False
+    hurt = vis[:, 5] & (cpos[5] >= (pos // chunk * chunk))
+    q, gate, hb = rng.standard_normal((T, H, D)).astype(np.float32), rng.standard_normal((T, H)).astype(np.float32), rng.standard_normal(H).astype(np.float32)
+    for loud in (False, True):
+        if loud:
+            vc[5, 0, 3] = np.inf
+        for weights in (0, 1, 2):
+            d = [U.Dev(a) for a in (q, kc, vc, cpos, pack_mask(vis, n_kv), pos, hb, gate, np.array([0, n_kv, T, 0], np.int32))]
+            od = U.Dev(nbytes=4 * T * H * V)
+            L.check(lib.pi_op_chunk_attention_ex(d[0].ptr, H * D, d[1].ptr, d[2].ptr, d[3].ptr, d[4].ptr, d[5].ptr, d[6].ptr, d[7].ptr, H, SIGMOID, 0.21, -1.5, weights, softcap, chunk, H, G, D, V, T, n_kv, od.ptr, H * V, d[8].ptr, None))
+            got, want = od.get(np.float32, (T, H, V)), np.zeros((T, H, V))
+            for t in range(T):
+                js = np.nonzero(vis[t] & (cpos >= pos[t] // chunk * chunk))[0]
+                for h in range(H):
+                    s = kc[js, h // (H // G)].astype(np.float64) @ q[t, h].astype(np.float64) * np.float32(0.21) + hb[h]
+                    s = softcap * np.tanh(s / softcap) if softcap and weights else s
+                    w = O.sigmoid(s) if weights == 0 else np.exp(s) / (np.exp(s).sum() + (weights == 2)) if len(js) else s
+                    want[t, h] = vc[js, h // (H // G)].T.astype(np.float64) @ w * O.sigmoid(gate[t, h]) * -1.5
+            fine = np.isfinite(want)
+            assert np.array_equal(fine, np.isfinite(got)) and np.array_equal(got[~fine], want[~fine].astype(np.float32)) and (fine.all() or (loud and hurt.any()))
+            assert rel_rms(np.where(fine, got, 0), np.where(fine, want, 0)) < 1e-5, (weights, loud)
