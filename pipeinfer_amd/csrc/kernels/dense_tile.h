@@ -14,7 +14,8 @@ typedef __bf16 dt_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float dt_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dt_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t dt_u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t dt_offs __attribute__((ext_vector_type(4)));          // offsets of up to four rows from a first one, in elements (an array of pointers would not stay in registers)
+typedef uint32_t dt_offs __attribute__((ext_vector_type(4)));          // offsets of up to four rows from a first one, in elements (an array of pointers would not stay in registers); rows of X that are gathered from a wide range take 64 bits each
+typedef uint64_t dt_offs64 __attribute__((ext_vector_type(4)));
 
 // two fp32 values as bfloat16, nearest even (v_cvt_pk_bf16_f32)
 static __device__ __forceinline__ uint32_t dt_pack(float a, float b) { const dt_bf16x2 v = { (__bf16) a, (__bf16) b }; return __builtin_bit_cast(uint32_t, v); }
@@ -28,8 +29,8 @@ static __device__ __forceinline__ dt_f32x4 dt_mfma(dt_u32x4 a, dt_u32x4 b, dt_f3
 // PL = 3: X is not rounded but taken apart into three bfloat16 values that add up to it, three products instead of one: the products are exact, as an fp32 one of the two factors is.
 // PAIR: an X value is join(x[k], x[k + pair_off]) of two fp32 values (the two halves of a gated hidden layer).  On return lane l of wave (wn, wt) holds in acc[a][b] the rows
 // wn BN / WN + 16 a + 4 (l / 16) .. + 3 of token wt BT / WT + 16 b + l % 16.
-template <int BN, int BT, int WN, int WT, int D, int KG, bool PAIR, int PL = 1, class Join>
-static __device__ __forceinline__ void dt_tile(const uint16_t * __restrict__ w, dt_offs wo, const float * __restrict__ x, dt_offs xo, int64_t pair_off, Join join, int64_t K, uint8_t * lds,
+template <int BN, int BT, int WN, int WT, int D, int KG, bool PAIR, int PL = 1, class Offs, class Join>
+static __device__ __forceinline__ void dt_tile(const uint16_t * __restrict__ w, dt_offs wo, const float * __restrict__ x, Offs xo, int64_t pair_off, Join join, int64_t K, uint8_t * lds,
                                                dt_f32x4 (&acc)[BN / WN / 16][BT / WT / 16]) {
     static_assert(PL == 1 || KG == 1, "one group of waves where X is in three parts");
     static_assert(D % 2 == 0, "an even number of register sets: a step's buffer is known when the code is compiled");

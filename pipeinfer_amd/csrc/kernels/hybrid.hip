@@ -14,6 +14,7 @@
 #include "ops_common.h"
 #include "kernel_timing.h"
 #include "prompt_attention.h"
+#include "dense_tile.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1278,17 +1279,13 @@ extern "C" int pi_op_moe_experts_glu(const pi_weight * wup, const pi_weight * wd
 }
 
 // ---- the same for a prompt's worth of tokens: grouped by expert, on the matrix cores ---------------------------------------------------------------------
-// k_moe_group sorts the (token, choice) slots of a pass by expert (a counting sort in one workgroup) and cuts every expert's run into tiles of 64 slots; k_moe_up_mfma /
-// k_moe_down_mfma compute 64 slots x 64 rows per workgroup with v_mfma_f32_16x16x32_bf16 (operand layout as k_dense_mfma: A = 16 weight rows, B = 16 slots, 8 consecutive k per
-// lane) — an expert's matrices are read once per 64 of its tokens instead of once per token; k_moe_combine sums a token's weighted choices (identity experts: the input itself).
+// k_moe_group sorts the (token, choice) slots of a pass by expert (a counting sort in one workgroup) and cuts every expert's run into tiles of 64 or 128 slots; k_moe_tile computes the products of a tile with
+// its expert's rows on the matrix cores — an expert's matrices are read once per tile of its tokens instead of once per token; k_moe_combine sums a token's weighted choices (identity experts: the input itself).
 // idx layout (int32): [0] number of tiles | tile expert [max_tiles] | tile start [max_tiles] | tile length [max_tiles] | order [n_slots]
-typedef __bf16 hy_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float hy_f32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t hy_u16x8 __attribute__((ext_vector_type(8)));
 #define MOE_GROUP_MAX_EXPERTS 1024
 static inline int moe_max_tiles(int n_slots, int n_exp) { return (n_slots + 63) / 64 + std::min(n_exp, n_slots); }
 
-__global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ sel, int n_slots, int n_exp, int max_tiles, int32_t * __restrict__ idx, const int32_t * __restrict__ abort_w) {
+__global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ sel, int n_slots, int n_exp, int max_tiles, int tile_len, int32_t * __restrict__ idx, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w)) return;
     __shared__ int cnt[MOE_GROUP_MAX_EXPERTS], cur[MOE_GROUP_MAX_EXPERTS];
     int32_t * tile_e = idx + 1, * tile_s = tile_e + max_tiles, * tile_n = tile_s + max_tiles, * order = tile_n + max_tiles;
@@ -1300,7 +1297,7 @@ __global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ 
         int at = 0, nt = 0;
         for (int e = 0; e < n_exp; e++) {
             cur[e] = at;
-            for (int k = 0; k < cnt[e]; k += 64) { tile_e[nt] = e; tile_s[nt] = at + k; tile_n[nt] = min(64, cnt[e] - k); nt++; }
+            for (int k = 0; k < cnt[e]; k += tile_len) { tile_e[nt] = e; tile_s[nt] = at + k; tile_n[nt] = min(tile_len, cnt[e] - k); nt++; }
             at += cnt[e];
         }
         idx[0] = nt;
@@ -1309,65 +1306,46 @@ __global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ 
     for (int i = threadIdx.x; i < n_slots; i += 256) { const int e = sel[i]; if (e >= 0 && e < n_exp) order[atomicAdd(&cur[e], 1)] = i; }
 }
 
-// acc[j] += W[rows j*16 + (l % 16)][k] * B[slot (l % 16)][k] over K (K % 8 == 0); brow: this lane's B row (nullptr: zeros), wrow[j]: this lane's A rows (nullptr: zeros)
-// glu_off > 0: the B value at k is silu(brow[k]) * brow[glu_off + k] (a gated hidden layer whose two halves were stored raw)
-static __device__ __forceinline__ void hy_mfma_rows(const uint16_t * const wrow[4], const float * brow, int64_t K, int kb, hy_f32x4 acc[4], int64_t glu_off = 0, int glu = PI_GLU_SILU, float limit = 0.0f) {
-    for (int64_t k0 = 0; k0 < K; k0 += 32) {
-        const int64_t k = k0 + kb * 8;
-        const bool k_ok = k < K;
-        hy_u16x8 b = hy_u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (k_ok && brow) {
-            const float4 v0 = *(const float4 *) (brow + k), v1 = *(const float4 *) (brow + k + 4);
-            float f[8] = { v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w };
-            if (glu_off > 0) {
-                const float4 u0 = *(const float4 *) (brow + glu_off + k), u1 = *(const float4 *) (brow + glu_off + k + 4);
-                const float uf[8] = { u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w };
-#pragma unroll
-                for (int i = 0; i < 8; i++) f[i] = hy_glu(f[i], uf[i], glu, limit);
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++) { const uint32_t u = __float_as_uint(f[i]); b[i] = (uint16_t) ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16); }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            hy_u16x8 a = hy_u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (k_ok && wrow[j]) a = *(const hy_u16x8 *) (wrow[j] + k);
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(hy_bf16x8, a), __builtin_bit_cast(hy_bf16x8, b), acc[j], 0, 0, 0);
-        }
-    }
-}
-
-// UP: B rows are the tokens' inputs x[slot / top], A rows W_up[e], out up[slot][f] = relu(.)^2;  !UP: B rows up[slot] (K = ff), A rows W_down[e], out dn[slot][n].
-// glu: UP leaves the 2 * ff rows [gate | up] of an expert raw, !UP forms silu(gate) * up while it reads them (bs = 2 * ff, K = ff)
-template <bool UP>
-__global__ void __launch_bounds__(256) k_moe_mfma(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,
-                                                  int max_tiles, int glu, float limit, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
+// A tile of slots x BN rows of its expert's matrix (dense_tile.h).  UP: X rows are the tokens' inputs x[slot / top], W rows W_up[e], out up[slot][f] = relu(.)^2; !UP: X rows up[slot] (K = ff), W rows W_down[e],
+// out dn[slot][n].  glu: UP leaves the 2 * ff rows [gate | up] of an expert raw, !UP (PAIR) joins them while it stages them (bs = 2 * ff, K = ff).  What bounds it: as k_dense_tile, whose tiles these are.  Operands
+// straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048, 44 and 23 us for 24 tokens' of 1024 x 512.
+template <int BN, int BT, int KG, bool UP, bool PAIR>
+__global__ void __launch_bounds__(256 * KG, 2) k_moe_tile(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,
+                                                          int max_tiles, int glu, float limit, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 1)) return;
-    const int tile = blockIdx.y;
-    if (tile >= idx[0]) return;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES(BN, BT, KG)];
+    // workgroup n runs on XCD n % 8: an XCD takes a contiguous run of the work, eight tiles of slots (mostly one expert's) by all of its rows
+    const int row_blocks = (rows + BN - 1) / BN, total = idx[0] * row_blocks, per = (total + 7) / 8, at = (int) (blockIdx.x >> 3), work = (int) (blockIdx.x & 7) * per + at;
+    if (at >= per || work >= total) return;
+    const int grp = work / (8 * row_blocks), in_grp = work % (8 * row_blocks), gsz = min(8, idx[0] - 8 * grp), tile = 8 * grp + in_grp % gsz, n0 = in_grp / gsz * BN;
     const int32_t * tile_e = idx + 1, * tile_s = tile_e + max_tiles, * tile_n = tile_s + max_tiles, * order = tile_n + max_tiles;
     const int e = tile_e[tile], start = tile_s[tile], len = tile_n[tile];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kb = lane >> 4;
-    if (wave * 16 >= len) return;                                  // (whole waves: no barrier follows)
-    const int si = wave * 16 + li;
-    const int slot = si < len ? order[start + si] : -1;
-    const float * brow = slot < 0 ? nullptr : B + (int64_t) (UP ? slot / top : slot) * bs;
-    const int n0 = blockIdx.x * 64;
-    const uint16_t * wrow[4];
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+    const int nr = min(n0 + (tid >> 3), rows - 1);
+    dt_offs wo; dt_offs64 xo;                                          // the rows this thread stages
 #pragma unroll
-    for (int j = 0; j < 4; j++) { const int r = n0 + j * 16 + li; wrow[j] = r < rows ? W + ((int64_t) e * rows + r) * K : nullptr; }
-    hy_f32x4 acc[4];
+    for (int i = 0; i < BN / 32; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, rows - 1) - nr) * K);
 #pragma unroll
-    for (int j = 0; j < 4; j++) acc[j] = hy_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    hy_mfma_rows(wrow, brow, K, kb, acc, !UP && glu ? K : 0, glu, limit);
-    if (slot < 0) return;
+    for (int i = 0; i < BT / 32; i++) { const int slot = order[start + min((tid >> 3) + 32 * i, len - 1)]; xo[i] = (uint64_t) (UP ? slot / top : slot) * (uint64_t) bs; }
+    dt_f32x4 acc[BN / 2 / 16][BT / 2 / 16];
+    dt_tile<BN, BT, 2, 2, 2, KG, PAIR>(W + ((int64_t) e * rows + nr) * K, wo, B, xo, K, [=](float a, float b) { return hy_glu(a, b, glu, limit); }, K, lds, acc);
+    if (KG > 1 && threadIdx.x >= 256) return;
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int b = 0; b < BT / 2 / 16; b++) {
+        const int si = (wave & 1) * (BT / 2) + b * 16 + (lane & 15);
+        if (si >= len) continue;
+        float * o = out + (int64_t) order[start + si] * rows;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = n0 + j * 16 + kb * 4 + r;
-            if (row < rows) { float v = acc[j][r]; if (UP && !glu) { v = fmaxf(v, 0.0f); v *= v; } out[(int64_t) slot * rows + row] = v; }
+        for (int a = 0; a < BN / 2 / 16; a++) {
+            const int row = n0 + (wave >> 1) * (BN / 2) + a * 16 + (lane >> 4) * 4;
+            dt_f32x4 v = acc[a][b];
+            if (UP && !glu) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) { v[r] = fmaxf(v[r], 0.0f); v[r] *= v[r]; }
+            }
+            if (row < rows) *(dt_f32x4 *) (o + row) = v;               // (rows % 8 == 0)
         }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ dn, int64_t width, int n_exp, int top, const float * __restrict__ x, int64_t xs, const int32_t * __restrict__ sel,
@@ -1384,6 +1362,23 @@ __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ 
     out[(int64_t) t * os + n] = acc;
 }
 
+// slots of a tile
+static int moe_tile_len(int n_slots, int n_exp) { return n_slots / n_exp >= 256 ? 128 : 64; }
+// rows of a tile: as for k_dense_tile, the largest that gives every compute unit a workgroup; where none does, two groups of waves share K
+template <bool UP>
+static void moe_tile_launch(const uint16_t * w, int64_t K, int rows, const float * b, int64_t bs, int top, const int32_t * idx, int mt, int tl, int est, int glu, float limit, float * out, int nta, double bytes, hipStream_t s) {
+#define MOE_GO2(BN, BT, KG, PAIR) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, bytes, (k_moe_tile<BN, BT, KG, UP, PAIR>), dim3((unsigned) ((mt * ((rows + BN - 1) / BN) + 7) / 8 * 8)), dim3(256 * KG), 0, s, \
+                                               w, K, rows, b, bs, top, idx, mt, glu, limit, out, pi_abort_word())
+#define MOE_GO(BN, BT, KG) do { if constexpr (UP) MOE_GO2(BN, BT, KG, false); else if (glu) MOE_GO2(BN, BT, KG, true); else MOE_GO2(BN, BT, KG, false); } while (0)
+    const int wg128 = est * ((rows + 127) / 128);
+    if (tl == 128 && !UP && glu) MOE_GO2(64, 128, 1, !UP);            // (two values for each of X: the registers do not hold the larger tile)
+    else if (tl == 128) MOE_GO2(128, 128, 1, false);
+    else if (wg128 >= 256) MOE_GO(128, 64, 1);
+    else if (wg128 >= 128) MOE_GO(128, 64, 2);
+    else MOE_GO(64, 64, 2);
+#undef MOE_GO
+#undef MOE_GO2
+}
 // ints of index scratch the grouped path needs for a pass of n_tok tokens
 extern "C" size_t pi_op_moe_grouped_index_ints(int n_tok, int top, int n_exp) { const int ns = n_tok * top; return (size_t) 1 + 3 * (size_t) moe_max_tiles(ns, n_exp) + (size_t) ns; }
 // whether a pass of this shape takes the grouped matrix-core path (otherwise pi_op_moe_experts: gathered mat-vecs)
@@ -1415,13 +1410,13 @@ extern "C" int pi_op_moe_experts_grouped_glu(const pi_weight * wup, const pi_wei
     const int64_t width = wup->ne0;
     const int ns = n_tok * top, mt = moe_max_tiles(ns, n_exp), nta = std::min(n_tok, PI_KT_MAXNT - 1);
     const double wbytes = std::min<double>(ns, n_exp) * 2.0 * ff * width * (glu ? 1.5 : 1.0);
-    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 8.0 * ns, k_moe_group, dim3(1), dim3(256), 0, s, sel_dev, ns, n_exp, mt, idx_dev, pi_abort_word());
+    const int tl = moe_tile_len(ns, n_exp), est = (ns + tl - 1) / tl + std::min(n_exp, ns) / 2;      // (tiles, if the experts' runs end in the middle of one)
+    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 8.0 * ns, k_moe_group, dim3(1), dim3(256), 0, s, sel_dev, ns, n_exp, mt, tl, idx_dev, pi_abort_word());
     PI_CHECK_LAUNCH();
-    PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, wbytes + 4.0 * ns * (width + ff), k_moe_mfma<true>, dim3((unsigned) ((ff * upr + 63) / 64), (unsigned) mt), dim3(256), 0, s,
-                 (const uint16_t *) wup->p0, width, ff * upr, x, x_stride, top, idx_dev, mt, glu, limit, up_dev, pi_abort_word());
+    const double bytes = wbytes + 4.0 * ns * (width + ff);
+    moe_tile_launch<true>((const uint16_t *) wup->p0, width, ff * upr, x, x_stride, top, idx_dev, mt, tl, est, glu, limit, up_dev, nta, bytes, s);
     PI_CHECK_LAUNCH();
-    PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, wbytes + 4.0 * ns * (width + ff), k_moe_mfma<false>, dim3((unsigned) ((width + 63) / 64), (unsigned) mt), dim3(256), 0, s,
-                 (const uint16_t *) wdown->p0, (int64_t) ff, (int) width, up_dev, (int64_t) ff * upr, top, idx_dev, mt, glu, limit, dn_dev, pi_abort_word());
+    moe_tile_launch<false>((const uint16_t *) wdown->p0, ff, (int) width, up_dev, (int64_t) ff * upr, top, idx_dev, mt, tl, est, glu, limit, dn_dev, nta, bytes, s);
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 4.0 * n_tok * width * (top + 2), k_moe_combine, dim3((unsigned) ((width + 255) / 256), (unsigned) n_tok), dim3(256), 0, s,
                  dn_dev, width, n_exp, top, x, x_stride, sel_dev, selw_dev, out, out_stride, pi_abort_word());

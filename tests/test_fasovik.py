@@ -432,6 +432,43 @@ def test_router_and_experts(E, I, top, ff, width, exact):
     assert rel_rms(got, want) < (1e-5 if exact else 2e-3)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,I,ff,width,T,top", [(2, 1, 136, 200, 300, 2), (8, 2, 64, 3080, 200, 2), (8, 0, 72, 1544, 210, 2), (70, 3, 16, 72, 40, 6), (1, 0, 8, 8, 33, 1), (3, 0, 24, 136, 700, 2)])
+@pytest.mark.parametrize("glu", [0, 1])
+def test_grouped_experts_tiles(E, I, ff, width, T, top, glu):
+    """every tile of the grouped path (64 and 128 slots, 64 and 128 rows, K shared by two groups of waves), runs and rows that end inside a tile, choices that nobody made, identity experts; both products
+    against fp64 sums of what entered them (fp32 sums of at most 3080 terms: 3e-6 of the rows' mean)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(E + T)
+    n = 2 if glu else 1
+    x = O.bf16_round(rng.standard_normal((T, width)).astype(np.float32))
+    ups, downs = bf(rng, E, n * ff, width, s=width ** -0.5), bf(rng, E, width, ff, s=ff ** -0.5)
+    sel = np.stack([rng.permutation(E + I)[:top] for _ in range(T)]).astype(np.int32)
+    sel[sel == 1] = 0 if E > 3 else 1                                  # (an expert without tokens)
+    selw = rng.uniform(0.1, 1.0, (T, top)).astype(np.float32)
+    ud, dd, xd, sd, wd = upload_bf16(lib, ups.reshape(E * n * ff, width)), upload_bf16(lib, downs.reshape(E * width, ff)), U.Dev(x), U.Dev(sel), U.Dev(selw)
+    hd, nd, od = U.Dev(np.zeros((T * top, n * ff), np.float32)), U.Dev(nbytes=4 * T * top * width), U.Dev(nbytes=4 * T * width)
+    idx = U.Dev(nbytes=4 * lib.pi_op_moe_grouped_index_ints(T, top, E))
+    assert lib.pi_op_moe_grouped_ok(ud, dd, E, ff, glu, T, top, 0)
+    L.check(lib.pi_op_moe_experts_grouped_act(ud, dd, E, ff, glu, xd.ptr, width, sd.ptr, wd.ptr, T, top, hd.ptr, nd.ptr, idx.ptr, od.ptr, width, None))
+    hidden, got = hd.get(np.float32, (T, top, n * ff)), od.get(np.float32, (T, width))
+    want_h, want = np.zeros((T, top, n * ff)), np.zeros((T, width))
+    h64 = hidden.astype(np.float64)
+    joined = h64[..., :ff] / (1 + np.exp(-h64[..., :ff])) * h64[..., ff:] if glu else h64
+    joined = O.bf16_round(joined.astype(np.float32)).astype(np.float64)
+    for t in range(T):
+        for k in range(top):
+            e = sel[t, k]
+            if e < E:
+                h = ups[e].astype(np.float64) @ x[t].astype(np.float64)
+                want_h[t, k] = h if glu else np.maximum(h, 0) ** 2
+            want[t] += selw[t, k] * (x[t] if e >= E else downs[e].astype(np.float64) @ joined[t, k])
+    assert rel_rms(hidden, want_h) < 3e-6
+    assert rel_rms(got, want) < (2e-4 if glu else 3e-6)                # (a gate's exponential may move a hidden value over a border of bfloat16: 2^-9 of it, one in hundreds)
+    for h in (ud, dd):
+        lib.pi_weight_free(h)
+
+
 # ---- whole models through llama_decode ------------------------------------------------------------------------------------------------------
 VARIANTS = {
     "mixed": None,
