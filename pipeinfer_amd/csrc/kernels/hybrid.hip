@@ -584,7 +584,195 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
         for (int ii = 0; ii < DPT; ii++) { const int i = sp * DPT + ii; if (i < dim) S_to[(int64_t) i * vdim + j] = S[ii]; }
 }
 
+// The pieces of a long pass on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), 64 tokens long, for key widths of 32 DI <= 128.  What bounds the token loop of k_linear_attention is its chain: a token's state
+// value waits for the one before, two products per state value on the vector units.  Per head and piece, with a_t = lambda_1 .. lambda_t and D[t][j] = lambda_{j+1} .. lambda_t (products only, no quotients):
+//   states   L = sum_j (lambda_{j+1} .. lambda_64 s_j k_j) v_j^T                 (as mode 1)
+//   outputs  O = a_t (Q S_in) + (Q K^T o D s) V;  a run's last piece also leaves a_64 S_in + L   (as mode 2)
+// 2048 tokens, 32 heads of 128 x 128: 2 x 759 us -> 98 + 124, the scan between them 58 -> 34 (half the pieces, half the memory); 512 tokens, 16 heads: 2 x 93 -> 27 + 48, 11 -> 7.
+#define LM_TB 64
+#define LM_MAX_TOKENS 16384                       // (the pass's slot words in LDS beside the 54 KB of a piece)
+typedef float hy_f32x4 __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ hy_f32x4 hy_mfma(float a, float b, hy_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+// base[i] with a 32-bit offset from a uniform base (an address per load in flight would not stay in registers)
+static __device__ __forceinline__ float lm_at(const float * __restrict__ base, uint32_t i) { return *(const float *) ((const char *) base + i * 4u); }
+// the value of token j of the piece in column c: the values end at vstored, a further column is ones
+static __device__ __forceinline__ float lm_value(const float * __restrict__ vp, uint32_t j, uint32_t stride, int c, int vstored) { const float x = lm_at(vp, j * stride + (uint32_t) min(c, vstored - 1)); return c < vstored ? x : 1.0f; }
+template <int DI, bool OUTPUTS>
+__global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim, int vstored,
+                                                       const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
+                                                       float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    constexpr int DIM = 32 * DI, PITCH = DIM + 4, PP = LM_TB + 4;
+    __shared__ __attribute__((aligned(16))) float qk[LM_TB * PITCH];  // the piece's queries (OUTPUTS), then, where its state is wanted, its keys
+    __shared__ __attribute__((aligned(16))) float pt[OUTPUTS ? LM_TB * PP : 4];
+    __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
+    __shared__ float lam[LM_TB], sc[LM_TB], upto[LM_TB], from[LM_TB], pre[LM_TB], suf[LM_TB], whole[4];     // decay, factor on k v^T; products: 1 .. t, t + 1 .. 64, and the same inside a tile of 16; a tile's
+    extern __shared__ int lm_recs[];              // the slot words of the pass
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+    for (int t = tid; t < n_tok; t += 256) lm_recs[t] = rec[t];
+    __syncthreads();
+    const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
+    if (tid == 0) {
+        int first = 0, len = 0, word = -1, last = 1;
+        if (!la_find_piece(lm_recs, n_tok, bnd, n_runs, LM_TB, blockIdx.y, first, len, word, last)) len = 0;
+        seg[0] = first; seg[1] = len; seg[2] = word; seg[3] = last;
+    }
+    __syncthreads();
+    const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
+    if (len == 0 || word < 0 || (!OUTPUTS && last)) return;
+    const int hq = h / hpg;
+    const float * qp = q + (int64_t) first * stride + (int64_t) hq * DIM, * kp = k + (int64_t) first * stride + (int64_t) hq * DIM, * vp = v + (int64_t) first * stride + (int64_t) h * vstored;
+    auto stage = [&](const float * src) {                             // rows behind the last repeat it: nothing of theirs is used
+        for (int i = tid; i < LM_TB * DIM; i += 256) { const int t = i / DIM, d = i % DIM; qk[t * PITCH + d] = src[(int64_t) min(t, len - 1) * stride + d]; }
+    };
+    stage(OUTPUTS ? qp : kp);
+    if (wave == 0) {
+        const int64_t at = (int64_t) (first + min(lane, len - 1)) * tds + h;
+        const float l = lane >= len ? 1.0f : tdecay ? tdecay[at] : decay[h];
+        float a = l, b = l;                                            // products of the tile up to this token, and from it on
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) { const float x = __shfl_up(a, o, 16), y = __shfl_down(b, o, 16); if (n >= o) a *= x; if (n + o < 16) b *= y; }
+        const float after = __shfl_down(b, 1, 16);
+        float w[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) w[i] = __shfl(a, 16 * i + 15, 64);
+        float before = 1.0f, behind = 1.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) { if (i < g) before *= w[i]; if (i > g) behind *= w[i]; }
+        const float s1 = n == 15 ? 1.0f : after;
+        lam[lane] = l; sc[lane] = lane < len ? (tscale ? tscale[at] : 1.0f) : 0.0f;
+        pre[lane] = a; suf[lane] = s1; upto[lane] = before * a; from[lane] = s1 * behind;
+        if (n == 15) whole[g] = a;
+    }
+    __syncthreads();
+    const int64_t per = (int64_t) DIM * vdim;
+    float * S_scr = scratch + ((int64_t) blockIdx.y * heads + h) * per;
+    const int n_tiles = (vdim + 15) / 16;
+    if constexpr (OUTPUTS) {
+        // (Q K^T o D s) transposed: tiles (rows j, columns t) on and below the diagonal, shared out among the waves; a lane's four rows are consecutive values of row t of pt
+        for (int i = wave; i < 10; i += 4) {
+            const int tt = i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3, jt = i - tt * (tt + 1) / 2, j = 16 * jt + n;
+            const float * kr = kp + (int64_t) min(j, len - 1) * stride;
+            hy_f32x4 a = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+            for (int s = 0; s < 2 * DI; s++) {
+                const hy_f32x4 qv = *(const hy_f32x4 *) &qk[(16 * tt + n) * PITCH + 16 * s + 4 * g];
+#pragma unroll
+                for (int c = 0; c < 4; c++) a = hy_mfma(kr[16 * s + 4 * g + c], qv[c], a);
+            }
+            const int t = 16 * tt + n;
+            float between = 1.0f;
+            for (int m = jt + 1; m < tt; m++) between *= whole[m];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int jr = 16 * jt + 4 * g + r;
+                float d = 1.0f;
+                if (jt < tt) d = suf[jr] * between * pre[t];
+                else for (int m = jr + 1; m <= t; m++) d *= lam[m];
+                a[r] = jr <= t && jr < len ? a[r] * d * sc[jr] : 0.0f;
+            }
+            *(hy_f32x4 *) &pt[t * PP + 16 * jt + 4 * g] = a;
+        }
+        __syncthreads();
+        for (int nt = wave; nt < n_tiles; nt += 4) {
+            const int c = 16 * nt + n, cc = min(c, vdim - 1);
+            float sv[8 * DI];                                          // S_in: rows 16 s + 4 g + i of column c
+#pragma unroll
+            for (int s = 0; s < 2 * DI; s++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) sv[4 * s + i] = lm_at(S_scr, (uint32_t) (16 * s + 4 * g + i) * (uint32_t) vdim + (uint32_t) cc);
+            float vv[16];                                              // values: rows 16 jt + 4 g + r
+#pragma unroll
+            for (int i = 0; i < 16; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored); }
+            hy_f32x4 acc[4];
+#pragma unroll
+            for (int m = 0; m < 4; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+            for (int s = 0; s < 2 * DI; s++) {
+                __builtin_amdgcn_sched_barrier(0);
+                hy_f32x4 qv[4];
+#pragma unroll
+                for (int m = 0; m < 4; m++) qv[m] = *(const hy_f32x4 *) &qk[(16 * m + n) * PITCH + 16 * s + 4 * g];
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int m = 0; m < 4; m++) acc[m] = hy_mfma(qv[m][i], sv[4 * s + i], acc[m]);
+            }
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[m][r] *= upto[16 * m + 4 * g + r];
+#pragma unroll
+            for (int jt = 0; jt < 4; jt++) {
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t big = 0;                                      // (an infinity or a NaN among the values must not meet the zero weights of the tokens before it)
+#pragma unroll
+                for (int r = 0; r < 4; r++) big = max(big, __float_as_uint(vv[4 * jt + r]) & 0x7fffffffu);
+                const bool odd = __any(big >= 0x7f800000u);
+#pragma unroll
+                for (int m = jt; m < 4; m++) {
+                    if (m == jt && odd) {
+                        for (int j = 16 * jt; j < min(16 * jt + 16, len); j++) {
+                            const float x = lm_value(vp, j, (uint32_t) stride, cc, vstored);
+#pragma unroll
+                            for (int r = 0; r < 4; r++) if (j <= 16 * m + 4 * g + r) acc[m][r] = fmaf(pt[(16 * m + 4 * g + r) * PP + j], x, acc[m][r]);
+                        }
+                        continue;
+                    }
+                    const hy_f32x4 pv = *(const hy_f32x4 *) &pt[(16 * m + n) * PP + 16 * jt + 4 * g];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[m] = hy_mfma(pv[r], vv[4 * jt + r], acc[m]);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int t = 16 * m + 4 * g + r;
+                    if (t >= len || c >= vdim) continue;
+                    __builtin_amdgcn_sched_barrier(0);
+                    float o = acc[m][r];
+                    if (skip) o = fmaf(skip[h], lm_value(vp, t, (uint32_t) stride, c, vstored), o);
+                    out[(int64_t) (first + t) * os + (int64_t) h * vdim + c] = o;
+                }
+        }
+        if (!last) return;
+        __syncthreads();
+        stage(kp);
+        __syncthreads();
+    }
+    // the state of the piece: from zero (scratch), or from S_in (the slot)
+    float * S_to = OUTPUTS ? state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per : S_scr;
+    const float all = upto[LM_TB - 1];
+    for (int nt = wave; nt < n_tiles; nt += 4) {
+        const int c = 16 * nt + n, cc = min(c, vdim - 1);
+        float vv[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = j < len ? lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored) * (from[j] * sc[j]) : 0.0f; }
+        hy_f32x4 acc[2 * DI];
+#pragma unroll
+        for (int m = 0; m < 2 * DI; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            __builtin_amdgcn_sched_barrier(0);
+            const float * kr = &qk[(16 * (i >> 2) + 4 * g + (i & 3)) * PITCH + n];
+#pragma unroll
+            for (int m = 0; m < 2 * DI; m++) acc[m] = hy_mfma(kr[16 * m], vv[i], acc[m]);
+        }
+        if (c < vdim)
+#pragma unroll
+            for (int m = 0; m < 2 * DI; m++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t at = ((uint32_t) (16 * m + 4 * g + r) * (uint32_t) vdim + (uint32_t) c) * 4u;
+                    if (OUTPUTS && r == 0) __builtin_amdgcn_sched_barrier(0);
+                    *(float *) ((char *) S_to + at) = OUTPUTS ? fmaf(all, *(const float *) ((const char *) S_scr + at), acc[m][r]) : acc[m][r];
+                }
+    }
+}
+
 // grid (head, blocks over dim * vdim, run): scratch[piece] holds L_p coming in and S_in(p) going out
+template <int TB>
 __global__ void __launch_bounds__(256) k_linear_state_scan(int heads, int dim, int vdim, const float * __restrict__ decay, const float * __restrict__ tdecay, int64_t tds, const float * __restrict__ state,
                                                            const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w)) return;
@@ -597,7 +785,7 @@ __global__ void __launch_bounds__(256) k_linear_state_scan(int heads, int dim, i
         int ord = 0, nsub = 0, word = -1, sub0 = 0, tfirst = 0;
         for (int r = 0; r < n_runs; r++) {
             const int t = bnd[r], e = r + 1 < n_runs ? bnd[r + 1] : n_tok;
-            const int ns = (e - t + LA_TB - 1) / LA_TB;
+            const int ns = (e - t + TB - 1) / TB;
             if (r == (int) blockIdx.z) { nsub = ns; word = recs[t]; sub0 = ord; tfirst = t; break; }
             ord += ns;
         }
@@ -609,20 +797,23 @@ __global__ void __launch_bounds__(256) k_linear_state_scan(int heads, int dim, i
     const int h = blockIdx.x, slot = word & ~LA_FRESH;
     const int64_t per = (int64_t) dim * vdim, idx = (int64_t) blockIdx.y * 256 + threadIdx.x;
     const bool in = idx < per;
-    __shared__ float lps[8];                                           // per-token decays: their products over eight pieces, a thread per token (LA_TB = 32 lanes meet per piece)
-    float lp = 1.0f;                                                   // lambda^LA_TB: every piece but a run's last has LA_TB tokens
-    if (!tdecay) for (int i = 0; i < LA_TB; i++) lp *= decay[h];
+    constexpr int ND = 256 / TB;                                       // pieces whose per-token decays are multiplied out in a round, a thread per token (the TB <= 64 lanes of a piece meet)
+    __shared__ float lps[8];
+    float lp = 1.0f;                                                   // lambda^TB: every piece but a run's last has TB tokens
+    if (!tdecay) for (int i = 0; i < TB; i++) lp *= decay[h];
     float run = !in || (word & LA_FRESH) ? 0.0f : state[((int64_t) slot * heads + h) * per + idx];
     for (int p0 = 0; p0 < nsub; p0 += 8) {                             // eight pieces at a time: their loads are in flight together, then the chain runs on registers
         float lpart[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) lpart[i] = in && p0 + i < nsub - 1 ? scratch[((int64_t) (sub0 + p0 + i) * heads + h) * per + idx] : 0.0f;
         if (tdecay) {
-            const int pi = threadIdx.x / LA_TB;                        // (256 threads: eight pieces; only whole pieces are multiplied out)
-            float d = p0 + pi < nsub - 1 ? tdecay[(int64_t) (tfirst + (p0 + pi) * LA_TB + threadIdx.x % LA_TB) * tds + h] : 1.0f;
-            for (int o = LA_TB >> 1; o > 0; o >>= 1) d *= __shfl_xor(d, o, PI_WAVE);
             __syncthreads();                                           // (the previous eight are no longer read)
-            if (threadIdx.x % LA_TB == 0) lps[pi] = d;
+            for (int pb = 0; pb < 8; pb += ND) {
+                const int pi = pb + threadIdx.x / TB;
+                float d = p0 + pi < nsub - 1 ? tdecay[(int64_t) (tfirst + (p0 + pi) * TB + threadIdx.x % TB) * tds + h] : 1.0f;        // (only whole pieces are multiplied out)
+                for (int o = TB >> 1; o > 0; o >>= 1) d *= __shfl_xor(d, o, PI_WAVE);
+                if (threadIdx.x % TB == 0) lps[pi] = d;
+            }
             __syncthreads();
         }
 #pragma unroll
@@ -642,6 +833,12 @@ extern "C" int pi_op_linear_attention_reserve(void) {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<8>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<16>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<32>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
+#define LM_RES(DI) PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_pieces<DI, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS)); \
+                   PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_pieces<DI, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS));
+    LM_RES(1) LM_RES(2) LM_RES(3) LM_RES(4)
+#undef LM_RES
+    PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_state_scan<LA_TB>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
+    PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_state_scan<LM_TB>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS));
     done = true;
     return 0;
 }
@@ -693,9 +890,26 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
 #define LA_GO(D, MODE) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_attention<D>, grid, dim3(threads), lds, s, q, k, v, stride, heads, hpg, dim, vdim, value_cols, R, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, state_dev, rec_dev, n_tok, MODE, scratch_dev, out, out_stride, pi_abort_word())
 #define LA_ANY(MODE) do { if (dpt == 8) LA_GO(8, MODE); else if (dpt == 16) LA_GO(16, MODE); else LA_GO(32, MODE); } while (0)
     if (!pieces) { LA_ANY(0); PI_CHECK_LAUNCH(); return 0; }
+    const unsigned gr = (unsigned) std::max(1, std::min(n_tok, max_segments)), gb = (unsigned) (((int64_t) dim * vdim + 255) / 256);
+    if (dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22)) {        // (32-bit offsets within a piece; pieces twice as long take half of the scratch that was asked for)
+        if (n_tok > 2048 && pi_op_linear_attention_reserve() != 0) return -1;
+        const dim3 pg((unsigned) heads, (unsigned) (n_tok / LM_TB + std::min(n_tok, std::max(1, max_segments)) + 1));
+#define LM_GO(DI, OUT) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_linear_pieces<DI, OUT>), pg, dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, \
+                                    state_dev, rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word())
+#define LM_ANY(OUT) do { if (dim == 32) LM_GO(1, OUT); else if (dim == 64) LM_GO(2, OUT); else if (dim == 96) LM_GO(3, OUT); else LM_GO(4, OUT); } while (0)
+        LM_ANY(false);
+        PI_CHECK_LAUNCH();
+        PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * pg.y * heads * dim * vdim, k_linear_state_scan<LM_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,
+                     heads, dim, vdim, decay_dev, tdecay_dev, t_stride, state_dev, rec_dev, n_tok, scratch_dev, pi_abort_word());
+        PI_CHECK_LAUNCH();
+        LM_ANY(true);
+#undef LM_ANY
+#undef LM_GO
+        PI_CHECK_LAUNCH(); return 0;
+    }
     LA_ANY(1);
     PI_CHECK_LAUNCH();
-    PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * gz * heads * dim * vdim, k_linear_state_scan, dim3((unsigned) heads, (unsigned) (((int64_t) dim * vdim + 255) / 256), (unsigned) std::max(1, std::min(n_tok, max_segments))), dim3(256), (size_t) 4 * n_tok, s,
+    PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * gz * heads * dim * vdim, k_linear_state_scan<LA_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,
                  heads, dim, vdim, decay_dev, tdecay_dev, t_stride, state_dev, rec_dev, n_tok, scratch_dev, pi_abort_word());
     PI_CHECK_LAUNCH();
     LA_ANY(2);
@@ -1308,7 +1522,8 @@ __global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ 
 
 // A tile of slots x BN rows of its expert's matrix (dense_tile.h).  UP: X rows are the tokens' inputs x[slot / top], W rows W_up[e], out up[slot][f] = relu(.)^2; !UP: X rows up[slot] (K = ff), W rows W_down[e],
 // out dn[slot][n].  glu: UP leaves the 2 * ff rows [gate | up] of an expert raw, !UP (PAIR) joins them while it stages them (bs = 2 * ff, K = ff).  What bounds it: as k_dense_tile, whose tiles these are.  Operands
-// straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048, 44 and 23 us for 24 tokens' of 1024 x 512.
+// straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048 (now 116 and 125: 475 and 440 TFLOP/s), 44 and 23 us for 24 tokens' of 1024 x 512
+// (10 and 7).
 template <int BN, int BT, int KG, bool UP, bool PAIR>
 __global__ void __launch_bounds__(256 * KG, 2) k_moe_tile(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,
                                                           int max_tiles, int glu, float limit, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
