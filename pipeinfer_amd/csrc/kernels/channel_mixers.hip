@@ -444,6 +444,333 @@ __global__ void __launch_bounds__(256) k_channel_state_scan_diag(int heads, int 
     }
 }
 
+// ---- long passes on the fp32 matrix cores -----------------------------------------------------------------------------------------------------------------------
+// What bounds the walks above: a token's chain (two dependent sums over the key, then the state) at one column per R lanes, and for the delta rule a dim x dim transition matrix per piece, built by as many extra
+// columns and chained by a scan of its own.  Written for a piece of 32 tokens at a time, with G_t the decays' product from the piece's start (v_mfma_f32_16x16x4_f32 throughout):
+//   (I + A) U = beta (V - W S_in),  W_t = G_t k_t,  A[t][j] = beta_t sum_i k_t k_j (g_{j+1} .. g_t)_i for j < t      (bonus rule: U = V)
+//   O = Q' S_in + P U,  Q'_t = G_t q_t,  P[t][j] = sum_i q_t k_j (g_{j+1} .. g_t)_i for j <= t                     (bonus rule: products up to t - 1, the bonus on the diagonal)
+//   S_out = G_32 S_in + K' U,  K'_j = k_j (g_{j+1} .. g_32)
+//   k_channel_pieces  per (head, piece), side by side: everything that does not know S_in, T = (I + A)^-1 applied to beta V and beta W.  Decays are products of factors only, never quotients: inside a tile of 16
+//                     tokens they are multiplied up pair by pair, across the two tiles they meet at the border between them (a decay of 1e-30 per token is as good as any other).  Unit keys and beta <= 1
+//                     bound T's entries by 1; keys as they come (qk_unit = 0) of the delta rule stay with the walks
+//   k_channel_walk    per (head, 16 value columns, run): one wave takes the run's pieces in order, the state in registers all the way - a product's result is laid out as the next one's operand.
+//                     An infinity or a NaN in a piece would meet zeros of tokens before it: such a piece is walked token by token
+// 333 tokens of one sequence, delta rule, 16 heads of 128 x 128: 2 x 271 us + scan 331 -> 42 + 48; bonus rule, 32 heads of 64 x 64: 2 x 129 + scan 22 -> 21 + 27.
+#define CP_TB 32
+typedef float cm_f32x4 __attribute__((ext_vector_type(4)));
+static __device__ __forceinline__ cm_f32x4 cm_mfma(float a, float b, cm_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+static __device__ __forceinline__ cm_f32x4 cm_mfma4(cm_f32x4 a, cm_f32x4 b, cm_f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) c = cm_mfma(a[i], b[i], c);
+    return c;
+}
+// a piece's block in scratch, in floats: operands as the lanes hold them, [tile][lane][4]:  Q' [2][dim / 16], K' [dim / 16][2], -T beta W [2][dim / 16], P [3], G_32 [dim], a flag, T beta V [2][vdim / 16]
+// (flagged: q, k, g as rows [32][dim] in the first three places, beta [32] and the scalar of the token's own write [32] in P's)
+struct cp_layout { int q, k, w, p, g, flag, u, total; };
+static __host__ __device__ __forceinline__ cp_layout cp_of(int dim, int vdim) {
+    cp_layout l;
+    l.q = 0; l.k = CP_TB * dim; l.w = 2 * CP_TB * dim; l.p = 3 * CP_TB * dim; l.g = l.p + 768; l.flag = l.g + dim; l.u = l.flag + 4; l.total = l.u + CP_TB * vdim;
+    return l;
+}
+template <int DI, int RULE>
+__global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs, const float * __restrict__ draw, int64_t ds,
+                                                        int decay_mode, const float * __restrict__ dbias, const float * __restrict__ a_log, const float * __restrict__ braw, int64_t bs, const float * __restrict__ bonus,
+                                                        int qk_unit, float q_mult, int heads, int hpg, int vdim, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    constexpr int DIM = 16 * DI, PITCH = DIM + 4, SL = 2 * DI;        // SL: the eighth of the channels that a thread of the diagonal tiles takes
+    __shared__ __attribute__((aligned(16))) float qt[CP_TB * PITCH], kt[CP_TB * PITCH], gt[CP_TB * PITCH], Am[CP_TB][36], Pm[CP_TB][36], Tm[CP_TB][36], whole[2][DIM];
+    __shared__ float beta[CP_TB], dot[CP_TB];
+    __shared__ int seg[3], bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+    const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd);
+    if (tid == 0) {
+        int ord = 0;
+        seg[1] = 0;
+        for (int r = 0; r < n_runs; r++) {
+            const int t = sorted[r], e = r + 1 < n_runs ? sorted[r + 1] : n_tok, nsub = (e - t + CP_TB - 1) / CP_TB, pc = (int) blockIdx.y - ord;
+            if (pc < nsub) { seg[0] = t + pc * CP_TB; seg[1] = min(CP_TB, e - seg[0]); seg[2] = rec[t]; break; }
+            ord += nsub;
+        }
+    }
+    __syncthreads();
+    const int first = seg[0], len = seg[1];
+    if (len == 0 || seg[2] < 0) return;
+    const cp_layout L = cp_of(DIM, vdim);
+    float * blk = scratch + ((int64_t) blockIdx.y * heads + h) * L.total;
+    const float ah = decay_mode == 2 ? expf(a_log[h]) : 0.0f;
+    uint32_t big = 0;
+    for (int idx = tid; idx < CP_TB * DIM; idx += 256) {
+        const int t = idx / DIM, i = idx % DIM;
+        const int64_t tok = first + min(t, len - 1);
+        float qv = q[tok * qs + (int64_t) (h / hpg) * DIM + i], kv = k[tok * ks + (int64_t) (h / hpg) * DIM + i], d = draw[tok * ds + (int64_t) h * DIM + i];
+        if (decay_mode == 1) d = expf(-expf(d + (dbias ? dbias[h * DIM + i] : 0.0f)));
+        else if (decay_mode == 2) d = expf(-ah * cm_softplus(d + (dbias ? dbias[h * DIM + i] : 0.0f)));
+        if (t >= len) { qv = 0.0f; kv = 0.0f; d = 1.0f; }
+        qt[t * PITCH + i] = qv; kt[t * PITCH + i] = kv; gt[t * PITCH + i] = d;
+        big = max(big, max(__float_as_uint(d) & 0x7fffffffu, max(__float_as_uint(qv) & 0x7fffffffu, __float_as_uint(kv) & 0x7fffffffu)));
+    }
+    if (tid < CP_TB) {
+        const float b = tid >= len ? 0.0f : braw ? cm_sigmoid(braw[(int64_t) (first + tid) * bs + h]) : 1.0f;
+        beta[tid] = b; big = max(big, __float_as_uint(b) & 0x7fffffffu);
+    }
+    for (int idx = tid; idx < len * vdim; idx += 256) big = max(big, __float_as_uint(v[(int64_t) (first + idx / vdim) * vs + (int64_t) h * vdim + idx % vdim]) & 0x7fffffffu);
+    for (int idx = tid; idx < CP_TB * 36; idx += 256) { (&Am[0][0])[idx] = 0.0f; (&Pm[0][0])[idx] = 0.0f; (&Tm[0][0])[idx] = 0.0f; }
+    const bool odd = __syncthreads_or(big >= 0x7f800000u);
+    for (int t = wave; t < CP_TB; t += 4) {                           // unit vectors, and the scalar of the token's own write
+        float * qr = qt + t * PITCH, * kr = kt + t * PITCH;
+        if (qk_unit) {
+            float sq = 0.0f, sk = 0.0f;
+            for (int i = lane; i < DIM; i += 64) { sq = fmaf(qr[i], qr[i], sq); sk = fmaf(kr[i], kr[i], sk); }
+            const float iq = q_mult / sqrtf(pi_lanes_sum<64>(sq) + 1e-6f), ik = 1.0f / sqrtf(pi_lanes_sum<64>(sk) + 1e-6f);
+            for (int i = lane; i < DIM; i += 64) { qr[i] *= iq; kr[i] *= ik; }
+        } else if (q_mult != 1.0f) for (int i = lane; i < DIM; i += 64) qr[i] *= q_mult;
+        float d = 0.0f;
+        for (int i = lane; i < DIM; i += 64) d = fmaf(RULE == 1 && bonus ? qr[i] * bonus[h * DIM + i] : qr[i], kr[i], d);
+        d = pi_lanes_sum<64>(d);
+        if (lane == 0) dot[t] = d;
+    }
+    __syncthreads();
+    if (tid == 0) *(int *) (blk + L.flag) = odd ? 1 : 0;
+    if (odd) {
+        for (int idx = tid; idx < CP_TB * DIM; idx += 256) { const int at = idx / DIM * PITCH + idx % DIM; blk[L.q + idx] = qt[at]; blk[L.k + idx] = kt[at]; blk[L.w + idx] = gt[at]; }
+        if (tid < CP_TB) { blk[L.p + tid] = beta[tid]; blk[L.p + CP_TB + tid] = dot[tid]; }
+        return;
+    }
+    {   // the tiles on the diagonal: eight threads share a column j, walk down from it and keep k_j decayed to where they are
+        const int sl = tid & 7, j = tid >> 3 & 15, t0 = tid >> 7 << 4;
+        cm_f32x4 r[SL / 4];
+#pragma unroll
+        for (int i = 0; i < SL / 4; i++) r[i] = *(const cm_f32x4 *) &kt[(t0 + j) * PITCH + SL * sl + 4 * i];
+        for (int t = j; t < 16; t++) {
+            const int at = (t0 + t) * PITCH + SL * sl;
+            float a = 0.0f, p = 0.0f;
+#pragma unroll
+            for (int i = 0; i < SL / 4; i++) {
+                const cm_f32x4 qv = *(const cm_f32x4 *) &qt[at + 4 * i], kv = *(const cm_f32x4 *) &kt[at + 4 * i], gv = *(const cm_f32x4 *) &gt[at + 4 * i];
+                if (RULE == 0 && t > j) r[i] *= gv;
+#pragma unroll
+                for (int e = 0; e < 4; e++) { if (RULE == 0) a = fmaf(r[i][e], kv[e], a); p = fmaf(r[i][e], qv[e], p); }
+                if (RULE == 1 && t > j) r[i] *= gv;
+            }
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) { if (RULE == 0) a += __shfl_xor(a, o, 64); p += __shfl_xor(p, o, 64); }
+            if (sl == 0) { if (t > j) Am[t0 + t][t0 + j] = a; Pm[t0 + t][t0 + j] = t > j ? p : dot[t0 + j]; }
+        }
+    }
+    __syncthreads();
+    if (tid < 2 * DIM) {                                               // a thread per channel and tile: gt <- k to the tile's start, qt <- q to it (both decayed), kt <- k to the tile's end
+        const int i = tid % DIM, t0 = tid / DIM << 4;
+        float gv[16], w = 1.0f;
+#pragma unroll
+        for (int t = 0; t < 16; t++) gv[t] = gt[(t0 + t) * PITCH + i];
+#pragma unroll
+        for (int t = 0; t < 16; t++) {
+            const int at = (t0 + t) * PITCH + i;
+            if (RULE == 1) qt[at] *= w;
+            w *= gv[t];
+            if (RULE == 0) { qt[at] *= w; gt[at] = kt[at] * w; }
+        }
+        whole[t0 >> 4][i] = w;
+        w = 1.0f;
+#pragma unroll
+        for (int t = 15; t >= 0; t--) { kt[(t0 + t) * PITCH + i] *= w; w *= gv[t]; }
+    }
+    __syncthreads();
+    if (wave < 2 && (RULE == 0 || wave == 1)) {                       // the tile below them
+        const float * rows = wave == 0 ? gt : qt;
+        cm_f32x4 a = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int s = 0; s < DI; s++) a = cm_mfma4(*(const cm_f32x4 *) &rows[(16 + n) * PITCH + 16 * s + 4 * g], *(const cm_f32x4 *) &kt[n * PITCH + 16 * s + 4 * g], a);
+#pragma unroll
+        for (int r = 0; r < 4; r++) (wave == 0 ? Am : Pm)[16 + 4 * g + r][n] = a[r];
+    }
+    __syncthreads();
+    if constexpr (RULE == 0) {
+        for (int idx = tid; idx < CP_TB * CP_TB; idx += 256) Am[idx >> 5][idx & 31] *= beta[idx >> 5];
+        __syncthreads();
+        if (tid < 32) {                                                // T on the diagonal: a thread per column, forward substitution
+            const int t0 = tid & 16, c = tid & 15;
+            float x[16];
+#pragma unroll
+            for (int t = 0; t < 16; t++) {
+                float y = t == c ? 1.0f : 0.0f;
+#pragma unroll
+                for (int j = 0; j < t; j++) y = fmaf(-Am[t0 + t][t0 + j], x[j], y);
+                x[t] = y;
+                Tm[t0 + t][t0 + c] = y;
+            }
+        }
+        __syncthreads();
+        const int t = tid >> 4, c = tid & 15;                          // below it: -T_11 (A_10 T_00)
+        float m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 16; j++) m = fmaf(Am[16 + t][j], Tm[j][c], m);
+        Am[t][16 + c] = m;
+        __syncthreads();
+        m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 16; j++) m = fmaf(Tm[16 + t][16 + j], Am[j][16 + c], m);
+        Tm[16 + t][c] = -m;
+        __syncthreads();
+        for (int s = wave; s < DI; s += 4) {                           // -(T beta W), transposed: a lane's four rows are four channels of one token
+            const int i = 16 * s + n;
+            const float w0 = whole[0][i];
+            cm_f32x4 a[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
+#pragma unroll
+            for (int jt = 0; jt < 2; jt++) {
+                cm_f32x4 w;
+#pragma unroll
+                for (int r = 0; r < 4; r++) { const int j = 16 * jt + 4 * g + r; w[r] = -beta[j] * gt[j * PITCH + i] * (jt ? w0 : 1.0f); }
+#pragma unroll
+                for (int mt = jt; mt < 2; mt++) a[mt] = cm_mfma4(w, *(const cm_f32x4 *) &Tm[16 * mt + n][16 * jt + 4 * g], a[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) *(cm_f32x4 *) (blk + L.w + ((mt * DI + s) * 64 + lane) * 4) = a[mt];
+        }
+        const int nvt = vdim / 16;
+        for (int vt = wave; vt < nvt; vt += 4) {
+            cm_f32x4 a[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
+#pragma unroll
+            for (int jt = 0; jt < 2; jt++) {
+                cm_f32x4 x;
+#pragma unroll
+                for (int r = 0; r < 4; r++) { const int j = 16 * jt + 4 * g + r; x[r] = beta[j] * v[(int64_t) (first + min(j, len - 1)) * vs + (int64_t) h * vdim + 16 * vt + n]; }       // (beta = 0 behind the end)
+#pragma unroll
+                for (int mt = jt; mt < 2; mt++) a[mt] = cm_mfma4(*(const cm_f32x4 *) &Tm[16 * mt + n][16 * jt + 4 * g], x, a[mt]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) *(cm_f32x4 *) (blk + L.u + ((mt * nvt + vt) * 64 + lane) * 4) = a[mt];
+        }
+    }
+    for (int idx = tid; idx < 2 * DI * 64; idx += 256) {
+        const int tile = idx >> 6, ln = idx & 15, lg = idx >> 4 & 3;
+        const int t = 16 * (tile / DI) + ln, i = 16 * (tile % DI) + 4 * lg;
+        cm_f32x4 x = *(const cm_f32x4 *) &qt[t * PITCH + i];
+        if (tile / DI) x *= *(const cm_f32x4 *) &whole[0][i];
+        *(cm_f32x4 *) (blk + L.q + idx * 4) = x;
+        const int c = 16 * (tile >> 1) + ln, j = 16 * (tile & 1) + 4 * lg;
+        cm_f32x4 y;
+#pragma unroll
+        for (int r = 0; r < 4; r++) y[r] = kt[(j + r) * PITCH + c] * (tile & 1 ? 1.0f : whole[1][c]);
+        *(cm_f32x4 *) (blk + L.k + idx * 4) = y;
+    }
+    if (wave < 3) *(cm_f32x4 *) (blk + L.p + tid * 4) = *(const cm_f32x4 *) &Pm[(wave ? 16 : 0) + n][(wave == 2 ? 16 : 0) + 4 * g];
+    for (int i = tid; i < DIM; i += 256) blk[L.g + i] = whole[0][i] * whole[1][i];
+}
+
+template <int DI, int RULE>
+__global__ void __launch_bounds__(64, 1) k_channel_walk(const float * __restrict__ v, int64_t vs, int heads, int vdim, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, const float * __restrict__ scratch,
+                                                        float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    constexpr int DIM = 16 * DI;
+    __shared__ int bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;
+    const int h = blockIdx.x, vt = blockIdx.y, lane = threadIdx.x, n = lane & 15, g = lane >> 4, c = 16 * vt + n;
+    const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd);
+    if ((int) blockIdx.z >= n_runs) return;
+    int ord = 0;
+    for (int r = 0; r < (int) blockIdx.z; r++) ord += ((r + 1 < n_runs ? sorted[r + 1] : n_tok) - sorted[r] + CP_TB - 1) / CP_TB;
+    const int start = sorted[blockIdx.z], end = (int) blockIdx.z + 1 < n_runs ? sorted[blockIdx.z + 1] : n_tok, word = rec[start], np = (end - start + CP_TB - 1) / CP_TB;
+    if (word < 0) return;
+    const cp_layout L = cp_of(DIM, vdim);
+    const int nvt = vdim / 16;
+    const float * blk = scratch + ((int64_t) ord * heads + h) * L.total;
+    const int64_t step = (int64_t) heads * L.total;
+    float * S_hbm = state + ((int64_t) (word & ~CM_FRESH) * heads + h) * DIM * vdim + c;
+    cm_f32x4 S[DI];                                                   // rows 16 m + 4 g + r of column c: as a product leaves them, and as the next one takes them
+#pragma unroll
+    for (int m = 0; m < DI; m++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) S[m][r] = word & CM_FRESH ? 0.0f : S_hbm[(int64_t) (16 * m + 4 * g + r) * vdim];
+    cm_f32x4 W[RULE == 0 ? 2 * DI : 1], U[2];
+    int flag;
+    auto ahead = [&](const float * b, int at) {                       // what the piece's first product reads
+        flag = *(const int *) (b + L.flag);
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            if constexpr (RULE == 0) U[m] = *(const cm_f32x4 *) (b + L.u + ((m * nvt + vt) * 64 + lane) * 4);
+            else
+#pragma unroll
+                for (int r = 0; r < 4; r++) U[m][r] = v[(int64_t) min(at + 16 * m + 4 * g + r, end - 1) * vs + (int64_t) h * vdim + c];      // (behind the end: met by keys of zero)
+        }
+        if constexpr (RULE == 0)
+#pragma unroll
+            for (int i = 0; i < 2 * DI; i++) W[i] = *(const cm_f32x4 *) (b + L.w + (i * 64 + lane) * 4);
+    };
+    ahead(blk, start);
+    for (int p = 0; p < np; p++, blk += step) {
+        const int at = start + p * CP_TB, len = min(CP_TB, end - at);
+        if (flag) {
+            for (int t = 0; t < len; t++) {
+                cm_f32x4 kv[DI];
+                float a = 0.0f, o = 0.0f;
+#pragma unroll
+                for (int m = 0; m < DI; m++) {
+                    kv[m] = *(const cm_f32x4 *) (blk + L.k + t * DIM + 16 * m + 4 * g);
+                    const cm_f32x4 qv = *(const cm_f32x4 *) (blk + L.q + t * DIM + 16 * m + 4 * g), gv = *(const cm_f32x4 *) (blk + L.w + t * DIM + 16 * m + 4 * g);
+                    if (RULE == 0) S[m] *= gv;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) { a = fmaf(S[m][r], kv[m][r], a); o = fmaf(S[m][r], qv[r], o); }
+                    if (RULE == 1) S[m] *= gv;
+                }
+                a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64); o += __shfl_xor(o, 16, 64); o += __shfl_xor(o, 32, 64);
+                const float x = v[(int64_t) (at + t) * vs + (int64_t) h * vdim + c], u = RULE == 0 ? blk[L.p + t] * (x - a) : x;
+#pragma unroll
+                for (int m = 0; m < DI; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) S[m][r] = fmaf(kv[m][r], u, S[m][r]);
+                if (g == 0) out[(int64_t) (at + t) * os + (int64_t) h * vdim + c] = fmaf(u, blk[L.p + CP_TB + t], o);
+            }
+            const float * nb = p + 1 < np ? blk + step : blk;
+            ahead(nb, p + 1 < np ? at + CP_TB : at);
+            continue;
+        }
+        cm_f32x4 Q[2 * DI], K[2 * DI], P[3], G[DI], O[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
+#pragma unroll
+        for (int i = 0; i < 2 * DI; i++) Q[i] = *(const cm_f32x4 *) (blk + L.q + (i * 64 + lane) * 4);
+#pragma unroll
+        for (int i = 0; i < 3; i++) P[i] = *(const cm_f32x4 *) (blk + L.p + (i * 64 + lane) * 4);
+#pragma unroll
+        for (int i = 0; i < 2 * DI; i++) K[i] = *(const cm_f32x4 *) (blk + L.k + (i * 64 + lane) * 4);
+#pragma unroll
+        for (int m = 0; m < DI; m++) G[m] = *(const cm_f32x4 *) (blk + L.g + 16 * m + 4 * g);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (RULE == 0)
+#pragma unroll
+            for (int s = 0; s < DI; s++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) { U[0] = cm_mfma(W[s][i], S[s][i], U[0]); U[1] = cm_mfma(W[DI + s][i], S[s][i], U[1]); }
+        const cm_f32x4 U0 = U[0], U1 = U[1];
+        __builtin_amdgcn_sched_barrier(0);
+        ahead(p + 1 < np ? blk + step : blk, p + 1 < np ? at + CP_TB : at);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < DI; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) { O[0] = cm_mfma(Q[s][i], S[s][i], O[0]); O[1] = cm_mfma(Q[DI + s][i], S[s][i], O[1]); }
+#pragma unroll
+        for (int m = 0; m < DI; m++) S[m] *= G[m];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int m = 0; m < DI; m++) S[m] = cm_mfma(K[2 * m][i], U0[i], S[m]);
+        O[0] = cm_mfma4(P[0], U0, O[0]);
+        O[1] = cm_mfma4(P[1], U0, O[1]);
+        O[1] = cm_mfma4(P[2], U1, O[1]);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int m = 0; m < DI; m++) S[m] = cm_mfma(K[2 * m + 1][i], U1[i], S[m]);
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) { const int t = 16 * m + 4 * g + r; if (t < len) out[(int64_t) (at + t) * os + (int64_t) h * vdim + c] = O[m][r]; }
+    }
+#pragma unroll
+    for (int m = 0; m < DI; m++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) S_hbm[(int64_t) (16 * m + 4 * g + r) * vdim] = S[m][r];
+}
+
 #define CR_LDS_MAX (150 * 1024)
 template <int DPT, int RULE> static int cr_reserve_one() { PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_recurrence<DPT, RULE>, hipFuncAttributeMaxDynamicSharedMemorySize, CR_LDS_MAX)); return 0; }
 extern "C" int pi_op_channel_recurrence_reserve(void) {
@@ -457,9 +784,15 @@ extern "C" int pi_op_channel_recurrence_reserve(void) {
     return 0;
 }
 static int cr_max_pieces(int n_tok, int max_segments, int piece = CR_TB) { return n_tok / piece + std::min(n_tok, std::max(1, max_segments)) + 1; }
+// whether the matrix cores take a pass (of pieces), and the floats of scratch it needs for them
+static bool cp_takes(int dim, int vdim) { return (dim == 32 || dim == 64 || dim == 128) && vdim % 16 == 0; }
+static size_t cp_floats(int heads, int dim, int vdim, int n_tok, int max_segments) { return (size_t) cr_max_pieces(n_tok, max_segments) * heads * cp_of(dim, vdim).total; }
+// floats of scratch that the walks need
+static size_t cr_floats(int heads, int dim, int vdim, int n_tok, int max_segments) { return (n_tok <= CR_TB || dim > CR_SCAN_MAXDIM) ? 0 : (size_t) cr_max_pieces(n_tok, max_segments) * heads * dim * (vdim + dim); }
 // passes of more than 32 tokens cut the runs into pieces that run side by side: floats of scratch they need (0: such a pass is walked in one piece per run)
 extern "C" size_t pi_op_channel_recurrence_scratch_floats(int heads, int dim, int vdim, int n_tok, int max_segments) {      // (sized for the delta rule, which needs more)
-    return (n_tok <= CR_TB || dim > CR_SCAN_MAXDIM) ? 0 : (size_t) cr_max_pieces(n_tok, max_segments) * heads * dim * (vdim + dim);
+    const size_t need = cr_floats(heads, dim, vdim, n_tok, max_segments);
+    return need > 0 && cp_takes(dim, vdim) ? std::max(need, cp_floats(heads, dim, vdim, n_tok, max_segments)) : need;
 }
 extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_stride, const float * k, int64_t k_stride, const float * v, int64_t v_stride, const float * decay_raw, int64_t decay_stride, int decay_mode,
                                         const float * decay_bias_dev, const float * a_log_dev, const float * beta_raw, int64_t beta_stride, const float * bonus_dev, int qk_unit, float q_mult,
@@ -473,7 +806,7 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
     if (max_segments > CR_MAXRUNS) { pi_set_error("pi_op_channel_recurrence: at most %d sequences in a pass", CR_MAXRUNS); return -1; }
     const int dpt = dim <= 8 ? 8 : dim <= 16 ? 16 : 32;                // state values a thread keeps in registers
     int R = 1; while (R * dpt < dim) R *= 2;
-    const size_t need = pi_op_channel_recurrence_scratch_floats(heads, dim, vdim, n_tok, max_segments);
+    const size_t need = cr_floats(heads, dim, vdim, n_tok, max_segments);
     const bool pieces = need > 0 && scratch_dev && scratch_floats >= need;       // (without scratch a long pass is still right, only serial)
     const int runs = std::max(1, std::min(n_tok, max_segments));
     const double bytes = 4.0 * n_tok * heads * (3.0 * dim + 2.0 * vdim) + 8.0 * heads * dim * vdim;
@@ -501,6 +834,19 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
         PI_CHECK_LAUNCH(); return 0;
     };
     if (!pieces) return launch(0);
+    if (cp_takes(dim, vdim) && (rule == PI_RULE_BONUS || qk_unit) && scratch_floats >= cp_floats(heads, dim, vdim, n_tok, max_segments) && ((uintptr_t) scratch_dev & 15) == 0) {
+        const dim3 pg((unsigned) heads, (unsigned) cr_max_pieces(n_tok, max_segments, CP_TB)), wg((unsigned) heads, (unsigned) (vdim / 16), (unsigned) runs);
+        const double blocks = 4.0 * pg.y * heads * cp_of(dim, vdim).total;
+#define CP_GO(DI, RL) do { PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_pieces<DI, RL>), pg, dim3(256), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
+                                        beta_raw, beta_stride, bonus_dev, qk_unit, q_mult, heads, heads / qk_heads, vdim, rec_dev, n_tok, scratch_dev, pi_abort_word()); \
+                           PI_CHECK_LAUNCH(); \
+                           PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_walk<DI, RL>), wg, dim3(64), 0, s, v, v_stride, heads, vdim, state_dev, rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word()); } while (0)
+#define CP_RULE(RL) do { if (dim == 32) CP_GO(2, RL); else if (dim == 64) CP_GO(4, RL); else CP_GO(8, RL); } while (0)
+        if (rule == PI_RULE_DELTA) CP_RULE(0); else CP_RULE(1);
+#undef CP_RULE
+#undef CP_GO
+        PI_CHECK_LAUNCH(); return 0;
+    }
     if (launch(1) != 0) return -1;
     const int n_pieces = cr_max_pieces(n_tok, max_segments, piece);
     if (rule == PI_RULE_BONUS) {

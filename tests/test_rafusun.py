@@ -358,6 +358,47 @@ def test_channel_recurrence_rules_decays_and_passes(H, G, D, V, rule, pieces):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 16), (3, 3, 64, 64), (4, 2, 128, 48), (1, 1, 128, 128)])
+@pytest.mark.parametrize("rule", [DELTA, BONUS])
+def test_channel_recurrence_pieces_on_the_matrix_cores(H, G, D, V, rule):
+    """the sizes that long passes take the matrix cores for: the same plan of passes"""
+    test_channel_recurrence_rules_decays_and_passes(H, G, D, V, rule, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rule,qk_unit", [(DELTA, 1), (BONUS, 0), (DELTA, 0)])
+def test_channel_recurrence_pieces_against_the_walk(rule, qk_unit):
+    """against the walk token by token: decays of nothing and of one, equal keys (every entry of the piece's triangle as large as it gets), a state that was there; values, keys and decays that are no numbers
+    reach their own token's outputs and later ones, and no others"""
+    U, lib = gpu()
+    H, D, V, T, slots = 2, 64, 32, 150, 2
+    rng = np.random.default_rng(rule + qk_unit)
+    q, k, v = (rng.standard_normal((T, H * n)).astype(np.float32) * 0.3 for n in (D, D, V))
+    k[40:60] = k[40]
+    raw, braw, bonus = rng.choice([0.0, 1e-30, 1e-6, 0.5, 0.999, 1.0], (T, H * D)).astype(np.float32), (rng.standard_normal((T, H)) * 4).astype(np.float32), rng.standard_normal((H, D)).astype(np.float32)
+    raw[64:96] = 1.0
+    state = rng.standard_normal((slots, H, D, V)).astype(np.float32)
+    rec = np.array([0] * 113 + [1 | F] + [1] * 36, np.int32)
+    n = int(lib.pi_op_channel_recurrence_scratch_floats(H, D, V, T, slots))
+    for where in (None, "v", "k", "g"):
+        a = {"q": q.copy(), "k": k.copy(), "v": v.copy(), "g": raw.copy()}
+        if where:
+            a[where][50, 3] = np.inf if where != "g" else np.nan
+        outs, states = [], []
+        for pieces in (True, False):
+            ds = [U.Dev(x) for x in (a["q"], a["k"], a["v"], a["g"], braw, bonus, rec)]
+            sd, od, scr = U.Dev(state), U.Dev(nbytes=4 * T * H * V), U.Dev(np.full(n, np.nan, np.float32))
+            L.check(lib.pi_op_channel_recurrence(rule, ds[0].ptr, H * D, ds[1].ptr, H * D, ds[2].ptr, H * V, ds[3].ptr, H * D, 0, None, None, ds[4].ptr, H, ds[5].ptr, qk_unit, 0.7, H, H, D, V, sd.ptr, ds[6].ptr, T, slots,
+                                                 scr.ptr if pieces else None, n if pieces else 0, od.ptr, H * V, None))
+            outs.append(od.get(np.float32, (T, H, V)))
+            states.append(sd.get(np.float32, state.shape))
+        for got, want in zip((outs[0], states[0]), (outs[1], states[1])):
+            fine = np.isfinite(want)
+            assert np.array_equal(np.isfinite(got), fine) and rel_rms(np.where(fine, got, 0), np.where(fine, want, 0)) < 1e-5, where
+        assert np.isfinite(outs[0][:50]).all() and np.isfinite(outs[0][113:]).all() and (where is None) == bool(np.isfinite(outs[0]).all())
+
+
+@pytest.mark.gpu
 def test_delta_rule_keeps_a_far_value_and_replaces_it():
     """a value written under one key 300 tokens back (decays of one, other keys orthogonal) is read back exactly; written again, the new value replaces the old one"""
     U, lib = gpu()
