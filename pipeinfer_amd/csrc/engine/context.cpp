@@ -1003,13 +1003,25 @@ static int n_segments(const llama_context * ctx) {
 }
 bool hop_store(void * dst, const void * src, size_t bytes, hipStream_t s);
 // x_in (device, [n_tokens][n_embd]) replaces the embedding lookup on stages after the first
-static bool launch_inputs(llama_context * ctx, int n_tokens, const void * meta, const float * x_in) {
+// in_place: meta is a page-locked block that the device reads itself, in one launch; arm (nullable): that launch arms the abort word for this run
+static bool launch_inputs(llama_context * ctx, int n_tokens, const void * meta, const float * x_in, bool in_place = false, const pi_run * arm = nullptr) {
     const int words = (ctx->n_ctx + 31) / 32;
     // block: tokens[n] | pos[n] | {kv_head, n_kv, n, has_table} | (cell[n], n_kv[n] when has_table: a pass that carries several runs) | mask[n][words]
     const int32_t * h_tok = (const int32_t *) meta, * h_pos = h_tok + n_tokens, * h_dyn = h_pos + n_tokens;
     const size_t n_table = h_dyn[3] ? (size_t) 2 * n_tokens : 0;
     const uint32_t * h_mask = (const uint32_t *) (h_dyn + 4 + n_table);
     hipStream_t s = ctx->stream;
+    if (in_place) {
+        void * dst[PI_COPY_IN_PARTS] = { ctx->tokens_dev, ctx->pos_dev, ctx->dyn_dev, ctx->mask_dev, ctx->rec_dev, ctx->pair_dev };
+        const int64_t words_of[PI_COPY_IN_PARTS] = { n_tokens, n_tokens, 4 + (int64_t) n_table, (int64_t) n_tokens * words, ctx->rec_dev || ctx->pair_dev ? n_tokens : 0, ctx->pair_dev ? n_tokens : 0 };
+        const bool word = arm && ctx->abort_dev;
+        if (pi_op_copy_in(meta, PI_COPY_IN_PARTS, dst, words_of, word ? ctx->abort_dev : nullptr, word ? arm->run_id : 0, word ? ctx->abort_host + (arm->run_id & 255) : nullptr, s) != 0) {
+            ctx->last_error = std::string("pi_op_copy_in: ") + pi_last_error();
+            return false;
+        }
+        if (x_in && !hop_store(ctx->x, x_in, (size_t) 4 * n_tokens * ctx->model->hparams.n_embd, s)) { ctx->last_error = "H2D of batch metadata failed"; return false; }
+        return true;
+    }
     bool ok = hipMemcpyAsync(ctx->tokens_dev, h_tok, (size_t) 4 * n_tokens, hipMemcpyHostToDevice, s) == hipSuccess &&
               hipMemcpyAsync(ctx->pos_dev, h_pos, (size_t) 4 * n_tokens, hipMemcpyHostToDevice, s) == hipSuccess &&
               hipMemcpyAsync(ctx->dyn_dev, h_dyn, 16 + 4 * n_table, hipMemcpyHostToDevice, s) == hipSuccess &&
@@ -1115,8 +1127,8 @@ static bool launch_outputs(llama_context * ctx, pi_run * run) {
     if (!ok) ctx->last_error = "D2H of logits failed";
     return ok;
 }
-static bool launch_forward(llama_context * ctx, int n_tokens, const void * meta, const float * x_in, pi_kt_sink ** sink_out) {
-    if (!launch_inputs(ctx, n_tokens, meta, x_in)) return false;
+static bool launch_forward(llama_context * ctx, int n_tokens, const void * meta, const float * x_in, pi_kt_sink ** sink_out, bool in_place = false, const pi_run * arm = nullptr) {
+    if (!launch_inputs(ctx, n_tokens, meta, x_in, in_place, arm)) return false;
     const int kv_head = ((const int32_t *) meta)[2 * n_tokens];
     const int n_kv = ((const int32_t *) meta)[2 * n_tokens + 1];
     for (int seg = 0, n = n_segments(ctx); seg < n; seg++) if (!launch_segment(ctx, n_tokens, kv_head, seg, sink_out, false, false, n_kv)) return false;
@@ -1234,7 +1246,7 @@ static void feed_pass(llama_context * ctx, const std::shared_ptr<pi_pass> & pass
         const void * meta = runs.size() == 1 ? (const void *) runs[0]->meta_host : compose_pass(ctx, runs, pass->n_tokens);
         ok = ok && meta != nullptr;
         const int nseg = n_segments(ctx), kv_head = ok ? ((const int32_t *) meta)[2 * n] : 0;
-        if (ok) ok = launch_inputs(ctx, n, meta, nullptr);
+        if (ok) ok = launch_inputs(ctx, n, meta, nullptr, true);
         int seg = 0;
         for (; ok && seg < nseg; seg++) {
             if (seg >= 2) (void) hipEventSynchronize(seg_done[seg & 1]);       // at most two segments ahead of the GPU
@@ -1467,8 +1479,7 @@ pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & 
         return run;
     }
     if (!run->canceled) {                                                     // a cancelled run still occupies its cells and completes "empty" (llama.cpp:5627-5716)
-        ok = launch_abort_begin(ctx, run->run_id);
-        if (ok) ok = launch_forward(ctx, n_tokens, run->meta_host, nullptr, &run->sink);
+        ok = launch_forward(ctx, n_tokens, run->meta_host, nullptr, &run->sink, !run->host_plain, run);
         if (ok) ok = launch_outputs(ctx, run);
         run->launched = ok;
     }

@@ -117,13 +117,14 @@ static thread_local int g_cu_count = 256;
 int pi_cu_count() { return g_cu_count; }
 extern "C" void pi_set_cu_count(int n) { g_cu_count = n > 0 && n <= 256 ? n : 256; }
 // device-scope atomics only: the exchange at a run's start and the compare-and-swap of a cancel never tear, whichever stream runs first
-__global__ void k_abort_begin(int32_t * word, int32_t run_id, const int32_t * host_flag) {
+static __device__ __forceinline__ void abort_begin(int32_t * word, int32_t run_id, const int32_t * host_flag) {
     const int32_t f = host_flag ? __hip_atomic_load(host_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : 0;
     // (a later segment of the SAME run keeps an abort the word already carries: one inherited from the upstream stage has no host flag behind it)
     const int32_t old = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int32_t keep = (old >> 1) == run_id ? (old & 1) : 0;
     __hip_atomic_exchange(word, (run_id << 1) | (f != 0) | keep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__global__ void k_abort_begin(int32_t * word, int32_t run_id, const int32_t * host_flag) { abort_begin(word, run_id, host_flag); }
 // ---- arrival flags of the stage transport (transport.cpp): the activations of a run cross a stage boundary with no host thread on the critical path.
 // A flag lives in page-locked host memory that both processes map: {ticket << 1 | aborted, -, realtime stamp}.  The producing stage's stream writes it right behind its peer
 // store (k_flag_publish); the consuming stage has enqueued its run already, behind k_abort_begin_wait, which polls the flag from the device and arms the run's abort word —
@@ -205,6 +206,41 @@ extern "C" int pi_op_copy_out(const float * logits_dev, float * logits_host, int
     const int64_t per_wg = 256 * 4 * 4;                                       // four 16-byte stores per thread
     const unsigned grid = (unsigned) std::max<int64_t>(1, std::min<int64_t>(256, (n_logits + per_wg - 1) / per_wg));
     hipLaunchKernelGGL(k_copy_out, dim3(grid), dim3(256), 0, (hipStream_t) stream, logits_dev, logits_host, (size_t) n_logits, ids_dev, ids_host, vals_dev, vals_host, sum_dev, sum_host, n_tok);
+    PI_CHECK_LAUNCH();
+    return 0;
+}
+
+// ---- and a pass's inputs come in through one ------------------------------------------------------------------------------------------------------
+// Tokens, positions, cells, mask rows and slot words lie behind each other in the run's page-locked block; copied part by part they were four to six launches of the runtime's copy kernel, each one
+// with a gap behind it, ahead of the first kernel of every pass (COPYIN_US)
+struct rt_parts { uint32_t * dst[PI_COPY_IN_PARTS]; long long end[PI_COPY_IN_PARTS]; };
+__global__ void __launch_bounds__(256) k_copy_in(const uint32_t * __restrict__ block, rt_parts parts, int32_t * word, int32_t run_id, const int32_t * host_flag) {
+    if (word && blockIdx.x == 0 && threadIdx.x == 0) abort_begin(word, run_id, host_flag);
+    const long long total = parts.end[PI_COPY_IN_PARTS - 1], step = (long long) gridDim.x * 256;
+    for (long long i0 = (long long) blockIdx.x * 256 + threadIdx.x; i0 < total; i0 += 4 * step) {
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = block[min(i0 + u * step, total - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const long long i = i0 + u * step;
+            long long from = 0;
+#pragma unroll
+            for (int p = 0; p < PI_COPY_IN_PARTS; p++) { if (parts.dst[p] && i >= from && i < parts.end[p]) parts.dst[p][i - from] = v[u]; from = parts.end[p]; }
+        }
+    }
+}
+extern "C" int pi_op_copy_in(const void * block_host, int parts, void * const * dst_dev, const int64_t * n, int32_t * abort_word_dev, int32_t run_id, const int32_t * host_flag, void * stream) {
+    if (parts < 1 || parts > PI_COPY_IN_PARTS || !block_host) { pi_set_error("pi_op_copy_in: %d parts (1 .. %d) of a page-locked block", parts, PI_COPY_IN_PARTS); return -1; }
+    rt_parts a;
+    long long end = 0;
+    for (int i = 0; i < PI_COPY_IN_PARTS; i++) {
+        if (i < parts && n[i] < 0) { pi_set_error("pi_op_copy_in: part %d of %lld words", i, (long long) n[i]); return -1; }
+        if (i < parts) end += n[i];
+        a.dst[i] = i < parts ? (uint32_t *) dst_dev[i] : nullptr; a.end[i] = end;
+    }
+    const unsigned grid = (unsigned) std::max<long long>(1, std::min<long long>(256, (end + 1023) / 1024));
+    hipLaunchKernelGGL(k_copy_in, dim3(grid), dim3(256), 0, (hipStream_t) stream, (const uint32_t *) block_host, a, abort_word_dev, run_id & 0x3fffffff, host_flag);
     PI_CHECK_LAUNCH();
     return 0;
 }

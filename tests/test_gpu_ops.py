@@ -875,3 +875,34 @@ def test_copy_out_writes_the_page_locked_buffers(gpu, n_tok, nv, skew):
         assert (tail == 0xA5).all(), "the kernel wrote past the buffers it was given"
     finally:
         hip.hipHostFree(host)
+
+
+@pytest.mark.parametrize("counts", [(1, 1, 4, 8), (7, 7, 18, 35, 7, 7), (513, 513, 4, 300001, 513, 0), (0, 0, 0, 0), (5,)])
+def test_copy_in_reads_the_page_locked_block(gpu, counts):
+    """pi_op_copy_in (runtime.hip): the parts of a page-locked block at their places, none of them past its end, a part without a place skipped; the abort word armed as pi_op_abort_begin arms it"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]; hip.hipHostFree.argtypes = [C.c_void_p]
+    total = sum(counts)
+    block = np.random.default_rng(total).integers(0, 2 ** 32, max(total, 1), dtype=np.uint32)
+    host = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(host), 4 * block.size, 0) == 0
+    try:
+        C.memmove(host, block.ctypes.data, 4 * block.size)
+        sentinel = np.uint32(0xA5A5A5A5)
+        dst = [U.Dev(np.full(n + 3, sentinel, np.uint32)) for n in counts]
+        skipped = len(counts) - 2 if len(counts) > 4 else None
+        ptrs = (C.c_void_p * len(counts))(*[None if i == skipped else d.ptr for i, d in enumerate(dst)])
+        word, flag = U.Dev(np.zeros(16, np.int32)), U.Dev(np.ones(1, np.int32))
+        L.check(lib.pi_op_copy_in(host, len(counts), ptrs, (C.c_int64 * len(counts))(*counts), word.ptr, 9, flag.ptr, None))
+        L.check(lib.pi_stream_sync(None))
+        at = 0
+        for i, (d, n) in enumerate(zip(dst, counts)):
+            got = d.get(np.uint32)
+            assert np.array_equal(got[:n], block[at:at + n] if i != skipped else np.full(n, sentinel)) and (got[n:] == sentinel).all()
+            at += n
+        assert word.get(np.int32)[0] == (9 << 1) | 1
+        assert lib.pi_op_copy_in(host, 7, ptrs, (C.c_int64 * len(counts))(*counts), None, 0, None, None) != 0
+    finally:
+        hip.hipHostFree(host)
