@@ -212,7 +212,7 @@ extern "C" int pi_op_copy_out(const float * logits_dev, float * logits_host, int
 
 // ---- and a pass's inputs come in through one ------------------------------------------------------------------------------------------------------
 // Tokens, positions, cells, mask rows and slot words lie behind each other in the run's page-locked block; copied part by part they were four to six launches of the runtime's copy kernel, each one
-// with a gap behind it, ahead of the first kernel of every pass (COPYIN_US)
+// with a gap behind it, ahead of the first kernel of every pass (10 us of a pass)
 struct rt_parts { uint32_t * dst[PI_COPY_IN_PARTS]; long long end[PI_COPY_IN_PARTS]; };
 __global__ void __launch_bounds__(256) k_copy_in(const uint32_t * __restrict__ block, rt_parts parts, int32_t * word, int32_t run_id, const int32_t * host_flag) {
     if (word && blockIdx.x == 0 && threadIdx.x == 0) abort_begin(word, run_id, host_flag);
