@@ -31,6 +31,8 @@ llama_context::~llama_context() {
         for (void * b : hb) if (b) { if (r->host_plain) free(b); else (void) hipHostFree(b); }
         delete r;
     }
+    free(logits);
+    if (logits_own) { if (remote) free(logits_own); else (void) hipHostFree(logits_own); }
     for (auto & kv : graphs) if (kv.second.exec) (void) hipGraphExecDestroy(kv.second.exec);
     for (hipEvent_t e : seg_events) if (e) (void) hipEventDestroy(e);
     if (pass_event) (void) hipEventDestroy(pass_event);
@@ -283,7 +285,7 @@ static bool context_prepare_impl(llama_context * ctx, std::string & err) {
     return true;
 }
 
-static pi_run * acquire_run(llama_context * ctx, int n_tokens, size_t meta_bytes) {
+static pi_run * acquire_run(llama_context * ctx, int n_tokens, int rows, size_t meta_bytes, bool until_done) {      // rows: of logits, that the run's buffer has to hold
     pi_run * r = nullptr;
     if (!ctx->pool.empty()) { r = ctx->pool.back(); ctx->pool.pop_back(); }
     else {
@@ -292,16 +294,24 @@ static pi_run * acquire_run(llama_context * ctx, int n_tokens, size_t meta_bytes
     }
     auto host_alloc = [&](void ** p, size_t bytes) { if (r->host_plain) { *p = malloc(bytes); return *p != nullptr; } return hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess; };
     auto host_free = [&](void * p) { if (r->host_plain) free(p); else (void) hipHostFree(p); };
-    const size_t need = ctx->is_last ? (size_t) n_tokens * ctx->model->hparams.n_vocab : 0;
+    const size_t need = ctx->is_last ? (size_t) rows * ctx->model->hparams.n_vocab : 0;
+    // (the buffer that the caller read the last run's rows in comes back where those rows are not read any more: such callers never pay for a second one)
+    if (need > r->logits_cap && until_done && ctx->logits_own_cap >= need) { std::swap(ctx->logits_own, r->logits_host); std::swap(ctx->logits_own_cap, r->logits_cap); }
     if (need > r->logits_cap) {
         if (r->logits_host) host_free(r->logits_host);
+        r->logits_host = nullptr; r->logits_cap = 0;
+        const size_t cap = std::max(need, (size_t) 16 * ctx->model->hparams.n_vocab);
+        if (!host_alloc((void **) &r->logits_host, cap * 4)) { r->logits_host = nullptr; ctx->pool.push_back(r); return nullptr; }
+        r->logits_cap = cap;
+    }
+    if (ctx->is_last && n_tokens > r->topk_rows) {                             // (apart from the rows: a finished run's logits buffer may go to the caller)
         if (r->topk_ids) host_free(r->topk_ids);
-        r->logits_cap = std::max(need, (size_t) 16 * ctx->model->hparams.n_vocab);
-        const size_t rows = r->logits_cap / ctx->model->hparams.n_vocab;
-        if (!host_alloc((void **) &r->logits_host, r->logits_cap * 4)) return nullptr;
-        if (!host_alloc((void **) &r->topk_ids, rows * (8 * 4 + 8 * 4 + 4))) return nullptr;
+        r->topk_ids = nullptr; r->topk_rows = 0;
+        const size_t rows = (size_t) std::max(n_tokens, 16);
+        if (!host_alloc((void **) &r->topk_ids, rows * (8 * 4 + 8 * 4 + 4))) { r->topk_ids = nullptr; ctx->pool.push_back(r); return nullptr; }
         r->topk_vals = (float *) (r->topk_ids + rows * 8);
         r->topk_sum  = r->topk_vals + rows * 8;
+        r->topk_rows = (int) rows;
     }
     if (meta_bytes > r->meta_cap) {
         if (r->meta_host) host_free(r->meta_host);
@@ -1093,13 +1103,13 @@ static bool launch_segment(llama_context * ctx, int n_tokens, int kv_head, int s
     pi_set_abort_word(nullptr);
     return fwd;
 }
+static bool outputs_by_memcpy() { static const bool on = getenv("PIPEINFER_COPY_OUT") && !strcmp(getenv("PIPEINFER_COPY_OUT"), "memcpy"); return on; }
 static bool launch_outputs(llama_context * ctx, pi_run * run) {
     if (!ctx->is_last) return true;
     hipStream_t s = ctx->stream;
     const size_t nv = ctx->model->hparams.n_vocab, r0 = (size_t) run->row0; const int n_tokens = run->n_tokens;
     // by a kernel that writes the run's page-locked buffers (pi_op_copy_out: a copy-engine transfer waits for the OTHER context's kernels); PIPEINFER_COPY_OUT=memcpy: plain copies of all rows
-    static const bool by_memcpy = getenv("PIPEINFER_COPY_OUT") && !strcmp(getenv("PIPEINFER_COPY_OUT"), "memcpy");
-    if (!by_memcpy && !run->host_plain) {
+    if (!outputs_by_memcpy() && !run->host_plain) {
         // the rows that phase 1 hands back (all of them for a tap): consecutive ones in one launch, the first launch brings the top-8 of every row.  A 512-token prompt that wants its last row brings
         // 128 KB over the bus instead of 65 MB (1.2 ms at the bus's 56 GB/s, a fifth of such a pass)
         auto wanted = [&](int i) { return run->all_rows || (run->last_only ? i == n_tokens - 1 : run->want_logits[(size_t) i] != 0); };
@@ -1107,10 +1117,13 @@ static bool launch_outputs(llama_context * ctx, pi_run * run) {
         for (int i = 0; i < n_tokens; i++) if (wanted(i)) { low = std::min(low, i); high = i + 1; ranges += i == 0 || !wanted(i - 1); }
         const bool whole = ranges > 8;                                          // (scattered rows: from the first to the last in one launch)
         bool first = true;
+        int at = 0;
         auto copy = [&](int a, int b) {
             const int tops = first ? n_tokens : 0;
             first = false;
-            return pi_op_copy_out(ctx->logits_dev + (r0 + (size_t) a) * nv, run->logits_host + (size_t) a * nv, (int64_t) (b - a) * (int64_t) nv, ctx->topk_ids_dev + r0 * 8, run->topk_ids, ctx->topk_vals_dev + r0 * 8,
+            float * to = run->logits_host + (size_t) (run->compact ? at : a) * nv;
+            at += b - a;
+            return pi_op_copy_out(ctx->logits_dev + (r0 + (size_t) a) * nv, to, (int64_t) (b - a) * (int64_t) nv, ctx->topk_ids_dev + r0 * 8, run->topk_ids, ctx->topk_vals_dev + r0 * 8,
                                   run->topk_vals, ctx->topk_sum_dev + r0, run->topk_sum, tops, s) == 0;
         };
         bool ok = true;
@@ -1347,7 +1360,7 @@ static void feeder_main(llama_context * ctx) {
     }
 }
 
-pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & rc) {
+pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & rc, bool until_done) {
     rc = -1;
     std::string err;
     if (!context_prepare(ctx, err)) { ctx->last_error = err; fprintf(stderr, "llama_decode: %s\n", err.c_str()); return nullptr; }
@@ -1414,7 +1427,12 @@ pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & 
         }
     }
     const size_t meta_bytes = (size_t) n_tokens * 8 + 16 + (size_t) n_tokens * words * 4 + (recurrent ? (size_t) n_tokens * 4 : 0) + (pairs ? (size_t) n_tokens * 4 : 0);
-    pi_run * run = acquire_run(ctx, n_tokens, meta_bytes);
+    // the rows that come back: the flagged ones (the last one without flags); room for them alone where they are few consecutive stretches
+    const bool all_rows = ctx->run_tap != nullptr, last_only = !batch_in.logits && !ctx->cparams.logits_all;
+    int wanted = 0, ranges = 0;
+    for (int i = 0; i < n_tokens; i++) if (last_only ? i == n_tokens - 1 : !batch_in.logits || batch_in.logits[i] != 0) { wanted++; ranges += i == 0 || last_only || (batch_in.logits && batch_in.logits[i - 1] == 0); }
+    const bool compact = !all_rows && !ctx->remote && !outputs_by_memcpy() && ranges <= 8;
+    pi_run * run = acquire_run(ctx, n_tokens, compact ? wanted : n_tokens, meta_bytes, until_done);
     // (a run that cannot be started gives the cells find_slot just allotted back: nothing was or will be written to them)
     auto give_back = [&]() { ctx->cells->release_cells(kv_head, n_tokens); for (int sl : fresh_taken) ctx->slots->mark_fresh(sl); for (auto it = last_before.rbegin(); it != last_before.rend(); ++it) ctx->slots->set_last_token(it->first, it->second); };
     if (!run) { ctx->last_error = "out of pinned host memory"; give_back(); return nullptr; }
@@ -1431,10 +1449,9 @@ pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & 
     if (!ctx->remote && ctx->seg_layers == 0 && hipEventRecord(run->begin, ctx->stream) != hipSuccess) { ctx->last_error = "hipEventRecord failed"; give_back(); ctx->pool.push_back(run); return nullptr; }
     // which rows phase 1 hands back (llama.cpp:5776-5789): flagged rows, or all with logits_all, or only the last one (stored at row 0)
     run->want_logits.assign(n_tokens, 1);
-    run->last_only = false;
-    run->all_rows = ctx->run_tap != nullptr;
+    run->last_only = last_only;
+    run->all_rows = all_rows; run->compact = compact;
     if (batch_in.logits) for (int i = 0; i < n_tokens; i++) run->want_logits[i] = batch_in.logits[i] != 0;
-    else if (!ctx->cparams.logits_all) run->last_only = true;
     int32_t * h_tok = (int32_t *) run->meta_host, * h_pos = h_tok + n_tokens, * h_dyn = h_pos + n_tokens; uint32_t * h_mask = (uint32_t *) (h_dyn + 4);
     memcpy(h_tok, batch_in.token, (size_t) 4 * n_tokens);
     memcpy(h_pos, pos, (size_t) 4 * n_tokens);
@@ -1820,10 +1837,25 @@ int context_finish(llama_context * ctx, pi_run * run) {
     const int n = run->n_tokens;
     if (ctx->run_tap) ctx->run_tap(ctx->run_tap_user, run->run_id, run->batch_id, n, run->meta_host, run->meta_bytes, run->launched && ctx->is_last && !run->canceled && run->all_rows ? run->logits_host : nullptr);
     if (ctx->is_last) {
-        ctx->logits.resize(run->last_only ? nv : (size_t) n * nv);             // llama.cpp:5734-5743
+        size_t wanted = run->last_only ? 1 : 0;
+        if (!run->last_only) for (int i = 0; i < n; i++) wanted += run->want_logits[i] != 0;
+        // many rows (a scored text): the run's buffer itself goes to the caller (333 rows of 32000 copied: 2 ms of a 4 ms pass)
+        const bool take = run->launched && !run->last_only && wanted * nv * 4 >= ((size_t) 4 << 20) && (!run->compact || wanted == (size_t) n);
+        if (take) { std::swap(ctx->logits_own, run->logits_host); std::swap(ctx->logits_own_cap, run->logits_cap); ctx->logits_out = ctx->logits_own; }
+        else {                                                                 // llama.cpp:5734-5743
+            const size_t size = run->last_only ? nv : (size_t) n * nv;
+            if (size > ctx->logits_size) {                                     // (zeros that cost nothing until somebody reads them: a prompt's caller looks at its last row)
+                float * bigger = (float *) calloc(size, 4);
+                if (!bigger) { ctx->last_error = "out of host memory (logits)"; run->launched = false; }
+                else { if (ctx->logits) memcpy(bigger, ctx->logits, ctx->logits_size * 4); free(ctx->logits); ctx->logits = bigger; ctx->logits_size = size; }
+            }
+            ctx->logits_out = size <= ctx->logits_size ? ctx->logits : nullptr;
+        }
         if (run->launched) {
-            if (run->last_only) memcpy(ctx->logits.data(), run->logits_host + (size_t) (n - 1) * nv, nv * 4);
-            else for (int i = 0; i < n; i++) if (run->want_logits[i]) memcpy(ctx->logits.data() + (size_t) i * nv, run->logits_host + (size_t) i * nv, nv * 4);
+            const float * from = run->logits_host;
+            if (take) {}
+            else if (run->last_only) memcpy(ctx->logits, from + (run->compact ? 0 : (size_t) (n - 1) * nv), nv * 4);
+            else for (int i = 0; i < n; i++) if (run->want_logits[i]) { memcpy(ctx->logits + (size_t) i * nv, run->compact ? from : from + (size_t) i * nv, nv * 4); if (run->compact) from += nv; }
             ctx->last_topk_ids.assign(run->topk_ids, run->topk_ids + (size_t) n * 8);
             ctx->last_topk_vals.assign(run->topk_vals, run->topk_vals + (size_t) n * 8);
             ctx->last_topk_sum.assign(run->topk_sum, run->topk_sum + n);

@@ -240,8 +240,10 @@ struct pi_run {                                // one llama_start_async_decode .
     hipEvent_t done = nullptr, begin = nullptr;
     float * logits_host = nullptr;            // pinned [n_tokens][n_vocab]
     size_t logits_cap = 0;
+    bool compact = false;                     // logits_host holds the wanted rows only, one behind the other
     bool all_rows = false;                    // every row comes back to logits_host, not only the wanted ones (a run tap was set when the run was started)
-    int32_t * topk_ids = nullptr; float * topk_vals = nullptr; float * topk_sum = nullptr;   // pinned [n_tokens][8], [n_tokens]
+    int32_t * topk_ids = nullptr; float * topk_vals = nullptr; float * topk_sum = nullptr;   // pinned [topk_rows][8], [topk_rows]
+    int topk_rows = 0;
     uint8_t * meta_host = nullptr; size_t meta_cap = 0;                                       // pinned staging for tokens/pos/mask
     int64_t t_start_us = 0;
     pi_kt_sink * sink = nullptr;            // kernel-timing samples of the graph this run replayed
@@ -360,7 +362,9 @@ struct llama_context {
     std::deque<pi_run *> inflight;            // oldest at front
     std::vector<pi_run *> pool;
     std::set<int32_t> canceled_batches;
-    std::vector<float> logits;                // API-visible buffer (llama_get_logits)
+    float * logits = nullptr; size_t logits_size = 0;             // API-visible buffer (llama_get_logits): the rows of a run that wanted few,
+    float * logits_own = nullptr; size_t logits_own_cap = 0;      // or a whole run's page-locked buffer, taken over from it (the run gets the one before),
+    float * logits_out = nullptr;             // whichever of the two the last finished run's rows are in
     std::vector<int32_t> last_topk_ids; std::vector<float> last_topk_vals, last_topk_sum; int last_n_tokens = 0;
 
     // timings (llama.cpp:10170-10206)
@@ -385,7 +389,7 @@ extern bool g_timeline_on;
 void timeline_note(const char * tag, int a, int b, int c);
 inline void tl(const char * tag, int a = 0, int b = 0, int c = 0) { if (g_timeline_on) timeline_note(tag, a, b, c); }
 bool context_prepare(llama_context * ctx, std::string & err);          // uploads weights, allocates KV + scratch
-pi_run * context_start(llama_context * ctx, const llama_batch & batch, int & rc);   // rc: 0 ok, 1 no slot, <0 error
+pi_run * context_start(llama_context * ctx, const llama_batch & batch, int & rc, bool until_done = false);   // rc: 0 ok, 1 no slot, <0 error; until_done: the caller finishes the run before it reads any logits again
 int  context_finish(llama_context * ctx, pi_run * run);
 bool context_poll_oldest(llama_context * ctx);
 bool context_precapture(llama_context * ctx, int max_tokens);             // captures the graphs of passes of 1..max_tokens tokens now (idle context, calling thread)

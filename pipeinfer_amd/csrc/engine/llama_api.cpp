@@ -122,13 +122,13 @@ extern "C" int llama_finish_async_decode(struct llama_context * ctx, struct llam
 extern "C" int llama_decode(struct llama_context * ctx, struct llama_batch batch) {
     if (ctx->node_id < 0) return 0;                                                                 // llama.cpp:10007-10008
     int rc;
-    pi_run * run = pi::context_start(ctx, batch, rc);
+    pi_run * run = pi::context_start(ctx, batch, rc, true);
     if (!run) return rc;
     return pi::context_finish(ctx, run) == 1 ? 0 : -1;
 }
 
-extern "C" float * llama_get_logits(struct llama_context * ctx) { return ctx->logits.data(); }
-extern "C" float * llama_get_logits_ith(struct llama_context * ctx, int32_t i) { return ctx->logits.data() + (size_t) i * ctx->model->hparams.n_vocab; }
+extern "C" float * llama_get_logits(struct llama_context * ctx) { return ctx->logits_out; }
+extern "C" float * llama_get_logits_ith(struct llama_context * ctx, int32_t i) { return ctx->logits_out + (size_t) i * ctx->model->hparams.n_vocab; }
 
 // ---- batches (llama.cpp:9839-9898) ------------------------------------------------------------------------------------------
 extern "C" struct llama_batch llama_batch_get_one(llama_token * tokens, int32_t n_tokens, llama_pos pos_0, llama_seq_id seq_id) {

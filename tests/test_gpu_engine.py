@@ -890,3 +890,24 @@ def test_only_the_wanted_rows_come_back(LL, wanted):
     ctx.set_run_tap(None)
     assert len(seen) == 2 and seen[0] is None and np.array_equal(seen[1].view(np.uint32), full.view(np.uint32))
     ctx.free(); m.free()
+
+
+def test_many_rows_are_handed_over_without_a_copy(LL):
+    """a run that wants 4 MB of rows and more hands its own page-locked buffer to the caller: the rows that came back, behind passes that are wider, narrower and below that (the buffers change hands)"""
+    m = LL.Model(os.path.join(GOLD, "tiny_llama_q4_k_m.gguf"))
+    n = (4 << 20) // (4 * m.n_vocab) + 12
+    toks = [int(t) for t in np.random.default_rng(6).integers(3, m.n_vocab, n)]
+    ctx = LL.Context(m, n_ctx=n + 40, n_batch=n)
+    seen, tops = {}, {}
+    ctx.set_run_tap(lambda run_id, batch_id, k, block, rows: seen.__setitem__(k, rows))
+    for count in (n, n - 12, 700, n - 1, 5, n):
+        ctx.kv_clear()
+        got = ctx.decode(toks[:count], list(range(count)), [[0]] * count)
+        assert np.array_equal(got.view(np.uint32), seen[count].view(np.uint32)), count
+        best = ctx.topk(count - 1)
+        assert best[0][0] == int(np.argmax(got[-1])) and tops.setdefault(count, best) == best
+        one = ctx.decode(toks[count - 1:count], [count - 1], [[1]])                     # (a sequence of its own: nothing of the others is seen)
+        ctx.seq_rm(1, -1, -1)
+        assert np.array_equal(one.view(np.uint32), seen[1].view(np.uint32)) and np.isfinite(one).all()
+    ctx.set_run_tap(None)
+    ctx.free(); m.free()

@@ -215,3 +215,22 @@ def test_hand_worked_placement():
     assert st[3][1] == (7, (2,)) and st[3][0] == (0, (0, 2))
     m = e.mask(st[2], [8], [[2]])
     assert m[0, 0] and m[0, 1] and not m[0, 6]                 # seq 2 sees its own cells and the copied prefix, not seq 1's cell
+
+
+def test_mask_of_a_sequence_s_consecutive_tokens():
+    """runs of tokens of one sequence (their rows are built from the one before): positions rising, repeated, falling back, cells out of position order, shared cells, several runs in a batch, ids that no cell has"""
+    rng = np.random.default_rng(3)
+    for _ in range(60):
+        dev = Eng()
+        for _ in range(int(rng.integers(1, 6))):
+            n = int(rng.integers(1, 5))
+            dev.decode([int(p) for p in rng.integers(0, 12, n)], [sorted(set(int(x) for x in rng.integers(0, 4, rng.integers(1, 3)))) for _ in range(n)])
+        if rng.random() < 0.5:
+            dev.lib.pi_kvcells_seq_rm(dev.h, int(rng.integers(0, 4)), 0, int(rng.integers(1, 8)))
+        n_kv = int(rng.integers(1, N_CTX + 1))
+        runs = [(int(rng.integers(0, 6)), int(rng.integers(1, 9))) for _ in range(int(rng.integers(1, 4)))]
+        seqs = [[s] for s, n in runs for _ in range(n)]
+        pos = [int(p) for p in (np.sort(rng.integers(0, 14, len(seqs))) if rng.random() < 0.5 else rng.integers(0, 14, len(seqs)))]
+        got = dev.mask(n_kv, pos, seqs)
+        for j, (p, s) in enumerate(zip(pos, seqs)):
+            assert [bool(b) for b in got[j]] == [dev.lib.pi_kvcells_nseq(dev.h, c) > 0 and bool(dev.lib.pi_kvcells_has(dev.h, c, s[0])) and dev.lib.pi_kvcells_pos(dev.h, c) <= p for c in range(n_kv)]
