@@ -54,9 +54,10 @@ __global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restri
 static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
-// weights of the cells 4 g + c of a tile of 16, and of the sums the outputs 4 NV (4 g + c) + j
-template <int NK, int NV, int MAPS>
-__global__ void __launch_bounds__(256, NK + 4 * NV > 16 ? 1 : 2) k_prompt_attention(const pa_args A, const int32_t * __restrict__ abort_w) {
+// weights of the cells 4 g + c of a tile of 16, and of the sums the outputs 4 NV (4 g + c) + j.  N1 > 0: whole steps only (dim1 = 16 N1, dim2 = 16 (NK - N1), vdim = 64 NV) and 32-bit offsets, so that a row's
+// loads differ by constants: with an address apiece the registers held no more than one load at a time (2048 tokens, 32 heads of 128: 546 us, 495 this way)
+template <int NK, int N1, int NV, int MAPS>
+__global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_prompt_attention(const pa_args A, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 5)) return;
     constexpr int NJ = 4 * NV, VW = 64 * NV, PARTS = 4 / MAPS;
     __shared__ __attribute__((aligned(16))) float meet[4][16][VW];
@@ -65,7 +66,7 @@ __global__ void __launch_bounds__(256, NK + 4 * NV > 16 ? 1 : 2) k_prompt_attent
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, map = wave % MAPS, part = wave / MAPS;
     const int h = blockIdx.x, t0 = (int) (gridDim.y - 1 - blockIdx.y) * 32;       // (the last tokens, which see the most, first)
     const int n_kv = min(A.dyn ? A.dyn[1] : A.n_kv, A.n_kv), c_end = min(n_kv, A.cell1), words = (A.n_kv + 31) / 32;
-    const int n1 = (A.dim1 + 15) / 16;
+    const int n1 = N1 > 0 ? N1 : (A.dim1 + 15) / 16;
     const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * A.dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
     const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
     pa_f32x4 q[2][NK], acc[2][NJ];
@@ -124,23 +125,37 @@ __global__ void __launch_bounds__(256, NK + 4 * NV > 16 ? 1 : 2) k_prompt_attent
             if (!here) continue;
             const int cb = c0 + 16 * half, spare = __ffs(here) - 1;
             const int ck = cb + (here >> n & 1u ? n : spare);
-            const float * kr1 = k1 + (int64_t) (ck - A.cell0) * A.k1_row, * kr2 = A.k2 + (int64_t) ck * A.k2_row;
             pa_f32x4 kf[NK], vf[4][NV];
+            if constexpr (N1 > 0) {
+                const uint32_t o1 = ((uint32_t) (ck - A.cell0) * (uint32_t) A.k1_row + 4u * g) * 4u, o2 = ((uint32_t) ck * (uint32_t) A.k2_row + 4u * g) * 4u;
 #pragma unroll
-            for (int i = 0; i < NK; i++) {
-                const int d = (i < n1 ? i : i - n1) * 16 + 4 * g;
-                kf[i] = i < n1 || A.dim2 == 0 ? *(const pa_f32x4 *) (kr1 + min(d, A.dim1 - 4)) : *(const pa_f32x4 *) (kr2 + min(d, A.dim2 - 4));
+                for (int i = 0; i < NK; i++) kf[i] = i < N1 ? *(const pa_f32x4 *) ((const char *) k1 + o1 + 64 * i) : *(const pa_f32x4 *) ((const char *) A.k2 + o2 + 64 * (i - N1));
+            } else {
+                const float * kr1 = k1 + (int64_t) (ck - A.cell0) * A.k1_row, * kr2 = A.k2 + (int64_t) ck * A.k2_row;
+#pragma unroll
+                for (int i = 0; i < NK; i++) {
+                    const int d = (i < n1 ? i : i - n1) * 16 + 4 * g;
+                    kf[i] = i < n1 || A.dim2 == 0 ? *(const pa_f32x4 *) (kr1 + min(d, A.dim1 - 4)) : *(const pa_f32x4 *) (kr2 + min(d, A.dim2 - 4));
+                }
             }
             auto values = [&]() {
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    const float * vr = vb + (int64_t) (cb + (here >> (4 * g + c) & 1u ? 4 * g + c : spare) - A.cell0) * A.v_row;
+                    const int cell = cb + (here >> (4 * g + c) & 1u ? 4 * g + c : spare) - A.cell0;
+                    if constexpr (N1 > 0) {
+                        const uint32_t o = ((uint32_t) cell * (uint32_t) A.v_row + (uint32_t) (NJ * n)) * 4u;
 #pragma unroll
-                    for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, A.vdim - 4));
+                        for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) ((const char *) vb + o + 16 * j);
+                    } else {
+                        const float * vr = vb + (int64_t) cell * A.v_row;
+#pragma unroll
+                        for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, A.vdim - 4));
+                    }
                 }
             };
             constexpr bool LATE = NK + 4 * NV > 16;                   // (the registers do not hold the keys and the values of a tile at a time)
             if constexpr (!LATE) values();
+            if constexpr (N1 > 0) __builtin_amdgcn_sched_barrier(0);  // (all of them on their way before the first product)
             pa_f32x4 s[2] = { pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }, pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f } };
 #pragma unroll
             for (int i = 0; i < NK; i++)
@@ -313,16 +328,21 @@ bool pa_takes(const pa_args & a, int maps, int min_tokens) {
     return a.n_tok >= min_tokens && pa_steps(a) <= 12 && a.vdim <= 128 && a.dim1 >= 4 && a.vdim >= 4 && four(a.dim1) && four(a.dim2) && four(a.vdim) && four(a.k1_row) && four(a.k1_head) && four(a.k2_row) && four(a.v_row) &&
            four(a.v_head) && ((uintptr_t) a.k1 & 15) == 0 && ((uintptr_t) a.k2 & 15) == 0 && ((uintptr_t) a.v & 15) == 0 && (maps == 1 || a.dim2 == 0);
 }
-template <int NK, int NV>
+template <int NK, int N1, int NV>
 static void pa_go(const pa_args & a, int maps, double bytes, hipStream_t s) {
     const dim3 grid((unsigned) a.heads, (unsigned) ((a.n_tok + 31) / 32));
     const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
-    if (maps == 2) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, NV, 2>), grid, dim3(256), 0, s, a, pi_abort_word());
-    else PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, NV, 1>), grid, dim3(256), 0, s, a, pi_abort_word());
+    if constexpr (N1 == 0 || N1 == NK)                                 // (two maps: no part that the heads share)
+        if (maps == 2) { PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, N1, NV, 2>), grid, dim3(256), 0, s, a, pi_abort_word()); return; }
+    PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_prompt_attention<NK, N1, NV, 1>), grid, dim3(256), 0, s, a, pi_abort_word());
 }
 void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s) {
-    const int nk = pa_steps(a);
-#define PA_NK(NV) do { if (nk <= 4) pa_go<4, NV>(a, maps, bytes, s); else if (nk <= 6) pa_go<6, NV>(a, maps, bytes, s); else if (nk <= 8) pa_go<8, NV>(a, maps, bytes, s); else pa_go<12, NV>(a, maps, bytes, s); } while (0)
+    const int nk = pa_steps(a), n1 = a.dim1 / 16;
+    const int64_t most = (int64_t) 1 << 30;                            // floats within 32-bit byte offsets
+    const bool whole = a.dim1 % 16 == 0 && a.dim2 % 16 == 0 && (a.vdim == 64 || a.vdim == 128) && (a.cell1 - a.cell0) * a.k1_row < most && (a.cell1 - a.cell0) * a.v_row < most && a.cell1 * a.k2_row < most;
+#define PA_NK(NV) do { if (whole && nk == 4 && n1 == 4) pa_go<4, 4, NV>(a, maps, bytes, s); else if (whole && nk == 8 && n1 == 8) pa_go<8, 8, NV>(a, maps, bytes, s); \
+                       else if (whole && nk == 6 && n1 == 4) pa_go<6, 4, NV>(a, maps, bytes, s); else if (whole && nk == 12 && n1 == 8) pa_go<12, 8, NV>(a, maps, bytes, s); \
+                       else if (nk <= 4) pa_go<4, 0, NV>(a, maps, bytes, s); else if (nk <= 8) pa_go<8, 0, NV>(a, maps, bytes, s); else pa_go<12, 0, NV>(a, maps, bytes, s); } while (0)
     if (a.vdim <= 64) PA_NK(1); else PA_NK(2);
 #undef PA_NK
 }

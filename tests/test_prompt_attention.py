@@ -7,7 +7,7 @@ from tests.test_letevik import HALVES, NEIGHBOURS, SIGMOID, O, diff_attention_re
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,D,R,V,rank,T,n_kv", [(3, 8, 4, 12, 24, 9, 33), (32, 8, 4, 12, 24, 33, 33), (32, 64, 0, 64, 72, 32, 300), (8, 128, 64, 128, 512, 130, 200), (11, 20, 36, 68, 136, 95, 161), (4, 64, 0, 64, 256, 300, 2500), (64, 4, 2, 4, 8, 70, 97)])
+@pytest.mark.parametrize("H,D,R,V,rank,T,n_kv", [(3, 8, 4, 12, 24, 9, 33), (32, 8, 4, 12, 24, 33, 33), (32, 64, 0, 64, 72, 32, 300), (8, 128, 64, 128, 512, 130, 200), (16, 64, 32, 64, 256, 50, 80), (11, 20, 36, 68, 136, 95, 161), (4, 64, 0, 64, 256, 300, 2500), (64, 4, 2, 4, 8, 70, 97)])
 def test_latent_prompt(H, D, R, V, rank, T, n_kv):
     """tiles that are not full (tokens, cells, key and output values), both pairings, every kind of gate, with and without a sink; the long one takes two launches over the cells (its scratch memory holds the
     keys and values of 1600)"""
