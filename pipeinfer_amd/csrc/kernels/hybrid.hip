@@ -957,6 +957,10 @@ static lat_plan latent_plan(int heads, int rank, int rot, int n_tok, int n_ctx) 
     return p;
 }
 
+// passes that take k_latent_rows: a few tokens (more of them: prompt_attention.hip), ranks of whole tiles
+static bool lat_rows_takes(int rank, int rot, int n_tok) { return n_tok <= 8 && (rank == 256 || rank == 512) && rot <= 64 && (rot & 3) == 0; }
+static size_t lat_rows_floats(int heads, int rank, int rot, int n_tok, int n_ctx) { return (size_t) n_tok * heads * ((size_t) (rank + rot) + (size_t) (n_ctx + 31) / 32 * (rank + 2)); }
+
 // grid (token tile of 4, head, 64 values of the rank, then 64 values of the rotated part): lane = one rank value, the four waves take a quarter of the head's dim each and meet in LDS.  A query head is
 // [dim values | rot values]; the last are turned in pairs by the token's position (cs: the rotation table) and go behind the rank values
 __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict__ q, int64_t qs, const uint16_t * __restrict__ wuk, float scale, int heads, int dim, int rank, int rot, const float2 * __restrict__ cs, int n_pos,
@@ -1156,18 +1160,122 @@ __global__ void __launch_bounds__(256) k_latent_scores(const float * __restrict_
     }
 }
 
+// The same for a few tokens on the fp32 matrix cores, sixteen rows (token, head) and a split of 32 cells per workgroup.  What bounds it: one trip to memory and back - every load of the workgroup goes out before the first
+// product.  With a lane per cell and a chain of loads each, 4 tokens x 16 heads over 700 cells of 512 + 64 took 20 us (now 11.5); 1 token x 16 heads of 256, 32 cells: 9.7 (6.4).
+// NJ: a wave sums 16 NJ of the rank's values (rank = 64 NJ); EX: steps of 16 values behind the rank.  Lane l holds, with n = l % 16 and g = l / 16, of the scores row n and the wave's cells 4 g + r, of the sums
+// row n and the values NJ (4 g + r) + j.  (Splits of 64 cells, every wave its sixteen over the whole width: 17 us.)
+template <int NJ, int EX>
+__global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int W, int n_rows, int n_kv_arg, int S,
+                                                        float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 5)) return;
+    constexpr int RANK = 64 * NJ, NS = RANK / 16 + EX, NH = NS / 2;
+    __shared__ __attribute__((aligned(16))) float ps[16][36], half[2][16][20];
+    __shared__ float top[2][16], sum[2][16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, split = blockIdx.y, c0 = split * 32, ct = wave & 1, wh = wave >> 1;
+    const int row = min((int) blockIdx.x * 16 + n, n_rows - 1), words = (n_kv_arg + 31) / 32, n_kv = min(dyn ? dyn[1] : n_kv_arg, n_kv_arg);
+    uint32_t vis = 0;
+    if (c0 < n_kv) {
+        vis = mask[(int64_t) (row / heads) * words + split];
+        if (n_kv - c0 < 32) vis &= (1u << (n_kv - c0)) - 1u;
+    }
+    uint32_t some = vis;                                              // the cells that any row sees; what the others hold is not read
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
+    float * pml_r = pml + ((int64_t) ((int) blockIdx.x * 16 + n) * S + split) * 2;
+    const bool real = (int) blockIdx.x * 16 + n < n_rows;
+    if (!some) {                                                      // (the same in every lane: the rows of a tile are the same sixteen in all four)
+        if (tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
+        return;
+    }
+    const int spare = __ffs(some) - 1;
+    auto cell = [&](int c) { return (uint32_t) (c0 + ((some >> c) & 1u ? c : spare)); };
+    hy_f32x4 kf[NH], qf[NH], vf[2][4][NJ / 4];
+    {   // a wave scores sixteen cells over half of the row's width
+        const uint32_t ko = cell(16 * ct + n) * (uint32_t) W, qo = (uint32_t) row * (uint32_t) W;
+#pragma unroll
+        for (int i = 0; i < NH; i++) {
+            const uint32_t d = 16u * (wh * NH + i) + 4u * g, at = EX == 0 ? d : min(d, (uint32_t) W - 4u);
+            kf[i] = *(const hy_f32x4 *) (cache + ko + at); qf[i] = *(const hy_f32x4 *) (qa + qo + at);
+            if (EX && d >= (uint32_t) W) qf[i] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+        }
+    }
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const uint32_t o = cell(16 * jt + 4 * g + c) * (uint32_t) W + (uint32_t) (wave * (RANK / 4) + NJ * n);
+#pragma unroll
+            for (int j = 0; j < NJ / 4; j++) vf[jt][c][j] = *(const hy_f32x4 *) (cache + o + 4 * j);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+    hy_f32x4 s0 = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+    for (int i = 0; i < NH; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) s0 = hy_mfma(kf[i][c], qf[i][c], s0);
+    if (wh) *(hy_f32x4 *) &half[ct][n][4 * g] = s0;
+    __syncthreads();
+    const uint32_t mine = vis >> (16 * ct + 4 * g);
+    float m = -INFINITY;
+    if (!wh) {
+        s0 += *(const hy_f32x4 *) &half[ct][n][4 * g];
+#pragma unroll
+        for (int r = 0; r < 4; r++) if (mine >> r & 1u) m = fmaxf(m, s0[r]);
+        m = fmaxf(m, __shfl_xor(m, 16, 64)); m = fmaxf(m, __shfl_xor(m, 32, 64));
+        if (g == 0) top[ct][n] = m;
+    }
+    __syncthreads();
+    m = fmaxf(top[0][n], top[1][n]);
+    if (!wh) {
+        float l = 0.0f;
+        hy_f32x4 p;
+#pragma unroll
+        for (int r = 0; r < 4; r++) { p[r] = mine >> r & 1u ? expf(s0[r] - m) : 0.0f; l += p[r]; }
+        l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+        if (g == 0) sum[ct][n] = l;
+        *(hy_f32x4 *) &ps[n][16 * ct + 4 * g] = p;
+    }
+    __syncthreads();
+    if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
+    hy_f32x4 acc[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+    for (int jt = 0; jt < 2; jt++) {
+        const hy_f32x4 w = *(const hy_f32x4 *) &ps[n][16 * jt + 4 * g];
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
+    }
+    if (!real || vis == 0) return;
+    float * o = pol + ((int64_t) row * S + split) * RANK + wave * (RANK / 4);
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int j = 0; j < NJ; j += 4) *(hy_f32x4 *) (o + NJ * (4 * g + r) + j) = hy_f32x4{ acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r] };
+}
+
 // grid (token tile of 4, head, 16 output values): merges the splits (with the sink if there is one), normalises, applies its rows of W_uv[h], then the gate if there is one: one value per head, or (gate_width = vdim)
 // one per output value
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
-                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, float * __restrict__ out, int64_t os,
+                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 5)) return;
-    extern __shared__ float ol[];                                     // [4][rank]
+    extern __shared__ __attribute__((aligned(16))) float ol[];                                     // [4][rank]
     __shared__ float wgt[4][64];                                      // per token: weight of the splits that hold something, 64 splits at a time,
     __shared__ int num[4][64], cnt[4];                                // their numbers, how many they are
     __shared__ float gsh[4];                                          // per token: the head's gate (one value per head)
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nt = min(4, n_tok - t0);
+    hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (vec: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
+    if (vec) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)) * rank + min(lane * 8, rank - 8));
+        if (gate && gate_width > 1)
+#pragma unroll
+            for (int k = 0; k < 4; k++) gv[k] = gate[(int64_t) (t0 + min(lane, nt - 1)) * gs + (int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)];
+    }
     for (int idx = tid; idx < 4 * rank; idx += 256) ol[idx] = 0.0f;
     if (tid < 4) {
         float g = 1.0f;
@@ -1196,6 +1304,24 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             if (lane == 0) cnt[wave] = __popcll(some);
         }
         __syncthreads();
+        if (vec) {                                                     // four values of the rank per thread, eight splits on their way at a time (one by one, every split was a trip to memory: 23 us for 11 of 4 tokens)
+            for (int idx = tid; idx < nt * (rank >> 2); idx += 256) {
+                const int tt = idx / (rank >> 2), r = idx % (rank >> 2) * 4, n = cnt[tt];
+                if (n == 0) continue;
+                const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + r;
+                float4 v = *(const float4 *) (ol + tt * rank + r);
+                for (int s0 = 0; s0 < n; s0 += 8) {
+                    float4 x[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) x[u] = *(const float4 *) (p + (int64_t) num[tt][min(s0 + u, n - 1)] * rank);
+#pragma unroll
+                    for (int u = 0; u < 8; u++)
+                        if (s0 + u < n) { const float w = wgt[tt][s0 + u]; v.x = fmaf(w, x[u].x, v.x); v.y = fmaf(w, x[u].y, v.y); v.z = fmaf(w, x[u].z, v.z); v.w = fmaf(w, x[u].w, v.w); }
+                }
+                *(float4 *) (ol + tt * rank + r) = v;
+            }
+            continue;
+        }
         for (int idx = tid; idx < nt * rank; idx += 256) {
             const int tt = idx / rank, r = idx % rank;
             const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + r;
@@ -1207,6 +1333,39 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         }
     }
     __syncthreads();
+    if (vec) {
+        const int v0 = blockIdx.z * 16 + wave;
+        float a[4][4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++) a[k][tt] = 0.0f;
+        for (int rb = 0; rb < rank; rb += 512) {
+            const int r = rb + lane * 8;
+            if (r >= rank) break;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const hy_u16x8v w = rb == 0 ? wrow[k] : *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min(v0 + 4 * k, vdim - 1)) * rank + r);
+#pragma unroll
+                for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+                    for (int i = 0; i < 8; i++) a[k][tt] = fmaf(hy_widen(w[i]), ol[tt * rank + r + i], a[k][tt]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int vv = v0 + 4 * k;
+            if (vv >= vdim) break;
+            float v = 0.0f;
+#pragma unroll
+            for (int tt = 0; tt < 4; tt++) { const float s = pi_lanes_sum<64>(a[k][tt]); if (lane == tt) v = s; }
+            if (lane >= nt) continue;
+            float g = gsh[lane];
+            if (gate && gate_width > 1) { g = gv[k]; if (gate_act == PI_ACT_SIGMOID) g = 1.0f / (1.0f + expf(-g)); }
+            out[(int64_t) (t0 + lane) * os + (int64_t) h * vdim + vv] = v * g;
+        }
+        return;
+    }
     for (int vv = blockIdx.z * 16 + wave; vv < min(vdim, (int) blockIdx.z * 16 + 16); vv += 4) {
         const uint16_t * wv = wuv + ((int64_t) h * vdim + vv) * rank;
         float a[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
@@ -1233,7 +1392,8 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
 extern "C" int pi_op_latent_attention_max_cells(int rank) { (void) rank; return 1 << 22; }       // (long contexts are cut into splits: no score row has to fit LDS whole)
 extern "C" size_t pi_op_latent_attention_scratch_floats(int heads, int rank, int n_tok, int n_ctx) { return pi_op_latent_attention_rot_scratch_floats(heads, rank, 0, n_tok, n_ctx); }
 extern "C" size_t pi_op_latent_attention_rot_scratch_floats(int heads, int rank, int rot_dim, int n_tok, int n_ctx) {
-    return std::max(latent_plan(heads, rank, rot_dim, n_tok, n_ctx).scratch, latent_plan(heads, rank, rot_dim, std::min(n_tok, 8), n_ctx).scratch);
+    const int few = std::min(n_tok, 8);
+    return std::max(std::max(latent_plan(heads, rank, rot_dim, n_tok, n_ctx).scratch, latent_plan(heads, rank, rot_dim, few, n_ctx).scratch), lat_rows_takes(rank, rot_dim, few) ? lat_rows_floats(heads, rank, rot_dim, few, n_ctx) : 0);
 }
 template <int M, int RPT> static int latent_reserve_one() {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_latent_scores<M, RPT>, hipFuncAttributeMaxDynamicSharedMemorySize, LAT_LDS_BUDGET + 4096));
@@ -1304,7 +1464,7 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
         pi_set_error("pi_op_latent_attention: the up-projections must be bfloat16 [heads * dim][rank] and [heads * vdim][rank]"); return -1;
     }
     if (rank > 1024) { pi_set_error("pi_op_latent_attention: latent width %d above 1024", rank); return -1; }
-    const lat_plan p = latent_plan(heads, rank, rot, n_tok, n_kv);
+    lat_plan p = latent_plan(heads, rank, rot, n_tok, n_kv);
     if (p.scratch > scratch_floats) { pi_set_error("pi_op_latent_attention: %zu floats of scratch needed, %zu given", p.scratch, scratch_floats); return -1; }
     if (p.lds > LAT_LDS_BUDGET + 4096 || (size_t) 4 * rank * 4 > 64 * 1024) { pi_set_error("pi_op_latent_attention: LDS plan does not fit"); return -1; }
     if (pi_op_latent_attention_reserve() != 0) return -1;
@@ -1322,14 +1482,27 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     PI_CHECK_LAUNCH();
     const dim3 grid((unsigned) n_tok, (unsigned) ((heads + p.M - 1) / p.M), (unsigned) p.S);
     const double bytes = 4.0 * acct * (rank + rot) + 4.0 * n_tok * heads * (rank + rot + (double) rank * p.S);
+    // few tokens, sizes of whole steps: the matrix cores (more scratch memory than the other kernel's: its size is pi_op_latent_attention_rot_scratch_floats')
+    const int S32 = (n_kv + 31) / 32;
+    const bool whole = lat_rows_takes(rank, rot, n_tok) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats && (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
+    if (whole) {
+        p.S = S32;
+        pml = pol + (size_t) n_tok * heads * p.S * rank;
+        const dim3 rgrid((unsigned) ((n_tok * heads + 15) / 16), (unsigned) p.S);
+#define LAT_ROWS(NJ, EX) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_rows<NJ, EX>), rgrid, dim3(256), 0, s, qa, cache, mask, heads, rank + rot, n_tok * heads, n_kv, p.S, pol, pml, dyn_dev, pi_abort_word())
+        if (rank == 256) { if (rot) LAT_ROWS(4, 4); else LAT_ROWS(4, 0); } else { if (rot) LAT_ROWS(8, 4); else LAT_ROWS(8, 0); }
+#undef LAT_ROWS
+    } else {
 #define LAT_GO(M) do { if (p.RPT == 1) latent_scores_launch<M, 1>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); \
                        else if (p.RPT == 2) latent_scores_launch<M, 2>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); \
                        else latent_scores_launch<M, 4>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); } while (0)
     switch (p.M) { case 16: LAT_GO(16); break; case 8: LAT_GO(8); break; case 4: LAT_GO(4); break; case 2: LAT_GO(2); break; default: LAT_GO(1); }
 #undef LAT_GO
+    }
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), dim3(256), (size_t) 16 * rank, s,
-                 pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok, out, out_stride, pi_abort_word());
+                 pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok,
+                 (int) ((rank & 7) == 0 && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0), out, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 

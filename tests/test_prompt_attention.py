@@ -1,8 +1,9 @@
-"""Passes of many tokens (prompt_attention.hip): 32 tokens of a head at a time, keys and values of a latent written out first.  Against the explicit fp64 sums that the per-token kernels are tested with."""
+"""Attention on the matrix cores.  Passes of many tokens (prompt_attention.hip): 32 tokens of a head at a time, keys and values of a latent written out first; few tokens over a latent (hybrid.hip).  Against the explicit fp64 sums that the per-token kernels are tested with."""
 import numpy as np
 import pytest
 
 from pipeinfer_amd import lib as L
+from tests import test_fasovik as fasovik
 from tests.test_letevik import HALVES, NEIGHBOURS, SIGMOID, O, diff_attention_ref, gpu, latent_case, pack_mask, rel_rms, run_diff
 
 
@@ -17,6 +18,26 @@ def test_latent_prompt(H, D, R, V, rank, T, n_kv):
     for pairing, width, sink in ((HALVES, V, True), (NEIGHBOURS, 1, False)) if n_kv > 1000 else ((HALVES, V, True), (NEIGHBOURS, V, False), (HALVES, 1, True), (HALVES, 0, False)):
         got, want = latent_case(U, lib, rng, H, D, R, V, rank, n_kv, pos, 500.0, pairing, width, rng.standard_normal(H) * 2 if sink else None, (D + R) ** -0.5)
         assert rel_rms(got, want) < 1e-5, (pairing, width, sink)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,D,R,V,rank", [(16, 8, 64, 24, 512), (5, 20, 36, 17, 512), (3, 8, 0, 33, 256), (7, 4, 4, 8, 256)])
+@pytest.mark.parametrize("T,n_kv", [(1, 33), (1, 700), (4, 64), (8, 130), (3, 4200)])
+def test_latent_few_tokens(H, D, R, V, rank, T, n_kv):
+    """sixteen rows (token, head) at a time over splits of 64 cells: rows and splits that are not full, more than 64 splits, a rotated part that ends inside a step"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H * 100 + n_kv)
+    pos = np.arange(n_kv - T, n_kv)
+    for pairing, width, sink in ((HALVES, V, True), (NEIGHBOURS, 1, False)):
+        got, want = latent_case(U, lib, rng, H, D, R, V, rank, n_kv, pos, 500.0, pairing, width, rng.standard_normal(H) * 2 if sink else None, (D + R) ** -0.5)
+        assert rel_rms(got, want) < 1e-5, (pairing, width, sink)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,rank,T,n_kv", [(6, 256, 5, 700), (16, 512, 4, 200), (1, 256, 1, 64), (5, 512, 8, 100)])
+def test_latent_few_tokens_over_scattered_cells(H, rank, T, n_kv):
+    """what a token sees is any set of cells; what lies behind the cells in use is no number"""
+    fasovik.test_latent_attention_against_explicit_keys_and_values(H, 16, 24, rank, T, n_kv)
 
 
 def scattered(rng, T, n_kv, n_ctx):
