@@ -34,9 +34,10 @@ static __device__ __forceinline__ float cm_block_sum(float v, float * red) {    
 // ---- embedding: token row * scale + a row of a second table ---------------------------------------------------------------------------------------------
 __global__ void k_embed_pair(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, const uint16_t * __restrict__ table2, int64_t n_rows2,
                              const int32_t * __restrict__ rows2, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x;
     const int64_t row = tokens[t], row2 = rows2[t];
+    if (pi_abort_late(gone, abort_w)) return;
     const bool ok = row >= 0 && row < n_rows, ok2 = row2 >= 0 && row2 < n_rows2;
     for (int64_t i = threadIdx.x; i < width; i += blockDim.x)
         out[(int64_t) t * width + i] = (ok ? cm_widen(table[row * width + i]) * scale : 0.0f) + (ok2 ? cm_widen(table2[row2 * width + i]) : 0.0f);
@@ -57,7 +58,7 @@ template <int NPT, bool PRE>
 __global__ void __launch_bounds__(256) k_rms_post(const float * __restrict__ a, int64_t as, const float * __restrict__ wa, const float * __restrict__ b, int64_t bs, const float * __restrict__ wb, float mb,
                                                   const float * __restrict__ ls, const float * __restrict__ x, int64_t xs, float alpha, const float * __restrict__ w, float eps, int n,
                                                   float * __restrict__ out, int64_t os, const float * __restrict__ w_next, float * __restrict__ out_next, int64_t ons, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x;
     float m[NPT], v[NPT];
@@ -90,6 +91,7 @@ __global__ void __launch_bounds__(256) k_rms_post(const float * __restrict__ a, 
     }
     ss = cm_block_sum(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float) n + eps);
+    if (pi_abort_late(gone, abort_w)) return;
     float s2 = 0.0f;
 #pragma unroll
     for (int j = 0; j < NPT; j++) { const int i = j * 256 + tid; if (i < n) { v[j] = v[j] * inv * (PRE ? pw[j] : w[i]); out[(int64_t) t * os + i] = v[j]; s2 = fmaf(v[j], v[j], s2); } }
@@ -139,10 +141,11 @@ __global__ void __launch_bounds__(256) k_token_shift_state(const float * __restr
 // short passes in ONE launch: the thread of a run's first token walks the run for its value and leaves the state, so nothing it writes is read by another thread
 __global__ void __launch_bounds__(256) k_token_shift_walk(const float * __restrict__ h, int64_t hs, int n, const float * __restrict__ mu, int n_mix, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok,
                                                           float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, i = blockIdx.y * 256 + threadIdx.x;
     const int word = rec[t], slot = word & ~CM_FRESH;
     if (i >= n || (t > 0 && (rec[t - 1] & ~CM_FRESH) == slot)) return;
+    if (pi_abort_late(gone, abort_w)) return;                          // (behind the slot words)
     float prev = (word & CM_FRESH) ? 0.0f : state[(int64_t) slot * n + i];
     for (int tt = t; tt < n_tok && (rec[tt] & ~CM_FRESH) == slot; tt++) {
         const float cur = h[(int64_t) tt * hs + i], d = prev - cur;
@@ -209,7 +212,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
                                                             const float * __restrict__ braw, int64_t bs, const float * __restrict__ bonus, int qk_unit, float q_mult,
                                                             int heads, int hpg, int dim, int vdim, int R, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, int mode, int tb, int piece,
                                                             float * __restrict__ scratch, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ float lds[];                // q [CR_TB][dp] | k [CR_TB][dp] | g [CR_TB][dp] | v [CR_TB][cols];  a row is R parts of DPT values, DPT + 4 floats apart (the parts of one wave-wide read then fall into different banks), dp = R * (DPT + 4); rows end in zeros so that the token loop needs no bounds
     __shared__ int seg[4], bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;      // seg: first token, length, slot word of this workgroup's piece, whether it is its run's last
     __shared__ float beta_t[CR_TB], dot_t[CR_TB];
@@ -233,6 +236,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
     __syncthreads();
     const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
+    if (pi_abort_late(gone, abort_w)) return;
     if (len == 0 || word < 0 || (mode == 1 && last)) return;
     const int slot = word & ~CM_FRESH;
     const int cols = blockDim.x / R;
@@ -872,10 +876,33 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
 // out[t][h][i] = y[t][h][i] / sqrt(mean_i(y[t][h]^2) + eps) * w[(w_per_head ? h * n : 0) + i] * act(gate[t][h][i]);  a wave per (token, head); out may be y
 __global__ void __launch_bounds__(256) k_head_norm_gate(const float * __restrict__ y, int64_t ys, int heads, int n, const float * __restrict__ w, int w_per_head, const float * __restrict__ gate, int64_t gs, int gate_act,
                                                         float eps, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (h >= heads) return;
     const float * yr = y + (int64_t) t * ys + (int64_t) h * n;
+    if (n <= 128) {                                                   // (two values a lane: what the row needs is on its way before its sum)
+        float yv[2], wv[2], gv[2], ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int i = min(lane + 64 * j, n - 1);
+            yv[j] = yr[i]; wv[j] = w[(w_per_head ? h * n : 0) + i]; gv[j] = gate ? gate[(int64_t) t * gs + (int64_t) h * n + i] : 1.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) if (lane + 64 * j < n) ss = fmaf(yv[j], yv[j], ss);
+        const float inv = 1.0f / sqrtf(pi_lanes_sum<64>(ss) / (float) n + eps);
+        if (pi_abort_late(gone, abort_w)) return;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int i = lane + 64 * j;
+            if (i >= n) break;
+            float g = gv[j];
+            if (gate && gate_act == PI_ACT_SIGMOID) g = cm_sigmoid(g);
+            else if (gate && gate_act == PI_ACT_SILU) g = g / (1.0f + expf(-g));
+            out[(int64_t) t * os + (int64_t) h * n + i] = yv[j] * inv * wv[j] * g;
+        }
+        return;
+    }
+    if (pi_abort_late(gone, abort_w)) return;
     float ss = 0.0f;
     for (int i = lane; i < n; i += 64) ss = fmaf(yr[i], yr[i], ss);
     const float inv = 1.0f / sqrtf(pi_lanes_sum<64>(ss) / (float) n + eps);

@@ -173,13 +173,14 @@ static __device__ __forceinline__ void wave_emit_frags(const q8k_frags & F, cons
 }
 
 __global__ void __launch_bounds__(64) k_quantize_q8_K(const float * __restrict__ x, int64_t k, int8_t * __restrict__ qs, float * __restrict__ dd, int16_t * __restrict__ bsums, const q8k_frags F, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 3)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.y, blk = blockIdx.x, lane = threadIdx.x;
     const int64_t nb = k >> 8;
     const float4 v = *(const float4 *) (x + (int64_t) t * k + (int64_t) blk * 256 + lane * 4);
     const float xs[4] = { v.x, v.y, v.z, v.w };
     int q[4], s;
     const float d = pi_wave_q8K(xs, lane, q, s);
+    if (pi_abort_late(gone, abort_w, 3)) return;
     pi_wave_q8K_store(q, s, d, lane, (int64_t) t * nb + blk, qs, dd, bsums);
     wave_emit_frags(F, q, s, d, lane, t, blk, nb);
 }
@@ -194,7 +195,7 @@ static __device__ __forceinline__ void q8_0_store_scale(const int q[4], float d,
 
 // one wave = 8 blocks of 32 = two groups of 4 blocks; values past k belong to the zero padding of the last group
 __global__ void __launch_bounds__(64) k_quantize_q8_0(const float * __restrict__ x, int64_t k, int64_t ng, uint32_t * __restrict__ qs, uint16_t * __restrict__ dd, float * __restrict__ ss, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 3)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.y, lane = threadIdx.x;
     const int64_t e0 = (int64_t) blockIdx.x * 256 + lane * 4;
     if (e0 >= ng * 128) return;
@@ -208,6 +209,7 @@ __global__ void __launch_bounds__(64) k_quantize_q8_0(const float * __restrict__
 #pragma unroll
     for (int i = 0; i < 4; i++) { int r = __float2int_rn(xs[i] * id); q[i] = r > 127 ? 127 : (r < -128 ? -128 : r); }
     const int64_t blk = e0 >> 5, grp = (int64_t) t * ng + (blk >> 2); const int bi = (int) (blk & 3), kk = lane & 7;
+    if (pi_abort_late(gone, abort_w, 3)) return;
     qs[(grp * 8 + kk) * 4 + bi] = (uint32_t) (q[0] & 0xff) | (uint32_t) (q[1] & 0xff) << 8 | (uint32_t) (q[2] & 0xff) << 16 | (uint32_t) (q[3] & 0xff) << 24;
     q8_0_store_scale(q, d, kk, grp, bi, dd, ss);
 }
@@ -438,7 +440,7 @@ extern "C" int pi_op_norm_quantize(const float * x, const float * w, const float
 // act(gate) [* up] straight into the quantised activation planes: which = 0 silu(gate)*up, 1 gelu(gate).  One wave per 256 values.
 __global__ void __launch_bounds__(256) k_act_quant(const float * __restrict__ g, const float * __restrict__ u, int which, int64_t n, int vdt, int64_t ng,
                                                     const uint16_t * __restrict__ tab, uint8_t * __restrict__ qs, uint8_t * __restrict__ dd, int16_t * __restrict__ bsums, const q8k_frags F, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 4)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t c0 = ((int64_t) blockIdx.x * 4 + wave) * 256, e0 = c0 + lane * 4;
     const int64_t n_pad = vdt == PI_Q8_K ? n : ng * 128;
@@ -455,6 +457,7 @@ __global__ void __launch_bounds__(256) k_act_quant(const float * __restrict__ g,
             else { const float a = pi_h2f(tab[pi_f2h(gs[i])]); ys[i] = which == 0 ? a * us[i] : a; }
         }
     }
+    if (pi_abort_late(gone, abort_w, 4)) return;
     if (vdt == PI_Q8_K) wave_quantize_q8_K(ys, lane, t, c0 >> 8, n >> 8, (int8_t *) qs, (float *) dd, bsums, F);
     else if (e0 < n_pad) wave_quantize_q8_0(ys, lane, (int64_t) t * ng, e0, (uint32_t *) qs, (uint16_t *) dd, vdt == PI_Q8_1 ? (float *) bsums : nullptr);
 }
@@ -701,7 +704,7 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
 }
 template <int VPT>
 __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, lane = threadIdx.x & 63, ch = blockIdx.y * 4 + (threadIdx.x >> 6);
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per);
     const float * l = logits + (int64_t) t * n_vocab;
@@ -724,10 +727,12 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     } else for (int i = lo + lane, w = 0; i < hi; i += 64, w = (w + 1) & 3) { const float e = expf(l[i] - first); s[0] += w == 0 ? e : 0.0f; s[1] += w == 1 ? e : 0.0f; s[2] += w == 2 ? e : 0.0f; s[3] += w == 3 ? e : 0.0f; }
 #pragma unroll
     for (int w = 0; w < 4; w++) s[w] = pi_lanes_sum<64>(s[w]);
+    if (pi_abort_late(gone, abort_w)) return;
     if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
     const int64_t out = ((int64_t) t * TOPK_NCH + ch) * k;
+    int own = 0x7fffffff;                                             // lane r keeps the r-th: their values are read back together, not one by one between the rounds
     for (int r = 0; ; r++) {
-        if (lane == 0) { cid[out + r] = wi; cval[out + r] = wk ? l[wi] : -INFINITY; }
+        if (lane == r) own = wi;
         if (r + 1 >= k) break;
         if (wk != 0 && wi == lo + lane + 64 * bm) {                     // its owner looks for its next one
             bk = 0;
@@ -745,16 +750,18 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         wk = bk; wi = bk ? lo + lane + 64 * bm : 0x7fffffff;
         topk_best(wk, wi);
     }
+    if (lane < k) { cid[out + lane] = own; cval[out + lane] = own != 0x7fffffff ? l[own] : -INFINITY; }
 }
 __global__ void __launch_bounds__(64) k_topk2(int k, const int32_t * __restrict__ cid, const float * __restrict__ cval, const float * __restrict__ cmax, const float * __restrict__ csum,
                                                int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, lane = threadIdx.x;
     const int n = TOPK_NCH * k;                                        // <= 256: four candidates per lane
     float cv[4]; int ci[4]; uint32_t key[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) { const int i = lane + 64 * j; cv[j] = i < n ? cval[(int64_t) t * n + i] : -INFINITY; ci[j] = i < n ? cid[(int64_t) t * n + i] : 0x7fffffff; key[j] = ci[j] != 0x7fffffff ? topk_key(cv[j]) : 0u; }
     const float pm = lane < TOPK_NCH ? cmax[t * TOPK_NCH + lane] : -INFINITY, ps = lane < TOPK_NCH ? csum[t * TOPK_NCH + lane] : 0.0f;
+    if (pi_abort_late(gone, abort_w)) return;
     for (int r = 0; r < k; r++) {
         uint32_t bk = 0; int bi = 0x7fffffff; float bv = -INFINITY;     // this lane's best
 #pragma unroll

@@ -62,6 +62,40 @@ static __device__ __forceinline__ float hy_block_max(float v, float * red) {
 }
 
 // ---- RMS norm with its usual companions ---------------------------------------------------------------------------------------------------------
+// rows of up to 1024 NV aligned values: everything the row needs is on its way before its sum (a row that was read again behind the sum: one more trip to memory, 3.4 us a launch instead of 3.1)
+template <int NV>
+__global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n, const float * __restrict__ gate, int64_t gs,
+                                                        const float * __restrict__ res, int64_t rs, float mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    __shared__ float red[4];
+    const int t = blockIdx.x;
+    const int64_t orow = to_cells ? pi_cell_of(dyn, 0, t) : t;
+    float4 xv[NV], wv[NV], gv[NV], rv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = min((int) threadIdx.x * 4 + 1024 * j, n - 4);
+        xv[j] = *(const float4 *) (x + (int64_t) t * xs + i); wv[j] = *(const float4 *) (w + i);
+        if (gate) gv[j] = *(const float4 *) (gate + (int64_t) t * gs + i);
+        if (res) rv[j] = *(const float4 *) (res + (int64_t) t * rs + i);
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) if ((int) threadIdx.x * 4 + 1024 * j < n) { ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss); ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss); }
+    ss = hy_block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float) n + eps);
+    if (pi_abort_late(gone, abort_w)) return;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = (int) threadIdx.x * 4 + 1024 * j;
+        if (i >= n) break;
+        float y[4] = { xv[j].x * inv * (wv[j].x + w_off), xv[j].y * inv * (wv[j].y + w_off), xv[j].z * inv * (wv[j].z + w_off), xv[j].w * inv * (wv[j].w + w_off) };
+        if (gate) { y[0] *= gv[j].x; y[1] *= gv[j].y; y[2] *= gv[j].z; y[3] *= gv[j].w; }
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] *= mult;
+        if (res) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
+        *(float4 *) (out + orow * os + i) = make_float4(y[0], y[1], y[2], y[3]);
+    }
+}
 __global__ void __launch_bounds__(256) k_rms_scale(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n,
                                                    const float * __restrict__ gate, int64_t gs, const float * __restrict__ res, int64_t rs, float mult,
                                                    float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, int vec, const int32_t * __restrict__ abort_w) {
@@ -102,6 +136,12 @@ extern "C" int pi_op_rms_scale(const float * x, int64_t x_stride, const float * 
     if (to_cells && !dyn_dev) { pi_set_error("pi_op_rms_scale: rows go to cache cells but no cell table was given"); return -1; }
     auto al = [](const void * p, int64_t stride) { return !p || (((uintptr_t) p % 16) == 0 && stride % 4 == 0); };
     const int vec = n % 4 == 0 && al(x, x_stride) && al(w, 0) && al(gate, gate_stride) && al(residual, residual_stride) && al(out, out_stride);
+#define RS_GO(NV) do { PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale_once<NV>, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride, residual, \
+                                    residual_stride, mult, out, out_stride, dyn_dev, to_cells, pi_abort_word()); PI_CHECK_LAUNCH(); return 0; } while (0)
+    if (vec && n <= 1024) RS_GO(1);
+    if (vec && n <= 2048) RS_GO(2);
+    if (vec && n <= 4096) RS_GO(4);
+#undef RS_GO
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride,
                  residual, residual_stride, mult, out, out_stride, dyn_dev, to_cells, vec, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
@@ -335,9 +375,11 @@ extern "C" int pi_op_softcap(float * x, int64_t n, float cap, void * stream) {
 
 // out[t][f] = in[t][f] * in[t][ff + f]  (a gated feed-forward whose gate and up rows are one matrix; the gate's activation ran in the projection's epilogue)
 __global__ void k_glu_mul(const float * __restrict__ in, int64_t is, int ff, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
-    const int t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
-    if (f < ff) out[(int64_t) t * os + f] = in[(int64_t) t * is + f] * in[(int64_t) t * is + ff + f];
+    const int gone = pi_abort_peek(abort_w), t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
+    if (f >= ff) return;
+    const float y = in[(int64_t) t * is + f] * in[(int64_t) t * is + ff + f];
+    if (pi_abort_late(gone, abort_w)) return;
+    out[(int64_t) t * os + f] = y;
 }
 extern "C" int pi_op_glu_mul(const float * in, int64_t in_stride, int ff, int n_tok, float * out, int64_t out_stride, void * stream) {
     if (n_tok <= 0 || ff <= 0) return 0;
@@ -354,12 +396,12 @@ static __device__ __forceinline__ float hy_glu(float g, float u, int glu, float 
     return glu == PI_GLU_SILU ? g / (1.0f + expf(-g)) * u : g * u;
 }
 __global__ void k_glu_mul_ex(const float * __restrict__ in, int64_t is, int ff, int glu, float limit, int64_t gate_col, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
-    const int t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
+    const int gone = pi_abort_peek(abort_w), t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
     if (f >= ff) return;
     const float * r = in + (int64_t) t * is;
     float y = hy_glu(r[f], r[ff + f], glu, limit);
     if (gate_col >= 0) y *= 1.0f / (1.0f + expf(-r[gate_col]));
+    if (pi_abort_late(gone, abort_w)) return;
     out[(int64_t) t * os + f] = y;
 }
 extern "C" int pi_op_glu_mul_ex(const float * in, int64_t in_stride, int ff, int glu, float limit, int64_t gate_col, int n_tok, float * out, int64_t out_stride, void * stream) {
@@ -491,12 +533,14 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
                                                           const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
                                                           float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, int mode, float * __restrict__ scratch,
                                                           float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ float lds[];                // q tile [LA_TB][dim] | k tile [LA_TB][dim] | v tile [LA_TB][cols] | the slot words of the pass [n_tok]
     __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd; // seg: first token, length, slot word, last piece of its run
     __shared__ float lam_t[LA_TB], sc_t[LA_TB];   // per token of the tile: decay and the factor on k v^T
     const int h = blockIdx.x, tid = threadIdx.x;
     int * recs = (int *) (lds + 2 * LA_TB * dim + LA_TB * (blockDim.x / R));
+    if (n_tok == 1) { if (tid == 0) { seg[0] = 0; seg[1] = blockIdx.z == 0; seg[2] = rec[0]; seg[3] = 1; } }      // (a single token is its own run: no search)
+    else {
     for (int t = tid; t < n_tok; t += blockDim.x) recs[t] = rec[t];
     __syncthreads();
     const int n_runs = la_runs(recs, n_tok, bnd, &nbnd);
@@ -505,8 +549,10 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
         if (!la_find_piece(recs, n_tok, bnd, n_runs, mode ? LA_TB : 0, blockIdx.z, first, len, word, last)) len = 0;
         seg[0] = first; seg[1] = len; seg[2] = word; seg[3] = last;
     }
+    }
     __syncthreads();
     const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
+    if (pi_abort_late(gone, abort_w)) return;
     if (len == 0 || word < 0 || (mode == 1 && last)) return;
     const int slot = word & ~LA_FRESH;
     const int cols = blockDim.x / R;
@@ -965,7 +1011,7 @@ static size_t lat_rows_floats(int heads, int rank, int rot, int n_tok, int n_ctx
 // [dim values | rot values]; the last are turned in pairs by the token's position (cs: the rotation table) and go behind the rank values
 __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict__ q, int64_t qs, const uint16_t * __restrict__ wuk, float scale, int heads, int dim, int rank, int rot, const float2 * __restrict__ cs, int n_pos,
                                                        int pairing, const int32_t * __restrict__ pos, int n_tok, float * __restrict__ qa, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 5)) return;
+    const int gone = pi_abort_peek(abort_w);
     __shared__ float part[4][4][64];
     extern __shared__ float4 qsh[];                                    // [dim]: the head's query values of the four tokens, side by side
     const int t0 = blockIdx.x * 4, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.z * 64 + lane;
@@ -977,6 +1023,7 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
         const pi_turn u = pi_turn_of(d, rot / 2, pairing);
         const float2 c = cs[(int64_t) min(pos[t], n_pos - 1) * (rot / 2) + u.angle];
         const float own = qr[d], other = qr[u.mate];
+        if (pi_abort_late(gone, abort_w, 5)) return;
         qa[((int64_t) t * heads + h) * (rank + rot) + rank + d] = (u.lead ? own * c.x - other * c.y : own * c.x + other * c.y) * scale;
         return;
     }
@@ -998,6 +1045,7 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
     for (int tt = 0; tt < 4; tt++) part[wave][tt][lane] = acc[tt];
     __syncthreads();
     const int tt = wave;                                              // wave tt writes token t0 + tt
+    if (pi_abort_late(gone, abort_w, 5)) return;
     if (t0 + tt < n_tok && r < rank) qa[((int64_t) (t0 + tt) * heads + h) * (rank + rot) + r] = (part[0][tt][lane] + part[1][tt][lane] + part[2][tt][lane] + part[3][tt][lane]) * scale;
 }
 
@@ -1167,7 +1215,7 @@ __global__ void __launch_bounds__(256) k_latent_scores(const float * __restrict_
 template <int NJ, int EX>
 __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int W, int n_rows, int n_kv_arg, int S,
                                                         float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 5)) return;
+    const int gone = pi_abort_peek(abort_w);
     constexpr int RANK = 64 * NJ, NS = RANK / 16 + EX, NH = NS / 2;
     __shared__ __attribute__((aligned(16))) float ps[16][36], half[2][16][20];
     __shared__ float top[2][16], sum[2][16];
@@ -1184,7 +1232,7 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
     float * pml_r = pml + ((int64_t) ((int) blockIdx.x * 16 + n) * S + split) * 2;
     const bool real = (int) blockIdx.x * 16 + n < n_rows;
     if (!some) {                                                      // (the same in every lane: the rows of a tile are the same sixteen in all four)
-        if (tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
+        if (!pi_abort_late(gone, abort_w, 5) && tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
         return;
     }
     const int spare = __ffs(some) - 1;
@@ -1236,6 +1284,7 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
         *(hy_f32x4 *) &ps[n][16 * ct + 4 * g] = p;
     }
     __syncthreads();
+    if (pi_abort_late(gone, abort_w, 5)) return;
     if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
     hy_f32x4 acc[NJ];
 #pragma unroll
@@ -1261,7 +1310,7 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
                                                         const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 5)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ __attribute__((aligned(16))) float ol[];                                     // [4][rank]
     __shared__ float wgt[4][64];                                      // per token: weight of the splits that hold something, 64 splits at a time,
     __shared__ int num[4][64], cnt[4];                                // their numbers, how many they are
@@ -1333,6 +1382,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         }
     }
     __syncthreads();
+    if (pi_abort_late(gone, abort_w, 5)) return;
     if (vec) {
         const int v0 = blockIdx.z * 16 + wave;
         float a[4][4];
@@ -1507,22 +1557,22 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
 }
 
 // ---- routed feed-forward ------------------------------------------------------------------------------------------------------------------------------
-// one workgroup per token: logits of all router outputs (a wave per output), soft-max, choice = score + correction, `top` rounds of arg-max (lowest index wins a tie)
+// one workgroup per token: logits of all router outputs (a wave per output; few tokens: up to sixteen waves, so that ten outputs are one trip to memory: 7.2 us on four, 5.4 so), soft-max, choice = score + correction, `top` rounds of arg-max (lowest index wins a tie)
 // n_groups > 0: the scores are sigmoid(logit), consecutive outputs are bundled into n_groups groups of equal size, a group is ranked by top1 + top2 of its members' scores, and the
 // choice is restricted to members of the `keep` highest-ranked groups (then by their own score; lowest index wins a tie, among groups as among outputs)
-__global__ void __launch_bounds__(256) k_moe_route(const uint16_t * __restrict__ router, int64_t width, int n_out, const float * __restrict__ corr, const float * __restrict__ x, int64_t xs,
+__global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict__ router, int64_t width, int n_out, const float * __restrict__ corr, const float * __restrict__ x, int64_t xs,
                                                    int top, int exact, int vec, int n_groups, int keep, int32_t * __restrict__ sel, float * __restrict__ selw, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ float z[];                  // [n_out] logits -> scores | [n_out] choice | [n_groups] group scores
     float * ch = z + n_out, * gsc = ch + n_out;
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const float * xr = x + (int64_t) t * xs;
-    for (int e = wave; e < n_out; e += 4) {
+    for (int e = wave; e < n_out; e += (int) (blockDim.x >> 6)) {
         const float a = pi_lanes_sum<64>(hy_dot_lane(router + (int64_t) e * width, xr, width, lane, exact != 0, vec != 0));
         if (lane == 0) z[e] = a;
     }
     __syncthreads();
-    if (wave != 0) return;
+    if (wave != 0 || pi_abort_late(gone, abort_w)) return;
     if (n_groups < 0) {                           // by logit (+ bias); the weights are worked out over the chosen ones below
         for (int e = lane; e < n_out; e += 64) { z[e] += corr ? corr[e] : 0.0f; ch[e] = z[e]; }
     } else if (n_groups > 0) {
@@ -1576,7 +1626,7 @@ __global__ void __launch_bounds__(256) k_moe_route(const uint16_t * __restrict__
 // glu: an expert's first matrix holds 2 * ff rows [gate | up] and up[t][kk][f] = silu(gate_f . x) * (up_f . x)
 __global__ void __launch_bounds__(256) k_moe_up(const uint16_t * __restrict__ wup, int64_t width, int ff, int n_exp, const float * __restrict__ x, int64_t xs, const int32_t * __restrict__ sel,
                                                 int top, int exact, int vec, int glu, float limit, float * __restrict__ up, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 0)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int lane = threadIdx.x & 63, f = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int slot = blockIdx.y, e = sel[slot];
     if (f >= ff || e >= n_exp) return;
@@ -1585,17 +1635,17 @@ __global__ void __launch_bounds__(256) k_moe_up(const uint16_t * __restrict__ wu
     if (glu) {
         const float g = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * 2 * ff + f) * width, xr, width, lane, exact != 0, vec != 0));
         const float u = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * 2 * ff + ff + f) * width, xr, width, lane, exact != 0, vec != 0));
-        if (lane == 0) up[(int64_t) slot * ff + f] = hy_glu(g, u, glu, limit);
+        if (!pi_abort_late(gone, abort_w, 0) && lane == 0) up[(int64_t) slot * ff + f] = hy_glu(g, u, glu, limit);
         return;
     }
     const float a = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * ff + f) * width, xr, width, lane, exact != 0, vec != 0));
-    if (lane == 0) { const float r = fmaxf(a, 0.0f); up[(int64_t) slot * ff + f] = r * r; }
+    if (!pi_abort_late(gone, abort_w, 0) && lane == 0) { const float r = fmaxf(a, 0.0f); up[(int64_t) slot * ff + f] = r * r; }
 }
 // out[t][n] = sum_kk w_kk * (identity ? x[t][n] : W_down[e_kk][n] . up[t][kk]); a wave per output n
 __global__ void __launch_bounds__(256) k_moe_down(const uint16_t * __restrict__ wdown, int64_t width, int ff, int n_exp, int top, const float * __restrict__ x, int64_t xs,
                                                   const int32_t * __restrict__ sel, const float * __restrict__ selw, const float * __restrict__ up, int exact, int vec, float * __restrict__ out, int64_t os,
                                                   const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 0)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int lane = threadIdx.x & 63;
     const int64_t n = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
     const int t = blockIdx.y;
@@ -1608,13 +1658,13 @@ __global__ void __launch_bounds__(256) k_moe_down(const uint16_t * __restrict__ 
         const float a = pi_lanes_sum<64>(hy_dot_lane(wdown + ((int64_t) e * width + n) * ff, up + ((int64_t) t * top + kk) * ff, ff, lane, exact != 0, vec != 0));
         acc = fmaf(wgt, a, acc);
     }
-    if (lane == 0) out[(int64_t) t * os + n] = acc;
+    if (!pi_abort_late(gone, abort_w, 0) && lane == 0) out[(int64_t) t * os + n] = acc;
 }
 
 static int moe_route_launch(const pi_weight * router, const float * correction_dev, const float * x, int64_t x_stride, int n_tok, int top, int exact, int n_groups, int keep, int32_t * sel_dev, float * selw_dev, void * stream) {
     if (n_tok <= 0) return 0;
     if (!router || router->type != PI_BF16 || top < 1 || top > router->ne1 || router->ne1 > 8192) { pi_set_error("pi_op_moe_route: a bfloat16 router of at most 8192 outputs and 1 <= top <= outputs are required"); return -1; }
-    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 2.0 * router->ne0 * router->ne1 + 4.0 * n_tok * router->ne0, k_moe_route, dim3((unsigned) n_tok), dim3(256), (size_t) 8 * router->ne1 + (size_t) 4 * std::max(n_groups, 1), (hipStream_t) stream,
+    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 2.0 * router->ne0 * router->ne1 + 4.0 * n_tok * router->ne0, k_moe_route, dim3((unsigned) n_tok), dim3((unsigned) (64 * (n_tok <= 64 ? std::min<int64_t>(16, router->ne1) : 4))), (size_t) 8 * router->ne1 + (size_t) 4 * std::max(n_groups, 1), (hipStream_t) stream,
                  (const uint16_t *) router->p0, router->ne0, (int) router->ne1, correction_dev, x, x_stride, top, exact,
                  (int) (router->ne0 % 8 == 0 && ((uintptr_t) router->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0), n_groups, keep, sel_dev, selw_dev, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;

@@ -167,10 +167,11 @@ __global__ void __launch_bounds__(64) k_qkv_prepare_any(const float * __restrict
                                                         const float * __restrict__ kw, float eps, int H, int G, int GV, int D, int V, const float2 * __restrict__ rot, int half, int n_pos, int norm_first, int pairing, int v_norm, float temp_coef, int temp_every,
                                                         const int32_t * __restrict__ pos, float * __restrict__ q_out, int64_t qos, float * __restrict__ kc, float * __restrict__ vc,
                                                         int32_t * __restrict__ cell_pos, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, slot = blockIdx.y, lane = threadIdx.x;
     const int cell = pi_cell_of(dyn, 0, t);
     const int p = pos[t];
+    if (pi_abort_late(gone, abort_w)) return;                          // (behind the position, which everything waits for)
     if (k && slot == 0 && lane == 0) cell_pos[cell] = p;                // (queries alone: the cells belong to the layer whose keys are read)
     if (slot >= H + G) {
         const int g = slot - H - G;
@@ -317,11 +318,11 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
                                                          const uint32_t * __restrict__ mask, const int32_t * __restrict__ pos, const float * __restrict__ hbias, const float * __restrict__ gate, int64_t gs, int gate_act,
                                                          float scale, float out_mult, int weights, float softcap, int chunk, int H, int G, int D, int V, int n_kv_arg, int tile, int hps, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn,
                                                          const float * __restrict__ sink, int mask_kind, int pool, int pool_off, int pool_z, int n_hz, int n_cs, int split_cells, float * __restrict__ part, int keep_first, ca_maps mp, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 5)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ float lds[];                // q [hpg][D] | key tile [tile][D + 1], then the value tile [tile][V] in the same place | weights [tile][hpg]
     if (pool_z > 0 && (int) blockIdx.z == pool_z) {                   // the extra slice of workgroups: the pooled rows of the blocks this pass's tokens close (no token of the pass reads them: the host checked n_tok <= window)
         const int p = pos[blockIdx.x];
-        if ((p + 1) % pool != 0) return;
+        if (pi_abort_late(gone, abort_w, 5) || (p + 1) % pool != 0) return;
         pm_pool_block((float *) kc, (float *) vc, cell_pos, mask + (int64_t) blockIdx.x * ((n_kv_arg + 31) / 32), p, pool, pool_off, G, blockIdx.y, D, V, min(dyn ? dyn[1] : n_kv_arg, n_kv_arg), pi_cell_of(dyn, 0, blockIdx.x), (int *) lds);
         return;
     }
@@ -347,6 +348,7 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
     // the first position the token sees as itself: the start of its block of `chunk` positions, or of the window of `chunk` positions that ends with the token
     const int first_pos = chunk <= 0 ? 0 : mask_kind == PI_MASK_WINDOW ? p - chunk + 1 : p / chunk * chunk;
     for (int i = tid; i < nr * D; i += 256) qsh[i] = q[(int64_t) t * qs + (int64_t) h0 * KD + i];
+    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the queries, requested after it)
     float acc[CA_MAXOUT];
 #pragma unroll
     for (int i = 0; i < CA_MAXOUT; i++) acc[i] = 0.0f;
@@ -456,7 +458,7 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
 // the cell splits of a token's head merged: M = max(maxima, sink), out = sum_s e^(m_s - M) sums_s / (e^(sink - M) + sum_s e^(m_s - M) l_s), in split order; grid (token, head)
 __global__ void __launch_bounds__(128) k_attention_combine(const float * __restrict__ part, int n_cs, int H, int V, const float * __restrict__ sink, int weights, const float * __restrict__ gate, int64_t gs, int gate_act,
                                                            float out_mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, h = blockIdx.y;
     const float * pr = part + ((int64_t) t * H + h) * n_cs * (V + 2);
     const bool has_sink = sink || weights == PI_WEIGHTS_SOFTMAX_SINK;
@@ -465,6 +467,7 @@ __global__ void __launch_bounds__(128) k_attention_combine(const float * __restr
     for (int s = 0; s < n_cs; s++) M = fmaxf(M, pr[(int64_t) s * (V + 2) + V]);
     float den = has_sink ? expf(sk - M) : 0.0f;
     for (int s = 0; s < n_cs; s++) { const float ms = pr[(int64_t) s * (V + 2) + V]; if (ms != -INFINITY) den = fmaf(pr[(int64_t) s * (V + 2) + V + 1], expf(ms - M), den); }
+    if (pi_abort_late(gone, abort_w)) return;
     float gt = gate ? gate[(int64_t) t * gs + h] : 1.0f;
     if (gate && gate_act == PI_ACT_SIGMOID) gt = pm_sigmoid(gt);
     for (int v = threadIdx.x; v < V; v += 128) {
@@ -475,7 +478,7 @@ __global__ void __launch_bounds__(128) k_attention_combine(const float * __restr
 }
 // the same where a head is two maps: grid (token, head), both maps' splits merged into LDS, then joined by one wave
 __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __restrict__ part, int n_cs, int H, int V, ca_maps mp, float out_mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     extern __shared__ float maps_lds[];                               // [2][V]
     const int t = blockIdx.x, h = blockIdx.y, map = threadIdx.x >> 6, lane = threadIdx.x & 63;        // a wave per map
     const float * pr = part + (((int64_t) t * H + h) * 2 + map) * n_cs * (V + 2);
@@ -487,13 +490,20 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
     for (int v0 = 0; v0 < V; v0 += 64) {
         const int v = v0 + lane;
         float a = 0.0f;
-        for (int s = 0; s < n_cs; s++) {
-            const float f = __shfl(f_l, s, 64);
-            if (f > 0.0f && v < V) a = fmaf(pr[(int64_t) s * (V + 2) + v], f, a);
+        for (int s0 = 0; s0 < n_cs; s0 += 8) {                         // eight splits on their way at a time
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = pr[(int64_t) min(s0 + u, n_cs - 1) * (V + 2) + min(v, V - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const float f = s0 + u < n_cs ? __shfl(f_l, s0 + u, 64) : 0.0f;
+                if (f > 0.0f) a = fmaf(x[u], f, a);
+            }
         }
         if (v < V) maps_lds[map * V + v] = den > 0.0f ? a / den : 0.0f;
     }
     __syncthreads();
+    if (pi_abort_late(gone, abort_w)) return;
     if (map == 0) ca_join_maps(maps_lds, maps_lds + V, V, mp, out_mult, out + (int64_t) t * os + (int64_t) h * V, lane);
 }
 // cell splits of a pass of n_tok tokens over n_kv cells: how many, and the floats of scratch they need (0 splits: the pass is wide enough to fill the device by itself)
@@ -681,9 +691,10 @@ __global__ void __launch_bounds__(256) k_causal_conv_walk(const float * __restri
                                                           float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, int act, float * __restrict__ out, int64_t os, int cblocks,
                                                           const float * __restrict__ raw, int64_t raws, const float * __restrict__ dt_bias, const float * __restrict__ a_log, int heads,
                                                           float * __restrict__ dt, float * __restrict__ decay, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x;
     if ((int) blockIdx.y == cblocks) {                                // step sizes and decays of token t
+        if (pi_abort_late(gone, abort_w)) return;
         for (int h = threadIdx.x; h < heads; h += 256) {
             const float z = raw[(int64_t) t * raws + h] + dt_bias[h];
             const float sp = z > 20.0f ? z : log1pf(expf(z));
@@ -703,6 +714,7 @@ __global__ void __launch_bounds__(256) k_causal_conv_walk(const float * __restri
 #pragma unroll
     for (int l = 0; l < CV_MAXTAPS; l++) wt[l] = l >= off ? w[(int64_t) c * taps + (l - off)] : 0.0f;
     const float b0 = bias ? bias[c] : 0.0f;
+    if (pi_abort_late(gone, abort_w)) return;
     for (int tt = t; tt < n_tok && (rec[tt] & ~PM_FRESH) == slot; tt++) {
         const float v = x[(int64_t) tt * xs + c];
         float a = b0;

@@ -90,6 +90,13 @@ static __device__ __forceinline__ bool pi_aborted(const int32_t * w, int fam = 6
     return true;
 }
 
+// the same for a small launch, whose own loads take no longer than the word's: requested at the top (pi_abort_peek), looked at just ahead of the first store (a trip to memory of its own at the top: 0.3 us of 3.4)
+static __device__ __forceinline__ bool pi_abort_late(int peek, const int32_t * w, int fam = 6) {
+    if ((peek & 1) == 0) return false;
+    pi_abort_note(w, fam);
+    return true;
+}
+
 // KV cell of token i of a pass.  dyn (device memory, refreshed per call so that one captured graph serves every call): {kv_head, n_kv, n_tokens, has_table, cell[0..n_tokens)}.
 // A run's tokens sit in consecutive cells from kv_head (find_slot, llama.cpp:1593-1644); a pass that carries several runs at once (context.cpp: coalescing) brings a table.
 static __device__ __forceinline__ int pi_cell_of(const int32_t * dyn, int kv_head, int i) { return dyn ? (dyn[3] ? dyn[4 + i] : dyn[0] + i) : kv_head + i; }

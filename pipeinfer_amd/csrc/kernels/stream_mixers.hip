@@ -24,10 +24,16 @@ template <int S, int VEC, int NG>
 __global__ void __launch_bounds__(1024) k_hyper_step(const float * xin, int64_t xts, int64_t xss, int ns, const float * __restrict__ y, int64_t ys, const float * __restrict__ mix, const float * __restrict__ outc,
                                                      const float * __restrict__ in_next, const float * __restrict__ shift, const float * __restrict__ w, float eps, int n, float * xo, float * __restrict__ h, int64_t hs,
                                                      const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     __shared__ float red[16];
     const int t = blockIdx.x;
     float u[NG][VEC], ss = 0.0f;
+    float wn[NG][VEC];                                                // the norm's weight is on its way with the streams
+#pragma unroll
+    for (int g = 0; g < NG; g++) {
+        const int i = min((int) (threadIdx.x + g * blockDim.x) * VEC, n - VEC);
+        if constexpr (VEC == 4) { const float4 v = *(const float4 *) (w + i); wn[g][0] = v.x; wn[g][1] = v.y; wn[g][2] = v.z; wn[g][3] = v.w; } else wn[g][0] = w[i];
+    }
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         const int i = (threadIdx.x + g * blockDim.x) * VEC;
@@ -69,7 +75,7 @@ __global__ void __launch_bounds__(1024) k_hyper_step(const float * xin, int64_t 
 #pragma unroll
                 for (int e = 0; e < VEC; e++) v[e] += shift[i + e];
             }
-            if (xo) {
+            if (xo && !(gone & 1)) {
                 float * dst = xo + ((int64_t) t * ns + d) * n + i;
                 if constexpr (VEC == 4) *(float4 *) dst = make_float4(v[0], v[1], v[2], v[3]); else dst[0] = v[0];
             }
@@ -85,14 +91,15 @@ __global__ void __launch_bounds__(1024) k_hyper_step(const float * xin, int64_t 
     __syncthreads();
     float tot = 0.0f;
     for (int i = 0; i < (int) (blockDim.x >> 6); i++) tot += red[i];
+    if (pi_abort_late(gone, abort_w)) return;
     const float inv = 1.0f / sqrtf(tot / (float) n + eps);
 #pragma unroll
     for (int g = 0; g < NG; g++) {
         const int i = (threadIdx.x + g * blockDim.x) * VEC;
         if (i >= n) continue;
         float * dst = h + (int64_t) t * hs + i;
-        if constexpr (VEC == 4) { const float4 wv = *(const float4 *) (w + i); *(float4 *) dst = make_float4(u[g][0] * inv * wv.x, u[g][1] * inv * wv.y, u[g][2] * inv * wv.z, u[g][3] * inv * wv.w); }
-        else dst[0] = u[g][0] * inv * w[i];
+        if constexpr (VEC == 4) *(float4 *) dst = make_float4(u[g][0] * inv * wn[g][0], u[g][1] * inv * wn[g][1], u[g][2] * inv * wn[g][2], u[g][3] * inv * wn[g][3]);
+        else dst[0] = u[g][0] * inv * wn[g][0];
     }
 }
 static int hyper_step(const float * x_in, int64_t token_stride, int64_t stream_stride, int streams, const float * y, int64_t y_stride, const float * mix_dev, const float * out_dev, const float * in_next_dev,
@@ -243,7 +250,7 @@ extern "C" int pi_op_window_mask(const uint32_t * mask_dev, const int32_t * pos_
 __global__ void __launch_bounds__(256) k_latent_prepare(const float * __restrict__ p, int64_t ps, int q_rank, const float * __restrict__ qw, int rank, const float * __restrict__ kw, int rot, const float2 * __restrict__ cs,
                                                         int n_pos, int pairing, float eps, const int32_t * __restrict__ pos, float * __restrict__ cq, int64_t cqs, float * __restrict__ cache, const int32_t * __restrict__ dyn,
                                                         const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x;
     const bool is_q = blockIdx.y == 0;
@@ -254,6 +261,7 @@ __global__ void __launch_bounds__(256) k_latent_prepare(const float * __restrict
     ss = pi_lanes_sum<64>(ss);
     if ((tid & 63) == 0) red[tid >> 6] = ss;
     __syncthreads();
+    if (pi_abort_late(gone, abort_w)) return;
     const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float) n + eps);
     float * dst = is_q ? cq + (int64_t) t * cqs : cache + (int64_t) pi_cell_of(dyn, 0, t) * (rank + rot);
     for (int i = tid; i < n; i += 256) dst[i] = src[i] * inv * w[i];
