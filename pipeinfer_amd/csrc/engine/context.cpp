@@ -147,6 +147,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
                 in_w = std::max(in_w, (size_t) A.in_rows() + (size_t) 5 * width);
                 att_w = std::max(att_w, (size_t) A.heads * (A.dim + A.vdim) + (size_t) 7 * R.inner() + (size_t) R.decay_rank);
                 ctx->rec_scratch_floats = std::max(ctx->rec_scratch_floats, pi_op_channel_recurrence_scratch_floats(R.heads, R.dim, R.dim, nb, ctx->slots->size()));
+                ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_window_attention_scratch_floats(A.heads, A.vdim, nb));
                 positions = true;
             }
             ctx->rec_off[i] = rec; rec += (size_t) ctx->slots->size() * H.state_floats();
@@ -169,6 +170,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
             ctx->lat_off[i] = lat; lat += (size_t) ctx->n_ctx * H.cell_floats();
             ctx->rec_off[i] = rec; rec += (size_t) ctx->slots->size() * H.state_floats();
             ctx->rec_scratch_floats = std::max(ctx->rec_scratch_floats, pi_op_linear_attention_scratch_floats(R.heads, R.state, R.vdim, nb, ctx->slots->size()));
+            ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_window_attention_scratch_floats(A.heads, A.vdim, nb));
             in_w = std::max(in_w, (size_t) std::max(H.in_rows(), std::max(H.mlp == PI_MLP_DENSE_RELU_SQR ? H.ff : 0, 3 * H.shared_ff)));
             att_w = std::max(att_w, (size_t) A.heads * (A.dim + A.vdim) + (size_t) R.channels() + (size_t) R.inner());
             step_w = std::max(step_w, (size_t) 2 * R.heads); positions = true;
@@ -386,8 +388,8 @@ static bool forward_parallel_mixer(llama_context * ctx, const pi_hybrid_layer & 
     if (ctx->branch_stream && (hipEventRecord(ctx->branch_events[2 * il], s_main) != hipSuccess || hipStreamWaitEvent(s2, ctx->branch_events[2 * il], 0) != hipSuccess)) { ctx->last_error = "fork of the mixer's branches failed"; return false; }
     // attention branch (its output already carries the branch's factor)
     OP_OK(pi_op_qkv_prepare(P, P + hd, P + hd + gd, pw, W.q_norm, W.k_norm, eps, A.heads, A.kv_heads, A.dim, A.vdim, W.rotary, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
-    OP_OK(pi_op_chunk_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, W.head_bias, P + hd + gd + gv, pw, PI_ACT_SIGMOID, A.scale, H.left_scale, A.chunk, A.heads, A.kv_heads, A.dim, A.vdim, n_tok, n_kv,
-                                O, ow, ctx->dyn_dev, s));
+    OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, W.head_bias, nullptr, P + hd + gd + gv, pw, PI_ACT_SIGMOID, A.scale, H.left_scale, PI_WEIGHTS_SIGMOID, 0.0f, PI_MASK_CHUNK, A.chunk, 0, 0, 0, A.heads,
+                                 A.kv_heads, A.dim, A.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, ow, ctx->dyn_dev, s));
     trace(ctx, "att", (int) il, O, hv, n_tok, ow);
     // recurrence branch
     const float * R0 = P + A.in_rows();                                   // z | x B C | dt
@@ -511,8 +513,8 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
             // attention branch
             OP_OK(pi_op_dense(W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
             OP_OK(pi_op_qkv_prepare_ex(P, P + hd, P + hd + gd, pw, nullptr, nullptr, eps, L.heads, L.kv_heads, L.dim, L.vdim, W.rotary, 0, PI_PAIR_NEIGHBOURS, 0, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
-            OP_OK(pi_op_chunk_attention_ex(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, 0, PI_ACT_NONE, L.scale, 1.0f, L.weights, L.softcap, L.chunk, L.heads, L.kv_heads, L.dim, L.vdim, n_tok, n_kv,
-                                           O, hv, ctx->dyn_dev, s));
+            OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, nullptr, 0, PI_ACT_NONE, L.scale, 1.0f, L.weights, L.softcap, PI_MASK_CHUNK, L.chunk, 0, 0, 0, L.heads, L.kv_heads, L.dim,
+                                         L.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
             trace(ctx, "att", (int) il, O, hv, n_tok);
             OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
             // time-mix branch

@@ -455,25 +455,36 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
     }
 }
 
-// the cell splits of a token's head merged: M = max(maxima, sink), out = sum_s e^(m_s - M) sums_s / (e^(sink - M) + sum_s e^(m_s - M) l_s), in split order; grid (token, head)
+// the cell splits of a token's head merged: M = max(maxima, sink), out = sum_s e^(m_s - M) sums_s / (e^(sink - M) + sum_s e^(m_s - M) l_s), in split order (sigmoid weights: the sums alone); grid (token, head)
 __global__ void __launch_bounds__(128) k_attention_combine(const float * __restrict__ part, int n_cs, int H, int V, const float * __restrict__ sink, int weights, const float * __restrict__ gate, int64_t gs, int gate_act,
                                                            float out_mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
-    const int t = blockIdx.x, h = blockIdx.y;
+    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
     const float * pr = part + ((int64_t) t * H + h) * n_cs * (V + 2);
-    const bool has_sink = sink || weights == PI_WEIGHTS_SOFTMAX_SINK;
-    const float sk = sink ? sink[h] : 0.0f;
-    float M = has_sink ? sk : -INFINITY;
-    for (int s = 0; s < n_cs; s++) M = fmaxf(M, pr[(int64_t) s * (V + 2) + V]);
-    float den = has_sink ? expf(sk - M) : 0.0f;
-    for (int s = 0; s < n_cs; s++) { const float ms = pr[(int64_t) s * (V + 2) + V]; if (ms != -INFINITY) den = fmaf(pr[(int64_t) s * (V + 2) + V + 1], expf(ms - M), den); }
-    if (pi_abort_late(gone, abort_w)) return;
+    const bool soft = weights != PI_WEIGHTS_SIGMOID, has_sink = soft && (sink || weights == PI_WEIGHTS_SOFTMAX_SINK);
+    const float sk = has_sink && sink ? sink[h] : 0.0f;
     float gt = gate ? gate[(int64_t) t * gs + h] : 1.0f;
+    // (a lane per split: n_cs <= CA_SPLIT_MAX <= 64)
+    const float ms_l = lane < n_cs ? pr[(int64_t) lane * (V + 2) + V] : -INFINITY, ls_l = lane < n_cs ? pr[(int64_t) lane * (V + 2) + V + 1] : 0.0f;
+    const float M = fmaxf(pi_wave_max(ms_l), has_sink ? sk : -INFINITY);
+    const float f_l = ms_l == -INFINITY ? 0.0f : soft ? expf(ms_l - M) : 1.0f;
+    const float den = pi_lanes_sum<64>(f_l > 0.0f ? ls_l * f_l : 0.0f) + (has_sink ? expf(sk - M) : 0.0f);
     if (gate && gate_act == PI_ACT_SIGMOID) gt = pm_sigmoid(gt);
-    for (int v = threadIdx.x; v < V; v += 128) {
+    if (pi_abort_late(gone, abort_w)) return;
+    for (int v0 = 0; v0 < V; v0 += 128) {
+        const int v = v0 + (int) threadIdx.x;
         float a = 0.0f;
-        for (int s = 0; s < n_cs; s++) { const float ms = pr[(int64_t) s * (V + 2) + V]; if (ms != -INFINITY) a = fmaf(pr[(int64_t) s * (V + 2) + v], expf(ms - M), a); }
-        out[(int64_t) t * os + (int64_t) h * V + v] = (den > 0.0f ? a / den : 0.0f) * gt * out_mult;
+        for (int s0 = 0; s0 < n_cs; s0 += 8) {                         // eight splits on their way at a time
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = pr[(int64_t) min(s0 + u, n_cs - 1) * (V + 2) + min(v, V - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const float f = s0 + u < n_cs ? __shfl(f_l, s0 + u, 64) : 0.0f;
+                if (f > 0.0f) a = fmaf(x[u], f, a);
+            }
+        }
+        if (v < V) out[(int64_t) t * os + (int64_t) h * V + v] = (!soft ? a : den > 0.0f ? a / den : 0.0f) * gt * out_mult;
     }
 }
 // the same where a head is two maps: grid (token, head), both maps' splits merged into LDS, then joined by one wave
@@ -572,12 +583,33 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
     if (maps * hpg * vdim > 256 * CA_MAXOUT || lds > 60 * 1024) { pi_set_error("pi_op_chunk_attention: %d query heads per key head of sizes %d / %d are beyond the kernel (LDS %zu bytes)", hpg, dim, vdim, lds); return -1; }
     const int acct = pi_account_n_kv() > 0 ? pi_account_n_kv() : n_kv;
     const double visible = chunk > 0 ? std::min(acct, chunk) + (pool > 0 ? std::max(acct - chunk, 0) / pool : std::min(std::max(acct - chunk, 0), keep_first)) : acct;
-    if (pool == 0 && !pool_here) {                                     // a prompt: 32 tokens of a head at a time
+    auto merge = [&]() -> int {                                        // the splits' shares, where there are any
+        if (maps == 2) {
+            PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * (2.0 * n_cs * (vdim + 2) + vdim), k_attention_combine_maps, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), (size_t) 2 * vdim * sizeof(float),
+                         (hipStream_t) stream, scratch, n_cs, heads, vdim, mp, out_mult, out, out_stride, pi_abort_word());
+            PI_CHECK_LAUNCH();
+        } else {
+            PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * ((double) n_cs * (vdim + 2) + vdim), k_attention_combine, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), 0, (hipStream_t) stream,
+                         scratch, n_cs, heads, vdim, sink_dev, weights, gate_dev, gate_stride, gate_act, out_mult, out, out_stride, pi_abort_word());
+            PI_CHECK_LAUNCH();
+        }
+        return 0;
+    };
+    if (pool == 0 && !pool_here) {                                     // a few tokens with splits; a prompt: 32 tokens of a head at a time
         pa_args a = {};
         a.q = q; a.qs = q_stride; a.k1 = k_cache; a.k1_row = (int64_t) kv_heads * maps * dim; a.k1_head = (int64_t) maps * dim; a.dim1 = dim; a.v = v_cache; a.v_row = (int64_t) kv_heads * vdim; a.v_head = vdim; a.vdim = vdim;
         a.cell1 = n_kv; a.heads = heads; a.per_kv = heads / kv_heads; a.n_tok = n_tok; a.n_kv = n_kv; a.dyn = dyn_dev; a.mask = mask_dev; a.cell_pos = cell_pos_dev; a.pos = pos_dev; a.mask_kind = mask_kind; a.chunk = chunk;
         a.keep_first = keep_first; a.scale = scale; a.hbias = head_bias_dev; a.softcap = softcap; a.weights = weights; a.sink = sink_dev; a.gate = gate_dev; a.gs = gate_stride; a.gate_act = gate_act; a.gate_width = 1;
         a.out_mult = out_mult; a.lam = mp.lam; a.eps = mp.eps; a.out = out; a.os = out_stride; a.first = a.last = 1;
+        a.state = scratch;
+        const double few_bytes = 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim);
+        if (const int few = pa_few_split(a, maps, scratch_floats, &split_cells)) {
+            pa_few_launch(a, maps, few, split_cells, few_bytes, (hipStream_t) stream);
+            PI_CHECK_LAUNCH();
+            n_cs = few;
+            return merge();
+        }
+        a.state = nullptr;
         if (pa_takes(a, maps, PA_CACHE_TOKENS)) { pa_launch(a, maps, 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (hipStream_t) stream); PI_CHECK_LAUNCH(); return 0; }
     }
 #define CA_GO(R, MP)     PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (k_chunk_attention<R, MP>), dim3((unsigned) n_tok, (unsigned) kv_heads, (unsigned) (n_z * n_cs + (pool_here ? 1 : 0))), dim3(256), lds, \
@@ -586,16 +618,7 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
     if (maps == 2) { CA_GO(4, 2); } else { CA_GO(4, 1); }              // (deeper rounds were measured for single tokens: no gain, the registers they take cost as much as the trips they save)
 #undef CA_GO
     PI_CHECK_LAUNCH();
-    if (split_cells > 0 && maps == 2) {
-        PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * (2.0 * n_cs * (vdim + 2) + vdim), k_attention_combine_maps, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), (size_t) 2 * vdim * sizeof(float),
-                     (hipStream_t) stream, scratch, n_cs, heads, vdim, mp, out_mult, out, out_stride, pi_abort_word());
-        PI_CHECK_LAUNCH();
-    } else if (split_cells > 0) {
-        PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * ((double) n_cs * (vdim + 2) + vdim), k_attention_combine, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), 0, (hipStream_t) stream,
-                     scratch, n_cs, heads, vdim, sink_dev, weights, gate_dev, gate_stride, gate_act, out_mult, out, out_stride, pi_abort_word());
-        PI_CHECK_LAUNCH();
-    }
-    return 0;
+    return split_cells > 0 ? merge() : 0;
 }
 
 // ---- pooled far blocks: one key / value per block of `pool` positions ------------------------------------------------------------------------------------------

@@ -30,3 +30,8 @@ void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s);
 #define PA_LATENT_TOKENS 9
 // keys [cell][heads * dim] and values [cell][heads * vdim] of the cells [cell0, cell1) from their latents (row stride `width` floats)
 void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, const int32_t * dyn, float * k, float * v, hipStream_t s);
+// a few tokens over keys and values in a cache: splits of 32 cells (or of several times 32), sixteen query heads of a key head at a time, every split's [vdim sums | maximum | denominator] per (token, head, map)
+// into a.state for the caller's merge.  pa_few_split: cells of a split and their number, 0: not for this kernel
+int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split_cells);
+void pa_few_launch(const pa_args & a, int maps, int n_cs, int split_cells, double bytes, hipStream_t s);
+#define PA_FEW_SPLITS 32

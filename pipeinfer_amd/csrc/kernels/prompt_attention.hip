@@ -351,3 +351,144 @@ void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * w
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, PI_KT_MAXNT - 1, 2.0 * rank * (wuk->ne1 + wuv->ne1) + 4.0 * std::min(cell1 - cell0, n_kv) * (double) (width + wuk->ne1 + wuv->ne1), k_latent_expand, dim3((unsigned) ((tiles + 7) / 8 * 8)), dim3(256), 0, s,
                  cache, width, (int64_t) rank, (const uint16_t *) wuk->p0, wuk->ne1, (const uint16_t *) wuv->p0, wuv->ne1, cell0, cell1, dyn, k, v, cell_blocks, tiles, pi_abort_word());
 }
+
+// ---- a few tokens ---------------------------------------------------------------------------------------------------------------------------------------------------
+// grid (token, key head; split).  A workgroup per token that stages keys, then scores them, then stages values, waits for memory at every one of these (29 us for 4 tokens of 16 differential heads in a window of 256
+// of 700 cells); here the keys and values of 32 cells are on their way together, the scores of the key head's query heads are one tile of a matrix product, and so is every 16 outputs of theirs (XX
+// merge 6.6 instead of 4.5 for there are more splits; 8 tokens of 32 sigmoid heads over 40 to 350 cells: 31 us, now 8.0 and a merge of 5).  Lane layout as above, rows = query heads: scores of row n and the cells 4 g + c, sums of row n and the outputs 16 NV wave + NV (4 g + r) + j
+template <int NK, int NV, int MAPS>
+__global__ void __launch_bounds__(256) k_few_attention(const pa_args A, int n_cs, int split_cells, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    constexpr int V = 64 * NV, STEPS = MAPS == 2 ? NK : NK / 2;       // one map: two waves share a tile's key values
+    typedef float vec __attribute__((ext_vector_type(NV)));
+    __shared__ __attribute__((aligned(16))) float ps[MAPS][16][36], half[2][16][20];
+    __shared__ float top[MAPS][2][16], sum[MAPS][2][16];
+    const int G = A.heads / A.per_kv, t = blockIdx.x / G, kvh = blockIdx.x % G, cs = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, ct = wave & 1, wm = wave >> 1;
+    const int n_kv = min(A.dyn ? A.dyn[1] : A.n_kv, A.n_kv), words = (A.n_kv + 31) / 32, c_end = min(n_kv, (cs + 1) * split_cells);
+    const int h = kvh * A.per_kv + min(n, A.per_kv - 1), p = A.pos[t], map = MAPS == 2 ? wm : 0, step0 = MAPS == 2 ? 0 : wm * STEPS;
+    const int first = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
+    const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
+    const float * qr = A.q + (int64_t) t * A.qs + (int64_t) (h * MAPS + map) * (16 * NK), * kb = A.k1 + (int64_t) kvh * A.k1_head + map * (16 * NK), * vb = A.v + (int64_t) kvh * A.v_head;
+    const float bias = A.hbias ? A.hbias[h] : 0.0f;
+    pa_f32x4 qf[STEPS], acc[MAPS][NV];
+#pragma unroll
+    for (int i = 0; i < STEPS; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) qf[i][c] = qr[16 * (step0 + i) + 4 * g + c];
+    float m_run[MAPS], l_run[MAPS];
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        m_run[mp] = -INFINITY; l_run[mp] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; j++) acc[mp][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
+    bool any = false;
+    for (int c0 = cs * split_cells; c0 < c_end; c0 += 32) {
+        const int mc = c0 + (lane & 31);
+        bool see = false;
+        if (mc < c_end) { const int cp = A.cell_pos[mc]; see = (A.mask[(int64_t) t * words + (c0 >> 5)] >> (lane & 31) & 1u) && (cp >= first || cp < A.keep_first); }
+        const uint32_t vis = (uint32_t) __ballot(see);
+        if (!vis) continue;
+        pa_f32x4 kf[STEPS]; vec vf[2][4];
+        {
+            const float * kr = kb + (int64_t) min(c0 + 16 * ct + n, c_end - 1) * A.k1_row + 16 * step0 + 4 * g;
+#pragma unroll
+            for (int i = 0; i < STEPS; i++) kf[i] = *(const pa_f32x4 *) (kr + 16 * i);
+        }
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) vf[jt][c] = *(const vec *) (vb + (int64_t) min(c0 + 16 * jt + 4 * g + c, c_end - 1) * A.v_row + 16 * NV * wave + NV * n);
+        __builtin_amdgcn_sched_barrier(0);
+        pa_f32x4 s = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < STEPS; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) s = pa_mfma(kf[i][c], qf[i][c], s);
+        if (any) __syncthreads();                                     // (the last round's weights are no longer read)
+        if constexpr (MAPS == 1) {
+            if (wm) *(pa_f32x4 *) &half[ct][n][4 * g] = s;
+            __syncthreads();
+            if (!wm) s += *(const pa_f32x4 *) &half[ct][n][4 * g];
+        }
+        const bool scores = MAPS == 2 || !wm;
+        const uint32_t mine = vis >> (16 * ct + 4 * g);
+        float m = -INFINITY;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            float x = s[c] * A.scale + bias;
+            if (soft && A.softcap > 0.0f) x = A.softcap * tanhf(x / A.softcap);
+            s[c] = x;
+            if (mine >> c & 1u) m = fmaxf(m, x);
+        }
+        if (soft) {
+            m = fmaxf(m, __shfl_xor(m, 16, 64)); m = fmaxf(m, __shfl_xor(m, 32, 64));
+            if (scores && g == 0) top[map][ct][n] = m;
+            __syncthreads();
+        }
+        float m_new[MAPS], f[MAPS];
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            m_new[mp] = soft ? fmaxf(m_run[mp], fmaxf(top[mp][0][n], top[mp][1][n])) : 0.0f;
+            f[mp] = !soft || m_run[mp] == m_new[mp] ? 1.0f : expf(m_run[mp] - m_new[mp]);
+            m_run[mp] = m_new[mp];
+        }
+        if (scores) {
+            float l = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; c++) { const float e = !(mine >> c & 1u) ? 0.0f : soft ? expf(s[c] - m_new[map]) : 1.0f / (1.0f + expf(-s[c])); s[c] = e; l += e; }
+            l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+            if (g == 0) sum[map][ct][n] = l;
+            *(pa_f32x4 *) &ps[map][n][16 * ct + 4 * g] = s;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) if (!(vis >> (16 * jt + 4 * g + c) & 1u)) vf[jt][c] = vec(0.0f);        // (a cell that the token does not see may hold anything)
+#pragma unroll
+        for (int mp = 0; mp < MAPS; mp++) {
+            l_run[mp] = fmaf(l_run[mp], f[mp], sum[mp][0][n] + sum[mp][1][n]);
+#pragma unroll
+            for (int j = 0; j < NV; j++) acc[mp][j] *= f[mp];
+#pragma unroll
+            for (int jt = 0; jt < 2; jt++) {
+                const pa_f32x4 w = *(const pa_f32x4 *) &ps[mp][n][16 * jt + 4 * g];
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int j = 0; j < NV; j++) { float x; if constexpr (NV == 1) x = vf[jt][c][0]; else x = vf[jt][c][j]; acc[mp][j] = pa_mfma(x, w[c], acc[mp][j]); }
+            }
+        }
+        any = true;
+    }
+    if (pi_abort_late(gone, abort_w, 5) || n >= A.per_kv) return;
+#pragma unroll
+    for (int mp = 0; mp < MAPS; mp++) {
+        float * pr = A.state + (((int64_t) (t * A.heads + h) * MAPS + mp) * n_cs + cs) * (V + 2);
+        if (wave == 0 && g == 0) { pr[V] = any ? m_run[mp] : -INFINITY; pr[V + 1] = l_run[mp]; }
+        if (any)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < NV; j++) pr[16 * NV * wave + NV * (4 * g + r) + j] = acc[mp][j][r];
+    }
+}
+int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split_cells) {
+    auto four = [](int64_t n) { return (n & 3) == 0; };
+    if (a.n_tok >= PA_CACHE_TOKENS || a.n_kv <= 64 || !a.state || a.per_kv > 16 || (a.dim1 != 64 && a.dim1 != 128) || (a.vdim != 64 && a.vdim != 128) || !four(a.k1_row) || !four(a.k1_head) || !four(a.v_row) || !four(a.v_head) ||
+        (((uintptr_t) a.k1 | (uintptr_t) a.v) & 15)) return 0;
+    const int chunks = (a.n_kv + 31) / 32, per = (chunks + PA_FEW_SPLITS - 1) / PA_FEW_SPLITS, n_cs = (chunks + per - 1) / per;
+    if ((size_t) a.n_tok * a.heads * maps * n_cs * (a.vdim + 2) > scratch_floats) return 0;
+    *split_cells = 32 * per;
+    return n_cs;
+}
+void pa_few_launch(const pa_args & a, int maps, int n_cs, int split_cells, double bytes, hipStream_t s) {
+    const dim3 grid((unsigned) (a.n_tok * (a.heads / a.per_kv)), (unsigned) n_cs);
+    const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
+#define FEW_GO(NK, NV) do { if (maps == 2) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_few_attention<NK, NV, 2>), grid, dim3(256), 0, s, a, n_cs, split_cells, pi_abort_word()); \
+                            else PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_few_attention<NK, NV, 1>), grid, dim3(256), 0, s, a, n_cs, split_cells, pi_abort_word()); } while (0)
+    if (a.dim1 == 64) { if (a.vdim == 64) FEW_GO(4, 1); else FEW_GO(4, 2); } else { if (a.vdim == 64) FEW_GO(8, 1); else FEW_GO(8, 2); }
+#undef FEW_GO
+}

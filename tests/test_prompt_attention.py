@@ -5,6 +5,7 @@ import pytest
 from pipeinfer_amd import lib as L
 from tests import test_fasovik as fasovik
 from tests.test_letevik import HALVES, NEIGHBOURS, SIGMOID, O, diff_attention_ref, gpu, latent_case, pack_mask, rel_rms, run_diff
+from tests.test_rarevik import CHUNK
 
 
 @pytest.mark.gpu
@@ -52,7 +53,7 @@ def scattered(rng, T, n_kv, n_ctx):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 4, 4, 3, 2, 40, 32), (8, 2, 64, 128, 256, 4, 700, 97), (3, 3, 36, 68, 0, 0, 130, 65), (4, 1, 128, 64, 9, 33, 333, 200), (4, 2, 192, 128, 50, 0, 161, 40)])
+@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 4, 4, 3, 2, 40, 32), (8, 2, 64, 128, 256, 4, 700, 97), (3, 3, 36, 68, 0, 0, 130, 65), (4, 1, 128, 64, 9, 33, 333, 200), (16, 1, 64, 128, 256, 4, 700, 4), (6, 2, 128, 64, 9, 33, 333, 31), (5, 5, 64, 64, 0, 0, 1200, 1), (4, 2, 192, 128, 50, 0, 161, 40)])
 @pytest.mark.parametrize("maps", [2, 1])
 def test_window_prompt(H, G, D, V, size, keep, n_kv, T, maps):
     """plain and differential heads over windows with kept positions, cells in any order, garbage behind the live cells"""
@@ -68,15 +69,16 @@ def test_window_prompt(H, G, D, V, size, keep, n_kv, T, maps):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,G,D,V,chunk,n_kv,T", [(2, 1, 16, 8, 32, 90, 33), (8, 2, 128, 128, 256, 600, 150), (40, 1, 8, 128, 9, 290, 32)])
+@pytest.mark.parametrize("H,G,D,V,chunk,n_kv,T", [(2, 1, 16, 8, 32, 90, 33), (8, 2, 128, 128, 256, 600, 150), (40, 1, 8, 128, 9, 290, 32), (1, 1, 64, 64, 7, 65, 1), (32, 2, 128, 64, 64, 300, 4), (24, 8, 64, 128, 300, 1100, 31),
+                                                   (30, 2, 128, 128, 700, 2100, 8)])
 @pytest.mark.parametrize("softcap", [0.0, 3.0])
 def test_weights_of_a_prompt(H, G, D, V, chunk, n_kv, T, softcap):
-    """sigmoid weights, a soft-max and one with a sink, a bias and a gate per head, capped scores (of a soft-max); a token that sees nothing; values that are no numbers reach the tokens that see them and no others"""
+    """passes of many tokens, and of few over splits of the cells (sixteen query heads of a key head or fewer, a split of one round and of several, splits that show nothing): sigmoid weights, a soft-max and one with a sink, a bias and a gate per head, capped scores (of a soft-max); a token that sees nothing; values that are no numbers reach the tokens that see them and no others"""
     U, lib = gpu()
     rng = np.random.default_rng(n_kv + T)
     kc, vc = rng.standard_normal((n_kv, G, D)).astype(np.float32), rng.standard_normal((n_kv, G, V)).astype(np.float32)
     cpos, pos, vis = scattered(rng, T, n_kv, n_kv)
-    vis[7] = False
+    vis[7:8] = False
     hurt = vis[:, 5] & (cpos[5] >= (pos // chunk * chunk))
     q, gate, hb = rng.standard_normal((T, H, D)).astype(np.float32), rng.standard_normal((T, H)).astype(np.float32), rng.standard_normal(H).astype(np.float32)
     for loud in (False, True):
@@ -85,7 +87,10 @@ def test_weights_of_a_prompt(H, G, D, V, chunk, n_kv, T, softcap):
         for weights in (0, 1, 2):
             d = [U.Dev(a) for a in (q, kc, vc, cpos, pack_mask(vis, n_kv), pos, hb, gate, np.array([0, n_kv, T, 0], np.int32))]
             od = U.Dev(nbytes=4 * T * H * V)
-            L.check(lib.pi_op_chunk_attention_ex(d[0].ptr, H * D, d[1].ptr, d[2].ptr, d[3].ptr, d[4].ptr, d[5].ptr, d[6].ptr, d[7].ptr, H, SIGMOID, 0.21, -1.5, weights, softcap, chunk, H, G, D, V, T, n_kv, od.ptr, H * V, d[8].ptr, None))
+            n_scr = lib.pi_op_window_attention_scratch_floats(H, V, T)
+            scr = U.Dev(np.full(n_scr, np.nan, np.float32))
+            L.check(lib.pi_op_window_attention(d[0].ptr, H * D, d[1].ptr, d[2].ptr, d[3].ptr, d[4].ptr, d[5].ptr, d[6].ptr, None, d[7].ptr, H, SIGMOID, 0.21, -1.5, weights, softcap, CHUNK, chunk, 0, 0, 0, H, G, D, V, T, n_kv,
+                                               scr.ptr, n_scr, od.ptr, H * V, d[8].ptr, None))
             got, want = od.get(np.float32, (T, H, V)), np.zeros((T, H, V))
             for t in range(T):
                 js = np.nonzero(vis[t] & (cpos >= pos[t] // chunk * chunk))[0]
