@@ -39,12 +39,25 @@ static __device__ __forceinline__ float dn_act(float v, int act) {
     }
 }
 
-__global__ void k_embed(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+// grid (token, 2048 values); vec: eight values of a thread in one 16-byte load (rows and output start 16-byte aligned), else one by one
+__global__ void __launch_bounds__(256) k_embed(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, int vec, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x;
-    const int64_t row = tokens[t];
-    if (row < 0 || row >= n_rows) { for (int64_t i = threadIdx.x; i < width; i += blockDim.x) out[(int64_t) t * width + i] = 0.0f; return; }
-    for (int64_t i = threadIdx.x; i < width; i += blockDim.x) out[(int64_t) t * width + i] = dn_widen(table[row * width + i]) * scale;
+    const int64_t row = tokens[t], i0 = (int64_t) blockIdx.y * 2048;
+    if (pi_abort_late(gone, abort_w)) return;
+    const bool ok = row >= 0 && row < n_rows;
+    if (vec) {
+        const int64_t i = i0 + 8 * threadIdx.x;
+        if (i >= width) return;
+        const dn_u16x8 a = *(const dn_u16x8 *) (table + (ok ? row : 0) * width + i);
+        float4 o[2];
+#pragma unroll
+        for (int c = 0; c < 8; c++) ((float *) o)[c] = ok ? dn_widen(a[c]) * scale : 0.0f;
+        float4 * dst = (float4 *) (out + (int64_t) t * width + i);
+        dst[0] = o[0]; dst[1] = o[1];
+        return;
+    }
+    for (int64_t i = i0 + threadIdx.x; i < min(width, i0 + 2048); i += 256) out[(int64_t) t * width + i] = ok ? dn_widen(table[row * width + i]) * scale : 0.0f;
 }
 
 // VW weights per lane and step (8: one 16-byte load, 4: 8 bytes, 1: any K and alignment)
@@ -201,7 +214,9 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
 extern "C" int pi_op_embed(const pi_weight * w, const int32_t * tokens, int n_tok, float scale, float * out, void * stream) {
     if (!w || w->type != PI_BF16) { pi_set_error("pi_op_embed: the table must be a bfloat16 weight"); return -1; }
     if (n_tok <= 0) return 0;
-    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * w->ne0 * n_tok, k_embed, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, (const uint16_t *) w->p0, w->ne0, w->ne1, tokens, scale, out, pi_abort_word());
+    const int vec = w->ne0 % 8 == 0 && w->ne1 > 0 && (((uintptr_t) w->p0 | (uintptr_t) out) & 15) == 0;
+    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * w->ne0 * n_tok, k_embed, dim3((unsigned) n_tok, (unsigned) ((w->ne0 + 2047) / 2048)), dim3(256), 0, (hipStream_t) stream, (const uint16_t *) w->p0, w->ne0, w->ne1, tokens, scale, vec, out,
+                 pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 

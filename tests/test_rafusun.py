@@ -202,6 +202,26 @@ def test_embedding_adds_the_pair_row():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("width", [8, 2048, 4104, 2050])
+def test_embedding_widths(width):
+    """eight values at a time and one by one, rows that are not full, tokens outside the tables (zeros): the same bits as the products and the sum in 32 bits"""
+    U, lib = gpu()
+    rng = np.random.default_rng(width)
+    table, table2 = O.bf16_round(rng.standard_normal((7, width)).astype(np.float32)), O.bf16_round(rng.standard_normal((5, width)).astype(np.float32))
+    toks, rows = np.array([6, -1, 0, 7, 3], np.int32), np.array([4, 0, 5, -1, 2], np.int32)
+    w, w2 = upload_bf16(lib, table), upload_bf16(lib, table2)
+    td, rd, od = U.Dev(toks), U.Dev(rows), U.Dev(nbytes=4 * 5 * width)
+    first = np.where(((toks >= 0) & (toks < 7))[:, None], table[np.clip(toks, 0, 6)] * np.float32(0.3), np.float32(0))
+    second = np.where(((rows >= 0) & (rows < 5))[:, None], table2[np.clip(rows, 0, 4)], np.float32(0))
+    L.check(lib.pi_op_embed(w, td.ptr, 5, 0.3, od.ptr, None))
+    assert np.array_equal(od.get(np.float32, (5, width)), first)
+    L.check(lib.pi_op_embed_pair(w, td.ptr, 5, 0.3, w2, rd.ptr, od.ptr, None))
+    assert np.array_equal(od.get(np.float32, (5, width)), first + second)
+    lib.pi_weight_free(w)
+    lib.pi_weight_free(w2)
+
+
+@pytest.mark.gpu
 def test_dense_epilogues_tanh_and_gelu():
     U, lib = gpu()
     rng = np.random.default_rng(2)
