@@ -7,7 +7,7 @@
 //
 //   k_dense_rows   one wave per output row, K spread over the lanes with 16 / 8 / 2-byte weight loads, TT tokens held in registers: the mat-vec of single tokens (weights streamed once from HBM:
 //                  6.7 TB/s at 32000 x 4096, 4.3 at 4096 x 4096, 4 us of launch below 1024 x 1024) and every width of the fp32 mode
-//   k_dense_split  serving precision, 2 .. 32 tokens: 16 or 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (4.6 TB/s at 32000 x 4096 and up to
+//   k_dense_split  serving precision, 2 .. 32 tokens: 4 .. 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (4.6 TB/s at 32000 x 4096 and up to
 //                  8 tokens).  On the mat-vec every row reads all tokens' activations again, 2 T times its own bytes: 28 us for 4096 x 4096 at 8 tokens, 11 here
 //   k_dense_tile   serving precision, more tokens: tiles of 64 .. 128 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory
 //                  (26 bytes a cycle of cold weights and activations), large ones by the shared levels of memory and the steps' latency: 730 TFLOP/s at 16384 x 4096 x 2048 tokens (the tiles without
@@ -142,23 +142,23 @@ __global__ void __launch_bounds__(256 * KG, 2) k_dense_tile(const uint16_t * __r
     }
 }
 
-// 2 .. 64 tokens: RT x 16 rows and TT x 16 tokens per workgroup, K split over its eight waves, which meet in LDS.  The weights are streamed once, straight from memory in the operand's lane layout: the
-// four lanes of a row take 64 consecutive bytes of it per product, the activations come from L2 once per workgroup.  Rows in segments: as k_dense_rows, whole tiles
+// 2 .. 32 tokens: up to RT x 16 rows (`rows`, a multiple of 4: the lanes of the others read the last one again, which costs no bytes) and TT x 16 tokens per workgroup, K split over its eight waves, which meet in LDS.  The weights are streamed once, straight from memory in the operand's lane layout: the
+// four lanes of a row take 64 consecutive bytes of it per product, the activations come from L2 once per workgroup.  Rows in segments: as k_dense_rows, whole workgroups
 // inside a segment (the host checks).
 template <int RT, int TT>
 __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
-                                                     int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int64_t seg_rows, int64_t seg_off, int seg_last, const int32_t * __restrict__ abort_w) {
+                                                     int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int64_t seg_rows, int64_t seg_off, int seg_last, int rows, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 0)) return;
     constexpr int KS = 8;
     __shared__ dt_f32x4 red[KS][RT * TT][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
-    const int64_t n0 = (int64_t) blockIdx.x * (16 * RT);
+    const int64_t n0 = (int64_t) blockIdx.x * rows;
     const int t0 = blockIdx.y * (16 * TT);
     if (seg_rows > 0) X += min(n0 / seg_rows, (int64_t) seg_last) * seg_off;
     const int64_t per = (K + 64 * KS - 1) / (64 * KS) * 64, k_begin = wave * per, k_end = min(K, k_begin + per);
     const uint16_t * wrow[RT]; const float * xrow[TT];
 #pragma unroll
-    for (int a = 0; a < RT; a++) wrow[a] = W + min(n0 + a * 16 + li, N - 1) * K + kb * 8;
+    for (int a = 0; a < RT; a++) wrow[a] = W + min(n0 + min(a * 16 + li, rows - 1), N - 1) * K + kb * 8;
 #pragma unroll
     for (int b = 0; b < TT; b++) xrow[b] = X + (int64_t) min(t0 + b * 16 + li, T - 1) * xs + kb * 8;
     dt_f32x4 acc[RT][TT];
@@ -206,8 +206,8 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
         dt_f32x4 v = red[0][tile][l];
 #pragma unroll
         for (int w = 1; w < KS; w++) v += red[w][tile][l];
-        const int64_t row = n0 + (tile / TT) * 16 + (l >> 4) * 4;
-        if (row < N) dn_store4(v, row, N, tok, Y, ys, act_a, rows_a, act_b, bias);
+        const int own = (tile / TT) * 16 + (l >> 4) * 4;
+        if (own < rows && n0 + own < N) dn_store4(v, n0 + own, N, tok, Y, ys, act_a, rows_a, act_b, bias);
     }
 }
 
@@ -236,12 +236,24 @@ static void launch_rows(const pi_weight * w, const float * x, int64_t xs, int n_
 //                          fill the chip and read the activations less often (32000 x 2048 at 24: 41 against 26)
 //   more                   k_dense_tile
 static bool dense_takes_split(int64_t rows, int64_t k, int n_tok) { return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32) && !(n_tok == 2 && rows * k <= (4 << 20)); }
-// 32 rows per workgroup where that still leaves a workgroup per compute unit; at up to four tokens long rows rather take twice the workgroups (8192 x 4096 at 2 tokens: 14.7 against 16.7; 32000 x 2048: 31 against 24)
+// Rows per workgroup: the chip's 256 compute units take a workgroup each at a time, and a round of them lasts about as long as 8 + rows (K 4096 at 8 tokens: 16 rows 7.8 us a round, 24 10, 32 13; the launch itself 4).  So
+// the split that needs the least, in steps of 4 rows, the larger one of two that need the same.  Against 16 rows (32 from 8192 rows on), us at 2 .. 4 / 8 / 32 tokens: 6144 x 4096 17.6 / 19.8 / 39.0, now 24 rows
+// 13.3 / 14.5 / 24.2; 5120 x 13824 46.6 / 59.3 / 123, now 20 rows 32.8 / 37.8 / 71.7; 16448 x 4096 at 8 41.5, now 24 rows 37.6; 32000 x 4096 at 4 63.8, now 32 rows 52.5; 2048 x 2048 6.5 / 7.0 / 11.8, now 8 rows
+// 5.9 / 6.4 / 11.2; 8192 x 4096 at 2 the one that loses, 16.2, now 32 rows 17.0 (at 4 17.8 and 17.0)
+static int split_rows(int64_t n, int64_t seg_rows) {
+    int best = 16; int64_t least = INT64_MAX;
+    for (int r = 32; r >= 4; r -= 4) {
+        const int64_t cost = ((n + r - 1) / r + 255) / 256 * (8 + r);
+        if (cost < least && (seg_rows <= 0 || seg_rows % r == 0)) { least = cost; best = r; }
+    }
+    return best;
+}
 static void launch_split(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias, int64_t seg_rows = 0,
                          int64_t seg_off = 0, int seg_last = 0) {
-    const bool two = w->ne1 >= 8192 && (n_tok > 4 || w->ne0 < 4096);
-#define DN_SPLIT(RT, TT) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_split<RT, TT>), dim3((unsigned) ((w->ne1 + 16 * RT - 1) / (16 * RT)), (unsigned) ((n_tok + 16 * TT - 1) / (16 * TT))), \
-                                     dim3(512), 0, s, (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word())
+    const int r = split_rows(w->ne1, seg_rows);
+    const bool two = r > 16;
+#define DN_SPLIT(RT, TT) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_split<RT, TT>), dim3((unsigned) ((w->ne1 + r - 1) / r), (unsigned) ((n_tok + 16 * TT - 1) / (16 * TT))), \
+                                     dim3(512), 0, s, (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, r, pi_abort_word())
     if (n_tok <= 16) { if (two) DN_SPLIT(2, 1); else DN_SPLIT(1, 1); }
     else { if (two) DN_SPLIT(2, 2); else DN_SPLIT(1, 2); }
 #undef DN_SPLIT

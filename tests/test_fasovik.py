@@ -187,9 +187,9 @@ def test_dense_every_kernel_and_width(K, N, T, exact):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("K,N,T", [(8, 1, 2), (72, 33, 16), (1096, 130, 17), (520, 8193, 32), (4104, 8200, 3), (64, 16, 33), (1000, 70, 65), (2048, 16390, 9),
-                                   (200, 2100, 520), (136, 4100, 600), (72, 8200, 600)])
+                                   (136, 3001, 3), (520, 5102, 20), (72, 6143, 17), (264, 7007, 8), (200, 2100, 520), (136, 4100, 600), (72, 8200, 600)])
 def test_dense_on_the_matrix_cores(K, N, T):
-    """16-byte aligned rows: k_dense_split (one / two tiles of rows and of tokens; K that ends inside a step, or before some of the waves' shares begin) and k_dense_tile (64 x 64 and 128 x 64 with K over
+    """16-byte aligned rows: k_dense_split (one / two tiles of rows and of tokens, tiles of rows that are not full; K that ends inside a step, or before some of the waves' shares begin) and k_dense_tile (64 x 64 and 128 x 64 with K over
     two groups of waves, 128 x 64 and 128 x 128), rows and tokens that end inside a tile, padded strides, a bias and both activations.  Sums of K products of bfloat16 values in fp32: 2e-6 as above"""
     U, lib = gpu()
     rng = np.random.default_rng(K + N + T)
