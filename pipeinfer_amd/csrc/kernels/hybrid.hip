@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 static __device__ __forceinline__ float hy_widen(uint16_t b) { return __uint_as_float((uint32_t) b << 16); }
 static __device__ __forceinline__ float hy_round(float f) { const uint32_t u = __float_as_uint(f); return __uint_as_float(((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16); }
@@ -493,7 +494,7 @@ extern "C" int pi_op_sum_tanh_norm_shift(const float * x, int64_t x_stride, cons
 // rec[t] = state slot of token t (| 1 << 30 on the first token of a sequence whose state starts from zero), tokens of one slot are consecutive.  Workgroup (head, column block,
 // piece): thread (column j, part sp of R) keeps S[i][j] for its DPT rows i in registers and walks the piece's tokens in order.
 // A pass of up to LA_TB tokens is one launch: a piece is a sequence's whole run, S comes from and goes back to HBM.  Longer passes cut every sequence's run into pieces of LA_TB
-// tokens and take three launches, so that the serial depth is two pieces instead of the whole prompt (the recurrence is linear in S):
+// tokens and take three launches (on the matrix cores: pieces of LM_TB, see there; a pass of as many tokens one launch), so that the serial depth is two pieces instead of the whole prompt (the recurrence is linear in S):
 //   mode 1  every piece but a run's last: the state it would build from ZERO, L_p = sum_j lambda^(len-1-j) k_j v_j^T, into scratch
 //   k_linear_state_scan  per run, piece by piece: S_in(p + 1) = lambda^len_p * S_in(p) + L_p, S_in(0) = the slot's state (or zero); scratch[p] <- S_in(p)
 //   mode 2  every piece from its true S_in(p): outputs; a run's last piece leaves the slot's new state
@@ -634,6 +635,7 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
 // value waits for the one before, two products per state value on the vector units.  Per head and piece, with a_t = lambda_1 .. lambda_t and D[t][j] = lambda_{j+1} .. lambda_t (products only, no quotients):
 //   states   L = sum_j (lambda_{j+1} .. lambda_64 s_j k_j) v_j^T                 (as mode 1)
 //   outputs  O = a_t (Q S_in) + (Q K^T o D s) V;  a run's last piece also leaves a_64 S_in + L   (as mode 2)
+// A piece of up to 16 or 32 tokens takes as many tiles (a run of 16 tokens alone: 42 us with all four, 23).
 // 2048 tokens, 32 heads of 128 x 128: 2 x 759 us -> 98 + 124, the scan between them 58 -> 34 (half the pieces, half the memory); 512 tokens, 16 heads: 2 x 93 -> 27 + 48, 11 -> 7.
 #define LM_TB 64
 #define LM_MAX_TOKENS 16384                       // (the pass's slot words in LDS beside the 54 KB of a piece)
@@ -668,8 +670,9 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
     if (len == 0 || word < 0 || (!OUTPUTS && last)) return;
     const int hq = h / hpg;
     const float * qp = q + (int64_t) first * stride + (int64_t) hq * DIM, * kp = k + (int64_t) first * stride + (int64_t) hq * DIM, * vp = v + (int64_t) first * stride + (int64_t) h * vstored;
+    const int tiles = len <= 16 ? 1 : len <= 32 ? 2 : 4;              // of 16 tokens
     auto stage = [&](const float * src) {                             // rows behind the last repeat it: nothing of theirs is used
-        for (int i = tid; i < LM_TB * DIM; i += 256) { const int t = i / DIM, d = i % DIM; qk[t * PITCH + d] = src[(int64_t) min(t, len - 1) * stride + d]; }
+        for (int i = tid; i < 16 * tiles * DIM; i += 256) { const int t = i / DIM, d = i % DIM; qk[t * PITCH + d] = src[(int64_t) min(t, len - 1) * stride + d]; }
     };
     stage(OUTPUTS ? qp : kp);
     if (wave == 0) {
@@ -693,10 +696,12 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
     __syncthreads();
     const int64_t per = (int64_t) DIM * vdim;
     float * S_scr = scratch + ((int64_t) blockIdx.y * heads + h) * per;
+    const float * S_in = OUTPUTS && !scratch ? state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per : S_scr;      // (no scratch: a piece is its sequence's whole run)
+    const bool zero = OUTPUTS && !scratch && (word & LA_FRESH);
     const int n_tiles = (vdim + 15) / 16;
     if constexpr (OUTPUTS) {
         // (Q K^T o D s) transposed: tiles (rows j, columns t) on and below the diagonal, shared out among the waves; a lane's four rows are consecutive values of row t of pt
-        for (int i = wave; i < 10; i += 4) {
+        for (int i = wave; i < tiles * (tiles + 1) / 2; i += 4) {
             const int tt = i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3, jt = i - tt * (tt + 1) / 2, j = 16 * jt + n;
             const float * kr = kp + (int64_t) min(j, len - 1) * stride;
             hy_f32x4 a = { 0.0f, 0.0f, 0.0f, 0.0f };
@@ -720,68 +725,74 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
             *(hy_f32x4 *) &pt[t * PP + 16 * jt + 4 * g] = a;
         }
         __syncthreads();
-        for (int nt = wave; nt < n_tiles; nt += 4) {
-            const int c = 16 * nt + n, cc = min(c, vdim - 1);
-            float sv[8 * DI];                                          // S_in: rows 16 s + 4 g + i of column c
+        auto outputs = [&](auto n_mt) {
+            constexpr int MT = decltype(n_mt)::value;
+            for (int nt = wave; nt < n_tiles; nt += 4) {
+                const int c = 16 * nt + n, cc = min(c, vdim - 1);
+                float sv[8 * DI];                                          // S_in: rows 16 s + 4 g + i of column c
 #pragma unroll
-            for (int s = 0; s < 2 * DI; s++)
+                for (int s = 0; s < 2 * DI; s++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) sv[4 * s + i] = lm_at(S_scr, (uint32_t) (16 * s + 4 * g + i) * (uint32_t) vdim + (uint32_t) cc);
-            float vv[16];                                              // values: rows 16 jt + 4 g + r
+                    for (int i = 0; i < 4; i++) { const float x = lm_at(S_in, (uint32_t) (16 * s + 4 * g + i) * (uint32_t) vdim + (uint32_t) cc); sv[4 * s + i] = zero ? 0.0f : x; }
+                float vv[4 * MT];                                          // values: rows 16 jt + 4 g + r
 #pragma unroll
-            for (int i = 0; i < 16; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored); }
-            hy_f32x4 acc[4];
+                for (int i = 0; i < 4 * MT; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored); }
+                hy_f32x4 acc[MT];
 #pragma unroll
-            for (int m = 0; m < 4; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+                for (int m = 0; m < MT; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-            for (int s = 0; s < 2 * DI; s++) {
-                __builtin_amdgcn_sched_barrier(0);
-                hy_f32x4 qv[4];
-#pragma unroll
-                for (int m = 0; m < 4; m++) qv[m] = *(const hy_f32x4 *) &qk[(16 * m + n) * PITCH + 16 * s + 4 * g];
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int m = 0; m < 4; m++) acc[m] = hy_mfma(qv[m][i], sv[4 * s + i], acc[m]);
-            }
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc[m][r] *= upto[16 * m + 4 * g + r];
-#pragma unroll
-            for (int jt = 0; jt < 4; jt++) {
-                __builtin_amdgcn_sched_barrier(0);
-                uint32_t big = 0;                                      // (an infinity or a NaN among the values must not meet the zero weights of the tokens before it)
-#pragma unroll
-                for (int r = 0; r < 4; r++) big = max(big, __float_as_uint(vv[4 * jt + r]) & 0x7fffffffu);
-                const bool odd = __any(big >= 0x7f800000u);
-#pragma unroll
-                for (int m = jt; m < 4; m++) {
-                    if (m == jt && odd) {
-                        for (int j = 16 * jt; j < min(16 * jt + 16, len); j++) {
-                            const float x = lm_value(vp, j, (uint32_t) stride, cc, vstored);
-#pragma unroll
-                            for (int r = 0; r < 4; r++) if (j <= 16 * m + 4 * g + r) acc[m][r] = fmaf(pt[(16 * m + 4 * g + r) * PP + j], x, acc[m][r]);
-                        }
-                        continue;
-                    }
-                    const hy_f32x4 pv = *(const hy_f32x4 *) &pt[(16 * m + n) * PP + 16 * jt + 4 * g];
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[m] = hy_mfma(pv[r], vv[4 * jt + r], acc[m]);
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int t = 16 * m + 4 * g + r;
-                    if (t >= len || c >= vdim) continue;
+                for (int s = 0; s < 2 * DI; s++) {
                     __builtin_amdgcn_sched_barrier(0);
-                    float o = acc[m][r];
-                    if (skip) o = fmaf(skip[h], lm_value(vp, t, (uint32_t) stride, c, vstored), o);
-                    out[(int64_t) (first + t) * os + (int64_t) h * vdim + c] = o;
+                    hy_f32x4 qv[MT];
+#pragma unroll
+                    for (int m = 0; m < MT; m++) qv[m] = *(const hy_f32x4 *) &qk[(16 * m + n) * PITCH + 16 * s + 4 * g];
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+#pragma unroll
+                        for (int m = 0; m < MT; m++) acc[m] = hy_mfma(qv[m][i], sv[4 * s + i], acc[m]);
                 }
-        }
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[m][r] *= upto[16 * m + 4 * g + r];
+#pragma unroll
+                for (int jt = 0; jt < MT; jt++) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    uint32_t big = 0;                                      // (an infinity or a NaN among the values must not meet the zero weights of the tokens before it)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) big = max(big, __float_as_uint(vv[4 * jt + r]) & 0x7fffffffu);
+                    const bool odd = __any(big >= 0x7f800000u);
+#pragma unroll
+                    for (int m = jt; m < MT; m++) {
+                        if (m == jt && odd) {
+                            for (int j = 16 * jt; j < min(16 * jt + 16, len); j++) {
+                                const float x = lm_value(vp, j, (uint32_t) stride, cc, vstored);
+#pragma unroll
+                                for (int r = 0; r < 4; r++) if (j <= 16 * m + 4 * g + r) acc[m][r] = fmaf(pt[(16 * m + 4 * g + r) * PP + j], x, acc[m][r]);
+                            }
+                            continue;
+                        }
+                        const hy_f32x4 pv = *(const hy_f32x4 *) &pt[(16 * m + n) * PP + 16 * jt + 4 * g];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) acc[m] = hy_mfma(pv[r], vv[4 * jt + r], acc[m]);
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int t = 16 * m + 4 * g + r;
+                        if (t >= len || c >= vdim) continue;
+                        __builtin_amdgcn_sched_barrier(0);
+                        float o = acc[m][r];
+                        if (skip) o = fmaf(skip[h], lm_value(vp, t, (uint32_t) stride, c, vstored), o);
+                        out[(int64_t) (first + t) * os + (int64_t) h * vdim + c] = o;
+                    }
+            }
+        };
+        if (tiles == 1) outputs(std::integral_constant<int, 1>{});
+        else if (tiles == 2) outputs(std::integral_constant<int, 2>{});
+        else outputs(std::integral_constant<int, 4>{});
         if (!last) return;
         __syncthreads();
         stage(kp);
@@ -790,31 +801,37 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
     // the state of the piece: from zero (scratch), or from S_in (the slot)
     float * S_to = OUTPUTS ? state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per : S_scr;
     const float all = upto[LM_TB - 1];
-    for (int nt = wave; nt < n_tiles; nt += 4) {
-        const int c = 16 * nt + n, cc = min(c, vdim - 1);
-        float vv[16];
+    auto states = [&](auto n_mt) {
+        constexpr int MT = decltype(n_mt)::value;
+        for (int nt = wave; nt < n_tiles; nt += 4) {
+            const int c = 16 * nt + n, cc = min(c, vdim - 1);
+            float vv[4 * MT];
 #pragma unroll
-        for (int i = 0; i < 16; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = j < len ? lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored) * (from[j] * sc[j]) : 0.0f; }
-        hy_f32x4 acc[2 * DI];
+            for (int i = 0; i < 4 * MT; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = j < len ? lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored) * (from[j] * sc[j]) : 0.0f; }
+            hy_f32x4 acc[2 * DI];
 #pragma unroll
-        for (int m = 0; m < 2 * DI; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+            for (int m = 0; m < 2 * DI; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            __builtin_amdgcn_sched_barrier(0);
-            const float * kr = &qk[(16 * (i >> 2) + 4 * g + (i & 3)) * PITCH + n];
+            for (int i = 0; i < 4 * MT; i++) {
+                __builtin_amdgcn_sched_barrier(0);
+                const float * kr = &qk[(16 * (i >> 2) + 4 * g + (i & 3)) * PITCH + n];
 #pragma unroll
-            for (int m = 0; m < 2 * DI; m++) acc[m] = hy_mfma(kr[16 * m], vv[i], acc[m]);
+                for (int m = 0; m < 2 * DI; m++) acc[m] = hy_mfma(kr[16 * m], vv[i], acc[m]);
+            }
+            if (c < vdim)
+#pragma unroll
+                for (int m = 0; m < 2 * DI; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const uint32_t at = ((uint32_t) (16 * m + 4 * g + r) * (uint32_t) vdim + (uint32_t) c) * 4u;
+                        if (OUTPUTS && r == 0) __builtin_amdgcn_sched_barrier(0);
+                        *(float *) ((char *) S_to + at) = !OUTPUTS || zero ? acc[m][r] : fmaf(all, *(const float *) ((const char *) S_in + at), acc[m][r]);
+                    }
         }
-        if (c < vdim)
-#pragma unroll
-            for (int m = 0; m < 2 * DI; m++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const uint32_t at = ((uint32_t) (16 * m + 4 * g + r) * (uint32_t) vdim + (uint32_t) c) * 4u;
-                    if (OUTPUTS && r == 0) __builtin_amdgcn_sched_barrier(0);
-                    *(float *) ((char *) S_to + at) = OUTPUTS ? fmaf(all, *(const float *) ((const char *) S_scr + at), acc[m][r]) : acc[m][r];
-                }
-    }
+    };
+    if (tiles == 1) states(std::integral_constant<int, 1>{});
+    else if (tiles == 2) states(std::integral_constant<int, 2>{});
+    else states(std::integral_constant<int, 4>{});
 }
 
 // grid (head, blocks over dim * vdim, run): scratch[piece] holds L_p coming in and S_in(p) going out
@@ -935,24 +952,33 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
     const int nta = std::min(n_tok, PI_KT_MAXNT - 1);
 #define LA_GO(D, MODE) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_attention<D>, grid, dim3(threads), lds, s, q, k, v, stride, heads, hpg, dim, vdim, value_cols, R, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, state_dev, rec_dev, n_tok, MODE, scratch_dev, out, out_stride, pi_abort_word())
 #define LA_ANY(MODE) do { if (dpt == 8) LA_GO(8, MODE); else if (dpt == 16) LA_GO(16, MODE); else LA_GO(32, MODE); } while (0)
-    if (!pieces) { LA_ANY(0); PI_CHECK_LAUNCH(); return 0; }
+    const bool matrix = dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22);       // (32-bit offsets within a piece; pieces twice as long take half of the scratch that was asked for)
     const unsigned gr = (unsigned) std::max(1, std::min(n_tok, max_segments)), gb = (unsigned) (((int64_t) dim * vdim + 255) / 256);
-    if (dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22)) {        // (32-bit offsets within a piece; pieces twice as long take half of the scratch that was asked for)
+#define LM_GO(DI, OUT, SCR) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_linear_pieces<DI, OUT>), pg, dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, \
+                                    state_dev, rec_dev, n_tok, SCR, out, out_stride, pi_abort_word())
+#define LM_ANY(OUT, SCR) do { if (dim == 32) LM_GO(1, OUT, SCR); else if (dim == 64) LM_GO(2, OUT, SCR); else if (dim == 96) LM_GO(3, OUT, SCR); else LM_GO(4, OUT, SCR); } while (0)
+    // Up to 64 tokens every run is one piece: one launch from the slots' states to the slots' states.  Beyond LA_TB always (32 heads of 128 x 128, three launches against it: a run of 64 tokens 55 -> 48 us, 64 runs of a
+    // token 1115 -> 150, for the scan looked for its run in every workgroup); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
+    // (24 tokens 53 -> 29, 9 about even; eight runs of a token or two 14 .. 18, here 25 .. 29)
+    if (matrix && n_tok <= LM_TB && (pieces || n_tok > 8 * gr)) {
+        const dim3 pg((unsigned) heads, gr);
+        LM_ANY(true, nullptr);
+        PI_CHECK_LAUNCH(); return 0;
+    }
+    if (!pieces) { LA_ANY(0); PI_CHECK_LAUNCH(); return 0; }
+    if (matrix) {
         if (n_tok > 2048 && pi_op_linear_attention_reserve() != 0) return -1;
         const dim3 pg((unsigned) heads, (unsigned) (n_tok / LM_TB + std::min(n_tok, std::max(1, max_segments)) + 1));
-#define LM_GO(DI, OUT) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_linear_pieces<DI, OUT>), pg, dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, \
-                                    state_dev, rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word())
-#define LM_ANY(OUT) do { if (dim == 32) LM_GO(1, OUT); else if (dim == 64) LM_GO(2, OUT); else if (dim == 96) LM_GO(3, OUT); else LM_GO(4, OUT); } while (0)
-        LM_ANY(false);
+        LM_ANY(false, scratch_dev);
         PI_CHECK_LAUNCH();
         PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * pg.y * heads * dim * vdim, k_linear_state_scan<LM_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,
                      heads, dim, vdim, decay_dev, tdecay_dev, t_stride, state_dev, rec_dev, n_tok, scratch_dev, pi_abort_word());
         PI_CHECK_LAUNCH();
-        LM_ANY(true);
-#undef LM_ANY
-#undef LM_GO
+        LM_ANY(true, scratch_dev);
         PI_CHECK_LAUNCH(); return 0;
     }
+#undef LM_ANY
+#undef LM_GO
     LA_ANY(1);
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * gz * heads * dim * vdim, k_linear_state_scan<LA_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,

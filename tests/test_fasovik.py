@@ -310,7 +310,7 @@ def test_linear_attention_states_segments_and_slots(H, D, V):
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,G,D,V,per_token,key_sum", [(3, 3, 32, 5, False, 0), (4, 2, 64, 64, True, 0), (2, 1, 96, 33, True, 1), (4, 4, 128, 128, False, 0), (6, 3, 128, 47, True, 1)])
 def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_sum):
-    """passes longer than 32 tokens in pieces of 64: whole pieces, one token more, one less, several sequences, states carried and from nothing; decays per head and per token (very small ones and zeros among
+    """passes longer than 32 tokens in pieces of 64 (up to 64 tokens, and shorter ones of few sequences, every sequence is one piece): whole pieces, one token more, one less, several sequences, states carried and from nothing; decays per head and per token (very small ones and zeros among
     them), factors on the keys, a skip, a column of ones; a value that is no number reaches its own token and the later ones only"""
     U, lib = gpu()
     rng = np.random.default_rng(H * D + V)
@@ -320,7 +320,7 @@ def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_
     ref = state.astype(np.float64)
     sd, lam, skip = U.Dev(state), np.linspace(0.4, 0.999, H).astype(np.float32), rng.standard_normal(H).astype(np.float32)
 
-    def run(rec, hurt=None):
+    def run(rec, hurt=None, most=slots):
         T = len(rec)
         buf = (rng.standard_normal((T, stride)) * 0.5).astype(np.float32)
         dec, fac = np.exp(-np.exp(rng.standard_normal((T, H)) * 3 - 4)).astype(np.float32), rng.uniform(0.1, 2.0, (T, H)).astype(np.float32)
@@ -331,10 +331,10 @@ def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_
         if key_sum:
             v = np.concatenate([v, np.ones((T, H, 1))], -1)
         ds = [U.Dev(a) for a in (buf, np.array(rec, np.int32), lam, dec, fac, skip)]
-        od, n = U.Dev(nbytes=4 * T * H * VC), lib.pi_op_linear_attention_scratch_floats(H, D, VC, T, slots)
+        od, n = U.Dev(nbytes=4 * T * H * VC), lib.pi_op_linear_attention_scratch_floats(H, D, VC, T, most)
         scr = U.Dev(np.full(max(n, 1), np.nan, np.float32))
         L.check(lib.pi_op_linear_attention_keysum(ds[0].ptr, ds[0].ptr + 4 * G * D, ds[0].ptr + 8 * G * D, stride, H, G, D, V, key_sum, None if per_token else ds[2].ptr, ds[3].ptr if per_token else None,
-                                                  ds[4].ptr if per_token else None, H, ds[5].ptr if per_token else None, sd.ptr, ds[1].ptr, T, slots, scr.ptr, n, od.ptr, H * VC, None))
+                                                  ds[4].ptr if per_token else None, H, ds[5].ptr if per_token else None, sd.ptr, ds[1].ptr, T, most, scr.ptr, n, od.ptr, H * VC, None))
         got, want = od.get(np.float32, (T, H, VC)), np.zeros((T, H, VC))
         g = np.arange(H) // (H // G)
         with np.errstate(invalid="ignore"):
@@ -352,8 +352,13 @@ def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_
     run([0] * 130 + [1 | F] + [1] * 63 + [2] * 65 + [3])
     run([1] * 127 + [0] * 2)
     run([0] * 64)
+    run([0] * 5 + [1 | F] + [1] * 20 + [2] * 16 + [3 | F])
+    run([2] * 24, most=1)
+    run([3 | F] + [3] * 8, most=1)
+    run([3] + [1] * 31, most=2)
     assert rel_rms(sd.get(np.float32, state.shape), ref) < 1e-5
     run([3] * 3 + [0] * 150, hurt=75)
+    run([0 | F] + [0] * 40 + [2] * 2, hurt=9)
 
 
 def latent_ref(q, cache, vis, wuk, wuv, sink, scale, H, D, V):
