@@ -1650,22 +1650,24 @@ __global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict_
 
 // up[t][kk][f] = relu(W_up[e] x_t)^2 for the kk-th chosen expert e of token t (nothing for identity experts); a wave per row f.
 // glu: an expert's first matrix holds 2 * ff rows [gate | up] and up[t][kk][f] = silu(gate_f . x) * (up_f . x)
+// (this kernel and the next: the abort word and the choice leave together, and the word is looked at before the choice is used.  In a cancelled run the router has written none: what stands there may be anything, and
+// an expert's matrix is not read for nothing.  A choice below zero is nobody's)
 __global__ void __launch_bounds__(256) k_moe_up(const uint16_t * __restrict__ wup, int64_t width, int ff, int n_exp, const float * __restrict__ x, int64_t xs, const int32_t * __restrict__ sel,
                                                 int top, int exact, int vec, int glu, float limit, float * __restrict__ up, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     const int lane = threadIdx.x & 63, f = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int slot = blockIdx.y, e = sel[slot];
-    if (f >= ff || e >= n_exp) return;
+    if (pi_abort_late(gone, abort_w, 0) || f >= ff || (uint32_t) e >= (uint32_t) n_exp) return;
     const int t = slot / top;
     const float * xr = x + (int64_t) t * xs;
     if (glu) {
         const float g = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * 2 * ff + f) * width, xr, width, lane, exact != 0, vec != 0));
         const float u = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * 2 * ff + ff + f) * width, xr, width, lane, exact != 0, vec != 0));
-        if (!pi_abort_late(gone, abort_w, 0) && lane == 0) up[(int64_t) slot * ff + f] = hy_glu(g, u, glu, limit);
+        if (lane == 0) up[(int64_t) slot * ff + f] = hy_glu(g, u, glu, limit);
         return;
     }
     const float a = pi_lanes_sum<64>(hy_dot_lane(wup + ((int64_t) e * ff + f) * width, xr, width, lane, exact != 0, vec != 0));
-    if (!pi_abort_late(gone, abort_w, 0) && lane == 0) { const float r = fmaxf(a, 0.0f); up[(int64_t) slot * ff + f] = r * r; }
+    if (lane == 0) { const float r = fmaxf(a, 0.0f); up[(int64_t) slot * ff + f] = r * r; }
 }
 // out[t][n] = sum_kk w_kk * (identity ? x[t][n] : W_down[e_kk][n] . up[t][kk]); a wave per output n
 __global__ void __launch_bounds__(256) k_moe_down(const uint16_t * __restrict__ wdown, int64_t width, int ff, int n_exp, int top, const float * __restrict__ x, int64_t xs,
@@ -1675,16 +1677,19 @@ __global__ void __launch_bounds__(256) k_moe_down(const uint16_t * __restrict__ 
     const int lane = threadIdx.x & 63;
     const int64_t n = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
     const int t = blockIdx.y;
-    if (n >= width) return;
+    const int32_t * own = sel + (int64_t) t * top;
+    int e = own[0];
+    if (pi_abort_late(gone, abort_w, 0) || n >= width) return;
     float acc = 0.0f;
     for (int kk = 0; kk < top; kk++) {
-        const int e = sel[(int64_t) t * top + kk];
+        if (kk > 0) e = own[kk];
         const float wgt = selw[(int64_t) t * top + kk];
+        if (e < 0) continue;
         if (e >= n_exp) { acc = fmaf(wgt, x[(int64_t) t * xs + n], acc); continue; }
         const float a = pi_lanes_sum<64>(hy_dot_lane(wdown + ((int64_t) e * width + n) * ff, up + ((int64_t) t * top + kk) * ff, ff, lane, exact != 0, vec != 0));
         acc = fmaf(wgt, a, acc);
     }
-    if (!pi_abort_late(gone, abort_w, 0) && lane == 0) out[(int64_t) t * os + n] = acc;
+    if (lane == 0) out[(int64_t) t * os + n] = acc;
 }
 
 static int moe_route_launch(const pi_weight * router, const float * correction_dev, const float * x, int64_t x_stride, int n_tok, int top, int exact, int n_groups, int keep, int32_t * sel_dev, float * selw_dev, void * stream) {

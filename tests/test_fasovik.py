@@ -487,6 +487,45 @@ def test_router_and_experts(E, I, top, ff, width, exact):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("glu", [0, 1])
+@pytest.mark.parametrize("T", [1, 3])
+def test_experts_of_a_cancelled_run(T, glu):
+    """a run that is cancelled before its router: the choices were never written, the expert kernels look at nothing and write nothing, and both launches are counted whatever the first choice is.  In a run that goes
+    on, a choice below zero adds nothing"""
+    U, lib = gpu()
+    E, ff, width, top, n = 3, 24, 72, 2, 2 if glu else 1
+    rng = np.random.default_rng(T)
+    x = O.bf16_round(rng.standard_normal((T, width)).astype(np.float32))
+    ups, downs = bf(rng, E * n * ff, width, s=0.2), bf(rng, E * width, ff, s=0.2)
+    selw = rng.uniform(0.2, 1.0, (T, top)).astype(np.float32)
+    ud, dd, xd, wd, word = upload_bf16(lib, ups), upload_bf16(lib, downs), U.Dev(x), U.Dev(selw), U.Dev(np.zeros(16, np.int32))
+
+    def run(sel):
+        sd, hd, od = U.Dev(sel), U.Dev(np.full(T * top * ff, 777.0, np.float32)), U.Dev(np.full((T, width), 555.0, np.float32))
+        lib.pi_set_abort_word(word.ptr)
+        try:
+            L.check(lib.pi_op_moe_experts_act(ud, dd, E, ff, glu, xd.ptr, width, sd.ptr, wd.ptr, T, top, 1, hd.ptr, od.ptr, width, None))
+        finally:
+            lib.pi_set_abort_word(None)
+        return hd.get(np.float32), od.get(np.float32, (T, width))
+
+    nobody = np.full((T, top), -1, np.int32)
+    L.check(lib.pi_op_abort_begin(word.ptr, 7, None, None))
+    hidden, got = run(nobody)
+    assert np.all(hidden == 777.0) and np.all(got == 0.0)
+    one = np.stack([[-1, t % E] for t in range(T)]).astype(np.int32)
+    hidden, got = run(one)
+    want_h = hidden.reshape(T, top, ff)[:, 1].astype(np.float64)
+    want = np.stack([selw[t, 1] * (downs.reshape(E, width, ff)[t % E].astype(np.float64) @ want_h[t]) for t in range(T)])
+    assert np.all(hidden.reshape(T, top, ff)[:, 0] == 777.0) and rel_rms(got, want) < 1e-6            # (fp32 sums of 24 terms)
+    L.check(lib.pi_op_abort_cancel(word.ptr, 7, None))
+    for i, sel in enumerate((nobody, np.full((T, top), -2 ** 31, np.int32), np.full((T, top), E, np.int32), np.zeros((T, top), np.int32))):
+        hidden, got = run(sel)
+        assert np.all(hidden == 777.0) and np.all(got == 555.0)
+        assert word.get(np.int32)[8] == 2 * (i + 1)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,I,ff,width,T,top", [(2, 1, 136, 200, 300, 2), (8, 2, 64, 3080, 200, 2), (8, 0, 72, 1544, 210, 2), (70, 3, 16, 72, 40, 6), (1, 0, 8, 8, 33, 1), (3, 0, 24, 136, 700, 2)])
 @pytest.mark.parametrize("glu", [0, 1])
 def test_grouped_experts_tiles(E, I, ff, width, T, top, glu):
