@@ -47,8 +47,9 @@ PI_API int     pi_device_sync(void);
 
 /* Kernel-granular early cancellation (reference: the abort callback polled between graph nodes, ggml.c:15748-15811, llama.cpp:5614-5628, 5665-5687).
  * word_dev: the first int32 of a 64-byte block in device memory (zeroed by the owner) holding (run id << 1 | aborted); words 8..14 of the block count, per kernel family
- * (enum order of pi_kt_row.family), the launches that found the run aborted and returned on entry.  Every hot-path kernel launched — or captured into a
- * graph — by the calling thread after pi_set_abort_word(word_dev) reads it on entry and returns at once when bit 0 is set (NULL: no check).
+ * (enum order of pi_kt_row.family), the launches that found the run aborted and returned without a result.  Every hot-path kernel launched — or captured into a
+ * graph — by the calling thread after pi_set_abort_word(word_dev) asks for it on entry and, when bit 0 is set, returns before it writes anything and before it streams weights or
+ * walks cells (NULL: no check).
  *   pi_op_abort_begin   (in stream order, ahead of a run's kernels)  word = run_id << 1 | (*host_flag != 0); host_flag: pinned host memory, nullable
  *   pi_op_abort_cancel  (any stream, any time)                        if word == run_id << 1 then word |= 1: only the run that is executing NOW is hit */
 PI_API void    pi_set_abort_word(const int32_t * word_dev);

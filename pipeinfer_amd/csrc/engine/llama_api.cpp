@@ -453,7 +453,7 @@ extern "C" void pipeinfer_reset_stats(struct llama_context * ctx) { ctx->stat_ca
     if (ctx->hop_dev && ctx->stream) { (void) hipMemsetAsync(ctx->hop_dev, 0, 64, ctx->stream); (void) hipStreamSynchronize(ctx->stream); }
     ctx->stat_flag_seen_us = 0.0; ctx->stat_flag_wait_ms = 0.0; ctx->stat_flag_runs = 0;
 }
-// launches of this context since pipeinfer_reset_stats that found their run aborted (llama_cancel_run after the start) and returned on entry, per kernel family
+// launches of this context since pipeinfer_reset_stats that found their run aborted (llama_cancel_run after the start) and returned without a result, per kernel family
 // (index = pi_kt_row.family); synchronises the context's control stream.  Returns the number of families written (<= cap), -1 on error
 extern "C" int pipeinfer_get_aborted_launches(struct llama_context * ctx, uint64_t * out, int cap) {
     const int n = std::min(cap, (int) PI_KT_NFAM);

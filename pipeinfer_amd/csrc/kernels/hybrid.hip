@@ -1058,6 +1058,7 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
         ((float *) qsh)[d * 4 + tt] = q[(int64_t) min(t0 + tt, n_tok - 1) * qs + (int64_t) h * hw + d];
     }
     __syncthreads();
+    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the queries, requested after it)
     const int dq = (dim + 3) / 4, d0 = wave * dq, d1 = min(dim, d0 + dq);
     float acc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
     const uint16_t * w = wuk + (int64_t) h * dim * rank + min(r, rank - 1);
@@ -1071,7 +1072,6 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
     for (int tt = 0; tt < 4; tt++) part[wave][tt][lane] = acc[tt];
     __syncthreads();
     const int tt = wave;                                              // wave tt writes token t0 + tt
-    if (pi_abort_late(gone, abort_w, 5)) return;
     if (t0 + tt < n_tok && r < rank) qa[((int64_t) (t0 + tt) * heads + h) * (rank + rot) + r] = (part[0][tt][lane] + part[1][tt][lane] + part[2][tt][lane] + part[3][tt][lane]) * scale;
 }
 
@@ -1257,8 +1257,9 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
     for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
     float * pml_r = pml + ((int64_t) ((int) blockIdx.x * 16 + n) * S + split) * 2;
     const bool real = (int) blockIdx.x * 16 + n < n_rows;
+    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the mask, requested after it)
     if (!some) {                                                      // (the same in every lane: the rows of a tile are the same sixteen in all four)
-        if (!pi_abort_late(gone, abort_w, 5) && tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
+        if (tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
         return;
     }
     const int spare = __ffs(some) - 1;
@@ -1310,7 +1311,6 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
         *(hy_f32x4 *) &ps[n][16 * ct + 4 * g] = p;
     }
     __syncthreads();
-    if (pi_abort_late(gone, abort_w, 5)) return;
     if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
     hy_f32x4 acc[NJ];
 #pragma unroll
@@ -1369,6 +1369,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         for (int s = lane; s < S; s += 64) { const float ms = pml_t[s * 2]; if (ms != -INFINITY) d += pml_t[s * 2 + 1] * expf(ms - mstar); }
         den = pi_lanes_sum<64>(d) + (sink ? expf(sk - mstar) : 0.0f);
     }
+    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the splits' maxima, requested after it)
     for (int sb = 0; sb < S; sb += 64) {
         __syncthreads();
         if (wave < nt) {
@@ -1408,7 +1409,6 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         }
     }
     __syncthreads();
-    if (pi_abort_late(gone, abort_w, 5)) return;
     if (vec) {
         const int v0 = blockIdx.z * 16 + wave;
         float a[4][4];
@@ -1595,6 +1595,7 @@ __global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict_
     const float * xr = x + (int64_t) t * xs;
     for (int e = wave; e < n_out; e += (int) (blockDim.x >> 6)) {
         const float a = pi_lanes_sum<64>(hy_dot_lane(router + (int64_t) e * width, xr, width, lane, exact != 0, vec != 0));
+        if (gone & 1) break;                                           // (no further outputs for a cancelled run)
         if (lane == 0) z[e] = a;
     }
     __syncthreads();

@@ -498,6 +498,7 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
     const float M = pi_wave_max(ms_l);
     const float f_l = ms_l != -INFINITY ? expf(ms_l - M) : 0.0f;
     const float den = pi_lanes_sum<64>(f_l > 0.0f ? pr[(int64_t) lane * (V + 2) + V + 1] * f_l : 0.0f);
+    if (pi_abort_late(gone, abort_w)) return;
     for (int v0 = 0; v0 < V; v0 += 64) {
         const int v = v0 + lane;
         float a = 0.0f;
@@ -514,7 +515,6 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
         if (v < V) maps_lds[map * V + v] = den > 0.0f ? a / den : 0.0f;
     }
     __syncthreads();
-    if (pi_abort_late(gone, abort_w)) return;
     if (map == 0) ca_join_maps(maps_lds, maps_lds + V, V, mp, out_mult, out + (int64_t) t * os + (int64_t) h * V, lane);
 }
 // cell splits of a pass of n_tok tokens over n_kv cells: how many, and the floats of scratch they need (0 splits: the pass is wide enough to fill the device by itself)

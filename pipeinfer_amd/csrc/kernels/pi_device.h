@@ -79,7 +79,7 @@ static __device__ __forceinline__ float pi_wave_max(float v) {
 // weights look at the value only after their first loads are in flight (vmcnt retires in order, so the wait costs them nothing).
 static __device__ __forceinline__ int pi_abort_peek(const int32_t * w) { return w ? __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0; }
 // The word is the first int32 of a 64-byte block (include/pipeinfer_ops.h): words 8..14 count, per kernel family (kernel_timing.h: pi_kt_family), the LAUNCHES that found
-// the run aborted and returned — one thread of a launch adds one, on the abort path only.  bench.py's roofline keeps those launches apart from the ones that did the work.
+// the run aborted and returned without a result — one thread of a launch adds one, on the abort path only.  bench.py's roofline keeps those launches apart from the ones that did the work.
 static __device__ __forceinline__ void pi_abort_note(const int32_t * w, int fam) {
     if ((threadIdx.x | threadIdx.y | threadIdx.z | blockIdx.x | blockIdx.y | blockIdx.z) == 0)
         __hip_atomic_fetch_add(const_cast<int32_t *>(w) + 8 + fam, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -90,7 +90,9 @@ static __device__ __forceinline__ bool pi_aborted(const int32_t * w, int fam = 6
     return true;
 }
 
-// the same for a small launch, whose own loads take no longer than the word's: requested at the top (pi_abort_peek), looked at just ahead of the first store (a trip to memory of its own at the top: 0.3 us of 3.4)
+// the same for a launch that asks for the word at the top (pi_abort_peek) and goes on loading (a trip to memory of its own at the top: 0.3 us of 3.4).  A kernel of one trip to memory looks at it ahead of its first
+// store; one that streams weights, walks cells or loops over its values looks once its first loads are on their way, ahead of the loop, so that a cancelled run costs it no more than those.  What such a kernel
+// takes an address from before it has looked comes from the pass's own inputs: a launch before it in a cancelled run may have written nothing
 static __device__ __forceinline__ bool pi_abort_late(int peek, const int32_t * w, int fam = 6) {
     if ((peek & 1) == 0) return false;
     pi_abort_note(w, fam);

@@ -389,6 +389,7 @@ __global__ void __launch_bounds__(256) k_few_attention(const pa_args A, int n_cs
         bool see = false;
         if (mc < c_end) { const int cp = A.cell_pos[mc]; see = (A.mask[(int64_t) t * words + (c0 >> 5)] >> (lane & 31) & 1u) && (cp >= first || cp < A.keep_first); }
         const uint32_t vis = (uint32_t) __ballot(see);
+        if (gone & 1) break;                                          // (a cancelled run: its keys and values are not read)
         if (!vis) continue;
         pa_f32x4 kf[STEPS]; vec vf[2][4];
         {

@@ -755,7 +755,7 @@ def test_two_weight_types_share_one_matrix_core_launch(gpu, types, k, n_tok, n_h
 
 def test_abort_word_stops_kernels_of_the_cancelled_run_only(gpu):
     """Kernel-granular early cancellation (reference: the abort callback polled between graph nodes, ggml.c:15748-15811, llama.cpp:5665-5687): every hot-path
-    kernel launched under pi_set_abort_word reads (run id << 1 | aborted) on entry.  pi_op_abort_cancel is a compare-and-swap on the run id: it stops the run that
+    kernel launched under pi_set_abort_word asks for (run id << 1 | aborted) on entry and writes nothing once it is aborted.  pi_op_abort_cancel is a compare-and-swap on the run id: it stops the run that
     is executing, never another one; a run that is not aborted computes the oracle's bits."""
     from pipeinfer_amd import lib as L
     lib, U = gpu
@@ -765,7 +765,7 @@ def test_abort_word_stops_kernels_of_the_cancelled_run_only(gpu):
     act = rng.standard_normal((n_tok, k)).astype(np.float32)
     want = O.Impl("oracle").mul_mat(t, blocks, k, rows, act)
     w = upload_weight(lib, t, rows, k, blocks)
-    word = U.Dev(np.zeros(16, np.int32))                               # the abort block: word 0 = (run id << 1 | aborted), words 8..14 = launches aborted on entry, per kernel family
+    word = U.Dev(np.zeros(16, np.int32))                               # the abort block: word 0 = (run id << 1 | aborted), words 8..14 = launches that returned without a result, per kernel family
     xd = U.Dev(act)
     sentinel = np.full((n_tok, rows), 12345.0, np.float32)
 

@@ -102,3 +102,39 @@ def test_weights_of_a_prompt(H, G, D, V, chunk, n_kv, T, softcap):
             fine = np.isfinite(want)
             assert np.array_equal(fine, np.isfinite(got)) and np.array_equal(got[~fine], want[~fine].astype(np.float32)) and (fine.all() or (loud and hurt.any()))
             assert rel_rms(np.where(fine, got, 0), np.where(fine, want, 0)) < 1e-5, (weights, loud)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 3, 40])
+def test_launches_of_a_cancelled_run(T):
+    """kernels that ask for the abort word and go on loading: a run that is cancelled ahead of them writes neither results nor partial sums, and every launch is counted once (a single token, a few, a prompt)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(T)
+    H, G, D, V, rank, E, top, n_kv = 4, 2, 64, 64, 256, 5, 2, 300
+    word = U.Dev(np.zeros(16, np.int32))
+    f = lambda *shape: U.Dev(rng.standard_normal(shape).astype(np.float32))
+    w = lambda n, k: fasovik.upload_bf16(lib, fasovik.bf(rng, n, k, s=0.1))
+    q, kc, vc, cache, x = f(T, H * 2 * D), f(n_kv, G, 2 * D), f(n_kv, G, V), f(n_kv, rank), f(T, rank)
+    pos, cpos, mask = U.Dev(np.arange(n_kv - T, n_kv, dtype=np.int32)), U.Dev(np.arange(n_kv, dtype=np.int32)), U.Dev(pack_mask(np.ones((T, n_kv), bool), n_kv))
+    dyn, hb, uk, uv, router, corr = U.Dev(np.array([0, n_kv, T, 0], np.int32)), f(H), w(H * D, rank), w(H * V, rank), w(E, rank), f(E)
+    n_scr = max(lib.pi_op_window_attention_scratch_floats(2 * H, V, T), lib.pi_op_latent_attention_rot_scratch_floats(H, rank, 0, max(T, 8), n_kv))
+    out, scr, sel = U.Dev(np.full((T, H * V), 555.0, np.float32)), U.Dev(np.full(n_scr, 777.0, np.float32)), U.Dev(np.full(T * top, 333, np.int32))
+    calls = {
+        "differential heads": lambda: lib.pi_op_diff_attention(q.ptr, 2 * H * D, kc.ptr, vc.ptr, cpos.ptr, mask.ptr, pos.ptr, 0.1, 0, 0, 2, 0.4, 1.0, 1e-5, H, G, D, V, T, n_kv, scr.ptr, n_scr, out.ptr, H * V, dyn.ptr, None),
+        "window": lambda: lib.pi_op_window_attention(q.ptr, H * D, kc.ptr, vc.ptr, cpos.ptr, mask.ptr, pos.ptr, hb.ptr, None, None, 0, 0, 0.1, 1.0, 1, 0.0, CHUNK, 0, 0, 0, 0, H, G, D, V, T, n_kv, scr.ptr, n_scr, out.ptr, H * V,
+                                                     dyn.ptr, None),
+        "latent": lambda: lib.pi_op_latent_attention(q.ptr, H * D, cache.ptr, mask.ptr, uk, uv, hb.ptr, 0.1, H, D, V, rank, T, n_kv, scr.ptr, n_scr, out.ptr, H * V, dyn.ptr, None),
+        "router": lambda: lib.pi_op_moe_route(router, corr.ptr, x.ptr, rank, T, top, 0, sel.ptr, out.ptr, None),
+    }
+    L.check(lib.pi_op_abort_begin(word.ptr, 3, None, None))
+    L.check(lib.pi_op_abort_cancel(word.ptr, 3, None))
+    for name, call in calls.items():
+        before = word.get(np.int32)[8:15].sum()
+        lib.pi_set_abort_word(word.ptr)
+        try:
+            L.check(call())
+        finally:
+            lib.pi_set_abort_word(None)
+        assert np.all(out.get(np.float32) == 555.0) and np.all(scr.get(np.float32) == 777.0) and np.all(sel.get(np.int32) == 333), name
+        launches = {"differential heads": 1 if T >= 32 else 2, "window": 1 if T >= 32 else 2, "latent": 2 if T > 8 else 3, "router": 1}[name]
+        assert word.get(np.int32)[8:15].sum() - before == launches, name
