@@ -1312,6 +1312,21 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
     }
     __syncthreads();
     if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
+    // an infinity or a NaN must not meet the zero weight of a row that does not see its cell (rows of several tokens share a tile, a cell that nobody sees repeats another): it joins at the end
+    bool odd = false;
+    if (__any(vis != 0xffffffffu)) {
+        uint32_t big = 0;
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) big = max(big, __float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu);
+        odd = __any(big >= 0x7f800000u);
+        if (odd)
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[i >> 2][i & 3][j >> 2][j & 3] = 0.0f;
+    }
     hy_f32x4 acc[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
@@ -1324,6 +1339,15 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
             for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
     }
     if (!real || vis == 0) return;
+    if (odd)
+        for (int c = 0; c < 32; c++) {
+            if (!(vis >> c & 1u)) continue;
+            const float * row = cache + cell(c) * (uint32_t) W + wave * (RANK / 4) + NJ * 4 * g;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) if ((__float_as_uint(row[NJ * r + j]) & 0x7fffffffu) >= 0x7f800000u) acc[j][r] += row[NJ * r + j];
+        }
     float * o = pol + ((int64_t) row * S + split) * RANK + wave * (RANK / 4);
 #pragma unroll
     for (int r = 0; r < 4; r++)

@@ -41,6 +41,20 @@ def test_latent_few_tokens_over_scattered_cells(H, rank, T, n_kv):
     fasovik.test_latent_attention_against_explicit_keys_and_values(H, 16, 24, rank, T, n_kv)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,R,rank,T,n_kv", [(6, 4, 256, 5, 70), (16, 0, 512, 3, 33), (3, 0, 256, 8, 200), (5, 64, 512, 4, 64), (6, 4, 64, 12, 90)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_latents_that_are_no_numbers(H, R, rank, T, n_kv, bad):
+    """rows of several tokens share a tile, and some of them see a latent that is no number: it reaches those and no others"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H * 100 + n_kv)
+    cache = rng.standard_normal((n_kv, rank + R)).astype(np.float32)
+    cache[n_kv - 2, 1] = bad
+    with np.errstate(invalid="ignore"):
+        got, want = latent_case(U, lib, rng, H, 8, R, 12, rank, n_kv, np.arange(n_kv - T, n_kv), 500.0, HALVES, 12, None, (8 + R) ** -0.5, cache=cache)
+    assert rel_rms(got[:-2], want[:-2]) < 1e-5 and not np.isfinite(got[-2:]).any()
+
+
 def scattered(rng, T, n_kv, n_ctx):
     """positions of cells in any order, tokens' positions, what the mask shows (a token sees at least itself)"""
     cpos = rng.permutation(n_ctx).astype(np.int32)
