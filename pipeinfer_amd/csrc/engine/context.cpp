@@ -296,32 +296,48 @@ static pi_run * acquire_run(llama_context * ctx, int n_tokens, int rows, size_t 
     }
     auto host_alloc = [&](void ** p, size_t bytes) { if (r->host_plain) { *p = malloc(bytes); return *p != nullptr; } return hipHostMalloc(p, bytes, hipHostMallocDefault) == hipSuccess; };
     auto host_free = [&](void * p) { if (r->host_plain) free(p); else (void) hipHostFree(p); };
-    const size_t need = ctx->is_last ? (size_t) rows * ctx->model->hparams.n_vocab : 0;
-    // (the buffer that the caller read the last run's rows in comes back where those rows are not read any more: such callers never pay for a second one)
-    if (need > r->logits_cap && until_done && ctx->logits_own_cap >= need) { std::swap(ctx->logits_own, r->logits_host); std::swap(ctx->logits_own_cap, r->logits_cap); }
-    if (need > r->logits_cap) {
-        if (r->logits_host) host_free(r->logits_host);
-        r->logits_host = nullptr; r->logits_cap = 0;
-        const size_t cap = std::max(need, (size_t) 16 * ctx->model->hparams.n_vocab);
-        if (!host_alloc((void **) &r->logits_host, cap * 4)) { r->logits_host = nullptr; ctx->pool.push_back(r); return nullptr; }
-        r->logits_cap = cap;
-    }
+    r->lent = false;
+    auto none = [&]() -> pi_run * { ctx->pool.push_back(r); return nullptr; };
     if (ctx->is_last && n_tokens > r->topk_rows) {                             // (apart from the rows: a finished run's logits buffer may go to the caller)
         if (r->topk_ids) host_free(r->topk_ids);
         r->topk_ids = nullptr; r->topk_rows = 0;
         const size_t rows = (size_t) std::max(n_tokens, 16);
-        if (!host_alloc((void **) &r->topk_ids, rows * (8 * 4 + 8 * 4 + 4))) { r->topk_ids = nullptr; ctx->pool.push_back(r); return nullptr; }
+        if (!host_alloc((void **) &r->topk_ids, rows * (8 * 4 + 8 * 4 + 4))) { r->topk_ids = nullptr; return none(); }
         r->topk_vals = (float *) (r->topk_ids + rows * 8);
         r->topk_sum  = r->topk_vals + rows * 8;
         r->topk_rows = (int) rows;
     }
     if (meta_bytes > r->meta_cap) {
         if (r->meta_host) host_free(r->meta_host);
-        r->meta_cap = std::max(meta_bytes, (size_t) 4096);
-        if (!host_alloc((void **) &r->meta_host, r->meta_cap)) return nullptr;
+        r->meta_host = nullptr; r->meta_cap = 0;
+        const size_t cap = std::max(meta_bytes, (size_t) 4096);
+        if (!host_alloc((void **) &r->meta_host, cap)) { r->meta_host = nullptr; return none(); }
+        r->meta_cap = cap;
+    }
+    const size_t need = ctx->is_last ? (size_t) rows * ctx->model->hparams.n_vocab : 0;
+    // (the buffer that the caller read the last run's rows in comes back where those rows are not read any more: such callers never pay for a second one.  Behind everything else that can fail; take_back for what
+    // can fail later)
+    if (need > r->logits_cap && until_done && ctx->logits_own_cap >= need) {
+        r->lent = ctx->logits_out && ctx->logits_out == ctx->logits_own;
+        if (r->lent) ctx->logits_out = nullptr;
+        std::swap(ctx->logits_own, r->logits_host); std::swap(ctx->logits_own_cap, r->logits_cap);
+    }
+    if (need > r->logits_cap) {
+        if (r->logits_host) host_free(r->logits_host);
+        r->logits_host = nullptr; r->logits_cap = 0;
+        const size_t cap = std::max(need, (size_t) 16 * ctx->model->hparams.n_vocab);
+        if (!host_alloc((void **) &r->logits_host, cap * 4)) { r->logits_host = nullptr; return none(); }
+        r->logits_cap = cap;
     }
     r->canceled = r->launched = r->finished = r->failed = false;
     return r;
+}
+// a run that wrote no rows: the ones that were to be read before it are to be read again
+static void take_back(llama_context * ctx, pi_run * r) {
+    if (!r->lent) return;
+    std::swap(ctx->logits_own, r->logits_host); std::swap(ctx->logits_own_cap, r->logits_cap);
+    ctx->logits_out = ctx->logits_own;
+    r->lent = false;
 }
 
 // ---- the forward pass of this stage: layers [l0, l1) ----------------------------------------------------------------------
@@ -1436,7 +1452,8 @@ pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & 
     const bool compact = !all_rows && !ctx->remote && !outputs_by_memcpy() && ranges <= 8;
     pi_run * run = acquire_run(ctx, n_tokens, compact ? wanted : n_tokens, meta_bytes, until_done);
     // (a run that cannot be started gives the cells find_slot just allotted back: nothing was or will be written to them)
-    auto give_back = [&]() { ctx->cells->release_cells(kv_head, n_tokens); for (int sl : fresh_taken) ctx->slots->mark_fresh(sl); for (auto it = last_before.rbegin(); it != last_before.rend(); ++it) ctx->slots->set_last_token(it->first, it->second); };
+    bool rows_written = false;                                                 // whether anything may write the run's rows yet
+    auto give_back = [&]() { if (run && !rows_written) take_back(ctx, run); ctx->cells->release_cells(kv_head, n_tokens); for (int sl : fresh_taken) ctx->slots->mark_fresh(sl); for (auto it = last_before.rbegin(); it != last_before.rend(); ++it) ctx->slots->set_last_token(it->first, it->second); };
     if (!run) { ctx->last_error = "out of pinned host memory"; give_back(); return nullptr; }
     run->batch_id = batch_in.batch_id; run->n_tokens = n_tokens; run->t_start_us = time_us(); run->sink = nullptr;
     run->run_id = (++ctx->run_counter) & 0x3fffffff; run->kv_head = kv_head; run->n_kv = n_kv;
@@ -1499,7 +1516,7 @@ pi_run * context_start(llama_context * ctx, const llama_batch & batch_in, int & 
     }
     if (!run->canceled) {                                                     // a cancelled run still occupies its cells and completes "empty" (llama.cpp:5627-5716)
         ok = launch_forward(ctx, n_tokens, run->meta_host, nullptr, &run->sink, !run->host_plain, run);
-        if (ok) ok = launch_outputs(ctx, run);
+        if (ok) { rows_written = true; ok = launch_outputs(ctx, run); }
         run->launched = ok;
     }
     if (ok) ok = hipEventRecord(run->done, ctx->stream) == hipSuccess;
@@ -1790,6 +1807,7 @@ int stage_run_pass(llama_context * ctx, int n_members, const void * const * meta
 
 int context_finish(llama_context * ctx, pi_run * run) {
     if (!run) return -1;
+    bool written = false;                                                      // whether the run wrote rows, results or not
     if (ctx->remote) {
         if (run->launched) {
             const int rc = ctx->remote_ops.wait(ctx->remote_ops.user, run->run_seq, run->logits_host, run->topk_ids, run->topk_vals, run->topk_sum);
@@ -1833,8 +1851,11 @@ int context_finish(llama_context * ctx, pi_run * run) {
                 if (run->pass_tokens == run->n_tokens && hipEventElapsedTime(&ms, run->begin, run->done) == hipSuccess) ctx->stat_cancel_gpu_ms += ms;
             }
         }
+        written = run->launched;
         if (cut) run->launched = false;
     }
+    if (!run->launched && !written) take_back(ctx, run);
+    run->lent = false;
     const size_t nv = ctx->model->hparams.n_vocab;
     const int n = run->n_tokens;
     if (ctx->run_tap) ctx->run_tap(ctx->run_tap_user, run->run_id, run->batch_id, n, run->meta_host, run->meta_bytes, run->launched && ctx->is_last && !run->canceled && run->all_rows ? run->logits_host : nullptr);
@@ -1846,12 +1867,18 @@ int context_finish(llama_context * ctx, pi_run * run) {
         if (take) { std::swap(ctx->logits_own, run->logits_host); std::swap(ctx->logits_own_cap, run->logits_cap); ctx->logits_out = ctx->logits_own; }
         else {                                                                 // llama.cpp:5734-5743
             const size_t size = run->last_only ? nv : (size_t) n * nv;
-            if (size > ctx->logits_size) {                                     // (zeros that cost nothing until somebody reads them: a prompt's caller looks at its last row)
-                float * bigger = (float *) calloc(size, 4);
-                if (!bigger) { ctx->last_error = "out of host memory (logits)"; run->launched = false; }
-                else { if (ctx->logits) memcpy(bigger, ctx->logits, ctx->logits_size * 4); free(ctx->logits); ctx->logits = bigger; ctx->logits_size = size; }
+            const bool own = ctx->logits_out && ctx->logits_out == ctx->logits_own;
+            // (no result: the rows of the run before stay where they are, unless the buffer has to be longer)
+            if (run->launched || !own || size > ctx->logits_own_cap) {
+                const float * keep = own && !run->launched ? ctx->logits_own : ctx->logits;
+                const size_t n_keep = own && !run->launched ? ctx->logits_own_cap : ctx->logits_size;
+                if (size > ctx->logits_size || keep != ctx->logits) {          // (zeros that cost nothing until somebody reads them: a prompt's caller looks at its last row)
+                    float * bigger = (float *) calloc(std::max(size, n_keep), 4);
+                    if (!bigger) { ctx->last_error = "out of host memory (logits)"; run->launched = false; }
+                    else { if (keep) memcpy(bigger, keep, n_keep * 4); free(ctx->logits); ctx->logits = bigger; ctx->logits_size = std::max(size, n_keep); }
+                }
+                ctx->logits_out = size <= ctx->logits_size ? ctx->logits : nullptr;
             }
-            ctx->logits_out = size <= ctx->logits_size ? ctx->logits : nullptr;
         }
         if (run->launched) {
             const float * from = run->logits_host;

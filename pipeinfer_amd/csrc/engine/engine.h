@@ -244,6 +244,7 @@ struct pi_run {                                // one llama_start_async_decode .
     bool all_rows = false;                    // every row comes back to logits_host, not only the wanted ones (a run tap was set when the run was started)
     int32_t * topk_ids = nullptr; float * topk_vals = nullptr; float * topk_sum = nullptr;   // pinned [topk_rows][8], [topk_rows]
     int topk_rows = 0;
+    bool lent = false;                        // logits_host holds the rows that llama_get_logits showed before this run (context_start of a synchronous decode): they go back where the run writes none
     uint8_t * meta_host = nullptr; size_t meta_cap = 0;                                       // pinned staging for tokens/pos/mask
     int64_t t_start_us = 0;
     pi_kt_sink * sink = nullptr;            // kernel-timing samples of the graph this run replayed
