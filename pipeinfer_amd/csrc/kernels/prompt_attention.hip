@@ -177,9 +177,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                     top = fmaxf(top, __shfl_xor(top, 16, 64)); top = fmaxf(top, __shfl_xor(top, 32, 64));
                     const float m_new = fmaxf(m_run[u], top);
                     const float f = m_run[u] == m_new ? 1.0f : expf(m_run[u] - m_new);            // (nothing seen yet: expf(-inf) = 0, or both -inf)
+                    const float from = m_new == -INFINITY ? 0.0f : m_new;                         // (scores of minus infinity alone: no weight, not a NaN)
                     float sum = 0.0f;
 #pragma unroll
-                    for (int c = 0; c < 4; c++) { const float e = mine >> c & 1u ? expf(s[u][c] - m_new) : 0.0f; s[u][c] = e; sum += e; }
+                    for (int c = 0; c < 4; c++) { const float e = mine >> c & 1u ? expf(s[u][c] - from) : 0.0f; s[u][c] = e; sum += e; }
                     l_run[u] = fmaf(l_run[u], f, sum); m_run[u] = m_new;                          // (a lane's own cells; the four of a query meet at the end)
                     if (__any(f != 1.0f))
 #pragma unroll
@@ -428,17 +429,18 @@ __global__ void __launch_bounds__(256) k_few_attention(const pa_args A, int n_cs
             if (scores && g == 0) top[map][ct][n] = m;
             __syncthreads();
         }
-        float m_new[MAPS], f[MAPS];
+        float m_new[MAPS], f[MAPS], from[MAPS];
 #pragma unroll
         for (int mp = 0; mp < MAPS; mp++) {
             m_new[mp] = soft ? fmaxf(m_run[mp], fmaxf(top[mp][0][n], top[mp][1][n])) : 0.0f;
             f[mp] = !soft || m_run[mp] == m_new[mp] ? 1.0f : expf(m_run[mp] - m_new[mp]);
             m_run[mp] = m_new[mp];
+            from[mp] = m_new[mp] == -INFINITY ? 0.0f : m_new[mp];     // (scores of minus infinity alone: no weight, not a NaN)
         }
         if (scores) {
             float l = 0.0f;
 #pragma unroll
-            for (int c = 0; c < 4; c++) { const float e = !(mine >> c & 1u) ? 0.0f : soft ? expf(s[c] - m_new[map]) : 1.0f / (1.0f + expf(-s[c])); s[c] = e; l += e; }
+            for (int c = 0; c < 4; c++) { const float e = !(mine >> c & 1u) ? 0.0f : soft ? expf(s[c] - from[map]) : 1.0f / (1.0f + expf(-s[c])); s[c] = e; l += e; }
             l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
             if (g == 0) sum[map][ct][n] = l;
             *(pa_f32x4 *) &ps[map][n][16 * ct + 4 * g] = s;

@@ -152,3 +152,26 @@ def test_launches_of_a_cancelled_run(T):
         assert np.all(out.get(np.float32) == 555.0) and np.all(scr.get(np.float32) == 777.0) and np.all(sel.get(np.int32) == 333), name
         launches = {"differential heads": 1 if T >= 32 else 2, "window": 1 if T >= 32 else 2, "latent": 2 if T > 8 else 3, "router": 1}[name]
         assert word.get(np.int32)[8:15].sum() - before == launches, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n_kv", [(40, 300), (33, 64), (2, 1100), (8, 200)])
+@pytest.mark.parametrize("maps", [1, 2])
+def test_scores_of_minus_infinity(T, n_kv, maps):
+    """cells whose scores overflow to minus infinity have no weight, wherever they lie: at the start of every wave's and every split's range, or in all of it; a token that sees nothing else gets zeros"""
+    U, lib = gpu()
+    H, G, D, V = 4, 2, 64, 64
+    rng = np.random.default_rng(n_kv + T)
+    q = np.abs(rng.standard_normal((T, H, maps, D))).astype(np.float32) + 0.1
+    kc, vc = rng.standard_normal((n_kv, G, maps, D)).astype(np.float32), rng.standard_normal((n_kv, G, V)).astype(np.float32)
+    far = (np.arange(n_kv) % 64 < 32) & (np.arange(n_kv) < n_kv - T)
+    kc[far] = -3e38
+    cpos, pos, vis = np.arange(n_kv, dtype=np.int32), np.arange(n_kv - T, n_kv, dtype=np.int32), np.arange(n_kv)[None, :] <= np.arange(n_kv - T, n_kv)[:, None]
+    vis[T - 1] = far
+    args = [vis, pos, 3.0, 0, 0, maps, 0.45, 0.7, 1e-3, H, G]
+    got = run_diff(U, lib, q, kc, vc, cpos, *args, True)
+    near = ~far
+    args[0] = vis[:T - 1][:, near]
+    args[1] = pos[:T - 1]
+    want = diff_attention_ref(q[:T - 1], kc[near], vc[near], cpos[near], *args)
+    assert rel_rms(got[:T - 1], want) < 1e-5 and np.all(got[T - 1] == 0.0)
