@@ -501,7 +501,8 @@ extern "C" int pi_op_sum_tanh_norm_shift(const float * x, int64_t x_stride, cons
 #define LA_TB 32                                  // tokens of a piece; q, k and v of a piece are staged in LDS
 #define LA_FRESH (1 << 30)
 #define LA_MAXRUNS 256                            // sequences a pass may carry (the host checks)
-// the first tokens of the pass's runs, in order (every thread of the block calls; bnd / nb in LDS): a thread looks at its own tokens only, one thread sorts the few it found
+// the first tokens of the pass's runs, in order (every thread of the block, 64 at least, calls; bnd / nb in LDS): a thread looks at its own tokens only, then every run finds its place by counting the ones ahead of
+// it.  (One thread that sorted them: with 64 runs 200 us and more of every launch, 16 heads of 64 x 64, 96 tokens: 719 us for the three, now 75)
 static __device__ __forceinline__ int la_runs(const int * recs, int n_tok, int * bnd, int * nb) {
     if (threadIdx.x == 0) *nb = 0;
     __syncthreads();
@@ -509,25 +510,50 @@ static __device__ __forceinline__ int la_runs(const int * recs, int n_tok, int *
         if (t == 0 || (recs[t] & ~LA_FRESH) != (recs[t - 1] & ~LA_FRESH)) { const int k = atomicAdd(nb, 1); if (k < LA_MAXRUNS) bnd[k] = t; }
     __syncthreads();
     const int n = min(*nb, LA_MAXRUNS);
-    if (threadIdx.x == 0)
-        for (int i = 1; i < n; i++) { const int v = bnd[i]; int j = i - 1; while (j >= 0 && bnd[j] > v) { bnd[j + 1] = bnd[j]; j--; } bnd[j + 1] = v; }
+    if (n > 1) {
+        int at[LA_MAXRUNS / 64], v[LA_MAXRUNS / 64];
+#pragma unroll
+        for (int k = 0; k < LA_MAXRUNS / 64; k++) {
+            const int i = threadIdx.x + k * blockDim.x;
+            at[k] = 0;
+            if (i < n) { v[k] = bnd[i]; for (int o = 0; o < n; o++) at[k] += bnd[o] < v[k]; }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < LA_MAXRUNS / 64; k++) if ((int) (threadIdx.x + k * blockDim.x) < n) bnd[at[k]] = v[k];
+    }
     __syncthreads();
     return n;
 }
-// piece number `want` of the pass (lseg = 0: pieces are whole runs): first token, length, slot word, whether it is its run's last piece
-static __device__ __forceinline__ bool la_find_piece(const int * recs, int n_tok, const int * bnd, int n_runs, int lseg, int want, int & first, int & len, int & word, int & last) {
-    int ord = 0;
-    for (int r = 0; r < n_runs; r++) {
-        const int t = bnd[r], e = r + 1 < n_runs ? bnd[r + 1] : n_tok;
-        const int nsub = lseg > 0 ? (e - t + lseg - 1) / lseg : 1;
-        if (want < ord + nsub) {
-            const int p = want - ord;
-            first = lseg > 0 ? t + p * lseg : t; len = lseg > 0 ? min(lseg, e - first) : e - t; word = recs[t]; last = p == nsub - 1;
-            return true;
-        }
-        ord += nsub;
+// The pieces of lseg tokens (0: pieces are whole runs) that lie ahead of a lane's four runs (the first wave calls; run 4 lane + k has own[k])
+static __device__ __forceinline__ int la_pieces_before(const int * bnd, int n_runs, int n_tok, int lseg, int (&own)[4]) {
+    const int lane = threadIdx.x;
+    int sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int r = 4 * lane + k;
+        own[k] = r >= n_runs ? 0 : lseg > 0 ? ((r + 1 < n_runs ? bnd[r + 1] : n_tok) - bnd[r] + lseg - 1) / lseg : 1;
+        sum += own[k];
     }
-    return false;
+    int upto = sum;
+    if (n_runs > 4)
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int x = __shfl_up(upto, o, 64); if (lane >= o) upto += x; }
+    return upto - sum;
+}
+static_assert(LA_MAXRUNS <= 4 * 64, "four runs to a lane");
+// piece number `want` of the pass into seg (LDS; the first wave calls): first token, length (0: there is none), slot word, whether it is its run's last piece
+static __device__ __forceinline__ void la_find_piece(const int * recs, int n_tok, const int * bnd, int n_runs, int lseg, int want, int * seg) {
+    int own[4], ord = la_pieces_before(bnd, n_runs, n_tok, lseg, own);
+    if (threadIdx.x == 0) { seg[0] = 0; seg[1] = 0; seg[2] = -1; seg[3] = 1; }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        if (want >= ord && want < ord + own[k]) {
+            const int r = 4 * (int) threadIdx.x + k, t = bnd[r], e = r + 1 < n_runs ? bnd[r + 1] : n_tok, p = want - ord, first = lseg > 0 ? t + p * lseg : t;
+            seg[0] = first; seg[1] = lseg > 0 ? min(lseg, e - first) : e - t; seg[2] = recs[t]; seg[3] = p == own[k] - 1;
+        }
+        ord += own[k];
+    }
 }
 template <int DPT>
 __global__ void __launch_bounds__(256) k_linear_attention(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int dim, int vdim, int vstored, int R,
@@ -545,11 +571,7 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
     for (int t = tid; t < n_tok; t += blockDim.x) recs[t] = rec[t];
     __syncthreads();
     const int n_runs = la_runs(recs, n_tok, bnd, &nbnd);
-    if (tid == 0) {
-        int first = 0, len = 0, word = -1, last = 1;
-        if (!la_find_piece(recs, n_tok, bnd, n_runs, mode ? LA_TB : 0, blockIdx.z, first, len, word, last)) len = 0;
-        seg[0] = first; seg[1] = len; seg[2] = word; seg[3] = last;
-    }
+    if (tid < 64) la_find_piece(recs, n_tok, bnd, n_runs, mode ? LA_TB : 0, blockIdx.z, seg);
     }
     __syncthreads();
     const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
@@ -660,11 +682,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
     for (int t = tid; t < n_tok; t += 256) lm_recs[t] = rec[t];
     __syncthreads();
     const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
-    if (tid == 0) {
-        int first = 0, len = 0, word = -1, last = 1;
-        if (!la_find_piece(lm_recs, n_tok, bnd, n_runs, LM_TB, blockIdx.y, first, len, word, last)) len = 0;
-        seg[0] = first; seg[1] = len; seg[2] = word; seg[3] = last;
-    }
+    if (tid < 64) la_find_piece(lm_recs, n_tok, bnd, n_runs, LM_TB, blockIdx.y, seg);
     __syncthreads();
     const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
     if (len == 0 || word < 0 || (!OUTPUTS && last)) return;
@@ -844,15 +862,15 @@ __global__ void __launch_bounds__(256) k_linear_state_scan(int heads, int dim, i
     for (int t = threadIdx.x; t < n_tok; t += 256) recs[t] = rec[t];
     __syncthreads();
     const int n_runs = la_runs(recs, n_tok, bnd, &nbnd);
-    if (threadIdx.x == 0) {
-        int ord = 0, nsub = 0, word = -1, sub0 = 0, tfirst = 0;
-        for (int r = 0; r < n_runs; r++) {
-            const int t = bnd[r], e = r + 1 < n_runs ? bnd[r + 1] : n_tok;
-            const int ns = (e - t + TB - 1) / TB;
-            if (r == (int) blockIdx.z) { nsub = ns; word = recs[t]; sub0 = ord; tfirst = t; break; }
-            ord += ns;
+    if (threadIdx.x < 64) {
+        int own[4], ord = la_pieces_before(bnd, n_runs, n_tok, TB, own);
+        if (threadIdx.x == 0) seg[2] = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int r = 4 * (int) threadIdx.x + k;
+            if (r == (int) blockIdx.z && r < n_runs) { seg[0] = recs[bnd[r]]; seg[1] = ord; seg[2] = own[k]; seg[3] = bnd[r]; }
+            ord += own[k];
         }
-        seg[0] = word; seg[1] = sub0; seg[2] = nsub; seg[3] = tfirst;
     }
     __syncthreads();
     const int word = seg[0], sub0 = seg[1], nsub = seg[2], tfirst = seg[3];
@@ -958,7 +976,7 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
                                     state_dev, rec_dev, n_tok, SCR, out, out_stride, pi_abort_word())
 #define LM_ANY(OUT, SCR) do { if (dim == 32) LM_GO(1, OUT, SCR); else if (dim == 64) LM_GO(2, OUT, SCR); else if (dim == 96) LM_GO(3, OUT, SCR); else LM_GO(4, OUT, SCR); } while (0)
     // Up to 64 tokens every run is one piece: one launch from the slots' states to the slots' states.  Beyond LA_TB always (32 heads of 128 x 128, three launches against it: a run of 64 tokens 55 -> 48 us, 64 runs of a
-    // token 1115 -> 150, for the scan looked for its run in every workgroup); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
+    // token 450 -> 123, for the pieces are walked twice and the scan starts for every run); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
     // (24 tokens 53 -> 29, 9 about even; eight runs of a token or two 14 .. 18, here 25 .. 29)
     if (matrix && n_tok <= LM_TB && (pieces || n_tok > 8 * gr)) {
         const dim3 pg((unsigned) heads, gr);

@@ -361,6 +361,29 @@ def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_
     run([0 | F] + [0] * 40 + [2] * 2, hurt=9)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 24])
+@pytest.mark.parametrize("lengths", [[1] * 5, [1] * 30, [2, 1, 3] * 40, [1] * 255 + [70], [1] * 3 + [130] + [1, 2] * 35 + [64, 65]])
+def test_linear_attention_of_many_sequences(D, lengths):
+    """up to 256 sequences in a pass, more than a wave has lanes and fewer than four: every piece finds its run (pieces of a wave on the matrix cores and of the walk)"""
+    U, lib = gpu()
+    H, V, F, slots = 2, 16, 1 << 30, len(lengths)
+    rng = np.random.default_rng(slots + D)
+    order = rng.permutation(slots)
+    rec = np.concatenate([[s | (F if s % 3 == 0 else 0)] + [s] * (n - 1) for s, n in zip(order, lengths)]).astype(np.int32)
+    T, stride = len(rec), 2 * H * D + H * V
+    buf, state, decay = (rng.standard_normal((T, stride)) * 0.5).astype(np.float32), rng.standard_normal((slots, H, D, V)).astype(np.float32), np.linspace(0.5, 0.99, H).astype(np.float32)
+    n = lib.pi_op_linear_attention_scratch_floats(H, D, V, T, slots)
+    bd, rd, dd, sd, od, scr = U.Dev(buf), U.Dev(rec), U.Dev(decay), U.Dev(state), U.Dev(nbytes=4 * T * H * V), U.Dev(np.full(max(n, 1), np.nan, np.float32))
+    L.check(lib.pi_op_linear_attention(bd.ptr, bd.ptr + 4 * H * D, bd.ptr + 8 * H * D, stride, H, D, V, dd.ptr, sd.ptr, rd.ptr, T, slots, scr.ptr, n, od.ptr, H * V, None))
+    got, gs, at = od.get(np.float32, (T, H, V)), sd.get(np.float32, state.shape), 0
+    for s, n in zip(order, lengths):
+        q, k, v = (buf[at:at + n, a:b].reshape(n, H, -1).astype(np.float64) for a, b in ((0, H * D), (H * D, 2 * H * D), (2 * H * D, stride)))
+        ref = np.zeros((H, D, V)) if s % 3 == 0 else state[s].astype(np.float64)
+        assert rel_rms(got[at:at + n], lightning_ref(q, k, v, decay.astype(np.float64), ref)) < 1e-5 and rel_rms(gs[s], ref) < 1e-5, (s, at)
+        at += n
+
+
 def latent_ref(q, cache, vis, wuk, wuv, sink, scale, H, D, V):
     T = q.shape[0]
     out = np.zeros((T, H, V))
