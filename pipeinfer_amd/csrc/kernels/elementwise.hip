@@ -685,9 +685,11 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // stage 1: grid (n_tok, NCH) — each workgroup finds the k best of its slice of the vocabulary and its partial max / sum-exp
 // stage 2: one workgroup per token merges NCH*k candidates (same ordering) and the partial sums.
 #define TOPK_NCH 32
-// What bounds it: the k selection rounds (8 MB of logits a millisecond of reading is nothing beside them).  A slice belongs to ONE wave, its values in registers as order-preserving integers; a lane keeps its own
-// best, so a round is two wave reductions and one rescan of the lane that lost its best — no barrier, no rescan of everything.  (A workgroup per slice that looked at all its values in every round and met at a
-// barrier: 16.7 us for one row of 32000, 607 for 2048 rows; now 8.6 and 144.)  Slices of more than 64 * 32 values (a vocabulary above 65536) are re-read from memory in every round.
+// What bounds it: the k selection rounds (8 MB of logits a millisecond of reading is nothing beside them).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best, so a round is
+// two wave reductions and one rescan of the lane that lost its best — no barrier, no rescan of everything.  (A workgroup per slice that looked at all its values in every round and met at a barrier: 16.7 us for one
+// row of 32000, 607 for 2048 rows; now 8.6 and 144.)  WS waves share a slice.  One up to a vocabulary of 65536
+// (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
+// One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
 static __device__ __forceinline__ uint32_t topk_key(float v) {
     const uint32_t u = __float_as_uint(v + 0.0f);                       // (-0 ties with +0)
@@ -702,53 +704,79 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
     pi_butterfly<32>([&](auto o) { i = min(i, pi_partner<decltype(o)::value>(i)); });
     key = m; id = i;
 }
-template <int VPT>
+template <int VPT, int WS>
 __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
-    const int t = blockIdx.x, lane = threadIdx.x & 63, ch = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per);
+    constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
+    __shared__ uint32_t met_key[WS > 1 ? 32 : 1]; __shared__ int met_id[WS > 1 ? 32 : 1]; __shared__ float met_sum[4];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
+    const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per), own0 = lo + lane + (WS > 1 ? 64 * wave : 0);
     const float * l = logits + (int64_t) t * n_vocab;
     uint32_t key[VPT > 0 ? VPT : 1]; float rv[VPT > 0 ? VPT : 1];
     uint32_t bk = 0; int bm = 0;                                        // this lane's best among the ones not taken: key, number
     if constexpr (VPT > 0) {
 #pragma unroll
-        for (int m = 0; m < VPT; m++) { const int i = lo + lane + 64 * m; rv[m] = l[min(i, n_vocab - 1)]; }
+        for (int m = 0; m < VPT; m++) rv[m] = l[min(own0 + STEP * m, n_vocab - 1)];
 #pragma unroll
-        for (int m = 0; m < VPT; m++) { key[m] = lo + lane + 64 * m < hi ? topk_key(rv[m]) : 0u; if (key[m] > bk) { bk = key[m]; bm = m; } }
-    } else for (int i = lo + lane; i < hi; i += 64) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = (i - lo) / 64; } }
-    uint32_t wk = bk; int wi = bk ? lo + lane + 64 * bm : 0x7fffffff;
+        for (int m = 0; m < VPT; m++) { key[m] = own0 + STEP * m < hi ? topk_key(rv[m]) : 0u; if (key[m] > bk) { bk = key[m]; bm = m; } }
+    } else for (int i = own0, m = 0; i < hi; i += STEP, m++) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = m; } }
+    if (pi_abort_late(gone, abort_w)) return;
+    uint32_t wk = bk; int wi = bk ? own0 + STEP * bm : 0x7fffffff;
     topk_best(wk, wi);
-    const float first = topk_value(wk);
+    uint32_t top = wk;
+    if constexpr (WS > 1) {
+        if (lane == 0) met_key[wave] = wk;
+        __syncthreads();
+        top = max(max(met_key[0], met_key[1]), max(met_key[2], met_key[3]));
+        __syncthreads();
+    }
+    const float first = topk_value(top);
     // the slice's sum of exponentials, in the order of 256 threads of four waves
     float s[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
     if constexpr (VPT > 0) {
 #pragma unroll
-        for (int m = 0; m < VPT; m++) if (lo + lane + 64 * m < hi) s[m & 3] += expf(rv[m] - first);
-    } else for (int i = lo + lane, w = 0; i < hi; i += 64, w = (w + 1) & 3) { const float e = expf(l[i] - first); s[0] += w == 0 ? e : 0.0f; s[1] += w == 1 ? e : 0.0f; s[2] += w == 2 ? e : 0.0f; s[3] += w == 3 ? e : 0.0f; }
+        for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[WS > 1 ? 0 : m & 3] += expf(rv[m] - first);
+    } else for (int i = own0; i < hi; i += STEP) s[0] += expf(l[i] - first);
+    static_assert(VPT > 0 || WS > 1, "values that are read again: four waves");
+    if constexpr (WS == 1) {
 #pragma unroll
-    for (int w = 0; w < 4; w++) s[w] = pi_lanes_sum<64>(s[w]);
-    if (pi_abort_late(gone, abort_w)) return;
-    if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
+        for (int w = 0; w < 4; w++) s[w] = pi_lanes_sum<64>(s[w]);
+        if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
+    } else { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; }
     const int64_t out = ((int64_t) t * TOPK_NCH + ch) * k;
-    int own = 0x7fffffff;                                             // lane r keeps the r-th: their values are read back together, not one by one between the rounds
+    int own = 0x7fffffff; uint32_t own_key = 0;                       // lane r keeps the r-th: their values are read back together, not one by one between the rounds
     for (int r = 0; ; r++) {
-        if (lane == r) own = wi;
+        if (lane == r) { own = wi; own_key = wk; }
         if (r + 1 >= k) break;
-        if (wk != 0 && wi == lo + lane + 64 * bm) {                     // its owner looks for its next one
-            bk = 0;
-            if constexpr (VPT > 0) {
+        if constexpr (VPT > 0) {
+            if (wk != 0 && wi == own0 + STEP * bm) {                    // its owner looks for its next one
+                bk = 0;
                 const int taken = bm;
 #pragma unroll
                 for (int m = 0; m < VPT; m++) { if (m == taken) key[m] = 0; if (key[m] > bk) { bk = key[m]; bm = m; } }
-            } else {
-                for (int i = lo + lane; i < hi; i += 64) {
-                    const uint32_t q = topk_key(l[i]);
-                    if ((q < wk || (q == wk && i > wi)) && q > bk) { bk = q; bm = (i - lo) / 64; }
-                }
+            }
+        } else {                                                        // (every lane looks again: one lane's values alone would be a trip to memory each)
+            bk = 0;
+            for (int i = own0, m = 0; i < hi; i += STEP, m++) {
+                const uint32_t q = topk_key(l[i]);
+                if ((q < wk || (q == wk && i > wi)) && q > bk) { bk = q; bm = m; }
             }
         }
-        wk = bk; wi = bk ? lo + lane + 64 * bm : 0x7fffffff;
+        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
         topk_best(wk, wi);
+    }
+    if constexpr (WS > 1) {
+        if (lane < 8) { met_key[8 * wave + lane] = lane < k ? own_key : 0u; met_id[8 * wave + lane] = own; }
+        __syncthreads();
+        if (wave != 0) return;
+        uint32_t mk = lane < 32 ? met_key[lane] : 0u; const int mi = lane < 32 ? met_id[lane] : 0x7fffffff;
+        for (int r = 0; r < k; r++) {
+            wk = mk; wi = mi;
+            topk_best(wk, wi);
+            if (lane == r) own = wi;
+            if (mi == wi) mk = 0;
+        }
+        if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (met_sum[0] + met_sum[1]) + (met_sum[2] + met_sum[3]); }
     }
     if (lane < k) { cid[out + lane] = own; cval[out + lane] = own != 0x7fffffff ? l[own] : -INFINITY; }
 }
@@ -787,9 +815,11 @@ extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, i
     if (!scratch) { pi_set_error("pi_op_topk: scratch is NULL (needs pi_op_topk_scratch_bytes(n_tok) bytes)"); return -1; }
     int32_t * cid = (int32_t *) scratch; float * cval = (float *) (cid + (size_t) n_tok * TOPK_NCH * k);
     float * cmax = cval + (size_t) n_tok * TOPK_NCH * k, * csum = cmax + (size_t) n_tok * TOPK_NCH;
-    const int per_lane = ((n_vocab + TOPK_NCH - 1) / TOPK_NCH + 63) / 64;
-#define TOPK_GO(VPT) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, k_topk1<VPT>, dim3(n_tok, TOPK_NCH / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, cid, cval, cmax, csum, pi_abort_word())
-    if (per_lane <= 8) TOPK_GO(8); else if (per_lane <= 16) TOPK_GO(16); else if (per_lane <= 32) TOPK_GO(32); else TOPK_GO(0);
+    const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
+#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, cid, cval, cmax, csum, pi_abort_word())
+    if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4);
+    else if (per <= 64 * 8) TOPK_GO(8, 1); else if (per <= 64 * 16) TOPK_GO(16, 1); else if (per <= 64 * 32) TOPK_GO(32, 1);
+    else if (per <= 256 * 16) TOPK_GO(16, 4); else if (per <= 256 * 32) TOPK_GO(32, 4); else TOPK_GO(0, 4);
 #undef TOPK_GO
     PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2, dim3(n_tok), dim3(64), 0, (hipStream_t) stream, k, cid, cval, cmax, csum, ids, vals, sumexp, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;

@@ -439,6 +439,31 @@ def test_topk_edges(gpu, n_vocab):
             assert abs(gs[t] - want) / want < 1e-5
 
 
+@pytest.mark.parametrize("n_vocab", [131072, 131073, 262144, 262145])
+def test_topk_edges_of_large_vocabularies(gpu, n_vocab):
+    """the last vocabulary of every instance that four waves share a slice of, and the first of the next"""
+    test_topk_edges(gpu, n_vocab)
+
+
+@pytest.mark.parametrize("n_tok", [5, 17])
+@pytest.mark.parametrize("n_vocab", [3, 8192, 8193, 65536, 65537, 262145])
+def test_top_of_a_row_and_more(gpu, n_vocab, n_tok):
+    """fewer than eight: k = 1 (few rows: four waves a slice) and k = 3 are the first of the eight, with the same bits of the sum"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(n_vocab)
+    x = np.round(rng.standard_normal((n_tok, n_vocab)) * 6).astype(np.float32)
+    x[1] = np.nan
+    x[2, :] = -np.inf
+    ld, scr, res = U.Dev(x), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(n_tok)), {}
+    for k in (8, 3, 1):
+        ids, vals, se = U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok)
+        L.check(lib.pi_op_topk(ld.ptr, n_vocab, n_tok, k, ids.ptr, vals.ptr, se.ptr, scr.ptr, None))
+        res[k] = ids.get(np.int32, (n_tok, k)), vals.get(np.float32, (n_tok, k)), se.get(np.float32)
+        assert np.array_equal(res[k][0], res[8][0][:, :k]) and np.array_equal(res[k][1], res[8][1][:, :k]) and np.array_equal(res[k][2].view(np.uint32), res[8][2].view(np.uint32))
+    assert res[8][0][0, 0] == int(np.argmax(x[0]))
+
+
 @pytest.mark.parametrize("n_vocab", [512, 32000, 65024])
 def test_topk(gpu, n_vocab):
     lib, U = gpu
