@@ -1385,14 +1385,22 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     __shared__ float gsh[4];                                          // per token: the head's gate (one value per head)
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nt = min(4, n_tok - t0);
-    hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (vec: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
-    if (vec) {
+    hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (wide: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
+    const bool wide = vec && rank >= 256;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9)
+    if (wide) {
 #pragma unroll
         for (int k = 0; k < 4; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)) * rank + min(lane * 8, rank - 8));
         if (gate && gate_width > 1)
 #pragma unroll
             for (int k = 0; k < 4; k++) gv[k] = gate[(int64_t) (t0 + min(lane, nt - 1)) * gs + (int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)];
     }
+    // many splits: a thread per four values of the rank, for all tokens at a time or, where that leaves no second group of threads and the splits are many, for one token after the other; the groups take eight splits
+    // in turn (1 token of 8 heads, rank 256, over 16384 cells: 83 us with one group, now 43)
+    __shared__ __attribute__((aligned(16))) float4 shares[4][256];
+    const int cols = rank >> 2, at_once = nt * cols <= 128 ? nt : 1, per = at_once * cols, groups = vec && (at_once == nt ? S > 8 : S > 64) && per <= 128 ? 256 / per : 1, grp = tid / per, mine = tid % per / cols, col = tid % cols;
+    float4 share[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     for (int idx = tid; idx < 4 * rank; idx += 256) ol[idx] = 0.0f;
     if (tid < 4) {
         float g = 1.0f;
@@ -1422,6 +1430,22 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             if (lane == 0) cnt[wave] = __popcll(some);
         }
         __syncthreads();
+        if (groups > 1) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tt = min(i * at_once + mine, nt - 1), n = i * at_once < nt && grp < groups ? cnt[tt] : 0;
+                const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + col * 4;
+                for (int s0 = 8 * grp; s0 < n; s0 += 8 * groups) {
+                    float4 x[8];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) x[u] = *(const float4 *) (p + (int64_t) num[tt][min(s0 + u, n - 1)] * rank);
+#pragma unroll
+                    for (int u = 0; u < 8; u++)
+                        if (s0 + u < n) { const float w = wgt[tt][s0 + u]; share[i].x = fmaf(w, x[u].x, share[i].x); share[i].y = fmaf(w, x[u].y, share[i].y); share[i].z = fmaf(w, x[u].z, share[i].z); share[i].w = fmaf(w, x[u].w, share[i].w); }
+                }
+            }
+            continue;
+        }
         if (vec) {                                                     // four values of the rank per thread, eight splits on their way at a time (one by one, every split was a trip to memory: 23 us for 11 of 4 tokens)
             for (int idx = tid; idx < nt * (rank >> 2); idx += 256) {
                 const int tt = idx / (rank >> 2), r = idx % (rank >> 2) * 4, n = cnt[tt];
@@ -1450,8 +1474,19 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             ol[idx] = v;
         }
     }
+    if (groups > 1) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) if (i * at_once < nt) shares[i][tid] = share[i];
+        __syncthreads();
+        for (int idx = tid; idx < nt * cols; idx += 256) {
+            const float4 * from = shares[idx / per];
+            float4 v = from[idx % per];
+            for (int g = 1; g < groups; g++) { const float4 x = from[g * per + idx % per]; v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w; }
+            *(float4 *) (ol + idx / cols * rank + idx % cols * 4) = v;
+        }
+    }
     __syncthreads();
-    if (vec) {
+    if (wide) {
         const int v0 = blockIdx.z * 16 + wave;
         float a[4][4];
 #pragma unroll
@@ -1602,7 +1637,7 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     const double bytes = 4.0 * acct * (rank + rot) + 4.0 * n_tok * heads * (rank + rot + (double) rank * p.S);
     // few tokens, sizes of whole steps: the matrix cores (more scratch memory than the other kernel's: its size is pi_op_latent_attention_rot_scratch_floats')
     const int S32 = (n_kv + 31) / 32;
-    const bool whole = lat_rows_takes(rank, rot, n_tok) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats && (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
+    const bool whole = lat_rows_takes(rank, rot, n_tok) && (n_tok * heads >= 8 || n_kv < 4096) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats && (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
     if (whole) {
         p.S = S32;
         pml = pol + (size_t) n_tok * heads * p.S * rank;
@@ -1620,7 +1655,7 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), dim3(256), (size_t) 16 * rank, s,
                  pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok,
-                 (int) ((rank & 7) == 0 && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0), out, out_stride, pi_abort_word());
+                 (int) ((rank & 7) == 0 && (rank >= 256 || p.S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0)      /* (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3) */, out, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 

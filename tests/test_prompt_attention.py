@@ -35,6 +35,17 @@ def test_latent_few_tokens(H, D, R, V, rank, T, n_kv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rank", [40, 64, 256, 512, 768])
+@pytest.mark.parametrize("T,n_kv", [(1, 2600), (2, 300), (3, 2600), (4, 4500), (7, 900)])
+def test_latent_splits_are_merged(rank, T, n_kv):
+    """one to four tokens of a tile, splits that groups of threads share out (all tokens at once, one after the other) and that one group takes, rounds of 64 splits that are not full"""
+    U, lib = gpu()
+    rng = np.random.default_rng(rank + T)
+    got, want = latent_case(U, lib, rng, 5, 12, 0, 20, rank, n_kv, np.arange(n_kv - T, n_kv), 500.0, HALVES, 0, rng.standard_normal(5), 12 ** -0.5)
+    assert rel_rms(got, want) < 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,rank,T,n_kv", [(6, 256, 5, 700), (16, 512, 4, 200), (1, 256, 1, 64), (5, 512, 8, 100)])
 def test_latent_few_tokens_over_scattered_cells(H, rank, T, n_kv):
     """what a token sees is any set of cells; what lies behind the cells in use is no number"""
