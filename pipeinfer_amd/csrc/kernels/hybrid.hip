@@ -1076,7 +1076,6 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
         ((float *) qsh)[d * 4 + tt] = q[(int64_t) min(t0 + tt, n_tok - 1) * qs + (int64_t) h * hw + d];
     }
     __syncthreads();
-    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the queries, requested after it)
     const int dq = (dim + 3) / 4, d0 = wave * dq, d1 = min(dim, d0 + dq);
     float acc[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
     const uint16_t * w = wuk + (int64_t) h * dim * rank + min(r, rank - 1);
@@ -1090,6 +1089,7 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
     for (int tt = 0; tt < 4; tt++) part[wave][tt][lane] = acc[tt];
     __syncthreads();
     const int tt = wave;                                              // wave tt writes token t0 + tt
+    if (pi_abort_late(gone, abort_w, 5)) return;                       // (32 rows of 128 bytes per wave: an earlier look keeps them behind the queries, 4.7 us a launch instead of 3.8)
     if (t0 + tt < n_tok && r < rank) qa[((int64_t) (t0 + tt) * heads + h) * (rank + rot) + r] = (part[0][tt][lane] + part[1][tt][lane] + part[2][tt][lane] + part[3][tt][lane]) * scale;
 }
 
@@ -1394,13 +1394,18 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
 #pragma unroll
             for (int k = 0; k < 4; k++) gv[k] = gate[(int64_t) (t0 + min(lane, nt - 1)) * gs + (int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)];
     }
-    // many splits: a thread per four values of the rank, for all tokens at a time or, where that leaves no second group of threads and the splits are many, for one token after the other; the groups take eight splits
+    // many splits: a thread per four values of the rank, for all tokens at a time or, where that leaves some threads idle but no second group of them and the splits are many, for one token after the other; the groups take eight splits
     // in turn (1 token of 8 heads, rank 256, over 16384 cells: 83 us with one group, now 43)
     __shared__ __attribute__((aligned(16))) float4 shares[4][256];
-    const int cols = rank >> 2, at_once = nt * cols <= 128 ? nt : 1, per = at_once * cols, groups = vec && (at_once == nt ? S > 8 : S > 64) && per <= 128 ? 256 / per : 1, grp = tid / per, mine = tid % per / cols, col = tid % cols;
+    int groups = 1, per = 1, at_once = 1, grp = 0, mine = 0, col = 0;
     float4 share[4];
+    if (vec && S > 8) {
+        const int cols = rank >> 2;
+        at_once = nt * cols <= 128 ? nt : 1; per = at_once * cols;
+        if ((at_once == nt || (S > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
 #pragma unroll
-    for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
     for (int idx = tid; idx < 4 * rank; idx += 256) ol[idx] = 0.0f;
     if (tid < 4) {
         float g = 1.0f;
@@ -1478,6 +1483,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
 #pragma unroll
         for (int i = 0; i < 4; i++) if (i * at_once < nt) shares[i][tid] = share[i];
         __syncthreads();
+        const int cols = rank >> 2;
         for (int idx = tid; idx < nt * cols; idx += 256) {
             const float4 * from = shares[idx / per];
             float4 v = from[idx % per];
