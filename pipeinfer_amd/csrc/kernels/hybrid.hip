@@ -1047,9 +1047,15 @@ static lat_plan latent_plan(int heads, int rank, int rot, int n_tok, int n_ctx) 
     return p;
 }
 
-// passes that take k_latent_rows: a few tokens (more of them: prompt_attention.hip), ranks of whole tiles
-static bool lat_rows_takes(int rank, int rot, int n_tok) { return n_tok <= 8 && (rank == 256 || rank == 512) && rot <= 64 && (rot & 3) == 0; }
+// Passes that take k_latent_rows: ranks of whole tiles, up to eight tokens, and as many more as leave rows (token, head) x rank small: there the tiles of a prompt, a workgroup per head that walks all cells, leave most of
+// the chip idle (16 heads, rank 512, us of the per-token kernels / the tiles / here: 9 tokens alone 71 / 25 / 22, of 512 cells 178 / 54 / 28, of 4096 439 / 274 / 89, of 16384 510 / 1060 / 292; 32 tokens alone
+// 82 / 32 / 29, of 4096 cells 431 / 280 / 174).  Beyond 512 rows of rank 512 the shares of the splits cost more than the tiles of a short context (32 heads, 24 tokens alone 31, here 36).  The shares are kept to
+// 560 MB of scratch memory from nine tokens on.
 static size_t lat_rows_floats(int heads, int rank, int rot, int n_tok, int n_ctx) { return (size_t) n_tok * heads * ((size_t) (rank + rot) + (size_t) (n_ctx + 31) / 32 * (rank + 2)); }
+static bool lat_rows_takes(int heads, int rank, int rot, int n_tok, int n_ctx) {
+    return (rank == 256 || rank == 512) && rot <= 64 && (rot & 3) == 0 && (n_tok <= 8 || (n_tok <= 32 && (int64_t) n_tok * heads * rank <= 512 * 512 && lat_rows_floats(heads, rank, rot, n_tok, n_ctx) <= (size_t) 140 << 20 &&
+                                                                                                 (n_ctx >= 64 || (int64_t) n_tok * heads * rank <= 384 * 512)));
+}
 
 // grid (token tile of 4, head, 64 values of the rank, then 64 values of the rotated part): lane = one rank value, the four waves take a quarter of the head's dim each and meet in LDS.  A query head is
 // [dim values | rot values]; the last are turned in pairs by the token's position (cs: the rotation table) and go behind the rank values
@@ -1330,31 +1336,37 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
     }
     __syncthreads();
     if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
-    // an infinity or a NaN must not meet the zero weight of a row that does not see its cell (rows of several tokens share a tile, a cell that nobody sees repeats another): it joins at the end
+    hy_f32x4 acc[NJ];
+    auto sums = [&]() {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++) {
+            const hy_f32x4 w = *(const hy_f32x4 *) &ps[n][16 * jt + 4 * g];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
+        }
+    };
+    sums();
+    // an infinity or a NaN must not meet the zero weight of a row that does not see its cell (rows of several tokens share a tile, a cell that nobody sees repeats another): where a sum is no number it is left out of all
+    // of them and joins at the end
     bool odd = false;
     if (__any(vis != 0xffffffffu)) {
-        uint32_t big = 0;
+        hy_f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-        for (int i = 0; i < 8; i++)
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++) big = max(big, __float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu);
-        odd = __any(big >= 0x7f800000u);
-        if (odd)
+            for (int r = 0; r < 4; r++) z[r] = fmaf(acc[j][r], 0.0f, z[r]);
+        odd = __any((z[0] + z[1]) + (z[2] + z[3]) != 0.0f);
+        if (odd) {
 #pragma unroll
             for (int i = 0; i < 8; i++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[i >> 2][i & 3][j >> 2][j & 3] = 0.0f;
-    }
-    hy_f32x4 acc[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll
-    for (int jt = 0; jt < 2; jt++) {
-        const hy_f32x4 w = *(const hy_f32x4 *) &ps[n][16 * jt + 4 * g];
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
+            sums();
+        }
     }
     if (!real || vis == 0) return;
     if (odd)
@@ -1375,6 +1387,8 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
 
 // grid (token tile of 4, head, 16 output values): merges the splits (with the sink if there is one), normalises, applies its rows of W_uv[h], then the gate if there is one: one value per head, or (gate_width = vdim)
 // one per output value
+// MANY: more than eight splits (the code for them costs the launches of fewer 0.3 us of 9.5)
+template <bool MANY>
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
                                                         const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
@@ -1396,10 +1410,10 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     }
     // many splits: a thread per four values of the rank, for all tokens at a time or, where that leaves some threads idle but no second group of them and the splits are many, for one token after the other; the groups take eight splits
     // in turn (1 token of 8 heads, rank 256, over 16384 cells: 83 us with one group, now 43)
-    __shared__ __attribute__((aligned(16))) float4 shares[4][256];
+    __shared__ __attribute__((aligned(16))) float4 shares[MANY ? 4 : 1][MANY ? 256 : 1];
     int groups = 1, per = 1, at_once = 1, grp = 0, mine = 0, col = 0;
     float4 share[4];
-    if (vec && S > 8) {
+    if (MANY && vec) {
         const int cols = rank >> 2;
         at_once = nt * cols <= 128 ? nt : 1; per = at_once * cols;
         if ((at_once == nt || (S > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
@@ -1435,7 +1449,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             if (lane == 0) cnt[wave] = __popcll(some);
         }
         __syncthreads();
-        if (groups > 1) {
+        if (MANY && groups > 1) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int tt = min(i * at_once + mine, nt - 1), n = i * at_once < nt && grp < groups ? cnt[tt] : 0;
@@ -1479,7 +1493,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             ol[idx] = v;
         }
     }
-    if (groups > 1) {
+    if (MANY && groups > 1) {
 #pragma unroll
         for (int i = 0; i < 4; i++) if (i * at_once < nt) shares[i][tid] = share[i];
         __syncthreads();
@@ -1551,8 +1565,9 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
 extern "C" int pi_op_latent_attention_max_cells(int rank) { (void) rank; return 1 << 22; }       // (long contexts are cut into splits: no score row has to fit LDS whole)
 extern "C" size_t pi_op_latent_attention_scratch_floats(int heads, int rank, int n_tok, int n_ctx) { return pi_op_latent_attention_rot_scratch_floats(heads, rank, 0, n_tok, n_ctx); }
 extern "C" size_t pi_op_latent_attention_rot_scratch_floats(int heads, int rank, int rot_dim, int n_tok, int n_ctx) {
-    const int few = std::min(n_tok, 8);
-    return std::max(std::max(latent_plan(heads, rank, rot_dim, n_tok, n_ctx).scratch, latent_plan(heads, rank, rot_dim, few, n_ctx).scratch), lat_rows_takes(rank, rot_dim, few) ? lat_rows_floats(heads, rank, rot_dim, few, n_ctx) : 0);
+    size_t need = std::max(latent_plan(heads, rank, rot_dim, n_tok, n_ctx).scratch, latent_plan(heads, rank, rot_dim, std::min(n_tok, 8), n_ctx).scratch);
+    for (int few = 1; few <= std::min(n_tok, 32); few++) if (lat_rows_takes(heads, rank, rot_dim, few, n_ctx)) need = std::max(need, lat_rows_floats(heads, rank, rot_dim, few, n_ctx));
+    return need;
 }
 template <int M, int RPT> static int latent_reserve_one() {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_latent_scores<M, RPT>, hipFuncAttributeMaxDynamicSharedMemorySize, LAT_LDS_BUDGET + 4096));
@@ -1635,15 +1650,17 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     a.q = q; a.qs = q_stride; a.dim1 = dim; a.k2_row = rank + rot; a.dim2 = rot; a.vdim = vdim; a.heads = heads; a.per_kv = 1; a.n_tok = n_tok; a.n_kv = n_kv; a.dyn = dyn_dev; a.mask = mask; a.pos = rot > 0 ? pos_dev : nullptr;
     a.cs = cs; a.n_pos = n_pos; a.pairing = pairing; a.scale = scale; a.weights = PI_WEIGHTS_SOFTMAX; a.sink = sink_dev; a.gate = gate_dev; a.gs = gate_stride; a.gate_act = gate_act; a.gate_width = gate_width; a.out_mult = 1.0f;
     a.out = out; a.os = out_stride;
-    if (latent_prompt(a, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) { PI_CHECK_LAUNCH(); return 0; }
+    // few tokens, sizes of whole steps (more scratch memory than the per-token kernels': its size is pi_op_latent_attention_rot_scratch_floats'); fewer than eight rows over a long context: those (1 head, 1 token of 16384
+    // cells 34 us, 40 here)
+    const int S32 = (n_kv + 31) / 32;
+    const bool whole = lat_rows_takes(heads, rank, rot, n_tok, n_kv) && (n_tok * heads >= 8 || n_kv < 4096) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats &&
+                       (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
+    if (!whole && latent_prompt(a, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) { PI_CHECK_LAUNCH(); return 0; }
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * dim + 4.0 * n_tok * heads * (dim + rank + 2.0 * rot), k_latent_absorb, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((rank + 63) / 64 + (rot + 63) / 64)), dim3(256), (size_t) 16 * dim, s,
                  q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, pi_abort_word());
     PI_CHECK_LAUNCH();
     const dim3 grid((unsigned) n_tok, (unsigned) ((heads + p.M - 1) / p.M), (unsigned) p.S);
     const double bytes = 4.0 * acct * (rank + rot) + 4.0 * n_tok * heads * (rank + rot + (double) rank * p.S);
-    // few tokens, sizes of whole steps: the matrix cores (more scratch memory than the other kernel's: its size is pi_op_latent_attention_rot_scratch_floats')
-    const int S32 = (n_kv + 31) / 32;
-    const bool whole = lat_rows_takes(rank, rot, n_tok) && (n_tok * heads >= 8 || n_kv < 4096) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats && (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
     if (whole) {
         p.S = S32;
         pml = pol + (size_t) n_tok * heads * p.S * rank;
@@ -1659,9 +1676,11 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
 #undef LAT_GO
     }
     PI_CHECK_LAUNCH();
-    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), dim3(256), (size_t) 16 * rank, s,
-                 pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok,
-                 (int) ((rank & 7) == 0 && (rank >= 256 || p.S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0)      /* (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3) */, out, out_stride, pi_abort_word());
+    const int vec = (rank & 7) == 0 && (rank >= 256 || p.S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
+#define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
+                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok, vec, out, out_stride, pi_abort_word())
+    if (p.S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
+#undef LAT_COMBINE
     PI_CHECK_LAUNCH(); return 0;
 }
 

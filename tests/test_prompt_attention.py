@@ -35,6 +35,17 @@ def test_latent_few_tokens(H, D, R, V, rank, T, n_kv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,R,rank", [(16, 64, 512), (17, 0, 512), (7, 8, 256), (32, 0, 256), (33, 4, 256), (64, 4, 512)])
+@pytest.mark.parametrize("T,n_kv", [(9, 9), (16, 100), (17, 700), (31, 40), (32, 600), (33, 64)])
+def test_latent_rows_and_tiles(H, R, rank, T, n_kv):
+    """both sides of the line between splits of 32 cells and the tiles of a prompt (32 tokens; 512 rows of rank 512, 1024 of rank 256)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H + T)
+    got, want = latent_case(U, lib, rng, H, 8, R, 12, rank, n_kv, np.arange(n_kv - T, n_kv), 500.0, NEIGHBOURS, 1, None, (8 + R) ** -0.5)
+    assert rel_rms(got, want) < 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rank", [40, 64, 256, 512, 768])
 @pytest.mark.parametrize("T,n_kv", [(1, 2600), (2, 300), (3, 2600), (4, 4500), (7, 900)])
 def test_latent_splits_are_merged(rank, T, n_kv):
