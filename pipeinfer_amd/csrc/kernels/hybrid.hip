@@ -1262,127 +1262,133 @@ __global__ void __launch_bounds__(256) k_latent_scores(const float * __restrict_
 // product.  With a lane per cell and a chain of loads each, 4 tokens x 16 heads over 700 cells of 512 + 64 took 20 us (now 11.5); 1 token x 16 heads of 256, 32 cells: 9.7 (6.4).
 // NJ: a wave sums 16 NJ of the rank's values (rank = 64 NJ); EX: steps of 16 values behind the rank.  Lane l holds, with n = l % 16 and g = l / 16, of the scores row n and the wave's cells 4 g + r, of the sums
 // row n and the values NJ (4 g + r) + j.  (Splits of 64 cells, every wave its sixteen over the whole width: 17 us.)
-template <int NJ, int EX>
-__global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int W, int n_rows, int n_kv_arg, int S,
+// LOOP: fewer workgroups than splits, each takes several (a loop of one round costs 77 -> 85 us: 4 tokens x 16 heads, 16384 cells)
+template <int NJ, int EX, bool LOOP>
+__global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_rows(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int W, int n_rows, int n_kv_arg, int S,
                                                         float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int RANK = 64 * NJ, NS = RANK / 16 + EX, NH = NS / 2;
     __shared__ __attribute__((aligned(16))) float ps[16][36], half[2][16][20];
     __shared__ float top[2][16], sum[2][16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, split = blockIdx.y, c0 = split * 32, ct = wave & 1, wh = wave >> 1;
-    const int row = min((int) blockIdx.x * 16 + n, n_rows - 1), words = (n_kv_arg + 31) / 32, n_kv = min(dyn ? dyn[1] : n_kv_arg, n_kv_arg);
-    uint32_t vis = 0;
-    if (c0 < n_kv) {
-        vis = mask[(int64_t) (row / heads) * words + split];
+    const int words = (n_kv_arg + 31) / 32, n_kv = min(dyn ? dyn[1] : n_kv_arg, n_kv_arg);
+    const uint32_t first = mask[(int64_t) (min((int) (blockIdx.x * 16 + (threadIdx.x & 15)), n_rows - 1) / heads) * words + blockIdx.y];      // (on its way beside the number of live cells)
+    int split = blockIdx.y;
+    if (split * 32 >= n_kv) return;                                    // (cells of the context that hold nothing yet)
+    do {                                                               // (a barrier lies between a round's last look at the LDS and the next one's writes to the same place)
+        int tid = threadIdx.x;
+        if constexpr (LOOP) asm volatile("" : "+v"(tid));              // (queries and addresses are made again in every round: kept from one to the next they take the registers of a second workgroup)
+        const int lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, ct = wave & 1, wh = wave >> 1, row = min((int) blockIdx.x * 16 + n, n_rows - 1);
+        const int c0 = split * 32;
+        uint32_t vis = split == (int) blockIdx.y ? first : mask[(int64_t) (row / heads) * words + split];
         if (n_kv - c0 < 32) vis &= (1u << (n_kv - c0)) - 1u;
-    }
-    uint32_t some = vis;                                              // the cells that any row sees; what the others hold is not read
+        uint32_t some = vis;                                              // the cells that any row sees; what the others hold is not read
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
-    float * pml_r = pml + ((int64_t) ((int) blockIdx.x * 16 + n) * S + split) * 2;
-    const bool real = (int) blockIdx.x * 16 + n < n_rows;
-    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the mask, requested after it)
-    if (!some) {                                                      // (the same in every lane: the rows of a tile are the same sixteen in all four)
-        if (tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
-        return;
-    }
-    const int spare = __ffs(some) - 1;
-    auto cell = [&](int c) { return (uint32_t) (c0 + ((some >> c) & 1u ? c : spare)); };
-    hy_f32x4 kf[NH], qf[NH], vf[2][4][NJ / 4];
-    {   // a wave scores sixteen cells over half of the row's width
-        const uint32_t ko = cell(16 * ct + n) * (uint32_t) W, qo = (uint32_t) row * (uint32_t) W;
-#pragma unroll
-        for (int i = 0; i < NH; i++) {
-            const uint32_t d = 16u * (wh * NH + i) + 4u * g, at = EX == 0 ? d : min(d, (uint32_t) W - 4u);
-            kf[i] = *(const hy_f32x4 *) (cache + ko + at); qf[i] = *(const hy_f32x4 *) (qa + qo + at);
-            if (EX && d >= (uint32_t) W) qf[i] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+        for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
+        float * pml_r = pml + ((int64_t) ((int) blockIdx.x * 16 + n) * S + split) * 2;
+        const bool real = (int) blockIdx.x * 16 + n < n_rows;
+        if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the mask, requested after it)
+        if (!some) {                                                      // (the same in every lane: the rows of a tile are the same sixteen in all four)
+            if (tid < 16 && real) { pml_r[0] = -INFINITY; pml_r[1] = 0.0f; }
+            continue;
         }
-    }
+        const int spare = __ffs(some) - 1;
+        auto cell = [&](int c) { return (uint32_t) (c0 + ((some >> c) & 1u ? c : spare)); };
+        hy_f32x4 kf[NH], qf[NH], vf[2][4][NJ / 4];
+        {   // a wave scores sixteen cells over half of the row's width
+            const uint32_t ko = cell(16 * ct + n) * (uint32_t) W, qo = (uint32_t) row * (uint32_t) W;
 #pragma unroll
-    for (int jt = 0; jt < 2; jt++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint32_t o = cell(16 * jt + 4 * g + c) * (uint32_t) W + (uint32_t) (wave * (RANK / 4) + NJ * n);
-#pragma unroll
-            for (int j = 0; j < NJ / 4; j++) vf[jt][c][j] = *(const hy_f32x4 *) (cache + o + 4 * j);
+            for (int i = 0; i < NH; i++) {
+                const uint32_t d = 16u * (wh * NH + i) + 4u * g, at = EX == 0 ? d : min(d, (uint32_t) W - 4u);
+                kf[i] = *(const hy_f32x4 *) (cache + ko + at); qf[i] = *(const hy_f32x4 *) (qa + qo + at);
+                if (EX && d >= (uint32_t) W) qf[i] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+            }
         }
-    __builtin_amdgcn_sched_barrier(0);
-    hy_f32x4 s0 = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-    for (int i = 0; i < NH; i++)
+        for (int jt = 0; jt < 2; jt++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) s0 = hy_mfma(kf[i][c], qf[i][c], s0);
-    if (wh) *(hy_f32x4 *) &half[ct][n][4 * g] = s0;
-    __syncthreads();
-    const uint32_t mine = vis >> (16 * ct + 4 * g);
-    float m = -INFINITY;
-    if (!wh) {
-        s0 += *(const hy_f32x4 *) &half[ct][n][4 * g];
+            for (int c = 0; c < 4; c++) {
+                const uint32_t o = cell(16 * jt + 4 * g + c) * (uint32_t) W + (uint32_t) (wave * (RANK / 4) + NJ * n);
 #pragma unroll
-        for (int r = 0; r < 4; r++) if (mine >> r & 1u) m = fmaxf(m, s0[r]);
-        m = fmaxf(m, __shfl_xor(m, 16, 64)); m = fmaxf(m, __shfl_xor(m, 32, 64));
-        if (g == 0) top[ct][n] = m;
-    }
-    __syncthreads();
-    m = fmaxf(top[0][n], top[1][n]);
-    if (!wh) {
-        float l = 0.0f;
-        hy_f32x4 p;
+                for (int j = 0; j < NJ / 4; j++) vf[jt][c][j] = *(const hy_f32x4 *) (cache + o + 4 * j);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        hy_f32x4 s0 = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-        for (int r = 0; r < 4; r++) { p[r] = mine >> r & 1u ? expf(s0[r] - m) : 0.0f; l += p[r]; }
-        l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
-        if (g == 0) sum[ct][n] = l;
-        *(hy_f32x4 *) &ps[n][16 * ct + 4 * g] = p;
-    }
-    __syncthreads();
-    if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
-    hy_f32x4 acc[NJ];
-    auto sums = [&]() {
+        for (int i = 0; i < NH; i++)
 #pragma unroll
-        for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+            for (int c = 0; c < 4; c++) s0 = hy_mfma(kf[i][c], qf[i][c], s0);
+        if (wh) *(hy_f32x4 *) &half[ct][n][4 * g] = s0;
+        __syncthreads();
+        const uint32_t mine = vis >> (16 * ct + 4 * g);
+        float m = -INFINITY;
+        if (!wh) {
+            s0 += *(const hy_f32x4 *) &half[ct][n][4 * g];
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++) {
-            const hy_f32x4 w = *(const hy_f32x4 *) &ps[n][16 * jt + 4 * g];
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
+            for (int r = 0; r < 4; r++) if (mine >> r & 1u) m = fmaxf(m, s0[r]);
+            m = fmaxf(m, __shfl_xor(m, 16, 64)); m = fmaxf(m, __shfl_xor(m, 32, 64));
+            if (g == 0) top[ct][n] = m;
         }
-    };
-    sums();
-    // an infinity or a NaN must not meet the zero weight of a row that does not see its cell (rows of several tokens share a tile, a cell that nobody sees repeats another): where a sum is no number it is left out of all
-    // of them and joins at the end
-    bool odd = false;
-    if (__any(vis != 0xffffffffu)) {
-        hy_f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
+        __syncthreads();
+        m = fmaxf(top[0][n], top[1][n]);
+        if (!wh) {
+            float l = 0.0f;
+            hy_f32x4 p;
 #pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) z[r] = fmaf(acc[j][r], 0.0f, z[r]);
-        odd = __any((z[0] + z[1]) + (z[2] + z[3]) != 0.0f);
-        if (odd) {
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[i >> 2][i & 3][j >> 2][j & 3] = 0.0f;
-            sums();
+            for (int r = 0; r < 4; r++) { p[r] = mine >> r & 1u ? expf(s0[r] - m) : 0.0f; l += p[r]; }
+            l += __shfl_xor(l, 16, 64); l += __shfl_xor(l, 32, 64);
+            if (g == 0) sum[ct][n] = l;
+            *(hy_f32x4 *) &ps[n][16 * ct + 4 * g] = p;
         }
-    }
-    if (!real || vis == 0) return;
-    if (odd)
-        for (int c = 0; c < 32; c++) {
-            if (!(vis >> c & 1u)) continue;
-            const float * row = cache + cell(c) * (uint32_t) W + wave * (RANK / 4) + NJ * 4 * g;
+        __syncthreads();
+        if (tid < 16 && real) { pml_r[0] = m; pml_r[1] = sum[0][n] + sum[1][n]; }
+        hy_f32x4 acc[NJ];
+        auto sums = [&]() {
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+            for (int j = 0; j < NJ; j++) acc[j] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-                for (int j = 0; j < NJ; j++) if ((__float_as_uint(row[NJ * r + j]) & 0x7fffffffu) >= 0x7f800000u) acc[j][r] += row[NJ * r + j];
+            for (int jt = 0; jt < 2; jt++) {
+                const hy_f32x4 w = *(const hy_f32x4 *) &ps[n][16 * jt + 4 * g];
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) acc[j] = hy_mfma(vf[jt][c][j >> 2][j & 3], w[c], acc[j]);
+            }
+        };
+        sums();
+        // an infinity or a NaN must not meet the zero weight of a row that does not see its cell (rows of several tokens share a tile, a cell that nobody sees repeats another): where a sum is no number it is left out of all
+        // of them and joins at the end
+        bool odd = false;
+        if (__any(vis != 0xffffffffu)) {
+            hy_f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) z[r] = fmaf(acc[j][r], 0.0f, z[r]);
+            odd = __any((z[0] + z[1]) + (z[2] + z[3]) != 0.0f);
+            if (odd) {
+#pragma unroll
+                for (int i = 0; i < 8; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[i >> 2][i & 3][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[i >> 2][i & 3][j >> 2][j & 3] = 0.0f;
+                sums();
+            }
         }
-    float * o = pol + ((int64_t) row * S + split) * RANK + wave * (RANK / 4);
+        if (!real || vis == 0) continue;
+        if (odd)
+            for (int c = 0; c < 32; c++) {
+                if (!(vis >> c & 1u)) continue;
+                const float * row = cache + cell(c) * (uint32_t) W + wave * (RANK / 4) + NJ * 4 * g;
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+                for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int j = 0; j < NJ; j += 4) *(hy_f32x4 *) (o + NJ * (4 * g + r) + j) = hy_f32x4{ acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r] };
+                    for (int j = 0; j < NJ; j++) if ((__float_as_uint(row[NJ * r + j]) & 0x7fffffffu) >= 0x7f800000u) acc[j][r] += row[NJ * r + j];
+            }
+        float * o = pol + ((int64_t) row * S + split) * RANK + wave * (RANK / 4);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int j = 0; j < NJ; j += 4) *(hy_f32x4 *) (o + NJ * (4 * g + r) + j) = hy_f32x4{ acc[j][r], acc[j + 1][r], acc[j + 2][r], acc[j + 3][r] };
+    } while (LOOP && (split += gridDim.y) * 32 < n_kv);
 }
 
 // grid (token tile of 4, head, 16 output values): merges the splits (with the sink if there is one), normalises, applies its rows of W_uv[h], then the gate if there is one: one value per head, or (gate_width = vdim)
@@ -1390,7 +1396,7 @@ __global__ void __launch_bounds__(256, 1) k_latent_rows(const float * __restrict
 // MANY: more than eight splits (the code for them costs the launches of fewer 0.3 us of 9.5)
 template <bool MANY>
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
-                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int vec, float * __restrict__ out, int64_t os,
+                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, const int32_t * __restrict__ dyn, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     extern __shared__ __attribute__((aligned(16))) float ol[];                                     // [4][rank]
@@ -1398,7 +1404,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     __shared__ int num[4][64], cnt[4];                                // their numbers, how many they are
     __shared__ float gsh[4];                                          // per token: the head's gate (one value per head)
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nt = min(4, n_tok - t0);
+    const int nt = min(4, n_tok - t0), n_s = n_kv > 0 ? min(S, (min(dyn ? dyn[1] : n_kv, n_kv) + 31) / 32) : S;      // (n_kv > 0: splits of 32 cells, the ones behind the live cells hold nothing)
     hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (wide: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
     const bool wide = vec && rank >= 256;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9)
     if (wide) {
@@ -1416,7 +1422,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     if (MANY && vec) {
         const int cols = rank >> 2;
         at_once = nt * cols <= 128 ? nt : 1; per = at_once * cols;
-        if ((at_once == nt || (S > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
+        if ((at_once == nt || (n_s > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
 #pragma unroll
         for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
@@ -1430,20 +1436,21 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     float mstar = -INFINITY, den = 0.0f;
     const float sk = sink ? sink[h] : -INFINITY;
     const float * pml_t = pml + ((int64_t) (t0 + min(wave, nt - 1)) * heads + h) * S * 2;
+    const float m_own = lane < S ? pml_t[lane * 2] : -INFINITY, l_own = lane < S ? pml_t[lane * 2 + 1] : 0.0f;      // (on their way beside the number of live cells)
     {
-        float m = sk;
-        for (int s = lane; s < S; s += 64) m = fmaxf(m, pml_t[s * 2]);
+        float m = lane < n_s ? fmaxf(sk, m_own) : sk;
+        for (int s = lane + 64; s < n_s; s += 64) m = fmaxf(m, pml_t[s * 2]);
         mstar = pi_wave_max(m);
-        float d = 0.0f;
-        for (int s = lane; s < S; s += 64) { const float ms = pml_t[s * 2]; if (ms != -INFINITY) d += pml_t[s * 2 + 1] * expf(ms - mstar); }
+        float d = lane < n_s && m_own != -INFINITY ? l_own * expf(m_own - mstar) : 0.0f;
+        for (int s = lane + 64; s < n_s; s += 64) { const float ms = pml_t[s * 2]; if (ms != -INFINITY) d += pml_t[s * 2 + 1] * expf(ms - mstar); }
         den = pi_lanes_sum<64>(d) + (sink ? expf(sk - mstar) : 0.0f);
     }
     if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the splits' maxima, requested after it)
-    for (int sb = 0; sb < S; sb += 64) {
+    for (int sb = 0; sb < n_s; sb += 64) {
         __syncthreads();
         if (wave < nt) {
             const int s = sb + lane;
-            const float ms = s < S ? pml_t[s * 2] : -INFINITY;
+            const float ms = s >= n_s ? -INFINITY : sb == 0 ? m_own : pml_t[s * 2];
             const unsigned long long some = __ballot(ms != -INFINITY);
             if (ms != -INFINITY) { const int at = __popcll(some & ((1ull << lane) - 1ull)); wgt[wave][at] = expf(ms - mstar) / den; num[wave][at] = s; }
             if (lane == 0) cnt[wave] = __popcll(some);
@@ -1664,9 +1671,12 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     if (whole) {
         p.S = S32;
         pml = pol + (size_t) n_tok * heads * p.S * rank;
-        const dim3 rgrid((unsigned) ((n_tok * heads + 15) / 16), (unsigned) p.S);
-#define LAT_ROWS(NJ, EX) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_rows<NJ, EX>), rgrid, dim3(256), 0, s, qa, cache, mask, heads, rank + rot, n_tok * heads, n_kv, p.S, pol, pml, dyn_dev, pi_abort_word())
+        const unsigned row_tiles = (unsigned) ((n_tok * heads + 15) / 16);
+        const dim3 rgrid(row_tiles, std::min((unsigned) p.S, std::max(1u, 4096u / row_tiles)));      // (a context that holds less than it could: 8 tokens x 32 heads, 512 cells of 65536, a workgroup for each of the 2048 splits: 129 us, so 35)
+#define LAT_ROWS2(NJ, EX, LOOP) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_rows<NJ, EX, LOOP>), rgrid, dim3(256), 0, s, qa, cache, mask, heads, rank + rot, n_tok * heads, n_kv, p.S, pol, pml, dyn_dev, pi_abort_word())
+#define LAT_ROWS(NJ, EX) do { if (rgrid.y < (unsigned) p.S) LAT_ROWS2(NJ, EX, true); else LAT_ROWS2(NJ, EX, false); } while (0)
         if (rank == 256) { if (rot) LAT_ROWS(4, 4); else LAT_ROWS(4, 0); } else { if (rot) LAT_ROWS(8, 4); else LAT_ROWS(8, 0); }
+#undef LAT_ROWS2
 #undef LAT_ROWS
     } else {
 #define LAT_GO(M) do { if (p.RPT == 1) latent_scores_launch<M, 1>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); \
@@ -1678,7 +1688,7 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     PI_CHECK_LAUNCH();
     const int vec = (rank & 7) == 0 && (rank >= 256 || p.S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
 #define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
-                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok, vec, out, out_stride, pi_abort_word())
+                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok, whole ? n_kv : 0, dyn_dev, vec, out, out_stride, pi_abort_word())
     if (p.S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
 #undef LAT_COMBINE
     PI_CHECK_LAUNCH(); return 0;
