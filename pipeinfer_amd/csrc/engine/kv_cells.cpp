@@ -1,7 +1,6 @@
 #include "kv_cells.h"
 
 #include <algorithm>
-#include <utility>
 #include <climits>
 #include <cstring>
 
@@ -218,24 +217,21 @@ void kv_cells::build_mask(int n_kv, int n_tokens, const int32_t * pos, const int
     if (words32 <= 0) words32 = (n_kv + 31) / 32;          // row stride of the bitmap (the engine uses a fixed stride of n_ctx bits)
     memset(out, 0, (size_t) n_tokens * words32 * 4);
     std::vector<uint64_t> tmask((size_t) words_);
-    std::vector<std::pair<int32_t, int32_t>> own;          // (position, cell) of one sequence's cells, by position
     for (int j = 0; j < n_tokens; j++) {
         uint32_t * row = out + (size_t) j * words32;
         const int ns = n_seq_id[j];
-        // a prompt: one sequence's tokens, one behind the other.  A token sees what the one before it saw and the cells between their positions, so the table is walked once for all of them
-        // (2048 tokens, cell by cell for each: 3.4 ms of host time ahead of a 3.6 ms pass; 0.1 this way)
+        // a prompt: one sequence's tokens, one behind the other.  A token sees what the one before it saw and the cells between their positions, so the table is walked once for all of them: a cell goes to
+        // the first token that sees it, and the rows add up.  No order of the cells is needed: in a cache whose cells came round again sorting them took 237 us for 4 tokens of 4096 cells, the walk per token
+        // 37.  This way 4 / 8 / 512 tokens take 9 / 9 / 40 us, token by token 37 / 75 / 4680
         int end = j;
-        if (ns == 1) while (end < n_tokens && n_seq_id[end] == 1 && seq_id[end][0] == seq_id[j][0]) end++;
+        if (ns == 1) while (end < n_tokens && n_seq_id[end] == 1 && seq_id[end][0] == seq_id[j][0] && (end == j || pos[end] >= pos[end - 1])) end++;
         if (end - j >= 4) {
-            own.clear();
-            for (int c = 0; c < n_kv; c++) if (nseq_[c] != 0 && has(c, seq_id[j][0])) own.emplace_back(pos_[c], c);
-            if (!std::is_sorted(own.begin(), own.end())) std::sort(own.begin(), own.end());
-            size_t at = 0;
-            for (int t = j; t < end; t++, row += words32) {
-                if (t > j && pos[t] >= pos[t - 1]) memcpy(row, row - words32, (size_t) words32 * 4);
-                else at = 0;
-                for (; at < own.size() && own[at].first <= pos[t]; at++) row[own[at].second >> 5] |= 1u << (own[at].second & 31);
+            for (int c = 0; c < n_kv; c++) {
+                if (nseq_[c] == 0 || pos_[c] > pos[end - 1] || !has(c, seq_id[j][0])) continue;
+                const int t = pos_[c] <= pos[j] ? 0 : (int) (std::lower_bound(pos + j, pos + end, pos_[c]) - (pos + j));
+                row[(size_t) t * words32 + (c >> 5)] |= 1u << (c & 31);
             }
+            for (int t = j + 1; t < end; t++, row += words32) for (int w = 0; w < words32; w++) row[words32 + w] |= row[w];
             j = end - 1;
             continue;
         }

@@ -234,3 +234,33 @@ def test_mask_of_a_sequence_s_consecutive_tokens():
         got = dev.mask(n_kv, pos, seqs)
         for j, (p, s) in enumerate(zip(pos, seqs)):
             assert [bool(b) for b in got[j]] == [dev.lib.pi_kvcells_nseq(dev.h, c) > 0 and bool(dev.lib.pi_kvcells_has(dev.h, c, s[0])) and dev.lib.pi_kvcells_pos(dev.h, c) <= p for c in range(n_kv)]
+
+
+def test_mask_of_cells_that_came_round_again_costs_no_more_than_token_by_token():
+    """a cache of 4096 cells whose positions start in its middle (cells allotted again): the rows of 8 consecutive tokens together take no longer than one by one (a quarter of that here; sorted by position they took four times as long)"""
+    import time
+    lib, n, T = LL.api(), 4096, 8
+    h = lib.pi_kvcells_new(n)
+    pos = np.roll(np.arange(n - T, dtype=np.int32), n // 3)
+    one, ids = np.ones(n, np.int32), np.zeros(n * MAX_SEQ, np.int32)
+    assert lib.pi_kvcells_decode(h, n - T, O._ptr(pos), O._ptr(one), O._ptr(ids), MAX_SEQ) == 0
+    new = np.arange(n - T, n, dtype=np.int32)
+    assert lib.pi_kvcells_decode(h, T, O._ptr(new), O._ptr(one), O._ptr(ids), MAX_SEQ) >= 0
+    rows, singles = np.zeros((T, n // 32), np.uint32), np.zeros((T, n // 32), np.uint32)
+
+    def together():
+        lib.pi_kvcells_mask(h, n, T, O._ptr(new), O._ptr(one), O._ptr(ids), MAX_SEQ, O._ptr(rows))
+
+    def one_by_one():
+        for j in range(T):
+            lib.pi_kvcells_mask(h, n, 1, O._ptr(new[j:]), O._ptr(one), O._ptr(ids), MAX_SEQ, O._ptr(singles[j:]))
+
+    def best(f):
+        times = []
+        for _ in range(9):
+            t = time.perf_counter(); f(); times.append(time.perf_counter() - t)
+        return min(times)
+
+    a, b = best(together), best(one_by_one)
+    assert np.array_equal(rows, singles) and rows.any()
+    assert a < b, (a, b)
