@@ -22,8 +22,8 @@ struct pa_args {
 bool pa_takes(const pa_args & a, int maps, int min_tokens);
 void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s);
 // Which passes take tiles of 32 tokens rather than a workgroup per token (measured against each other over 9 .. 128 tokens, 16 and 32 heads, contexts of the pass's own tokens, 512 .. 1000 and 4096 cells, us):
-//   keys in a cache     from 32 tokens on: 16 heads of 128 over 4: 32 tokens in a window of 256 of 1000 cells 84 -> 47, all of 4096 cells 1082 -> 359, but 18 -> 23 where they are alone in the cache; 128 tokens
-//                       alone 38 -> 24.  With 16 tokens the per-token kernel cuts the cells into splits: 32 against 41
+//   keys in a cache     from 32 tokens on: 16 heads of 128 over 4: 32 tokens in a window of 256 of 1000 cells 76 -> 36, all of 4000 cells 1060 -> 251, alone in the
+//                       cache 15.7 -> 14.8; 128 tokens alone 38 -> 17.  Fewer tokens: k_few_attention (31 of them over all of 1000 cells 31)
 //   keys of a latent    from 9 tokens on, but for the passes that k_latent_rows (hybrid.hip: splits of 32 cells) takes: 16 heads of 128, rank 512, without those: 9 tokens alone 74 -> 27, of 512 cells 179 -> 65, of 4096
 //                       440 -> 379; 128 tokens 123 -> 38, 213 -> 69, 836 -> 374
 #define PA_CACHE_TOKENS 32

@@ -55,7 +55,8 @@ static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c)
 
 // NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
 // weights of the cells 4 g + c of a tile of 16, and of the sums the outputs 4 NV (4 g + c) + j.  N1 > 0: whole steps only (dim1 = 16 N1, dim2 = 16 (NK - N1), vdim = 64 NV) and 32-bit offsets, so that a row's
-// loads differ by constants: with an address apiece the registers held no more than one load at a time (2048 tokens, 32 heads of 128: 546 us, 495 this way)
+// loads differ by constants: with an address apiece the registers held no more than one load at a time (2048 tokens, 32 heads of 128: 546 us, 495 this way), and the queries and
+// the outputs have no test per value (32 tokens alone in a cache, 16 heads of 128 over 4: 20.2 us, 14.8 this way; a workgroup per token 15.7)
 template <int NK, int N1, int NV, int MAPS>
 __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_prompt_attention(const pa_args A, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 5)) return;
@@ -66,8 +67,8 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, map = wave % MAPS, part = wave / MAPS;
     const int h = blockIdx.x, t0 = (int) (gridDim.y - 1 - blockIdx.y) * 32;       // (the last tokens, which see the most, first)
     const int n_kv = min(A.dyn ? A.dyn[1] : A.n_kv, A.n_kv), c_end = min(n_kv, A.cell1), words = (A.n_kv + 31) / 32;
-    const int n1 = N1 > 0 ? N1 : (A.dim1 + 15) / 16;
-    const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * A.dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
+    const int dim1 = N1 > 0 ? 16 * N1 : A.dim1, dim2 = N1 > 0 ? 16 * (NK - N1) : A.dim2, vdim = N1 > 0 ? VW : A.vdim, n1 = (dim1 + 15) / 16;
+    const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
     const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
     pa_f32x4 q[2][NK], acc[2][NJ];
     float m_run[2] = { -INFINITY, -INFINITY }, l_run[2] = { 0.0f, 0.0f };
@@ -78,18 +79,18 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         const int t = min(t0 + 16 * u + n, A.n_tok - 1), p = A.pos ? A.pos[t] : 0;
         mrow[u] = A.mask + (int64_t) t * words;
         first_pos[u] = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
-        const float * qr = A.q + (int64_t) t * A.qs + (int64_t) (h * MAPS + map) * (A.dim1 + A.dim2);
+        const float * qr = A.q + (int64_t) t * A.qs + (int64_t) (h * MAPS + map) * (dim1 + dim2);
 #pragma unroll
         for (int i = 0; i < NK; i++)
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int d = (i < n1 ? i : i - n1) * 16 + 4 * g + c;
                 float x = 0.0f;                                       // (values past the end: the keys there repeat others)
-                if (i < n1) { if (d < A.dim1) x = qr[d]; }
-                else if (d < A.dim2) {
-                    const pi_turn r = pi_turn_of(d, A.dim2 / 2, A.pairing);
-                    const float2 t2 = A.cs[(int64_t) min(p, A.n_pos - 1) * (A.dim2 / 2) + r.angle];
-                    const float own = qr[A.dim1 + d], other = qr[A.dim1 + r.mate];
+                if (i < n1) { if (d < dim1) x = qr[d]; }
+                else if (d < dim2) {
+                    const pi_turn r = pi_turn_of(d, dim2 / 2, A.pairing);
+                    const float2 t2 = A.cs[(int64_t) min(p, A.n_pos - 1) * (dim2 / 2) + r.angle];
+                    const float own = qr[dim1 + d], other = qr[dim1 + r.mate];
                     x = r.lead ? own * t2.x - other * t2.y : own * t2.x + other * t2.y;
                 }
                 q[u][i][c] = x;
@@ -135,7 +136,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
                 for (int i = 0; i < NK; i++) {
                     const int d = (i < n1 ? i : i - n1) * 16 + 4 * g;
-                    kf[i] = i < n1 || A.dim2 == 0 ? *(const pa_f32x4 *) (kr1 + min(d, A.dim1 - 4)) : *(const pa_f32x4 *) (kr2 + min(d, A.dim2 - 4));
+                    kf[i] = i < n1 || dim2 == 0 ? *(const pa_f32x4 *) (kr1 + min(d, dim1 - 4)) : *(const pa_f32x4 *) (kr2 + min(d, dim2 - 4));
                 }
             }
             auto values = [&]() {
@@ -149,7 +150,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                     } else {
                         const float * vr = vb + (int64_t) cell * A.v_row;
 #pragma unroll
-                        for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, A.vdim - 4));
+                        for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, vdim - 4));
                     }
                 }
             };
@@ -224,10 +225,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         __syncthreads();
         const int r = tid >> 4, t = t0 + 16 * u + r, v0 = (tid & 15) * 4;
         pa_f32x4 o[MAPS][NV]; float M[MAPS], L[MAPS];
-        float * st = A.state ? A.state + ((int64_t) min(t, A.n_tok - 1) * A.heads + h) * (A.vdim + 2) : nullptr;
+        float * st = A.state ? A.state + ((int64_t) min(t, A.n_tok - 1) * A.heads + h) * (vdim + 2) : nullptr;
 #pragma unroll
         for (int mp = 0; mp < MAPS; mp++) {
-            M[mp] = st && !A.first ? st[A.vdim] : -INFINITY; L[mp] = 0.0f;
+            M[mp] = st && !A.first ? st[vdim] : -INFINITY; L[mp] = 0.0f;
             const float m_before = M[mp];
             if (soft) {
 #pragma unroll
@@ -237,12 +238,12 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             for (int j = 0; j < NV; j++) o[mp][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
             if (st && !A.first) {
                 const float f = !soft ? 1.0f : m_before == -INFINITY ? 0.0f : expf(m_before - M[mp]);
-                L[mp] = st[A.vdim + 1] * f;
+                L[mp] = st[vdim + 1] * f;
                 if (f > 0.0f)
 #pragma unroll
                     for (int j = 0; j < NV; j++)
 #pragma unroll
-                        for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) o[mp][j][e] = st[v0 + 64 * j + e] * f;
+                        for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < vdim) o[mp][j][e] = st[v0 + 64 * j + e] * f;
             }
 #pragma unroll
             for (int w = 0; w < PARTS; w++) {
@@ -262,7 +263,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                 if (A.cell_pos && A.cell_pos[cell] < fp && A.cell_pos[cell] >= A.keep_first) continue;
 #pragma unroll
                 for (int j = 0; j < NV; j++) {
-                    const pa_f32x4 x = *(const pa_f32x4 *) (vb + (int64_t) (cell - A.cell0) * A.v_row + min(v0 + 64 * j, A.vdim - 4));
+                    const pa_f32x4 x = *(const pa_f32x4 *) (vb + (int64_t) (cell - A.cell0) * A.v_row + min(v0 + 64 * j, vdim - 4));
 #pragma unroll
                     for (int e = 0; e < 4; e++)
                         if ((__float_as_uint(x[e]) & 0x7fffffffu) >= 0x7f800000u)
@@ -275,8 +276,8 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
             for (int j = 0; j < NV; j++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) st[v0 + 64 * j + e] = o[0][j][e];
-            if (v0 == 0) { st[A.vdim] = M[0]; st[A.vdim + 1] = L[0]; }
+                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < vdim) st[v0 + 64 * j + e] = o[0][j][e];
+            if (v0 == 0) { st[vdim] = M[0]; st[vdim + 1] = L[0]; }
             continue;
         }
         if (soft) {
@@ -297,10 +298,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
             for (int j = 0; j < NV; j++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < A.vdim) { const float x = o[0][j][e] - A.lam * o[1][j][e]; o[0][j][e] = x; ss = fmaf(x, x, ss); }
+                for (int e = 0; e < 4; e++) if (v0 + 64 * j + e < vdim) { const float x = o[0][j][e] - A.lam * o[1][j][e]; o[0][j][e] = x; ss = fmaf(x, x, ss); }
 #pragma unroll
             for (int s = 1; s < 16; s <<= 1) ss += __shfl_xor(ss, s, 64);
-            mult = A.out_mult / sqrtf(ss / (float) A.vdim + A.eps);
+            mult = A.out_mult / sqrtf(ss / (float) vdim + A.eps);
         } else if (A.gate && A.gate_width == 1) {
             float gt = A.gate[(int64_t) t * A.gs + h];
             if (A.gate_act == PI_ACT_SIGMOID) gt = 1.0f / (1.0f + expf(-gt));
@@ -311,14 +312,14 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const int v = v0 + 64 * j + e;
-                if (v >= A.vdim) continue;
+                if (v >= vdim) continue;
                 float x = o[0][j][e] * mult;
                 if (MAPS == 1 && A.gate && A.gate_width > 1) {
-                    float gt = A.gate[(int64_t) t * A.gs + (int64_t) h * A.vdim + v];
+                    float gt = A.gate[(int64_t) t * A.gs + (int64_t) h * vdim + v];
                     if (A.gate_act == PI_ACT_SIGMOID) gt = 1.0f / (1.0f + expf(-gt));
                     x *= gt;
                 }
-                A.out[(int64_t) t * A.os + (int64_t) h * A.vdim + v] = x;
+                A.out[(int64_t) t * A.os + (int64_t) h * vdim + v] = x;
             }
     }
 }
