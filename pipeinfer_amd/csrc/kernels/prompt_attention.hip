@@ -51,6 +51,18 @@ __global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restri
     }
 }
 
+// lane l: which of the 32 cells from c0 + step * l on lie at position `first` or behind it, or ahead of `keep` (the whole wave calls; two runs of 32 cells per load, so that a load is two lines of memory)
+static __device__ __forceinline__ uint32_t pa_near(const int32_t * __restrict__ cell_pos, int c0, int step, int c_end, int first, int keep, int lane) {
+    uint32_t near = 0;
+#pragma unroll 8
+    for (int i = 0; i < 32; i++) {
+        const int cp = cell_pos[min(c0 + step * (2 * i + (lane >> 5)) + (lane & 31), c_end - 1)];
+        const unsigned long long both = __ballot(cp >= first || cp < keep);
+        if (lane >> 1 == i) near = (uint32_t) (lane & 1 ? both >> 32 : both);
+    }
+    return near;
+}
+
 static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
@@ -100,7 +112,38 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         for (int j = 0; j < NJ; j++) acc[u][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
     }
     const float bias = A.hbias ? A.hbias[h] : 0.0f;
-    for (int c0 = (A.cell0 & ~31) + 32 * part; c0 < c_end; c0 += 32 * PARTS) {
+    // Contexts whose walk is long: a lane looks at a run of 32 cells, the wave at 64 of its runs at a time, and only those are walked that hold a cell which one of the tokens may see (32 tokens in a window of 256 of 60000
+    // cells: 160 us a workgroup per token, 630 with every run walked, 77 so; up to 64 runs of a wave the walk itself is as quick)
+    const int start = (A.cell0 & ~31) + 32 * __builtin_amdgcn_readfirstlane(part);
+    const bool far = c_end - start > 64 * 32 * PARTS;
+    int first_min = 0;
+    if (far) {
+        first_min = min(first_pos[0], first_pos[1]);
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) first_min = min(first_min, __shfl_xor(first_min, o, 64));
+        first_min = __builtin_amdgcn_readfirstlane(first_min);
+    }
+    unsigned long long todo = 0;
+    for (int c0 = start; c0 < c_end; c0 += 32 * PARTS) {
+        if (far) {
+            const int at = (c0 - start) / (32 * PARTS) & 63;
+            if (at == 0) {
+                const int c = c0 + 32 * PARTS * lane;
+                uint32_t any = 0;
+                if (c < c_end) {
+#pragma unroll 8
+                    for (int t = 0; t < 32; t++) any |= A.mask[(int64_t) min(t0 + t, A.n_tok - 1) * words + (c >> 5)];
+                }
+                if (A.cell_pos) any &= pa_near(A.cell_pos, c0, 32 * PARTS, c_end, first_min, A.keep_first, lane);
+                todo = __ballot(any != 0);
+            }
+            if (~todo) {
+                const unsigned long long rest = todo >> at;
+                const int skip = rest ? __ffsll(rest) - 1 : 63 - at;
+                c0 += 32 * PARTS * skip;
+                if (!rest) continue;
+            }
+        }
         uint32_t vis[2];
         const uint32_t in = (c_end - c0 >= 32 ? 0xffffffffu : (1u << (c_end - c0)) - 1u) & (c0 < A.cell0 ? 0xffffffffu << (A.cell0 - c0) : 0xffffffffu);
 #pragma unroll
@@ -356,9 +399,12 @@ void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * w
 
 // ---- a few tokens ---------------------------------------------------------------------------------------------------------------------------------------------------
 // grid (token, key head; split).  A workgroup per token that stages keys, then scores them, then stages values, waits for memory at every one of these (29 us for 4 tokens of 16 differential heads in a window of 256
-// of 700 cells); here the keys and values of 32 cells are on their way together, the scores of the key head's query heads are one tile of a matrix product, and so is every 16 outputs of theirs (XX
-// merge 6.6 instead of 4.5 for there are more splits; 8 tokens of 32 sigmoid heads over 40 to 350 cells: 31 us, now 8.0 and a merge of 5).  Lane layout as above, rows = query heads: scores of row n and the cells 4 g + c, sums of row n and the outputs 16 NV wave + NV (4 g + r) + j
-template <int NK, int NV, int MAPS>
+// of 700 cells); here the keys and values of 32 cells are on their way together, the scores of the key head's query heads are one tile of a matrix product, and so is every 16 outputs of theirs.  With the merge of the
+// splits, us: 4 tokens of 16 differential heads over 4 key heads in a window of 256 of 700 cells 34 -> 12.8; 8 tokens of 32 sigmoid heads in chunks of 64 of 350 cells 24 -> 8.9.
+// Lane layout as above, rows = query heads: scores of row n and the cells 4 g + c, sums of row n and the outputs 16 NV wave + NV (4 g + r) + j
+// FAR: splits of many runs of 32 cells: a lane looks at a run, the wave at 64 of them at a time (us for tokens in a window of 256 of 4000 cells, a context of 65536, 32 sigmoid heads: 35 with every run walked, 19 so; 16 tokens of 16 key heads in chunks of
+// 512 of 60000 cells: 108 with a workgroup per token, 149, 36)
+template <int NK, int NV, int MAPS, bool FAR>
 __global__ void __launch_bounds__(256) k_few_attention(const pa_args A, int n_cs, int split_cells, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int V = 64 * NV, STEPS = MAPS == 2 ? NK : NK / 2;       // one map: two waves share a tile's key values
@@ -386,11 +432,29 @@ __global__ void __launch_bounds__(256) k_few_attention(const pa_args A, int n_cs
         for (int j = 0; j < NV; j++) acc[mp][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
     }
     bool any = false;
-    for (int c0 = cs * split_cells; c0 < c_end; c0 += 32) {
-        const int mc = c0 + (lane & 31);
-        bool see = false;
-        if (mc < c_end) { const int cp = A.cell_pos[mc]; see = (A.mask[(int64_t) t * words + (c0 >> 5)] >> (lane & 31) & 1u) && (cp >= first || cp < A.keep_first); }
-        const uint32_t vis = (uint32_t) __ballot(see);
+    const int start = cs * split_cells;
+    uint32_t seen = 0;
+    for (int c0 = start; c0 < c_end; c0 += 32) {
+        uint32_t vis;
+        if constexpr (FAR) {
+            const int at = (c0 - start) >> 5 & 63;
+            if (at == 0) {
+                const int c = c0 + 32 * lane;
+                seen = c < c_end ? A.mask[(int64_t) t * words + (c >> 5)] : 0u;
+                if (c_end - c < 32 && c < c_end) seen &= (1u << (c_end - c)) - 1u;
+                seen &= pa_near(A.cell_pos, c0, 32, c_end, first, A.keep_first, lane);
+            }
+            const unsigned long long rest = __ballot(seen != 0) >> at;
+            const int skip = rest ? __ffsll(rest) - 1 : 63 - at;
+            c0 += 32 * skip;
+            if (!rest) continue;
+            vis = (uint32_t) __builtin_amdgcn_readlane((int) seen, at + skip);
+        } else {
+            const int mc = c0 + (lane & 31);
+            bool see = false;
+            if (mc < c_end) { const int cp = A.cell_pos[mc]; see = (A.mask[(int64_t) t * words + (c0 >> 5)] >> (lane & 31) & 1u) && (cp >= first || cp < A.keep_first); }
+            vis = (uint32_t) __ballot(see);
+        }
         if (gone & 1) break;                                          // (a cancelled run: its keys and values are not read)
         if (!vis) continue;
         pa_f32x4 kf[STEPS]; vec vf[2][4];
@@ -491,8 +555,10 @@ int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split
 void pa_few_launch(const pa_args & a, int maps, int n_cs, int split_cells, double bytes, hipStream_t s) {
     const dim3 grid((unsigned) (a.n_tok * (a.heads / a.per_kv)), (unsigned) n_cs);
     const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
-#define FEW_GO(NK, NV) do { if (maps == 2) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_few_attention<NK, NV, 2>), grid, dim3(256), 0, s, a, n_cs, split_cells, pi_abort_word()); \
-                            else PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_few_attention<NK, NV, 1>), grid, dim3(256), 0, s, a, n_cs, split_cells, pi_abort_word()); } while (0)
+#define FEW_GO2(NK, NV, MAPS, FAR) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_few_attention<NK, NV, MAPS, FAR>), grid, dim3(256), 0, s, a, n_cs, split_cells, pi_abort_word())
+#define FEW_GO(NK, NV) do { if (maps == 2) { if (far) FEW_GO2(NK, NV, 2, true); else FEW_GO2(NK, NV, 2, false); } else { if (far) FEW_GO2(NK, NV, 1, true); else FEW_GO2(NK, NV, 1, false); } } while (0)
+    const bool far = split_cells > 256;                                // (up to eight runs the walk is as quick)
     if (a.dim1 == 64) { if (a.vdim == 64) FEW_GO(4, 1); else FEW_GO(4, 2); } else { if (a.vdim == 64) FEW_GO(8, 1); else FEW_GO(8, 2); }
+#undef FEW_GO2
 #undef FEW_GO
 }

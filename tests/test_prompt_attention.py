@@ -25,7 +25,7 @@ def test_latent_prompt(H, D, R, V, rank, T, n_kv):
 @pytest.mark.parametrize("H,D,R,V,rank", [(16, 8, 64, 24, 512), (5, 20, 36, 17, 512), (3, 8, 0, 33, 256), (7, 4, 4, 8, 256)])
 @pytest.mark.parametrize("T,n_kv", [(1, 33), (1, 700), (4, 64), (8, 130), (3, 4200)])
 def test_latent_few_tokens(H, D, R, V, rank, T, n_kv):
-    """sixteen rows (token, head) at a time over splits of 64 cells: rows and splits that are not full, more than 64 splits, a rotated part that ends inside a step"""
+    """sixteen rows (token, head) at a time over splits of 32 cells: rows and splits that are not full, more than 64 splits, a rotated part that ends inside a step"""
     U, lib = gpu()
     rng = np.random.default_rng(H * 100 + n_kv)
     pos = np.arange(n_kv - T, n_kv)
@@ -129,6 +129,37 @@ def test_window_prompt(H, G, D, V, size, keep, n_kv, T, maps):
     args = (q, kc, vc, cpos, vis, pos, 0.6 * D ** -0.25, size, keep, maps, 0.45, 0.7, 1e-3, H, G)
     want = diff_attention_ref(*(a[:n_kv] if a is kc or a is vc or a is cpos else a for a in args))
     assert rel_rms(run_diff(U, lib, *args, True), want) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 64, 64, 60, 3, 9300, 33), (2, 2, 36, 68, 60, 0, 17001, 40), (3, 1, 64, 128, 60, 3, 9300, 5), (2, 2, 128, 64, 5000, 0, 70001, 2), (2, 1, 64, 64, 0, 0, 8225, 32)])
+@pytest.mark.parametrize("maps", [2, 1])
+def test_window_in_a_long_context(H, G, D, V, size, keep, n_kv, T, maps):
+    """walks that look at 64 runs of 32 cells at a time and visit the ones with something to see (more than 8192 cells, 4096 of two maps; splits of more than 256): every run and few, cells in any order, the last run and the
+    last 64 not full; an infinity that nobody sees stays out"""
+    U, lib = gpu()
+    rng = np.random.default_rng(n_kv + T)
+    kc, vc = (rng.standard_normal((n_kv + 13, G, maps, D)) * 1.5).astype(np.float32), rng.standard_normal((n_kv + 13, G, V)).astype(np.float32)
+    kc[n_kv:], vc[n_kv:] = np.nan, np.nan
+    cpos, pos, vis = scattered(rng, T, n_kv, n_kv + 13)
+    q = (rng.standard_normal((T, H, maps, D)) * 2).astype(np.float32)
+    hidden = np.nonzero(~(vis & ((cpos[None, :n_kv] > pos[:, None] - size) | (cpos[None, :n_kv] < keep) | (size == 0))).any(0))[0][-1]
+    vc[hidden] = np.inf                                                # (nobody sees it)
+    args = (q, kc, vc, cpos, vis, pos, 0.6 * D ** -0.25, size, keep, maps, 0.45, 0.7, 1e-3, H, G)
+    clean = vc.copy()
+    clean[hidden] = 0
+    want = diff_attention_ref(*(clean[:n_kv] if a is vc else a[:n_kv] if a is kc or a is cpos else a for a in args))
+    assert rel_rms(run_diff(U, lib, *args, True), want) < 1e-5
+
+
+@pytest.mark.gpu
+def test_latent_prompt_in_a_long_context():
+    """the walk of the mask alone (keys written out of a latent), in one launch and in several over the cells"""
+    U, lib = gpu()
+    rng = np.random.default_rng(5)
+    for n_kv, rank in ((9300, 264), (30000, 128)):
+        got, want = latent_case(U, lib, rng, 2, 12, 4, 12, rank, n_kv, np.arange(n_kv - 9, n_kv), 500.0, NEIGHBOURS, 1, None, 0.3)
+        assert rel_rms(got, want) < 1e-5, n_kv
 
 
 @pytest.mark.gpu
