@@ -547,7 +547,9 @@ int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split
     auto four = [](int64_t n) { return (n & 3) == 0; };
     if (a.n_tok >= PA_CACHE_TOKENS || a.n_kv <= 64 || !a.state || a.per_kv > 16 || (a.dim1 != 64 && a.dim1 != 128) || (a.vdim != 64 && a.vdim != 128) || !four(a.k1_row) || !four(a.k1_head) || !four(a.v_row) || !four(a.v_head) ||
         (((uintptr_t) a.k1 | (uintptr_t) a.v) & 15)) return 0;
-    const int chunks = (a.n_kv + 31) / 32, per = (chunks + PA_FEW_SPLITS - 1) / PA_FEW_SPLITS, n_cs = (chunks + per - 1) / per;
+    const int most = std::max(1, std::min(PA_FEW_SPLITS, 8192 / (a.n_tok * (a.heads / a.per_kv))));      // (more workgroups than that only wait for each other: 31 tokens of 16 key heads, 64 live cells of 1024: 16.1 us with a workgroup per token, 20.3 with 32 splits, 13.7 with 16; 16 tokens,
+                                                                                                          // 200 cells of 4096: 15.4, with half as many workgroups 19.4)
+    const int chunks = (a.n_kv + 31) / 32, per = (chunks + most - 1) / most, n_cs = (chunks + per - 1) / per;
     if ((size_t) a.n_tok * a.heads * maps * n_cs * (a.vdim + 2) > scratch_floats) return 0;
     *split_cells = 32 * per;
     return n_cs;

@@ -132,7 +132,7 @@ def test_window_prompt(H, G, D, V, size, keep, n_kv, T, maps):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 64, 64, 60, 3, 9300, 33), (2, 2, 36, 68, 60, 0, 17001, 40), (3, 1, 64, 128, 60, 3, 9300, 5), (2, 2, 128, 64, 5000, 0, 70001, 2), (2, 1, 64, 64, 0, 0, 8225, 32)])
+@pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(2, 1, 64, 64, 60, 3, 9300, 33), (2, 2, 36, 68, 60, 0, 17001, 40), (3, 1, 64, 128, 60, 3, 9300, 5), (2, 2, 128, 64, 5000, 0, 70001, 2), (2, 1, 64, 64, 0, 0, 8225, 32), (32, 32, 64, 64, 0, 0, 700, 31)])
 @pytest.mark.parametrize("maps", [2, 1])
 def test_window_in_a_long_context(H, G, D, V, size, keep, n_kv, T, maps):
     """walks that look at 64 runs of 32 cells at a time and visit the ones with something to see (more than 8192 cells, 4096 of two maps; splits of more than 256): every run and few, cells in any order, the last run and the
