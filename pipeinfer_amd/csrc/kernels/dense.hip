@@ -230,16 +230,10 @@ static void launch_rows(const pi_weight * w, const float * x, int64_t xs, int n_
     else PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, nt_acct, bytes, (k_dense_rows<8, VW, EXACT>), dim3(gx, (unsigned) ((n_tok + 7) / 8)), dim3(256), 0, s, W, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word());
 }
 
-// Which kernel takes a pass of serving precision (aligned rows; measured against each other over 512 .. 32000 rows, K 1024 .. 4096, us):
-//   1 token                the mat-vec; 2 tokens of a matrix of at most 4 M values too (2048 x 2048: 5.5, k_dense_split 5.7: both at the floor of a launch)
-//   .. 32 tokens           k_dense_split (4096 x 4096 at 4 / 8 / 16 / 32 tokens: 9.7 / 11 / 14 / 21; the mat-vec 15 / 28 at 4 / 8, k_dense_tile 27 at 32); of 16384 rows and more only .. 8 tokens, where the tiles
-//                          fill the chip and read the activations less often (32000 x 2048 at 24: 41 against 26)
-//   more                   k_dense_tile
-static bool dense_takes_split(int64_t rows, int64_t k, int n_tok) { return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32) && !(n_tok == 2 && rows * k <= (4 << 20)); }
 // Rows per workgroup: the chip's 256 compute units take a workgroup each at a time, and a round of them lasts about as long as 8 + rows (K 4096 at 8 tokens: 16 rows 7.8 us a round, 24 10, 32 13; the launch itself 4).  So
 // the split that needs the least, in steps of 4 rows, the larger one of two that need the same.  Against 16 rows (32 from 8192 rows on), us at 2 .. 4 / 8 / 32 tokens: 6144 x 4096 17.6 / 19.8 / 39.0, now 24 rows
 // 13.3 / 14.5 / 24.2; 5120 x 13824 46.6 / 59.3 / 123, now 20 rows 32.8 / 37.8 / 71.7; 16448 x 4096 at 8 41.5, now 24 rows 37.6; 32000 x 4096 at 4 63.8, now 32 rows 52.5; 2048 x 2048 6.5 / 7.0 / 11.8, now 8 rows
-// 5.9 / 6.4 / 11.2; 8192 x 4096 at 2 the one that loses, 16.2, now 32 rows 17.0 (at 4 17.8 and 17.0)
+// 5.9 / 6.4 / 11.2
 static int split_rows(int64_t n, int64_t seg_rows) {
     int best = 16; int64_t least = INT64_MAX;
     for (int r = 32; r >= 4; r -= 4) {
@@ -247,6 +241,16 @@ static int split_rows(int64_t n, int64_t seg_rows) {
         if (cost < least && (seg_rows <= 0 || seg_rows % r == 0)) { least = cost; best = r; }
     }
     return best;
+}
+// Which kernel takes a pass of serving precision (aligned rows; measured against each other over 512 .. 32000 rows, K 1024 .. 4096, us):
+//   1 token                the mat-vec; 2 tokens of a matrix of at most 4 M values too (2048 x 2048: 5.5, k_dense_split 5.7: both at the floor of a launch), and rows of 8 KB where
+//                          k_dense_split would take 32 of them a workgroup (their addresses meet: 8192 rows of 3968 / 4096 / 4224 values 12.6 / 16.4 / 13.3, the mat-vec 14.7 / 14.9 / 16.3; 32000 rows of 4096 52.7
+//                          and 47.1; from 3 tokens on the mat-vec is slower there too, 19.1 for 8192 rows)
+//   .. 32 tokens           k_dense_split (4096 x 4096 at 4 / 8 / 16 / 32 tokens: 9.7 / 11 / 14 / 21; the mat-vec 15 / 28 at 4 / 8, k_dense_tile 27 at 32); of 16384 rows and more only .. 8 tokens, where the tiles
+//                          fill the chip and read the activations less often (32000 x 2048 at 24: 41 against 26)
+//   more                   k_dense_tile
+static bool dense_takes_split(int64_t rows, int64_t k, int n_tok, int64_t seg_rows = 0) {
+    return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32) && !(n_tok == 2 && (rows * k <= (4 << 20) || (k == 4096 && split_rows(rows, seg_rows) == 32)));
 }
 static void launch_split(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias, int64_t seg_rows = 0,
                          int64_t seg_off = 0, int seg_last = 0) {
@@ -305,11 +309,11 @@ extern "C" int pi_op_dense_segments(const pi_weight * w, const float * x, int64_
     const int64_t K = w->ne0;
     if (x_stride < (int64_t) (n_seg - 1) * seg_off + K || out_stride < w->ne1) { pi_set_error("pi_op_dense_segments: row strides below the sizes"); return -1; }
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0 && seg_off % 4 == 0;
-    if (!exact && al16 && dense_takes_split(w->ne1, K, n_tok) && seg_rows % 32 == 0) {
+    if (!exact && al16 && dense_takes_split(w->ne1, K, n_tok, seg_rows) && seg_rows % 32 == 0) {
         launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, (hipStream_t) stream, 2.0 * K * w->ne1 + 4.0 * n_tok * (n_seg * K + w->ne1), nullptr, seg_rows, seg_off, n_seg - 1);
         PI_CHECK_LAUNCH(); return 0;
     }
-    if (exact || !al16 || n_tok < 16) {
+    if (exact || !al16 || n_tok < 16) {                                // (up to 15 tokens of segments that no split fits one launch of mat-vecs: 5 segments of 1000 rows, K 4096, 15 tokens 51 us, a launch each 55)
         const bool al8 = K % 4 == 0 && ((uintptr_t) w->p0 % 8) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0 && seg_off % 4 == 0;
         const double bytes = 2.0 * K * w->ne1 + 4.0 * n_tok * (n_seg * K + w->ne1);
         hipStream_t s = (hipStream_t) stream;

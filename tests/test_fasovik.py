@@ -167,6 +167,19 @@ def upload_bf16(lib, w):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [8192, 8191, 8224])
+def test_dense_two_tokens_of_rows_of_8_kb(N):
+    """4096 values a row, 32 rows and fewer per workgroup: on both sides of the line between the mat-vec and the split kernel (fp32 sums of 4096 exact products: 2e-6 of their mean)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(N)
+    w, x = bf(rng, N, 4096, s=0.02), rng.standard_normal((2, 4096)).astype(np.float32)
+    wd, xd, od = upload_bf16(lib, w), U.Dev(x), U.Dev(nbytes=8 * N)
+    L.check(lib.pi_op_dense(wd, xd.ptr, 4096, 2, od.ptr, N, 0, N, 0, 0, None))
+    assert rel_rms(od.get(np.float32, (2, N)), O.bf16_round(x).astype(np.float64) @ w.T.astype(np.float64)) < 2e-6
+    lib.pi_weight_free(wd)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K,N,T", [(40, 37, 1), (33, 10, 3), (512, 70, 5), (1024, 130, 8), (96, 200, 17), (64, 64, 64), (520, 33, 150), (256, 300, 200), (72, 130, 129)])
 @pytest.mark.parametrize("exact", [True, False])
 def test_dense_every_kernel_and_width(K, N, T, exact):
