@@ -1060,7 +1060,8 @@ static bool lat_rows_takes(int heads, int rank, int rot, int n_tok, int n_ctx) {
 // grid (token tile of 4, head, 64 values of the rank, then 64 values of the rotated part): lane = one rank value, the four waves take a quarter of the head's dim each and meet in LDS.  A query head is
 // [dim values | rot values]; the last are turned in pairs by the token's position (cs: the rotation table) and go behind the rank values
 __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict__ q, int64_t qs, const uint16_t * __restrict__ wuk, float scale, int heads, int dim, int rank, int rot, const float2 * __restrict__ cs, int n_pos,
-                                                       int pairing, const int32_t * __restrict__ pos, int n_tok, float * __restrict__ qa, const int32_t * __restrict__ abort_w) {
+                                                       int pairing, const int32_t * __restrict__ pos, int n_tok, float * __restrict__ qa, const int32_t * __restrict__ dyn, int live_min, const int32_t * __restrict__ abort_w) {
+    if (live_min > 0 && dyn[1] <= live_min) return;                    // (a pass that prompt_attention.hip takes: latent_tiles_to)
     const int gone = pi_abort_peek(abort_w);
     __shared__ float part[4][4][64];
     extern __shared__ float4 qsh[];                                    // [dim]: the head's query values of the four tokens, side by side
@@ -1101,8 +1102,8 @@ __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict_
 
 template <int M, int RPT>
 __global__ void __launch_bounds__(256) k_latent_scores(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int rank, int rot, int n_kv_arg,
-                                                       int cap, int S, float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 5)) return;
+                                                       int cap, int S, float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, int live_min, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 5) || (live_min > 0 && dyn[1] <= live_min)) return;
     extern __shared__ float lds[];
     const int t = blockIdx.x, h0 = blockIdx.y * M, split = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rthreads = (rank + RPT - 1) / RPT, G = max(1, 256 / rthreads);
@@ -1265,7 +1266,7 @@ __global__ void __launch_bounds__(256) k_latent_scores(const float * __restrict_
 // LOOP: fewer workgroups than splits, each takes several (a loop of one round costs 77 -> 85 us: 4 tokens x 16 heads, 16384 cells)
 template <int NJ, int EX, bool LOOP>
 __global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_rows(const float * __restrict__ qa, const float * __restrict__ cache, const uint32_t * __restrict__ mask, int heads, int W, int n_rows, int n_kv_arg, int S,
-                                                        float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
+                                                        float * __restrict__ pol, float * __restrict__ pml, const int32_t * __restrict__ dyn, int live_max, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int RANK = 64 * NJ, NS = RANK / 16 + EX, NH = NS / 2;
     __shared__ __attribute__((aligned(16))) float ps[16][36], half[2][16][20];
@@ -1273,7 +1274,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_r
     const int words = (n_kv_arg + 31) / 32, n_kv = min(dyn ? dyn[1] : n_kv_arg, n_kv_arg);
     const uint32_t first = mask[(int64_t) (min((int) (blockIdx.x * 16 + (threadIdx.x & 15)), n_rows - 1) / heads) * words + blockIdx.y];      // (on its way beside the number of live cells)
     int split = blockIdx.y;
-    if (split * 32 >= n_kv) return;                                    // (cells of the context that hold nothing yet)
+    if (split * 32 >= n_kv || (live_max > 0 && n_kv > live_max)) return;       // (cells of the context that hold nothing yet; a pass that the kernels per token take)
     do {                                                               // (a barrier lies between a round's last look at the LDS and the next one's writes to the same place)
         int tid = threadIdx.x;
         if constexpr (LOOP) asm volatile("" : "+v"(tid));              // (queries and addresses are made again in every round: kept from one to the next they take the registers of a second workgroup)
@@ -1396,8 +1397,9 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_r
 // MANY: more than eight splits (the code for them costs the launches of fewer 0.3 us of 9.5)
 template <bool MANY>
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
-                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, const int32_t * __restrict__ dyn, int vec, float * __restrict__ out, int64_t os,
+                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, const int32_t * __restrict__ dyn, int live_min, int live_max, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
+    if ((live_min > 0 && dyn[1] <= live_min) || (live_max > 0 && dyn[1] > live_max)) return;
     const int gone = pi_abort_peek(abort_w);
     extern __shared__ __attribute__((aligned(16))) float ol[];                                     // [4][rank]
     __shared__ float wgt[4][64];                                      // per token: weight of the splits that hold something, 64 splits at a time,
@@ -1591,8 +1593,8 @@ extern "C" int pi_op_latent_attention_reserve(void) {
 }
 template <int M, int RPT>
 static void latent_scores_launch(const lat_plan & p, dim3 grid, hipStream_t s, double bytes, int nta, const float * qa, const float * cache, const uint32_t * mask, int heads, int rank, int rot, int n_kv,
-                                 float * pol, float * pml, const int32_t * dyn) {
-    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_scores<M, RPT>), grid, dim3(256), p.lds, s, qa, cache, mask, heads, rank, rot, n_kv, p.cap, p.S, pol, pml, dyn, pi_abort_word());
+                                 float * pol, float * pml, const int32_t * dyn, int live_min) {
+    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_scores<M, RPT>), grid, dim3(256), p.lds, s, qa, cache, mask, heads, rank, rot, n_kv, p.cap, p.S, pol, pml, dyn, live_min, pi_abort_word());
 }
 extern "C" int pi_op_latent_attention(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev,
                                       float scale, int heads, int dim, int vdim, int rank, int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride,
@@ -1606,26 +1608,44 @@ extern "C" int pi_op_latent_attention_rot(const float * q, int64_t q_stride, con
     return pi_op_latent_attention_gated(q, q_stride, cache, mask, wuk, wuv, sink_dev, gate_dev, gate_stride, gate_act, 1, scale, heads, dim, rot, vdim, rank, rotary_table, PI_PAIR_NEIGHBOURS, pos_dev, n_tok, n_kv, scratch_dev,
                                         scratch_floats, out, out_stride, dyn_dev, stream);
 }
-// A prompt with its keys and values written out (prompt_attention.hip), in as few launches over the cells as the scratch memory allows; false: not for that kernel
-static bool latent_prompt(pa_args a, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, size_t scratch_floats, double bytes, hipStream_t s) {
-    if ((rank & 7) || (a.k2_row & 3) || ((uintptr_t) cache & 15) || ((uintptr_t) scratch & 15)) return false;
+// How many live cells the tiles of a prompt are the better for.  They walk all cells with a workgroup per head and 32 tokens: few heads and tokens over a long context leave most of the chip idle, where k_latent_scores has
+// a workgroup per token, tile of heads and 1280 .. 2048 cells.  Both by what was measured (8 .. 128 heads, ranks 128 .. 768, 9 .. 256 tokens, 40 .. 16000 cells), us: a tile's round of 128 cells 2 + 0.385 per step, the keys
+// and values written out at 1000 TFLOP/s, 8 for every pair of launches; a round of 256 workgroups per token 0.19 + 0.029 per head of the tile for 1000 cells x values.  The tiles give way where they are clearly slower:
+// tiles / workgroups per token 33 tokens of 16000 cells, 8 heads of rank 256 610 / 455, 16 of 512 + 64 1205 / 1060, 16 of 128 + 32 (in several launches) 1576 / 360, 9 tokens of them 1587 / 199; 128 heads, 9 tokens of
+// 4000 cells 751 / 480, of 300 100 / 184; 33 tokens of 512 of 65536, rank 512 114 / 202.
+// 0: none; n_kv: all.  The line between is looked at on the device, where the number of live cells is known: both sets of launches go out and one returns at once
+static int latent_tiles_to(const lat_plan & p, const pa_args & a, int rank, int launches) {
+    const double steps = (a.dim1 + 15) / 16 + (a.dim2 + 15) / 16 + 4 * ((a.vdim + 63) / 64);
+    const int64_t rounds = ((int64_t) a.heads * ((a.n_tok + 31) / 32) + 511) / 512, heads = (a.heads + p.M - 1) / p.M;
+    auto tiles = [&](int64_t live) { return (double) ((live + 127) / 128 * rounds) * (2.0 + 0.385 * steps) + 6e-9 * (double) live * a.heads * (a.dim1 + a.vdim) * rank + 8.0 * launches; };
+    auto tokens = [&](int64_t live) { return std::ceil((double) (a.n_tok * heads) * live / p.cap / 256) * (double) std::min<int64_t>(live, p.cap) * (rank + a.dim2) * (1.9e-4 + 2.9e-5 * p.M) + 25.0; };
+    int64_t to = a.n_kv, live = a.n_kv;                                // down from all cells as long as the tiles lose
+    while (live >= 64 && 0.72 * tiles(live) > tokens(live)) { to = live = live * 5 / 7; }
+    return live < 64 ? 0 : (int) to;
+}
+// A prompt with its keys and values written out (prompt_attention.hip), in as few launches over the cells as the scratch memory allows.  How many live cells it took the pass for: 0 none, a.n_kv any
+static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, size_t scratch_floats, double bytes, hipStream_t s) {
+    if ((rank & 7) || (a.k2_row & 3) || ((uintptr_t) cache & 15) || ((uintptr_t) scratch & 15)) return 0;
     const size_t per_cell = (size_t) a.heads * (a.dim1 + a.vdim), state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3;
     size_t cells = ((size_t) a.n_kv + 63) / 64 * 64;
     if (cells * per_cell > scratch_floats) {
         cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
-        if (cells < 1024) return false;
+        if (cells < 1024) return 0;
         a.state = scratch + cells * per_cell;
     }
     a.k1 = scratch; a.k1_row = (int64_t) a.heads * a.dim1; a.k1_head = a.dim1;
     a.v = scratch + cells * (size_t) a.k1_row; a.v_row = (int64_t) a.heads * a.vdim; a.v_head = a.vdim;
     a.k2 = cache + rank;
-    if (!pa_takes(a, 1, PA_LATENT_TOKENS)) return false;
-    for (size_t c = 0; c < (size_t) a.n_kv; c += cells) {
-        a.cell0 = (int) c; a.cell1 = (int) std::min((size_t) a.n_kv, c + cells); a.first = c == 0; a.last = c + cells >= (size_t) a.n_kv;
-        pa_expand(cache, a.k2_row, rank, wuk, wuv, a.cell0, a.cell1, a.n_kv, a.dyn, scratch, scratch + cells * (size_t) a.k1_row, s);
+    if (!pa_takes(a, 1, PA_LATENT_TOKENS)) return 0;
+    const int to = latent_tiles_to(p, a, rank, (int) (((size_t) a.n_kv + cells - 1) / cells));
+    if (to == 0 || (to < a.n_kv && !a.dyn)) return 0;
+    a.live_max = to < a.n_kv ? to : 0;
+    for (size_t c = 0; c < (size_t) to; c += cells) {
+        a.cell0 = (int) c; a.cell1 = (int) std::min((size_t) to, c + cells); a.first = c == 0; a.last = c + cells >= (size_t) to;
+        pa_expand(cache, a.k2_row, rank, wuk, wuv, a.cell0, a.cell1, a.n_kv, a.live_max, a.dyn, scratch, scratch + cells * (size_t) a.k1_row, s);
         pa_launch(a, 1, bytes, s);
     }
-    return true;
+    return to;
 }
 extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev, const float * gate_dev,
                                             int64_t gate_stride, int gate_act, int gate_width, float scale, int heads, int dim, int rot, int vdim, int rank, const void * rotary_table, int pairing, const int32_t * pos_dev,
@@ -1662,34 +1682,50 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     const int S32 = (n_kv + 31) / 32;
     const bool whole = lat_rows_takes(heads, rank, rot, n_tok, n_kv) && (n_tok * heads >= 8 || n_kv < 4096) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats &&
                        (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
-    if (!whole && latent_prompt(a, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) { PI_CHECK_LAUNCH(); return 0; }
+    int live_min = 0;                                                  // the launches below are for passes of more live cells
+    if (!whole && (live_min = latent_prompt(a, p, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) > 0) {
+        PI_CHECK_LAUNCH();
+        if (live_min >= n_kv) return 0;
+    }
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * dim + 4.0 * n_tok * heads * (dim + rank + 2.0 * rot), k_latent_absorb, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((rank + 63) / 64 + (rot + 63) / 64)), dim3(256), (size_t) 16 * dim, s,
-                 q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, pi_abort_word());
+                 q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, dyn_dev, live_min, pi_abort_word());
     PI_CHECK_LAUNCH();
-    const dim3 grid((unsigned) n_tok, (unsigned) ((heads + p.M - 1) / p.M), (unsigned) p.S);
     const double bytes = 4.0 * acct * (rank + rot) + 4.0 * n_tok * heads * (rank + rot + (double) rank * p.S);
+    // most rows and more shares of the splits than the 256 MB of the last cache: the kernels per token (32 tokens of 16 heads, rank 512 + 64, us here / per token: 6000 cells 327 / 482, 9000 611 / 510, 16000 1029 / 968; of
+    // 24 tokens, 384 rows, 16000 cells still 695 / 973)
+    const int64_t rows_to = n_tok > 8 && dyn_dev && (int64_t) n_tok * heads * rank > 448 * 512 ? ((int64_t) 1 << 31) / ((int64_t) n_tok * heads * rank) : n_kv;
+    const int live_max = whole && rows_to < n_kv ? (int) rows_to : 0;
+#define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
+                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, S, n_tok, rows ? n_kv : 0, dyn_dev, rows ? 0 : live_min, rows ? live_max : 0, \
+                 vec, out, out_stride, pi_abort_word())
+    auto combine = [&](int S, bool rows) -> int {
+        const int vec = (rank & 7) == 0 && (rank >= 256 || S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
+        if (S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
+        PI_CHECK_LAUNCH(); return 0;
+    };
     if (whole) {
-        p.S = S32;
-        pml = pol + (size_t) n_tok * heads * p.S * rank;
+        pml = pol + (size_t) n_tok * heads * S32 * rank;
         const unsigned row_tiles = (unsigned) ((n_tok * heads + 15) / 16);
-        const dim3 rgrid(row_tiles, std::min((unsigned) p.S, std::max(1u, 4096u / row_tiles)));      // (a context that holds less than it could: 8 tokens x 32 heads, 512 cells of 65536, a workgroup for each of the 2048 splits: 129 us, so 35)
-#define LAT_ROWS2(NJ, EX, LOOP) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_rows<NJ, EX, LOOP>), rgrid, dim3(256), 0, s, qa, cache, mask, heads, rank + rot, n_tok * heads, n_kv, p.S, pol, pml, dyn_dev, pi_abort_word())
-#define LAT_ROWS(NJ, EX) do { if (rgrid.y < (unsigned) p.S) LAT_ROWS2(NJ, EX, true); else LAT_ROWS2(NJ, EX, false); } while (0)
+        const dim3 rgrid(row_tiles, std::min((unsigned) S32, std::max(1u, 4096u / row_tiles)));      // (a context that holds less than it could: 8 tokens x 32 heads, 512 cells of 65536, a workgroup for each of the 2048 splits: 129 us, so 35)
+#define LAT_ROWS2(NJ, EX, LOOP) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, bytes, (k_latent_rows<NJ, EX, LOOP>), rgrid, dim3(256), 0, s, qa, cache, mask, heads, rank + rot, n_tok * heads, n_kv, S32, pol, pml, dyn_dev, live_max, pi_abort_word())
+#define LAT_ROWS(NJ, EX) do { if (rgrid.y < (unsigned) S32) LAT_ROWS2(NJ, EX, true); else LAT_ROWS2(NJ, EX, false); } while (0)
         if (rank == 256) { if (rot) LAT_ROWS(4, 4); else LAT_ROWS(4, 0); } else { if (rot) LAT_ROWS(8, 4); else LAT_ROWS(8, 0); }
 #undef LAT_ROWS2
 #undef LAT_ROWS
-    } else {
-#define LAT_GO(M) do { if (p.RPT == 1) latent_scores_launch<M, 1>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); \
-                       else if (p.RPT == 2) latent_scores_launch<M, 2>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); \
-                       else latent_scores_launch<M, 4>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev); } while (0)
+        PI_CHECK_LAUNCH();
+        if (combine(S32, true) != 0) return -1;
+        if (live_max == 0) return 0;
+        live_min = live_max;
+        pml = pol + (size_t) n_tok * heads * p.S * rank;
+    }
+    const dim3 grid((unsigned) n_tok, (unsigned) ((heads + p.M - 1) / p.M), (unsigned) p.S);
+#define LAT_GO(M) do { if (p.RPT == 1) latent_scores_launch<M, 1>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev, live_min); \
+                       else if (p.RPT == 2) latent_scores_launch<M, 2>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev, live_min); \
+                       else latent_scores_launch<M, 4>(p, grid, s, bytes, nta, qa, cache, mask, heads, rank, rot, n_kv, pol, pml, dyn_dev, live_min); } while (0)
     switch (p.M) { case 16: LAT_GO(16); break; case 8: LAT_GO(8); break; case 4: LAT_GO(4); break; case 2: LAT_GO(2); break; default: LAT_GO(1); }
 #undef LAT_GO
-    }
     PI_CHECK_LAUNCH();
-    const int vec = (rank & 7) == 0 && (rank >= 256 || p.S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
-#define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * p.S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
-                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, p.S, n_tok, whole ? n_kv : 0, dyn_dev, vec, out, out_stride, pi_abort_word())
-    if (p.S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
+    return combine(p.S, false);
 #undef LAT_COMBINE
     PI_CHECK_LAUNCH(); return 0;
 }

@@ -8,6 +8,7 @@ struct pa_args {
     const float * k2; int64_t k2_row; int dim2;                        // ... then dim2 values that the heads share
     const float * v; int64_t v_row, v_head; int vdim;
     int cell0, cell1;                                                  // the cells of this launch; k1 and v begin at cell0, everything else at cell 0
+    int live_max;                                                      // > 0: a launch for passes of no more live cells than that (others return)
     int heads, per_kv, n_tok, n_kv; const int32_t * dyn;
     const uint32_t * mask; const int32_t * cell_pos, * pos;            // cell_pos null: what a token sees is the mask's alone
     int mask_kind, chunk, keep_first;
@@ -24,12 +25,12 @@ void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s);
 // Which passes take tiles of 32 tokens rather than a workgroup per token (measured against each other over 9 .. 128 tokens, 16 and 32 heads, contexts of the pass's own tokens, 512 .. 1000 and 4096 cells, us):
 //   keys in a cache     from 32 tokens on: 16 heads of 128 over 4: 32 tokens in a window of 256 of 1000 cells 76 -> 36, all of 4000 cells 1060 -> 251, alone in the
 //                       cache 15.7 -> 14.8; 128 tokens alone 38 -> 17.  Fewer tokens: k_few_attention (31 of them over all of 1000 cells 31)
-//   keys of a latent    from 9 tokens on, but for the passes that k_latent_rows (hybrid.hip: splits of 32 cells) takes: 16 heads of 128, rank 512, without those: 9 tokens alone 74 -> 27, of 512 cells 179 -> 65, of 4096
+//   keys of a latent    from 9 tokens on, but for the long contexts of latent_tiles_to (hybrid.hip) and for the passes that k_latent_rows (hybrid.hip: splits of 32 cells) takes: 16 heads of 128, rank 512, without those: 9 tokens alone 74 -> 27, of 512 cells 179 -> 65, of 4096
 //                       440 -> 379; 128 tokens 123 -> 38, 213 -> 69, 836 -> 374
 #define PA_CACHE_TOKENS 32
 #define PA_LATENT_TOKENS 9
 // keys [cell][heads * dim] and values [cell][heads * vdim] of the cells [cell0, cell1) from their latents (row stride `width` floats)
-void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, const int32_t * dyn, float * k, float * v, hipStream_t s);
+void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, int live_max, const int32_t * dyn, float * k, float * v, hipStream_t s);
 // a few tokens over keys and values in a cache: splits of 32 cells (or of several times 32), sixteen query heads of a key head at a time, every split's [vdim sums | maximum | denominator] per (token, head, map)
 // into a.state for the caller's merge.  pa_few_split: cells of a split and their number, 0: not for this kernel
 int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split_cells);

@@ -17,7 +17,7 @@ typedef int pa_i32x4 __attribute__((ext_vector_type(4)));
 
 // tiles of 128 rows of the two matrices x 64 cells; an XCD takes a contiguous run of tiles, eight blocks of rows wide and then along the cells (k_dense_tile)
 __global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restrict__ cache, int64_t width, int64_t rank, const uint16_t * __restrict__ wuk, int64_t nk, const uint16_t * __restrict__ wuv, int64_t nv, int cell0, int cell1,
-                                                          const int32_t * __restrict__ dyn, float * __restrict__ ko, float * __restrict__ vo, int cell_blocks, int tiles, const int32_t * __restrict__ abort_w) {
+                                                          int live_max, const int32_t * __restrict__ dyn, float * __restrict__ ko, float * __restrict__ vo, int cell_blocks, int tiles, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 5)) return;
     __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES_PL(128, 64, 3)];
     const int tile = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
@@ -27,7 +27,7 @@ __global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restri
     const bool is_v = block >= k_blocks;
     const uint16_t * W = is_v ? wuv : wuk;
     const int64_t N = is_v ? nv : nk, n0 = (int64_t) (is_v ? block - k_blocks : block) * 128;
-    if (dyn) cell1 = min(cell1, dyn[1]);
+    if (dyn) { if (live_max > 0 && dyn[1] > live_max) return; cell1 = min(cell1, dyn[1]); }
     const int t0 = cell0 + (in_grp / gsz) * 64, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (t0 >= cell1) return;                                          // (cells of the context that hold nothing yet)
     const int64_t nr = min(n0 + (tid >> 3), N - 1); const int tr = min(t0 + (tid >> 3), cell1 - 1);
@@ -79,6 +79,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, map = wave % MAPS, part = wave / MAPS;
     const int h = blockIdx.x, t0 = (int) (gridDim.y - 1 - blockIdx.y) * 32;       // (the last tokens, which see the most, first)
     const int n_kv = min(A.dyn ? A.dyn[1] : A.n_kv, A.n_kv), c_end = min(n_kv, A.cell1), words = (A.n_kv + 31) / 32;
+    if (A.live_max > 0 && n_kv > A.live_max) return;
     const int dim1 = N1 > 0 ? 16 * N1 : A.dim1, dim2 = N1 > 0 ? 16 * (NK - N1) : A.dim2, vdim = N1 > 0 ? VW : A.vdim, n1 = (dim1 + 15) / 16;
     const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
     const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
@@ -391,10 +392,10 @@ void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s) {
     if (a.vdim <= 64) PA_NK(1); else PA_NK(2);
 #undef PA_NK
 }
-void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, const int32_t * dyn, float * k, float * v, hipStream_t s) {
+void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * wuk, const pi_weight * wuv, int cell0, int cell1, int n_kv, int live_max, const int32_t * dyn, float * k, float * v, hipStream_t s) {
     const int cell_blocks = (cell1 - cell0 + 63) / 64, tiles = cell_blocks * (int) ((wuk->ne1 + 127) / 128 + (wuv->ne1 + 127) / 128);
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, PI_KT_MAXNT - 1, 2.0 * rank * (wuk->ne1 + wuv->ne1) + 4.0 * std::min(cell1 - cell0, n_kv) * (double) (width + wuk->ne1 + wuv->ne1), k_latent_expand, dim3((unsigned) ((tiles + 7) / 8 * 8)), dim3(256), 0, s,
-                 cache, width, (int64_t) rank, (const uint16_t *) wuk->p0, wuk->ne1, (const uint16_t *) wuv->p0, wuv->ne1, cell0, cell1, dyn, k, v, cell_blocks, tiles, pi_abort_word());
+                 cache, width, (int64_t) rank, (const uint16_t *) wuk->p0, wuk->ne1, (const uint16_t *) wuv->p0, wuv->ne1, cell0, cell1, live_max, dyn, k, v, cell_blocks, tiles, pi_abort_word());
 }
 
 // ---- a few tokens ---------------------------------------------------------------------------------------------------------------------------------------------------

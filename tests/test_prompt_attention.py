@@ -73,6 +73,33 @@ def test_latent_context_that_holds_less_than_it_could(H, rank, T, live):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,rank,T", [(8, 264, 9), (7, 264, 40), (2, 64, 20), (16, 512, 30)])
+@pytest.mark.parametrize("live", [45, 7000, 8300, 8738, 8739, 11650, 11750, 16384])
+def test_latent_both_sides_of_the_line_between_tiles_and_tokens(H, rank, T, live):
+    """16384 cells: which kernels take a pass is decided on the device, by how many are live; the ones that do not take it leave nothing behind"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H + live)
+    D, V, cells, pos = 8, 12, 16384, np.arange(live - T, live)
+    wk, wv = (O.bf16_round((rng.standard_normal((H * n, rank)) / np.sqrt(rank)).astype(np.float32)) for n in (D, V))
+    cache = np.full((cells, rank), np.nan, np.float32)
+    cache[:live] = rng.standard_normal((live, rank))
+    q, vis = rng.standard_normal((T, H, D)).astype(np.float32), np.arange(cells)[None, :] <= pos[:, None]
+    uk, uv = fasovik.upload_bf16(lib, wk), fasovik.upload_bf16(lib, wv)
+    qd, cd, md, sd, dd, od = U.Dev(q), U.Dev(cache), U.Dev(pack_mask(vis, cells)), U.Dev(np.full(H, -30.0, np.float32)), U.Dev(np.array([0, live, T, 0], np.int32)), U.Dev(nbytes=4 * T * H * V)
+    n = max(lib.pi_op_latent_attention_rot_scratch_floats(H, rank, 0, T, cells), 1 << 22)
+    scr = U.Dev(np.full(n, np.nan, np.float32))
+    L.check(lib.pi_op_latent_attention(qd.ptr, H * D, cd.ptr, md.ptr, uk, uv, sd.ptr, 0.3, H, D, V, rank, T, cells, scr.ptr, n, od.ptr, H * V, dd.ptr, None))
+    got, c = od.get(np.float32, (T, H, V)), cache[:live].astype(np.float64)
+    for h in range(H):
+        s = (c @ wk.reshape(H, D, rank)[h].T.astype(np.float64)) @ q[:, h].T.astype(np.float64) * np.float32(0.3)
+        w = np.where(vis[:, :live].T, np.exp(s), 0)
+        want = (w / (w.sum(0) + np.exp(-30.0))).T @ (c @ wv.reshape(H, V, rank)[h].T.astype(np.float64))
+        assert rel_rms(got[:, h], want) < 1e-5
+    lib.pi_weight_free(uk)
+    lib.pi_weight_free(uv)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rank", [40, 64, 256, 512, 768])
 @pytest.mark.parametrize("T,n_kv", [(1, 2600), (2, 300), (3, 2600), (4, 4500), (7, 900)])
 def test_latent_splits_are_merged(rank, T, n_kv):
