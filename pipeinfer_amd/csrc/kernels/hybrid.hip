@@ -1397,7 +1397,7 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_r
 // MANY: more than eight splits (the code for them costs the launches of fewer 0.3 us of 9.5)
 template <bool MANY>
 __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
-                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, const int32_t * __restrict__ dyn, int live_min, int live_max, int vec, float * __restrict__ out, int64_t os,
+                                                        const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, int cap, const int32_t * __restrict__ dyn, int live_min, int live_max, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
     if ((live_min > 0 && dyn[1] <= live_min) || (live_max > 0 && dyn[1] > live_max)) return;
     const int gone = pi_abort_peek(abort_w);
@@ -1406,9 +1406,9 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     __shared__ int num[4][64], cnt[4];                                // their numbers, how many they are
     __shared__ float gsh[4];                                          // per token: the head's gate (one value per head)
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nt = min(4, n_tok - t0), n_s = n_kv > 0 ? min(S, (min(dyn ? dyn[1] : n_kv, n_kv) + 31) / 32) : S;      // (n_kv > 0: splits of 32 cells, the ones behind the live cells hold nothing)
+    const int nt = min(4, n_tok - t0), n_s = min(S, (min(dyn ? dyn[1] : n_kv, n_kv) + cap - 1) / cap);      // (splits of cap cells: the ones behind the live cells hold nothing)
     hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (wide: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
-    const bool wide = vec && rank >= 256;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9)
+    const bool wide = vec && rank > 64;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9; whole calls of rank 96 with one split 16.3 that way, 15.5 so)
     if (wide) {
 #pragma unroll
         for (int k = 0; k < 4; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)) * rank + min(lane * 8, rank - 8));
@@ -1424,7 +1424,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     if (MANY && vec) {
         const int cols = rank >> 2;
         at_once = nt * cols <= 128 ? nt : 1; per = at_once * cols;
-        if ((at_once == nt || (n_s > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
+        if (n_s > 16 && (at_once == nt || (n_s > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
 #pragma unroll
         for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
@@ -1696,10 +1696,10 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     const int64_t rows_to = n_tok > 8 && dyn_dev && (int64_t) n_tok * heads * rank > 448 * 512 ? ((int64_t) 1 << 31) / ((int64_t) n_tok * heads * rank) : n_kv;
     const int live_max = whole && rows_to < n_kv ? (int) rows_to : 0;
 #define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
-                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, S, n_tok, rows ? n_kv : 0, dyn_dev, rows ? 0 : live_min, rows ? live_max : 0, \
+                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, S, n_tok, n_kv, rows ? 32 : p.cap, dyn_dev, rows ? 0 : live_min, rows ? live_max : 0, \
                  vec, out, out_stride, pi_abort_word())
     auto combine = [&](int S, bool rows) -> int {
-        const int vec = (rank & 7) == 0 && (rank >= 256 || S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
+        const int vec = (rank & 7) == 0 && (rank > 64 || S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
         if (S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
         PI_CHECK_LAUNCH(); return 0;
     };
