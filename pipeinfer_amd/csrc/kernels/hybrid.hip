@@ -1023,8 +1023,9 @@ extern "C" int pi_op_copy_f32(const float * src, float * dst, int64_t n, void * 
 // (2) k_latent_scores, grid (token, head tile of M heads, split of the cell range): a thread owns a cell in the score phase — its latent row streams through registers once and
 // feeds M accumulators, the M queries come through wave-uniform (scalar) loads — and a slice of the latent's rank in the value phase, where the probabilities of a cell are
 // broadcast from LDS to M x RPT accumulators; every split leaves an un-normalised partial (max, sum, sum of p * c) in scratch.  (3) k_latent_combine merges the splits with
-// the sink term, normalises and applies the value up-projection.  K / V are never materialised; single tokens are spread over the chip by the splits (64 cells each),
-// longer passes take splits only when a score row would not fit LDS.  A pass of 9 tokens and more takes these kernels where sizes, alignment or scratch memory keep it off prompt_attention.hip.
+// the sink term, normalises and applies the value up-projection.  K / V are never materialised; passes of up to eight tokens are spread over the chip by the splits (64 cells each),
+// longer ones take splits only when a score row would not fit LDS.  k_latent_rows takes (2) for few tokens of ranks 256 and 512 (lat_rows_takes), prompt_attention.hip passes of nine tokens and more that are not
+// k_latent_rows's; where sizes, alignment or scratch memory keep a pass off both it comes here.
 // A cached row is [latent (rank) | rotated key part (rot values, shared by the heads; none by default)]: the folded query carries its own rotated part behind the rank values, so a score is one
 // dot product over the row's width; only the latent is summed with the probabilities.  Which cells a token sees is the mask's alone (a window of positions: pi_op_window_mask).
 // scratch (floats): qa [n_tok][heads][rank + rot] | pol [n_tok][heads][S][rank] | pml [n_tok][heads][S][2]
@@ -1408,7 +1409,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nt = min(4, n_tok - t0), n_s = min(S, (min(dyn ? dyn[1] : n_kv, n_kv) + cap - 1) / cap);      // (splits of cap cells: the ones behind the live cells hold nothing)
     hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (wide: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
-    const bool wide = vec && rank > 64;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9; whole calls of rank 96 with one split 16.3 that way, 15.5 so)
+    const bool wide = vec && rank > 64;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9; calls of rank 96 with one split, 4 tokens, 17.1 that way, 16.3 so)
     if (wide) {
 #pragma unroll
         for (int k = 0; k < 4; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)) * rank + min(lane * 8, rank - 8));

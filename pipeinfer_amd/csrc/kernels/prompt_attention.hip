@@ -1,8 +1,8 @@
 // Attention of a prompt: 32 tokens x one head per workgroup, scores and sums on the fp32 matrix cores.
 //
-// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; 62 reached at 2048 tokens x 32 heads of 128).  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
-// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  2048 tokens, 32 heads of 128, rank 512: 7.1 ms -> 0.63; 1000 tokens, 16 heads of 192: 2.4 ms -> 0.21;
-// 1000 tokens of 16 differential heads over a window of 256: 535 us -> 98; 333 tokens of 16 heads with capped scores: 139 us -> 42.
+// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; about 75 reached at 2048 tokens x 32 heads of 128).  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
+// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  Whole calls: 2048 tokens, 32 heads of 128, rank 512: 6.9 ms -> 0.46; 1000 tokens, 16 heads of 192: 1.11 ms -> 0.13;
+// 1000 tokens of 16 differential heads over a window of 256: 526 us -> 74; 333 tokens of 16 heads of 64: 382 us -> 21.
 //   k_latent_expand   the keys and values of the pass's cells written out once: an fp32 latent in three bfloat16 parts times the bfloat16 matrix on the matrix cores, exact products (dense_tile.h)
 //   k_prompt_attention  a wave owns 32 queries (two operand tiles, so a key is read for both) and every fourth run of 32 cells; no barrier until the four waves' sums meet at the end.  The scores are
 //                     computed transposed (rows = cells): what a lane then holds - four cells of one query - is already the operand of the product with the values, nothing crosses lanes but the maximum.

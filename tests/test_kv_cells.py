@@ -237,9 +237,9 @@ def test_mask_of_a_sequence_s_consecutive_tokens():
 
 
 def test_mask_of_cells_that_came_round_again_costs_no_more_than_token_by_token():
-    """a cache of 4096 cells whose positions start in its middle (cells allotted again): the rows of 8 consecutive tokens together take no longer than one by one (a quarter of that here; sorted by position they took four times as long)"""
+    """a cache of 4096 cells whose positions start in its middle (cells allotted again): the rows of 4 consecutive tokens together take no longer than one by one (sorted by position they took twice as long)"""
     import time
-    lib, n, T = LL.api(), 4096, 8
+    lib, n, T = LL.api(), 4096, 4
     h = lib.pi_kvcells_new(n)
     pos = np.roll(np.arange(n - T, dtype=np.int32), n // 3)
     one, ids = np.ones(n, np.int32), np.zeros(n * MAX_SEQ, np.int32)
