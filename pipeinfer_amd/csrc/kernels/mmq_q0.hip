@@ -177,9 +177,11 @@ __global__ void __launch_bounds__(64 * Q0_WAVES, 4) k_mmq_q0(const mmvq_args g, 
 }
 
 // from the first width that costs k_mmvq_q0 a second pass over the weights.  Measured, us there / here at 4096 x 4096, 11008 x 4096 and 4096 x 11008: 5 tokens 21 / 33, 27 / 35, 55 / 83;
-// 8 tokens 29 / 33, 37 / 35, 82 / 83; 9 tokens two passes, about 44 / 33, 57 / 35, 120 / 84
-bool pi_mmq_q0_wants(int type, int n_tok) {
+// 8 tokens 29 / 33, 37 / 35, 82 / 83; 9 tokens two passes, about 44 / 33, 57 / 35, 120 / 84.  The second pass of nine tokens has one token: quick where the rows are few and long, and Q4_0 has more to expand here than Q8_0 (9 tokens of
+// 2048 x 4096 30.0 / 31.9, 2048 x 11008 72.4 / 80.0, 1000 x 2048 17.6 / 17.7, 4096 x 4096 32.6 / 32.1; Q8_0 29.1 / 28.6, 73.6 / 71.4; 10 tokens of 2048 x 11008 88 / 80)
+bool pi_mmq_q0_wants(int type, int n_tok, int64_t rows, int64_t k) {
     static const int min_tok = getenv("PI_MMQ_Q0_MIN") ? atoi(getenv("PI_MMQ_Q0_MIN")) : 9;
+    if (type == PI_Q4_0 && n_tok == 9 && rows <= 2048 && k >= 4096) return false;
     return (type == PI_Q4_0 || type == PI_Q8_0) && n_tok >= min_tok;
 }
 

@@ -967,7 +967,7 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
     for (int i = 0; i < n_w; i++) mfma = mfma && ws[i]->mq != nullptr;
     size_t ofa = 0, ofb = 0, oax = 0;
     if (mfma || mixed_mfma) pi_q8_frag_layout(K, n_tok, &ofa, &ofb, &oax);
-    const bool q0 = pi_mmq_q0_wants(w0->type, n_tok);                          // Q4_0 / Q8_0 prompts: the whole pass in one launch on the matrix cores (n_w == 1 here)
+    const bool q0 = pi_mmq_q0_wants(w0->type, n_tok, w0->ne1, K);                          // Q4_0 / Q8_0 prompts: the whole pass in one launch on the matrix cores (n_w == 1 here)
     const int step = mfma ? pi_mmq_step(w0->type, n_tok, rows_all) : q0 ? n_tok : 8;
     for (int t0 = 0, adv = 0; t0 < n_tok; t0 += adv) {
         // (a two-type matrix-core launch walks up to 8 tokens — a verify pass — or, in a prompt pass, 64: four chunks, the pass's last launch with whatever is left)

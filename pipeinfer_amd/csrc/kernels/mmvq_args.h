@@ -49,6 +49,6 @@ int  pi_mmq_launch(int type, mmvq_launch & L, hipStream_t stream, hipEvent_t ea,
 bool pi_mmq2_applies(int type_b, int n_tok, int64_t rows_a, int64_t rows_b);
 int  pi_mmq_launch2(int type_b, int n_a, bool four_chunks, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
 // mmq_q0.hip: Q4_0 / Q8_0 prompts, the whole pass in one launch (seg[0]; g.aq / g.ad at the first token, g.nt tokens)
-bool pi_mmq_q0_wants(int type, int n_tok);
+bool pi_mmq_q0_wants(int type, int n_tok, int64_t rows, int64_t k);
 int  pi_mmq_q0_reserve();
 int  pi_mmq_q0_launch(int type, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);

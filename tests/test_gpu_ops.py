@@ -161,6 +161,17 @@ def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("k,rows", [(4096, 40), (4096, 2048), (4096, 2049), (4064, 40)])
+def test_mul_mat_q4_0_nine_tokens(gpu, k, rows):
+    """both sides of the line between two passes of the mat-vec and one of k_mmq_q0 (at most 2048 rows of 4096 values and more): the reference's bits"""
+    lib, U = gpu
+    blocks = synth.random_blocks(O.Q4_0, rows * k, np.random.default_rng(k + rows), 0.05).reshape(rows, -1)
+    act = np.stack([signal(k, s) for s in range(9)])
+    w = upload_weight(lib, O.Q4_0, rows, k, blocks)
+    assert np.array_equal(gpu_mul_mat(lib, U, O.Q4_0, w, k, rows, act).view(np.uint32), O.Impl("oracle").mul_mat(O.Q4_0, blocks, k, rows, act).view(np.uint32))
+    lib.pi_weight_free(w)
+
+
 @pytest.mark.parametrize("t", QTYPES)
 def test_mul_mat_integer_sums_exact(gpu, t):
     """Scales forced to powers of two and integer activations small enough that every partial sum is an integer < 2^24:
