@@ -1,5 +1,5 @@
-// Multi-token quantised mat-mat for verify batches and prompts (2 <= n_tok <= 16 per launch) on the matrix cores, BIT-EXACT with the
-// reference's x86 AVX2 arm — the same contract as mmvq.hip:
+// Multi-token quantised mat-mat for verify batches and short prompts (2 <= n_tok <= 16 per launch; 32 over few row groups, see mmq_prompt.hip) on the
+// matrix cores, BIT-EXACT with the reference's x86 AVX2 arm — the same contract as mmvq.hip:
 //
 //   out[t][row] = residual[t][row] + vec_dot(W[row], act[t])
 //
@@ -51,22 +51,6 @@ int pi_mmq_min_nt() {
     return v;
 }
 extern "C" int pi_op_mmq_min_tokens(void) { return pi_mmq_min_nt(); }
-// tokens one launch of the matrix-core kernel walks: 64 (four chunks of 16 over one weight stream, register-staged activations); PI_MMQ_CHUNKS=2 / 1: 32 / 16
-int pi_mmq_max_nt() {
-    static const int v = [] { const char * e = getenv("PI_MMQ_CHUNKS"); return e && atoi(e) == 1 ? 16 : e && atoi(e) == 2 ? 32 : 64; }();
-    return v;
-}
-// tokens per launch of a prompt pass over matrices of `rows` rows in all: 64 (four chunks over one weight stream, register-staged activations) — except for the tall launches
-// (> 1152 row groups: the fused up + gate), whose one-wave row groups walk two chunks at 2.7 TB/s and would have to be split over four waves for four (measured, 70B up + gate
-// per 64 tokens: 2 x 99 us in two-chunk launches, 218-260 us in one four-chunk launch; every shorter launch gains: ffn_down Q6_K 2 x 108 -> 143, Q4_K 2 x 83 -> 122, wo 2 x 27 -> 41)
-int pi_mmq_step(int type, int n_tok, int64_t rows) {
-    (void) type;
-    static const int force = getenv("PI_MMQ_STEP") ? atoi(getenv("PI_MMQ_STEP")) : 0;
-    if (force) return force;
-    if (n_tok <= 16) return 16;
-    const int64_t groups = (rows + 15) / 16 * 256 / pi_cu_count();
-    return groups > 1152 ? (pi_mmq_max_nt() < 32 ? pi_mmq_max_nt() : 32) : pi_mmq_max_nt();
-}
 bool pi_mmq_supported(int type) {
     static const bool q3 = !(getenv("PI_MMQ_Q3") && atoi(getenv("PI_MMQ_Q3")) == 0);      // PI_MMQ_Q3=0: Q3_K batches stay on the VALU kernel (A/B)
     return (type == PI_Q3_K && q3) || type == PI_Q4_K || type == PI_Q5_K || type == PI_Q6_K;
@@ -122,14 +106,10 @@ template <int TYPE, int S> struct mq_w { uint32_t dd, rec, rec2; mq_q<S> q; mq_q
 // PIPE (S >= 2, one chunk, Q4_K / Q5_K): the block step as a two-stage software pipeline — see "pipelined form" below
 // The kernel body as a device function (inlined into k_mmq_kq and into the two-type k_mmq_kq2t): workgroup `wg` of the launch's part that starts at row group `group0`
 // and ends at `n_groups` (both counted over the whole launch: the segments' wave0 are) walks row groups group0 + wg * R ..
-// STG (prompt passes, NC = 4: 33..64 tokens over ONE weight stream): the activation image of a block — NC x 9 KB — is staged through registers (global_load -> ds_write,
-// two LDS buffers, one barrier per block) instead of by LDS-DMA: three DMA buffers of that size would leave the first 64 KB of LDS, the range an M0-based DMA
-// destination can address.  The reference decodes a prompt as ONE batch of up to n_batch = 512 tokens (llama.cpp:5493-5496, speculative.cpp:235-239).
-template <int TYPE, int S, int R, int TB, bool NT8, int NC = 1, bool PIPE = false, bool STG = false>
+template <int TYPE, int S, int R, int TB, bool NT8, int NC = 1, bool PIPE = false>
 static __device__ __forceinline__ void mmq_kq_body(const mmvq_args & g, const int n_groups, const int wg, const int group0) {
     static_assert(!PIPE || (NC == 1 && S >= 2 && (TYPE == PI_Q4_K || TYPE == PI_Q5_K)), "pipelined form: one chunk, split row groups, Q4_K / Q5_K");
-    static_assert(NC == 1 || ((NC == 2 || NC == 4) && !NT8), "several chunks only for full 16-token chunks");
-    static_assert(STG == (NC == 4) && (!STG || (TB == 1 && !PIPE)), "four chunks: register-staged, one block per tile");
+    static_assert(NC == 1 || (NC == 2 && !NT8), "two chunks only for full 16-token chunks");
     static_assert(TYPE == PI_Q3_K || TYPE == PI_Q4_K || TYPE == PI_Q5_K || TYPE == PI_Q6_K, "types are added one by one");
     constexpr bool Q5 = TYPE == PI_Q5_K, Q6 = TYPE == PI_Q6_K, Q3 = TYPE == PI_Q3_K;
     constexpr uint32_t TILE = Q6 ? PI_MQ_TILE_Q6 : Q5 ? PI_MQ_TILE_Q5 : Q3 ? PI_MQ_TILE_Q3 : PI_MQ_TILE, QOFF = Q6 ? 1600 : (Q5 || Q3) ? 832 : 320;
@@ -308,112 +288,8 @@ static __device__ __forceinline__ void mmq_kq_body(const mmvq_args & g, const in
             }
         }
     };
-    // ---- four chunks (STG): the block's weight operands are built ONCE — they do not depend on the chunk — and the chunks then run one after the other, each with its own
-    //      d / fragments / MFMAs / chain updates, behind a scheduling barrier: the generic form below keeps every chunk's d and fragments live at once (402 VGPRs at S = 2) ----
-    auto compute_pp = [&](const mq_w<TYPE, S> & W, const uint8_t * blk) __attribute__((always_inline)) {
-        const pi_f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
-        if constexpr (Q6) {
-            const int n = gq >> 1, hh = gq & 1;
-            const float dx_h = pi_h2f((uint16_t) (W.dd & 0xffff)); const pi_f32x2 dP = mq_pair(dx_h, dx_h); const float dx = dP.x;
-            const uint32_t aoff = (uint32_t) (r + 32 * n) * 16 + 8 * hh;
-            uint4 b1[KS], b2[KS];
-#pragma unroll
-            for (int kk = 0; kk < KS; kk++) {
-                const int half = S == 1 ? (kk >> 2) : S == 2 ? s : (s >> 1);
-                const uint32_t selA = 0x04000400u + (uint32_t) half * 0x00010001u, selB = selA + 0x00020002u;
-                const uint32_t SLa = pk_add(__builtin_amdgcn_perm(0x64646464u, W.rec, selA), 0xE400E400u);
-                const uint32_t SHa = pk_fma(__builtin_amdgcn_perm(0x64646464u, W.rec2, selA), 0x4C004C00u, 0xF408F408u);
-                const uint32_t SLb = pk_fma(__builtin_amdgcn_perm(0x64646464u, W.rec, selB), 0x2C002C00u, 0xD400D400u);
-                const uint32_t SHb = pk_add(__builtin_amdgcn_perm(0x64646464u, W.rec2, selB), 0xE408E408u);
-                const uint32_t q = qdword(W, kk), q8 = q >> 8;
-                const uint32_t h = hdword(W, kk) >> (2 * hh), h8 = h >> 8;
-                const uint32_t w0 = pk_add((q & 0x000F000Fu) | magic | ((h & 0x00030003u) << 4), 0xE420E420u);
-                const uint32_t w1 = pk_add((q8 & 0x000F000Fu) | magic | ((h8 & 0x00030003u) << 4), 0xE420E420u);
-                const uint32_t w2 = pk_add((q & 0x00F000F0u) | magic | ((h & 0x00300030u) << 4), 0xE600E600u);
-                const uint32_t w3 = pk_add((q8 & 0x00F000F0u) | magic | ((h8 & 0x00300030u) << 4), 0xE600E600u);
-                b1[kk] = make_uint4(pk_mul(w0, SHa), pk_mul(w1, SHa), pk_mul(w2, SHb), pk_mul(w3, SHb));
-                b2[kk] = make_uint4(pk_mul(w0, SLa), pk_mul(w1, SLa), pk_mul(w2, SLb), pk_mul(w3, SLb));
-            }
-#pragma unroll
-            for (int ch = 0; ch < NC; ch++) {
-                const float4 dy4 = *(const float4 *) (blk + ch * CH_LDS + 8 * FRAG + 16 * gq);
-                const float d[4] = { dy4.x * dx, dy4.y * dx, dy4.z * dx, dy4.w * dx };
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++) {
-                    const uint8_t * fr = blk + ch * CH_LDS + (s * KS + kk) * FRAG + aoff;
-                    const uint2 a_lo = *(const uint2 *) fr, a_hi = *(const uint2 *) (fr + 16 * 16);
-                    const uint4 af = make_uint4(a_lo.x, a_lo.y, a_hi.x, a_hi.y);
-                    pi_f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pi_half8, af), __builtin_bit_cast(pi_half8, b1[kk]), z, 0, 0, 0);
-                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pi_half8, af), __builtin_bit_cast(pi_half8, b2[kk]), c, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[ch][kk][i] = fmaf(d[i], c[i], acc[ch][kk][i]);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-            const pi_f32x2 dP = mq_pair(pi_h2f((uint16_t) (W.dd & 0xffff)), pi_h2f((uint16_t) (W.dd >> 16))); const float dx = dP.x, dminx = dP.y;
-            const uint32_t S1 = pk_add(__builtin_amdgcn_perm(0x64646464u, W.rec, 0x04000400u), 0xE400E400u);
-            const uint32_t S2 = pk_fma(__builtin_amdgcn_perm(0x64646464u, W.rec, 0x04010401u), 0x2C002C00u, 0xD400D400u);
-            const uint32_t C1 = pk_mul(S1, 0xE400E400u), C2 = pk_mul(S2, 0xE400E400u);
-            uint4 bw[KS];
-#pragma unroll
-            for (int kk = 0; kk < KS; kk++) {
-                const uint32_t q = qdword(W, kk), qh = q >> 8;
-                if constexpr (Q5) {
-                    const uint32_t t = hdword(W, kk) >> (2 * gq), th = t >> 8;
-                    bw[kk].x = pk_fma((q & 0x000F000Fu) | magic | ((t & 0x00010001u) << 4), S1, C1);
-                    bw[kk].y = pk_fma((qh & 0x000F000Fu) | magic | ((th & 0x00010001u) << 4), S1, C1);
-                    bw[kk].z = pk_fma((q & 0x00F000F0u) | magic | ((t & 0x00020002u) << 7), S2, C2);
-                    bw[kk].w = pk_fma((qh & 0x00F000F0u) | magic | ((th & 0x00020002u) << 7), S2, C2);
-                } else {
-                    bw[kk].x = pk_fma((q & 0x000F000Fu) | magic, S1, C1);
-                    bw[kk].y = pk_fma((qh & 0x000F000Fu) | magic, S1, C1);
-                    bw[kk].z = pk_fma((q & 0x00F000F0u) | magic, S2, C2);
-                    bw[kk].w = pk_fma((qh & 0x00F000F0u) | magic, S2, C2);
-                }
-            }
-            const uint32_t M0 = pk_add(__builtin_amdgcn_perm(0x64646464u, W.rec, 0x04020402u), 0xE400E400u);
-            const uint32_t M1 = pk_add(__builtin_amdgcn_perm(0x64646464u, W.rec, 0x04030403u), 0xE400E400u);
-#pragma unroll
-            for (int ch = 0; ch < NC; ch++) {
-                const float4 dy4 = *(const float4 *) (blk + ch * CH_LDS + 8 * FRAG + 16 * gq);
-                const float dy[4] = { dy4.x, dy4.y, dy4.z, dy4.w };
-                float d[4], nd[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) { d[i] = dy[i] * dx; nd[i] = -dy[i] * dminx; }
-#pragma unroll
-                for (int kk = 0; kk < KS; kk++) {
-                    const uint4 af = *(const uint4 *) (blk + ch * CH_LDS + (s * KS + kk) * FRAG + lane * 16);
-                    const pi_f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(pi_half8, af), __builtin_bit_cast(pi_half8, bw[kk]), z, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) acc[ch][kk][i] = fmaf(d[i], c[i], acc[ch][kk][i]);
-                }
-                const uint2 bs = *(const uint2 *) (blk + ch * CH_LDS + 8 * FRAG + 64 + lane * 8);
-                const uint2 am = make_uint2(bs.x, bs.y);
-                if constexpr (Q5) {
-                    if (s == 0) {
-                        const uint2 bm = make_uint2(M0, M1);
-                        const pi_f32x4 cm = mq_mfma_k16(am, bm, z);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) { const float prod = nd[i] * cm[i]; accm[ch][0][i] = accm[ch][0][i] + prod; }
-                    }
-                } else {
-#pragma unroll
-                    for (int cc = 0; cc < CS; cc++) {
-                        const int c = s * CS + cc;
-                        const uint2 bm = make_uint2(M0 & own[c], M1 & own[c]);
-                        const pi_f32x4 cm = mq_mfma_k16(am, bm, z);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) accm[ch][cc][i] = fmaf(nd[i], cm[i], accm[ch][cc][i]);
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    };
     auto compute = [&](const mq_w<TYPE, S> & W, const uint8_t * blk, bool live) __attribute__((always_inline)) {
         if constexpr (Q3) { compute_q3(W, blk); return; }                   // (every width: the operands are built once per block, the chunks run one after the other)
-        if constexpr (STG) { compute_pp(W, blk); return; }
         if constexpr (Q6) { compute_q6(W, blk); return; }
         // ---- block scalars: d, dmin of the row; this lane's two scales and two mins, bytes of one record ----
         const uint32_t ddl = live ? W.dd : 0u;
@@ -573,67 +449,18 @@ static __device__ __forceinline__ void mmq_kq_body(const mmvq_args & g, const in
     static_assert(D == 2 * TB, "ring = two tiles");
     mq_w<TYPE, S> ring[D];
     const uint32_t lds0 = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) uint8_t *) lds;
-    if constexpr (!STG) {
 #pragma unroll
-        for (int u = 0; u < D; u++) load_w(u, ring[u]);
+    for (int u = 0; u < D; u++) load_w(u, ring[u]);
 #pragma unroll
-        for (int j = 0; j < NB - 1; j++) dma_tile(j, lds0 + j * TB * MQ_BLK_LDS);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        wg_barrier();
-    }
+    for (int j = 0; j < NB - 1; j++) dma_tile(j, lds0 + j * TB * MQ_BLK_LDS);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wg_barrier();
     // after the DMAs of tile T + NB - 1 a wave issues TB * LW refills in tile T; when tile T ends, the DMAs of tile T + 1 are older than
     // (NB - 2) tiles of refills + this tile's refills + at least floor(9 TB / NW) DMAs of each younger tile
     constexpr int DMA_MIN = (NP * TB) / NW, WAIT_N = (NB - 1) * TB * LW + (NB - 2) * DMA_MIN;
     // 2 NB tiles per trip: buffer (T % NB) and ring half (T % 2) are compile-time.  The uniform branches around a tile and around a block's
     // compute are deliberate: they are basic-block boundaries for the scheduler, which otherwise interleaves several blocks, doubles the
     // registers in use and spills (measured: 90 -> 124 VGPRs at S = 4, 170 -> 256 + 340 bytes of scratch at S = 1 without them)
-    if constexpr (STG) {
-        // ---- register-staged form: block b is computed from LDS buffer b & 1 while block b + 1's image travels global -> registers; it is written to the other buffer behind the
-        //      compute and one barrier ends the step (the buffer being written was last read in step b - 1, which every wave has left through the barrier that ended it).
-        //      No branch anywhere near a load: the source addresses are clamped (chunks past the launch's last one re-read that one: their results are never stored). ----
-        constexpr int NTHR = 64 * S * R, UNITS = NC * 576, NL = (UNITS + NTHR - 1) / NTHR;          // 16-byte units of one block image, per thread
-        const int nch = (nt + 15) >> 4;
-        // (addresses are recomputed per use: a handful of VALU per 16-byte unit, against ten registers held through the whole loop)
-        pi_u32x4 st[NL];                                                          // (a native vector type: an array of HIP's uint4 structs stayed in scratch memory)
-        auto stage_load = [&](int b) __attribute__((always_inline)) {
-            const uint32_t bb = (uint32_t) (b < nb ? b : nb - 1);
-#pragma unroll
-            for (int i = 0; i < NL; i++) {
-                const int u = i * NTHR + (int) threadIdx.x < UNITS ? i * NTHR + (int) threadIdx.x : UNITS - 1;
-                const int ch = u / 576, w = u - ch * 576, chs = ch < nch ? ch : nch - 1;
-                const size_t cb = (size_t) chs * nb + bb;
-                const uint8_t * src = w < 512 ? g.frag + cb * 8192 + (size_t) w * 16 : g.aux + cb * 1024 + (size_t) (w - 512) * 16;
-                st[i] = *(const pi_u32x4 *) src;
-            }
-        };
-        auto stage_store = [&](uint8_t * buf) __attribute__((always_inline)) {
-#pragma unroll
-            for (int i = 0; i < NL; i++) {
-                const int u = i * NTHR + (int) threadIdx.x < UNITS ? i * NTHR + (int) threadIdx.x : UNITS - 1;
-                const int ch = u / 576, w = u - ch * 576;
-                *(pi_u32x4 *) (buf + ch * CH_LDS + w * 16) = st[i];
-            }
-        };
-        mq_w<TYPE, S> W0, W1;
-        stage_load(0);
-        load_w(0, W0); load_w(1, W1);
-        stage_store(lds);
-        __syncthreads();
-        for (int b0 = 0; b0 < nb; b0 += 2) {
-            stage_load(b0 + 1);
-            compute(W0, lds, true);
-            load_w(b0 + 2, W0);
-            stage_store(lds + MQ_BLK_LDS);
-            __syncthreads();
-            if (b0 + 1 >= nb) break;
-            stage_load(b0 + 2);
-            compute(W1, lds + MQ_BLK_LDS, true);
-            load_w(b0 + 3, W1);
-            stage_store(lds);
-            __syncthreads();
-        }
-        __syncthreads();
-    } else
     if constexpr (PIPE) {
         static_assert(TB % 2 == 0, "the pending sets alternate with the block parity");
         mq_act A0, A1;
@@ -800,7 +627,7 @@ tiles_done:
 template <int TYPE, int S, int R, int TB, bool NT8, int NC = 1, bool PIPE = false>
 __global__ void __launch_bounds__(64 * S * R) k_mmq_kq(const mmvq_args g, const int n_groups) {
     if (pi_aborted(g.abort_w, 1)) return;
-    mmq_kq_body<TYPE, S, R, TB, NT8, NC, PIPE, NC == 4>(g, n_groups, (int) blockIdx.x, 0);
+    mmq_kq_body<TYPE, S, R, TB, NT8, NC, PIPE>(g, n_groups, (int) blockIdx.x, 0);
 }
 // Two weight types in ONE matrix-core launch (<= 8 tokens): the Q4_K_M mixtures keep attn_q / attn_k in Q4_K and put attn_v into Q5_K or Q6_K (llama.cpp:7923-7933).  At one
 // or two tokens k_mmvq_kq2 carries all three; from three tokens attn_v used to be a launch of its own behind q + k (64 row groups of the 70B model: 12-15 us on the VALU
@@ -810,15 +637,13 @@ __global__ void __launch_bounds__(64 * S * R) k_mmq_kq(const mmvq_args g, const 
 // RB: row groups per workgroup of the SECOND type's part.  The part is small (64 row groups of the 70B model) and, in Q6_K, slow per block: three row groups to a workgroup made
 // it the launch's long pole (27-29 us against 21 for q + k alone); with RB = 1 it spreads over 64 CUs, one wave per SIMD (the workgroup's other waves leave at once — a
 // terminated wave does not take part in barriers), and the launch is still one round: 192 + 64 workgroups.
-// NC = 4: the same for prompt passes (33..64 tokens, register-staged activations): attn_v's 64 row groups were a 37-41 us launch of their own per 64 tokens.
-template <int TA, int TB_, int S, int R, int RB, int TBA, int TBB, int NC = 1>
+template <int TA, int TB_, int S, int R, int RB, int TBA, int TBB>
 __global__ void __launch_bounds__(64 * S * R) k_mmq_kq2t(const mmvq_args g, const int groups_a, const int groups_all, const int wgs_a) {
-    static_assert(NC == 1 || (NC == 4 && TBA == 1 && TBB == 1), "verify widths (<= 8 tokens) or four chunks");
     if (pi_aborted(g.abort_w, 1)) return;
-    if ((int) blockIdx.x < wgs_a) mmq_kq_body<TA, S, R, TBA, NC == 1, NC, false, NC == 4>(g, groups_a, (int) blockIdx.x, 0);
+    if ((int) blockIdx.x < wgs_a) mmq_kq_body<TA, S, R, TBA, true>(g, groups_a, (int) blockIdx.x, 0);
     else {
         if constexpr (RB < R) { if ((int) threadIdx.x >= 64 * S * RB) return; }
-        mmq_kq_body<TB_, S, RB, TBB, NC == 1, NC, false, NC == 4>(g, groups_all, (int) blockIdx.x - wgs_a, groups_a);
+        mmq_kq_body<TB_, S, RB, TBB, true>(g, groups_all, (int) blockIdx.x - wgs_a, groups_a);
     }
 }
 
@@ -1048,9 +873,9 @@ tiles_done:
 static bool mmq_pipe_on() { static const bool on = !(getenv("PI_MMQ_PIPE") && atoi(getenv("PI_MMQ_PIPE")) == 0); return on; }
 template <int TYPE, int S, int R, int TB, bool NT8, int NC = 1, bool PIPE = false>
 static void mmq_go2(const mmvq_args & g, int groups, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-    constexpr size_t tiles = (size_t) (NC == 4 ? 2 : 3) * TB * NC * (8 * (NT8 ? 512 : 1024) + 1024), fold = (size_t) R * (8 * 16 * 17 + 4 * 16 * 17 + 256) * 4;
+    constexpr size_t tiles = (size_t) 3 * TB * NC * (8 * (NT8 ? 512 : 1024) + 1024), fold = (size_t) R * (8 * 16 * 17 + 4 * 16 * 17 + 256) * 4;
     constexpr size_t lds = tiles > fold ? tiles : fold;
-    static_assert(NC == 4 || tiles <= 65536, "LDS-DMA targets stay inside the first 64 KB");
+    static_assert(tiles <= 65536, "LDS-DMA targets stay inside the first 64 KB");
     // (Two blocks per scheduling region — the block-axis analogue of k_mmq_g2's two row groups — was built and measured too: no gain on any split-row-group shape,
     //  Q6_K 8192 x 28672 62.7 -> 67.5 us; removed.)
     // the pipelined block step pays at 9..16 tokens (same-box A/B, us per launch: 8192 x 8192 18.70 -> 17.66, 8192 x 28672 53.7 -> 50.2) and is a wash at <= 8 (17.02 / 17.17, 44.7 / 44.4)
@@ -1062,37 +887,20 @@ static void mmq_go2(const mmvq_args & g, int groups, hipStream_t stream, hipEven
     if (ea) hipExtLaunchKernelGGL((k_mmq_kq<TYPE, S, R, TB, NT8, NC, PIPE>), dim3(grid), dim3(64 * S * R), lds, stream, ea, eb, 0, g, groups);
     else    hipLaunchKernelGGL((k_mmq_kq<TYPE, S, R, TB, NT8, NC, PIPE>), dim3(grid), dim3(64 * S * R), lds, stream, g, groups);
 }
-// batches of <= 8 tokens stage half the fragment bytes and take twice the blocks per tile (TB8) in the same LDS; 17..32 tokens are two chunks over one weight
-// stream, one block per tile (the three tiles of two chunks are 54 KB)
+// batches of <= 8 tokens stage half the fragment bytes and take twice the blocks per tile (TB8) in the same LDS; 17..32 tokens over few row groups (one four-wave row group per workgroup) are two chunks over one
+// weight stream, one block per tile — everything else of more than 16 tokens is mmq_prompt.hip's
 template <int TYPE, int S, int R, int TB16, int TB8>
 static void mmq_go(const mmvq_args & g, int groups, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     if (g.nt <= 8) mmq_go2<TYPE, S, R, TB8, true>(g, groups, stream, ea, eb);
     else if (g.nt <= 16) mmq_go2<TYPE, S, R, TB16, false>(g, groups, stream, ea, eb);
-    else if (g.nt <= 32) mmq_go2<TYPE, S, R, 1, false, 2>(g, groups, stream, ea, eb);
-    else if constexpr (S == 4) mmq_go2<TYPE, S, R, 1, false, 4>(g, groups, stream, ea, eb);   // prompt passes: four chunks over one weight stream, register-staged activations
-    else if (!g.frag) mmq_go2<TYPE, S, R, 1, false, 2>(g, groups, stream, ea, eb);            // (pi_op_mul_mat_reserve walks every (cfg, width): nothing is launched)
-    else pi_set_error("mmq: a launch of %d tokens reached a %d-wave configuration (only four-wave row groups walk four chunks)", g.nt, S);   // not reached: mmq_dispatch_t sends launches of > 32 tokens to 41 / 42 / 43; an error, never half a result
+    else if constexpr (S == 4 && R == 1) mmq_go2<TYPE, S, R, 1, false, 2>(g, groups, stream, ea, eb);
+    else if (g.frag) pi_set_error("mmq: a launch of %d tokens reached configuration %d%d", g.nt, S, R);      // not reached: mmq_dispatch_t sends launches of 17..32 tokens to 41; an error, never half a result
 }
 
 template <int TYPE>
 static void mmq_dispatch_t(const mmvq_args & g, int groups, int cfg, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     constexpr int T8 = TYPE == PI_Q4_K ? 4 : 2;                 // blocks per tile at <= 8 tokens (Q5_K: the ring carries the fifth bits too)
-    // Two chunks double the chains a wave carries (96 accumulators on a one-wave row group).  Round 3 sent such launches to two-wave row groups (it spilled with the 8-block ring);
-    // with the one-block tiles of the two-chunk form (a 2-block ring) the one-wave instance fits — 254 VGPRs, no spill — and the tall launches stop repeating the block scalars in
-    // two waves and take two rounds of workgroups instead of 3.5.  Same-box A/B at 24 / 32 tokens, us per launch: 57344 x 8192 139.3 / 138.8 -> 102.2 / 100.7, 28672 x 8192
-    // 72.1 / 71.6 -> 54.6 / 53.3, 44032 x 4096 59.1 / 58.7 -> 56.2 / 55.8, Q6_K 32000 x 8192 78.0 / 75.2 -> 77.9 / 75.8; 70B prompts 987 -> 1 098 tok/s.  PI_MMQ_S1NC2=0: round 3's choice.
-    static const bool s1nc2 = !(getenv("PI_MMQ_S1NC2") && atoi(getenv("PI_MMQ_S1NC2")) == 0);
-    if (g.nt > 16 && (cfg == 17 || cfg == 18 || cfg == 14) && !s1nc2) cfg = 24;
-    // four chunks (33..64 tokens): a one-wave row group would carry 4 x 48 chain registers; two-wave row groups (4 x 24) keep them in registers
-    // four chunks: four-wave row groups (48 chain registers per wave; two-wave row groups need 96 + the staged block image: 256 VGPRs and ~90 spilled inside the loop).
-    // Tall launches (one-wave row groups) do not come here: pi_mmq_step keeps them at 32 tokens per launch.  PI_MMQ_PP_CFG overrides (A/B).
-    // (only the four-wave configurations walk four chunks: any other value would compute the first 32 tokens of a 33..64-token launch and leave the rest unwritten — refused, loudly, once)
-    static const int pp_cfg = [] {
-        const int v = getenv("PI_MMQ_PP_CFG") ? atoi(getenv("PI_MMQ_PP_CFG")) : 0;
-        if (v && v != 41 && v != 42 && v != 43) { fprintf(stderr, "PI_MMQ_PP_CFG=%d ignored: launches of more than 32 tokens need a four-wave configuration (41, 42, 43)\n", v); return 0; }
-        return v;
-    }();
-    if (g.nt > 32) { if (pp_cfg) cfg = pp_cfg; else if (cfg != 41 && cfg != 42 && cfg != 43) cfg = 43; }
+    if (g.nt > 16) cfg = 41;
     switch (cfg) {                                             // (S waves per row group)(R row groups per workgroup); blocks per tile for 16 / <= 8 tokens
         case 17: mmq_go<TYPE, 1, 7, 2, T8>(g, groups, stream, ea, eb); break;
         case 18: mmq_go<TYPE, 1, 8, 2, T8>(g, groups, stream, ea, eb); break;
@@ -1154,32 +962,15 @@ static void mmq_2t_go(const mmvq_args & g, int groups_a, int groups_all, hipStre
     if (ea) hipExtLaunchKernelGGL((k_mmq_kq2t<PI_Q4_K, TB_, 4, R, RB, TBA, TBB>), dim3((unsigned) (wgs_a + wgs_b)), dim3(64 * 4 * R), lds, stream, ea, eb, 0, g, groups_a, groups_all, wgs_a);
     else    hipLaunchKernelGGL((k_mmq_kq2t<PI_Q4_K, TB_, 4, R, RB, TBA, TBB>), dim3((unsigned) (wgs_a + wgs_b)), dim3(64 * 4 * R), lds, stream, g, groups_a, groups_all, wgs_a);
 }
-// four chunks.  The kernel's register budget is that of its block size (R = 3: 168 VGPRs): a second part with ONE row group per workgroup stages nine 16-byte units per
-// thread instead of three and spills (Q5_K: 97 registers; the fused launch then took 120 us against 48 + 37 apart), so the second part keeps R row groups per workgroup
-// (measured, q + k + v of a 70B layer per 64 tokens: Q6_K 54 us fused against 117 apart).  A prompt launch is many rounds long anyway.
-template <int TB_, int R>
-static void mmq_2t_go4(const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-    constexpr int RB = R;
-    constexpr size_t tiles = (size_t) 2 * 4 * (8 * 1024 + 1024), fold = (size_t) R * (8 * 16 * 17 + 4 * 16 * 17 + 256) * 4;
-    constexpr size_t lds = tiles > fold ? tiles : fold;
-    if (!g.frag) { (void) hipFuncSetAttribute((const void *) k_mmq_kq2t<PI_Q4_K, TB_, 4, R, RB, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds); return; }
-    const int wgs_a = (groups_a + R - 1) / R, wgs_b = (groups_all - groups_a + RB - 1) / RB;
-    if (ea) hipExtLaunchKernelGGL((k_mmq_kq2t<PI_Q4_K, TB_, 4, R, RB, 1, 1, 4>), dim3((unsigned) (wgs_a + wgs_b)), dim3(64 * 4 * R), lds, stream, ea, eb, 0, g, groups_a, groups_all, wgs_a);
-    else    hipLaunchKernelGGL((k_mmq_kq2t<PI_Q4_K, TB_, 4, R, RB, 1, 1, 4>), dim3((unsigned) (wgs_a + wgs_b)), dim3(64 * 4 * R), lds, stream, g, groups_a, groups_all, wgs_a);
-}
 template <int TB_>
-static void mmq_2t_dispatch_t(int r, int rb, bool four, const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-    if (four) {                                                                             // (launches of a prompt pass: up to 64 tokens, four chunks)
-        if (r == 1) mmq_2t_go4<TB_, 1>(g, groups_a, groups_all, stream, ea, eb); else if (r == 2) mmq_2t_go4<TB_, 2>(g, groups_a, groups_all, stream, ea, eb); else mmq_2t_go4<TB_, 3>(g, groups_a, groups_all, stream, ea, eb);
-        return;
-    }
+static void mmq_2t_dispatch_t(int r, int rb, const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     if (r == 1) mmq_2t_go<TB_, 1, 1>(g, groups_a, groups_all, stream, ea, eb);
     else if (r == 2) { if (rb == 1) mmq_2t_go<TB_, 2, 1>(g, groups_a, groups_all, stream, ea, eb); else mmq_2t_go<TB_, 2, 2>(g, groups_a, groups_all, stream, ea, eb); }
     else             { if (rb == 1) mmq_2t_go<TB_, 3, 1>(g, groups_a, groups_all, stream, ea, eb); else mmq_2t_go<TB_, 3, 3>(g, groups_a, groups_all, stream, ea, eb); }
 }
-static void mmq_2t_dispatch(int type_b, int r, int rb, bool four, const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-    if (type_b == PI_Q6_K) mmq_2t_dispatch_t<PI_Q6_K>(r, rb, four, g, groups_a, groups_all, stream, ea, eb);
-    else                   mmq_2t_dispatch_t<PI_Q5_K>(r, rb, four, g, groups_a, groups_all, stream, ea, eb);
+static void mmq_2t_dispatch(int type_b, int r, int rb, const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
+    if (type_b == PI_Q6_K) mmq_2t_dispatch_t<PI_Q6_K>(r, rb, g, groups_a, groups_all, stream, ea, eb);
+    else                   mmq_2t_dispatch_t<PI_Q5_K>(r, rb, g, groups_a, groups_all, stream, ea, eb);
 }
 // row groups per workgroup (S = 4) the single-type dispatcher would give the Q4_K part; 0: that part is not one of the short-matrix configurations (no two-type launch)
 static int mmq_2t_rows_per_wg(int64_t rows_a) {
@@ -1195,17 +986,15 @@ static int mmq_2t_rows_per_wg_b(int r, int64_t rows_a, int64_t rows_b) {
 }
 // may a launch of n_a Q4_K matrices (rows_a rows in all) followed by matrices of type_b (rows_b rows) go out as ONE matrix-core launch?  PI_MMQ_2T=0 switches it off.
 // (Only while both parts fit one round of workgroups: the 7B model's attn_v has as many rows as attn_k — fused, q + k + v would be a round and a half.)
-// n_tok: the PASS's tokens.  Verify widths (<= 8) and prompt passes (> 32: launches of 64 tokens, four chunks; a tail of <= 32 tokens goes out in launches of 8).
+// n_tok: the PASS's tokens, a verify pass of 8 at most (prompts: pi_mmq_prompt_wants).
 bool pi_mmq2_applies(int type_b, int n_tok, int64_t rows_a, int64_t rows_b) {
     static const bool on = !(getenv("PI_MMQ_2T") && atoi(getenv("PI_MMQ_2T")) == 0);
-    if (!on || (type_b != PI_Q5_K && type_b != PI_Q6_K) || (n_tok > 8 && n_tok <= 32)) return false;
+    if (!on || (type_b != PI_Q5_K && type_b != PI_Q6_K) || n_tok > 8) return false;
     const int r = mmq_2t_rows_per_wg(rows_a);
-    if (n_tok > 32) return r > 0 && pi_mmq_max_nt() >= 64;
     return pi_mmq_wants(PI_Q4_K, n_tok, rows_a, 0) && r > 0 && mmq_2t_rows_per_wg_b(r, rows_a, rows_b) > 0;
 }
-// L: segments [0, n_a) Q4_K, [n_a, nseg) of type_b, all with tile-major copies; g.frag / g.aux / g.nt set.  four: a launch of a prompt pass (g.nt <= 64 tokens, a multiple
-// of 64 tokens into the pass: the four-chunk instance, whatever is left of the pass); else g.nt <= 8
-int pi_mmq_launch2(int type_b, int n_a, bool four, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
+// L: segments [0, n_a) Q4_K, [n_a, nseg) of type_b, all with tile-major copies; g.frag / g.aux / g.nt (<= 8) set
+int pi_mmq_launch2(int type_b, int n_a, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     if (pi_op_mul_mat_reserve() != 0) return -1;
     mmvq_args & g = L.g;
     int groups = 0, groups_a = 0; int64_t rows_a = 0, rows_b = 0;
@@ -1214,13 +1003,12 @@ int pi_mmq_launch2(int type_b, int n_a, bool four, mmvq_launch & L, hipStream_t 
         else { g.seg[i] = g.seg[0]; g.seg[i].wave0 = 0x7fffffff; }
     }
     // (the second part's row groups are counted per matrix: each of its matrices starts a row group, like the first part's)
-    int r = mmq_2t_rows_per_wg(rows_a);
-    if (four && type_b == PI_Q5_K && r == 3) r = 2;                                          // (the Q5_K body of the four-chunk form spills 62 registers under the 168 of a 12-wave workgroup; 8 waves: 229, none)
-    int rb = four ? r : r > 0 ? mmq_2t_rows_per_wg_b(r, rows_a, rows_b) : 0;
+    const int r = mmq_2t_rows_per_wg(rows_a);
+    int rb = r > 0 ? mmq_2t_rows_per_wg_b(r, rows_a, rows_b) : 0;
     if (r > 0 && rb <= 0) rb = r;                                                           // (more than one round: still correct, pi_mmq2_applies does not choose it)
-    if (r <= 0 || n_a <= 0 || n_a >= L.nseg || g.nt > (four ? 64 : 8)) { pi_set_error("pi_mmq_launch2: not a two-type launch"); return -1; }
+    if (r <= 0 || n_a <= 0 || n_a >= L.nseg || g.nt > 8) { pi_set_error("pi_mmq_launch2: not a two-type launch"); return -1; }
     g.dbg = 0;
-    mmq_2t_dispatch(type_b, r, rb, four, g, groups_a, groups, stream, ea, eb);
+    mmq_2t_dispatch(type_b, r, rb, g, groups_a, groups, stream, ea, eb);
     PI_CHECK_LAUNCH();
     return 0;
 }
@@ -1231,9 +1019,9 @@ extern "C" int pi_op_mul_mat_reserve(void) {
     static bool done = false;
     if (done) return 0;
     mmvq_args g; memset(&g, 0, sizeof g);                      // g.frag == nullptr: the instances only set their attribute
-    for (int type : { PI_Q3_K, PI_Q4_K, PI_Q5_K, PI_Q6_K }) for (int cfg : mmq_cfgs) for (int nt : { 8, 16, 32, 64 }) { g.nt = nt; mmq_dispatch(type, g, 0, cfg, nullptr, nullptr, nullptr); }
-    for (int type_b : { PI_Q5_K, PI_Q6_K }) for (int r : { 1, 2, 3 }) for (int rb : { 1, r }) for (bool four : { false, true }) mmq_2t_dispatch(type_b, r, rb, four, g, 0, 0, nullptr, nullptr, nullptr);
-    if (pi_mmq_q0_reserve() != 0) return -1;
+    for (int type : { PI_Q3_K, PI_Q4_K, PI_Q5_K, PI_Q6_K }) for (int cfg : mmq_cfgs) for (int nt : { 8, 16, 32 }) { g.nt = nt; mmq_dispatch(type, g, 0, cfg, nullptr, nullptr, nullptr); }
+    for (int type_b : { PI_Q5_K, PI_Q6_K }) for (int r : { 1, 2, 3 }) for (int rb : { 1, r }) mmq_2t_dispatch(type_b, r, rb, g, 0, 0, nullptr, nullptr, nullptr);
+    if (pi_mmq_q0_reserve() != 0 || pi_mmq_prompt_reserve() != 0) return -1;
     done = true;
     PI_CHECK_LAUNCH();
     return 0;

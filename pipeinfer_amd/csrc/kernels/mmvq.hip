@@ -932,13 +932,14 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
     const bool all_b = type_b >= 0 && type_b_mask == (1 << n_w) - 1;            // a single type that is not Q4_K
     const bool mixed = type_b >= 0 && !all_b;
     // ... or, at 3..8 tokens, on the matrix cores (k_mmq_kq2t): the Q4_K matrices first, the second type's behind them
-    bool mixed_mfma = false; int n_a = 0;
+    bool mixed_mfma = false, prompt = false; int n_a = 0;          // prompt: k_mmq_prompt
     if (mixed && vdt == PI_Q8_K) {
         while (n_a < n_w && ws[n_a]->type == PI_Q4_K) n_a++;
         bool suffix = n_a > 0 && type_b_mask == (((1 << n_w) - 1) & ~((1 << n_a) - 1)), copies = true;
         int64_t rows_a = 0, rows_b = 0;
         for (int i = 0; i < n_w; i++) { copies = copies && ws[i]->mq != nullptr; if (i < n_a) rows_a += ws[i]->ne1; else rows_b += ws[i]->ne1; }
-        mixed_mfma = suffix && copies && n_tok >= pi_mmq_min_nt() && pi_mmq2_applies(type_b, n_tok, rows_a, rows_b);
+        prompt = suffix && copies && (type_b == PI_Q5_K || type_b == PI_Q6_K) && pi_mmq_prompt_wants(PI_Q4_K, n_tok, rows_a + rows_b);
+        mixed_mfma = prompt || (suffix && copies && n_tok >= pi_mmq_min_nt() && pi_mmq2_applies(type_b, n_tok, rows_a, rows_b));
     }
     if (type_b == -2 || (mixed && !mixed_mfma && !mmvq2_applies(PI_Q4_K, type_b, n_tok, (int) (w0->ne0 / 256)))) {
         bool same = true;
@@ -959,19 +960,19 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
     const uint8_t * base = (const uint8_t *) q8;
     const int64_t K = w0->ne0;
     const int64_t nbq = vdt == PI_Q8_K ? K / 256 : w0->ng;
-    // batches of PI_MMQ_MIN_NT tokens and more go to the matrix cores, 16 tokens per pass over the weights (mmq_mfma.hip); everything else
+    // batches of PI_MMQ_MIN_NT tokens and more go to the matrix cores (mmq_mfma.hip: 16 or 32 tokens per pass over the weights; mmq_prompt.hip: the whole pass at once); everything else
     // (single tokens, types without an MFMA kernel) takes the VALU mat-vec, 8 tokens per pass
     int64_t rows_all = 0;
     for (int i = 0; i < n_w; i++) rows_all += ws[i]->ne1;
     bool mfma = !mixed && vdt == PI_Q8_K && pi_mmq_wants(w0->type, n_tok, rows_all, K);
     for (int i = 0; i < n_w; i++) mfma = mfma && ws[i]->mq != nullptr;
+    if (mfma && pi_mmq_prompt_wants(w0->type, n_tok, rows_all)) { prompt = true; n_a = n_w; }
     size_t ofa = 0, ofb = 0, oax = 0;
     if (mfma || mixed_mfma) pi_q8_frag_layout(K, n_tok, &ofa, &ofb, &oax);
     const bool q0 = pi_mmq_q0_wants(w0->type, n_tok, w0->ne1, K);                          // Q4_0 / Q8_0 prompts: the whole pass in one launch on the matrix cores (n_w == 1 here)
-    const int step = mfma ? pi_mmq_step(w0->type, n_tok, rows_all) : q0 ? n_tok : 8;
+    const int step = prompt || q0 ? n_tok : mfma ? (n_tok <= 16 ? 16 : 32) : 8;
     for (int t0 = 0, adv = 0; t0 < n_tok; t0 += adv) {
-        // (a two-type matrix-core launch walks up to 8 tokens — a verify pass — or, in a prompt pass, 64: four chunks, the pass's last launch with whatever is left)
-        const int step_now = mixed_mfma ? (n_tok > 8 ? 64 : 8) : step;
+        const int step_now = mixed_mfma ? (prompt ? 64 : 8) : step;    // (a two-type launch walks up to 8 tokens of a verify pass, 64 of a prompt)
         const int nt = n_tok - t0 < step_now ? n_tok - t0 : step_now;
         adv = nt;
         mmvq_launch L;
@@ -999,13 +1000,23 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
             else { L.g.ad = base + od + (size_t) t0 * nbq * 8; L.g.abs_ = nullptr; }
         }
         int rc = -1;
+        if (prompt) {
+            L.g.frag = base + ofa + (size_t) (t0 / 16) * nbq * 8192; L.g.aux = base + oax + (size_t) (t0 / 16) * nbq * 1024;
+            L.g.type_b_mask = 0;
+            hipEvent_t ea = nullptr, eb = nullptr;
+            const bool sample = kt_begin(w0->type, nt, L, ea, eb, PI_KT_MMQ);
+            rc = pi_mmq_prompt_launch(w0->type, type_b, n_a, L, stream, ea, eb);
+            if (sample) kt_end(w0->type, nt, L, ea, eb, PI_KT_MMQ);
+            if (rc) return rc;
+            continue;
+        }
         if (mixed_mfma) {
             L.g.frag = base + ofa + (size_t) (t0 / 16) * nbq * 8192;
             L.g.aux = base + oax + (size_t) (t0 / 16) * nbq * 1024;
             L.g.type_b_mask = 0;
             hipEvent_t ea = nullptr, eb = nullptr;
             const bool sample = kt_begin(PI_Q4_K, nt, L, ea, eb, PI_KT_MMQ);
-            rc = pi_mmq_launch2(type_b, n_a, n_tok > 8, L, stream, ea, eb);
+            rc = pi_mmq_launch2(type_b, n_a, L, stream, ea, eb);
             if (sample) kt_end(PI_Q4_K, nt, L, ea, eb, PI_KT_MMQ);
             if (rc) return rc;
             continue;
@@ -1091,7 +1102,7 @@ extern "C" int pi_op_mul_mat_qkv_rope(const pi_weight * wq, const pi_weight * wk
         // (and from three tokens on the matrix cores, when the Q4_K matrices come first: k_mmq_kq2t)
         int64_t rows_a = 0, rows_b = 0; bool copies = true, a_first = true;
         for (int j = 0; j < 3; j++) { copies = copies && ws[j]->mq != nullptr; if (ws[j]->type == PI_Q4_K) { rows_a += ws[j]->ne1; a_first = a_first && j < n_a; } else rows_b += ws[j]->ne1; }
-        const bool on_mfma = a_first && copies && n_tok >= pi_mmq_min_nt() && pi_mmq2_applies(tb_type, n_tok, rows_a, rows_b);
+        const bool on_mfma = a_first && copies && n_tok >= pi_mmq_min_nt() && (pi_mmq2_applies(tb_type, n_tok, rows_a, rows_b) || ((tb_type == PI_Q5_K || tb_type == PI_Q6_K) && pi_mmq_prompt_wants(PI_Q4_K, n_tok, rows_a + rows_b)));
         if (ok2 && n_a > 0 && n_a < 3 && (mmvq2_applies(PI_Q4_K, tb_type, n_tok, (int) (wq->ne0 / 256)) || on_mfma)) {
             mmvq_rope r;
             r.pos = pos; r.cs = tb->cs; r.dyn = dyn_dev; r.kv_head = kv_head; r.hd = hd;

@@ -47,7 +47,11 @@ bool pi_mmq_wants(int type, int n_tok, int64_t rows, int64_t k);      // k: row 
 int  pi_mmq_launch(int type, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
 // two weight types in one matrix-core launch (k_mmq_kq2t): n_a Q4_K segments followed by segments of type_b (Q5_K / Q6_K), 3..8 tokens
 bool pi_mmq2_applies(int type_b, int n_tok, int64_t rows_a, int64_t rows_b);
-int  pi_mmq_launch2(int type_b, int n_a, bool four_chunks, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
+int  pi_mmq_launch2(int type_b, int n_a, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
+// mmq_prompt.hip: K-quant prompts, the whole pass in one launch (segments [0, n_a) of type_a, the others of type_b; g.frag / g.aux at the first token, g.nt tokens)
+bool pi_mmq_prompt_wants(int type, int n_tok, int64_t rows);      // type: the first segments'; rows: of all
+int  pi_mmq_prompt_reserve();
+int  pi_mmq_prompt_launch(int type_a, int type_b, int n_a, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
 // mmq_q0.hip: Q4_0 / Q8_0 prompts, the whole pass in one launch (seg[0]; g.aq / g.ad at the first token, g.nt tokens)
 bool pi_mmq_q0_wants(int type, int n_tok, int64_t rows, int64_t k);
 int  pi_mmq_q0_reserve();

@@ -75,8 +75,6 @@ static __device__ __forceinline__ pi_turn pi_turn_of(int i, int half, int pairin
 // smallest batch width that takes the MFMA kernel (mmq_mfma.hip) instead of the VALU mat-vec; the quantisers write its operand
 // planes from the same width on.  PI_MMQ_MIN_NT overrides (tuning / A-B tests; read once).
 int pi_mmq_min_nt();
-int pi_mmq_max_nt();
-int pi_mmq_step(int type, int n_tok, int64_t rows);             // tokens per matrix-core launch of a pass of n_tok tokens over matrices of `rows` rows in all
 
 static inline bool pi_type_is_legacy(int t) { return t == PI_Q4_1 || t == PI_Q5_0 || t == PI_Q5_1; }
 static inline int pi_type_blck(int t) {

@@ -161,6 +161,23 @@ def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("t", [O.Q3_K, O.Q4_K, O.Q5_K, O.Q6_K])
+@pytest.mark.parametrize("k,rows,n_tok", [(256, 1, 33), (512, 40, 47), (768, 16, 65), (256, 8200, 100), (512, 8190, 90), (512, 8176, 60), (768, 8193, 64), (256, 8222, 128), (512, 8192, 121), (768, 24600, 17), (512, 24577, 32), (256, 16400, 34)])
+def test_mul_mat_k_quants_prompt(gpu, t, k, rows, n_tok):
+    """k_mmq_prompt in every tile shape its rule chooses (two to four chunks of tokens, one or two waves a row group, four and eight waves a workgroup): one block, two, an odd number; rows and tokens that end
+    inside a tile and inside a workgroup's row groups — the reference's bits, with and without a residual"""
+    lib, U = gpu
+    rng = np.random.default_rng(k + rows + n_tok)
+    blocks = synth.random_blocks(t, rows * k, rng, 0.05).reshape(rows, -1)
+    act = np.stack([signal(k, s + n_tok) for s in range(n_tok)])
+    res = rng.standard_normal((n_tok, rows)).astype(np.float32)
+    w = upload_weight(lib, t, rows, k, blocks)
+    want = O.Impl("oracle").mul_mat(t, blocks, k, rows, act)
+    assert np.array_equal(gpu_mul_mat(lib, U, t, w, k, rows, act).view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(gpu_mul_mat(lib, U, t, w, k, rows, act, residual=res).view(np.uint32), (res + want).view(np.uint32))
+    lib.pi_weight_free(w)
+
+
 @pytest.mark.parametrize("k,rows", [(4096, 40), (4096, 2048), (4096, 2049), (4064, 40)])
 def test_mul_mat_q4_0_nine_tokens(gpu, k, rows):
     """both sides of the line between two passes of the mat-vec and one of k_mmq_q0 (at most 2048 rows of 4096 values and more): the reference's bits"""
