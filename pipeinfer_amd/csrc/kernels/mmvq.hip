@@ -951,7 +951,9 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
             return 0;
         }
     }
-    if (vdt != PI_Q8_K && n_w > 1) {
+    bool q0 = true;                                             // Q4_0 / Q8_0 prompts: the whole pass of all matrices in one launch on the matrix cores (mmq_q0.hip)
+    for (int i = 0; i < n_w; i++) q0 = q0 && ws[i]->type == w0->type && pi_mmq_q0_wants(ws[i]->type, n_tok);
+    if (vdt != PI_Q8_K && n_w > 1 && !q0) {
         for (int i = 0; i < n_w; i++) { const int rc = mul_mat_multi_impl(1, ws + i, q8, n_tok, outs + i, ress ? ress + i : nullptr, nullptr, stream_); if (rc) return rc; }
         return 0;
     }
@@ -969,7 +971,6 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
     if (mfma && pi_mmq_prompt_wants(w0->type, n_tok, rows_all)) { prompt = true; n_a = n_w; }
     size_t ofa = 0, ofb = 0, oax = 0;
     if (mfma || mixed_mfma) pi_q8_frag_layout(K, n_tok, &ofa, &ofb, &oax);
-    const bool q0 = pi_mmq_q0_wants(w0->type, n_tok, w0->ne1, K);                          // Q4_0 / Q8_0 prompts: the whole pass in one launch on the matrix cores (n_w == 1 here)
     const int step = prompt || q0 ? n_tok : mfma ? (n_tok <= 16 ? 16 : 32) : 8;
     for (int t0 = 0, adv = 0; t0 < n_tok; t0 += adv) {
         const int step_now = mixed_mfma ? (prompt ? 64 : 8) : step;    // (a two-type launch walks up to 8 tokens of a verify pass, 64 of a prompt)

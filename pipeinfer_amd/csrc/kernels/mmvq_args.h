@@ -52,7 +52,7 @@ int  pi_mmq_launch2(int type_b, int n_a, mmvq_launch & L, hipStream_t stream, hi
 bool pi_mmq_prompt_wants(int type, int n_tok, int64_t rows);      // type: the first segments'; rows: of all
 int  pi_mmq_prompt_reserve();
 int  pi_mmq_prompt_launch(int type_a, int type_b, int n_a, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);
-// mmq_q0.hip: Q4_0 / Q8_0 prompts, the whole pass in one launch (seg[0]; g.aq / g.ad at the first token, g.nt tokens)
-bool pi_mmq_q0_wants(int type, int n_tok, int64_t rows, int64_t k);
+// mmq_q0.hip: Q4_0 / Q8_0 prompts, the whole pass in one launch (all segments of one type; g.aq / g.ad at the first token, g.nt tokens)
+bool pi_mmq_q0_wants(int type, int n_tok);
 int  pi_mmq_q0_reserve();
 int  pi_mmq_q0_launch(int type, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb);

@@ -161,6 +161,27 @@ def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("t", [O.Q4_0, O.Q8_0])
+@pytest.mark.parametrize("k,rows,n_tok", [(128, (33, 1, 31), 16), (160, (4090,), 121), (256, (4095, 1), 250), (160, (2000, 2081), 333), (32, (4001,), 385), (288, (1, 130, 96), 17), (384, (128, 128, 128), 1000)])
+def test_mul_mat_32_blocks_prompt_tiles(gpu, t, k, rows, n_tok):
+    """k_mmq_q0 in every tile shape its rule chooses, one to three matrices in a launch (one may end inside a workgroup's rows): the reference's bits"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(k + sum(rows) + n_tok)
+    act = np.stack([signal(k, s + n_tok) for s in range(n_tok)])
+    blocks = [synth.random_blocks(t, m * k, rng, 0.05).reshape(m, -1) for m in rows]
+    ws = [upload_weight(lib, t, m, k, b) for m, b in zip(rows, blocks)]
+    xd, q8 = U.Dev(act), U.Dev(nbytes=lib.pi_q8_nbytes(O.Q8_0, k, n_tok))
+    L.check(lib.pi_op_quantize(O.Q8_0, xd.ptr, k, n_tok, q8.ptr, None))
+    outs = [U.Dev(nbytes=4 * n_tok * m) for m in rows]
+    L.check(lib.pi_op_mul_mat_multi(len(ws), (C.c_void_p * len(ws))(*ws), q8.ptr, n_tok, (C.c_void_p * len(ws))(*[o.ptr for o in outs]), None, None))
+    for m, b, dv in zip(rows, blocks, outs):
+        want = O.Impl("oracle").mul_mat(t, b, k, m, act)
+        assert np.array_equal(dv.get(np.uint32, (n_tok, m)), want.view(np.uint32))
+    for w in ws:
+        lib.pi_weight_free(w)
+
+
 @pytest.mark.parametrize("t", [O.Q3_K, O.Q4_K, O.Q5_K, O.Q6_K])
 @pytest.mark.parametrize("k,rows,n_tok", [(256, 1, 33), (512, 40, 47), (768, 16, 65), (256, 8200, 100), (512, 8190, 90), (512, 8176, 60), (768, 8193, 64), (256, 8222, 128), (512, 8192, 121), (768, 24600, 17), (512, 24577, 32), (256, 16400, 34)])
 def test_mul_mat_k_quants_prompt(gpu, t, k, rows, n_tok):
