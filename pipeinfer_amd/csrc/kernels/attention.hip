@@ -39,6 +39,7 @@ struct att_args {
     const int32_t * dyn;                                    // optional {kv_head, n_kv} in device memory: lets one captured graph serve every call
     const int32_t * abort_w;                                // abort word of the run (pi_device.h), nullable
     const float * alibi_m;                                  // ALiBi slope of every query head (ggml_alibi, ggml.c:10736-10793), nullable
+    int tile_cells;                                         // k_attention_tiles, launched ahead, takes a pass of up to this many cells (0: none)
     int per_token;                                          // the pass may carry several runs: dyn = {.., n_kv of the widest, n, has_table, cell[n], n_kv[n]} and a workgroup's rows belong to ONE token
 };
 
@@ -59,6 +60,7 @@ __global__ void __launch_bounds__(256) k_attention(const att_args ga) {
     __shared__ float redf[RW][4];
     __shared__ unsigned long long redu[RW][4];
     att_args g = ga;
+    if (ga.tile_cells > 0 && ga.dyn[1] <= ga.tile_cells) return;
     const int s_stride = ga.n_kv;                           // LDS rows keep the static stride
     const int hk = blockIdx.x, chunk = blockIdx.y;
     const int r = g.n_head / g.n_head_kv;                   // query heads per kv head (broadcast rule i02 = i12 / r2, ggml.c:9425)
@@ -317,6 +319,268 @@ __global__ void __launch_bounds__(256) k_attention(const att_args ga) {
 }
 
 // =================================================================================================================
+// k_attention_tiles — passes of many rows (head widths 64 and 128): the chains on the fp32 matrix cores.
+//
+// An accumulator of ggml_vec_dot_f16 is a chain of fma, and for one accumulator a the scores of 16 rows with 16 cells are an outer product per step: q[row][32 st + a] times k[cell][32 st + a] onto a 16 x 16 tile.  That is
+// v_mfma_f32_16x16x1_4b_f32 with its K of one, four accumulators (blocks) at a time: it rounds each product onto the sum once, as fmaf does (tests/test_gpu_ops.py holds the kernel against the reference bit for bit; a
+// comparison of 7.5e10 products and sums, f16 denormals, zeros of both signs, cancellations and infinities among them, found no difference).  The values of f16 products and of their sums are multiples of 2^-48: nothing is
+// ever denormal.  The same for the values: accumulator a of 16 rows x 16 dimensions takes cells 32 w + a.
+//   What bounded k_attention in a prompt was VALU issue: 350 lane-instructions per (row, cell) for the score (folds across lanes among them) and 130 for the values.  Here 128 + 128 products are 8 cycles of a SIMD's matrix
+// core, and the folds, 31 additions per result, run on the VALU beside them: the four blocks of an instruction are accumulators l, l + 16, l + 8, l + 24, so a block fold is three additions in the reference's order.
+//   A workgroup is 16 rows (token-major: row = t * r + gq) of a kv head.  Scores: a wave takes 16 cells at a time; runs of 16 that no row of the tile sees are minus infinity without being computed.  Values: wave l has
+// accumulators l, l + 16, l + 8, l + 24 of all dimensions (a lane's 8 bytes of a cell are the operands of four tiles), the eight waves meet in LDS.  Words of 32 cells outside the rows' visible ones are left out - each product
+// would add 0 * v to a sum that is never -0 - unless such a value is infinite or not a number, which makes the sum one in the reference too: they are looked through for those.
+// Measured, us before / now (prompt without cells ahead): 32 heads of 128, 128 tokens 39 / 16, 333: 198 / 47, 480: 230 / 64; 64 heads over 8, 128: 70 / 23, 480: 640 / 122; 32 heads of 64 over 4, 333: 114 / 29.  (One score per
+// lane with keys through scalar loads, everything on the VALU: 97 at 333.)  Now the matrix cores are busy in 25 % of the cycles; the VALU's 45 % are conversions, folds and the soft max.
+// =================================================================================================================
+#define ATT_TILE_CELLS 2240                                  // 16 score rows of so many cells in LDS
+using att_f32x16 = __attribute__((ext_vector_type(16))) float;
+using att_f32x4 = __attribute__((ext_vector_type(4))) float;
+static __host__ __device__ constexpr int att_tile_stride(int cells) { return (cells + 31) / 32 * 32 + 4; }
+static __device__ __forceinline__ float att_half(uint32_t u, int hi) { return pi_h2f((uint16_t) (hi ? u >> 16 : u & 0xffff)); }
+// (D0 + D1) + (D2 + D3) of the four blocks
+static __device__ __forceinline__ att_f32x4 att_blocks(const att_f32x16 & d) {
+    att_f32x4 x;
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = (d[i] + d[4 + i]) + (d[8 + i] + d[12 + i]);
+    return x;
+}
+template <int HD>
+__global__ void __launch_bounds__(512, 4) k_attention_tiles(const att_args g, const int cells) {
+    extern __shared__ float smem[];
+    const int n_kv = g.dyn ? g.dyn[1] : g.n_kv;
+    if (n_kv > cells) return;                                // (k_attention, launched behind, takes the pass)
+    constexpr int NS = HD / 32, DH = HD / 64;                // 32-element steps of a head; 64 dimensions at a time
+    float * S = smem;                                        // [16][stride] scores, then probabilities; at the end the waves' sums
+    const int stride = att_tile_stride(n_kv);
+    __shared__ int range[2];                                 // first word of 32 cells that matters to any row, end
+    __shared__ float tail[16][32];                           // probabilities of the n_kv % 32 last cells
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, blk = lane >> 4, off = (blk & 1) * 16 + (blk & 2) * 4;      // block's accumulators: off + l
+    const int hk = blockIdx.x, r = g.n_head / g.n_head_kv, rows = g.n_tok * r, row0 = ((int) gridDim.y - 1 - (int) blockIdx.y) * 16;                                      // (the last rows, which see most, first)
+    const int n_gqa = g.n_head_kv * HD, n_embd = g.n_head * HD, words = (n_kv + 31) >> 5, np = n_kv & ~31;
+    if (tid == 0) { range[0] = words; range[1] = 0; }
+    // ---- phase 1: scores ----
+    float q[NS][8];
+    {
+        const int row = min(row0 + j, rows - 1), t = row / r;
+        const uint16_t * qp = g.q16 + (int64_t) t * n_embd + (hk * r + row % r) * HD + off;
+#pragma unroll
+        for (int st = 0; st < NS; st++) {
+            const uint4 v = *(const uint4 *) (qp + 32 * st);
+            const uint32_t d[4] = { v.x, v.y, v.z, v.w };
+#pragma unroll
+            for (int l = 0; l < 8; l++) q[st][l] = att_half(d[l >> 1], l & 1);
+        }
+    }
+    const int tiles = (n_kv + 15) >> 4;
+    uint4 k[NS];
+    auto load_k = [&](int tile) __attribute__((always_inline)) {
+        const uint8_t * kp = (const uint8_t *) (g.kc + (int64_t) 16 * tile * n_gqa + hk * HD);       // (the same for all lanes; theirs is a 32-bit offset)
+        const uint32_t at = ((uint32_t) min(j, n_kv - 1 - 16 * tile) * n_gqa + off) * 2;
+#pragma unroll
+        for (int st = 0; st < NS; st++) k[st] = *(const uint4 *) (kp + (at + 64 * st));
+    };
+    uint32_t mw[4];                                          // visibility of the tile's word: a lane's four rows
+    const uint32_t * mrow[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) mrow[i] = g.mask + (int64_t) (min(row0 + 4 * blk + i, rows - 1) / r) * g.mask_words;
+    auto load_m = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) mw[i] = mrow[i][tile >> 1];
+    };
+    load_m(min(wv, tiles - 1));
+    load_k(min(wv, tiles - 1));
+    const int aborted = pi_abort_peek(g.abort_w);
+    __syncthreads();
+    int first = words, last = 0;
+    for (int tile = wv; tile < tiles; tile += 8) {
+        // the tile's 16 bits of the rows' visibility words (a lane's four rows: 4 blk ..), and of any row
+        const int w = tile >> 1, sh = (tile & 1) * 16;
+        uint32_t m[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) m[i] = mw[i] >> sh;
+        load_m(min(tile + 8, tiles - 1));
+        const int c = 16 * tile + j;
+        const uint32_t live = 16 * tile + 16 <= n_kv ? 0xffffu : (1u << (n_kv - 16 * tile)) - 1u;
+        float * s = S + 4 * blk * stride + c;
+        if (__ballot(((m[0] | m[1] | m[2] | m[3]) & live) != 0) == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) s[i * stride] = -INFINITY;                     // (cells past n_kv: inside the row's padding)
+            load_k(min(tile + 8, tiles - 1));
+            continue;
+        }
+        first = min(first, w); last = w + 1;
+        uint32_t d[NS][4];
+#pragma unroll
+        for (int st = 0; st < NS; st++) { d[st][0] = k[st].x; d[st][1] = k[st].y; d[st][2] = k[st].z; d[st][3] = k[st].w; }
+        load_k(min(tile + 8, tiles - 1));
+        const att_f32x16 z = { 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f };
+        att_f32x4 u, sum;
+#pragma unroll
+        for (int p = 0; p < 4; p++) {                        // t[p] = x[p] + x[p + 4]
+            att_f32x16 a = z, b = z;
+#pragma unroll
+            for (int st = 0; st < NS; st++) {
+                a = __builtin_amdgcn_mfma_f32_16x16x1f32(q[st][p], att_half(d[st][p >> 1], p & 1), a, 0, 0, 0);
+                b = __builtin_amdgcn_mfma_f32_16x16x1f32(q[st][p + 4], att_half(d[st][(p + 4) >> 1], p & 1), b, 0, 0, 0);
+            }
+            const att_f32x4 x = att_blocks(a), y = att_blocks(b);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {                    // (t0 + t1) + (t2 + t3)
+                const float T = x[i] + y[i];
+                if (p == 0 || p == 2) u[i] = T; else if (p == 1) sum[i] = u[i] + T; else sum[i] = sum[i] + (u[i] + T);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            s[i * stride] = (m[i] & live) >> j & 1 ? sum[i] * g.scale : -INFINITY;
+        }
+    }
+    if (lane == 0 && last > 0) { atomicMin(&range[0], first); atomicMax(&range[1], last); }
+    __syncthreads();
+    // ---- phase 2: soft max over the visible words, 32 threads per row; and the values of words that no row sees, for any that is not finite ----
+    {
+        const int lo = range[0], hi = range[1], from = 32 * lo, to = min(32 * hi, n_kv), rr = tid >> 5, c0 = tid & 31;
+        float * s = S + rr * stride;
+        constexpr int TPC = HD / 8, CPT = 512 / TPC;         // (sixteen bytes a thread, CPT cells a step, four steps on their way together)
+        using u16x2 = __attribute__((ext_vector_type(2))) uint16_t;
+        u16x2 top = { 0, 0 };                                // largest exponent fields
+        auto look = [&](int a, int b) __attribute__((always_inline)) {
+            for (int c = a + tid / TPC; c < b; c += 4 * CPT) {
+                uint4 v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) v[u] = *(const uint4 *) (g.vc + (int64_t) min(c + u * CPT, b - 1) * n_gqa + hk * HD + 8 * (tid % TPC));
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t d[4] = { v[u].x, v[u].y, v[u].z, v[u].w };
+#pragma unroll
+                    for (int i = 0; i < 4; i++) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, d[i] & 0x7C007C00u));
+                }
+            }
+        };
+        look(0, min(from, np));
+        look(32 * hi, np);
+        float mx = -INFINITY;
+        for (int c = from + c0; c < to; c += 32) mx = fmaxf(mx, s[c]);
+        pi_butterfly<16>([&](auto o) { mx = fmaxf(mx, pi_partner<decltype(o)::value>(mx)); });
+        uint32_t part = 0;                                   // in units of 2^-24: exact (at most ATT_TILE_CELLS / 32 values of one)
+        constexpr int U = 4;                                 // (table values that are on their way together)
+        for (int c = from + c0; c < to; c += 32 * U) {
+            float x[U]; uint16_t e[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) { x[u] = c + 32 * u < to ? s[c + 32 * u] : -INFINITY; e[u] = g.exp_tab[pi_f2h(x[u] - mx)]; }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const float v = x[u] != -INFINITY ? pi_h2f(e[u]) : 0.0f;
+                part += (uint32_t) (v * 16777216.0f);
+                if (c + 32 * u < to) s[c + 32 * u] = v;
+            }
+        }
+        unsigned long long isum = part;
+        pi_butterfly<16>([&](auto o) { isum += pi_partner<decltype(o)::value>(isum); });
+        const float inv = (float) (1.0 / ((double) isum * (1.0 / 16777216.0))), none = pi_h2f(pi_f2h(0.0f * inv));      // none: what a masked cell gets
+        for (int c = from + c0; c < to; c += 32) s[c] = pi_h2f(pi_f2h(s[c] * inv));      // P rounded to f16 as the V.P mul_mat does
+        if (np + c0 < n_kv) tail[rr][c0] = np + c0 >= from && np + c0 < to ? s[np + c0] : none;      // (from and np are multiples of 32: cell np + c0 is this thread's own)
+        __syncthreads();                                     // (every thread has read the range)
+        if (top[0] == 0x7C00 || top[1] == 0x7C00 || isum == 0) { range[0] = 0; range[1] = words; }      // (whoever gets here writes the same.  A row without a visible cell: not a number over all cells, as 0 * infinity makes it)
+        __syncthreads();
+        if (range[0] != lo || range[1] != hi) {              // the words that were left out, after all
+            for (int c = c0; c < np; c += 32) if (c < from || c >= to) s[c] = none;
+            __syncthreads();
+        }
+    }
+    if (aborted & 1) { pi_abort_note(g.abort_w, 5); return; }
+    // ---- phase 3: wave l: accumulators off + l of out[row][e] = ggml_vec_dot_f16(n_kv, V[:, e], P[row, :]), 64 dimensions at a time: lane (j, blk) has dimensions 4 j .. + 3 of cells 32 w + off + l ----
+    const int lo = __builtin_amdgcn_readfirstlane(range[0]), hi = __builtin_amdgcn_readfirstlane(min(range[1], np >> 5));
+    const float * P = S + j * stride + off + wv;
+    const uint32_t v_off = ((uint32_t) (off + wv) * n_gqa + 4 * j) * 2;
+    auto load_v = [&](int w, int dh) __attribute__((always_inline)) { return *(const uint2 *) ((const uint8_t *) (g.vc + (int64_t) 32 * w * n_gqa + hk * HD + 64 * dh) + v_off); };
+    att_f32x4 X[DH][4];                                      // x[l] of rows 4 blk .. + 3 (component), dimension 64 dh + 4 j + e
+#pragma unroll
+    for (int dh = 0; dh < DH; dh++) {
+        att_f32x16 a[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) a[e][i] = 0.0f;
+        constexpr int D = 3;                                 // words in flight
+        uint2 v[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) v[d] = lo < hi ? load_v(min(lo + d, hi - 1), dh) : make_uint2(0, 0);
+        auto word = [&](int w, int d) __attribute__((always_inline)) {
+            const float p = P[32 * w];
+            const uint2 x = v[d];
+            v[d] = load_v(min(w + D, hi - 1), dh);
+            a[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(p, att_half(x.x, 0), a[0], 0, 0, 0);
+            a[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(p, att_half(x.x, 1), a[1], 0, 0, 0);
+            a[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(p, att_half(x.y, 0), a[2], 0, 0, 0);
+            a[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(p, att_half(x.y, 1), a[3], 0, 0, 0);
+        };
+        int w = lo;
+        for (; w + D <= hi; w += D)
+#pragma unroll
+            for (int d = 0; d < D; d++) word(w + d, d);
+        if (w < hi) { word(w, 0); if (w + 1 < hi) { word(w + 1, 1); if (D > 3 && w + 2 < hi) word(w + 2, 2); } }
+#pragma unroll
+        for (int e = 0; e < 4; e++) X[dh][e] = att_blocks(a[e]);
+    }
+    constexpr int OPT = 16 * HD / 512;                       // outputs that a thread finishes: row tid / 32, dimensions OPT (tid % 32) ..
+    const int orow = row0 + (tid >> 5), oe = OPT * (tid & 31);
+    __syncthreads();
+    // t[p] = x[p] + x[p + 4]: waves 4 .. 7 hand theirs over, then waves 0 .. 3 the sums
+    float * F = smem;                                        // [4][16 rows][HD]
+    auto at = [&](int p, int dh, int e, int i) __attribute__((always_inline)) { return (p * 16 + 4 * blk + i) * HD + 64 * dh + 4 * j + e; };
+    if (wv >= 4)
+#pragma unroll
+        for (int dh = 0; dh < DH; dh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) *(float4 *) (F + at(wv - 4, dh, 0, i)) = make_float4(X[dh][0][i], X[dh][1][i], X[dh][2][i], X[dh][3][i]);
+    __syncthreads();
+    if (wv < 4)
+#pragma unroll
+        for (int dh = 0; dh < DH; dh++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                float4 * f = (float4 *) (F + at(wv, dh, 0, i));
+                const float4 y = *f;
+                *f = make_float4(X[dh][0][i] + y.x, X[dh][1][i] + y.y, X[dh][2][i] + y.z, X[dh][3][i] + y.w);
+            }
+    __syncthreads();
+    if (orow >= rows) return;
+    const int ot = orow / r, oh = hk * r + orow % r;
+    float out[OPT];
+#pragma unroll
+    for (int e = 0; e < OPT; e++) {
+        const float * f = F + (tid >> 5) * HD + oe + e;
+        out[e] = (f[0] + f[16 * HD]) + (f[32 * HD] + f[48 * HD]);
+    }
+    if (np < n_kv) {
+        double sd[OPT];
+#pragma unroll
+        for (int e = 0; e < OPT; e++) sd[e] = (double) out[e];
+        const uint16_t * vt = g.vc + hk * HD + oe;          // the last cells, one by one in double
+        for (int c = np; c < n_kv; c += 8) {                 // (eight on their way together)
+            uint32_t d[8][OPT / 2];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int e = 0; e < OPT / 2; e++) d[u][e] = *(const uint32_t *) (vt + (int64_t) min(c + u, n_kv - 1) * n_gqa + 2 * e);
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (c + u < n_kv) {
+                    const float p = tail[tid >> 5][c + u - np];
+#pragma unroll
+                    for (int e = 0; e < OPT; e++) sd[e] += (double) (att_half(d[u][e >> 1], e & 1) * p);
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < OPT; e++) out[e] = (float) sd[e];
+    }
+    float * o = g.out + (int64_t) ot * n_embd + oh * HD + oe;
+    if constexpr (OPT == 4) *(float4 *) o = make_float4(out[0], out[1], out[2], out[3]); else *(float2 *) o = make_float2(out[0], out[1]);
+}
+
+// =================================================================================================================
 // k_attention_any — every OTHER head width (even, <= 256; e.g. StableLM-3B's 80): the reference takes any n_embd_head (llama.cpp:3698-3778).  The same arithmetic written
 // plainly, not tuned: one workgroup per (kv head, query row); phase 1 one thread per cell, phase 3 one thread per output dimension, each running ggml_vec_dot_f16's 32
 // accumulators itself (4 registers x 8 lanes, fma in element order, folds (0 += 2, 1 += 3, 0 += 1), lanes l + (l + 4), two hadds) and — what the 64 / 128 instances never
@@ -436,6 +700,16 @@ static size_t att_lds_cap(int rw) { return (size_t) (rw == 1 ? 146 : 156) * 1024
 // Long contexts: the score rows of a workgroup live in LDS, so the rows per workgroup shrink as the context grows — 8 rows up to 4 840 cells, 4 up to 9 680, 2 up to
 // 19 360, one row up to 36 200 (the reference has no bound, llama.cpp:8729-8748; K/V are then re-read from L2 by more workgroups, nothing else changes).
 extern "C" int pi_op_attention_max_cells(void) { int n = 36200; while (att_lds_bytes(1, n) > att_lds_cap(1)) n--; return n; }
+static size_t att_tile_lds(int hd, int cells) { const size_t s = (size_t) 16 * att_tile_stride(cells) * 4, f = (size_t) 4 * 16 * hd * 4; return s > f ? s : f; }
+// k_attention_tiles may ask for the LDS of ATT_TILE_CELLS cells (once per process, outside any capture: pi_op_attention_reserve)
+static int att_tile_reserve() {
+    static const int rc = [] {
+        PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention_tiles<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) att_tile_lds(128, ATT_TILE_CELLS)));
+        PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention_tiles<64>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) att_tile_lds(64, ATT_TILE_CELLS)));
+        return 0;
+    }();
+    return rc;
+}
 extern "C" int pi_op_attention_reserve(int hd, int n_kv_max) {
     if (att_lds_bytes(1, n_kv_max) > att_lds_cap(1)) { pi_set_error("pi_op_attention_reserve: n_kv=%d needs %zu B of LDS for ONE score row (> 146 KiB): contexts beyond %d cells are not supported", n_kv_max, att_lds_bytes(1, n_kv_max), pi_op_attention_max_cells()); return -1; }
     if (hd != 64 && hd != 128) {                                          // the plain kernel of the other head widths: one score row + the mask words + the query row
@@ -445,6 +719,7 @@ extern "C" int pi_op_attention_reserve(int hd, int n_kv_max) {
         PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention_any<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) (b < att_lds_cap(1) ? b : att_lds_cap(1))));
         return 0;
     }
+    if (att_tile_reserve() != 0) return -1;
     if (att_lds_bytes(ATT_ROWS, n_kv_max) <= 60 * 1024) return 0;
     int rc = 0;
     auto want = [&](int rw) { const size_t b = att_lds_bytes(rw, n_kv_max), cap = att_lds_cap(rw); return b < cap ? b : cap; };
@@ -462,21 +737,31 @@ static void att_launch(const att_args & g, int rows, int rw, hipStream_t stream)
     const int nt = g.n_tok > 0 ? g.n_tok : 1;
     const int n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv;      // (eager launches of the engine: the pass's own n_kv)
     const double bytes = (double) n_kv_priced * g.n_head_kv * HD * 2 * 2 + (double) nt * g.n_head * HD * (2 + 4);
+    // (a launch behind k_attention_tiles is not counted: one of the two does the work)
+#define ATT_GO(...) do { if (g.tile_cells > 0) hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(256), lds, stream, g); else PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (__VA_ARGS__), grid, dim3(256), lds, stream, g); } while (0)
     if (g.alibi_m) {
         switch (rw) {
-            case 1: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 1, true>), grid, dim3(256), lds, stream, g); break;
-            case 2: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 2, true>), grid, dim3(256), lds, stream, g); break;
-            case 4: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 4, true>), grid, dim3(256), lds, stream, g); break;
-            default: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 8, true>), grid, dim3(256), lds, stream, g); break;
+            case 1: ATT_GO(k_attention<HD, 1, true>); break;
+            case 2: ATT_GO(k_attention<HD, 2, true>); break;
+            case 4: ATT_GO(k_attention<HD, 4, true>); break;
+            default: ATT_GO(k_attention<HD, 8, true>); break;
         }
         return;
     }
     switch (rw) {
-        case 1: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 1>), grid, dim3(256), lds, stream, g); break;
-        case 2: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 2>), grid, dim3(256), lds, stream, g); break;
-        case 4: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 4>), grid, dim3(256), lds, stream, g); break;
-        default: PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention<HD, 8>), grid, dim3(256), lds, stream, g); break;
+        case 1: ATT_GO(k_attention<HD, 1>); break;
+        case 2: ATT_GO(k_attention<HD, 2>); break;
+        case 4: ATT_GO(k_attention<HD, 4>); break;
+        default: ATT_GO(k_attention<HD, 8>); break;
     }
+}
+#undef ATT_GO
+// passes of many rows of up to ATT_TILE_CELLS cells; g.n_kv may be the bound of a captured graph
+template <int HD>
+static void att_tile_launch(const att_args & g, int rows, hipStream_t stream) {
+    const int nt = g.n_tok, cells = g.n_kv < ATT_TILE_CELLS ? g.n_kv : ATT_TILE_CELLS, n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv;
+    const double bytes = (double) n_kv_priced * g.n_head_kv * HD * 2 * 2 + (double) nt * g.n_head * HD * (2 + 4);
+    PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention_tiles<HD>), dim3(g.n_head_kv, (rows + 15) / 16), dim3(512), att_tile_lds(HD, cells), stream, g, cells);
 }
 
 extern "C" int pi_op_attention(const uint16_t * q16, const uint16_t * kc, const uint16_t * vc, const uint32_t * mask, int hd, int n_head, int n_head_kv,
@@ -504,7 +789,7 @@ extern "C" int pi_op_attention_alibi(const uint16_t * q16, const uint16_t * kc, 
     g.n_head = n_head; g.n_head_kv = n_head_kv; g.n_tok = n_tok; g.n_kv = n_kv; g.mask_words = (n_kv + 31) / 32;
     g.exp_tab = pi_get_tables().exp_f16;
     g.scale = 1.0f / sqrtf((float) hd);                      // KQ_scale, llama.cpp:5189-5193
-    g.dyn = dyn_dev; g.abort_w = pi_abort_word(); g.per_token = per_token_kv && dyn_dev ? 1 : 0;
+    g.tile_cells = 0; g.dyn = dyn_dev; g.abort_w = pi_abort_word(); g.per_token = per_token_kv && dyn_dev ? 1 : 0;
     const int rows = n_tok * (n_head / n_head_kv);
     // rows per workgroup.  K/V are re-read (from L2) by every workgroup of a kv head, so more rows per workgroup mean fewer bytes through L2 — but a workgroup walks its rows'
     // phases one after the other, and at the contexts of a generation (a few hundred cells) it is that chain, not L2, that a launch waits for.  Round 6, 70B (8 kv heads x 8 query
@@ -522,6 +807,15 @@ extern "C" int pi_op_attention_alibi(const uint16_t * q16, const uint16_t * kc, 
     if (g.per_token) { const int r = n_head / n_head_kv; while (rw > 1 && r % rw) rw >>= 1; }      // a workgroup's rows stay inside one token (rows are token-major)
     while (rw > 1 && att_lds_bytes(rw, n_kv) > att_lds_cap(rw)) rw >>= 1;               // long contexts: fewer score rows per workgroup (they live in LDS)
     if ((size_t) rw * (n_kv + g.mask_words) * sizeof(float) > att_lds_cap(rw)) { pi_set_error("pi_op_attention: n_kv=%d needs more than %d KiB of LDS", n_kv, rw == 1 ? 146 : 156); return -1; }
+    // from 1536 query rows: below, a workgroup's chain of phases (12 us at 32 cells of 128 values) is longer than k_attention's launch.  us there / here, no cells and 100 cells ahead: 32 heads of 128, 32 tokens 9.1 / 12.0
+    // and 17.5 / 16.3, 48: 14.2 / 14.2 and 22 / 18; 64 heads over 8, 16 tokens 11 / 13 and 15 / 17, 24: 13.3 / 14.3 and 18.5 / 17.8, 48: 25 / 15 and 39 / 19; 32 heads of 64 over 4, 48 tokens 10.7 / 8.5 and 15 / 11
+    static const int tile_min = getenv("PI_ATT_TILE_MIN") ? atoi(getenv("PI_ATT_TILE_MIN")) : 1536;
+    if ((hd == 128 || hd == 64) && !alibi_slopes_dev && !g.per_token && (int64_t) n_tok * n_head >= tile_min && (dyn_dev || n_kv <= ATT_TILE_CELLS) && (((uintptr_t) q16 | (uintptr_t) out | (uintptr_t) kc | (uintptr_t) vc) & 15) == 0) {
+        if (att_tile_reserve() != 0) return -1;
+        if (hd == 128) att_tile_launch<128>(g, rows, (hipStream_t) stream); else att_tile_launch<64>(g, rows, (hipStream_t) stream);
+        if (n_kv <= ATT_TILE_CELLS) { PI_CHECK_LAUNCH(); return 0; }
+        g.tile_cells = ATT_TILE_CELLS;                       // a captured graph's bound: longer passes go on with k_attention
+    }
     if (hd == 128) att_launch<128>(g, rows, rw, (hipStream_t) stream);
     else if (hd == 64) att_launch<64>(g, rows, rw, (hipStream_t) stream);
     else if (hd > 0 && hd <= 256 && hd % 2 == 0) {                       // every other head width: the plain kernel, one workgroup per (kv head, query row)

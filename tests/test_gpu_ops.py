@@ -436,6 +436,47 @@ def test_attention_vs_oracle(gpu, hd, n_head, n_head_kv, n_kv, n_tok):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()      # vec_dot_f16 order + exact soft-max sum
 
 
+@pytest.mark.parametrize("hd,n_head,n_head_kv,n_kv,n_tok,bound", [(128, 32, 32, 48, 48, 0), (128, 64, 8, 333, 25, 0), (64, 71, 1, 97, 65, 0), (64, 32, 4, 300, 64, 0), (128, 16, 16, 130, 130, 192), (128, 16, 2, 31, 100, 0),
+                                                                   (64, 24, 3, 2240, 64, 0), (128, 16, 16, 500, 100, 4096), (64, 16, 4, 2300, 97, 4096), (128, 4, 4, 1, 400, 0)])
+def test_attention_tiles(gpu, hd, n_head, n_head_kv, n_kv, n_tok, bound):
+    """k_attention_tiles (passes of 1536 query rows and more) == k_attention (the same tokens, a few at a time), bit for bit: tiles of rows and cells that are not full, cells past whole words, holes, rows that see nothing, values
+    outside every row's view that are infinite or no numbers; and behind a captured graph's bound of cells both kernels are launched and one of them does the work"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(hd + n_kv + n_tok)
+    words, row = (max(n_kv, bound) + 31) // 32, n_head * hd
+    k, v, q = (rng.standard_normal((n, h * hd)).astype(np.float16) for n, h in ((n_kv, n_head_kv), (n_kv, n_head_kv), (n_tok, n_head)))
+    kd, qd = U.Dev(k), U.Dev(q)
+    L.check(lib.pi_op_attention_reserve(hd, max(n_kv, bound)))
+    bits = np.zeros((n_tok, words * 32), np.uint8)
+    for t in range(n_tok):
+        bits[t, :max(1, n_kv - n_tok + t + 1)] = 1
+    bits[:, 40:75] = 0                                                         # a hole that holds a whole word
+    bits[:, n_kv:] = 0
+    odd = v.copy()
+    odd[min(n_kv - 1, 50), :3] = np.float16(np.inf)
+    odd[min(n_kv - 1, 64), hd - 1] = np.float16(np.nan)
+    blind = bits.copy()
+    blind[n_tok // 2] = 0
+    late = bits.copy()
+    late[:, min(64, n_kv - 1):n_kv - 1] = 0                                    # most words are outside every view
+    for name, vals, seen in (("plain", v, bits), ("not finite", odd, bits), ("blind row", v, blind), ("not finite, far", odd * np.float16(1), late), ("blind row, not finite", odd, blind)):
+        vd, md = U.Dev(vals), U.Dev(np.packbits(seen.reshape(n_tok, words, 32), axis=2, bitorder="little").view(np.uint32).reshape(n_tok, words))
+        step = max(1, 1535 // n_head // 4)
+        outs = []
+        for width in (n_tok, step):
+            out = U.Dev(nbytes=4 * n_tok * row)
+            for t0 in range(0, n_tok, width):
+                n = min(width, n_tok - t0)
+                dyn = U.Dev(np.array([0, n_kv, n, 0], np.int32)) if bound else None
+                L.check(lib.pi_op_attention(qd.ptr + 2 * t0 * row, kd.ptr, vd.ptr, md.ptr + 4 * t0 * words, hd, n_head, n_head_kv, n, bound or n_kv, out.ptr + 4 * t0 * row, dyn.ptr if bound else None, None))
+                lib.pi_device_sync()
+            outs.append(out.get(np.float32, (n_tok, row)))
+        a, b = outs
+        assert np.array_equal(np.isnan(a), np.isnan(b)), name
+        assert np.array_equal(np.where(np.isnan(a), 0, a).view(np.uint32), np.where(np.isnan(b), 0, b).view(np.uint32)), name
+
+
 def test_elementwise_exact(gpu):
     lib, U = gpu
     from pipeinfer_amd import lib as L
