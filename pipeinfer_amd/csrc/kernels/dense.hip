@@ -7,8 +7,8 @@
 //
 //   k_dense_rows   one wave per output row, K spread over the lanes with 16 / 8 / 2-byte weight loads, TT tokens held in registers: the mat-vec of single tokens (weights streamed once from HBM:
 //                  6.7 TB/s at 32000 x 4096, 4.3 at 4096 x 4096, 4 us of launch below 1024 x 1024) and every width of the fp32 mode
-//   k_dense_split  serving precision, 2 .. 32 tokens: 4 .. 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (4.6 TB/s at 32000 x 4096 and up to
-//                  8 tokens).  On the mat-vec every row reads all tokens' activations again, 2 T times its own bytes: 28 us for 4096 x 4096 at 8 tokens, 11 here
+//   k_dense_split  serving precision, 2 .. 32 tokens: 4 .. 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (5.8 TB/s at 32000 x 4096 and 2
+//                  tokens, 4.6 at 8) and by the address unit.  On the mat-vec every row reads all tokens' activations again, 2 T times its own bytes: 28 us for 4096 x 4096 at 8 tokens, 11 here
 //   k_dense_tile   serving precision, more tokens: tiles of 64 .. 128 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory
 //                  (26 bytes a cycle of cold weights and activations), large ones by the shared levels of memory and the steps' latency: 730 TFLOP/s at 16384 x 4096 x 2048 tokens (the tiles without
 //                  deeper prefetch and in plain order: 472), 17 us for 2048 x 2048 x 512 (82 before)
@@ -101,6 +101,9 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
     }
 }
 
+// the value of the lane N further on in the row of 16 (what the last N lanes get is of no use)
+template <int N>
+static __device__ __forceinline__ uint32_t dn_from_lane(uint32_t v) { return (uint32_t) __builtin_amdgcn_update_dpp(0, (int) v, 0x100 + N, 0xf, 0xf, true); }
 // one float4 of results (four rows of one token): bias, activation, store
 static __device__ __forceinline__ void dn_store4(dt_f32x4 v4, int64_t row, int64_t N, int tok, float * __restrict__ Y, int64_t ys, int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias) {
     float v[4] = { v4[0], v4[1], v4[2], v4[3] };
@@ -145,10 +148,14 @@ __global__ void __launch_bounds__(256 * KG, 2) k_dense_tile(const uint16_t * __r
 // 2 .. 32 tokens: up to RT x 16 rows (`rows`, a multiple of 4: the lanes of the others read the last one again, which costs no bytes) and TT x 16 tokens per workgroup, K split over its eight waves, which meet in LDS.  The weights are streamed once, straight from memory in the operand's lane layout: the
 // four lanes of a row take 64 consecutive bytes of it per product, the activations come from L2 once per workgroup.  Rows in segments: as k_dense_rows, whole workgroups
 // inside a segment (the host checks).
-template <int RT, int TT>
+// XS: tokens that a product's sixteen columns stand for.  With 8 (4) the lanes of the other columns load the rest of the tokens' values, which a move across the lanes then brings to their columns: half
+// (a quarter of) the loads of activations, which would otherwise be most of what the address unit works through (16 rows of weights are two loads a step, their sixteen columns of activations four).  us at 2 / 8 tokens, before: 4096 x 4096 9.4 / 11.1, now 8.3 / 10.4;
+// 2048 x 5632 10.8 / 12.8, 8.2 / 11.4; 5120 x 13824 31.8 / 35.6, 26.1 / 32.7 (reading the weights alone takes 6.3 us for 4096 x 4096).
+template <int RT, int TT, int XS>
 __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
                                                      int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int64_t seg_rows, int64_t seg_off, int seg_last, int rows, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 0)) return;
+    static_assert(XS == 16 || TT == 1, "one group of columns where they share a token");
+    const int gone = pi_abort_peek(abort_w);
     constexpr int KS = 8;
     __shared__ dt_f32x4 red[KS][RT * TT][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
@@ -156,50 +163,69 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
     const int t0 = blockIdx.y * (16 * TT);
     if (seg_rows > 0) X += min(n0 / seg_rows, (int64_t) seg_last) * seg_off;
     const int64_t per = (K + 64 * KS - 1) / (64 * KS) * 64, k_begin = wave * per, k_end = min(K, k_begin + per);
+    constexpr int NX = XS / 4;                                         // loads of activations per step and group of columns
+    const int part = li / XS;                                          // of the step's values: this lane's
+    const int x_at = XS == 16 ? kb * 8 : XS == 8 ? kb * 8 + part * 32 : kb * 8 + (part >> 1) * 32 + (part & 1) * 4;
     const uint16_t * wrow[RT]; const float * xrow[TT];
 #pragma unroll
     for (int a = 0; a < RT; a++) wrow[a] = W + min(n0 + min(a * 16 + li, rows - 1), N - 1) * K + kb * 8;
 #pragma unroll
-    for (int b = 0; b < TT; b++) xrow[b] = X + (int64_t) min(t0 + b * 16 + li, T - 1) * xs + kb * 8;
+    for (int b = 0; b < TT; b++) xrow[b] = X + (int64_t) min(t0 + b * 16 + li % XS, T - 1) * xs + x_at;
     dt_f32x4 acc[RT][TT];
 #pragma unroll
     for (int a = 0; a < RT; a++)
 #pragma unroll
         for (int b = 0; b < TT; b++) acc[a][b] = dt_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     const dt_u32x4 zero4 = { 0, 0, 0, 0 }; const dt_f32x4 zerof = { 0.0f, 0.0f, 0.0f, 0.0f };
-    constexpr int U = RT * TT == 1 ? 4 : RT * TT == 2 ? 2 : 1;                   // steps of 64 whose loads go out together
-    auto steps = [&](auto n_steps, int64_t k, bool ok0, bool ok1) {
+    constexpr int U = RT * TT == 1 ? 4 : RT * TT == 2 ? 2 : 1;                                            // steps of 64 whose loads go out together
+    auto steps = [&](auto n_steps, int64_t k, bool ok0, bool ok1) __attribute__((always_inline)) {
         constexpr int NS = decltype(n_steps)::value;
-        dt_u32x4 af[NS][RT][2]; dt_f32x4 xf[NS][TT][4];
+        const bool okx = XS == 16 || (XS == 8 ? part : part >> 1) == 0 ? ok0 : ok1;     // (fewer columns: of this lane's own values)
+        dt_u32x4 af[NS][RT][2]; dt_f32x4 xf[NS][TT][NX];
 #pragma unroll
         for (int u = 0; u < NS; u++) {
 #pragma unroll
-            for (int a = 0; a < RT; a++) { af[u][a][0] = ok0 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u) : zero4; af[u][a][1] = ok1 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u + 32) : zero4; }
-#pragma unroll
             for (int b = 0; b < TT; b++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) xf[u][b][i] = (i < 2 ? ok0 : ok1) ? *(const dt_f32x4 *) (xrow[b] + k + 64 * u + (i < 2 ? 0 : 24) + 4 * i) : zerof;
+                for (int i = 0; i < NX; i++) xf[u][b][i] = (i < 2 ? okx : ok1) ? *(const dt_f32x4 *) (xrow[b] + k + 64 * u + (i < 2 ? 0 : 24) + 4 * i) : zerof;
+#pragma unroll
+            for (int a = 0; a < RT; a++) { af[u][a][0] = ok0 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u) : zero4; af[u][a][1] = ok1 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u + 32) : zero4; }
         }
         __builtin_amdgcn_sched_barrier(0);                             // (all of them issued before the first product waits)
 #pragma unroll
         for (int u = 0; u < NS; u++)
 #pragma unroll
             for (int b = 0; b < TT; b++) {
-                const dt_u32x4 b0 = dt_pack8(xf[u][b][0], xf[u][b][1]), b1 = dt_pack8(xf[u][b][2], xf[u][b][3]);
+                dt_u32x4 b0, b1;
+                if constexpr (XS == 16) { b0 = dt_pack8(xf[u][b][0], xf[u][b][1]); b1 = dt_pack8(xf[u][b][2], xf[u][b][3]); }
+                else if constexpr (XS == 8) {
+                    b0 = dt_pack8(xf[u][b][0], xf[u][b][1]);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) b1[i] = dn_from_lane<8>(b0[i]);
+                } else {
+                    const uint32_t p0 = dt_pack(xf[u][b][0][0], xf[u][b][0][1]), p1 = dt_pack(xf[u][b][0][2], xf[u][b][0][3]);
+                    b0 = dt_u32x4{ p0, p1, dn_from_lane<4>(p0), dn_from_lane<4>(p1) };
+                    b1 = dt_u32x4{ dn_from_lane<8>(p0), dn_from_lane<8>(p1), dn_from_lane<12>(p0), dn_from_lane<12>(p1) };
+                }
 #pragma unroll
                 for (int a = 0; a < RT; a++) { acc[a][b] = dt_mfma(af[u][a][0], b0, acc[a][b]); acc[a][b] = dt_mfma(af[u][a][1], b1, acc[a][b]); }
             }
     };
     using one = std::integral_constant<int, 1>;
-    int64_t k = k_begin;
-    if constexpr (U > 1) for (; k + 64 * U <= k_end; k += 64 * U) steps(std::integral_constant<int, U>{}, k, true, true);
-    for (; k + 64 <= k_end; k += 64) steps(one{}, k, true, true);
+    // Where the waves' parts begin a multiple of 4 KB apart (K 16384), all of them and all rows ask the same memory channel at a time: there workgroups begin at steps of their own and go round
+    // (4096 x 16384 at 2 / 8 / 16 tokens: 40.6 / 43.6 / 49.8 us, with this and the shared columns 23.3 / 31.3 / 44.6; at K 4096 and 8192 it gives nothing and the order stays)
+    const int turns = k_begin < K ? (int) ((k_end - k_begin) / (64 * U)) : 0, turn = per % 2048 == 0 ? (int) (((uint64_t) ((blockIdx.x >> 3) * 0x9E3779B1u) * (uint32_t) turns) >> 32) : 0;
+    for (int i = turn; i < turns; i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
+    for (int i = 0; i < turn; i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
+    int64_t k = k_begin + 64 * U * (int64_t) turns;
+    if constexpr (U > 1) for (; k + 64 <= k_end; k += 64) steps(one{}, k, true, true);
     if (k < k_end) steps(one{}, k, k + kb * 8 < K, k + kb * 8 + 32 < K);       // (K % 8 == 0)
 #pragma unroll
     for (int a = 0; a < RT; a++)
 #pragma unroll
         for (int b = 0; b < TT; b++) red[wave][a * TT + b][lane] = acc[a][b];
     __syncthreads();
+    if (pi_abort_late(gone, abort_w, 0)) return;                       // (asked for at the top, looked at here: on its own the trip to memory was 0.4 us of every launch)
     for (int i = tid; i < RT * TT * 64; i += 512) {
         const int tile = i >> 6, l = i & 63, tok = t0 + (tile % TT) * 16 + (l & 15);
         if (tok >= T) continue;
@@ -230,36 +256,37 @@ static void launch_rows(const pi_weight * w, const float * x, int64_t xs, int n_
     else PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, nt_acct, bytes, (k_dense_rows<8, VW, EXACT>), dim3(gx, (unsigned) ((n_tok + 7) / 8)), dim3(256), 0, s, W, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, pi_abort_word());
 }
 
-// Rows per workgroup: the chip's 256 compute units take a workgroup each at a time, and a round of them lasts about as long as 8 + rows (K 4096 at 8 tokens: 16 rows 7.8 us a round, 24 10, 32 13; the launch itself 4).  So
-// the split that needs the least, in steps of 4 rows, the larger one of two that need the same.  Against 16 rows (32 from 8192 rows on), us at 2 .. 4 / 8 / 32 tokens: 6144 x 4096 17.6 / 19.8 / 39.0, now 24 rows
-// 13.3 / 14.5 / 24.2; 5120 x 13824 46.6 / 59.3 / 123, now 20 rows 32.8 / 37.8 / 71.7; 16448 x 4096 at 8 41.5, now 24 rows 37.6; 32000 x 4096 at 4 63.8, now 32 rows 52.5; 2048 x 2048 6.5 / 7.0 / 11.8, now 8 rows
-// 5.9 / 6.4 / 11.2
-static int split_rows(int64_t n, int64_t seg_rows) {
+// Rows per workgroup: the chip's 256 compute units take a workgroup each at a time, and a round of them lasts about as long as `base` + rows, the base being the activations (K 4096, us a round at 8 / 16 / 24 / 32 rows:
+// 2 tokens 3.7 / 5.0 / 7.7 / 11.3, 8 tokens 5.7 / 7.6 / 9.8 / 12.2, 16 tokens 9.0 / 11.0 / 12.8 / 15, 32 tokens 16 / 17.2 / 19.4 / 24; K 2048 at 2 tokens - / 3.6 / 5.0 / 6.2).  So the split that needs the least,
+// in steps of 4 rows, the larger one of two that need the same.  The addresses of rows of whole 8 KB meet, which is what a round of many of them at few tokens waits for (16384 x 4096 at 2 tokens: 32 rows 27.9, 16 rows
+// 23.5; 32000 x 4096 51.1 and 44.7, but 32000 x 2048 25.5 and 28.7).
+static int split_rows(int64_t n, int64_t k, int n_tok, int64_t seg_rows) {
+    const int base = n_tok <= 4 ? 6 : n_tok <= 8 ? 13 : n_tok <= 16 ? 28 : 70;
     int best = 16; int64_t least = INT64_MAX;
     for (int r = 32; r >= 4; r -= 4) {
-        const int64_t cost = ((n + r - 1) / r + 255) / 256 * (8 + r);
+        const int64_t cost = ((n + r - 1) / r + 255) / 256 * (base + r + (n_tok <= 4 && k % 4096 == 0 && r > 16 ? (r - 16) / 2 : 0));
         if (cost < least && (seg_rows <= 0 || seg_rows % r == 0)) { least = cost; best = r; }
     }
     return best;
 }
 // Which kernel takes a pass of serving precision (aligned rows; measured against each other over 512 .. 32000 rows, K 1024 .. 4096, us):
-//   1 token                the mat-vec; 2 tokens of a matrix of at most 4 M values too (2048 x 2048: 5.5, k_dense_split 5.7: both at the floor of a launch), and rows of 8 KB where
-//                          k_dense_split would take 32 of them a workgroup (their addresses meet: 8192 rows of 3968 / 4096 / 4224 values 12.6 / 16.4 / 13.3, the mat-vec 14.7 / 14.9 / 16.3; 32000 rows of 4096 52.7
-//                          and 47.1; from 3 tokens on the mat-vec is slower there too, 19.1 for 8192 rows)
-//   .. 32 tokens           k_dense_split (4096 x 4096 at 4 / 8 / 16 / 32 tokens: 9.7 / 11 / 14 / 21; the mat-vec 15 / 28 at 4 / 8, k_dense_tile 27 at 32); of 16384 rows and more only .. 8 tokens, where the tiles
+//   1 token                the mat-vec (at 2 the split kernel is ahead everywhere: 2048 x 2048 4.6 and 5.5, 8192 x 4096 13.3 and 20.1, 32000 x 4096 45 and 70; equal below 1024 x 1024)
+//   .. 32 tokens           k_dense_split (4096 x 4096 at 4 / 8 / 16 / 32 tokens: 8.8 / 10.4 / 14 / 21; the mat-vec 15 / 28 at 4 / 8, k_dense_tile 27 at 32); of 16384 rows and more only .. 8 tokens, where the tiles
 //                          fill the chip and read the activations less often (32000 x 2048 at 24: 41 against 26)
 //   more                   k_dense_tile
-static bool dense_takes_split(int64_t rows, int64_t k, int n_tok, int64_t seg_rows = 0) {
-    return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32) && !(n_tok == 2 && (rows * k <= (4 << 20) || (k == 4096 && split_rows(rows, seg_rows) == 32)));
+static bool dense_takes_split(int64_t rows, int n_tok) {
+    return n_tok > 1 && n_tok <= (rows >= 16384 ? 8 : 32);
 }
 static void launch_split(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias, int64_t seg_rows = 0,
                          int64_t seg_off = 0, int seg_last = 0) {
-    const int r = split_rows(w->ne1, seg_rows);
+    const int r = split_rows(w->ne1, w->ne0, n_tok, seg_rows);
     const bool two = r > 16;
-#define DN_SPLIT(RT, TT) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_split<RT, TT>), dim3((unsigned) ((w->ne1 + r - 1) / r), (unsigned) ((n_tok + 16 * TT - 1) / (16 * TT))), \
+#define DN_SPLIT(RT, TT, XS) PI_KT_LAUNCH(PI_KT_MATVEC, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_split<RT, TT, XS>), dim3((unsigned) ((w->ne1 + r - 1) / r), (unsigned) ((n_tok + 16 * TT - 1) / (16 * TT))), \
                                      dim3(512), 0, s, (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, seg_rows, seg_off, seg_last, r, pi_abort_word())
-    if (n_tok <= 16) { if (two) DN_SPLIT(2, 1); else DN_SPLIT(1, 1); }
-    else { if (two) DN_SPLIT(2, 2); else DN_SPLIT(1, 2); }
+    if (n_tok <= 4)       { if (two) DN_SPLIT(2, 1, 4); else DN_SPLIT(1, 1, 4); }
+    else if (n_tok <= 8)  { if (two) DN_SPLIT(2, 1, 8); else DN_SPLIT(1, 1, 8); }
+    else if (n_tok <= 16) { if (two) DN_SPLIT(2, 1, 16); else DN_SPLIT(1, 1, 16); }
+    else                  { if (two) DN_SPLIT(2, 2, 16); else DN_SPLIT(1, 2, 16); }
 #undef DN_SPLIT
 }
 // The largest tile that gives the chip's 256 compute units one workgroup each; where the next larger one would not, two groups of waves share K (measured at 512 .. 32000 rows x 24 .. 2048 tokens; the crossings:
@@ -288,8 +315,8 @@ extern "C" int pi_op_dense_bias(const pi_weight * w, const float * bias, const f
     const double bytes = 2.0 * K * w->ne1 + 4.0 * n_tok * (K + w->ne1);
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
     const bool al8  = K % 4 == 0 && ((uintptr_t) w->p0 % 8) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
-    if (!exact && al16 && (n_tok > 2 || dense_takes_split(w->ne1, K, n_tok))) {
-        if (dense_takes_split(w->ne1, K, n_tok)) launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
+    if (!exact && al16 && n_tok > 1) {
+        if (dense_takes_split(w->ne1, n_tok)) launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
         else launch_tile(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
         PI_CHECK_LAUNCH(); return 0;
     }
@@ -309,7 +336,7 @@ extern "C" int pi_op_dense_segments(const pi_weight * w, const float * x, int64_
     const int64_t K = w->ne0;
     if (x_stride < (int64_t) (n_seg - 1) * seg_off + K || out_stride < w->ne1) { pi_set_error("pi_op_dense_segments: row strides below the sizes"); return -1; }
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0 && seg_off % 4 == 0;
-    if (!exact && al16 && dense_takes_split(w->ne1, K, n_tok, seg_rows) && seg_rows % 32 == 0) {
+    if (!exact && al16 && dense_takes_split(w->ne1, n_tok) && seg_rows % 32 == 0) {
         launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, (hipStream_t) stream, 2.0 * K * w->ne1 + 4.0 * n_tok * (n_seg * K + w->ne1), nullptr, seg_rows, seg_off, n_seg - 1);
         PI_CHECK_LAUNCH(); return 0;
     }

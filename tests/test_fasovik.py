@@ -180,6 +180,27 @@ def test_dense_two_tokens_of_rows_of_8_kb(N):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [2, 4, 5, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(8, 5), (504, 33), (2056, 300), (16384, 70), (16392, 9), (4096, 4100)])
+def test_dense_few_tokens_share_columns(K, N, T):
+    """both sides of the lines at 4, 8 and 16 tokens, K below a wave's step, ragged and in parts that begin 4 KB apart; each token's result stays its own when another one is not finite
+    (fp32 sums of at most 16392 exact products: 4e-6 of their mean)"""
+    U, lib = gpu()
+    rng = np.random.default_rng(K + N + T)
+    w, x = bf(rng, N, K, s=0.2), rng.standard_normal((T, K + 4)).astype(np.float32)
+    wd, xd, od = upload_bf16(lib, w), U.Dev(x), U.Dev(nbytes=4 * T * (N + 3))
+    L.check(lib.pi_op_dense(wd, xd.ptr, K + 4, T, od.ptr, N + 3, 0, N, 0, 0, None))
+    got = od.get(np.float32, (T, N + 3))[:, :N].copy()
+    assert rel_rms(got, O.bf16_round(x[:, :K]).astype(np.float64) @ w.T.astype(np.float64)) < 4e-6
+    x[T // 2, K // 2], x[T // 2, 0] = np.inf, np.nan
+    xd = U.Dev(x)
+    L.check(lib.pi_op_dense(wd, xd.ptr, K + 4, T, od.ptr, N + 3, 0, N, 0, 0, None))
+    bad = od.get(np.float32, (T, N + 3))[:, :N]
+    assert np.isnan(bad[T // 2]).all() and np.array_equal(np.delete(bad, T // 2, 0), np.delete(got, T // 2, 0))
+    lib.pi_weight_free(wd)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("K,N,T", [(40, 37, 1), (33, 10, 3), (512, 70, 5), (1024, 130, 8), (96, 200, 17), (64, 64, 64), (520, 33, 150), (256, 300, 200), (72, 130, 129)])
 @pytest.mark.parametrize("exact", [True, False])
 def test_dense_every_kernel_and_width(K, N, T, exact):
