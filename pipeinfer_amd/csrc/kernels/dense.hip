@@ -9,9 +9,9 @@
 //                  6.7 TB/s at 32000 x 4096, 4.3 at 4096 x 4096, 4 us of launch below 1024 x 1024) and every width of the fp32 mode
 //   k_dense_split  serving precision, 2 .. 32 tokens: 4 .. 32 rows x all tokens per workgroup on the matrix cores, K over its eight waves.  Bound by the weight stream (5.8 TB/s at 32000 x 4096 and 2
 //                  tokens, 4.6 at 8) and by the address unit.  On the mat-vec every row reads all tokens' activations again, 2 T times its own bytes: 28 us for 4096 x 4096 at 8 tokens, 11 here
-//   k_dense_tile   serving precision, more tokens: tiles of 64 .. 128 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory
-//                  (26 bytes a cycle of cold weights and activations), large ones by the shared levels of memory and the steps' latency: 730 TFLOP/s at 16384 x 4096 x 2048 tokens (the tiles without
-//                  deeper prefetch and in plain order: 472), 17 us for 2048 x 2048 x 512 (82 before)
+//   k_dense_tile   serving precision, more tokens: tiles of 64 .. 256 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory and by the
+//                  latency of a step, large ones by the shared levels of memory: 850 TFLOP/s at 16384 x 4096 x 2048 tokens (128 x 128 tiles with a step's parts one after another: 710), 14 us for
+//                  2048 x 2048 x 512 (17)
 //   k_embed        rows of the table gathered, widened and scaled
 #include "ops_common.h"
 #include "dense_tile.h"
@@ -118,7 +118,7 @@ static __device__ __forceinline__ void dn_store4(dt_f32x4 v4, int64_t row, int64
 // BN rows x BT tokens per workgroup (dense_tile.h).  Workgroup n runs on XCD n % 8: an XCD takes a contiguous run of tiles, eight blocks of rows wide and then along the tokens, so that the 64 tiles it
 // works on at a time are 8 x 8 and share the rows and tokens that pass through its L2
 template <int BN, int BT, int WN, int WT, int KG>
-__global__ void __launch_bounds__(256 * KG, 2) k_dense_tile(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
+__global__ void __launch_bounds__(64 * WN * WT * KG, 2) k_dense_tile(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
                                                        int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int tok_blocks, int tiles, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 1)) return;
     __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES(BN, BT, KG)];
@@ -126,16 +126,15 @@ __global__ void __launch_bounds__(256 * KG, 2) k_dense_tile(const uint16_t * __r
     if (tile >= tiles) return;
     const int row_blocks = tiles / tok_blocks, grp = tile / (8 * tok_blocks), in_grp = tile % (8 * tok_blocks), gsz = min(8, row_blocks - 8 * grp);
     const int64_t n0 = (int64_t) (8 * grp + in_grp % gsz) * BN;
-    const int t0 = (in_grp / gsz) * BT, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    const int64_t nr = min(n0 + (tid >> 3), N - 1); const int tr = min(t0 + (tid >> 3), T - 1);
-    dt_offs wo, xo;                                                    // the rows this thread stages, from the first
+    const int t0 = (in_grp / gsz) * BT, tid = threadIdx.x % (64 * WN * WT), lane = tid & 63, wave = tid >> 6;
+    dt_offs wo, xo;                                                    // the rows this thread stages, from the tile's first
 #pragma unroll
-    for (int i = 0; i < BN / 32; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, N - 1) - nr) * K);
+    for (int i = 0; i < BN / (8 * WN * WT); i++) wo[i] = (uint32_t) ((min(n0 + (tid >> 3) + 8 * WN * WT * i, N - 1) - n0) * K);
 #pragma unroll
-    for (int i = 0; i < BT / 32; i++) xo[i] = (uint32_t) ((min(tr + 32 * i, T - 1) - tr) * xs);
+    for (int i = 0; i < BT / (8 * WN * WT); i++) xo[i] = (uint32_t) ((min(t0 + (tid >> 3) + 8 * WN * WT * i, T - 1) - t0) * xs);
     dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
-    dt_tile<BN, BT, WN, WT, 2, KG, false>(W + nr * K, wo, X + (int64_t) tr * xs, xo, 0, [](float a, float) { return a; }, K, lds, acc);
-    if (KG > 1 && threadIdx.x >= 256) return;
+    dt_tile<BN, BT, WN, WT, 2, KG, false>(W + n0 * K, wo, X + (int64_t) t0 * xs, xo, 0, [](float a, float) { return a; }, K, lds, acc);
+    if (KG > 1 && threadIdx.x >= 64 * WN * WT) return;
 #pragma unroll
     for (int b = 0; b < BT / WT / 16; b++) {
         const int tok = t0 + (wave % WT) * (BT / WT) + b * 16 + (lane & 15);
@@ -289,17 +288,23 @@ static void launch_split(const pi_weight * w, const float * x, int64_t xs, int n
     else                  { if (two) DN_SPLIT(2, 2, 16); else DN_SPLIT(1, 2, 16); }
 #undef DN_SPLIT
 }
-// The largest tile that gives the chip's 256 compute units one workgroup each; where the next larger one would not, two groups of waves share K (measured at 512 .. 32000 rows x 24 .. 2048 tokens; the crossings:
-// 2048 x 2048 at 512 tokens 64 x 64 in two groups 17.1, one 18.6, 128 x 64 21.1; at 1000 128 x 64 in two groups 24.3, one 25.9, 64 x 64 27.9, 128 x 128 34.6; 6144 x 2048 at 512 128 x 64 39.1, 128 x 128 41.9;
-// 8192 x 4096 at 1000 128 x 128 108, 128 x 64 129)
+// The tile that needs the least time, by rounds of 256 workgroups (one per compute unit; us a round at K 2048): 64 x 64 and 128 x 64 in two groups of waves that share K 14.2 and 23, 128 x 128 by eight waves 29.6,
+// 256 x 128 by eight 47; of 128 x 128 by four waves two fit a compute unit and a last round that is not full costs less: 15 + 23.5 a round, from the second on.  Measured at 512 .. 32000 rows x 64 .. 2048 tokens; the crossings, K 2048:
+// 2048 rows at 1000 tokens 128 x 64 19.9, 128 x 128 by eight 25.6, at 2048 32.7 (by four) and 29.6; 6144 at 1000 128 x 128 by four 48.0, by eight 54.3, 256 x 128 46.4, at 2048 80.6 / 85.1 / 84.4; K 4096: 4608 rows
+// at 2048 132 / 139 / 136, 16384 at 512 118 / 124 / 89.5, at 2048 376 / 390 / 323
 static void launch_tile(const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, double bytes, const float * bias) {
     auto tiles = [&](int bn, int bt) { return (w->ne1 + bn - 1) / bn * ((n_tok + bt - 1) / bt); };
-#define DN_TILE(BN, BT, KG) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_tile<BN, BT, 2, 2, KG>), dim3((unsigned) ((tiles(BN, BT) + 7) / 8 * 8)), dim3(256 * KG), 0, s, \
+#define DN_TILE(BN, BT, WN, WT, KG) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_tile<BN, BT, WN, WT, KG>), dim3((unsigned) ((tiles(BN, BT) + 7) / 8 * 8)), dim3(64 * WN * WT * KG), 0, s, \
                      (const uint16_t *) w->p0, w->ne0, w->ne1, x, xs, n_tok, out, os, act_a, rows_a, act_b, bias, (n_tok + BT - 1) / BT, (int) tiles(BN, BT), pi_abort_word())
-    if (tiles(64, 64) <= 256) DN_TILE(64, 64, 2);
-    else if (tiles(128, 64) <= 256) DN_TILE(128, 64, 2);
-    else if (tiles(128, 128) <= 256) DN_TILE(128, 64, 1);
-    else DN_TILE(128, 128, 1);
+    auto rounds = [&](int bn, int bt) { return (double) ((tiles(bn, bt) + 255) / 256); };
+    const double cost[5] = { 14.2 * rounds(64, 64), 23.0 * rounds(128, 64), 29.6 * rounds(128, 128), 47.0 * rounds(256, 128), tiles(128, 128) <= 256 ? 1e30 : 15.0 + 23.5 * (double) tiles(128, 128) / 256 };
+    switch ((int) (std::min_element(cost, cost + 5) - cost)) {
+        case 0:  DN_TILE(64, 64, 2, 2, 2); break;
+        case 1:  DN_TILE(128, 64, 2, 2, 2); break;
+        case 2:  DN_TILE(128, 128, 4, 2, 1); break;
+        case 3:  DN_TILE(256, 128, 4, 2, 1); break;
+        default: DN_TILE(128, 128, 2, 2, 1);
+    }
 #undef DN_TILE
 }
 
@@ -315,7 +320,7 @@ extern "C" int pi_op_dense_bias(const pi_weight * w, const float * bias, const f
     const double bytes = 2.0 * K * w->ne1 + 4.0 * n_tok * (K + w->ne1);
     const bool al16 = K % 8 == 0 && ((uintptr_t) w->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
     const bool al8  = K % 4 == 0 && ((uintptr_t) w->p0 % 8) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0;
-    if (!exact && al16 && n_tok > 1) {
+    if (!exact && al16 && n_tok > 1 && (dense_takes_split(w->ne1, n_tok) || (K < (1 << 22) && x_stride < (1 << 22)))) {      // (a tile's offsets in 32 bits)
         if (dense_takes_split(w->ne1, n_tok)) launch_split(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
         else launch_tile(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias);
         PI_CHECK_LAUNCH(); return 0;

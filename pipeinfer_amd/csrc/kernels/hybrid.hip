@@ -1928,8 +1928,8 @@ __global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ 
 // out dn[slot][n].  glu: UP leaves the 2 * ff rows [gate | up] of an expert raw, !UP (PAIR) joins them while it stages them (bs = 2 * ff, K = ff).  What bounds it: as k_dense_tile, whose tiles these are.  Operands
 // straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048 (now 116 and 125: 475 and 440 TFLOP/s), 44 and 23 us for 24 tokens' of 1024 x 512
 // (10 and 7).
-template <int BN, int BT, int KG, bool UP, bool PAIR>
-__global__ void __launch_bounds__(256 * KG, 2) k_moe_tile(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,
+template <int BN, int BT, int WN, int WT, int KG, bool UP, bool PAIR>
+__global__ void __launch_bounds__(64 * WN * WT * KG, 2) k_moe_tile(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,
                                                           int max_tiles, int glu, float limit, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 1)) return;
     __shared__ __attribute__((aligned(16))) uint8_t lds[DT_LDS_BYTES(BN, BT, KG)];
@@ -1939,24 +1939,24 @@ __global__ void __launch_bounds__(256 * KG, 2) k_moe_tile(const uint16_t * __res
     const int grp = work / (8 * row_blocks), in_grp = work % (8 * row_blocks), gsz = min(8, idx[0] - 8 * grp), tile = 8 * grp + in_grp % gsz, n0 = in_grp / gsz * BN;
     const int32_t * tile_e = idx + 1, * tile_s = tile_e + max_tiles, * tile_n = tile_s + max_tiles, * order = tile_n + max_tiles;
     const int e = tile_e[tile], start = tile_s[tile], len = tile_n[tile];
-    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-    const int nr = min(n0 + (tid >> 3), rows - 1);
+    constexpr int SR = 8 * WN * WT;
+    const int tid = threadIdx.x % (64 * WN * WT), lane = tid & 63, wave = tid >> 6;
     dt_offs wo; dt_offs64 xo;                                          // the rows this thread stages
 #pragma unroll
-    for (int i = 0; i < BN / 32; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, rows - 1) - nr) * K);
+    for (int i = 0; i < BN / SR; i++) wo[i] = (uint32_t) ((min(n0 + (tid >> 3) + SR * i, rows - 1) - n0) * K);
 #pragma unroll
-    for (int i = 0; i < BT / 32; i++) { const int slot = order[start + min((tid >> 3) + 32 * i, len - 1)]; xo[i] = (uint64_t) (UP ? slot / top : slot) * (uint64_t) bs; }
-    dt_f32x4 acc[BN / 2 / 16][BT / 2 / 16];
-    dt_tile<BN, BT, 2, 2, 2, KG, PAIR>(W + ((int64_t) e * rows + nr) * K, wo, B, xo, K, [=](float a, float b) { return hy_glu(a, b, glu, limit); }, K, lds, acc);
-    if (KG > 1 && threadIdx.x >= 256) return;
+    for (int i = 0; i < BT / SR; i++) { const int slot = order[start + min((tid >> 3) + SR * i, len - 1)]; xo[i] = (uint64_t) (UP ? slot / top : slot) * (uint64_t) bs; }
+    dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
+    dt_tile<BN, BT, WN, WT, 2, KG, PAIR>(W + ((int64_t) e * rows + n0) * K, wo, B, xo, K, [=](float a, float b) { return hy_glu(a, b, glu, limit); }, K, lds, acc);
+    if (KG > 1 && threadIdx.x >= 64 * WN * WT) return;
 #pragma unroll
-    for (int b = 0; b < BT / 2 / 16; b++) {
-        const int si = (wave & 1) * (BT / 2) + b * 16 + (lane & 15);
+    for (int b = 0; b < BT / WT / 16; b++) {
+        const int si = (wave % WT) * (BT / WT) + b * 16 + (lane & 15);
         if (si >= len) continue;
         float * o = out + (int64_t) order[start + si] * rows;
 #pragma unroll
-        for (int a = 0; a < BN / 2 / 16; a++) {
-            const int row = n0 + (wave >> 1) * (BN / 2) + a * 16 + (lane >> 4) * 4;
+        for (int a = 0; a < BN / WN / 16; a++) {
+            const int row = n0 + (wave / WT) * (BN / WN) + a * 16 + (lane >> 4) * 4;
             dt_f32x4 v = acc[a][b];
             if (UP && !glu) {
 #pragma unroll
@@ -1986,12 +1986,12 @@ static int moe_tile_len(int n_slots, int n_exp) { return n_slots / n_exp >= 256 
 // rows of a tile: as for k_dense_tile, the largest that gives every compute unit a workgroup; where none does, two groups of waves share K
 template <bool UP>
 static void moe_tile_launch(const uint16_t * w, int64_t K, int rows, const float * b, int64_t bs, int top, const int32_t * idx, int mt, int tl, int est, int glu, float limit, float * out, int nta, double bytes, hipStream_t s) {
-#define MOE_GO2(BN, BT, KG, PAIR) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, bytes, (k_moe_tile<BN, BT, KG, UP, PAIR>), dim3((unsigned) ((mt * ((rows + BN - 1) / BN) + 7) / 8 * 8)), dim3(256 * KG), 0, s, \
+#define MOE_GO2(BN, BT, WN, WT, KG, PAIR) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, bytes, (k_moe_tile<BN, BT, WN, WT, KG, UP, PAIR>), dim3((unsigned) ((mt * ((rows + BN - 1) / BN) + 7) / 8 * 8)), dim3(64 * WN * WT * KG), 0, s, \
                                                w, K, rows, b, bs, top, idx, mt, glu, limit, out, pi_abort_word())
-#define MOE_GO(BN, BT, KG) do { if constexpr (UP) MOE_GO2(BN, BT, KG, false); else if (glu) MOE_GO2(BN, BT, KG, true); else MOE_GO2(BN, BT, KG, false); } while (0)
+#define MOE_GO(BN, BT, KG) do { if constexpr (UP) MOE_GO2(BN, BT, 2, 2, KG, false); else if (glu) MOE_GO2(BN, BT, 2, 2, KG, true); else MOE_GO2(BN, BT, 2, 2, KG, false); } while (0)
     const int wg128 = est * ((rows + 127) / 128);
-    if (tl == 128 && !UP && glu) MOE_GO2(64, 128, 1, !UP);            // (two values for each of X: the registers do not hold the larger tile)
-    else if (tl == 128) MOE_GO2(128, 128, 1, false);
+    if (tl == 128 && !UP && glu) MOE_GO2(64, 128, 2, 4, 1, !UP);            // (two values for each of X: the registers do not hold the larger tile)
+    else if (tl == 128) MOE_GO2(128, 128, 4, 2, 1, false);
     else if (wg128 >= 256) MOE_GO(128, 64, 1);
     else if (wg128 >= 128) MOE_GO(128, 64, 2);
     else MOE_GO(64, 64, 2);

@@ -30,14 +30,13 @@ __global__ void __launch_bounds__(256, 2) k_latent_expand(const float * __restri
     if (dyn) { if (live_max > 0 && dyn[1] > live_max) return; cell1 = min(cell1, dyn[1]); }
     const int t0 = cell0 + (in_grp / gsz) * 64, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (t0 >= cell1) return;                                          // (cells of the context that hold nothing yet)
-    const int64_t nr = min(n0 + (tid >> 3), N - 1); const int tr = min(t0 + (tid >> 3), cell1 - 1);
     dt_offs wo, xo;
 #pragma unroll
-    for (int i = 0; i < 4; i++) wo[i] = (uint32_t) ((min(nr + 32 * i, N - 1) - nr) * rank);
+    for (int i = 0; i < 4; i++) wo[i] = (uint32_t) ((min(n0 + (tid >> 3) + 32 * i, N - 1) - n0) * rank);
 #pragma unroll
-    for (int i = 0; i < 2; i++) xo[i] = (uint32_t) ((min(tr + 32 * i, cell1 - 1) - tr) * width);
+    for (int i = 0; i < 2; i++) xo[i] = (uint32_t) ((min(t0 + (tid >> 3) + 32 * i, cell1 - 1) - t0) * width);
     dt_f32x4 acc[4][2];
-    dt_tile<128, 64, 2, 2, 2, 1, false, 3>(W + nr * rank, wo, cache + (int64_t) tr * width, xo, 0, [](float a, float) { return a; }, rank, lds, acc);
+    dt_tile<128, 64, 2, 2, 2, 1, false, 3>(W + n0 * rank, wo, cache + (int64_t) t0 * width, xo, 0, [](float a, float) { return a; }, rank, lds, acc);
     float * out = is_v ? vo : ko;
 #pragma unroll
     for (int b = 0; b < 2; b++) {
