@@ -54,19 +54,20 @@ template <int CTRL> static __device__ __forceinline__ float dpp_add(float x) {
 #endif
 }
 
-template <int HD, int RW, bool ALIBI = false>
+// BEHIND: launched behind k_attention_tiles, which does a pass of up to tile_cells cells (an instance of its own: the look alone cost a single token's launch 0.4 us of 8.7)
+template <int HD, int RW, bool ALIBI = false, bool BEHIND = false>
 __global__ void __launch_bounds__(256) k_attention(const att_args ga) {
     extern __shared__ float smem[];
     __shared__ float redf[RW][4];
     __shared__ unsigned long long redu[RW][4];
     att_args g = ga;
-    if (ga.tile_cells > 0 && ga.dyn[1] <= ga.tile_cells) return;
     const int s_stride = ga.n_kv;                           // LDS rows keep the static stride
     const int hk = blockIdx.x, chunk = blockIdx.y;
     const int r = g.n_head / g.n_head_kv;                   // query heads per kv head (broadcast rule i02 = i12 / r2, ggml.c:9425)
     // kv_self.n of the run this workgroup's token belongs to (llama.cpp:5571): the reference's vec_dot_f16 sums the last n % 32 cells apart, in double, so every token
     // must see exactly the n its own run was started with — a pass that carries several runs brings one n per token (the launcher keeps a workgroup inside one token)
     if (ga.dyn) g.n_kv = (ga.per_token && ga.dyn[3]) ? ga.dyn[4 + ga.dyn[2] + (chunk * RW) / r] : ga.dyn[1];
+    if constexpr (BEHIND) if (g.n_kv <= ga.tile_cells) return;
     const int n_rows_total = g.n_tok * r;
     const int row0 = chunk * RW;
     const int n_rows = min(RW, n_rows_total - row0);
@@ -691,6 +692,7 @@ __global__ void __launch_bounds__(256) k_attention_any(const att_args ga, const 
 // raises the dynamic-LDS limit of the kernel for contexts longer than ~2000 cells; call once outside any graph capture
 template <int HD, int RW> static int att_set_lds(size_t lds) {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention<HD, RW, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+    PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention<HD, RW, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_attention<HD, RW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
     return 0;
 }
@@ -737,8 +739,16 @@ static void att_launch(const att_args & g, int rows, int rw, hipStream_t stream)
     const int nt = g.n_tok > 0 ? g.n_tok : 1;
     const int n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv;      // (eager launches of the engine: the pass's own n_kv)
     const double bytes = (double) n_kv_priced * g.n_head_kv * HD * 2 * 2 + (double) nt * g.n_head * HD * (2 + 4);
-    // (a launch behind k_attention_tiles is not counted: one of the two does the work)
-#define ATT_GO(...) do { if (g.tile_cells > 0) hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(256), lds, stream, g); else PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (__VA_ARGS__), grid, dim3(256), lds, stream, g); } while (0)
+    if (g.tile_cells > 0) {                                  // behind k_attention_tiles (without ALiBi): not counted, one of the two does the work
+        switch (rw) {
+            case 1: hipLaunchKernelGGL((k_attention<HD, 1, false, true>), grid, dim3(256), lds, stream, g); break;
+            case 2: hipLaunchKernelGGL((k_attention<HD, 2, false, true>), grid, dim3(256), lds, stream, g); break;
+            case 4: hipLaunchKernelGGL((k_attention<HD, 4, false, true>), grid, dim3(256), lds, stream, g); break;
+            default: hipLaunchKernelGGL((k_attention<HD, 8, false, true>), grid, dim3(256), lds, stream, g); break;
+        }
+        return;
+    }
+#define ATT_GO(...) PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (__VA_ARGS__), grid, dim3(256), lds, stream, g)
     if (g.alibi_m) {
         switch (rw) {
             case 1: ATT_GO(k_attention<HD, 1, true>); break;
