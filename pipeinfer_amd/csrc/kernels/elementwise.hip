@@ -685,9 +685,9 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // stage 1: grid (n_tok, NCH) — each workgroup finds the k best of its slice of the vocabulary and its partial max / sum-exp
 // stage 2: one workgroup per token merges NCH*k candidates (same ordering) and the partial sums.
 #define TOPK_NCH 32
-// What bounds it: the k selection rounds (8 MB of logits a millisecond of reading is nothing beside them).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best, so a round is
-// two wave reductions and one rescan of the lane that lost its best — no barrier, no rescan of everything.  (A workgroup per slice that looked at all its values in every round and met at a barrier: 16.7 us for one
-// row of 32000, 607 for 2048 rows; now 8.6 and 144.)  WS waves share a slice.  One up to a vocabulary of 65536
+// What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One wave to a
+// slice: the least of eight lane groups' bests is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  Four: a round for each of the k, two wave reductions and one rescan of the lane
+// that lost its best.  (Rounds for one wave as well, two kernels together: 13.0 us for one row of 32000, 44 for 512, 142 for 2048, now 12.3, 33 and 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
 // (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
 // One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
@@ -708,7 +708,8 @@ template <int VPT, int WS>
 __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
-    __shared__ uint32_t met_key[WS > 1 ? 32 : 1]; __shared__ int met_id[WS > 1 ? 32 : 1]; __shared__ float met_sum[4];
+    constexpr int MET = WS > 1 ? 32 : 256;                              // the four waves' bests; a wave's own candidates
+    __shared__ uint32_t met_key[MET]; __shared__ int met_id[MET]; __shared__ float met_sum[4], met_val[WS > 1 ? 1 : MET];
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per), own0 = lo + lane + (WS > 1 ? 64 * wave : 0);
     const float * l = logits + (int64_t) t * n_vocab;
@@ -722,8 +723,12 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     } else for (int i = own0, m = 0; i < hi; i += STEP, m++) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = m; } }
     if (pi_abort_late(gone, abort_w)) return;
     uint32_t wk = bk; int wi = bk ? own0 + STEP * bm : 0x7fffffff;
-    topk_best(wk, wi);
-    uint32_t top = wk;
+    uint32_t top = bk, low = 0;                                         // low: at least eight values are not below it — the least of the bests of eight lanes each (lanes of the same number mod 8)
+    if constexpr (WS == 1) {
+        top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<8>((int) top));
+        low = top;
+        pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); low = min(low, (uint32_t) pi_partner<O>((int) low)); });
+    } else { topk_best(wk, wi); top = wk; }
     if constexpr (WS > 1) {
         if (lane == 0) met_key[wave] = wk;
         __syncthreads();
@@ -744,6 +749,37 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
     } else { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; }
     const int64_t out = ((int64_t) t * TOPK_NCH + ch) * k;
+    if constexpr (WS == 1) {
+        // what is not below `low` goes to a lane each, which counts those ahead of it
+        const uint32_t least = max(k == 1 ? top : low, 1u);
+        uint64_t who[VPT]; int n = 0;
+#pragma unroll
+        for (int m = 0; m < VPT; m++) { who[m] = __ballot(key[m] >= least); n += __popcll(who[m]); }
+        if (n <= 64) {                                                  // (else, a crowd of equal values: the rounds below)
+            int base = 0;
+#pragma unroll
+            for (int m = 0; m < VPT; m++) {
+                if (key[m] >= least) {
+                    const int at = base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[m], 0));
+                    met_key[64 * wave + at] = key[m]; met_id[64 * wave + at] = lo + lane + 64 * m; met_val[64 * wave + at] = rv[m];
+                }
+                base += __popcll(who[m]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t ck = lane < n ? met_key[64 * wave + lane] : 0u; const int ci = lane < n ? met_id[64 * wave + lane] : 0x7fffffff;
+            const float cv = lane < n ? met_val[64 * wave + lane] : -INFINITY;
+            int ahead = 0;
+#pragma unroll 4
+            for (int j = 0; j < n; j++) {
+                const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(ci, j);
+                ahead += kj > ck || (kj == ck && ij < ci);
+            }
+            if (lane < n ? ahead < k : lane < k) { const int64_t at = out + (lane < n ? ahead : lane); cid[at] = ci; cval[at] = cv; }
+            return;
+        }
+        topk_best(wk, wi);
+    }
     int own = 0x7fffffff; uint32_t own_key = 0;                       // lane r keeps the r-th: their values are read back together, not one by one between the rounds
     for (int r = 0; ; r++) {
         if (lane == r) { own = wi; own_key = wk; }
