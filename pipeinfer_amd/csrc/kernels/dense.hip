@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) k_embed(const uint16_t * __restrict__ tab
 template <int TT, int VW, bool EXACT>
 __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict__ W, int64_t K, int64_t N, const float * __restrict__ X, int64_t xs, int T, float * __restrict__ Y, int64_t ys,
                                                     int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int64_t seg_rows, int64_t seg_off, int seg_last, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w, 0)) return;
+    const int gone = pi_abort_peek(abort_w);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t row = (int64_t) blockIdx.x * 4 + wave;
     if (row >= N) return;
@@ -74,6 +74,28 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
 #pragma unroll
     for (int i = 0; i < TT; i++) acc[i] = 0.0f;
     const uint16_t * w = W + row * K;
+    if constexpr (TT == 1 && VW == 8) {
+        // one token: two steps of 512 values go out together (a step at a time 32000 x 1024 / 2048 took 15.1 / 25.8 us, now 13.4 / 23.5).  Rows of 8 KB and more keep single steps: 32000 x 4096 48.7, in pairs 50.1;
+        // 5120 x 13824 27.5, in pairs 31.6
+        const float * x0 = X + (int64_t) t0 * xs + lane * 8;
+        const uint16_t * w0 = w + lane * 8;
+        auto steps = [&](auto n_steps, int64_t k) __attribute__((always_inline)) {
+            constexpr int U = decltype(n_steps)::value;
+            dn_u16x8 wv[U]; float4 xv[U][2];
+#pragma unroll
+            for (int u = 0; u < U; u++) { xv[u][0] = *(const float4 *) (x0 + k + 512 * u); xv[u][1] = *(const float4 *) (x0 + k + 512 * u + 4); wv[u] = *(const dn_u16x8 *) (w0 + k + 512 * u); }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const float xf[8] = { xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w, xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w };
+#pragma unroll
+                for (int i = 0; i < 8; i++) acc[0] = fmaf(dn_widen(wv[u][i]), EXACT ? xf[i] : dn_round(xf[i]), acc[0]);
+            }
+        };
+        int64_t k = 0;
+        if (K < 4096) for (; k + 1024 <= K; k += 1024) steps(std::integral_constant<int, 2>{}, k);
+        for (; k < K; k += 512) if (k + lane * 8 < K) steps(std::integral_constant<int, 1>{}, k);
+    } else
     for (int64_t k = (int64_t) lane * VW; k < K; k += 64 * VW) {
         float wf[VW];
         if constexpr (VW == 8) { const dn_u16x8 v = *(const dn_u16x8 *) (w + k); for (int i = 0; i < 8; i++) wf[i] = dn_widen(v[i]); }
@@ -93,6 +115,7 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
         }
     }
     const int act = row < rows_a ? act_a : act_b;
+    if (pi_abort_late(gone, abort_w, 0)) return;
 #pragma unroll
     for (int tt = 0; tt < TT; tt++) {
         if (t0 + tt >= T) break;
