@@ -8,8 +8,6 @@
 static int absent(const char * what) { pi_set_error("%s: this library was built with the dense-weight kernels only (make -C pipeinfer_amd/csrc builds the full one)", what); return -1; }
 
 int pi_mmq_min_nt() { return INT_MAX; }
-int pi_mmq_max_nt() { return 0; }
-int pi_mmq_step(int, int n_tok, int64_t) { return n_tok; }
 
 extern "C" int pi_op_mmq_min_tokens(void) { return INT_MAX; }
 extern "C" int pi_op_mul_mat_reserve(void) { return 0; }
