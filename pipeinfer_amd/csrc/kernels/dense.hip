@@ -93,25 +93,27 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
             }
         };
         int64_t k = 0;
-        if (K < 4096) for (; k + 1024 <= K; k += 1024) steps(std::integral_constant<int, 2>{}, k);
-        for (; k < K; k += 512) if (k + lane * 8 < K) steps(std::integral_constant<int, 1>{}, k);
-    } else
-    for (int64_t k = (int64_t) lane * VW; k < K; k += 64 * VW) {
-        float wf[VW];
-        if constexpr (VW == 8) { const dn_u16x8 v = *(const dn_u16x8 *) (w + k); for (int i = 0; i < 8; i++) wf[i] = dn_widen(v[i]); }
-        else if constexpr (VW == 4) { const uint2 v = *(const uint2 *) (w + k); wf[0] = __uint_as_float(v.x << 16); wf[1] = __uint_as_float(v.x & 0xffff0000u); wf[2] = __uint_as_float(v.y << 16); wf[3] = __uint_as_float(v.y & 0xffff0000u); }
-        else wf[0] = dn_widen(w[k]);
+        if (K < 4096) for (; k + 1024 <= K && (k == 0 || !(gone & 1)); k += 1024) steps(std::integral_constant<int, 2>{}, k);
+        for (; k < K && (k == 0 || !(gone & 1)); k += 512) if (k + lane * 8 < K) steps(std::integral_constant<int, 1>{}, k);
+    } else {
+        if (pi_abort_late(gone, abort_w, 0)) return;
+        for (int64_t k = (int64_t) lane * VW; k < K; k += 64 * VW) {
+            float wf[VW];
+            if constexpr (VW == 8) { const dn_u16x8 v = *(const dn_u16x8 *) (w + k); for (int i = 0; i < 8; i++) wf[i] = dn_widen(v[i]); }
+            else if constexpr (VW == 4) { const uint2 v = *(const uint2 *) (w + k); wf[0] = __uint_as_float(v.x << 16); wf[1] = __uint_as_float(v.x & 0xffff0000u); wf[2] = __uint_as_float(v.y << 16); wf[3] = __uint_as_float(v.y & 0xffff0000u); }
+            else wf[0] = dn_widen(w[k]);
 #pragma unroll
-        for (int tt = 0; tt < TT; tt++) {
-            if (t0 + tt >= T) break;
-            const float * x = X + (int64_t) (t0 + tt) * xs + k;
-            float xf[VW];
-            if constexpr (VW >= 4) {
+            for (int tt = 0; tt < TT; tt++) {
+                if (t0 + tt >= T) break;
+                const float * x = X + (int64_t) (t0 + tt) * xs + k;
+                float xf[VW];
+                if constexpr (VW >= 4) {
 #pragma unroll
-                for (int i = 0; i < VW; i += 4) { const float4 v = *(const float4 *) (x + i); xf[i] = v.x; xf[i + 1] = v.y; xf[i + 2] = v.z; xf[i + 3] = v.w; }
-            } else xf[0] = x[0];
+                    for (int i = 0; i < VW; i += 4) { const float4 v = *(const float4 *) (x + i); xf[i] = v.x; xf[i + 1] = v.y; xf[i + 2] = v.z; xf[i + 3] = v.w; }
+                } else xf[0] = x[0];
 #pragma unroll
-            for (int i = 0; i < VW; i++) acc[tt] = fmaf(wf[i], EXACT ? xf[i] : dn_round(xf[i]), acc[tt]);
+                for (int i = 0; i < VW; i++) acc[tt] = fmaf(wf[i], EXACT ? xf[i] : dn_round(xf[i]), acc[tt]);
+            }
         }
     }
     const int act = row < rows_a ? act_a : act_b;
@@ -237,8 +239,9 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
     // Where the waves' parts begin a multiple of 4 KB apart (K 16384), all of them and all rows ask the same memory channel at a time: there workgroups begin at steps of their own and go round
     // (4096 x 16384 at 2 / 8 / 16 tokens: 40.6 / 43.6 / 49.8 us, with this and the shared columns 23.3 / 31.3 / 44.6; at K 4096 and 8192 it gives nothing and the order stays)
     const int turns = k_begin < K ? (int) ((k_end - k_begin) / (64 * U)) : 0, turn = per % 2048 == 0 ? (int) (((uint64_t) ((blockIdx.x >> 3) * 0x9E3779B1u) * (uint32_t) turns) >> 32) : 0;
-    for (int i = turn; i < turns; i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
-    for (int i = 0; i < turn; i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
+    // The abort word is asked for at the top and looked at behind the first round of loads: on its own the trip to memory was 0.2 us of every launch (and between loads and products it costs the larger forms 10 %)
+    for (int i = turn; i < turns && (i == turn || !(gone & 1)); i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
+    for (int i = 0; i < turn && !(gone & 1); i++) steps(std::integral_constant<int, U>{}, k_begin + 64 * U * (int64_t) i, true, true);
     int64_t k = k_begin + 64 * U * (int64_t) turns;
     if constexpr (U > 1) for (; k + 64 <= k_end; k += 64) steps(one{}, k, true, true);
     if (k < k_end) steps(one{}, k, k + kb * 8 < K, k + kb * 8 + 32 < K);       // (K % 8 == 0)
@@ -247,7 +250,7 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
 #pragma unroll
         for (int b = 0; b < TT; b++) red[wave][a * TT + b][lane] = acc[a][b];
     __syncthreads();
-    if (pi_abort_late(gone, abort_w, 0)) return;                       // (asked for at the top, looked at here: on its own the trip to memory was 0.4 us of every launch)
+    if (pi_abort_late(gone, abort_w, 0)) return;
     for (int i = tid; i < RT * TT * 64; i += 512) {
         const int tile = i >> 6, l = i & 63, tok = t0 + (tile % TT) * 16 + (l & 15);
         if (tok >= T) continue;
