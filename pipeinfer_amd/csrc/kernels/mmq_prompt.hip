@@ -407,7 +407,7 @@ int pi_mmq_prompt_reserve() {
 // 4096 x 4096 15.2 / 15.7, 8192 x 8192 30.7 / 28.6, 57344 x 8192 109.7 / 94.5; Q6_K 2048 x 5632 20.5 / 21.1, 4096 x 11008 42.4 / 38.1, 8192 x 8192 39.3 / 32.0; from 33 tokens everything is faster here (48 tokens: Q4_K
 // 2048 x 2048 15.1 / 10.2, 1024 x 8192 41.6 / 26.1, 57344 x 8192 191 / 180; Q6_K 1024 x 8192 42.3 / 28.5)
 bool pi_mmq_prompt_wants(int type, int n_tok, int64_t rows) {
-    if (!pi_mmq_supported(type)) return false;
+    if (!pi_mmq_supported(type) || n_tok < pi_mmq_min_nt()) return false;            // (below that the quantisers write no operand planes)
     if (n_tok > 32) return true;
     return n_tok > 16 && (rows + 15) / 16 * 256 / pi_cu_count() >= (type == PI_Q6_K ? 256 : 384);
 }

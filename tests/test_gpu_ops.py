@@ -868,6 +868,39 @@ def test_two_weight_types_share_one_matrix_core_launch(gpu, types, k, n_tok, n_h
         lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q5_K), (O.Q4_K, O.Q6_K, O.Q6_K), (O.Q4_K, O.Q4_K, O.Q4_K)])
+def test_prompts_below_the_first_width_of_the_matrix_cores(gpu, types):
+    """PI_MMQ_MIN_NT=64: the quantisers write no operand planes below 64 tokens, and nothing reads them there - one or two weight types, the widths at which k_mmq_prompt would begin (17 tokens of many rows, 33 of
+    few) and both sides of 64.  The buffer is full of NaNs beforehand; the oracle's bits.  (A process of its own: the variable is read once)"""
+    import subprocess
+    import sys
+    code = """
+import ctypes as C, sys
+import numpy as np
+from tests import gpu_util as U, oracle_lib as O
+from pipeinfer_amd import lib as L
+from pipeinfer_amd.tools import synth
+lib, types, k = U.init(), [int(t) for t in sys.argv[1:]], 512
+assert lib.pi_op_mmq_min_tokens() == 64
+for rows, n_tok in (((100, 33, 17), 40), ((6200, 40, 33), 20), ((100, 33, 17), 63), ((100, 33, 17), 64)):
+    rng = np.random.default_rng(n_tok)
+    act = rng.standard_normal((n_tok, k)).astype(np.float32)
+    blocks = [synth.random_blocks(t, m * k, rng, 0.05).reshape(m, -1) for t, m in zip(types, rows)]
+    ws = [lib.pi_weight_upload(t, k, m, b.ctypes.data_as(C.c_void_p), None) for t, m, b in zip(types, rows, blocks)]
+    xd, q8 = U.Dev(act), U.Dev(np.full(lib.pi_q8_nbytes(O.Q8_K, k, n_tok), 255, np.uint8))
+    L.check(lib.pi_op_quantize(O.Q8_K, xd.ptr, k, n_tok, q8.ptr, None))
+    outs = [U.Dev(nbytes=4 * n_tok * m) for m in rows]
+    L.check(lib.pi_op_mul_mat_multi(3, (C.c_void_p * 3)(*ws), q8.ptr, n_tok, (C.c_void_p * 3)(*[o.ptr for o in outs]), None, None))
+    for t, m, b, dv in zip(types, rows, blocks, outs):
+        assert np.array_equal(dv.get(np.uint32, (n_tok, m)), O.Impl("oracle").mul_mat(t, b, k, m, act).view(np.uint32)), (rows, n_tok, t)
+    for w in ws:
+        lib.pi_weight_free(w)
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code] + [str(t) for t in types], cwd=root, env={**os.environ, "PI_MMQ_MIN_NT": "64"}, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_abort_word_stops_kernels_of_the_cancelled_run_only(gpu):
     """Kernel-granular early cancellation (reference: the abort callback polled between graph nodes, ggml.c:15748-15811, llama.cpp:5665-5687): every hot-path
     kernel launched under pi_set_abort_word asks for (run id << 1 | aborted) on entry and writes nothing once it is aborted.  pi_op_abort_cancel is a compare-and-swap on the run id: it stops the run that
