@@ -685,9 +685,9 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // stage 1: grid (n_tok, NCH) — each workgroup finds the k best of its slice of the vocabulary and its partial max / sum-exp
 // stage 2: one workgroup per token merges NCH*k candidates (same ordering) and the partial sums.
 #define TOPK_NCH 32
-// What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One wave to a
-// slice: the least of eight lane groups' bests is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  Four: a round for each of the k, two wave reductions and one rescan of the lane
-// that lost its best.  (Rounds for one wave as well, two kernels together: 13.0 us for one row of 32000, 44 for 512, 142 for 2048, now 12.3, 33 and 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
+// What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One way
+// to go on is a round for each of the k, two wave reductions and one rescan of the lane that lost its best.  The other, for one wave to a slice and many rounds (the rule is at the launch): the least of eight lane groups' bests
+// is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
 // (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
 // One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
@@ -705,7 +705,7 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
     key = m; id = i;
 }
 template <int VPT, int WS>
-__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
+__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int candidates, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
     constexpr int MET = WS > 1 ? 32 : 256;                              // the four waves' bests; a wave's own candidates
@@ -724,7 +724,7 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     if (pi_abort_late(gone, abort_w)) return;
     uint32_t wk = bk; int wi = bk ? own0 + STEP * bm : 0x7fffffff;
     uint32_t top = bk, low = 0;                                         // low: at least eight values are not below it — the least of the bests of eight lanes each (lanes of the same number mod 8)
-    if constexpr (WS == 1) {
+    if (WS == 1 && candidates) {
         top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<8>((int) top));
         low = top;
         pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); low = min(low, (uint32_t) pi_partner<O>((int) low)); });
@@ -749,9 +749,9 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
     } else { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; }
     const int64_t out = ((int64_t) t * TOPK_NCH + ch) * k;
-    if constexpr (WS == 1) {
+    if constexpr (WS == 1) if (candidates) {
         // what is not below `low` goes to a lane each, which counts those ahead of it
-        const uint32_t least = max(k == 1 ? top : low, 1u);
+        const uint32_t least = max(low, 1u);
         uint64_t who[VPT]; int n = 0;
 #pragma unroll
         for (int m = 0; m < VPT; m++) { who[m] = __ballot(key[m] >= least); n += __popcll(who[m]); }
@@ -852,7 +852,11 @@ extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, i
     int32_t * cid = (int32_t *) scratch; float * cval = (float *) (cid + (size_t) n_tok * TOPK_NCH * k);
     float * cmax = cval + (size_t) n_tok * TOPK_NCH * k, * csum = cmax + (size_t) n_tok * TOPK_NCH;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
-#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, cid, cval, cmax, csum, pi_abort_word())
+    // One wave to a slice: candidates cost the same for every k, rounds some 0.8 us each of them, and 1 / 3 us less at the start of 64 / 256 rows.  us by rounds / candidates, vocabulary 32000: 512 rows k = 1 20.1 / 28.7,
+    // 4 30.6 / 30.2, 5 34.3 / 30.8, 8 44.5 / 32.5; 256 rows k = 5 21.0 / 20.6; 128 rows k = 6 15.0 / 15.0, 7 16.3 / 15.5; 64 rows k = 7 12.6 / 13.2; k = 8 of one row 12.7 / 11.4, 6 rows 13.4 / 13.1, 16 11.7 / 12.7,
+    // 32 11.9 / 12.8, 48 13.5 / 13.6; of 65536 8 rows 15.6 / 14.7, 16 14.8 / 15.0
+    const int candidates = n_tok >= 256 ? k >= 5 : n_tok >= 128 ? k >= 7 : k == 8 && (n_tok <= (per > 1024 ? 12 : 7) || n_tok > 32);
+#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, candidates, cid, cval, cmax, csum, pi_abort_word())
     if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4);
     else if (per <= 64 * 8) TOPK_GO(8, 1); else if (per <= 64 * 16) TOPK_GO(16, 1); else if (per <= 64 * 32) TOPK_GO(32, 1);
     else if (per <= 256 * 16) TOPK_GO(16, 4); else if (per <= 256 * 32) TOPK_GO(32, 4); else TOPK_GO(0, 4);

@@ -554,6 +554,27 @@ def test_top_of_a_row_and_more(gpu, n_vocab, n_tok):
     assert res[8][0][0, 0] == int(np.argmax(x[0]))
 
 
+@pytest.mark.parametrize("n_vocab", [1000, 32768, 32769])
+def test_topk_rounds_and_candidates(gpu, n_vocab):
+    """both sides of every line between the two ways to pick the k best: the same order (ties go to the lower id, what is no number comes last) and the same bits of the sum whichever way a pass goes"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    x = np.round(np.random.default_rng(n_vocab).standard_normal((256, n_vocab)) * 40).astype(np.float32)
+    x[3], x[5], x[6, 4:] = np.nan, 2.0, np.nan                       # (6: fewer numbers than k)
+    order = np.lexsort((np.broadcast_to(np.arange(n_vocab), x.shape), -np.nan_to_num(x, nan=-np.inf)), axis=1)[:, :8].astype(np.int32)
+    want = np.where(np.isnan(np.take_along_axis(x, order, 1)), 0x7fffffff, order)
+    ld, sums = U.Dev(x), None
+    for n_tok, k in ((7, 8), (8, 8), (12, 8), (13, 8), (32, 8), (33, 8), (127, 7), (127, 8), (128, 6), (128, 7), (255, 6), (256, 4), (256, 5)):
+        ids, vals, se, scr = U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(n_tok))
+        L.check(lib.pi_op_topk(ld.ptr, n_vocab, n_tok, k, ids.ptr, vals.ptr, se.ptr, scr.ptr, None))
+        assert np.array_equal(ids.get(np.int32, (n_tok, k)), want[:n_tok, :k]), (n_tok, k)
+        top = np.take_along_axis(x, order, 1)[:n_tok, :k]
+        assert np.array_equal(vals.get(np.float32, (n_tok, k)), np.where(np.isnan(top), -np.inf, top)), (n_tok, k)
+        got = se.get(np.uint32)
+        sums = got if sums is None else sums
+        assert np.array_equal(got[:7], sums[:7]), (n_tok, k)
+
+
 @pytest.mark.parametrize("n_vocab", [512, 32000, 65024])
 def test_topk(gpu, n_vocab):
     lib, U = gpu
