@@ -12,8 +12,8 @@
 // A lane of a wave (row r, c) needs lanes k = c and c + 4 of its row: 16 contiguous bytes of a group of four blocks, which go from memory to its registers and are converted there, once for the TT token tiles that the wave
 // owns.  The tokens' operands are converted once per workgroup, into LDS; a group has one barrier, loads are a group ahead, LDS reads a block (a single tile: two).  Few tokens: two waves share a row tile's lanes k, so that a
 // block's serial chain is half as long.  Matrices that share their activations (q, k, v; up and gate) are one launch: its rounds fill better.
-// Measured (Q4_0, us for 4096 x 4096 / 11008 x 4096, before / now): 16 tokens 34 / 25, 35 / 34; 32: 41 / 25, 44 / 36; 64: 60 / 34, 64 / 51; 128: 62 / 40, 110 / 89; 333: 114 / 75, 266 / 207; 512: 123 / 96 (179 TFLOP/s),
-// 327 / 269; Q8_0 4096 x 4096 16 tokens 31 / 27, 333: 112 / 81.  In a full round of 128 rows x 64 tokens the VALU issues in 86 % of the cycles.
+// Measured (Q4_0, us for 4096 x 4096 / 11008 x 4096, before / now): 16 tokens 34 / 25, 35 / 30; 32: 41 / 25, 44 / 36; 64: 60 / 34, 64 / 51; 128: 62 / 40, 110 / 89; 333: 114 / 75, 266 / 207; 512: 123 / 96 (179 TFLOP/s),
+// 327 / 269; Q8_0 4096 x 4096 16 tokens 31 / 27, 333: 112 / 81, 11008 x 4096 16 tokens 33 / 31, 32: 41 / 36.  In a full round of 128 rows x 64 tokens the VALU issues in 86 % of the cycles.
 #include "mmvq_args.h"
 #include <hip/hip_ext.h>
 
@@ -211,7 +211,7 @@ template <int TYPE, int WR, int TT, int KS>
 static int launch_q0(mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     mmvq_args & g = L.g;
     constexpr int NTHR = 64 * WR * KS, U = (TT * 256 + NTHR - 1) / NTHR, UB = U == 3 ? 4 : U;
-    constexpr size_t lds = 3 * (size_t) (NTHR * UB * 16 + NTHR * 4);
+    constexpr size_t image = 3 * (size_t) (NTHR * UB * 16 + NTHR * 4), fold = KS == 2 ? (size_t) WR * TT * 4096 : 0, lds = image > fold ? image : fold;
     if (!g.aq) { PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_mmq_q0<TYPE, WR, TT, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); return 0; }      // pi_mmq_q0_reserve
     int rb = 0;
     for (int i = 0; i < MMVQ_MAX_SEG; i++) {
@@ -229,21 +229,29 @@ template <int TYPE>
 static int launch_q0_cfg(int cfg, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     switch (cfg) {
         case 212: return launch_q0<TYPE, 2, 1, 2>(L, stream, ea, eb);
+        case 412: return launch_q0<TYPE, 4, 1, 2>(L, stream, ea, eb);
+        case 422: if constexpr (TYPE == PI_Q8_0) return launch_q0<TYPE, 4, 2, 2>(L, stream, ea, eb); else break;      // (Q4_0: 128 x 16 takes as long: 36.1 and 36.6 for 11008 x 4096 at 32 tokens)
         case 81: return launch_q0<TYPE, 8, 1, 1>(L, stream, ea, eb);
         case 83: return launch_q0<TYPE, 8, 3, 1>(L, stream, ea, eb);
         case 84: return launch_q0<TYPE, 8, 4, 1>(L, stream, ea, eb);
-        default: return launch_q0<TYPE, 8, 2, 1>(L, stream, ea, eb);
+        case 82: return launch_q0<TYPE, 8, 2, 1>(L, stream, ea, eb);
     }
+    pi_set_error("mmq_q0: configuration %d", cfg);
+    return -1;
 }
 // Which tiles: the shortest estimate of  rounds of workgroups x time of a round, as in mmq_prompt.hip.  A round's time (us for 128 blocks, launch taken off, 4096 columns): rows x tokens of a workgroup 32 x 16 (two of them
-// fit a CU; few tokens: a block is the shortest serial chain), 128 x 16, x 32, x 48, x 64 (the wider, the fewer instructions per tile)
+// fit a CU; few tokens: a block is the shortest serial chain), 64 x 16 and x 32 (the same chain, and one round where the smallest tile needs more than one to a CU), 128 x 16, x 32, x 48, x 64 (the wider, the fewer
+// instructions per tile).  The 64-row tiles against the others' best, us: Q8_0 11008 x 4096 at 9 / 16 / 24 / 32 tokens 29.4 / 31.2 / 36 / 36 and 35.7 / 36.3 / 46 / 48, 6144 x 4096 at 64 36.4 and 46.1; Q4_0 11008 x 4096 at
+// 16 30.1 and 33.5, 4096 x 4096 at 48 30.4 and 33.5.  (Where they do not help, Q8_0 22016 and 32000 x 4096 at 16 tokens take 50.7 and 55; the kernel that
+// converted its weights once per workgroup, in LDS, took 47.8 and 51: there a wave's conversions serve one tile of tokens.)
 static int q0_choose(int type, const mmvq_launch & L) {
-    static const struct { int cfg, wr, tt, per_cu; float one, full; } cfgs[2][5] = {
-        { { 212, 2, 1, 2, 20.0f, 30.0f }, { 81, 8, 1, 1, 32.0f, 32.0f }, { 82, 8, 2, 1, 47.0f, 47.0f }, { 83, 8, 3, 1, 69.0f, 69.0f }, { 84, 8, 4, 1, 89.0f, 89.0f } },      // Q4_0
-        { { 212, 2, 1, 2, 23.0f, 30.5f }, { 81, 8, 1, 1, 41.0f, 41.0f }, { 82, 8, 2, 1, 54.0f, 54.0f }, { 83, 8, 3, 1, 74.0f, 74.0f }, { 84, 8, 4, 1, 95.0f, 95.0f } },      // Q8_0
-    };
+    struct tiles { int cfg, wr, tt, per_cu; float one, full; };
+    static const tiles q4[] = { { 212, 2, 1, 2, 20.0f, 30.0f }, { 412, 4, 1, 1, 25.0f, 25.0f }, { 81, 8, 1, 1, 32.0f, 32.0f }, { 82, 8, 2, 1, 47.0f, 47.0f }, { 83, 8, 3, 1, 69.0f, 69.0f }, { 84, 8, 4, 1, 89.0f, 89.0f } };
+    static const tiles q8[] = { { 212, 2, 1, 2, 23.0f, 30.5f }, { 412, 4, 1, 1, 27.0f, 27.0f }, { 422, 4, 2, 1, 33.0f, 33.0f }, { 81, 8, 1, 1, 41.0f, 41.0f }, { 82, 8, 2, 1, 54.0f, 54.0f }, { 83, 8, 3, 1, 74.0f, 74.0f }, { 84, 8, 4, 1, 95.0f, 95.0f } };
+    const tiles * cfgs = type == PI_Q8_0 ? q8 : q4; const int n_cfgs = type == PI_Q8_0 ? 7 : 6;
     int best = 83; float best_t = 1e30f;
-    for (const auto & c : cfgs[type == PI_Q8_0]) {
+    for (int n = 0; n < n_cfgs; n++) {
+        const tiles & c = cfgs[n];
         int64_t rb = 0;
         for (int i = 0; i < L.nseg; i++) rb += (L.g.seg[i].M + c.wr * 16 - 1) / (c.wr * 16);
         const int64_t wgs = rb * ((L.g.nt + c.tt * 16 - 1) / (c.tt * 16)), slots = (int64_t) pi_cu_count() * c.per_cu, whole = wgs / slots, rest = wgs % slots;
@@ -256,8 +264,8 @@ static int q0_choose(int type, const mmvq_launch & L) {
 // once per process and outside any stream capture (pi_op_mul_mat_reserve): the instances' dynamic LDS is more than a kernel gets by default
 int pi_mmq_q0_reserve() {
     mmvq_launch L; memset(&L.g, 0, sizeof L.g);                        // g.aq == nullptr: the instances only set their attribute
-    for (int cfg : { 212, 81, 82, 83, 84 })
-        if (launch_q0_cfg<PI_Q4_0>(cfg, L, nullptr, nullptr, nullptr) != 0 || launch_q0_cfg<PI_Q8_0>(cfg, L, nullptr, nullptr, nullptr) != 0) return -1;
+    for (int cfg : { 212, 412, 422, 81, 82, 83, 84 })
+        if ((cfg != 422 && launch_q0_cfg<PI_Q4_0>(cfg, L, nullptr, nullptr, nullptr) != 0) || launch_q0_cfg<PI_Q8_0>(cfg, L, nullptr, nullptr, nullptr) != 0) return -1;
     return 0;
 }
 // the whole pass in one launch (up to three matrices of one type; g.aq / g.ad at the first token, g.nt tokens)

@@ -162,9 +162,11 @@ def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
 
 
 @pytest.mark.parametrize("t", [O.Q4_0, O.Q8_0])
-@pytest.mark.parametrize("k,rows,n_tok", [(128, (33, 1, 31), 16), (160, (4090,), 121), (256, (4095, 1), 250), (160, (2000, 2081), 333), (32, (4001,), 385), (288, (1, 130, 96), 17), (384, (128, 128, 128), 1000)])
+@pytest.mark.parametrize("k,rows,n_tok", [(128, (33, 1, 31), 16), (160, (4090,), 121), (256, (4095, 1), 250), (160, (2000, 2081), 333), (32, (4001,), 385), (288, (1, 130, 96), 17), (384, (128, 128, 128), 1000),
+                                            (288, (9001,), 12), (160, (4001,), 47), (160, (6001,), 50), (256, (8990, 17), 32), (256, (4090,), 220), (160, (8200, 2700), 40), (32, (2030, 2050), 200), (288, (2000, 2081), 100), (32, (5500, 5500), 100)])
 def test_mul_mat_32_blocks_prompt_tiles(gpu, t, k, rows, n_tok):
-    """k_mmq_q0 in every tile shape its rule chooses, one to three matrices in a launch (one may end inside a workgroup's rows): the reference's bits"""
+    """k_mmq_q0 in every tile shape its rule chooses for either type on 256 compute units (rows x tokens 32 x 16, 64 x 16, Q8_0 64 x 32, 128 x 16 .. 64), one to three matrices in a launch (one may end inside a
+    workgroup's rows), with and without a residual: the reference's bits"""
     lib, U = gpu
     from pipeinfer_amd import lib as L
     rng = np.random.default_rng(k + sum(rows) + n_tok)
@@ -175,9 +177,14 @@ def test_mul_mat_32_blocks_prompt_tiles(gpu, t, k, rows, n_tok):
     L.check(lib.pi_op_quantize(O.Q8_0, xd.ptr, k, n_tok, q8.ptr, None))
     outs = [U.Dev(nbytes=4 * n_tok * m) for m in rows]
     L.check(lib.pi_op_mul_mat_multi(len(ws), (C.c_void_p * len(ws))(*ws), q8.ptr, n_tok, (C.c_void_p * len(ws))(*[o.ptr for o in outs]), None, None))
-    for m, b, dv in zip(rows, blocks, outs):
-        want = O.Impl("oracle").mul_mat(t, b, k, m, act)
+    wants = [O.Impl("oracle").mul_mat(t, b, k, m, act) for m, b in zip(rows, blocks)]
+    for m, want, dv in zip(rows, wants, outs):
         assert np.array_equal(dv.get(np.uint32, (n_tok, m)), want.view(np.uint32))
+    res = [rng.standard_normal((n_tok, m)).astype(np.float32) for m in rows]
+    rd = [U.Dev(r) for r in res]
+    L.check(lib.pi_op_mul_mat_multi(len(ws), (C.c_void_p * len(ws))(*ws), q8.ptr, n_tok, (C.c_void_p * len(ws))(*[o.ptr for o in outs]), (C.c_void_p * len(ws))(*[r.ptr for r in rd]), None))
+    for m, want, r, dv in zip(rows, wants, res, outs):
+        assert np.array_equal(dv.get(np.uint32, (n_tok, m)), (r + want).view(np.uint32))
     for w in ws:
         lib.pi_weight_free(w)
 
