@@ -75,26 +75,27 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
     for (int i = 0; i < TT; i++) acc[i] = 0.0f;
     const uint16_t * w = W + row * K;
     if constexpr (TT == 1 && VW == 8) {
-        // one token: two steps of 512 values go out together (a step at a time 32000 x 1024 / 2048 took 15.1 / 25.8 us, now 13.4 / 23.5).  Rows of 8 KB and more keep single steps: 32000 x 4096 48.7, in pairs 50.1;
-        // 5120 x 13824 27.5, in pairs 31.6
-        const float * x0 = X + (int64_t) t0 * xs + lane * 8;
-        const uint16_t * w0 = w + lane * 8;
-        auto steps = [&](auto n_steps, int64_t k) __attribute__((always_inline)) {
-            constexpr int U = decltype(n_steps)::value;
-            dn_u16x8 wv[U]; float4 xv[U][2];
+        // one token: of rows below 8 KB two steps of 512 values go out together (a step at a time 32000 x 1024 / 2048 took 15.1 / 25.8 us, now 13.4 / 23.5).  Longer rows keep single steps, which the compiler may run into
+        // each other (4096 x 4096 9.1, with a step's loads held together 9.5; 32000 x 4096 48.9, in pairs 50.1; 5120 x 13824 27.1, in pairs 31.6)
+        const float * x0 = X + (int64_t) t0 * xs;
+        auto product = [&](const dn_u16x8 & v, const float4 & lo, const float4 & hi) __attribute__((always_inline)) {
+            const float xf[8] = { lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w };
 #pragma unroll
-            for (int u = 0; u < U; u++) { xv[u][0] = *(const float4 *) (x0 + k + 512 * u); xv[u][1] = *(const float4 *) (x0 + k + 512 * u + 4); wv[u] = *(const dn_u16x8 *) (w0 + k + 512 * u); }
+            for (int i = 0; i < 8; i++) acc[0] = fmaf(dn_widen(v[i]), EXACT ? xf[i] : dn_round(xf[i]), acc[0]);
+        };
+        int64_t k = lane * 8;
+        if (K < 4096) for (; k - lane * 8 + 1024 <= K && (k < 512 || !(gone & 1)); k += 1024) {
+            dn_u16x8 wv[2]; float4 xv[2][2];
+#pragma unroll
+            for (int u = 0; u < 2; u++) { xv[u][0] = *(const float4 *) (x0 + k + 512 * u); xv[u][1] = *(const float4 *) (x0 + k + 512 * u + 4); wv[u] = *(const dn_u16x8 *) (w + k + 512 * u); }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const float xf[8] = { xv[u][0].x, xv[u][0].y, xv[u][0].z, xv[u][0].w, xv[u][1].x, xv[u][1].y, xv[u][1].z, xv[u][1].w };
-#pragma unroll
-                for (int i = 0; i < 8; i++) acc[0] = fmaf(dn_widen(wv[u][i]), EXACT ? xf[i] : dn_round(xf[i]), acc[0]);
-            }
-        };
-        int64_t k = 0;
-        if (K < 4096) for (; k + 1024 <= K && (k == 0 || !(gone & 1)); k += 1024) steps(std::integral_constant<int, 2>{}, k);
-        for (; k < K && (k == 0 || !(gone & 1)); k += 512) if (k + lane * 8 < K) steps(std::integral_constant<int, 1>{}, k);
+            for (int u = 0; u < 2; u++) product(wv[u], xv[u][0], xv[u][1]);
+        }
+        for (; k < K && (k < 512 || !(gone & 1)); k += 512) {
+            const float4 lo = *(const float4 *) (x0 + k), hi = *(const float4 *) (x0 + k + 4);
+            product(*(const dn_u16x8 *) (w + k), lo, hi);
+        }
     } else {
         if (pi_abort_late(gone, abort_w, 0)) return;
         for (int64_t k = (int64_t) lane * VW; k < K; k += 64 * VW) {
@@ -208,12 +209,18 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
         dt_u32x4 af[NS][RT][2]; dt_f32x4 xf[NS][TT][NX];
 #pragma unroll
         for (int u = 0; u < NS; u++) {
+            auto load_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int b = 0; b < TT; b++)
+                for (int b = 0; b < TT; b++)
 #pragma unroll
-                for (int i = 0; i < NX; i++) xf[u][b][i] = (i < 2 ? okx : ok1) ? *(const dt_f32x4 *) (xrow[b] + k + 64 * u + (i < 2 ? 0 : 24) + 4 * i) : zerof;
+                    for (int i = 0; i < NX; i++) xf[u][b][i] = (i < 2 ? okx : ok1) ? *(const dt_f32x4 *) (xrow[b] + k + 64 * u + (i < 2 ? 0 : 24) + 4 * i) : zerof;
+            };
+            // (16 rows and 32 tokens, where the activations are most of it: the weights first.  4096 x 11008 at 17 / 32 tokens 36.1 / 50.2 us, the other way round 39.0 / 53.5; 32 rows 8192 x 4096 at 24 22.6 and 22.1)
+            constexpr bool W_FIRST = RT == 1 && TT == 2;
+            if constexpr (!W_FIRST) load_x();
 #pragma unroll
             for (int a = 0; a < RT; a++) { af[u][a][0] = ok0 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u) : zero4; af[u][a][1] = ok1 ? *(const dt_u32x4 *) (wrow[a] + k + 64 * u + 32) : zero4; }
+            if constexpr (W_FIRST) load_x();
         }
         __builtin_amdgcn_sched_barrier(0);                             // (all of them issued before the first product waits)
 #pragma unroll
