@@ -730,49 +730,41 @@ extern "C" int pi_op_attention_reserve(int hd, int n_kv_max) {
     return rc;
 }
 
-template <int HD>
-static void att_launch(const att_args & g, int rows, int rw, hipStream_t stream) {
+// cells that a launch is priced with: the pass's own where the engine launches eagerly, else what it is launched with.  (A captured graph is launched with n_kv = n_ctx and reads the real n_kv from device memory: its
+// count carries the upper bound, bench.py prices attention from the call statistics instead.)
+static int att_priced(const att_args & g) { return pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv; }
+// algorithmic bytes: K and V of n_kv cells (f16) + the query rows + the fp32 output
+static double att_bytes(const att_args & g, int hd) { return (double) att_priced(g) * g.n_head_kv * hd * 2 * 2 + (double) g.n_tok * g.n_head * hd * (2 + 4); }
+// where k_attention stands behind k_attention_tiles, the one that does the pass of the priced cells is counted and timed
+#define ATT_GO(COUNTED, GRID, BLOCK, LDS, KERNEL, ...) do { \
+        if (COUNTED) PI_KT_LAUNCH(PI_KT_ATT, 0, g.n_tok, att_bytes(g, HD), KERNEL, GRID, BLOCK, LDS, stream, __VA_ARGS__); \
+        else hipLaunchKernelGGL(KERNEL, GRID, BLOCK, LDS, stream, __VA_ARGS__); \
+    } while (0)
+template <int HD, bool ALIBI, bool BEHIND>
+static void att_launch_rows(const att_args & g, int rows, int rw, hipStream_t stream) {
     const dim3 grid(g.n_head_kv, (rows + rw - 1) / rw);
     const size_t lds = (size_t) rw * (g.n_kv + g.mask_words) * sizeof(float);
-    // algorithmic bytes: K and V of n_kv cells (f16) + the query rows + the fp32 output.  (A captured graph is launched with n_kv = n_ctx and reads the real
-    // n_kv from device memory: its count carries the upper bound, bench.py prices attention from the call statistics instead.)
-    const int nt = g.n_tok > 0 ? g.n_tok : 1;
-    const int n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv;      // (eager launches of the engine: the pass's own n_kv)
-    const double bytes = (double) n_kv_priced * g.n_head_kv * HD * 2 * 2 + (double) nt * g.n_head * HD * (2 + 4);
-    if (g.tile_cells > 0) {                                  // behind k_attention_tiles (without ALiBi): not counted, one of the two does the work
-        switch (rw) {
-            case 1: hipLaunchKernelGGL((k_attention<HD, 1, false, true>), grid, dim3(256), lds, stream, g); break;
-            case 2: hipLaunchKernelGGL((k_attention<HD, 2, false, true>), grid, dim3(256), lds, stream, g); break;
-            case 4: hipLaunchKernelGGL((k_attention<HD, 4, false, true>), grid, dim3(256), lds, stream, g); break;
-            default: hipLaunchKernelGGL((k_attention<HD, 8, false, true>), grid, dim3(256), lds, stream, g); break;
-        }
-        return;
-    }
-#define ATT_GO(...) PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (__VA_ARGS__), grid, dim3(256), lds, stream, g)
-    if (g.alibi_m) {
-        switch (rw) {
-            case 1: ATT_GO(k_attention<HD, 1, true>); break;
-            case 2: ATT_GO(k_attention<HD, 2, true>); break;
-            case 4: ATT_GO(k_attention<HD, 4, true>); break;
-            default: ATT_GO(k_attention<HD, 8, true>); break;
-        }
-        return;
-    }
+    const bool counted = !BEHIND || att_priced(g) > g.tile_cells;
     switch (rw) {
-        case 1: ATT_GO(k_attention<HD, 1>); break;
-        case 2: ATT_GO(k_attention<HD, 2>); break;
-        case 4: ATT_GO(k_attention<HD, 4>); break;
-        default: ATT_GO(k_attention<HD, 8>); break;
+        case 1: ATT_GO(counted, grid, dim3(256), lds, (k_attention<HD, 1, ALIBI, BEHIND>), g); break;
+        case 2: ATT_GO(counted, grid, dim3(256), lds, (k_attention<HD, 2, ALIBI, BEHIND>), g); break;
+        case 4: ATT_GO(counted, grid, dim3(256), lds, (k_attention<HD, 4, ALIBI, BEHIND>), g); break;
+        default: ATT_GO(counted, grid, dim3(256), lds, (k_attention<HD, 8, ALIBI, BEHIND>), g); break;
     }
 }
-#undef ATT_GO
+template <int HD>
+static void att_launch(const att_args & g, int rows, int rw, hipStream_t stream) {
+    if (g.tile_cells > 0) att_launch_rows<HD, false, true>(g, rows, rw, stream);          // (never with ALiBi)
+    else if (g.alibi_m) att_launch_rows<HD, true, false>(g, rows, rw, stream);
+    else att_launch_rows<HD, false, false>(g, rows, rw, stream);
+}
 // passes of many rows of up to ATT_TILE_CELLS cells; g.n_kv may be the bound of a captured graph
 template <int HD>
 static void att_tile_launch(const att_args & g, int rows, hipStream_t stream) {
-    const int nt = g.n_tok, cells = g.n_kv < ATT_TILE_CELLS ? g.n_kv : ATT_TILE_CELLS, n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < g.n_kv ? pi_account_n_kv() : g.n_kv;
-    const double bytes = (double) n_kv_priced * g.n_head_kv * HD * 2 * 2 + (double) nt * g.n_head * HD * (2 + 4);
-    PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention_tiles<HD>), dim3(g.n_head_kv, (rows + 15) / 16), dim3(512), att_tile_lds(HD, cells), stream, g, cells);
+    const int cells = g.n_kv < ATT_TILE_CELLS ? g.n_kv : ATT_TILE_CELLS;
+    ATT_GO(att_priced(g) <= ATT_TILE_CELLS, dim3(g.n_head_kv, (rows + 15) / 16), dim3(512), att_tile_lds(HD, cells), (k_attention_tiles<HD>), g, cells);
 }
+#undef ATT_GO
 
 extern "C" int pi_op_attention(const uint16_t * q16, const uint16_t * kc, const uint16_t * vc, const uint32_t * mask, int hd, int n_head, int n_head_kv,
                                int n_tok, int n_kv, float * out, const int32_t * dyn_dev, void * stream) {
@@ -831,11 +823,9 @@ extern "C" int pi_op_attention_alibi(const uint16_t * q16, const uint16_t * kc, 
     else if (hd > 0 && hd <= 256 && hd % 2 == 0) {                       // every other head width: the plain kernel, one workgroup per (kv head, query row)
         const size_t lds = ((size_t) n_kv + g.mask_words + (size_t) hd) * sizeof(float);
         if (lds > att_lds_cap(1)) { pi_set_error("pi_op_attention: n_kv=%d needs more than 146 KiB of LDS", n_kv); return -1; }
-        const int nt = n_tok > 0 ? n_tok : 1;
-        const int n_kv_priced = pi_account_n_kv() > 0 && pi_account_n_kv() < n_kv ? pi_account_n_kv() : n_kv;
-        const double bytes = (double) n_kv_priced * n_head_kv * hd * 2 * 2 + (double) nt * n_head * hd * (2 + 4);
-        if (alibi_slopes_dev) PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention_any<true>), dim3(n_head_kv, rows), dim3(256), lds, (hipStream_t) stream, g, hd);
-        else                  PI_KT_LAUNCH(PI_KT_ATT, 0, nt, bytes, (k_attention_any<false>), dim3(n_head_kv, rows), dim3(256), lds, (hipStream_t) stream, g, hd);
+        const double bytes = att_bytes(g, hd);
+        if (alibi_slopes_dev) PI_KT_LAUNCH(PI_KT_ATT, 0, n_tok, bytes, (k_attention_any<true>), dim3(n_head_kv, rows), dim3(256), lds, (hipStream_t) stream, g, hd);
+        else                  PI_KT_LAUNCH(PI_KT_ATT, 0, n_tok, bytes, (k_attention_any<false>), dim3(n_head_kv, rows), dim3(256), lds, (hipStream_t) stream, g, hd);
     }
     else { pi_set_error("pi_op_attention: head_dim %d not supported (even, <= 256)", hd); return -1; }
     PI_CHECK_LAUNCH();

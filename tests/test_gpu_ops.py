@@ -484,6 +484,29 @@ def test_attention_tiles(gpu, hd, n_head, n_head_kv, n_kv, n_tok, bound):
         assert np.array_equal(np.where(np.isnan(a), 0, a).view(np.uint32), np.where(np.isnan(b), 0, b).view(np.uint32)), name
 
 
+def test_attention_accounting_behind_a_bound(gpu):
+    """a pass of many rows behind a bound of more cells than k_attention_tiles takes goes out as two launches, one of which returns at once: it is counted once, with the pass's own cells, and what is timed is the
+    launch that does the work (10 billion products and sums of 2400 cells: 64 us at the 157 TFLOP/s of fp32 that the chip has at most; an empty launch is a few us), whichever that is"""
+    lib, U = gpu
+    import bench as B
+    from pipeinfer_amd import lib as L
+    hd, n_head, n_head_kv, n_tok, bound, words = 128, 64, 8, 128, 4096, 128
+    zeros = U.Dev(nbytes=2 * bound * n_head_kv * hd)
+    q, out, mask = U.Dev(nbytes=2 * n_tok * n_head * hd), U.Dev(nbytes=4 * n_tok * n_head * hd), U.Dev(np.full((n_tok, words), 0xffffffff, np.uint32))
+    L.check(lib.pi_op_attention_reserve(hd, bound))
+    for n_kv in (2400, 2241, 2240, 500):
+        dyn = U.Dev(np.array([0, n_kv, n_tok, 0], np.int32))
+        lib.pi_set_account_n_kv(n_kv)
+        lib.pi_kernel_timing(1, 1)                                   # every launch is timed
+        L.check(lib.pi_op_attention(q.ptr, zeros.ptr, zeros.ptr, mask.ptr, hd, n_head, n_head_kv, n_tok, bound, out.ptr, dyn.ptr, None))
+        lib.pi_device_sync()
+        rows = [r for r in B.timing_rows(lib) if r["family"] == 5]
+        lib.pi_kernel_timing(0, 8)
+        lib.pi_set_account_n_kv(0)
+        assert len(rows) == 1 and rows[0]["launches"] == 1 and rows[0]["sampled"] == 1, rows
+        assert rows[0]["avg_us"] > 4.0 * n_tok * n_head * n_kv * hd / 157e6, (n_kv, rows)
+
+
 def test_elementwise_exact(gpu):
     lib, U = gpu
     from pipeinfer_amd import lib as L
