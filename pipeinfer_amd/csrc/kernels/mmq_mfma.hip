@@ -887,20 +887,18 @@ static void mmq_go2(const mmvq_args & g, int groups, hipStream_t stream, hipEven
     if (ea) hipExtLaunchKernelGGL((k_mmq_kq<TYPE, S, R, TB, NT8, NC, PIPE>), dim3(grid), dim3(64 * S * R), lds, stream, ea, eb, 0, g, groups);
     else    hipLaunchKernelGGL((k_mmq_kq<TYPE, S, R, TB, NT8, NC, PIPE>), dim3(grid), dim3(64 * S * R), lds, stream, g, groups);
 }
-// batches of <= 8 tokens stage half the fragment bytes and take twice the blocks per tile (TB8) in the same LDS; 17..32 tokens over few row groups (one four-wave row group per workgroup) are two chunks over one
-// weight stream, one block per tile — everything else of more than 16 tokens is mmq_prompt.hip's
+// batches of <= 8 tokens stage half the fragment bytes and take twice the blocks per tile (TB8) in the same LDS
 template <int TYPE, int S, int R, int TB16, int TB8>
 static void mmq_go(const mmvq_args & g, int groups, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     if (g.nt <= 8) mmq_go2<TYPE, S, R, TB8, true>(g, groups, stream, ea, eb);
-    else if (g.nt <= 16) mmq_go2<TYPE, S, R, TB16, false>(g, groups, stream, ea, eb);
-    else if constexpr (S == 4 && R == 1) mmq_go2<TYPE, S, R, 1, false, 2>(g, groups, stream, ea, eb);
-    else if (g.frag) pi_set_error("mmq: a launch of %d tokens reached configuration %d%d", g.nt, S, R);      // not reached: mmq_dispatch_t sends launches of 17..32 tokens to 41; an error, never half a result
+    else mmq_go2<TYPE, S, R, TB16, false>(g, groups, stream, ea, eb);
 }
 
 template <int TYPE>
 static void mmq_dispatch_t(const mmvq_args & g, int groups, int cfg, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     constexpr int T8 = TYPE == PI_Q4_K ? 4 : 2;                 // blocks per tile at <= 8 tokens (Q5_K: the ring carries the fifth bits too)
-    if (g.nt > 16) cfg = 41;
+    // 17..32 tokens over few row groups: two chunks over one weight stream, one block per tile, one four-wave row group per workgroup (everything else of more than 16 tokens is mmq_prompt.hip's)
+    if (g.nt > 16) { mmq_go2<TYPE, 4, 1, 1, false, 2>(g, groups, stream, ea, eb); return; }
     switch (cfg) {                                             // (S waves per row group)(R row groups per workgroup); blocks per tile for 16 / <= 8 tokens
         case 17: mmq_go<TYPE, 1, 7, 2, T8>(g, groups, stream, ea, eb); break;
         case 18: mmq_go<TYPE, 1, 8, 2, T8>(g, groups, stream, ea, eb); break;
@@ -1019,7 +1017,10 @@ extern "C" int pi_op_mul_mat_reserve(void) {
     static bool done = false;
     if (done) return 0;
     mmvq_args g; memset(&g, 0, sizeof g);                      // g.frag == nullptr: the instances only set their attribute
-    for (int type : { PI_Q3_K, PI_Q4_K, PI_Q5_K, PI_Q6_K }) for (int cfg : mmq_cfgs) for (int nt : { 8, 16, 32 }) { g.nt = nt; mmq_dispatch(type, g, 0, cfg, nullptr, nullptr, nullptr); }
+    for (int type : { PI_Q3_K, PI_Q4_K, PI_Q5_K, PI_Q6_K }) {
+        for (int cfg : mmq_cfgs) for (int nt : { 8, 16 }) { g.nt = nt; mmq_dispatch(type, g, 0, cfg, nullptr, nullptr, nullptr); }
+        g.nt = 32; mmq_dispatch(type, g, 0, 41, nullptr, nullptr, nullptr);
+    }
     for (int type_b : { PI_Q5_K, PI_Q6_K }) for (int r : { 1, 2, 3 }) for (int rb : { 1, r }) mmq_2t_dispatch(type_b, r, rb, g, 0, 0, nullptr, nullptr, nullptr);
     if (pi_mmq_q0_reserve() != 0 || pi_mmq_prompt_reserve() != 0) return -1;
     done = true;
@@ -1036,6 +1037,7 @@ int pi_mmq_launch(int type, mmvq_launch & L, hipStream_t stream, hipEvent_t ea, 
         else { g.seg[i] = g.seg[0]; g.seg[i].wave0 = 0x7fffffff; }
     }
     if (!pi_mmq_supported(type)) { pi_set_error("pi_mmq_launch: weight type %d has no MFMA kernel", type); return -1; }
+    if (g.nt > 32) { pi_set_error("pi_mmq_launch: %d tokens, a launch walks two chunks of 16 at most", g.nt); return -1; }
     static const int dbg_env = getenv("PI_MMQ_DBG") ? atoi(getenv("PI_MMQ_DBG")) : 0;
     g.dbg = dbg_env;
     // (waves per row group, row groups per workgroup).  One wave per row group needs the fewest instructions per weight byte (the block scalars
