@@ -147,8 +147,8 @@ def test_mul_mat_vs_oracle(gpu, t, k, rows, n_tok):
 @pytest.mark.parametrize("t", [O.Q4_0, O.Q8_0])
 @pytest.mark.parametrize("k,rows,n_tok", [(32, 1, 9), (96, 17, 16), (128, 64, 10), (160, 65, 17), (4544, 130, 32), (256, 63, 33), (4096, 129, 64), (1056, 68, 65), (2048, 1030, 130), (11008, 66, 47)])
 def test_mul_mat_32_blocks_prompt(gpu, t, k, rows, n_tok):
-    """k_mmq_q0 (prompts of the 32-value block types on the matrix cores), one instance per 16 / 32 / more tokens: last groups of less than four blocks, rows and tokens that end inside a tile, row
-    counts that are no multiple of four (scalar stores) — the reference's bits, with and without a residual"""
+    """k_mmq_q0 (prompts of the 32-value block types on the matrix cores) over few rows, which is its smallest tiles: last groups of less than four blocks, rows and tokens that end inside a tile - the reference's bits,
+    with and without a residual.  (Every tile: test_mul_mat_32_blocks_prompt_tiles)"""
     lib, U = gpu
     rng = np.random.default_rng(k + rows + n_tok)
     blocks = synth.random_blocks(t, rows * k, rng, 0.05).reshape(rows, -1)
@@ -190,9 +190,9 @@ def test_mul_mat_32_blocks_prompt_tiles(gpu, t, k, rows, n_tok):
 
 
 @pytest.mark.parametrize("t", [O.Q3_K, O.Q4_K, O.Q5_K, O.Q6_K])
-@pytest.mark.parametrize("k,rows,n_tok", [(256, 1, 33), (512, 40, 47), (768, 16, 65), (256, 8200, 100), (512, 8190, 90), (512, 8176, 60), (768, 8193, 64), (256, 8222, 128), (512, 8192, 121), (768, 24600, 17), (512, 24577, 32), (256, 16400, 34)])
+@pytest.mark.parametrize("k,rows,n_tok", [(256, 1, 33), (512, 40, 47), (768, 16, 65), (256, 8200, 100), (512, 8190, 90), (512, 8176, 60), (768, 8193, 64), (256, 8222, 128), (512, 8192, 121), (768, 24600, 17), (512, 24577, 32), (256, 16400, 34), (256, 527, 1663)])
 def test_mul_mat_k_quants_prompt(gpu, t, k, rows, n_tok):
-    """k_mmq_prompt in every tile shape its rule chooses (two to four chunks of tokens, one or two waves a row group, four and eight waves a workgroup): one block, two, an odd number; rows and tokens that end
+    """k_mmq_prompt in every tile shape its rule chooses for each type (two to four chunks of tokens, one or two waves a row group, four and eight waves a workgroup): one block, two, an odd number; rows and tokens that end
     inside a tile and inside a workgroup's row groups — the reference's bits, with and without a residual"""
     lib, U = gpu
     rng = np.random.default_rng(k + rows + n_tok)
@@ -208,7 +208,7 @@ def test_mul_mat_k_quants_prompt(gpu, t, k, rows, n_tok):
 
 @pytest.mark.parametrize("k,rows", [(4096, 40), (4096, 2048), (4096, 2049), (4064, 40)])
 def test_mul_mat_q4_0_nine_tokens(gpu, k, rows):
-    """both sides of the line between two passes of the mat-vec and one of k_mmq_q0 (at most 2048 rows of 4096 values and more): the reference's bits"""
+    """nine tokens, where the mat-vec would take a second pass over the weights (k_mmq_q0 takes them, as it does all from seven), around 2048 rows of 4096 values and a row of whole groups less one block: the reference's bits"""
     lib, U = gpu
     blocks = synth.random_blocks(O.Q4_0, rows * k, np.random.default_rng(k + rows), 0.05).reshape(rows, -1)
     act = np.stack([signal(k, s) for s in range(9)])
@@ -760,13 +760,14 @@ def test_mmq_two_row_groups_per_wave_fused_up_gate(gpu, n_tok):
 @pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q4_K), (O.Q4_K, O.Q4_K, O.Q6_K), (O.Q5_K, O.Q6_K, O.Q4_K)])
 @pytest.mark.parametrize("hd,n_head,n_head_kv,n_tok,kv_head", [(128, 8, 8, 1, 5), (64, 8, 2, 3, 0), (128, 4, 1, 8, 17), (64, 4, 4, 11, 2),
                                                                (128, 64, 8, 1, 3), (128, 64, 8, 2, 9), (128, 64, 8, 4, 1), (128, 40, 40, 1, 0),    # K = 8192 / 5120: the tile-per-wave instance with the RoPE epilogue
-                                                               (64, 4, 4, 20, 2), (128, 64, 8, 32, 1), (64, 8, 2, 27, 5)])                            # two chunks of 16 per launch of the matrix-core kernel
+                                                               (64, 4, 4, 20, 2), (128, 64, 8, 32, 1), (64, 8, 2, 27, 5),                             # two chunks of 16 per launch of the matrix-core kernel
+                                                               (64, 8, 2, 50, 5), (128, 64, 8, 47, 3), (128, 64, 8, 64, 1)])                            # k_mmq_prompt, the last one wave to a row group
 def test_qkv_rope_epilogue_equals_separate_launches(gpu, types, hd, n_head, n_head_kv, n_tok, kv_head):
     """RoPE + f16 rounding + KV-cache writes done by the projection's own waves == mat-vecs into fp32 + pi_op_rope_kv_store"""
     lib, U = gpu
     from pipeinfer_amd import lib as L
     rng = np.random.default_rng(hd + n_tok)
-    k, n_ctx = 512, 40
+    k, n_ctx = 512, max(40, kv_head + n_tok + 3)
     n_embd, n_gqa = n_head * hd, n_head_kv * hd
     ws = []
     for t, m in zip(types, (n_embd, n_gqa, n_gqa)):
@@ -853,8 +854,8 @@ def test_two_weight_types_share_one_launch(gpu, types, k, n_tok):
 
 @pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q5_K), (O.Q4_K, O.Q4_K, O.Q6_K), (O.Q4_K, O.Q6_K, O.Q6_K)])
 @pytest.mark.parametrize("k,n_tok,n_head,n_head_kv", [(2048, 3, 48, 2), (8192, 6, 48, 4), (4096, 8, 40, 8), (5120, 5, 32, 32), (8192, 4, 64, 8),
-                                                       # prompt passes: launches of 64 tokens (four chunks, register-staged activations), the last one with what is left
-                                                       (4096, 64, 48, 4), (2048, 40, 40, 8), (2048, 100, 48, 2), (1024, 130, 16, 16)])
+                                                       # prompt passes: launches of 64 tokens, the last one with what is left; with 64 / 8 heads one wave to a row group
+                                                       (4096, 64, 48, 4), (2048, 40, 40, 8), (2048, 100, 48, 2), (1024, 130, 16, 16), (512, 64, 64, 8), (768, 100, 64, 8)])
 def test_two_weight_types_share_one_matrix_core_launch(gpu, types, k, n_tok, n_head, n_head_kv):
     """The same mixture at verify widths (3..8 tokens): attn_v (Q5_K / Q6_K) rides in the q + k matrix-core launch (k_mmq_kq2t: the first workgroups walk the Q4_K row
     groups, the last ones the second type's, each with its own tile format) instead of being a launch of its own behind it.  Bits: the oracle's vec_dot per matrix
@@ -915,6 +916,34 @@ def test_two_weight_types_share_one_matrix_core_launch(gpu, types, k, n_tok, n_h
         assert np.array_equal(a, b), name
     assert res[0][1].any() and res[0][2].any()
     lib.pi_rope_table_free(table)
+    for w in ws:
+        lib.pi_weight_free(w)
+
+
+@pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q5_K), (O.Q4_K, O.Q4_K, O.Q6_K), (O.Q4_K, O.Q6_K, O.Q6_K)])
+@pytest.mark.parametrize("k,rows,n_tok,cus", [(256, (33, 7, 18), 33, 0), (768, (6200, 40, 33), 20, 0), (512, (5000, 35, 70), 64, 0), (512, (8176, 9, 33), 40, 0), (256, (8176, 9, 33), 63, 0), (256, (16000, 150, 149), 64, 255)])
+def test_two_weight_types_prompt_tiles(gpu, types, k, rows, n_tok, cus):
+    """k_mmq_prompt of two types in every tile shape that its rule chooses for a launch of up to 64 tokens (the last of an odd number of compute units only), rows that end inside a row group of either type, with and
+    without a residual: the oracle's bits"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(k + sum(rows) + n_tok)
+    act = rng.standard_normal((n_tok, k)).astype(np.float32)
+    blocks = [synth.random_blocks(t, m * k, rng, 0.05).reshape(m, -1) for t, m in zip(types, rows)]
+    ws = [upload_weight(lib, t, m, k, b) for t, m, b in zip(types, rows, blocks)]
+    wants = [O.Impl("oracle").mul_mat(t, b, k, m, act) for t, m, b in zip(types, rows, blocks)]
+    q8, outs = gpu_quantize(lib, U, O.Q8_K, act), [U.Dev(nbytes=4 * n_tok * m) for m in rows]
+    res = [rng.standard_normal((n_tok, m)).astype(np.float32) for m in rows]
+    rd = [U.Dev(r) for r in res]
+    wl, ol, rl = [(C.c_void_p * 3)(*p) for p in (ws, [o.ptr for o in outs], [r.ptr for r in rd])]
+    lib.pi_set_cu_count(cus)
+    try:
+        for ress in (None, rl):
+            L.check(lib.pi_op_mul_mat_multi(3, wl, q8.ptr, n_tok, ol, ress, None))
+            for m, want, r, dv in zip(rows, wants, res, outs):
+                assert np.array_equal(dv.get(np.uint32, (n_tok, m)), (want if ress is None else r + want).view(np.uint32))
+    finally:
+        lib.pi_set_cu_count(0)
     for w in ws:
         lib.pi_weight_free(w)
 
