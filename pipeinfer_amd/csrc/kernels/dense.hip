@@ -83,8 +83,9 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
 #pragma unroll
             for (int i = 0; i < 8; i++) acc[0] = fmaf(dn_widen(v[i]), EXACT ? xf[i] : dn_round(xf[i]), acc[0]);
         };
-        int64_t k = lane * 8;
-        if (K < 4096) for (; k - lane * 8 + 1024 <= K && (k < 512 || !(gone & 1)); k += 1024) {
+        int64_t done = 0;
+        if (K < 4096) for (; done + 1024 <= K && (done == 0 || !(gone & 1)); done += 1024) {
+            const int64_t k = done + lane * 8;
             dn_u16x8 wv[2]; float4 xv[2][2];
 #pragma unroll
             for (int u = 0; u < 2; u++) { xv[u][0] = *(const float4 *) (x0 + k + 512 * u); xv[u][1] = *(const float4 *) (x0 + k + 512 * u + 4); wv[u] = *(const dn_u16x8 *) (w + k + 512 * u); }
@@ -92,7 +93,7 @@ __global__ void __launch_bounds__(256) k_dense_rows(const uint16_t * __restrict_
 #pragma unroll
             for (int u = 0; u < 2; u++) product(wv[u], xv[u][0], xv[u][1]);
         }
-        for (; k < K && (k < 512 || !(gone & 1)); k += 512) {
+        for (int64_t k = done + lane * 8; k < K && (k < 512 || !(gone & 1)); k += 512) {
             const float4 lo = *(const float4 *) (x0 + k), hi = *(const float4 *) (x0 + k + 4);
             product(*(const dn_u16x8 *) (w + k), lo, hi);
         }
