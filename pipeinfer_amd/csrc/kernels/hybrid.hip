@@ -2005,6 +2005,7 @@ extern "C" int pi_op_moe_grouped_ok(const pi_weight * wup, const pi_weight * wdo
     (void) glu;
     static const int min_slots = getenv("PI_MOE_GROUPED_MIN") ? atoi(getenv("PI_MOE_GROUPED_MIN")) : 32;
     return !exact && n_exp > 0 && n_exp <= MOE_GROUP_MAX_EXPERTS && wup && wdown && n_tok * top >= min_slots && wup->ne0 % 8 == 0 && ff % 8 == 0 &&
+           wup->ne0 < (1 << 24) && ff < (1 << 24) &&                   // (a tile's 128 rows of weights in 32 bits, in bytes)
            ((uintptr_t) wup->p0 % 16) == 0 && ((uintptr_t) wdown->p0 % 16) == 0;
 }
 // up_dev: [n_tok * top][ff], dn_dev: [n_tok * top][width], idx_dev: pi_op_moe_grouped_index_ints ints

@@ -167,6 +167,19 @@ def upload_bf16(lib, w):
 
 
 @pytest.mark.gpu
+def test_experts_whose_tiles_outgrow_32_bit_offsets_stay_with_the_mat_vecs():
+    """127 rows of bfloat16 in a tile's 32-bit byte offsets: up to 2^24 - 8 values a row (either width of an expert), from 2^24 on pi_op_moe_experts takes the pass"""
+    U, lib = gpu()
+    small = upload_bf16(lib, np.zeros((1, 64), np.float32))
+    for k, ok in ((2 ** 24 - 8, 1), (2 ** 24, 0)):
+        w = lib.pi_weight_upload(BF16, k, 1, np.zeros(k, np.uint16).ctypes.data_as(C.c_void_p), None)
+        assert w and lib.pi_op_moe_grouped_ok(w, small, 4, 64, 0, 64, 2, 0) == ok
+        assert lib.pi_op_moe_grouped_ok(small, w, 4, k, 0, 64, 2, 0) == ok
+        lib.pi_weight_free(w)
+    lib.pi_weight_free(small)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N", [8192, 8191, 8224])
 def test_dense_two_tokens_of_rows_of_8_kb(N):
     """4096 values a row, 32 rows and fewer per workgroup: on both sides of the line between the mat-vec and the split kernel (fp32 sums of 4096 exact products: 2e-6 of their mean)"""
