@@ -1983,15 +1983,18 @@ __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ 
 
 // slots of a tile
 static int moe_tile_len(int n_slots, int n_exp) { return n_slots / n_exp >= 256 ? 128 : 64; }
-// rows of a tile: as for k_dense_tile, the largest that gives every compute unit a workgroup; where none does, two groups of waves share K
+// rows of a tile: as for k_dense_tile, the largest that gives every compute unit a workgroup; where none does, two groups of waves share K.  Of 128 slots 256 rows as soon as tiles of 128 rows would be more than a round
+// of workgroups (some more: the number of tiles is an estimate).  us for both products of top-2 of 8 experts, 128 / 256 rows: 4096 x 2048 at 1024 tokens 210 / 190, 2048 356 / 328, 4000 549 / 434; 2048 x 2048 at 1400
+// 113 / 96, 3000 227 / 200; and at less than a round 2048 x 1024 at 1400 the one of 208 workgroups + 8.7, the one of 416 - 5.7.  (128 rows by 4 x 2 waves instead of 2 x 4: 1 - 3 % more)
 template <bool UP>
 static void moe_tile_launch(const uint16_t * w, int64_t K, int rows, const float * b, int64_t bs, int top, const int32_t * idx, int mt, int tl, int est, int glu, float limit, float * out, int nta, double bytes, hipStream_t s) {
 #define MOE_GO2(BN, BT, WN, WT, KG, PAIR) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, bytes, (k_moe_tile<BN, BT, WN, WT, KG, UP, PAIR>), dim3((unsigned) ((mt * ((rows + BN - 1) / BN) + 7) / 8 * 8)), dim3(64 * WN * WT * KG), 0, s, \
                                                w, K, rows, b, bs, top, idx, mt, glu, limit, out, pi_abort_word())
 #define MOE_GO(BN, BT, KG) do { if constexpr (UP) MOE_GO2(BN, BT, 2, 2, KG, false); else if (glu) MOE_GO2(BN, BT, 2, 2, KG, true); else MOE_GO2(BN, BT, 2, 2, KG, false); } while (0)
     const int wg128 = est * ((rows + 127) / 128);
-    if (tl == 128 && !UP && glu) MOE_GO2(64, 128, 2, 4, 1, !UP);            // (two values for each of X: the registers do not hold the larger tile)
-    else if (tl == 128) MOE_GO2(128, 128, 4, 2, 1, false);
+    if constexpr (!UP) if (tl == 128 && glu) { MOE_GO2(64, 128, 2, 4, 1, true); return; }            // (two values for each of X: the registers do not hold the larger tile)
+    if (tl == 128 && wg128 > 280 && K < (1 << 23)) MOE_GO2(256, 128, 4, 2, 1, false);                 // (256 rows of weights in 32 bits, in bytes)
+    else if (tl == 128) MOE_GO2(128, 128, 2, 4, 1, false);
     else if (wg128 >= 256) MOE_GO(128, 64, 1);
     else if (wg128 >= 128) MOE_GO(128, 64, 2);
     else MOE_GO(64, 64, 2);

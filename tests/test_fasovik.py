@@ -615,10 +615,11 @@ def test_experts_of_a_cancelled_run(T, glu):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("E,I,ff,width,T,top", [(2, 1, 136, 200, 300, 2), (8, 2, 64, 3080, 200, 2), (8, 0, 72, 1544, 210, 2), (70, 3, 16, 72, 40, 6), (1, 0, 8, 8, 33, 1), (3, 0, 24, 136, 700, 2)])
+@pytest.mark.parametrize("E,I,ff,width,T,top", [(2, 1, 136, 200, 300, 2), (8, 2, 64, 3080, 200, 2), (8, 0, 72, 1544, 210, 2), (70, 3, 16, 72, 40, 6), (1, 0, 8, 8, 33, 1), (3, 0, 24, 136, 700, 2),
+                                                    (2, 0, 72, 1544, 1500, 2), (2, 0, 1480, 72, 1500, 2)])
 @pytest.mark.parametrize("glu", [0, 1])
 def test_grouped_experts_tiles(E, I, ff, width, T, top, glu):
-    """every tile of the grouped path (64 and 128 slots, 64 and 128 rows, K shared by two groups of waves), runs and rows that end inside a tile, choices that nobody made, identity experts; both products
+    """every tile of the grouped path (64 and 128 slots, 64, 128 and 256 rows, K shared by two groups of waves), runs and rows that end inside a tile, choices that nobody made, identity experts; both products
     against fp64 sums of what entered them (fp32 sums of at most 3080 terms: 3e-6 of the rows' mean)"""
     U, lib = gpu()
     rng = np.random.default_rng(E + T)
