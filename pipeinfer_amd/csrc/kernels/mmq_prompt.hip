@@ -351,24 +351,27 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
     }
 }
 
-// workgroup n runs on XCD n % 8: the token blocks of a row block go to one XCD one behind the other, so that its weights come from HBM once
-template <int TA, int TB, int S, int RG, int CH>
+// workgroup n runs on XCD n % 8: the token blocks of a row block go to one XCD one behind the other, so that its weights come from HBM once.
+// SB, RGB: waves per row group and row groups of the second type's workgroups.  They are few and come last, so the launch ends with one of them: where the first type keeps one wave to a row group the second takes two
+// (a Q6_K tile costs a wave 1.6 times a Q4_K one; 8192 + 1024 rows of Q4_K with 1024 of Q6_K, 8192 columns, 64 tokens: 57.6 us with one wave to all row groups, now 41.4; Q5_K 50 and 41.1)
+template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG>
 __global__ void __launch_bounds__(64 * S * RG) k_mmq_prompt(const mmvq_args g, const int groups_a, const int groups_all, const int blocks_a, const int row_blocks, const int tok_blocks) {
+    static_assert(S * RG == SB * RGB, "workgroups of one size");
     if (pi_aborted(g.abort_w, 1)) return;
     const int slot = blockIdx.x >> 3, rb = (blockIdx.x & 7) + 8 * (slot / tok_blocks), tb = slot % tok_blocks;
     if (rb >= row_blocks) return;
     if constexpr (TA != TB) {
-        if (rb >= blocks_a) { mmq_prompt_body<TB, S, RG, CH>(g, groups_all, groups_a + (rb - blocks_a) * RG, tb); return; }
+        if (rb >= blocks_a) { mmq_prompt_body<TB, SB, RGB, CH>(g, groups_all, groups_a + (rb - blocks_a) * RGB, tb); return; }
     }
     mmq_prompt_body<TA, S, RG, CH>(g, groups_a, rb * RG, tb);
 }
 
-template <int TA, int TB, int S, int RG, int CH>
+template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG>
 static int prompt_go(const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
-    constexpr size_t image = 3 * ((size_t) CH * 8192 + 64 * S * RG * 8), fold = S == 2 ? (size_t) S * RG * ((CH + 1) / 2) * 4 * 6 * 256 : 0, lds = image > fold ? image : fold;
-    const auto kernel = k_mmq_prompt<TA, TB, S, RG, CH>;
+    constexpr size_t image = 3 * ((size_t) CH * 8192 + 64 * S * RG * 8), fold = S == 2 || SB == 2 ? (size_t) S * RG * ((CH + 1) / 2) * 4 * 6 * 256 : 0, lds = image > fold ? image : fold;
+    const auto kernel = k_mmq_prompt<TA, TB, S, RG, CH, SB, RGB>;
     if (!g.frag) { PI_CHECK_HIP(hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); return 0; }       // pi_op_mul_mat_reserve
-    const int blocks_a = (groups_a + RG - 1) / RG, row_blocks = blocks_a + (groups_all - groups_a + RG - 1) / RG, tok_blocks = (g.nt + CH * 16 - 1) / (CH * 16);
+    const int blocks_a = (groups_a + RG - 1) / RG, row_blocks = blocks_a + (groups_all - groups_a + RGB - 1) / RGB, tok_blocks = (g.nt + CH * 16 - 1) / (CH * 16);
     const unsigned grid = (unsigned) ((row_blocks + 7) / 8 * 8) * (unsigned) tok_blocks;
     if (ea) hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(64 * S * RG), lds, stream, ea, eb, 0, g, groups_a, groups_all, blocks_a, row_blocks, tok_blocks);
     else    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * S * RG), lds, stream, g, groups_a, groups_all, blocks_a, row_blocks, tok_blocks);
@@ -382,7 +385,7 @@ static int prompt_cfg(int cfg, const mmvq_args & g, int groups_a, int groups_all
         case 243: return prompt_go<TA, TB, 2, 4, 3>(g, groups_a, groups_all, stream, ea, eb);
         case 244: return prompt_go<TA, TB, 2, 4, 4>(g, groups_a, groups_all, stream, ea, eb);
         case 222: return prompt_go<TA, TB, 2, 2, 2>(g, groups_a, groups_all, stream, ea, eb);
-        case 182: return prompt_go<TA, TB, 1, 8, 2>(g, groups_a, groups_all, stream, ea, eb);
+        case 182: if constexpr (TA != TB) return prompt_go<TA, TB, 1, 8, 2, 2, 4>(g, groups_a, groups_all, stream, ea, eb); else return prompt_go<TA, TB, 1, 8, 2>(g, groups_a, groups_all, stream, ea, eb);
     }
     pi_set_error("mmq_prompt: configuration %d", cfg);
     return -1;
@@ -412,19 +415,24 @@ bool pi_mmq_prompt_wants(int type, int n_tok, int64_t rows) {
     return n_tok > 16 && (rows + 15) / 16 * 256 / pi_cu_count() >= (type == PI_Q6_K ? 256 : 384);
 }
 // Which tiles: the shortest estimate of  rounds of workgroups x time of a round.  A round's time (us for 32 blocks, launch taken off; 8192 columns, measured per type on a full round) is about the same for all sizes:
-// what differs is how many tiles a wave's operand serves (4 chunks: least work per tile) against how well the launch fills its rounds.  [Q3_K, Q4_K, Q5_K, Q6_K]; two of the four-wave workgroups fit a CU
-static int prompt_choose(int type, int row_groups, int chunks) {
-    static const struct { int cfg, rg, ch, per_cu; float one, full; } cfgs[4][5] = {
+// what differs is how many tiles a wave's operand serves (4 chunks: least work per tile) against how well the launch fills its rounds.  [Q3_K, Q4_K, Q5_K, Q6_K]; two of the four-wave workgroups fit a CU.
+// Two types: the second one's workgroups come last, and what a round of them takes longer is added at the end
+static int prompt_choose(int type_a, int type_b, int groups_a, int groups_b, int chunks) {
+    struct tiles { int cfg, rg, ch, per_cu; float one, full; };
+    static const tiles cfgs[4][5] = {
         { { 222, 2, 2, 2, 24.0f, 36.0f }, { 242, 4, 2, 1, 28.0f, 28.0f }, { 243, 4, 3, 1, 35.0f, 35.0f }, { 244, 4, 4, 1, 43.5f, 43.5f }, { 182, 8, 2, 1, 48.7f, 48.7f } },
         { { 222, 2, 2, 2, 22.5f, 35.0f }, { 242, 4, 2, 1, 26.0f, 26.0f }, { 243, 4, 3, 1, 35.5f, 35.5f }, { 244, 4, 4, 1, 43.0f, 43.0f }, { 182, 8, 2, 1, 39.8f, 39.8f } },
         { { 222, 2, 2, 2, 26.0f, 39.0f }, { 242, 4, 2, 1, 33.0f, 33.0f }, { 243, 4, 3, 1, 40.0f, 40.0f }, { 244, 4, 4, 1, 51.0f, 51.0f }, { 182, 8, 2, 1, 51.0f, 51.0f } },
         { { 222, 2, 2, 2, 27.0f, 42.0f }, { 242, 4, 2, 1, 37.0f, 37.0f }, { 243, 4, 3, 1, 46.0f, 46.0f }, { 244, 4, 4, 1, 56.7f, 56.7f }, { 182, 8, 2, 1, 64.5f, 64.5f } },
     };
+    auto of = [](int type) { return cfgs[type == PI_Q3_K ? 0 : type == PI_Q4_K ? 1 : type == PI_Q5_K ? 2 : 3]; };
     int best = 244; float best_t = 1e30f;
-    for (const auto & c : cfgs[type == PI_Q3_K ? 0 : type == PI_Q4_K ? 1 : type == PI_Q5_K ? 2 : 3]) {
-        const int64_t wgs = (int64_t) ((row_groups + c.rg - 1) / c.rg) * ((chunks + c.ch - 1) / c.ch), slots = (int64_t) pi_cu_count() * c.per_cu, whole = wgs / slots, rest = wgs % slots;
+    for (int i = 0; i < 5; i++) {
+        const tiles & c = of(type_a)[i], & d = of(type_b)[groups_b > 0 && c.cfg == 182 ? 1 : i];          // (182: the second type's are 242, see the kernel)
+        const int64_t wgs = (int64_t) ((groups_a + c.rg - 1) / c.rg + (groups_b + d.rg - 1) / d.rg) * ((chunks + c.ch - 1) / c.ch), slots = (int64_t) pi_cu_count() * c.per_cu, whole = wgs / slots, rest = wgs % slots;
         // (up to three rounds the last one counts in full; behind more, workgroups of many rounds run past each other and about half a round is lost)
-        const float t = whole >= 3 ? c.full * ((float) wgs / slots + 0.5f) : c.full * whole + (rest == 0 ? 0.0f : rest <= pi_cu_count() ? c.one : c.full);
+        float t = whole >= 3 ? c.full * ((float) wgs / slots + 0.5f) : c.full * whole + (rest == 0 ? 0.0f : rest <= pi_cu_count() ? c.one : c.full);
+        if (groups_b > 0 && d.full > c.full) t += d.full - c.full;
         if (t < best_t) { best_t = t; best = c.cfg; }
     }
     return best;
@@ -438,5 +446,6 @@ int pi_mmq_prompt_launch(int type_a, int type_b, int n_a, mmvq_launch & L, hipSt
         if (i < L.nseg) { g.seg[i].wave0 = groups; groups += (g.seg[i].M + 15) / 16; if (i < n_a) groups_a = groups; }
         else { g.seg[i] = g.seg[0]; g.seg[i].wave0 = 0x7fffffff; }
     }
-    return prompt_types(type_a, n_a < L.nseg ? type_b : type_a, prompt_choose(type_a, groups, (g.nt + 15) / 16), g, groups_a, groups, stream, ea, eb);
+    if (n_a >= L.nseg) type_b = type_a;
+    return prompt_types(type_a, type_b, prompt_choose(type_a, type_b, groups_a, groups - groups_a, (g.nt + 15) / 16), g, groups_a, groups, stream, ea, eb);
 }

@@ -921,10 +921,10 @@ def test_two_weight_types_share_one_matrix_core_launch(gpu, types, k, n_tok, n_h
 
 
 @pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q5_K), (O.Q4_K, O.Q4_K, O.Q6_K), (O.Q4_K, O.Q6_K, O.Q6_K)])
-@pytest.mark.parametrize("k,rows,n_tok,cus", [(256, (33, 7, 18), 33, 0), (768, (6200, 40, 33), 20, 0), (512, (5000, 35, 70), 64, 0), (512, (8176, 9, 33), 40, 0), (256, (8176, 9, 33), 63, 0), (256, (16000, 150, 149), 64, 255)])
+@pytest.mark.parametrize("k,rows,n_tok,cus", [(256, (33, 7, 18), 33, 0), (768, (6200, 40, 33), 20, 0), (512, (5000, 35, 70), 64, 0), (512, (8176, 9, 33), 40, 0), (256, (8176, 9, 33), 63, 255), (512, (410, 409, 7990), 47, 0), (512, (410, 409, 7990), 50, 0)])
 def test_two_weight_types_prompt_tiles(gpu, types, k, rows, n_tok, cus):
-    """k_mmq_prompt of two types in every tile shape that its rule chooses for a launch of up to 64 tokens (the last of an odd number of compute units only), rows that end inside a row group of either type, with and
-    without a residual: the oracle's bits"""
+    """k_mmq_prompt of two types in every tile shape that its rule chooses for a launch of up to 64 tokens (and of a context confined to fewer compute units), rows that end inside a row group of either type, with and without
+    a residual: the oracle's bits"""
     lib, U = gpu
     from pipeinfer_amd import lib as L
     rng = np.random.default_rng(k + sum(rows) + n_tok)
