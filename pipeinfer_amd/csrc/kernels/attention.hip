@@ -334,7 +334,7 @@ __global__ void __launch_bounds__(256) k_attention(const att_args ga) {
 // Measured, us before / now (prompt without cells ahead): 32 heads of 128, 128 tokens 39 / 16, 333: 198 / 47, 480: 230 / 64; 64 heads over 8, 128: 70 / 23, 480: 640 / 122; 32 heads of 64 over 4, 333: 114 / 29.  (One score per
 // lane with keys through scalar loads, everything on the VALU: 97 at 333.)  Now the matrix cores are busy in 25 % of the cycles; the VALU's 45 % are conversions, folds and the soft max.
 // =================================================================================================================
-#define ATT_TILE_CELLS 2240                                  // 16 score rows of so many cells in LDS
+#define ATT_TILE_CELLS 2240                                  // 16 score rows of so many cells in LDS (128 tokens of 64 heads over 8: 137 us over 1628 cells, on k_attention 505 and, over 2428, 726)
 using att_f32x16 = __attribute__((ext_vector_type(16))) float;
 using att_f32x4 = __attribute__((ext_vector_type(4))) float;
 static __host__ __device__ constexpr int att_tile_stride(int cells) { return (cells + 31) / 32 * 32 + 4; }
@@ -810,7 +810,9 @@ extern "C" int pi_op_attention_alibi(const uint16_t * q16, const uint16_t * kc, 
     while (rw > 1 && att_lds_bytes(rw, n_kv) > att_lds_cap(rw)) rw >>= 1;               // long contexts: fewer score rows per workgroup (they live in LDS)
     if ((size_t) rw * (n_kv + g.mask_words) * sizeof(float) > att_lds_cap(rw)) { pi_set_error("pi_op_attention: n_kv=%d needs more than %d KiB of LDS", n_kv, rw == 1 ? 146 : 156); return -1; }
     // from 1536 query rows: below, a workgroup's chain of phases (12 us at 32 cells of 128 values) is longer than k_attention's launch.  us there / here, no cells and 100 cells ahead: 32 heads of 128, 32 tokens 9.1 / 12.0
-    // and 17.5 / 16.3, 48: 14.2 / 14.2 and 22 / 18; 64 heads over 8, 16 tokens 11 / 13 and 15 / 17, 24: 13.3 / 14.3 and 18.5 / 17.8, 48: 25 / 15 and 39 / 19; 32 heads of 64 over 4, 48 tokens 10.7 / 8.5 and 15 / 11
+    // and 17.5 / 16.3, 48: 14.2 / 14.2 and 22 / 18; 64 heads over 8, 16 tokens 11 / 13 and 15 / 17, 24: 13.3 / 14.3 and 18.5 / 17.8, 48: 25 / 15 and 39 / 19; 32 heads of 64 over 4, 48 tokens 10.7 / 8.5 and 15 / 11.
+    // Behind a bound of more cells k_attention is launched as well, which is 2 us, and alone would put several rows into a workgroup there: 64 heads over 8, bound 4096, 32 tokens with 0 / 100 / 700 / 1500 cells ahead 11.8 / 21.7
+    // / 56.7 / 103 there, 15.5 / 19.7 / 40.9 / 66 here; 32 heads of 128, 64 tokens 13.5 / 22.6 / 58 / 107 and 15.9 / 20.2 / 41 / 70
     static const int tile_min = getenv("PI_ATT_TILE_MIN") ? atoi(getenv("PI_ATT_TILE_MIN")) : 1536;
     if ((hd == 128 || hd == 64) && !alibi_slopes_dev && !g.per_token && (int64_t) n_tok * n_head >= tile_min && (dyn_dev || n_kv <= ATT_TILE_CELLS) && (((uintptr_t) q16 | (uintptr_t) out | (uintptr_t) kc | (uintptr_t) vc) & 15) == 0) {
         if (att_tile_reserve() != 0) return -1;

@@ -1926,7 +1926,7 @@ __global__ void __launch_bounds__(256) k_moe_group(const int32_t * __restrict__ 
 
 // A tile of slots x BN rows of its expert's matrix (dense_tile.h).  UP: X rows are the tokens' inputs x[slot / top], W rows W_up[e], out up[slot][f] = relu(.)^2; !UP: X rows up[slot] (K = ff), W rows W_down[e],
 // out dn[slot][n].  glu: UP leaves the 2 * ff rows [gate | up] of an expert raw, !UP (PAIR) joins them while it stages them (bs = 2 * ff, K = ff).  What bounds it: as k_dense_tile, whose tiles these are.  Operands
-// straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048 (now 116 and 125: 475 and 440 TFLOP/s), 44 and 23 us for 24 tokens' of 1024 x 512
+// straight from memory, 64 x 64 without prefetch, took 623 and 702 us for 2048 tokens' two choices of 8 experts 4096 x 2048 (now 91 and 98: 605 and 562 TFLOP/s), 44 and 23 us for 24 tokens' of 1024 x 512
 // (10 and 7).
 template <int BN, int BT, int WN, int WT, int KG, bool UP, bool PAIR>
 __global__ void __launch_bounds__(64 * WN * WT * KG, 2) k_moe_tile(const uint16_t * __restrict__ W, int64_t K, int rows, const float * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx,

@@ -1,4 +1,4 @@
-// Prompt passes of K-quant weights (Q3_K, Q4_K, Q5_K, Q6_K) on the matrix cores: a whole pass of any number of tokens in one launch, BIT-EXACT with the reference's x86 AVX2 arm (the contract of mmvq.hip).
+// Prompt passes of K-quant weights (Q3_K, Q4_K, Q5_K, Q6_K) on the matrix cores: a whole pass of any number of tokens in one launch (two types: whatever the caller gives a launch, 64 tokens), BIT-EXACT with the reference's x86 AVX2 arm (the contract of mmvq.hip).
 //
 //   out[t][row] = residual[t][row] + vec_dot(W[row], act[t])
 //

@@ -910,7 +910,7 @@ static int dispatch_nt(mmvq_launch & L, int nt, hipStream_t stream) {
 }
 
 // out[i][t][row] = residual[i][t][row] + vec_dot(W_i[row], act[t]) for n_w (<= 3) weight matrices of the same type and width
-// sharing one quantised activation.  Q4_0/Q8_0 weights are launched one by one.
+// sharing one quantised activation (or Q4_K followed by Q5_K or Q6_K).  Q4_0 / Q8_0 weights share a launch from seven tokens (mmq_q0.hip) and are launched one by one below.
 // RoPE / KV-store epilogue of a grouped launch: per weight where its rows go (mmvq_seg::store), plus what the epilogue reads
 struct mmvq_rope { int store[MMVQ_MAX_SEG]; uint16_t * dst16[MMVQ_MAX_SEG]; int stride16[MMVQ_MAX_SEG]; const int32_t * pos; const float * cs; const int32_t * dyn; int kv_head, hd; };
 
@@ -931,7 +931,7 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
     }
     const bool all_b = type_b >= 0 && type_b_mask == (1 << n_w) - 1;            // a single type that is not Q4_K
     const bool mixed = type_b >= 0 && !all_b;
-    // ... or, at 3..8 tokens, on the matrix cores (k_mmq_kq2t): the Q4_K matrices first, the second type's behind them
+    // ... or on the matrix cores, at 3..8 tokens (k_mmq_kq2t) and in prompts (k_mmq_prompt): the Q4_K matrices first, the second type's behind them
     bool mixed_mfma = false, prompt = false; int n_a = 0;          // prompt: k_mmq_prompt
     if (mixed && vdt == PI_Q8_K) {
         while (n_a < n_w && ws[n_a]->type == PI_Q4_K) n_a++;
@@ -945,7 +945,7 @@ static int mul_mat_multi_impl(int n_w, const pi_weight * const * ws, const void 
         bool same = true;
         for (int i = 1; i < n_w; i++) same = same && ws[i]->type == w0->type;
         if (!same) {
-            if (rope) { pi_set_error("pi_op_mul_mat_multi: weights differ in type (Q4_K with Q5_K or Q6_K share a launch at 1-2 tokens, and at 3-8 on the matrix cores)"); return -1; }
+            if (rope) { pi_set_error("pi_op_mul_mat_multi: weights differ in type (Q4_K with Q5_K or Q6_K share a launch at 1-2 tokens, and on the matrix cores at 3-8 and in prompts)"); return -1; }
             // plain outputs: the matrices that cannot share a launch go out one by one
             for (int i = 0; i < n_w; i++) { const int rc = mul_mat_multi_impl(1, ws + i, q8, n_tok, outs + i, ress ? ress + i : nullptr, nullptr, stream_); if (rc) return rc; }
             return 0;
