@@ -102,6 +102,7 @@ PI_API const void * pi_weight_data(const pi_weight * w); /* device address of th
 /* reads [p, p + bytes) once with up to `workgroups` workgroups (0: as many as the bytes need): warms the memory-side Infinity Cache */
 PI_API int     pi_op_prefetch(const void * p, size_t bytes, int workgroups, void * stream);
 PI_API int     pi_weight_type(const pi_weight * w);
+PI_API int64_t pi_weight_columns(const pi_weight * w);   /* values of a row */
 
 /* type the activations must be quantised to for this weight type (type_traits[].vec_dot_type, ggml.c:415-600) */
 PI_API int     pi_vec_dot_type(int weight_type);
@@ -288,6 +289,12 @@ PI_API int pi_op_embed_pair(const pi_weight * table, const int32_t * tokens_dev,
  * remaining rows (projections of DIFFERENT inputs of one width in one launch where the pass has few tokens) */
 PI_API int pi_op_dense_segments(const pi_weight * w, const float * x_dev, int64_t x_stride, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out_dev, int64_t out_stride, int act_a, int64_t rows_a,
                                 int act_b, int exact, void * stream);
+/* the same products from activations that are bfloat16 in memory (what serving precision rounds them to anyway), for passes of more tokens than the kernels that share K out take: pi_op_dense_rounded_ok says for which; n_seg > 1:
+ * segments as above, in one launch.  pi_op_round_bf16: rows of fp32 values rounded to nearest even (n % 8 == 0, 16-byte aligned rows) */
+PI_API int pi_op_round_bf16(const float * x_dev, int64_t x_stride, int64_t n, int n_tok, uint16_t * out_dev, int64_t out_stride, void * stream);
+PI_API int pi_op_dense_rounded_ok(const pi_weight * w, int64_t x_stride, int n_tok);
+PI_API int pi_op_dense_rounded(const pi_weight * w, const float * bias_dev, const uint16_t * x_dev, int64_t x_stride, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out_dev, int64_t out_stride, int act_a,
+                               int64_t rows_a, int act_b, void * stream);
 /* the end of a sublayer, R(y) = y / sqrt(mean(y^2) + eps):  m = b ? mean_mult * (R(a) * wa + R(b) * wb) : a;  out = R(alpha * x + layer_scale * m) * w  (layer_scale nullable: 1);
  * w_next != NULL: out_next = R(out) * w_next (the norm of whatever reads the stream next).  out may be x.  Rows of at most 8192 values */
 PI_API int pi_op_rms_post(const float * a_dev, int64_t a_stride, const float * wa_dev, const float * b_dev, int64_t b_stride, const float * wb_dev, float mean_mult, const float * layer_scale_dev,

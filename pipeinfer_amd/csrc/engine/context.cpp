@@ -44,7 +44,7 @@ llama_context::~llama_context() {
     if (hop_host) (void) hipHostFree(hop_host);
     pi_free(hop_dev);
     pi_free(abort_dev);
-    void * bufs[] = { cell_pos, hist, h_out2, h_out3, x_pair, ssd_dt, lat_cache, rec_state, rec_dev, pair_dev, h_in, h_att, h_out, moe_w, moe_up, moe_dn, lat_scratch, rec_scratch, moe_sel, moe_idx, k_cache, v_cache, x, x2, nx, nx2, qkv, att, up, gate, logits_dev, q16, q8a, q8b, q8c, tokens_dev, pos_dev, dyn_dev, mask_dev, topk_ids_dev, topk_vals_dev, topk_sum_dev, topk_scratch_dev };
+    void * bufs[] = { act_h, cell_pos, hist, h_out2, h_out3, x_pair, ssd_dt, lat_cache, rec_state, rec_dev, pair_dev, h_in, h_att, h_out, moe_w, moe_up, moe_dn, lat_scratch, rec_scratch, moe_sel, moe_idx, k_cache, v_cache, x, x2, nx, nx2, qkv, att, up, gate, logits_dev, q16, q8a, q8b, q8c, tokens_dev, pos_dev, dyn_dev, mask_dev, topk_ids_dev, topk_vals_dev, topk_sum_dev, topk_scratch_dev };
     for (void * b : bufs) pi_free(b);
     for (auto & kv : window_masks) pi_free(kv.second);
     if (rope) pi_rope_table_free(rope);
@@ -199,6 +199,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
     if (!(ctx->x = (float *) dev((size_t) 4 * nb * width * std::max(1, hp.streams))) || !(ctx->nx = (float *) dev((size_t) 4 * nb * width)) || !(ctx->h_out = (float *) dev((size_t) 4 * nb * width)) ||
         !(ctx->h_in = (float *) dev((size_t) 4 * nb * in_w)) || !(ctx->h_att = (float *) dev((size_t) 4 * nb * att_w)) || !(ctx->moe_up = (float *) dev((size_t) 4 * nb * up_w)) ||
         !(ctx->moe_w = (float *) dev((size_t) 4 * nb * sel_w)) || !(ctx->moe_dn = (float *) dev((size_t) 4 * nb * sel_w * width)) || !(ctx->moe_idx = (int32_t *) dev((size_t) 4 * idx_n)) || !(ctx->moe_sel = (int32_t *) dev((size_t) 4 * nb * sel_w)) || (ctx->slots && !(ctx->rec_dev = (int32_t *) dev((size_t) 4 * nb))) || (hp.pair_buckets > 0 && !(ctx->pair_dev = (int32_t *) dev((size_t) 4 * nb))) ||
+        !(ctx->act_h = (uint16_t *) dev((size_t) 2 * nb * (ctx->act_h_row = std::max(std::max(in_w, att_w), (size_t) 2 * width)))) ||
         !(ctx->tokens_dev = (int32_t *) dev((size_t) 4 * nb)) || !(ctx->pos_dev = (int32_t *) dev((size_t) 4 * nb)) || !(ctx->dyn_dev = (int32_t *) dev((size_t) 4 * (4 + 2 * nb))))
         return false;
     {   // abort word + cancel flags + the control stream cancels travel on
@@ -377,6 +378,24 @@ static bool mul_mat_grouped(int n, const pi_weight * const * ws, const void * co
     return true;
 }
 
+// A product of the serving precision in a pass of many tokens reads activations that are bfloat16 already: xh, where a kernel ahead wrote them, or rounded here, into the context's scratch (products of a context follow each other on
+// its stream).  Everything else goes to the operators that take fp32
+static int dense_segments(llama_context * ctx, const pi_weight * w, const float * x, int64_t xs, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s,
+                          const uint16_t * xh = nullptr, int64_t xhs = 0, const float * bias = nullptr) {
+    const int64_t n = (n_seg - 1) * seg_off + pi_weight_columns(w), hs = xh ? xhs : n;
+    const bool whole = xh || (xs % 4 == 0 && (uintptr_t) x % 16 == 0 && n % 8 == 0 && (size_t) n <= ctx->act_h_row);
+    if (ctx->exact || !whole || (n_seg > 1 && (seg_off % 8 || seg_rows % 4)) || !pi_op_dense_rounded_ok(w, hs, n_tok))
+        return n_seg > 1 ? pi_op_dense_segments(w, x, xs, seg_rows, seg_off, n_seg, n_tok, out, os, act_a, rows_a, act_b, ctx->exact, s) : pi_op_dense_bias(w, bias, x, xs, n_tok, out, os, act_a, rows_a, act_b, ctx->exact, s);
+    if (!xh) {
+        if (pi_op_round_bf16(x, xs, n, n_tok, ctx->act_h, n, s) != 0) return -1;
+        xh = ctx->act_h;
+    }
+    return pi_op_dense_rounded(w, bias, xh, hs, seg_rows, seg_off, n_seg, n_tok, out, os, act_a, rows_a, act_b, s);
+}
+static int dense(llama_context * ctx, const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, const uint16_t * xh = nullptr, int64_t xhs = 0, const float * bias = nullptr) {
+    return dense_segments(ctx, w, x, xs, 0, 0, 1, n_tok, out, os, act_a, rows_a, act_b, s, xh, xhs, bias);
+}
+
 // A hybrid model's pass: per layer  x += m * N1(mixer(x)),  x += m * N2(moe(x))  — the norm sits on the sublayer's output, the sublayers read x itself; everything between the
 // matrix products is fp32.  Kernel sequence: fused input projection (activations in its epilogue) -> mixer kernel -> output projection -> norm + scale + residual; router ->
 // experts -> norm + scale + residual; final norm -> logits against the embedding table itself.
@@ -389,7 +408,7 @@ static bool mul_mat_grouped(int n, const pi_weight * const * ws, const void * co
 static bool forward_parallel_mixer(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
     const pi_hparams & hp = ctx->model->hparams;
     hipStream_t s = ctx->stream;
-    const int width = hp.n_embd, ex = ctx->exact, nb = ctx->n_batch;
+    const int width = hp.n_embd, nb = ctx->n_batch;
     const float eps = hp.f_norm_eps;
     const pi_gate_attention & A = H.left; const pi_ssd & R = H.right;
     const int inner = R.inner(), gn = R.groups * R.state;
@@ -398,7 +417,7 @@ static bool forward_parallel_mixer(llama_context * ctx, const pi_hybrid_layer & 
     float * P = ctx->h_in, * Q = ctx->h_att, * O = Q + (size_t) nb * hd, * S = O + hv, * C = O + (size_t) nb * ow;
     float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
     float * ssm = ctx->rec_state + ctx->rec_off[il], * conv_state = ssm + (size_t) ctx->slots->size() * R.heads * R.state * R.vdim;
-    OP_OK(pi_op_dense(W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
     // the recurrence branch goes to the branch stream (behind the projection), the attention branch stays; they meet again in front of the output projection
     hipStream_t s_main = s, s2 = ctx->branch_stream ? ctx->branch_stream : s;
     if (ctx->branch_stream && (hipEventRecord(ctx->branch_events[2 * il], s_main) != hipSuccess || hipStreamWaitEvent(s2, ctx->branch_events[2 * il], 0) != hipSuccess)) { ctx->last_error = "fork of the mixer's branches failed"; return false; }
@@ -417,7 +436,7 @@ static bool forward_parallel_mixer(llama_context * ctx, const pi_hybrid_layer & 
     OP_OK(pi_op_gate_group_norm(S, ow, R0, pw, W.mix_norm, eps, H.right_scale, inner, R.norm_groups, n_tok, S, ow, s2));
     if (ctx->branch_stream && (hipEventRecord(ctx->branch_events[2 * il + 1], s2) != hipSuccess || hipStreamWaitEvent(s_main, ctx->branch_events[2 * il + 1], 0) != hipSuccess)) { ctx->last_error = "join of the mixer's branches failed"; return false; }
     trace(ctx, "ssd", (int) il, S, inner, n_tok, ow);
-    OP_OK(pi_op_dense(W.w_o, O, ow, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));          // a * W_o att + b * W_o' rec
+    OP_OK(dense(ctx, W.w_o, O, ow, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));          // a * W_o att + b * W_o' rec
     return true;
 }
 
@@ -450,8 +469,8 @@ static bool forward_pre_post_blocks(llama_context * ctx, int n_tok, int n_kv) {
             OP_OK(pi_op_norm_chain(Y, width, 1.0f, nullptr, 0, 0.0f, W.post1, W.post1_b, eps, width, n_tok, x, width, ctx->x, width, nullptr, 0, 0, nullptr, nullptr, 0, W.norm2, W.norm2_b, N, width, s));   // + the feed-forward's pre-norm
             x = ctx->x;
             if (H.mlp == PI_MLP_DENSE_RELU_SQR) {
-                OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, H.ff, PI_ACT_RELU_SQR, H.ff, PI_ACT_RELU_SQR, ex, s));
-                OP_OK(pi_op_dense(W.ff_down, P, H.ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+                OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, H.ff, PI_ACT_RELU_SQR, H.ff, PI_ACT_RELU_SQR, s));
+                OP_OK(dense(ctx, W.ff_down, P, H.ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
                 OP_OK(block_end(Y, nullptr, W.post2, W.post2_b, x));
             } else {
                 OP_OK(pi_op_moe_route_groups(W.router, N, width, n_tok, H.top, H.route_groups, H.route_keep, ex, ctx->moe_sel, ctx->moe_w, s));
@@ -462,9 +481,9 @@ static bool forward_pre_post_blocks(llama_context * ctx, int n_tok, int n_kv) {
                 if (H.shared_ff > 0) {                                     // the expert every token uses: silu(gate) in the projection's epilogue, * up, down
                     const int sf = H.shared_ff;
                     float * G = P + (size_t) nb * 2 * sf;
-                    OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, 2 * sf, PI_ACT_SILU, sf, PI_ACT_NONE, ex, s));
+                    OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, 2 * sf, PI_ACT_SILU, sf, PI_ACT_NONE, s));
                     OP_OK(pi_op_glu_mul(P, 2 * sf, sf, n_tok, G, sf, s));
-                    OP_OK(pi_op_dense(W.ff_down, G, sf, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+                    OP_OK(dense(ctx, W.ff_down, G, sf, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
                 }
                 OP_OK(block_end(Y, H.shared_ff > 0 ? Y2 : nullptr, W.post2, W.post2_b, x));
             }
@@ -472,7 +491,7 @@ static bool forward_pre_post_blocks(llama_context * ctx, int n_tok, int n_kv) {
         x = ctx->x;
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    OP_OK(pi_op_dense(hp.own_head ? m->output : m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, hp.own_head ? m->output : m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     if (hp.logit_softcap > 0.0f) OP_OK(pi_op_softcap(ctx->logits_dev, (int64_t) n_tok * hp.n_vocab, hp.logit_softcap, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
@@ -489,7 +508,7 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
     llama_model * m = ctx->model;
     const pi_hparams & hp = m->hparams;
     hipStream_t s = ctx->stream;
-    const int width = hp.n_embd, ex = ctx->exact, nb = ctx->n_batch, n_slots = ctx->slots->size();
+    const int width = hp.n_embd, nb = ctx->n_batch, n_slots = ctx->slots->size();
     const float eps = hp.f_norm_rms_eps, alpha = hp.post_alpha;
     const size_t n_layer = hp.hybrid.size();
     float * x = ctx->x, * P = ctx->h_in, * A = ctx->h_att, * Y = ctx->h_out, * Y2 = ctx->h_out2;
@@ -506,18 +525,18 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
             const int64_t aw = hd + hv;                                                                // a token's row of [raw decays | raw gate]
             float * C = A, * A2 = C + (size_t) nb * ch, * G2 = A2 + hd, * O = A2 + (size_t) nb * aw;
             float * S = ctx->rec_state + ctx->rec_off[il], * conv_state = S + (size_t) n_slots * D.matrix_floats();
-            OP_OK(pi_op_dense(W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
             OP_OK(pi_op_causal_conv(P, pw, (int) ch, D.conv, W.conv_w, nullptr, conv_state, ctx->rec_dev, n_tok, PI_ACT_SILU, C, ch, s));
-            if (!W.w_g2) OP_OK(pi_op_dense_segments(W.w_a2, P + ch, pw, hd, D.decay_rank, 2, n_tok, A2, aw, PI_ACT_NONE, aw, PI_ACT_NONE, ex, s));
+            if (!W.w_g2) OP_OK(dense_segments(ctx, W.w_a2, P + ch, pw, hd, D.decay_rank, 2, n_tok, A2, aw, PI_ACT_NONE, aw, PI_ACT_NONE, s));
             else {
-                OP_OK(pi_op_dense(W.w_a2, P + ch, pw, n_tok, A2, aw, PI_ACT_NONE, hd, PI_ACT_NONE, ex, s));
-                OP_OK(pi_op_dense(W.w_g2, P + ch + D.decay_rank, pw, n_tok, G2, aw, PI_ACT_NONE, hv, PI_ACT_NONE, ex, s));
+                OP_OK(dense(ctx, W.w_a2, P + ch, pw, n_tok, A2, aw, PI_ACT_NONE, hd, PI_ACT_NONE, s));
+                OP_OK(dense(ctx, W.w_g2, P + ch + D.decay_rank, pw, n_tok, G2, aw, PI_ACT_NONE, hv, PI_ACT_NONE, s));
             }
             OP_OK(pi_op_channel_recurrence(PI_RULE_DELTA, C, ch, C + gd, ch, C + 2 * gd, ch, A2, aw, 2, W.dt_bias, W.a_log, P + ch + D.decay_rank + D.gate_rank, pw, nullptr, 1, 1.0f / sqrtf((float) D.dim), D.heads, D.kv_heads, D.dim, D.vdim,
                                            S, ctx->rec_dev, n_tok, n_slots, ctx->rec_scratch, ctx->rec_scratch_floats, O, hv, s));
             trace(ctx, "rec", (int) il, O, hv, n_tok);
             OP_OK(pi_op_head_norm_gate(O, hv, D.heads, D.vdim, W.mix_norm, 0, G2, aw, PI_ACT_SIGMOID, eps, n_tok, O, hv, s));
-            OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
         } else if (H.mixer == PI_MIXER_PARALLEL_SHIFT) {
             const pi_gate_attention & L = H.left; const pi_time_mix & R = H.shift;
             const int64_t pw = L.in_rows(), hd = (int64_t) L.heads * L.dim, hv = (int64_t) L.heads * L.vdim, gd = (int64_t) L.kv_heads * L.dim, inner = R.inner(), mw = (int64_t) 5 * width;
@@ -527,36 +546,36 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
             float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
             float * S = ctx->rec_state + ctx->rec_off[il], * shift_state = S + (size_t) n_slots * R.matrix_floats();
             // attention branch
-            OP_OK(pi_op_dense(W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
             OP_OK(pi_op_qkv_prepare_ex(P, P + hd, P + hd + gd, pw, nullptr, nullptr, eps, L.heads, L.kv_heads, L.dim, L.vdim, W.rotary, 0, PI_PAIR_NEIGHBOURS, 0, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
             OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, nullptr, 0, PI_ACT_NONE, L.scale, 1.0f, L.weights, L.softcap, PI_MASK_CHUNK, L.chunk, 0, 0, 0, L.heads, L.kv_heads, L.dim,
                                          L.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
             trace(ctx, "att", (int) il, O, hv, n_tok);
-            OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
             // time-mix branch
             OP_OK(pi_op_token_shift(x, width, width, W.mu, 5, shift_state, ctx->rec_dev, n_tok, M, mw, s));
             // r | k | v | g | w1 from their own mixes: rows of ONE matrix in five segments; tanh on w1's rows, the gate's silu waits for the head norm
-            OP_OK(pi_op_dense_segments(W.w_r, M, mw, inner, width, 5, n_tok, RK, rkw, PI_ACT_NONE, 4 * inner, PI_ACT_TANH, ex, s));
-            OP_OK(pi_op_dense(W.w_w2, RK + 4 * inner, rkw, n_tok, WD, inner, PI_ACT_NONE, inner, PI_ACT_NONE, ex, s));
+            OP_OK(dense_segments(ctx, W.w_r, M, mw, inner, width, 5, n_tok, RK, rkw, PI_ACT_NONE, 4 * inner, PI_ACT_TANH, s));
+            OP_OK(dense(ctx, W.w_w2, RK + 4 * inner, rkw, n_tok, WD, inner, PI_ACT_NONE, inner, PI_ACT_NONE, s));
             OP_OK(pi_op_channel_recurrence(PI_RULE_BONUS, RK, rkw, RK + inner, rkw, RK + 2 * inner, rkw, WD, inner, 1, W.w0, nullptr, nullptr, 0, W.bonus, 0, 1.0f, R.heads, R.heads, R.dim, R.dim,
                                            S, ctx->rec_dev, n_tok, n_slots, ctx->rec_scratch, ctx->rec_scratch_floats, O2, inner, s));
             trace(ctx, "rec", (int) il, O2, inner, n_tok);
             OP_OK(pi_op_head_norm_gate(O2, inner, R.heads, R.dim, W.mix_norm, 1, RK + 3 * inner, rkw, PI_ACT_SILU, eps, n_tok, O2, inner, s));
-            OP_OK(pi_op_dense(W.w_o2, O2, inner, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.w_o2, O2, inner, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
             yb = Y2;
         } else { ctx->last_error = "blocks with the norm after the sum are built for the channel-delta and the attention + time-mix mixers"; return false; }
         OP_OK(pi_op_rms_post(ya, width, W.left_out, yb, width, W.right_out, 0.5f, W.ls1, x, width, alpha, W.norm1, eps, width, n_tok, x, width, last_sub_is_mixer ? m->output_norm : nullptr, ctx->nx, width, s));
         if (H.has_mlp) {
             const int ff = H.ff;
             float * G = P + (size_t) nb * 2 * ff;
-            OP_OK(pi_op_dense(W.ff_up, x, width, n_tok, P, 2 * ff, PI_ACT_GELU_TANH, ff, PI_ACT_NONE, ex, s));        // gelu(gate) | up
+            OP_OK(dense(ctx, W.ff_up, x, width, n_tok, P, 2 * ff, PI_ACT_GELU_TANH, ff, PI_ACT_NONE, s));        // gelu(gate) | up
             OP_OK(pi_op_glu_mul(P, 2 * ff, ff, n_tok, G, ff, s));
-            OP_OK(pi_op_dense(W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
             OP_OK(pi_op_rms_post(Y, width, nullptr, nullptr, 0, nullptr, 1.0f, W.ls2, x, width, alpha, W.norm2, eps, width, n_tok, x, width, il + 1 == n_layer ? m->output_norm : nullptr, ctx->nx, width, s));
         }
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    OP_OK(pi_op_dense(m->output, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, m->output, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -588,7 +607,7 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
     auto enter = [&](size_t il, const float * a, const float * b, const float * c) {
         const pi_hybrid_weights & W = m->hweights[(size_t) hp.hybrid[il].weights];
         if (pi_op_sum_tanh_norm(x, width, a, width, b, width, c, width, width, n_tok, XP, 2 * width, nullptr, nullptr, nullptr, nullptr, 0, s) != 0) return false;
-        if (pi_op_dense(W.w_loop, XP, 2 * width, n_tok, x, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s) != 0) return false;
+        if (dense(ctx, W.w_loop, XP, 2 * width, n_tok, x, width, PI_ACT_NONE, width, PI_ACT_NONE, s) != 0) return false;
         return norm_shift(il, nullptr, nullptr, nullptr, nullptr) == 0;
     };
     {
@@ -604,7 +623,7 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
         float * C = ctx->h_att, * Q = C + (size_t) nb * ch, * O = Q + (size_t) nb * hd;
         float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) A.cell_rows() * ctx->n_ctx * gd;
         float * conv_state = ctx->rec_state + ctx->rec_off[il] + (size_t) n_slots * width;         // (behind the run's shifted-token rows)
-        OP_OK(pi_op_dense(W.w_in, M, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+        OP_OK(dense(ctx, W.w_in, M, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
         const float * qkv = P; int64_t qs = pw;
         if (A.conv > 0) { OP_OK(pi_op_causal_conv(P, pw, (int) ch, A.conv, W.conv_w, nullptr, conv_state, ctx->rec_dev, n_tok, PI_ACT_NONE, C, ch, s)); qkv = C; qs = ch; }
         OP_OK(pi_op_qkv_prepare_ex(qkv, qkv + hd, qkv + hd + gd, qs, W.q_norm, W.k_norm, eps, A.heads, A.kv_heads, A.dim, A.vdim, W.rotary, A.qk_norm, A.pairing, A.v_norm ? 1 : 0, ctx->pos_dev, n_tok, Q, hd, kc, vc,
@@ -614,11 +633,11 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
         OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, W.sink, A.gated ? P + ch : nullptr, pw, PI_ACT_SIGMOID, A.scale, 1.0f, A.weights, A.softcap, A.mask_kind, A.chunk,
                                      pooled ? A.pool : 0, ctx->n_ctx, pool_here ? 1 : 0, A.heads, A.kv_heads, A.dim, A.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
         trace(ctx, "att", (int) il, O, hv, n_tok);
-        OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+        OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
         const float * y2 = nullptr, * y3 = nullptr;
         if (H.mlp == PI_MLP_DENSE_GELU) {
-            OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, H.ff, PI_ACT_GELU_ERF, H.ff, PI_ACT_GELU_ERF, ex, s));
-            OP_OK(pi_op_dense(W.ff_down, P, H.ff, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, H.ff, PI_ACT_GELU_ERF, H.ff, PI_ACT_GELU_ERF, s));
+            OP_OK(dense(ctx, W.ff_down, P, H.ff, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
             y2 = Y2;
         } else if (H.mlp == PI_MLP_MOE_CLIPPED) {
             OP_OK(pi_op_moe_route_top_logits(W.router, W.correction, N, width, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s));
@@ -630,9 +649,9 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
             if (H.shared_ff > 0) {                                         // the expert every token uses: [gate | up | token gate] in one projection, the clipped product times sigmoid(token gate), down
                 const int sf = H.shared_ff; const int64_t sw = 2 * (int64_t) sf + 1;
                 float * G = P + (size_t) nb * sw;
-                OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, sw, PI_ACT_NONE, sw, PI_ACT_NONE, ex, s));
+                OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, sw, PI_ACT_NONE, sw, PI_ACT_NONE, s));
                 OP_OK(pi_op_glu_mul_ex(P, sw, sf, PI_GLU_CLIPPED, H.shared_limit, 2 * (int64_t) sf, n_tok, G, sf, s));
-                OP_OK(pi_op_dense(W.ff_down, G, sf, n_tok, Y3, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+                OP_OK(dense(ctx, W.ff_down, G, sf, n_tok, Y3, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
                 y3 = Y3;
             }
         }
@@ -646,7 +665,7 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
         else OP_OK(pi_op_sum_tanh_norm(x, width, Y, width, y2, width, y3, width, width, n_tok, x, width, m->output_norm_alpha, m->output_norm, m->output_norm_b, N, width, s));
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    OP_OK(pi_op_dense(m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -663,57 +682,57 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
 static bool forward_memory(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok) {
     hipStream_t s = ctx->stream;
     const pi_memory & M = H.memory;
-    const int width = ctx->model->hparams.n_embd, ex = ctx->exact, nb = ctx->n_batch, n_slots = ctx->slots->size();
+    const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch, n_slots = ctx->slots->size();
     const int64_t pw = row_of_4(M.in_rows()), hd = (int64_t) M.heads * M.dim, hv = (int64_t) M.heads * M.vdim, hv1 = hv + M.heads;
     float * P = ctx->h_in, * O = ctx->h_att, * Z = O + (size_t) nb * hv, * forget = Z + (size_t) nb * hv1, * put = forget + (size_t) nb * M.heads, * flo = put + (size_t) nb * M.heads;
     float * S = ctx->rec_state + ctx->rec_off[il], * m_run = S + (size_t) n_slots * M.matrix_floats();
-    OP_OK(pi_op_dense(W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
     OP_OK(pi_op_memory_gates(P + 2 * hd + 2 * hv, P + 2 * hd + 2 * hv + M.heads, pw, W.gate_bias, W.gate_bias + M.heads, M.cap, M.heads, m_run, ctx->rec_dev, n_tok, forget, put, flo, s));
     OP_OK(pi_op_linear_attention_keysum(P, P + hd, P + 2 * hd, pw, M.heads, M.heads, M.dim, M.vdim, 1, nullptr, forget, put, M.heads, nullptr, S, ctx->rec_dev, n_tok, n_slots, ctx->rec_scratch, ctx->rec_scratch_floats, Z, hv1, s));
     OP_OK(pi_op_memory_norm(Z, hv1, flo, 1.0f / sqrtf((float) M.dim), 1e-6f, M.heads, M.vdim, ctx->model->hparams.f_norm_rms_eps, W.mix_norm, P + 2 * hd + hv, pw, PI_ACT_SIGMOID, n_tok, O, hv, s));
     trace(ctx, "mem", (int) il, O, hv, n_tok);
-    OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
     return true;
 }
 static bool forward_temp_attention(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
     hipStream_t s = ctx->stream;
     const pi_gate_attention & A = H.left;
-    const int width = ctx->model->hparams.n_embd, ex = ctx->exact, nb = ctx->n_batch;
+    const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch;
     const bool own = H.kv_from < 0;
     const int64_t pw = row_of_4(H.in_rows()), hd = (int64_t) A.heads * A.dim, hv = (int64_t) A.heads * A.vdim, gd = (int64_t) A.kv_heads * A.dim;
     float * P = ctx->h_in, * Q = ctx->h_att, * O = Q + (size_t) nb * hd;
     float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
-    OP_OK(pi_op_dense_bias(W.w_in, W.in_bias, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, nullptr, 0, W.in_bias));
     OP_OK(pi_op_qkv_prepare_temp(P, own ? P + hd : nullptr, own ? P + hd + gd : nullptr, pw, nullptr, nullptr, ctx->model->hparams.f_norm_rms_eps, A.heads, A.kv_heads, A.dim, A.vdim, W.rotary, A.qk_norm, A.pairing,
                                  A.v_norm ? 1 : 0, A.temp_coef, A.temp_every, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
     OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, nullptr, 0, PI_ACT_NONE, A.scale, 1.0f, A.weights, A.softcap, A.mask_kind, A.chunk, 0, 0, 0, A.heads, A.kv_heads, A.dim,
                                  A.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
     trace(ctx, "att", (int) il, O, hv, n_tok);
-    OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
     return true;
 }
 static bool forward_query_latent(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
     hipStream_t s = ctx->stream;
     const pi_latent & A = H.latent;
-    const int width = ctx->model->hparams.n_embd, ex = ctx->exact, nb = ctx->n_batch, R = A.rot_dim;
+    const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch, R = A.rot_dim;
     const int64_t pw = row_of_4(H.in_rows()), cw = row_of_4(A.q_rank), qw = (int64_t) H.heads * (H.dim + R), hv = (int64_t) H.heads * H.vdim;
     float * P = ctx->h_in, * C = ctx->h_att, * Q = C + (size_t) nb * cw, * O = Q + (size_t) nb * qw;
     float * cache = ctx->lat_cache + ctx->lat_off[il];
     const uint32_t * mask = A.window > 0 ? ctx->window_masks.at(A.window) : ctx->mask_dev;
-    OP_OK(pi_op_dense(W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
     OP_OK(pi_op_latent_prepare_ex(P, pw, A.q_rank, W.q_norm, H.kv_rank, W.mix_norm, R, W.rotary, A.pairing, ctx->model->hparams.f_norm_rms_eps, ctx->pos_dev, n_tok, C, cw, cache, ctx->dyn_dev, s));
-    OP_OK(pi_op_dense(W.w_uq, C, cw, n_tok, Q, qw, PI_ACT_NONE, qw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_uq, C, cw, n_tok, Q, qw, PI_ACT_NONE, qw, PI_ACT_NONE, s));
     OP_OK(pi_op_latent_attention_gated(Q, qw, cache, mask, W.w_uk, W.w_uv, W.sink, A.gated ? P + A.q_rank + H.kv_rank + R : nullptr, pw, PI_ACT_SIGMOID, A.gate_width, H.scale, H.heads, H.dim, R, H.vdim, H.kv_rank, W.rotary,
                                        A.pairing, ctx->pos_dev, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
     trace(ctx, "lat", (int) il, O, hv, n_tok);
-    OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
     return true;
 }
 static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
     llama_model * m = ctx->model;
     const pi_hparams & hp = m->hparams;
     hipStream_t s = ctx->stream;
-    const int width = hp.n_embd, ex = ctx->exact, nb = ctx->n_batch, ns = hp.streams;
+    const int width = hp.n_embd, nb = ctx->n_batch, ns = hp.streams;
     const float eps = hp.f_norm_rms_eps;
     const size_t n_layer = hp.hybrid.size();
     float * X = ctx->x, * N = ctx->nx, * Y = ctx->h_out, * P = ctx->h_in;
@@ -743,14 +762,14 @@ static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
             OP_OK(pi_op_hyper_step(X, (int64_t) ns * width, width, ns, Y, width, W.hc_mix[0], W.hc_out[0], W.hc_in[1], W.norm2, eps, width, n_tok, X, N, width, s));
             const int ff = H.ff;
             float * G = P + (size_t) nb * 2 * ff;
-            OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_SILU, ff, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_SILU, ff, PI_ACT_NONE, s));
             OP_OK(pi_op_glu_mul(P, 2 * (int64_t) ff, ff, n_tok, G, ff, s));
-            OP_OK(pi_op_dense(W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
             OP_OK(step_out(1));
         }
         trace(ctx, "lout", (int) il, X, (int64_t) ns * width, n_tok);
     }
-    OP_OK(pi_op_dense(m->output, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, m->output, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -765,25 +784,25 @@ static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
 static bool forward_diff_attention(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
     hipStream_t s = ctx->stream;
     const pi_gate_attention & A = H.left;
-    const int width = ctx->model->hparams.n_embd, ex = ctx->exact, nb = ctx->n_batch, ch = A.channels();
+    const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch, ch = A.channels();
     const int64_t pw = row_of_4(H.in_rows()), cw = row_of_4(ch), hd = (int64_t) A.heads * A.maps * A.dim, hv = (int64_t) A.heads * A.vdim, gd = (int64_t) A.kv_heads * A.maps * A.dim;
     float * P = ctx->h_in, * Q = ctx->h_att, * O = Q + (size_t) nb * hd, * C = O + (size_t) nb * hv;
     float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
-    OP_OK(pi_op_dense(W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
     const float * qkv = P; int64_t qs = pw;
     if (A.conv > 0) { OP_OK(pi_op_causal_conv(P, pw, ch, A.conv, W.conv_w, nullptr, ctx->rec_state + ctx->rec_off[il], ctx->rec_dev, n_tok, PI_ACT_NONE, C, cw, s)); qkv = C; qs = cw; }
     OP_OK(pi_op_qkv_prepare_maps(qkv, qkv + hd, qkv + hd + gd, qs, A.heads, A.kv_heads, A.maps, A.dim, A.vdim, W.rotary, A.pairing, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
     OP_OK(pi_op_diff_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, A.scale, A.chunk, A.keep_first, A.maps, W.lam, 1.0f - A.diff, ctx->model->hparams.f_norm_rms_eps, A.heads, A.kv_heads, A.dim, A.vdim, n_tok,
                                n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
     trace(ctx, "att", (int) il, O, hv, n_tok);
-    OP_OK(pi_op_dense(W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
     return true;
 }
 static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
     llama_model * m = ctx->model;
     const pi_hparams & hp = m->hparams;
     hipStream_t s = ctx->stream;
-    const int width = hp.n_embd, ex = ctx->exact, nb = ctx->n_batch;
+    const int width = hp.n_embd, nb = ctx->n_batch;
     const float eps = hp.f_norm_rms_eps;
     const size_t n_layer = hp.hybrid.size();
     float * x = ctx->x, * N = ctx->nx, * Y = ctx->h_out, * P = ctx->h_in;
@@ -815,13 +834,13 @@ static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
             const int ff = H.ff;
             float * G = P + (size_t) nb * 2 * ff;
             OP_OK(pi_op_residual_norm(x, Y, width, nullptr, W.norm2, eps, width, n_tok, x, N, width, s));
-            OP_OK(pi_op_dense(W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_NONE, 2 * (int64_t) ff, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_NONE, 2 * (int64_t) ff, PI_ACT_NONE, s));
             OP_OK(pi_op_glu_mul_ex(P, 2 * (int64_t) ff, ff, PI_GLU_CLIPPED, H.glu_limit, -1, n_tok, G, ff, s));
-            OP_OK(pi_op_dense(W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
         }
         OP_OK(step_to(il + 1, Y));
     }
-    OP_OK(pi_op_dense(m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -845,17 +864,17 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         const int64_t hd = (int64_t) H.heads * H.dim, hv = (int64_t) H.heads * H.vdim, pw = H.in_rows();
         if (H.mixer == PI_MIXER_LATENT_ATTENTION) {
             float * cache = ctx->lat_cache + ctx->lat_off[il];
-            OP_OK(pi_op_dense(W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, ex, s));                                               // q | W_dkv h
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));                                               // q | W_dkv h
             OP_OK(pi_op_rms_scale(P + hd, pw, W.mix_norm, 0.0f, eps, H.kv_rank, n_tok, nullptr, 0, nullptr, 0, 1.0f, cache, H.kv_rank, ctx->dyn_dev, 1, s));   // the latent, into its cell
             OP_OK(pi_op_latent_attention(P, pw, cache, ctx->mask_dev, W.w_uk, W.w_uv, W.sink, H.scale, H.heads, H.dim, H.vdim, H.kv_rank, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, A, hv, ctx->dyn_dev, s));
         } else {
             float * state = ctx->rec_state + ctx->rec_off[il];
-            OP_OK(pi_op_dense(W.w_in, x, width, n_tok, P, pw, PI_ACT_SILU, 2 * hd + hv, PI_ACT_SIGMOID, ex, s));                                   // silu(q | k | v) | sigmoid(g)
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_SILU, 2 * hd + hv, PI_ACT_SIGMOID, s));                                   // silu(q | k | v) | sigmoid(g)
             OP_OK(pi_op_linear_attention(P, P + hd, P + 2 * hd, pw, H.heads, H.dim, H.vdim, W.decay, state, ctx->rec_dev, n_tok, ctx->slots->size(), ctx->rec_scratch, ctx->rec_scratch_floats, A, hv, s));
             OP_OK(pi_op_rms_scale(A, hv, W.mix_norm, 0.0f, eps, (int) hv, n_tok, P + 2 * hd + hv, pw, nullptr, 0, 1.0f, A, hv, nullptr, 0, s));    // norm over all heads, * gate
         }
         trace(ctx, "mix", (int) il, A, hv, n_tok);
-        OP_OK(pi_op_dense(W.w_o, A, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, ex, s));
+        OP_OK(dense(ctx, W.w_o, A, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
         OP_OK(pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s));
         if (H.has_mlp) {
             OP_OK(pi_op_moe_route(W.router, W.correction, x, width, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s));
@@ -868,7 +887,7 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
     OP_OK(pi_op_rms_scale(x, width, m->output_norm, 1.0f, eps, width, n_tok, nullptr, 0, nullptr, 0, 1.0f, ctx->nx, width, nullptr, 0, s));
-    OP_OK(pi_op_dense(m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, ex, s));
+    OP_OK(dense(ctx, m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }

@@ -12,9 +12,11 @@
 //   k_dense_tile   serving precision, more tokens: tiles of 64 .. 256 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory and by the
 //                  latency of a step, large ones by the shared levels of memory: 850 TFLOP/s at 16384 x 4096 x 2048 tokens (128 x 128 tiles with a step's parts one after another: 710), 14 us for
 //                  2048 x 2048 x 512 (17)
+//   k_dense_async  the same from activations that are bfloat16 in memory (dense_async.h): what the engine's passes of more than 32 tokens take; k_round_bf16 makes such activations where no kernel ahead writes them
 //   k_embed        rows of the table gathered, widened and scaled
 #include "ops_common.h"
 #include "dense_tile.h"
+#include "dense_async.h"
 #include "kernel_timing.h"
 
 #include <algorithm>
@@ -270,6 +272,41 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
     }
 }
 
+// Tiles as k_dense_tile's, activations in bfloat16 (dense_async.h).  Rows in segments: as k_dense_rows, tiles inside a segment (blocks_of: tiles of rows to a segment; the last one takes the rest)
+template <int BN, int BT, int WN, int WT, int S>
+__global__ void __launch_bounds__(64 * WN * WT, WN * WT == 8 && BN * BT >= 32768 ? 2 : 1) k_dense_async(const uint16_t * __restrict__ W, int64_t K, int64_t N, const uint16_t * __restrict__ X, int64_t xs, int T, float * __restrict__ Y,
+                                                       int64_t ys, int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int blocks_of, int64_t seg_rows, int64_t seg_off, int seg_last, int tok_blocks, int tiles,
+                                                       const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 1)) return;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[DA_LDS_BYTES(BN, BT, S)];
+    const int tile = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int row_blocks = tiles / tok_blocks, grp = tile / (8 * tok_blocks), in_grp = tile % (8 * tok_blocks), gsz = min(8, row_blocks - 8 * grp), block = 8 * grp + in_grp % gsz;
+    const int seg = seg_rows > 0 ? min(block / blocks_of, seg_last) : 0;
+    const int64_t n0 = seg_rows > 0 ? seg * seg_rows + (int64_t) (block - seg * blocks_of) * BN : (int64_t) block * BN, n_end = seg_rows > 0 && seg < seg_last ? (seg + 1) * seg_rows : N;
+    const int t0 = (in_grp / gsz) * BT, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
+    da_tile<BN, BT, WN, WT, S>(W + n0 * K, [&](int r) { return (uint32_t) (min((int64_t) r, n_end - 1 - n0) * K * 2); }, X + seg * seg_off + (int64_t) t0 * xs, [&](int r) { return (uint32_t) ((int64_t) min(r, T - 1 - t0) * xs * 2); },
+                               (int) (K / 64), lds, acc);
+#pragma unroll
+    for (int b = 0; b < BT / WT / 16; b++) {
+        const int tok = t0 + (wave % WT) * (BT / WT) + b * 16 + (lane & 15);
+        if (tok >= T) continue;
+#pragma unroll
+        for (int a = 0; a < BN / WN / 16; a++) dn_store4(acc[a][b], n0 + (wave / WT) * (BN / WN) + a * 16 + (lane >> 4) * 4, n_end, tok, Y, ys, act_a, rows_a, act_b, bias);
+    }
+}
+
+// rows of fp32 values as bfloat16, nearest even: grid (2048 values, row), eight of a thread (n % 8 == 0)
+__global__ void __launch_bounds__(256) k_round_bf16(const float * __restrict__ x, int64_t xs, int64_t n, uint16_t * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    const int64_t i = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 8, t = blockIdx.y;
+    if (i >= n) return;
+    const dt_f32x4 lo = *(const dt_f32x4 *) (x + t * xs + i), hi = *(const dt_f32x4 *) (x + t * xs + i + 4);
+    if (pi_abort_late(gone, abort_w)) return;
+    *(dt_u32x4 *) (out + t * os + i) = dt_pack8(lo, hi);
+}
+
 extern "C" int pi_op_embed(const pi_weight * w, const int32_t * tokens, int n_tok, float scale, float * out, void * stream) {
     if (!w || w->type != PI_BF16) { pi_set_error("pi_op_embed: the table must be a bfloat16 weight"); return -1; }
     if (n_tok <= 0) return 0;
@@ -362,6 +399,64 @@ extern "C" int pi_op_dense_bias(const pi_weight * w, const float * bias, const f
     if (al16 && K >= 512) { if (exact) launch_rows<8, true>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); else launch_rows<8, false>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); }
     else if (al8)         { if (exact) launch_rows<4, true>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); else launch_rows<4, false>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); }
     else                  { if (exact) launch_rows<1, true>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); else launch_rows<1, false>(w, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, s, bytes, bias); }
+    PI_CHECK_LAUNCH(); return 0;
+}
+
+extern "C" int pi_op_round_bf16(const float * x, int64_t x_stride, int64_t n, int n_tok, uint16_t * out, int64_t out_stride, void * stream) {
+    if (n_tok <= 0 || n <= 0) return 0;
+    if (n % 8 || x_stride < n || out_stride < n || x_stride % 4 || out_stride % 8 || ((uintptr_t) x % 16) || ((uintptr_t) out % 16)) { pi_set_error("pi_op_round_bf16: rows of a multiple of 8 values, 16-byte aligned"); return -1; }
+    for (int t = 0; t < n_tok; t += 65535)                             // (rows are the grid's second dimension)
+        PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * n * n_tok, k_round_bf16, dim3((unsigned) ((n + 2047) / 2048), (unsigned) std::min(65535, n_tok - t)), dim3(256), 0, (hipStream_t) stream, x + (int64_t) t * x_stride, x_stride, n,
+                     out + (int64_t) t * out_stride, out_stride, pi_abort_word());
+    PI_CHECK_LAUNCH(); return 0;
+}
+// The tile that needs the least time, by rounds of 256 workgroups: 2.5 us + K / 2048 * rounds * the cost of one (us at K 2048 on weights from memory, measured over 1024 .. 32000 rows x 64 .. 2048 tokens):
+// 32 x 64 4.6, 64 x 64 6.3, 64 x 96 8.5, 128 x 128 19.5, 128 x 192 26, 128 x 256 31, 256 x 256 58.  Both sides of the crossings: 2048 x 2048 at 200 tokens 32 x 64 7.1, 64 x 64 8.2, at 333 9.0 / 8.7; at 700 64 x 64 13.2,
+// 64 x 96 10.5; 4096 x 4096 at 512 64 x 96 30.8, 128 x 128 34.6, at 1000 49.1 / 36.3; 12288 x 4096 at 200 64 x 64 46.6, 128 x 128 37.2, at 700 128 x 128 92, 128 x 192 77; 32000 x 1024 at 200 128 x 128 27.6, 128 x 256 21.2;
+// 32000 x 2048 at 512 128 x 192 79, 256 x 256 61
+static int async_tile_of(int64_t rows, int64_t K, int n_tok, int64_t seg_rows, int n_seg, int & row_blocks, int & tok_blocks, int & blocks_of) {
+    static const struct { int bn, bt; double us; } shape[] = { { 32, 64, 4.6 }, { 64, 64, 6.3 }, { 64, 96, 8.5 }, { 128, 128, 19.5 }, { 128, 192, 26.0 }, { 128, 256, 31.0 }, { 256, 256, 58.0 } };
+    int best = 0; double least = 1e30;
+    for (int i = 0; i < 7; i++) {
+        const int64_t seg_blocks = seg_rows > 0 ? (seg_rows + shape[i].bn - 1) / shape[i].bn : 0, blocks = seg_rows > 0 ? (n_seg - 1) * seg_blocks + (rows - (n_seg - 1) * seg_rows + shape[i].bn - 1) / shape[i].bn : (rows + shape[i].bn - 1) / shape[i].bn;
+        const int64_t toks = (n_tok + shape[i].bt - 1) / shape[i].bt, tiles = blocks * toks;
+        if (tiles > INT32_MAX / 2) continue;
+        const double cost = 2.5 + (double) K / 2048 * (double) ((tiles + 255) / 256) * shape[i].us;
+        if (cost < least) { least = cost; best = i; row_blocks = (int) blocks; tok_blocks = (int) toks; blocks_of = (int) seg_blocks; }
+    }
+    return best;
+}
+// whether a pass takes the products of bfloat16 activations: more tokens than the kernels that share K out take, whole steps of K, offsets inside a tile in 32 bits
+extern "C" int pi_op_dense_rounded_ok(const pi_weight * w, int64_t x_stride, int n_tok) {
+    return w && w->type == PI_BF16 && n_tok > 1 && !dense_takes_split(w->ne1, n_tok) && w->ne0 > 0 && w->ne0 % 64 == 0 && ((uintptr_t) w->p0 % 16) == 0 && w->ne0 < (1 << 22) && x_stride < (1 << 22) && w->ne1 <= INT32_MAX;
+}
+// x: bfloat16 rows.  n_seg > 1: rows of the matrix in segments of seg_rows, each with an input of its own, x + g * seg_off (pi_op_dense_segments), in one launch
+extern "C" int pi_op_dense_rounded(const pi_weight * w, const float * bias, const uint16_t * x, int64_t x_stride, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out, int64_t out_stride, int act_a, int64_t rows_a,
+                                   int act_b, void * stream) {
+    if (!w || w->type != PI_BF16) { pi_set_error("pi_op_dense_rounded: the weight must be bfloat16"); return -1; }
+    if (n_tok <= 0 || w->ne1 <= 0) return 0;
+    if (n_seg < 1 || (n_seg > 1 && (seg_rows < 1 || (int64_t) (n_seg - 1) * seg_rows >= w->ne1 || seg_rows % 4))) { pi_set_error("pi_op_dense_rounded: %d segments of %lld rows do not fit %lld rows", n_seg, (long long) seg_rows, (long long) w->ne1); return -1; }
+    if (n_seg == 1) seg_rows = seg_off = 0;
+    if (x_stride < (int64_t) (n_seg - 1) * seg_off + w->ne0 || out_stride < w->ne1) { pi_set_error("pi_op_dense_rounded: row strides (%lld, %lld) below the sizes (%lld, %lld)", (long long) x_stride, (long long) out_stride, (long long) w->ne0, (long long) w->ne1); return -1; }
+    if (w->ne0 % 64 || ((uintptr_t) w->p0 % 16) || ((uintptr_t) x % 16) || x_stride % 8 || seg_off % 8 || seg_off < 0 || w->ne0 >= (1 << 22) || x_stride >= (1 << 22) || w->ne1 > INT32_MAX) {
+        pi_set_error("pi_op_dense_rounded: rows of whole steps of 64 values, 16-byte aligned, of less than 2^22 values"); return -1;
+    }
+    hipStream_t s = (hipStream_t) stream;
+    int row_blocks = 0, tok_blocks = 0, blocks_of = 0;
+    const int which = async_tile_of(w->ne1, w->ne0, n_tok, seg_rows, n_seg, row_blocks, tok_blocks, blocks_of), tiles = row_blocks * tok_blocks;
+    const double bytes = 2.0 * w->ne0 * w->ne1 + 2.0 * n_tok * n_seg * w->ne0 + 4.0 * n_tok * w->ne1;
+#define DN_ASYNC(BN, BT, WN, WT, S) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_async<BN, BT, WN, WT, S>), dim3((unsigned) ((tiles + 7) / 8 * 8)), dim3(64 * WN * WT), 0, s, \
+                     (const uint16_t *) w->p0, w->ne0, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, blocks_of, seg_rows, seg_off, n_seg - 1, tok_blocks, tiles, pi_abort_word())
+    switch (which) {
+        case 0:  DN_ASYNC(32, 64, 2, 2, 4); break;
+        case 1:  DN_ASYNC(64, 64, 4, 2, 4); break;
+        case 2:  DN_ASYNC(64, 96, 2, 2, 4); break;
+        case 3:  DN_ASYNC(128, 128, 4, 2, 4); break;
+        case 4:  DN_ASYNC(128, 192, 2, 4, 3); break;
+        case 5:  DN_ASYNC(128, 256, 2, 4, 3); break;
+        default: DN_ASYNC(256, 256, 4, 2, 2);
+    }
+#undef DN_ASYNC
     PI_CHECK_LAUNCH(); return 0;
 }
 

@@ -572,6 +572,7 @@ extern "C" int pi_op_prefetch(const void * p, size_t bytes, int workgroups, void
 }
 extern "C" const void * pi_weight_data(const pi_weight * w) { return w->base; }
 extern "C" int pi_weight_type(const pi_weight * w) { return w->type; }
+extern "C" int64_t pi_weight_columns(const pi_weight * w) { return w->ne0; }
 
 extern "C" int pi_vec_dot_type(int t) {
     switch (t) {
