@@ -290,7 +290,12 @@ PI_API int pi_op_embed_pair(const pi_weight * table, const int32_t * tokens_dev,
 PI_API int pi_op_dense_segments(const pi_weight * w, const float * x_dev, int64_t x_stride, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out_dev, int64_t out_stride, int act_a, int64_t rows_a,
                                 int act_b, int exact, void * stream);
 /* the same products from activations that are bfloat16 in memory (what serving precision rounds them to anyway), for passes of more tokens than the kernels that share K out take: pi_op_dense_rounded_ok says for which; n_seg > 1:
- * segments as above, in one launch.  pi_op_round_bf16: rows of fp32 values rounded to nearest even (n % 8 == 0, 16-byte aligned rows) */
+ * segments as above, in one launch.  pi_op_round_bf16: rows of fp32 values rounded to nearest even (n % 8 == 0, 16-byte aligned rows of out) */
+/* Where an operator's result is such an input, the operator itself can write the rounded values: pi_set_rounded_output names a place for columns [from, from + n) of the next operator's rows (h, 16-byte aligned rows of `stride`
+ * values, n % 8 == 0) on the calling thread, only: nobody reads the fp32 result.  pi_rounded_output_written takes the request back and says whether the operator has met it (1; then, with `only`, the fp32 result may not be there) or
+ * not (0: it wrote fp32 alone).  Met by the norms, gates, embeddings, token shifts, prompt attentions and dense products of passes that pi_op_dense_rounded takes */
+PI_API void pi_set_rounded_output(uint16_t * h_dev, int64_t stride, int64_t from, int64_t n, int only);
+PI_API int pi_rounded_output_written(void);
 PI_API int pi_op_round_bf16(const float * x_dev, int64_t x_stride, int64_t n, int n_tok, uint16_t * out_dev, int64_t out_stride, void * stream);
 PI_API int pi_op_dense_rounded_ok(const pi_weight * w, int64_t x_stride, int n_tok);
 PI_API int pi_op_dense_rounded(const pi_weight * w, const float * bias_dev, const uint16_t * x_dev, int64_t x_stride, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out_dev, int64_t out_stride, int act_a,

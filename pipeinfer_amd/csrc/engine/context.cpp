@@ -110,7 +110,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) { err = "hipStreamCreate failed"; return false; }
     auto dev = [&](size_t bytes) -> void * { void * p = pi_malloc(std::max<size_t>(bytes, 16)); if (!p) err = pi_last_error(); return p; };
     const int nb = ctx->n_batch, width = hp.n_embd;
-    size_t lat = 0, rec = 0, in_w = 1, att_w = 1, up_w = 1, sel_w = 1, idx_n = 1, step_w = 0; bool positions = false;
+    size_t lat = 0, rec = 0, in_w = 1, att_w = 1, up_w = 1, sel_w = 1, idx_n = 1, step_w = 0, mid_w = 0; bool positions = false;
     ctx->lat_off.assign(hp.hybrid.size(), 0); ctx->rec_off.assign(hp.hybrid.size(), 0);
     if (hp.n_recurrent() > 0 || hp.pair_buckets > 0) ctx->slots.reset(new state_slots(std::max(1, ctx->n_state_slots)));      // (the previous token of a pair embedding is per-sequence state as well)
     for (size_t i = 0; i < hp.hybrid.size(); i++) {
@@ -138,13 +138,13 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
         if (H.mixer == PI_MIXER_CHANNEL_DELTA || H.mixer == PI_MIXER_PARALLEL_SHIFT) {        // scratch rows as forward_post_norm_blocks lays them out
             if (H.mixer == PI_MIXER_CHANNEL_DELTA) {
                 const pi_channel_delta & D = H.delta;
-                in_w = std::max(in_w, (size_t) D.in_rows());
+                in_w = std::max(in_w, (size_t) D.in_rows()); mid_w = std::max(mid_w, (size_t) D.decay_rank + (size_t) std::max(D.decay_rank, D.gate_rank));
                 att_w = std::max(att_w, (size_t) D.channels() + (size_t) D.heads * D.dim + (size_t) 2 * D.heads * D.vdim);
                 ctx->rec_scratch_floats = std::max(ctx->rec_scratch_floats, pi_op_channel_recurrence_scratch_floats(D.heads, D.dim, D.vdim, nb, ctx->slots->size()));
             } else {
                 const pi_gate_attention & A = H.left; const pi_time_mix & R = H.shift;
                 ctx->lat_off[i] = lat; lat += (size_t) ctx->n_ctx * H.cell_floats();
-                in_w = std::max(in_w, (size_t) A.in_rows() + (size_t) 5 * width);
+                in_w = std::max(in_w, (size_t) A.in_rows() + (size_t) 5 * width); mid_w = std::max(mid_w, (size_t) R.decay_rank);
                 att_w = std::max(att_w, (size_t) A.heads * (A.dim + A.vdim) + (size_t) 7 * R.inner() + (size_t) R.decay_rank);
                 ctx->rec_scratch_floats = std::max(ctx->rec_scratch_floats, pi_op_channel_recurrence_scratch_floats(R.heads, R.dim, R.dim, nb, ctx->slots->size()));
                 ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_window_attention_scratch_floats(A.heads, A.vdim, nb));
@@ -186,6 +186,8 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
         in_w = std::max(in_w, (size_t) H.in_rows()); att_w = std::max(att_w, (size_t) H.heads * H.vdim);
         if (H.has_mlp) { up_w = std::max(up_w, (size_t) H.top * std::max(H.ff, 1)); sel_w = std::max(sel_w, (size_t) H.top); idx_n = std::max(idx_n, pi_op_moe_grouped_index_ints(nb, H.top, H.n_expert)); }
     }
+    ctx->act_h_row = (std::max(std::max(in_w, att_w), (size_t) 2 * width) + 7) / 8 * 8;
+    const size_t x_w = ((size_t) width + 7) / 8 * 8; mid_w = (mid_w + 7) / 8 * 8;      // (act_h | x_h | mid_h in one allocation)
     if (!(ctx->rec_scratch = (float *) dev(ctx->rec_scratch_floats * 4)) || !(ctx->lat_scratch = (float *) dev(ctx->lat_scratch_floats * 4)) || !(ctx->lat_cache = (float *) dev(lat * 4)) || !(ctx->rec_state = (float *) dev(rec * 4))) return false;
     pi_memset(ctx->lat_cache, 0, std::max<size_t>(lat * 4, 16), nullptr); pi_memset(ctx->rec_state, 0, std::max<size_t>(rec * 4, 16), nullptr);
     if (positions) { if (!(ctx->cell_pos = (int32_t *) dev((size_t) 4 * ctx->n_ctx)) || !(ctx->h_out2 = (float *) dev((size_t) 4 * nb * width)) || !(ctx->ssd_dt = (float *) dev((size_t) 4 * nb * step_w))) return false; pi_memset(ctx->cell_pos, 0, (size_t) 4 * ctx->n_ctx, nullptr); }
@@ -199,9 +201,10 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
     if (!(ctx->x = (float *) dev((size_t) 4 * nb * width * std::max(1, hp.streams))) || !(ctx->nx = (float *) dev((size_t) 4 * nb * width)) || !(ctx->h_out = (float *) dev((size_t) 4 * nb * width)) ||
         !(ctx->h_in = (float *) dev((size_t) 4 * nb * in_w)) || !(ctx->h_att = (float *) dev((size_t) 4 * nb * att_w)) || !(ctx->moe_up = (float *) dev((size_t) 4 * nb * up_w)) ||
         !(ctx->moe_w = (float *) dev((size_t) 4 * nb * sel_w)) || !(ctx->moe_dn = (float *) dev((size_t) 4 * nb * sel_w * width)) || !(ctx->moe_idx = (int32_t *) dev((size_t) 4 * idx_n)) || !(ctx->moe_sel = (int32_t *) dev((size_t) 4 * nb * sel_w)) || (ctx->slots && !(ctx->rec_dev = (int32_t *) dev((size_t) 4 * nb))) || (hp.pair_buckets > 0 && !(ctx->pair_dev = (int32_t *) dev((size_t) 4 * nb))) ||
-        !(ctx->act_h = (uint16_t *) dev((size_t) 2 * nb * (ctx->act_h_row = std::max(std::max(in_w, att_w), (size_t) 2 * width)))) ||
+        !(ctx->act_h = (uint16_t *) dev((size_t) 2 * nb * (ctx->act_h_row + x_w + mid_w))) ||
         !(ctx->tokens_dev = (int32_t *) dev((size_t) 4 * nb)) || !(ctx->pos_dev = (int32_t *) dev((size_t) 4 * nb)) || !(ctx->dyn_dev = (int32_t *) dev((size_t) 4 * (4 + 2 * nb))))
         return false;
+    ctx->x_h = ctx->act_h + (size_t) nb * ctx->act_h_row; ctx->mid_h = ctx->x_h + (size_t) nb * x_w;
     {   // abort word + cancel flags + the control stream cancels travel on
         if (!(ctx->abort_dev = (int32_t *) dev(256))) return false;
         pi_memset(ctx->abort_dev, 0, 256, nullptr);
@@ -383,8 +386,7 @@ static bool mul_mat_grouped(int n, const pi_weight * const * ws, const void * co
 static int dense_segments(llama_context * ctx, const pi_weight * w, const float * x, int64_t xs, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s,
                           const uint16_t * xh = nullptr, int64_t xhs = 0, const float * bias = nullptr) {
     const int64_t n = (n_seg - 1) * seg_off + pi_weight_columns(w), hs = xh ? xhs : n;
-    const bool whole = xh || (xs % 4 == 0 && (uintptr_t) x % 16 == 0 && n % 8 == 0 && (size_t) n <= ctx->act_h_row);
-    if (ctx->exact || !whole || (n_seg > 1 && (seg_off % 8 || seg_rows % 4)) || !pi_op_dense_rounded_ok(w, hs, n_tok))
+    if (!xh && (ctx->exact || n % 8 || (size_t) n > ctx->act_h_row || (n_seg > 1 && (seg_off % 8 || seg_rows % 4)) || !pi_op_dense_rounded_ok(w, hs, n_tok)))      // (with xh: x may not be there)
         return n_seg > 1 ? pi_op_dense_segments(w, x, xs, seg_rows, seg_off, n_seg, n_tok, out, os, act_a, rows_a, act_b, ctx->exact, s) : pi_op_dense_bias(w, bias, x, xs, n_tok, out, os, act_a, rows_a, act_b, ctx->exact, s);
     if (!xh) {
         if (pi_op_round_bf16(x, xs, n, n_tok, ctx->act_h, n, s) != 0) return -1;
@@ -394,6 +396,17 @@ static int dense_segments(llama_context * ctx, const pi_weight * w, const float 
 }
 static int dense(llama_context * ctx, const pi_weight * w, const float * x, int64_t xs, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s, const uint16_t * xh = nullptr, int64_t xhs = 0, const float * bias = nullptr) {
     return dense_segments(ctx, w, x, xs, 0, 0, 1, n_tok, out, os, act_a, rows_a, act_b, s, xh, xhs, bias);
+}
+
+// h where the product of a pass of n_tok tokens with w reads bfloat16 (the operator ahead then writes it there, op_rounded), else null
+static uint16_t * reads_rounded(const llama_context * ctx, const pi_weight * w, int n_tok, uint16_t * h) { return !ctx->exact && w && pi_op_dense_rounded_ok(w, pi_weight_columns(w), n_tok) ? h : nullptr; }
+// an operator whose columns [from, from + n) of out the next product reads in bfloat16 (h null: in fp32); only: nobody reads them in fp32
+template <class Op>
+static int op_rounded(llama_context * ctx, uint16_t * h, const float * out, int64_t out_stride, int64_t from, int64_t n, int n_tok, bool only, hipStream_t s, Op op) {
+    if (!h) return op();
+    pi_set_rounded_output(h, n, from, n, only && !trace_enabled());
+    const int rc = op();
+    return !pi_rounded_output_written() && rc == 0 ? pi_op_round_bf16(out + from, out_stride, n, n_tok, h, n, s) : rc;
 }
 
 // A hybrid model's pass: per layer  x += m * N1(mixer(x)),  x += m * N2(moe(x))  — the norm sits on the sublayer's output, the sublayers read x itself; everything between the
@@ -512,31 +525,39 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
     const float eps = hp.f_norm_rms_eps, alpha = hp.post_alpha;
     const size_t n_layer = hp.hybrid.size();
     float * x = ctx->x, * P = ctx->h_in, * A = ctx->h_att, * Y = ctx->h_out, * Y2 = ctx->h_out2;
-    if (m->pair_embd) OP_OK(pi_op_embed_pair(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, m->pair_embd, ctx->pair_dev, x, s));
-    else OP_OK(pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s));
+    // the stream in bfloat16, where the next projection reads it so (behind the last sublayer: its final norm, for the head)
+    auto x_rounded = [&](size_t il) { return reads_rounded(ctx, il < n_layer ? m->hweights[(size_t) hp.hybrid[il].weights].w_in : m->output, n_tok, ctx->x_h); };
+    uint16_t * xh = x_rounded(0);
+    OP_OK(op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] {
+        return m->pair_embd ? pi_op_embed_pair(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, m->pair_embd, ctx->pair_dev, x, s) : pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s);
+    }));
     for (size_t il = 0; il < n_layer; il++) {
         const pi_hybrid_layer & H = hp.hybrid[il];
         const pi_hybrid_weights & W = m->hweights[(size_t) H.weights];
         const bool last_sub_is_mixer = il + 1 == n_layer && !H.has_mlp;
         const float * ya = Y, * yb = nullptr;
+        uint16_t * oh = reads_rounded(ctx, W.w_o, n_tok, ctx->act_h);
         if (H.mixer == PI_MIXER_CHANNEL_DELTA) {
             const pi_channel_delta & D = H.delta;
             const int64_t pw = D.in_rows(), gd = (int64_t) D.kv_heads * D.dim, hd = (int64_t) D.heads * D.dim, hv = (int64_t) D.heads * D.vdim, ch = D.channels();
             const int64_t aw = hd + hv;                                                                // a token's row of [raw decays | raw gate]
             float * C = A, * A2 = C + (size_t) nb * ch, * G2 = A2 + hd, * O = A2 + (size_t) nb * aw;
             float * S = ctx->rec_state + ctx->rec_off[il], * conv_state = S + (size_t) n_slots * D.matrix_floats();
-            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
+            // (the inputs of both low-rank projections, side by side in a row of P, in bfloat16 as well)
+            const int64_t lw = W.w_g2 ? (int64_t) D.decay_rank + D.gate_rank : 2 * (int64_t) D.decay_rank;
+            uint16_t * lh = xh && ch % 8 == 0 && D.decay_rank % 8 == 0 && lw % 8 == 0 && pw % 4 == 0 && hd % 4 == 0 && reads_rounded(ctx, W.w_a2, n_tok, ctx->mid_h) && (!W.w_g2 || reads_rounded(ctx, W.w_g2, n_tok, ctx->mid_h)) ? ctx->mid_h : nullptr;
+            OP_OK(op_rounded(ctx, lh, P, pw, ch, lw, n_tok, false, s, [&] { return dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, xh, width); }));
             OP_OK(pi_op_causal_conv(P, pw, (int) ch, D.conv, W.conv_w, nullptr, conv_state, ctx->rec_dev, n_tok, PI_ACT_SILU, C, ch, s));
-            if (!W.w_g2) OP_OK(dense_segments(ctx, W.w_a2, P + ch, pw, hd, D.decay_rank, 2, n_tok, A2, aw, PI_ACT_NONE, aw, PI_ACT_NONE, s));
+            if (!W.w_g2) OP_OK(dense_segments(ctx, W.w_a2, P + ch, pw, hd, D.decay_rank, 2, n_tok, A2, aw, PI_ACT_NONE, aw, PI_ACT_NONE, s, lh, lw));
             else {
-                OP_OK(dense(ctx, W.w_a2, P + ch, pw, n_tok, A2, aw, PI_ACT_NONE, hd, PI_ACT_NONE, s));
-                OP_OK(dense(ctx, W.w_g2, P + ch + D.decay_rank, pw, n_tok, G2, aw, PI_ACT_NONE, hv, PI_ACT_NONE, s));
+                OP_OK(dense(ctx, W.w_a2, P + ch, pw, n_tok, A2, aw, PI_ACT_NONE, hd, PI_ACT_NONE, s, lh, lw));
+                OP_OK(dense(ctx, W.w_g2, P + ch + D.decay_rank, pw, n_tok, G2, aw, PI_ACT_NONE, hv, PI_ACT_NONE, s, lh ? lh + D.decay_rank : nullptr, lw));
             }
             OP_OK(pi_op_channel_recurrence(PI_RULE_DELTA, C, ch, C + gd, ch, C + 2 * gd, ch, A2, aw, 2, W.dt_bias, W.a_log, P + ch + D.decay_rank + D.gate_rank, pw, nullptr, 1, 1.0f / sqrtf((float) D.dim), D.heads, D.kv_heads, D.dim, D.vdim,
                                            S, ctx->rec_dev, n_tok, n_slots, ctx->rec_scratch, ctx->rec_scratch_floats, O, hv, s));
             trace(ctx, "rec", (int) il, O, hv, n_tok);
-            OP_OK(pi_op_head_norm_gate(O, hv, D.heads, D.vdim, W.mix_norm, 0, G2, aw, PI_ACT_SIGMOID, eps, n_tok, O, hv, s));
-            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+            OP_OK(op_rounded(ctx, oh, O, hv, 0, hv, n_tok, true, s, [&] { return pi_op_head_norm_gate(O, hv, D.heads, D.vdim, W.mix_norm, 0, G2, aw, PI_ACT_SIGMOID, eps, n_tok, O, hv, s); }));
+            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, oh, hv));
         } else if (H.mixer == PI_MIXER_PARALLEL_SHIFT) {
             const pi_gate_attention & L = H.left; const pi_time_mix & R = H.shift;
             const int64_t pw = L.in_rows(), hd = (int64_t) L.heads * L.dim, hv = (int64_t) L.heads * L.vdim, gd = (int64_t) L.kv_heads * L.dim, inner = R.inner(), mw = (int64_t) 5 * width;
@@ -546,36 +567,50 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
             float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
             float * S = ctx->rec_state + ctx->rec_off[il], * shift_state = S + (size_t) n_slots * R.matrix_floats();
             // attention branch
-            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, xh, width));
             OP_OK(pi_op_qkv_prepare_ex(P, P + hd, P + hd + gd, pw, nullptr, nullptr, eps, L.heads, L.kv_heads, L.dim, L.vdim, W.rotary, 0, PI_PAIR_NEIGHBOURS, 0, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
-            OP_OK(pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, nullptr, 0, PI_ACT_NONE, L.scale, 1.0f, L.weights, L.softcap, PI_MASK_CHUNK, L.chunk, 0, 0, 0, L.heads, L.kv_heads, L.dim,
-                                         L.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
+            OP_OK(op_rounded(ctx, oh, O, hv, 0, hv, n_tok, true, s, [&] {
+                return pi_op_window_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, nullptr, nullptr, nullptr, 0, PI_ACT_NONE, L.scale, 1.0f, L.weights, L.softcap, PI_MASK_CHUNK, L.chunk, 0, 0, 0, L.heads, L.kv_heads, L.dim,
+                                              L.vdim, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s);
+            }));
             trace(ctx, "att", (int) il, O, hv, n_tok);
-            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+            OP_OK(dense(ctx, W.w_o, O, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, oh, hv));
             // time-mix branch
-            OP_OK(pi_op_token_shift(x, width, width, W.mu, 5, shift_state, ctx->rec_dev, n_tok, M, mw, s));
+            uint16_t * mh = width % 8 == 0 && inner % 4 == 0 ? reads_rounded(ctx, W.w_r, n_tok, ctx->act_h) : nullptr;
+            uint16_t * dh = mh && R.decay_rank % 8 == 0 ? reads_rounded(ctx, W.w_w2, n_tok, ctx->mid_h) : nullptr;
+            OP_OK(op_rounded(ctx, mh, M, mw, 0, mw, n_tok, true, s, [&] { return pi_op_token_shift(x, width, width, W.mu, 5, shift_state, ctx->rec_dev, n_tok, M, mw, s); }));
             // r | k | v | g | w1 from their own mixes: rows of ONE matrix in five segments; tanh on w1's rows, the gate's silu waits for the head norm
-            OP_OK(dense_segments(ctx, W.w_r, M, mw, inner, width, 5, n_tok, RK, rkw, PI_ACT_NONE, 4 * inner, PI_ACT_TANH, s));
-            OP_OK(dense(ctx, W.w_w2, RK + 4 * inner, rkw, n_tok, WD, inner, PI_ACT_NONE, inner, PI_ACT_NONE, s));
+            OP_OK(op_rounded(ctx, dh, RK, rkw, 4 * inner, R.decay_rank, n_tok, false, s, [&] { return dense_segments(ctx, W.w_r, M, mw, inner, width, 5, n_tok, RK, rkw, PI_ACT_NONE, 4 * inner, PI_ACT_TANH, s, mh, mw); }));
+            OP_OK(dense(ctx, W.w_w2, RK + 4 * inner, rkw, n_tok, WD, inner, PI_ACT_NONE, inner, PI_ACT_NONE, s, dh, R.decay_rank));
             OP_OK(pi_op_channel_recurrence(PI_RULE_BONUS, RK, rkw, RK + inner, rkw, RK + 2 * inner, rkw, WD, inner, 1, W.w0, nullptr, nullptr, 0, W.bonus, 0, 1.0f, R.heads, R.heads, R.dim, R.dim,
                                            S, ctx->rec_dev, n_tok, n_slots, ctx->rec_scratch, ctx->rec_scratch_floats, O2, inner, s));
             trace(ctx, "rec", (int) il, O2, inner, n_tok);
-            OP_OK(pi_op_head_norm_gate(O2, inner, R.heads, R.dim, W.mix_norm, 1, RK + 3 * inner, rkw, PI_ACT_SILU, eps, n_tok, O2, inner, s));
-            OP_OK(dense(ctx, W.w_o2, O2, inner, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+            uint16_t * o2h = reads_rounded(ctx, W.w_o2, n_tok, ctx->act_h);
+            OP_OK(op_rounded(ctx, o2h, O2, inner, 0, inner, n_tok, true, s, [&] { return pi_op_head_norm_gate(O2, inner, R.heads, R.dim, W.mix_norm, 1, RK + 3 * inner, rkw, PI_ACT_SILU, eps, n_tok, O2, inner, s); }));
+            OP_OK(dense(ctx, W.w_o2, O2, inner, n_tok, Y2, width, PI_ACT_NONE, width, PI_ACT_NONE, s, o2h, inner));
             yb = Y2;
         } else { ctx->last_error = "blocks with the norm after the sum are built for the channel-delta and the attention + time-mix mixers"; return false; }
-        OP_OK(pi_op_rms_post(ya, width, W.left_out, yb, width, W.right_out, 0.5f, W.ls1, x, width, alpha, W.norm1, eps, width, n_tok, x, width, last_sub_is_mixer ? m->output_norm : nullptr, ctx->nx, width, s));
+        // (behind the sublayer that ends the model the rounded row is the final norm's)
+        uint16_t * uh = H.has_mlp ? reads_rounded(ctx, W.ff_up, n_tok, ctx->x_h) : nullptr;
+        xh = x_rounded(il + 1);
+        OP_OK(op_rounded(ctx, H.has_mlp ? uh : xh, last_sub_is_mixer ? ctx->nx : x, width, 0, width, n_tok, last_sub_is_mixer, s, [&] {
+            return pi_op_rms_post(ya, width, W.left_out, yb, width, W.right_out, 0.5f, W.ls1, x, width, alpha, W.norm1, eps, width, n_tok, x, width, last_sub_is_mixer ? m->output_norm : nullptr, ctx->nx, width, s);
+        }));
         if (H.has_mlp) {
             const int ff = H.ff;
             float * G = P + (size_t) nb * 2 * ff;
-            OP_OK(dense(ctx, W.ff_up, x, width, n_tok, P, 2 * ff, PI_ACT_GELU_TANH, ff, PI_ACT_NONE, s));        // gelu(gate) | up
-            OP_OK(pi_op_glu_mul(P, 2 * ff, ff, n_tok, G, ff, s));
-            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
-            OP_OK(pi_op_rms_post(Y, width, nullptr, nullptr, 0, nullptr, 1.0f, W.ls2, x, width, alpha, W.norm2, eps, width, n_tok, x, width, il + 1 == n_layer ? m->output_norm : nullptr, ctx->nx, width, s));
+            uint16_t * gh = reads_rounded(ctx, W.ff_down, n_tok, ctx->act_h);
+            const bool last = il + 1 == n_layer;
+            OP_OK(dense(ctx, W.ff_up, x, width, n_tok, P, 2 * ff, PI_ACT_GELU_TANH, ff, PI_ACT_NONE, s, uh, width));        // gelu(gate) | up
+            OP_OK(op_rounded(ctx, gh, G, ff, 0, ff, n_tok, true, s, [&] { return pi_op_glu_mul(P, 2 * ff, ff, n_tok, G, ff, s); }));
+            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, gh, ff));
+            OP_OK(op_rounded(ctx, xh, last ? ctx->nx : x, width, 0, width, n_tok, last, s, [&] {
+                return pi_op_rms_post(Y, width, nullptr, nullptr, 0, nullptr, 1.0f, W.ls2, x, width, alpha, W.norm2, eps, width, n_tok, x, width, last ? m->output_norm : nullptr, ctx->nx, width, s);
+            }));
         }
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    OP_OK(dense(ctx, m->output, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
+    OP_OK(dense(ctx, m->output, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, xh, width));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -711,7 +746,7 @@ static bool forward_temp_attention(llama_context * ctx, const pi_hybrid_layer & 
     OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
     return true;
 }
-static bool forward_query_latent(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
+static bool forward_query_latent(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, const uint16_t * Nh, int n_tok, int n_kv) {
     hipStream_t s = ctx->stream;
     const pi_latent & A = H.latent;
     const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch, R = A.rot_dim;
@@ -719,13 +754,18 @@ static bool forward_query_latent(llama_context * ctx, const pi_hybrid_layer & H,
     float * P = ctx->h_in, * C = ctx->h_att, * Q = C + (size_t) nb * cw, * O = Q + (size_t) nb * qw;
     float * cache = ctx->lat_cache + ctx->lat_off[il];
     const uint32_t * mask = A.window > 0 ? ctx->window_masks.at(A.window) : ctx->mask_dev;
-    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
-    OP_OK(pi_op_latent_prepare_ex(P, pw, A.q_rank, W.q_norm, H.kv_rank, W.mix_norm, R, W.rotary, A.pairing, ctx->model->hparams.f_norm_rms_eps, ctx->pos_dev, n_tok, C, cw, cache, ctx->dyn_dev, s));
-    OP_OK(dense(ctx, W.w_uq, C, cw, n_tok, Q, qw, PI_ACT_NONE, qw, PI_ACT_NONE, s));
-    OP_OK(pi_op_latent_attention_gated(Q, qw, cache, mask, W.w_uk, W.w_uv, W.sink, A.gated ? P + A.q_rank + H.kv_rank + R : nullptr, pw, PI_ACT_SIGMOID, A.gate_width, H.scale, H.heads, H.dim, R, H.vdim, H.kv_rank, W.rotary,
-                                       A.pairing, ctx->pos_dev, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
+    uint16_t * ch = reads_rounded(ctx, W.w_uq, n_tok, ctx->act_h), * oh = reads_rounded(ctx, W.w_o, n_tok, ctx->act_h);
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, Nh, width));
+    OP_OK(op_rounded(ctx, ch, C, cw, 0, A.q_rank, n_tok, true, s, [&] {
+        return pi_op_latent_prepare_ex(P, pw, A.q_rank, W.q_norm, H.kv_rank, W.mix_norm, R, W.rotary, A.pairing, ctx->model->hparams.f_norm_rms_eps, ctx->pos_dev, n_tok, C, cw, cache, ctx->dyn_dev, s);
+    }));
+    OP_OK(dense(ctx, W.w_uq, C, cw, n_tok, Q, qw, PI_ACT_NONE, qw, PI_ACT_NONE, s, ch, A.q_rank));
+    OP_OK(op_rounded(ctx, oh, O, hv, 0, hv, n_tok, true, s, [&] {
+        return pi_op_latent_attention_gated(Q, qw, cache, mask, W.w_uk, W.w_uv, W.sink, A.gated ? P + A.q_rank + H.kv_rank + R : nullptr, pw, PI_ACT_SIGMOID, A.gate_width, H.scale, H.heads, H.dim, R, H.vdim, H.kv_rank, W.rotary,
+                                            A.pairing, ctx->pos_dev, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s);
+    }));
     trace(ctx, "lat", (int) il, O, hv, n_tok);
-    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s, oh, hv));
     return true;
 }
 static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
@@ -753,7 +793,7 @@ static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
         switch (H.mixer) {
             case PI_MIXER_MEMORY:           ok = forward_memory(ctx, H, W, il, N, n_tok); break;
             case PI_MIXER_WINDOW_ATTENTION: ok = forward_temp_attention(ctx, H, W, il, N, n_tok, n_kv); break;
-            case PI_MIXER_LATENT_ATTENTION: ok = forward_query_latent(ctx, H, W, il, N, n_tok, n_kv); break;
+            case PI_MIXER_LATENT_ATTENTION: ok = forward_query_latent(ctx, H, W, il, N, nullptr, n_tok, n_kv); break;
             default: ctx->last_error = "blocks over residual streams are built for the matrix-memory, attention and latent-attention mixers";
         }
         if (!ok) return false;
@@ -781,21 +821,25 @@ static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
 //   latent attention         forward_query_latent, with a sink and a gate per output value
 //   feed-forward             [gate | up] -> clipped product -> down
 // A sublayer ends in ONE row kernel (pi_op_residual_norm): the sum (with the pass's vector where the next layer opens one) and the norm of what reads it next; behind the last one the model's norm.
-static bool forward_diff_attention(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, int n_tok, int n_kv) {
+// (N: the normed stream; Nh: in bfloat16, where the projection reads it so)
+static bool forward_diff_attention(llama_context * ctx, const pi_hybrid_layer & H, const pi_hybrid_weights & W, size_t il, const float * N, const uint16_t * Nh, int n_tok, int n_kv) {
     hipStream_t s = ctx->stream;
     const pi_gate_attention & A = H.left;
     const int width = ctx->model->hparams.n_embd, nb = ctx->n_batch, ch = A.channels();
     const int64_t pw = row_of_4(H.in_rows()), cw = row_of_4(ch), hd = (int64_t) A.heads * A.maps * A.dim, hv = (int64_t) A.heads * A.vdim, gd = (int64_t) A.kv_heads * A.maps * A.dim;
     float * P = ctx->h_in, * Q = ctx->h_att, * O = Q + (size_t) nb * hd, * C = O + (size_t) nb * hv;
     float * kc = ctx->lat_cache + ctx->lat_off[il], * vc = kc + (size_t) ctx->n_ctx * gd;
-    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));
+    uint16_t * oh = reads_rounded(ctx, W.w_o, n_tok, ctx->act_h);
+    OP_OK(dense(ctx, W.w_in, N, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, Nh, width));
     const float * qkv = P; int64_t qs = pw;
     if (A.conv > 0) { OP_OK(pi_op_causal_conv(P, pw, ch, A.conv, W.conv_w, nullptr, ctx->rec_state + ctx->rec_off[il], ctx->rec_dev, n_tok, PI_ACT_NONE, C, cw, s)); qkv = C; qs = cw; }
     OP_OK(pi_op_qkv_prepare_maps(qkv, qkv + hd, qkv + hd + gd, qs, A.heads, A.kv_heads, A.maps, A.dim, A.vdim, W.rotary, A.pairing, ctx->pos_dev, n_tok, Q, hd, kc, vc, ctx->cell_pos, ctx->dyn_dev, s));
-    OP_OK(pi_op_diff_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, A.scale, A.chunk, A.keep_first, A.maps, W.lam, 1.0f - A.diff, ctx->model->hparams.f_norm_rms_eps, A.heads, A.kv_heads, A.dim, A.vdim, n_tok,
-                               n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s));
+    OP_OK(op_rounded(ctx, oh, O, hv, 0, hv, n_tok, true, s, [&] {
+        return pi_op_diff_attention(Q, hd, kc, vc, ctx->cell_pos, ctx->mask_dev, ctx->pos_dev, A.scale, A.chunk, A.keep_first, A.maps, W.lam, 1.0f - A.diff, ctx->model->hparams.f_norm_rms_eps, A.heads, A.kv_heads, A.dim, A.vdim, n_tok,
+                                    n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, O, hv, ctx->dyn_dev, s);
+    }));
     trace(ctx, "att", (int) il, O, hv, n_tok);
-    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+    OP_OK(dense(ctx, W.w_o, O, hv, n_tok, ctx->h_out, width, PI_ACT_NONE, width, PI_ACT_NONE, s, oh, hv));
     return true;
 }
 static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
@@ -807,15 +851,17 @@ static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
     const size_t n_layer = hp.hybrid.size();
     float * x = ctx->x, * N = ctx->nx, * Y = ctx->h_out, * P = ctx->h_in;
     // x + y (+ the vector of the pass that run `next` opens) -> x, the norm that run `next` (or the model's output) reads -> N
+    uint16_t * nh = nullptr;                                                   // N in bfloat16, where its reader takes it so
     auto step_to = [&](size_t next, const float * y) {
         const bool last = next == n_layer;
+        nh = reads_rounded(ctx, last ? m->tok_embd : m->hweights[(size_t) hp.hybrid[next].weights].w_in, n_tok, ctx->x_h);
         const float * w = last ? m->output_norm : m->hweights[(size_t) hp.hybrid[next].weights].norm1, * shift = !last && hp.hybrid[next].loop_entry ? m->loop_step + (size_t) hp.hybrid[next].loop_pass * width : nullptr;
         if (trace_enabled() && y) {                                            // (the stream as the layer left it)
             if (pi_op_residual_norm(x, y, width, nullptr, w, eps, width, n_tok, x, N, width, s) != 0) return -1;
             trace(ctx, "lout", (int) next - 1, x, width, n_tok);
             y = nullptr;
         }
-        return pi_op_residual_norm(x, y, width, shift, w, eps, width, n_tok, x, N, width, s);
+        return op_rounded(ctx, nh, N, width, 0, width, n_tok, true, s, [&] { return pi_op_residual_norm(x, y, width, shift, w, eps, width, n_tok, x, N, width, s); });
     };
     if (m->pair_embd) OP_OK(pi_op_embed_pair(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, m->pair_embd, ctx->pair_dev, x, s));
     else OP_OK(pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s));
@@ -825,22 +871,23 @@ static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
         const pi_hybrid_weights & W = m->hweights[(size_t) H.weights];
         bool ok = false;
         switch (H.mixer) {
-            case PI_MIXER_WINDOW_ATTENTION: ok = forward_diff_attention(ctx, H, W, il, N, n_tok, n_kv); break;
-            case PI_MIXER_LATENT_ATTENTION: ok = forward_query_latent(ctx, H, W, il, N, n_tok, n_kv); break;
+            case PI_MIXER_WINDOW_ATTENTION: ok = forward_diff_attention(ctx, H, W, il, N, nh, n_tok, n_kv); break;
+            case PI_MIXER_LATENT_ATTENTION: ok = forward_query_latent(ctx, H, W, il, N, nh, n_tok, n_kv); break;
             default: ctx->last_error = "plain pre-norm blocks are built for the window-attention and latent-attention mixers";
         }
         if (!ok) return false;
         if (H.has_mlp) {
             const int ff = H.ff;
             float * G = P + (size_t) nb * 2 * ff;
-            OP_OK(pi_op_residual_norm(x, Y, width, nullptr, W.norm2, eps, width, n_tok, x, N, width, s));
-            OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_NONE, 2 * (int64_t) ff, PI_ACT_NONE, s));
-            OP_OK(pi_op_glu_mul_ex(P, 2 * (int64_t) ff, ff, PI_GLU_CLIPPED, H.glu_limit, -1, n_tok, G, ff, s));
-            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
+            uint16_t * uh = reads_rounded(ctx, W.ff_up, n_tok, ctx->x_h), * gh = reads_rounded(ctx, W.ff_down, n_tok, ctx->act_h);
+            OP_OK(op_rounded(ctx, uh, N, width, 0, width, n_tok, true, s, [&] { return pi_op_residual_norm(x, Y, width, nullptr, W.norm2, eps, width, n_tok, x, N, width, s); }));
+            OP_OK(dense(ctx, W.ff_up, N, width, n_tok, P, 2 * (int64_t) ff, PI_ACT_NONE, 2 * (int64_t) ff, PI_ACT_NONE, s, uh, width));
+            OP_OK(op_rounded(ctx, gh, G, ff, 0, ff, n_tok, true, s, [&] { return pi_op_glu_mul_ex(P, 2 * (int64_t) ff, ff, PI_GLU_CLIPPED, H.glu_limit, -1, n_tok, G, ff, s); }));
+            OP_OK(dense(ctx, W.ff_down, G, ff, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, gh, ff));
         }
         OP_OK(step_to(il + 1, Y));
     }
-    OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
+    OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, nh, width));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }
@@ -857,37 +904,44 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
     const int width = hp.n_embd, ex = ctx->exact;
     const float eps = hp.f_norm_rms_eps, rm = hp.residual_mult;
     float * x = ctx->x, * P = ctx->h_in, * A = ctx->h_att, * Y = ctx->h_out;
-    OP_OK(pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s));
+    // the stream in bfloat16 where the next projection reads it so
+    auto x_rounded = [&](size_t il) { return il < hp.hybrid.size() ? reads_rounded(ctx, m->hweights[(size_t) hp.hybrid[il].weights].w_in, n_tok, ctx->x_h) : nullptr; };
+    uint16_t * xh = x_rounded(0);
+    OP_OK(op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s); }));
     for (size_t il = 0; il < hp.hybrid.size(); il++) {
         const pi_hybrid_layer & H = hp.hybrid[il];
         const pi_hybrid_weights & W = m->hweights[(size_t) H.weights];
         const int64_t hd = (int64_t) H.heads * H.dim, hv = (int64_t) H.heads * H.vdim, pw = H.in_rows();
+        uint16_t * ah = reads_rounded(ctx, W.w_o, n_tok, ctx->act_h);
         if (H.mixer == PI_MIXER_LATENT_ATTENTION) {
             float * cache = ctx->lat_cache + ctx->lat_off[il];
-            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s));                                               // q | W_dkv h
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, xh, width));                                    // q | W_dkv h
             OP_OK(pi_op_rms_scale(P + hd, pw, W.mix_norm, 0.0f, eps, H.kv_rank, n_tok, nullptr, 0, nullptr, 0, 1.0f, cache, H.kv_rank, ctx->dyn_dev, 1, s));   // the latent, into its cell
-            OP_OK(pi_op_latent_attention(P, pw, cache, ctx->mask_dev, W.w_uk, W.w_uv, W.sink, H.scale, H.heads, H.dim, H.vdim, H.kv_rank, n_tok, n_kv, ctx->lat_scratch, ctx->lat_scratch_floats, A, hv, ctx->dyn_dev, s));
+            OP_OK(op_rounded(ctx, ah, A, hv, 0, hv, n_tok, true, s, [&] { return pi_op_latent_attention(P, pw, cache, ctx->mask_dev, W.w_uk, W.w_uv, W.sink, H.scale, H.heads, H.dim, H.vdim, H.kv_rank, n_tok, n_kv, ctx->lat_scratch,
+                                                                                                        ctx->lat_scratch_floats, A, hv, ctx->dyn_dev, s); }));
         } else {
             float * state = ctx->rec_state + ctx->rec_off[il];
-            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_SILU, 2 * hd + hv, PI_ACT_SIGMOID, s));                                   // silu(q | k | v) | sigmoid(g)
+            OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_SILU, 2 * hd + hv, PI_ACT_SIGMOID, s, xh, width));                        // silu(q | k | v) | sigmoid(g)
             OP_OK(pi_op_linear_attention(P, P + hd, P + 2 * hd, pw, H.heads, H.dim, H.vdim, W.decay, state, ctx->rec_dev, n_tok, ctx->slots->size(), ctx->rec_scratch, ctx->rec_scratch_floats, A, hv, s));
-            OP_OK(pi_op_rms_scale(A, hv, W.mix_norm, 0.0f, eps, (int) hv, n_tok, P + 2 * hd + hv, pw, nullptr, 0, 1.0f, A, hv, nullptr, 0, s));    // norm over all heads, * gate
+            OP_OK(op_rounded(ctx, ah, A, hv, 0, hv, n_tok, true, s, [&] { return pi_op_rms_scale(A, hv, W.mix_norm, 0.0f, eps, (int) hv, n_tok, P + 2 * hd + hv, pw, nullptr, 0, 1.0f, A, hv, nullptr, 0, s); }));    // norm over all heads, * gate
         }
         trace(ctx, "mix", (int) il, A, hv, n_tok);
-        OP_OK(dense(ctx, W.w_o, A, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s));
-        OP_OK(pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s));
+        OP_OK(dense(ctx, W.w_o, A, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, ah, hv));
+        xh = x_rounded(il + 1);
+        OP_OK(op_rounded(ctx, H.has_mlp ? nullptr : xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
         if (H.has_mlp) {
             OP_OK(pi_op_moe_route(W.router, W.correction, x, width, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s));
             if (pi_op_moe_grouped_ok(W.e_up, W.e_down, H.n_expert, H.ff, 0, n_tok, H.top, ex))                                                     // prompts: by expert, on the matrix cores
                 OP_OK(pi_op_moe_experts_grouped(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
             else
                 OP_OK(pi_op_moe_experts(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ex, ctx->moe_up, Y, width, s));
-            OP_OK(pi_op_rms_scale(Y, width, W.norm2, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s));
+            OP_OK(op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm2, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
         }
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    OP_OK(pi_op_rms_scale(x, width, m->output_norm, 1.0f, eps, width, n_tok, nullptr, 0, nullptr, 0, 1.0f, ctx->nx, width, nullptr, 0, s));
-    OP_OK(dense(ctx, m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
+    uint16_t * nh = reads_rounded(ctx, m->tok_embd, n_tok, ctx->x_h);
+    OP_OK(op_rounded(ctx, nh, ctx->nx, width, 0, width, n_tok, true, s, [&] { return pi_op_rms_scale(x, width, m->output_norm, 1.0f, eps, width, n_tok, nullptr, 0, nullptr, 0, 1.0f, ctx->nx, width, nullptr, 0, s); }));
+    OP_OK(dense(ctx, m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, nh, width));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;
 }

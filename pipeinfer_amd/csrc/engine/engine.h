@@ -307,7 +307,8 @@ struct llama_context {
     int32_t * pair_dev = nullptr;                             // per token of the pass: its row of the pair-embedding table (models with pair_buckets > 0)
     int exact = 0;                                            // 1: dense operators keep fp32 activations (pipeinfer_context_set_precision)
     float * h_in = nullptr, * h_att = nullptr, * h_out = nullptr, * moe_w = nullptr, * moe_up = nullptr, * moe_dn = nullptr, * lat_scratch = nullptr, * rec_scratch = nullptr; size_t lat_scratch_floats = 0, rec_scratch_floats = 0; int32_t * moe_sel = nullptr, * moe_idx = nullptr;   // hybrid scratch
-    uint16_t * act_h = nullptr; size_t act_h_row = 0;         // activations of the product at hand in bfloat16 (values of a token's row)
+    // activations in bfloat16, as the products of many tokens read them: the stream or its norm, of the product at hand (act_h_row values of a token's row), of a product's result that the next one reads (parts of one allocation, act_h)
+    uint16_t * x_h = nullptr, * act_h = nullptr, * mid_h = nullptr; size_t act_h_row = 0;
     void * rope = nullptr;
     hipStream_t stream = nullptr;
     int stream_priority = 0;                 // > 0 high, < 0 low (pipeinfer_context_set_priority, before the first decode)

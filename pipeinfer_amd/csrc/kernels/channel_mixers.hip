@@ -36,7 +36,7 @@ static __device__ __forceinline__ float cm_block_sum(float v, float * red) {    
 // grid (token, 2048 values): eight values of a thread in one 16-byte load of each table (vec: rows and output start 16-byte aligned).  A thread that walked the row in 2-byte loads made a trip to memory at every one of
 // them: 18 us for 8 tokens of width 4096, now 4.3
 __global__ void __launch_bounds__(256) k_embed_pair(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, const uint16_t * __restrict__ table2, int64_t n_rows2,
-                             const int32_t * __restrict__ rows2, int vec, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
+                             const int32_t * __restrict__ rows2, int vec, float * __restrict__ out, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x;
     const int64_t row = tokens[t], row2 = rows2[t], i0 = (int64_t) blockIdx.y * 2048;
@@ -51,6 +51,7 @@ __global__ void __launch_bounds__(256) k_embed_pair(const uint16_t * __restrict_
         for (int c = 0; c < 8; c++) ((float *) o)[c] = (ok ? cm_widen(a[c]) * scale : 0.0f) + (ok2 ? cm_widen(b[c]) : 0.0f);
         float4 * dst = (float4 *) (out + (int64_t) t * width + i);
         dst[0] = o[0]; dst[1] = o[1];
+        if (rd.h) *(uint4 *) (rd.h + t * rd.stride + i) = make_uint4(pi_round_pair(o[0].x, o[0].y), pi_round_pair(o[0].z, o[0].w), pi_round_pair(o[1].x, o[1].y), pi_round_pair(o[1].z, o[1].w));
         return;
     }
     for (int64_t i = i0 + threadIdx.x; i < min(width, i0 + 2048); i += 256)
@@ -61,7 +62,7 @@ extern "C" int pi_op_embed_pair(const pi_weight * w, const int32_t * tokens, int
     if (n_tok <= 0) return 0;
     const int vec = w->ne0 % 8 == 0 && w->ne1 > 0 && w2->ne1 > 0 && (((uintptr_t) w->p0 | (uintptr_t) w2->p0 | (uintptr_t) out) & 15) == 0;
     PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 8.0 * w->ne0 * n_tok, k_embed_pair, dim3((unsigned) n_tok, (unsigned) ((w->ne0 + 2047) / 2048)), dim3(256), 0, (hipStream_t) stream, (const uint16_t *) w->p0, w->ne0, w->ne1, tokens, scale,
-                 (const uint16_t *) w2->p0, w2->ne1, rows2, vec, out, pi_abort_word());
+                 (const uint16_t *) w2->p0, w2->ne1, rows2, vec, out, vec ? pi_round_asked(0, w->ne0) : pi_round_dst{}, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 
@@ -72,7 +73,7 @@ extern "C" int pi_op_embed_pair(const pi_weight * w, const int32_t * tokens, int
 template <int NPT, bool PRE>
 __global__ void __launch_bounds__(256) k_rms_post(const float * __restrict__ a, int64_t as, const float * __restrict__ wa, const float * __restrict__ b, int64_t bs, const float * __restrict__ wb, float mb,
                                                   const float * __restrict__ ls, const float * __restrict__ x, int64_t xs, float alpha, const float * __restrict__ w, float eps, int n,
-                                                  float * __restrict__ out, int64_t os, const float * __restrict__ w_next, float * __restrict__ out_next, int64_t ons, const int32_t * __restrict__ abort_w) {
+                                                  float * __restrict__ out, int64_t os, const float * __restrict__ w_next, float * __restrict__ out_next, int64_t ons, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -110,11 +111,20 @@ __global__ void __launch_bounds__(256) k_rms_post(const float * __restrict__ a, 
     float s2 = 0.0f;
 #pragma unroll
     for (int j = 0; j < NPT; j++) { const int i = j * 256 + tid; if (i < n) { v[j] = v[j] * inv * (PRE ? pw[j] : w[i]); out[(int64_t) t * os + i] = v[j]; s2 = fmaf(v[j], v[j], s2); } }
-    if (!w_next) return;
+    if (!w_next) {
+        if (rd.h)
+#pragma unroll
+            for (int j = 0; j < NPT; j++) { const int i = j * 256 + tid; if (i < n) rd.h[t * rd.stride + i] = pi_round_one(v[j]); }
+        return;
+    }
     s2 = cm_block_sum(s2, red);
     const float inv2 = 1.0f / sqrtf(s2 / (float) n + eps);
 #pragma unroll
-    for (int j = 0; j < NPT; j++) { const int i = j * 256 + tid; if (i < n) out_next[(int64_t) t * ons + i] = v[j] * inv2 * (PRE ? pwn[j] : w_next[i]); }
+    for (int j = 0; j < NPT; j++) { const int i = j * 256 + tid; if (i < n) {
+        const float y = v[j] * inv2 * (PRE ? pwn[j] : w_next[i]);
+        if (!rd.only) out_next[(int64_t) t * ons + i] = y;
+        if (rd.h) rd.h[t * rd.stride + i] = pi_round_one(y);
+    } }
 }
 extern "C" int pi_op_rms_post(const float * a, int64_t a_stride, const float * wa, const float * b, int64_t b_stride, const float * wb, float mean_mult, const float * layer_scale, const float * x, int64_t x_stride,
                               float alpha, const float * w, float eps, int n, int n_tok, float * out, int64_t out_stride, const float * w_next, float * out_next, int64_t out_next_stride, void * stream) {
@@ -123,8 +133,9 @@ extern "C" int pi_op_rms_post(const float * a, int64_t a_stride, const float * w
     if (b && (!wa || !wb)) { pi_set_error("pi_op_rms_post: two inputs need the weights of their norms"); return -1; }
     if (w_next && !out_next) { pi_set_error("pi_op_rms_post: a second norm needs a place for its result"); return -1; }
     const double bytes = 4.0 * n * n_tok * (3.0 + (b ? 1 : 0) + (w_next ? 1 : 0));
+    const pi_round_dst rd = pi_round_asked(0, n);                      // (of the second norm where there is one)
 #define RP_GO(N, P) PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, (k_rms_post<N, P>), dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, a, a_stride, wa, b, b_stride, wb, mean_mult, layer_scale, x, x_stride, alpha, w, eps, n, \
-                              out, out_stride, w_next, out_next, out_next_stride, pi_abort_word())
+                              out, out_stride, w_next, out_next, out_next_stride, rd, pi_abort_word())
     if (n <= 256 * 2) RP_GO(2, true); else if (n <= 256 * 4) RP_GO(4, true); else if (n <= 256 * 8) RP_GO(8, true); else if (n <= 256 * 16) RP_GO(16, true); else RP_GO(32, false);
 #undef RP_GO
     PI_CHECK_LAUNCH(); return 0;
@@ -134,7 +145,7 @@ extern "C" int pi_op_rms_post(const float * a, int64_t a_stride, const float * w
 // out[t][s][i] = h[t][i] + (prev[i] - h[t][i]) * mu[s][i], s < n_mix; prev = h[t - 1] inside a sequence's run, the sequence's state (zeros on a fresh slot) at the run's first token.
 // rec as for the recurrences; state: [slots][n].  grid (token, blocks of 256 values)
 __global__ void __launch_bounds__(256) k_token_shift(const float * __restrict__ h, int64_t hs, int n, const float * __restrict__ mu, int n_mix, const float * __restrict__ state, const int32_t * __restrict__ rec,
-                                                     float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+                                                     float * __restrict__ out, int64_t os, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w)) return;
     const int t = blockIdx.x, i = blockIdx.y * 256 + threadIdx.x;
     if (i >= n) return;
@@ -143,7 +154,11 @@ __global__ void __launch_bounds__(256) k_token_shift(const float * __restrict__ 
     const float cur = h[(int64_t) t * hs + i];
     const float prev = inside ? h[(int64_t) (t - 1) * hs + i] : (word & CM_FRESH) ? 0.0f : state[(int64_t) slot * n + i];
     const float d = prev - cur;
-    for (int s = 0; s < n_mix; s++) out[(int64_t) t * os + (int64_t) s * n + i] = fmaf(d, mu[(int64_t) s * n + i], cur);
+    for (int s = 0; s < n_mix; s++) {
+        const float y = fmaf(d, mu[(int64_t) s * n + i], cur);
+        if (!rd.only) out[(int64_t) t * os + (int64_t) s * n + i] = y;
+        if (rd.h) rd.h[t * rd.stride + (int64_t) s * n + i] = pi_round_one(y);
+    }
 }
 // a run's last token becomes the sequence's state (its own launch: the run's first token reads the state in the launch above)
 __global__ void __launch_bounds__(256) k_token_shift_state(const float * __restrict__ h, int64_t hs, int n, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, const int32_t * __restrict__ abort_w) {
@@ -181,7 +196,7 @@ extern "C" int pi_op_token_shift(const float * h, int64_t h_stride, int n, const
         PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, k_token_shift_walk, grid, dim3(256), 0, s, h, h_stride, n, mu_dev, n_mix, state_dev, rec_dev, n_tok, out, out_stride, pi_abort_word());
         PI_CHECK_LAUNCH(); return 0;
     }
-    PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, k_token_shift, grid, dim3(256), 0, s, h, h_stride, n, mu_dev, n_mix, state_dev, rec_dev, out, out_stride, pi_abort_word());
+    PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, k_token_shift, grid, dim3(256), 0, s, h, h_stride, n, mu_dev, n_mix, state_dev, rec_dev, out, out_stride, pi_round_asked(0, (int64_t) n_mix * n), pi_abort_word());
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 8.0 * n, k_token_shift_state, grid, dim3(256), 0, s, h, h_stride, n, state_dev, rec_dev, n_tok, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
@@ -890,7 +905,7 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
 // ---- per-head RMS norm, weight, gate ------------------------------------------------------------------------------------------------------------------------------
 // out[t][h][i] = y[t][h][i] / sqrt(mean_i(y[t][h]^2) + eps) * w[(w_per_head ? h * n : 0) + i] * act(gate[t][h][i]);  a wave per (token, head); out may be y
 __global__ void __launch_bounds__(256) k_head_norm_gate(const float * __restrict__ y, int64_t ys, int heads, int n, const float * __restrict__ w, int w_per_head, const float * __restrict__ gate, int64_t gs, int gate_act,
-                                                        float eps, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+                                                        float eps, float * __restrict__ out, int64_t os, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x, h = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (h >= heads) return;
@@ -913,7 +928,9 @@ __global__ void __launch_bounds__(256) k_head_norm_gate(const float * __restrict
             float g = gv[j];
             if (gate && gate_act == PI_ACT_SIGMOID) g = cm_sigmoid(g);
             else if (gate && gate_act == PI_ACT_SILU) g = g / (1.0f + expf(-g));
-            out[(int64_t) t * os + (int64_t) h * n + i] = yv[j] * inv * wv[j] * g;
+            const float o = yv[j] * inv * wv[j] * g;
+            if (!rd.only) out[(int64_t) t * os + (int64_t) h * n + i] = o;
+            if (rd.h) rd.h[t * rd.stride + (int64_t) h * n + i] = pi_round_one(o);
         }
         return;
     }
@@ -925,13 +942,15 @@ __global__ void __launch_bounds__(256) k_head_norm_gate(const float * __restrict
         float g = gate ? gate[(int64_t) t * gs + (int64_t) h * n + i] : 1.0f;
         if (gate && gate_act == PI_ACT_SIGMOID) g = cm_sigmoid(g);
         else if (gate && gate_act == PI_ACT_SILU) g = g / (1.0f + expf(-g));
-        out[(int64_t) t * os + (int64_t) h * n + i] = yr[i] * inv * w[(w_per_head ? h * n : 0) + i] * g;
+        const float o = yr[i] * inv * w[(w_per_head ? h * n : 0) + i] * g;
+        if (!rd.only) out[(int64_t) t * os + (int64_t) h * n + i] = o;
+        if (rd.h) rd.h[t * rd.stride + (int64_t) h * n + i] = pi_round_one(o);
     }
 }
 extern "C" int pi_op_head_norm_gate(const float * y, int64_t y_stride, int heads, int n, const float * w_dev, int w_per_head, const float * gate, int64_t gate_stride, int gate_act, float eps, int n_tok,
                                     float * out, int64_t out_stride, void * stream) {
     if (n_tok <= 0 || heads <= 0 || n <= 0) return 0;
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n_tok * heads * n, k_head_norm_gate, dim3((unsigned) n_tok, (unsigned) ((heads + 3) / 4)), dim3(256), 0, (hipStream_t) stream, y, y_stride, heads, n, w_dev, w_per_head,
-                 gate, gate_stride, gate_act, eps, out, out_stride, pi_abort_word());
+                 gate, gate_stride, gate_act, eps, out, out_stride, pi_round_asked(0, (int64_t) heads * n), pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }

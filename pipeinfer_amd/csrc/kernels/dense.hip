@@ -42,7 +42,7 @@ static __device__ __forceinline__ float dn_act(float v, int act) {
 }
 
 // grid (token, 2048 values); vec: eight values of a thread in one 16-byte load (rows and output start 16-byte aligned), else one by one
-__global__ void __launch_bounds__(256) k_embed(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, int vec, float * __restrict__ out, const int32_t * __restrict__ abort_w) {
+__global__ void __launch_bounds__(256) k_embed(const uint16_t * __restrict__ table, int64_t width, int64_t n_rows, const int32_t * __restrict__ tokens, float scale, int vec, float * __restrict__ out, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     const int t = blockIdx.x;
     const int64_t row = tokens[t], i0 = (int64_t) blockIdx.y * 2048;
@@ -57,6 +57,7 @@ __global__ void __launch_bounds__(256) k_embed(const uint16_t * __restrict__ tab
         for (int c = 0; c < 8; c++) ((float *) o)[c] = ok ? dn_widen(a[c]) * scale : 0.0f;
         float4 * dst = (float4 *) (out + (int64_t) t * width + i);
         dst[0] = o[0]; dst[1] = o[1];
+        if (rd.h) *(dt_u32x4 *) (rd.h + t * rd.stride + i) = dt_pack8(*(const dt_f32x4 *) &o[0], *(const dt_f32x4 *) &o[1]);
         return;
     }
     for (int64_t i = i0 + threadIdx.x; i < min(width, i0 + 2048); i += 256) out[(int64_t) t * width + i] = ok ? dn_widen(table[row * width + i]) * scale : 0.0f;
@@ -276,7 +277,7 @@ __global__ void __launch_bounds__(512) k_dense_split(const uint16_t * __restrict
 template <int BN, int BT, int WN, int WT, int S>
 __global__ void __launch_bounds__(64 * WN * WT, WN * WT == 8 && BN * BT >= 32768 ? 2 : 1) k_dense_async(const uint16_t * __restrict__ W, int64_t K, int64_t N, const uint16_t * __restrict__ X, int64_t xs, int T, float * __restrict__ Y,
                                                        int64_t ys, int act_a, int64_t rows_a, int act_b, const float * __restrict__ bias, int blocks_of, int64_t seg_rows, int64_t seg_off, int seg_last, int tok_blocks, int tiles,
-                                                       const int32_t * __restrict__ abort_w) {
+                                                       const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w, 1)) return;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[DA_LDS_BYTES(BN, BT, S)];
     const int tile = (int) (blockIdx.x & 7) * (int) (gridDim.x >> 3) + (int) (blockIdx.x >> 3);
@@ -284,25 +285,43 @@ __global__ void __launch_bounds__(64 * WN * WT, WN * WT == 8 && BN * BT >= 32768
     const int row_blocks = tiles / tok_blocks, grp = tile / (8 * tok_blocks), in_grp = tile % (8 * tok_blocks), gsz = min(8, row_blocks - 8 * grp), block = 8 * grp + in_grp % gsz;
     const int seg = seg_rows > 0 ? min(block / blocks_of, seg_last) : 0;
     const int64_t n0 = seg_rows > 0 ? seg * seg_rows + (int64_t) (block - seg * blocks_of) * BN : (int64_t) block * BN, n_end = seg_rows > 0 && seg < seg_last ? (seg + 1) * seg_rows : N;
-    const int t0 = (in_grp / gsz) * BT, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = (in_grp / gsz) * BT, wave = threadIdx.x >> 6;
+    const bool vec = (ys & 3) == 0 && ((uintptr_t) Y & 15) == 0;
     dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
     da_tile<BN, BT, WN, WT, S>(W + n0 * K, [&](int r) { return (uint32_t) (min((int64_t) r, n_end - 1 - n0) * K * 2); }, X + seg * seg_off + (int64_t) t0 * xs, [&](int r) { return (uint32_t) ((int64_t) min(r, T - 1 - t0) * xs * 2); },
                                (int) (K / 64), lds, acc);
+    __syncthreads();                                                   // (the operands of every wave are read)
+    constexpr int SHARE = DA_LDS_BYTES(BN, BT, S) / (WN * WT) & ~15;
+    const int64_t row0 = n0 + (wave / WT) * (BN / WN); const int tok0 = t0 + (wave % WT) * (BT / WT);
+    da_rows<BN / WN / 16, BT / WT / 16, SHARE>(acc, lds + wave * SHARE, [&](int t, int r, dt_f32x4 v) __attribute__((always_inline)) {
+        const int64_t row = row0 + r; const int tok = tok0 + t;
+        if (tok >= T || row >= n_end) return;
+        if (bias)
 #pragma unroll
-    for (int b = 0; b < BT / WT / 16; b++) {
-        const int tok = t0 + (wave % WT) * (BT / WT) + b * 16 + (lane & 15);
-        if (tok >= T) continue;
+            for (int e = 0; e < 4; e++) v[e] += bias[min(row + e, n_end - 1)];
+        if (act_a != PI_ACT_NONE || act_b != PI_ACT_NONE) {
+            const int act = row < rows_a ? act_a : act_b, act3 = row + 3 < rows_a ? act_a : act_b;      // (a group of four that both activations share: one by one)
 #pragma unroll
-        for (int a = 0; a < BN / WN / 16; a++) dn_store4(acc[a][b], n0 + (wave / WT) * (BN / WN) + a * 16 + (lane >> 4) * 4, n_end, tok, Y, ys, act_a, rows_a, act_b, bias);
-    }
+            for (int e = 0; e < 4; e++) v[e] = dn_act(v[e], act == act3 ? act : row + e < rows_a ? act_a : act_b);
+        }
+        float * dst = Y + (int64_t) tok * ys + row;
+        if (row + 3 < n_end && vec) *(dt_f32x4 *) dst = v;
+        else for (int e = 0; e < 4; e++) if (row + e < n_end) dst[e] = v[e];
+        if (rd.h && row >= rd.from && row < rd.from + rd.n) pi_round_store4(rd, tok, row - rd.from, v[0], v[1], v[2], v[3]);
+    });
 }
 
 // rows of fp32 values as bfloat16, nearest even: grid (2048 values, row), eight of a thread (n % 8 == 0)
-__global__ void __launch_bounds__(256) k_round_bf16(const float * __restrict__ x, int64_t xs, int64_t n, uint16_t * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+__global__ void __launch_bounds__(256) k_round_bf16(const float * __restrict__ x, int64_t xs, int64_t n, int vec, uint16_t * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     const int64_t i = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 8, t = blockIdx.y;
     if (i >= n) return;
-    const dt_f32x4 lo = *(const dt_f32x4 *) (x + t * xs + i), hi = *(const dt_f32x4 *) (x + t * xs + i + 4);
+    dt_f32x4 lo, hi;
+    const float * r = x + t * xs + i;
+    if (vec) { lo = *(const dt_f32x4 *) r; hi = *(const dt_f32x4 *) (r + 4); }
+    else
+#pragma unroll
+        for (int e = 0; e < 4; e++) { lo[e] = r[e]; hi[e] = r[4 + e]; }
     if (pi_abort_late(gone, abort_w)) return;
     *(dt_u32x4 *) (out + t * os + i) = dt_pack8(lo, hi);
 }
@@ -312,7 +331,7 @@ extern "C" int pi_op_embed(const pi_weight * w, const int32_t * tokens, int n_to
     if (n_tok <= 0) return 0;
     const int vec = w->ne0 % 8 == 0 && w->ne1 > 0 && (((uintptr_t) w->p0 | (uintptr_t) out) & 15) == 0;
     PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * w->ne0 * n_tok, k_embed, dim3((unsigned) n_tok, (unsigned) ((w->ne0 + 2047) / 2048)), dim3(256), 0, (hipStream_t) stream, (const uint16_t *) w->p0, w->ne0, w->ne1, tokens, scale, vec, out,
-                 pi_abort_word());
+                 vec ? pi_round_asked(0, w->ne0) : pi_round_dst{}, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 
@@ -404,9 +423,10 @@ extern "C" int pi_op_dense_bias(const pi_weight * w, const float * bias, const f
 
 extern "C" int pi_op_round_bf16(const float * x, int64_t x_stride, int64_t n, int n_tok, uint16_t * out, int64_t out_stride, void * stream) {
     if (n_tok <= 0 || n <= 0) return 0;
-    if (n % 8 || x_stride < n || out_stride < n || x_stride % 4 || out_stride % 8 || ((uintptr_t) x % 16) || ((uintptr_t) out % 16)) { pi_set_error("pi_op_round_bf16: rows of a multiple of 8 values, 16-byte aligned"); return -1; }
+    if (n % 8 || x_stride < n || out_stride < n || out_stride % 8 || ((uintptr_t) out % 16)) { pi_set_error("pi_op_round_bf16: rows of a multiple of 8 values, 16-byte aligned where they are written"); return -1; }
+    const int vec = x_stride % 4 == 0 && ((uintptr_t) x % 16) == 0;
     for (int t = 0; t < n_tok; t += 65535)                             // (rows are the grid's second dimension)
-        PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * n * n_tok, k_round_bf16, dim3((unsigned) ((n + 2047) / 2048), (unsigned) std::min(65535, n_tok - t)), dim3(256), 0, (hipStream_t) stream, x + (int64_t) t * x_stride, x_stride, n,
+        PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 6.0 * n * n_tok, k_round_bf16, dim3((unsigned) ((n + 2047) / 2048), (unsigned) std::min(65535, n_tok - t)), dim3(256), 0, (hipStream_t) stream, x + (int64_t) t * x_stride, x_stride, n, vec,
                      out + (int64_t) t * out_stride, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
@@ -445,8 +465,10 @@ extern "C" int pi_op_dense_rounded(const pi_weight * w, const float * bias, cons
     int row_blocks = 0, tok_blocks = 0, blocks_of = 0;
     const int which = async_tile_of(w->ne1, w->ne0, n_tok, seg_rows, n_seg, row_blocks, tok_blocks, blocks_of), tiles = row_blocks * tok_blocks;
     const double bytes = 2.0 * w->ne0 * w->ne1 + 2.0 * n_tok * n_seg * w->ne0 + 4.0 * n_tok * w->ne1;
+    pi_round_dst rd = pi_round_take();
+    if (rd.h && (rd.from % 4 || rd.n % 4 || rd.from < 0 || rd.from + rd.n > w->ne1 || rd.stride % 4)) { pi_set_error("pi_op_dense_rounded: rounded columns [%lld, + %lld) of %lld rows", (long long) rd.from, (long long) rd.n, (long long) w->ne1); return -1; }
 #define DN_ASYNC(BN, BT, WN, WT, S) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, std::min(n_tok, PI_KT_MAXNT - 1), bytes, (k_dense_async<BN, BT, WN, WT, S>), dim3((unsigned) ((tiles + 7) / 8 * 8)), dim3(64 * WN * WT), 0, s, \
-                     (const uint16_t *) w->p0, w->ne0, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, blocks_of, seg_rows, seg_off, n_seg - 1, tok_blocks, tiles, pi_abort_word())
+                     (const uint16_t *) w->p0, w->ne0, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, blocks_of, seg_rows, seg_off, n_seg - 1, tok_blocks, tiles, rd, pi_abort_word())
     switch (which) {
         case 0:  DN_ASYNC(32, 64, 2, 2, 4); break;
         case 1:  DN_ASYNC(64, 64, 4, 2, 4); break;

@@ -20,6 +20,30 @@ static __device__ __forceinline__ void da_load(uint32_t lds, uint32_t offset, ui
 // all but the youngest N of this wave's loads have arrived, and its operand reads are done; then every wave's
 template <int N> static __device__ __forceinline__ void da_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory"); }
 
+// What lane l of a wave holds behind da_tile, four rows of sixteen tokens at a time, goes through the wave's own share of LDS, so that a store covers a token's RW rows (a store of four rows of sixteen tokens writes 64 bytes in
+// sixteen places) and what is done to a value on its way stands in the code once, not once per register: with silu and sigmoid 16384 x 4096 at 2048 tokens took 329 us, 207 without.  put(token, row, four values) of the wave's part.
+template <int RT, int TT, int BYTES, class Put>
+static __device__ __forceinline__ void da_rows(dt_f32x4 (&acc)[RT][TT], uint8_t * share, Put put) {
+    constexpr int RW = 16 * RT, ROW = RW + 4, NB = BYTES / (16 * ROW * 4) < TT ? BYTES / (16 * ROW * 4) : TT, LPT = RW / 4, TPI = 64 / LPT;
+    static_assert(NB > 0, "sixteen tokens fit");
+    const int lane = threadIdx.x & 63, li = lane & 15, kb = lane >> 4;
+    float * const own = (float *) share;
+#pragma unroll
+    for (int b0 = 0; b0 < TT; b0 += NB) {
+#pragma unroll
+        for (int b = b0; b < b0 + NB && b < TT; b++)
+#pragma unroll
+            for (int a = 0; a < RT; a++) *(dt_f32x4 *) (own + ((b - b0) * 16 + li) * ROW + a * 16 + kb * 4) = acc[a][b];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int n = 16 * (TT - b0 < NB ? TT - b0 : NB);
+#pragma unroll 1
+        for (int t = lane / LPT; t < n; t += TPI) put(b0 * 16 + t, (lane % LPT) * 4, *(const dt_f32x4 *) (own + t * ROW + (lane % LPT) * 4));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 #define DA_LDS_BYTES(BN, BT, S) ((S) * ((BN) + (BT)) * 128)
 
 // w, x: the same in all lanes, 16-byte aligned.  w_row(r), x_row(r): where row r of the tile begins, in bytes from w / x, below 2^32 (rows past the end repeat a valid one and are not stored).  steps = K / 64.

@@ -66,7 +66,7 @@ static __device__ __forceinline__ float hy_block_max(float v, float * red) {
 // rows of up to 1024 NV aligned values: everything the row needs is on its way before its sum (a row that was read again behind the sum: one more trip to memory, 3.4 us a launch instead of 3.1)
 template <int NV>
 __global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n, const float * __restrict__ gate, int64_t gs,
-                                                        const float * __restrict__ res, int64_t rs, float mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, const int32_t * __restrict__ abort_w) {
+                                                        const float * __restrict__ res, int64_t rs, float mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x;
@@ -94,7 +94,8 @@ __global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict
 #pragma unroll
         for (int k = 0; k < 4; k++) y[k] *= mult;
         if (res) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
-        *(float4 *) (out + orow * os + i) = make_float4(y[0], y[1], y[2], y[3]);
+        if (!rd.only) *(float4 *) (out + orow * os + i) = make_float4(y[0], y[1], y[2], y[3]);
+        if (rd.h) pi_round_store4(rd, t, i, y[0], y[1], y[2], y[3]);
     }
 }
 __global__ void __launch_bounds__(256) k_rms_scale(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n,
@@ -138,7 +139,7 @@ extern "C" int pi_op_rms_scale(const float * x, int64_t x_stride, const float * 
     auto al = [](const void * p, int64_t stride) { return !p || (((uintptr_t) p % 16) == 0 && stride % 4 == 0); };
     const int vec = n % 4 == 0 && al(x, x_stride) && al(w, 0) && al(gate, gate_stride) && al(residual, residual_stride) && al(out, out_stride);
 #define RS_GO(NV) do { PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale_once<NV>, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride, residual, \
-                                    residual_stride, mult, out, out_stride, dyn_dev, to_cells, pi_abort_word()); PI_CHECK_LAUNCH(); return 0; } while (0)
+                                    residual_stride, mult, out, out_stride, dyn_dev, to_cells, to_cells ? pi_round_dst{} : pi_round_asked(0, n), pi_abort_word()); PI_CHECK_LAUNCH(); return 0; } while (0)
     if (vec && n <= 1024) RS_GO(1);
     if (vec && n <= 2048) RS_GO(2);
     if (vec && n <= 4096) RS_GO(4);
@@ -374,6 +375,37 @@ extern "C" int pi_op_softcap(float * x, int64_t n, float cap, void * stream) {
     PI_CHECK_LAUNCH(); return 0;
 }
 
+// a gated hidden layer from its raw halves: PI_GLU_SILU silu(g) * u; PI_GLU_CLIPPED g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clip(u, -limit, limit) (limit <= 0: no bounds)
+static __device__ __forceinline__ float hy_glu(float g, float u, int glu, float limit) {
+    if (glu == PI_GLU_CLIPPED) {
+        if (limit > 0.0f) { g = fminf(g, limit); u = fminf(fmaxf(u, -limit), limit); }
+        return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
+    }
+    return glu == PI_GLU_SILU ? g / (1.0f + expf(-g)) * u : g * u;
+}
+// the same for passes of many tokens, whose result the down-projection reads in bfloat16: eight values of a thread (1000 tokens of 1408: 6.3 us and 5.2 for the rounding behind it, now 5)
+__global__ void __launch_bounds__(256) k_glu_rounded(const float * __restrict__ in, int64_t is, int ff, int glu, float limit, int64_t gate_col, float * __restrict__ out, int64_t os, const pi_round_dst rd,
+                                                     const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w), t = blockIdx.y, f = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (f >= ff) return;
+    const float * r = in + (int64_t) t * is + f;
+    float4 g[2] = { *(const float4 *) r, *(const float4 *) (r + 4) }, u[2] = { *(const float4 *) (r + ff), *(const float4 *) (r + ff + 4) };
+    const float m = gate_col >= 0 ? 1.0f / (1.0f + expf(-in[(int64_t) t * is + gate_col])) : 1.0f;
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) { y[i] = hy_glu(((const float *) g)[i], ((const float *) u)[i], glu, limit); if (gate_col >= 0) y[i] *= m; }
+    if (pi_abort_late(gone, abort_w)) return;
+    if (!rd.only) { float4 * o = (float4 *) (out + (int64_t) t * os + f); o[0] = make_float4(y[0], y[1], y[2], y[3]); o[1] = make_float4(y[4], y[5], y[6], y[7]); }
+    pi_round_store4(rd, t, f, y[0], y[1], y[2], y[3]); pi_round_store4(rd, t, f + 4, y[4], y[5], y[6], y[7]);
+}
+static bool glu_rounded(const float * in, int64_t is, int ff, int glu, float limit, int64_t gate_col, int n_tok, float * out, int64_t os, hipStream_t s) {
+    if (ff % 8 || is % 4 || os % 4 || (((uintptr_t) in | (uintptr_t) out) & 15)) return false;
+    const pi_round_dst rd = pi_round_asked(0, ff);
+    if (!rd.h) return false;
+    PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 10.0 * ff * n_tok, k_glu_rounded, dim3((unsigned) ((ff + 2047) / 2048), (unsigned) n_tok), dim3(256), 0, s, in, is, ff, glu, limit, gate_col, out, os, rd, pi_abort_word());
+    return true;
+}
+
 // out[t][f] = in[t][f] * in[t][ff + f]  (a gated feed-forward whose gate and up rows are one matrix; the gate's activation ran in the projection's epilogue)
 __global__ void k_glu_mul(const float * __restrict__ in, int64_t is, int ff, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w), t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
@@ -384,18 +416,11 @@ __global__ void k_glu_mul(const float * __restrict__ in, int64_t is, int ff, flo
 }
 extern "C" int pi_op_glu_mul(const float * in, int64_t in_stride, int ff, int n_tok, float * out, int64_t out_stride, void * stream) {
     if (n_tok <= 0 || ff <= 0) return 0;
+    if (glu_rounded(in, in_stride, ff, PI_GLU_OFF, 0.0f, -1, n_tok, out, out_stride, (hipStream_t) stream)) { PI_CHECK_LAUNCH(); return 0; }
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * ff * n_tok, k_glu_mul, dim3((unsigned) ((ff + 255) / 256), (unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, in, in_stride, ff, out, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
 
-// a gated hidden layer from its raw halves: PI_GLU_SILU silu(g) * u; PI_GLU_CLIPPED g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clip(u, -limit, limit) (limit <= 0: no bounds)
-static __device__ __forceinline__ float hy_glu(float g, float u, int glu, float limit) {
-    if (glu == PI_GLU_CLIPPED) {
-        if (limit > 0.0f) { g = fminf(g, limit); u = fminf(fmaxf(u, -limit), limit); }
-        return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
-    }
-    return glu == PI_GLU_SILU ? g / (1.0f + expf(-g)) * u : g * u;
-}
 __global__ void k_glu_mul_ex(const float * __restrict__ in, int64_t is, int ff, int glu, float limit, int64_t gate_col, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w), t = blockIdx.y, f = blockIdx.x * 256 + threadIdx.x;
     if (f >= ff) return;
@@ -408,6 +433,7 @@ __global__ void k_glu_mul_ex(const float * __restrict__ in, int64_t is, int ff, 
 extern "C" int pi_op_glu_mul_ex(const float * in, int64_t in_stride, int ff, int glu, float limit, int64_t gate_col, int n_tok, float * out, int64_t out_stride, void * stream) {
     if (n_tok <= 0 || ff <= 0) return 0;
     if (glu < PI_GLU_OFF || glu > PI_GLU_CLIPPED || gate_col >= in_stride) { pi_set_error("pi_op_glu_mul_ex: hidden layer of kind %d, gate column %lld of rows %lld floats apart", glu, (long long) gate_col, (long long) in_stride); return -1; }
+    if (glu_rounded(in, in_stride, ff, glu, limit, gate_col, n_tok, out, out_stride, (hipStream_t) stream)) { PI_CHECK_LAUNCH(); return 0; }
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * ff * n_tok, k_glu_mul_ex, dim3((unsigned) ((ff + 255) / 256), (unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, in, in_stride, ff, glu, limit, gate_col, out, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
@@ -1641,6 +1667,7 @@ static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int
     const int to = latent_tiles_to(p, a, rank, (int) (((size_t) a.n_kv + cells - 1) / cells));
     if (to == 0 || (to < a.n_kv && !a.dyn)) return 0;
     a.live_max = to < a.n_kv ? to : 0;
+    if (to == a.n_kv) a.rd = pi_round_asked(0, (int64_t) a.heads * a.vdim);      // (else other launches may be the ones that write)
     for (size_t c = 0; c < (size_t) to; c += cells) {
         a.cell0 = (int) c; a.cell1 = (int) std::min((size_t) to, c + cells); a.first = c == 0; a.last = c + cells >= (size_t) to;
         pa_expand(cache, a.k2_row, rank, wuk, wuv, a.cell0, a.cell1, a.n_kv, a.live_max, a.dyn, scratch, scratch + cells * (size_t) a.k1_row, s);

@@ -43,6 +43,14 @@ void pi_set_error(const char * fmt, ...);
 // abort word the calling thread's launches (and captures) hand to their kernels (pi_set_abort_word; nullptr: no check)
 const int32_t * pi_abort_word();
 int pi_account_n_kv();                                       // > 0: the cells an attention launch of this thread really reads (pi_set_account_n_kv)
+// a place for the rounded values of columns [from, from + n) of an operator's rows (pi_set_rounded_output); h null: none
+struct pi_round_dst { uint16_t * h; int64_t stride, from, n; int only; };
+pi_round_dst pi_round_take();                                // the calling thread's request, now met by the caller (who writes it); without one h is null
+pi_round_dst pi_round_asked(int64_t from, int64_t n);        // the same, unless it is about other columns: then it stays and h is null
+typedef __bf16 pi_bf16x2 __attribute__((ext_vector_type(2)));
+static __device__ __forceinline__ uint32_t pi_round_pair(float a, float b) { const pi_bf16x2 v = { (__bf16) a, (__bf16) b }; return __builtin_bit_cast(uint32_t, v); }
+static __device__ __forceinline__ uint16_t pi_round_one(float a) { return __builtin_bit_cast(uint16_t, (__bf16) a); }
+static __device__ __forceinline__ void pi_round_store4(const pi_round_dst & r, int64_t row, int64_t i, float a, float b, float c, float d) { *(uint2 *) (r.h + row * r.stride + i) = make_uint2(pi_round_pair(a, b), pi_round_pair(c, d)); }
 // compute units the launching context's stream may use (pipeinfer_context_set_cu_range -> hipExtStreamCreateWithCUMask; 256 without a mask): what "one round of workgroups" means
 int pi_cu_count();
 const pi_tables & pi_get_tables();

@@ -610,7 +610,7 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
             return merge();
         }
         a.state = nullptr;
-        if (pa_takes(a, maps, PA_CACHE_TOKENS)) { pa_launch(a, maps, 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (hipStream_t) stream); PI_CHECK_LAUNCH(); return 0; }
+        if (pa_takes(a, maps, PA_CACHE_TOKENS)) { a.rd = pi_round_asked(0, (int64_t) heads * vdim); pa_launch(a, maps, 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (hipStream_t) stream); PI_CHECK_LAUNCH(); return 0; }
     }
 #define CA_GO(R, MP)     PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * visible * kv_heads * (maps * dim + vdim) + 4.0 * n_tok * heads * (maps * dim + vdim), (k_chunk_attention<R, MP>), dim3((unsigned) n_tok, (unsigned) kv_heads, (unsigned) (n_z * n_cs + (pool_here ? 1 : 0))), dim3(256), lds, \
                  (hipStream_t) stream, q, q_stride, k_cache, v_cache, cell_pos_dev, mask_dev, pos_dev, head_bias_dev, gate_dev, gate_stride, gate_act, scale, out_mult, weights, softcap, chunk, heads, kv_heads, dim, vdim, n_kv, tile, hpg, out, out_stride, \

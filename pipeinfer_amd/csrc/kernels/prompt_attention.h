@@ -17,6 +17,7 @@ struct pa_args {
     const float * gate; int64_t gs; int gate_act, gate_width;
     float out_mult, lam, eps;
     float * out; int64_t os;
+    pi_round_dst rd;                                                   // of the output (the launch that writes it)
     float * state; int first, last;                                    // the cells in several launches: [token][head][vdim sums | maximum | denominator] between them
 };
 // a launch over the cells [cell0, cell1); maps = 2: see ca_join_maps.  false: sizes or alignment that the kernel does not take (pa_takes)

@@ -351,19 +351,26 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             mult *= gt;
         }
 #pragma unroll
-        for (int j = 0; j < NV; j++)
+        for (int j = 0; j < NV; j++) {
+            const int v = v0 + 64 * j;
+            if (v >= vdim) continue;                                  // (vdim % 4 == 0)
+            float x[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int v = v0 + 64 * j + e;
-                if (v >= vdim) continue;
-                float x = o[0][j][e] * mult;
+                x[e] = o[0][j][e] * mult;
                 if (MAPS == 1 && A.gate && A.gate_width > 1) {
-                    float gt = A.gate[(int64_t) t * A.gs + (int64_t) h * vdim + v];
+                    float gt = A.gate[(int64_t) t * A.gs + (int64_t) h * vdim + v + e];
                     if (A.gate_act == PI_ACT_SIGMOID) gt = 1.0f / (1.0f + expf(-gt));
-                    x *= gt;
+                    x[e] *= gt;
                 }
-                A.out[(int64_t) t * A.os + (int64_t) h * vdim + v] = x;
             }
+            if (!A.rd.only) {
+                float * dst = A.out + (int64_t) t * A.os + (int64_t) h * vdim + v;
+#pragma unroll
+                for (int e = 0; e < 4; e++) dst[e] = x[e];
+            }
+            if (A.rd.h) pi_round_store4(A.rd, t, (int64_t) h * vdim + v, x[0], x[1], x[2], x[3]);
+        }
     }
 }
 

@@ -114,6 +114,11 @@ static thread_local int g_account_n_kv = 0;
 int pi_account_n_kv() { return g_account_n_kv; }
 extern "C" void pi_set_account_n_kv(int n_kv) { g_account_n_kv = n_kv > 0 ? n_kv : 0; }
 static thread_local int g_cu_count = 256;
+static thread_local pi_round_dst g_round = { nullptr, 0, 0, 0, 0 };
+extern "C" void pi_set_rounded_output(uint16_t * h, int64_t stride, int64_t from, int64_t n, int only) { g_round = { h, stride, from, n, only }; }
+pi_round_dst pi_round_take() { const pi_round_dst r = g_round; g_round.h = nullptr; return r; }
+pi_round_dst pi_round_asked(int64_t from, int64_t n) { return g_round.h && g_round.from == from && g_round.n == n ? pi_round_take() : pi_round_dst{ nullptr, 0, 0, 0, 0 }; }
+extern "C" int pi_rounded_output_written(void) { const bool met = g_round.h == nullptr; g_round.h = nullptr; return met; }
 int pi_cu_count() { return g_cu_count; }
 extern "C" void pi_set_cu_count(int n) { g_cu_count = n > 0 && n <= 256 ? n : 256; }
 // device-scope atomics only: the exchange at a run's start and the compare-and-swap of a cancel never tear, whichever stream runs first

@@ -23,7 +23,7 @@ static __device__ __forceinline__ float sm_sigmoid(float v) { return 1.0f / (1.0
 template <int S, int VEC, int NG>
 __global__ void __launch_bounds__(1024) k_hyper_step(const float * xin, int64_t xts, int64_t xss, int ns, const float * __restrict__ y, int64_t ys, const float * __restrict__ mix, const float * __restrict__ outc,
                                                      const float * __restrict__ in_next, const float * __restrict__ shift, const float * __restrict__ w, float eps, int n, float * xo, float * __restrict__ h, int64_t hs,
-                                                     const int32_t * __restrict__ abort_w) {
+                                                     const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     __shared__ float red[16];
     const int t = blockIdx.x;
@@ -98,8 +98,11 @@ __global__ void __launch_bounds__(1024) k_hyper_step(const float * xin, int64_t 
         const int i = (threadIdx.x + g * blockDim.x) * VEC;
         if (i >= n) continue;
         float * dst = h + (int64_t) t * hs + i;
-        if constexpr (VEC == 4) *(float4 *) dst = make_float4(u[g][0] * inv * wn[g][0], u[g][1] * inv * wn[g][1], u[g][2] * inv * wn[g][2], u[g][3] * inv * wn[g][3]);
-        else dst[0] = u[g][0] * inv * wn[g][0];
+        if constexpr (VEC == 4) {
+            const float4 y = make_float4(u[g][0] * inv * wn[g][0], u[g][1] * inv * wn[g][1], u[g][2] * inv * wn[g][2], u[g][3] * inv * wn[g][3]);
+            if (!rd.only) *(float4 *) dst = y;
+            if (rd.h) pi_round_store4(rd, t, i, y.x, y.y, y.z, y.w);
+        } else dst[0] = u[g][0] * inv * wn[g][0];
     }
 }
 static int hyper_step(const float * x_in, int64_t token_stride, int64_t stream_stride, int streams, const float * y, int64_t y_stride, const float * mix_dev, const float * out_dev, const float * in_next_dev,
@@ -113,8 +116,9 @@ static int hyper_step(const float * x_in, int64_t token_stride, int64_t stream_s
     const int groups = (n + (vec ? 3 : 0)) / (vec ? 4 : 1), ng = groups <= 1024 ? 1 : groups <= 4096 ? 4 : 16;
     const int threads = ng > 1 ? 1024 : (groups + 63) / 64 * 64;
     const double bytes = 4.0 * n * n_tok * ((stream_stride ? streams : 1) + (y ? 1 : 0) + (x_out ? streams : 0) + 1);
+    const pi_round_dst rd = vec ? pi_round_asked(0, n) : pi_round_dst{};
 #define HS_GO(S, V, G) PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, (k_hyper_step<S, V, G>), dim3((unsigned) n_tok), dim3((unsigned) threads), 0, (hipStream_t) stream, x_in, token_stride, stream_stride, streams, y, y_stride, mix_dev, \
-                                    out_dev, in_next_dev, shift_dev, w_dev, eps, n, x_out, h_out, h_stride, pi_abort_word())
+                                    out_dev, in_next_dev, shift_dev, w_dev, eps, n, x_out, h_out, h_stride, rd, pi_abort_word())
 #define HS_S(V, G) do { if (streams == 1) HS_GO(1, V, G); else if (streams == 2) HS_GO(2, V, G); else if (streams == 3) HS_GO(3, V, G); else if (streams == 4) HS_GO(4, V, G); else if (streams <= 8) HS_GO(8, V, G); else HS_GO(16, V, G); } while (0)
     if (vec) { if (ng == 1) HS_S(4, 1); else HS_S(4, 4); }
     else { if (ng == 1) HS_S(1, 1); else if (ng == 4) HS_S(1, 4); else HS_S(1, 16); }
@@ -249,7 +253,7 @@ extern "C" int pi_op_window_mask(const uint32_t * mask_dev, const int32_t * pos_
 // grid (token, 2): the query latent; the key / value latent and the rotated key part
 __global__ void __launch_bounds__(256) k_latent_prepare(const float * __restrict__ p, int64_t ps, int q_rank, const float * __restrict__ qw, int rank, const float * __restrict__ kw, int rot, const float2 * __restrict__ cs,
                                                         int n_pos, int pairing, float eps, const int32_t * __restrict__ pos, float * __restrict__ cq, int64_t cqs, float * __restrict__ cache, const int32_t * __restrict__ dyn,
-                                                        const int32_t * __restrict__ abort_w) {
+                                                        const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x, tid = threadIdx.x;
@@ -264,7 +268,11 @@ __global__ void __launch_bounds__(256) k_latent_prepare(const float * __restrict
     if (pi_abort_late(gone, abort_w)) return;
     const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float) n + eps);
     float * dst = is_q ? cq + (int64_t) t * cqs : cache + (int64_t) pi_cell_of(dyn, 0, t) * (rank + rot);
-    for (int i = tid; i < n; i += 256) dst[i] = src[i] * inv * w[i];
+    for (int i = tid; i < n; i += 256) {
+        const float y = src[i] * inv * w[i];
+        if (!is_q || !rd.only) dst[i] = y;
+        if (is_q && rd.h) rd.h[t * rd.stride + i] = pi_round_one(y);
+    }
     if (is_q) return;
     const float2 * row = cs + (int64_t) min(pos[t], n_pos - 1) * (rot / 2);
     for (int i = tid; i < rot; i += 256) {
@@ -286,6 +294,6 @@ extern "C" int pi_op_latent_prepare_ex(const float * p, int64_t p_stride, int q_
     if (q_rank < 1 || kv_rank < 1 || rot_dim < 0 || (rot_dim & 1) || (rot_dim > 0 && (!cs || half != rot_dim / 2 || !pos_dev)) || (pairing != PI_PAIR_HALVES && pairing != PI_PAIR_NEIGHBOURS)) { pi_set_error("pi_op_latent_prepare: latents of %d and %d values, %d rotated ones with a table over them", q_rank, kv_rank, rot_dim); return -1; }
     if (p_stride < (int64_t) q_rank + kv_rank + rot_dim || q_latent_stride < q_rank || !dyn_dev || !q_norm_w || !kv_norm_w) { pi_set_error("pi_op_latent_prepare: row strides below the sizes, or no norm weights / cell table"); return -1; }
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 8.0 * n_tok * (q_rank + kv_rank + rot_dim), k_latent_prepare, dim3((unsigned) n_tok, 2), dim3(256), 0, (hipStream_t) stream, p, p_stride, q_rank, q_norm_w, kv_rank, kv_norm_w, rot_dim, cs, n_pos, pairing, eps, pos_dev,
-                 q_latent, q_latent_stride, cache_dev, dyn_dev, pi_abort_word());
+                 q_latent, q_latent_stride, cache_dev, dyn_dev, pi_round_asked(0, q_rank), pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }

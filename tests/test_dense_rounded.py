@@ -74,3 +74,73 @@ def test_what_the_rounded_products_refuse():
     assert lib.pi_op_dense_rounded_ok(W, 72, 64) == 0
     assert lib.pi_op_dense_rounded(W, None, x.ptr, 72, 0, 0, 1, 64, out.ptr, 64, 0, 64, 0, None) == -1
     lib.pi_weight_free(W)
+
+
+def _asked(lib, U, op, out, from_, n, rows, only):
+    """runs op() with its columns [from_, from_ + n) asked for in bfloat16 as well: (rounded values, whether the operator wrote them)"""
+    h = U.Dev(np.full((rows, n + 8), 0x1234, np.uint16))
+    lib.pi_set_rounded_output(h.ptr, n + 8, from_, n, only)
+    L.check(op())
+    met = lib.pi_rounded_output_written()
+    got = h.get(np.uint16, (rows, n + 8))
+    assert (got[:, n:] == 0x1234).all()
+    return got[:, :n], met
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,n", [(33, 64), (40, 1000), (35, 2048), (33, 4096)])
+def test_rounded_outputs_are_the_fp32_ones_rounded(T, n):
+    """norms, gates, shifts and embeddings: the rounded rows against the rounded fp32 result of the same call; asked for alone they leave the fp32 rows as they were"""
+    from tests import gpu_util as U
+    lib = U.init()
+    rng = np.random.default_rng([T, n])
+    x, y, g = (U.Dev(rng.standard_normal((T, n)).astype(np.float32)) for _ in range(3))
+    w = U.Dev(1 + 0.1 * rng.standard_normal(n).astype(np.float32))
+    two = U.Dev(rng.standard_normal((T, 2 * n)).astype(np.float32))
+    mu, state, rec = U.Dev(rng.random((3, n)).astype(np.float32)), U.Dev(np.zeros((2, n), np.float32)), U.Dev(np.full(T, 1 << 30, np.int32))
+    table = bf16(rng.standard_normal((50, n)))
+    W = lib.pi_weight_upload(30, n, 50, table.ctypes.data_as(C.c_void_p), None)
+    tok = U.Dev(rng.integers(0, 50, T).astype(np.int32))
+    out = U.Dev(nbytes=4 * T * 3 * n)
+    heads = n // 64 if n % 64 == 0 else n // 8
+    ops = {
+        "rms_scale": (n, lambda: lib.pi_op_rms_scale(x.ptr, n, w.ptr, 1.0, 1e-5, n, T, g.ptr, n, y.ptr, n, 0.5, out.ptr, n, None, 0, None)),
+        "residual_norm": (n, lambda: lib.pi_op_residual_norm(x.ptr, y.ptr, n, None, w.ptr, 1e-5, n, T, None, out.ptr, n, None)),
+        "rms_post": (n, lambda: lib.pi_op_rms_post(y.ptr, n, None, None, 0, None, 1.0, w.ptr, x.ptr, n, 2.0, w.ptr, 1e-5, n, T, out.ptr, n, None, None, 0, None)),
+        "rms_post, next norm": (n, lambda: lib.pi_op_rms_post(y.ptr, n, w.ptr, g.ptr, n, w.ptr, 0.5, w.ptr, x.ptr, n, 2.0, w.ptr, 1e-5, n, T, two.ptr, 2 * n, w.ptr, out.ptr, n, None)),
+        "head_norm_gate": (n, lambda: lib.pi_op_head_norm_gate(y.ptr, n, heads, n // heads, w.ptr, 1, g.ptr, n, 1, 1e-5, T, out.ptr, n, None)),
+        "token_shift": (3 * n, lambda: lib.pi_op_token_shift(x.ptr, n, n, mu.ptr, 3, state.ptr, rec.ptr, T, out.ptr, 3 * n, None)),
+        "glu_mul": (n, lambda: lib.pi_op_glu_mul(two.ptr, 2 * n, n, T, out.ptr, n, None)),
+        "glu_mul_ex": (n, lambda: lib.pi_op_glu_mul_ex(two.ptr, 2 * n, n, 2, 7.0, -1, T, out.ptr, n, None)),
+        "embed": (n, lambda: lib.pi_op_embed(W, tok.ptr, T, 0.7, out.ptr, None)),
+        "embed_pair": (n, lambda: lib.pi_op_embed_pair(W, tok.ptr, T, 0.7, W, tok.ptr, out.ptr, None)),
+    }
+    for name, (width, op) in ops.items():
+        got, met = _asked(lib, U, op, out, 0, width, T, 0)
+        full = out.get(np.float32, (T, width), 0, T * width)
+        assert met == 1, name
+        assert np.array_equal(got, bf16(full)), name
+        alone, met = _asked(lib, U, op, out, 0, width, T, 1)
+        assert met == 1 and np.array_equal(alone, got), name
+        _, met = _asked(lib, U, op, out, 0, width - 8, T, 0)      # not the operator's rows: not met, and not left behind for the next one
+        assert met == 0 and lib.pi_rounded_output_written() == 1, name
+        assert np.array_equal(out.get(np.float32, (T, width), 0, T * width), full), name
+    lib.pi_weight_free(W)
+
+
+@pytest.mark.gpu
+def test_a_products_columns_rounded_for_the_next():
+    from tests import gpu_util as U
+    lib = U.init()
+    rng = np.random.default_rng(3)
+    rows, K, T = 1000, 128, 77
+    w = bf16(rng.standard_normal((rows, K)))
+    W = lib.pi_weight_upload(30, K, rows, w.ctypes.data_as(C.c_void_p), None)
+    xh, out = U.Dev(bf16(rng.standard_normal((T, K)))), U.Dev(nbytes=4 * T * rows)
+    got, met = _asked(lib, U, lambda: lib.pi_op_dense_rounded(W, None, xh.ptr, K, 0, 0, 1, T, out.ptr, rows, 4, rows // 2, 0, None), out, 488, 64, T, 0)
+    assert met == 1 and np.array_equal(got, bf16(out.get(np.float32, (T, rows))[:, 488:552]))
+    odd = U.Dev(rng.standard_normal((T, 67)).astype(np.float32))      # rows that no 16-byte load can take
+    h = U.Dev(nbytes=2 * T * 64)
+    L.check(lib.pi_op_round_bf16(odd.ptr + 4, 67, 64, T, h.ptr, 64, None))
+    assert np.array_equal(h.get(np.uint16, (T, 64)), bf16(odd.get(np.float32, (T, 67))[:, 1:65]))
+    lib.pi_weight_free(W)
