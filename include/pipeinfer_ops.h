@@ -220,6 +220,10 @@ PI_API int pi_op_moe_experts(const pi_weight * w_up, const pi_weight * w_down, i
  * matrix cores 64 slots at a time.  up_dev: [n_tok * top][ff], dn_dev: [n_tok * top][width], idx_dev: pi_op_moe_grouped_index_ints(n_tok, top, n_exp) int32 */
 PI_API int pi_op_moe_grouped_ok(const pi_weight * w_up, const pi_weight * w_down, int n_exp, int ff, int glu, int n_tok, int top, int exact);
 PI_API size_t pi_op_moe_grouped_index_ints(int n_tok, int top, int n_exp);
+PI_API int pi_op_moe_rounded_ok(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, int64_t x_stride, int n_tok, int top);
+/* the same from inputs in bfloat16 (xh; x: the same in fp32, what identity experts hand on), up_dev [n_tok * top][ff] in bfloat16; pi_op_moe_rounded_ok says for which passes */
+PI_API int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh_dev, int64_t xh_stride, const float * x_dev, int64_t x_stride, const int32_t * sel_dev,
+                                     const float * selw_dev, int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out_dev, int64_t out_stride, void * stream);
 PI_API int pi_op_moe_experts_grouped(const pi_weight * w_up, const pi_weight * w_down, int n_exp, int ff, const float * x_dev, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev, int n_tok, int top,
                                      float * up_dev, float * dn_dev, int32_t * idx_dev, float * out_dev, int64_t out_stride, void * stream);
 

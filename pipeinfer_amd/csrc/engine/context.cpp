@@ -928,10 +928,14 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         trace(ctx, "mix", (int) il, A, hv, n_tok);
         OP_OK(dense(ctx, W.w_o, A, hv, n_tok, Y, width, PI_ACT_NONE, width, PI_ACT_NONE, s, ah, hv));
         xh = x_rounded(il + 1);
-        OP_OK(op_rounded(ctx, H.has_mlp ? nullptr : xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
+        // experts without a gate, a prompt: by expert on the matrix cores, from the stream in bfloat16
+        const bool moe_h = H.has_mlp && !ex && pi_op_moe_rounded_ok(W.e_up, W.e_down, H.n_expert, H.ff, width, n_tok, H.top);
+        OP_OK(op_rounded(ctx, H.has_mlp ? (moe_h ? ctx->x_h : nullptr) : xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
         if (H.has_mlp) {
             OP_OK(pi_op_moe_route(W.router, W.correction, x, width, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s));
-            if (pi_op_moe_grouped_ok(W.e_up, W.e_down, H.n_expert, H.ff, 0, n_tok, H.top, ex))                                                     // prompts: by expert, on the matrix cores
+            if (moe_h)
+                OP_OK(pi_op_moe_experts_rounded(W.e_up, W.e_down, H.n_expert, H.ff, ctx->x_h, width, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, (uint16_t *) ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
+            else if (pi_op_moe_grouped_ok(W.e_up, W.e_down, H.n_expert, H.ff, 0, n_tok, H.top, ex))
                 OP_OK(pi_op_moe_experts_grouped(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
             else
                 OP_OK(pi_op_moe_experts(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ex, ctx->moe_up, Y, width, s));

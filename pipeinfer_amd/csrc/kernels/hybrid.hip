@@ -15,6 +15,7 @@
 #include "kernel_timing.h"
 #include "prompt_attention.h"
 #include "dense_tile.h"
+#include "dense_async.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1994,6 +1995,35 @@ __global__ void __launch_bounds__(64 * WN * WT * KG, 2) k_moe_tile(const uint16_
     }
 }
 
+// The same tiles from inputs that are bfloat16 already (dense_async.h), the hidden layer left in bfloat16 for the second product: what the engine's prompts take where the experts have no gate.  us for both products of top-2 of 8
+// experts, k_moe_tile / these: 4096 x 2048 at 2048 tokens 88 + 98 / 71 + 81, 2048 x 1024 at 512 23.7 + 22 / 19.9 + 18.2
+template <int BN, int BT, int WN, int WT, int S, bool UP>
+__global__ void __launch_bounds__(64 * WN * WT, 1) k_moe_async(const uint16_t * __restrict__ W, int64_t K, int rows, const uint16_t * __restrict__ B, int64_t bs, int top, const int32_t * __restrict__ idx, int max_tiles,
+                                                               float * __restrict__ out, uint16_t * __restrict__ out_h, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w, 1)) return;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[DA_LDS_BYTES(BN, BT, S)];
+    const int row_blocks = (rows + BN - 1) / BN, total = idx[0] * row_blocks, per = (total + 7) / 8, at = (int) (blockIdx.x >> 3), work = (int) (blockIdx.x & 7) * per + at;
+    if (at >= per || work >= total) return;
+    const int grp = work / (8 * row_blocks), in_grp = work % (8 * row_blocks), gsz = min(8, idx[0] - 8 * grp), tile = 8 * grp + in_grp % gsz, n0 = in_grp / gsz * BN;
+    const int32_t * tile_e = idx + 1, * tile_s = tile_e + max_tiles, * tile_n = tile_s + max_tiles, * order = tile_n + max_tiles;
+    const int e = tile_e[tile], start = tile_s[tile], len = tile_n[tile], wave = threadIdx.x >> 6;
+    dt_f32x4 acc[BN / WN / 16][BT / WT / 16];
+    da_tile<BN, BT, WN, WT, S>(W + ((int64_t) e * rows + n0) * K, [&](int r) { return (uint32_t) (min(r, rows - 1 - n0) * K * 2); },
+                               B, [&](int r) { const int slot = order[start + min(r, len - 1)]; return (uint32_t) ((UP ? slot / top : slot) * bs * 2); }, (int) (K / 64), lds, acc);
+    __syncthreads();                                                   // (the operands of every wave are read)
+    constexpr int SHARE = DA_LDS_BYTES(BN, BT, S) / (WN * WT) & ~15;
+    const int row0 = n0 + (wave / WT) * (BN / WN), si0 = (wave % WT) * (BT / WT);
+    da_rows<BN / WN / 16, BT / WT / 16, SHARE>(acc, lds + wave * SHARE, [&](int t, int r, dt_f32x4 v) __attribute__((always_inline)) {
+        if (si0 + t >= len || row0 + r >= rows) return;               // (rows % 64 == 0)
+        const int64_t at = (int64_t) order[start + si0 + t] * rows + row0 + r;
+        if (UP) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) { v[i] = fmaxf(v[i], 0.0f); v[i] *= v[i]; }
+            *(uint2 *) (out_h + at) = make_uint2(pi_round_pair(v[0], v[1]), pi_round_pair(v[2], v[3]));
+        } else *(dt_f32x4 *) (out + at) = v;
+    });
+}
+
 __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ dn, int64_t width, int n_exp, int top, const float * __restrict__ x, int64_t xs, const int32_t * __restrict__ sel,
                                                      const float * __restrict__ selw, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w)) return;
@@ -2027,6 +2057,17 @@ static void moe_tile_launch(const uint16_t * w, int64_t K, int rows, const float
     else MOE_GO(64, 64, 2);
 #undef MOE_GO
 #undef MOE_GO2
+}
+// the tile that needs the least time by rounds of 256 workgroups, as async_tile_of (dense.hip)
+template <bool UP>
+static void moe_async_launch(const uint16_t * w, int64_t K, int rows, const uint16_t * b, int64_t bs, int top, const int32_t * idx, int mt, int tl, int est, float * out, uint16_t * out_h, int nta, double bytes, hipStream_t s) {
+    auto cost = [&](int bn, double us) { return std::max(1.0, (double) est * ((rows + bn - 1) / bn) / 256) * us; };      // (the number of tiles is an estimate: no whole rounds)
+#define MOE_GO(BN, BT, WN, WT, S) PI_KT_LAUNCH(PI_KT_MMQ, PI_BF16, nta, bytes, (k_moe_async<BN, BT, WN, WT, S, UP>), dim3((unsigned) (((int64_t) mt * ((rows + BN - 1) / BN) + 7) / 8 * 8)), dim3(64 * WN * WT), 0, s, \
+                                               w, K, rows, b, bs, top, idx, mt, out, out_h, pi_abort_word())
+    if (tl == 128) { if (cost(256, 31.0) < cost(128, 19.5)) MOE_GO(256, 128, 4, 2, 3); else MOE_GO(128, 128, 4, 2, 4); }
+    else if (cost(64, 6.3) < cost(32, 4.6)) MOE_GO(64, 64, 4, 2, 4);
+    else MOE_GO(32, 64, 2, 2, 4);
+#undef MOE_GO
 }
 // ints of index scratch the grouped path needs for a pass of n_tok tokens
 extern "C" size_t pi_op_moe_grouped_index_ints(int n_tok, int top, int n_exp) { const int ns = n_tok * top; return (size_t) 1 + 3 * (size_t) moe_max_tiles(ns, n_exp) + (size_t) ns; }
@@ -2067,6 +2108,32 @@ extern "C" int pi_op_moe_experts_grouped_glu(const pi_weight * wup, const pi_wei
     moe_tile_launch<true>((const uint16_t *) wup->p0, width, ff * upr, x, x_stride, top, idx_dev, mt, tl, est, glu, limit, up_dev, nta, bytes, s);
     PI_CHECK_LAUNCH();
     moe_tile_launch<false>((const uint16_t *) wdown->p0, ff, (int) width, up_dev, (int64_t) ff * upr, top, idx_dev, mt, tl, est, glu, limit, dn_dev, nta, bytes, s);
+    PI_CHECK_LAUNCH();
+    PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 4.0 * n_tok * width * (top + 2), k_moe_combine, dim3((unsigned) ((width + 255) / 256), (unsigned) n_tok), dim3(256), 0, s,
+                 dn_dev, width, n_exp, top, x, x_stride, sel_dev, selw_dev, out, out_stride, pi_abort_word());
+    PI_CHECK_LAUNCH(); return 0;
+}
+// whether pi_op_moe_experts_rounded takes the pass: whole steps of both products' K, offsets of a tile's rows in 32 bits
+extern "C" int pi_op_moe_rounded_ok(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, int64_t x_stride, int n_tok, int top) {
+    return pi_op_moe_grouped_ok(wup, wdown, n_exp, ff, PI_GLU_OFF, n_tok, top, 0) && wup->ne0 % 64 == 0 && ff % 64 == 0 && wup->ne0 < (1 << 22) && ff < (1 << 22) && (int64_t) n_tok * x_stride < (1ll << 31) && (int64_t) n_tok * top * ff < (1ll << 31);
+}
+// pi_op_moe_experts_grouped from inputs in bfloat16 (xh); x: the same in fp32, what identity experts hand on.  up_dev holds the hidden layer, bfloat16 [n_tok * top][ff]
+extern "C" int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh, int64_t xh_stride, const float * x, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev,
+                                         int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out, int64_t out_stride, void * stream) {
+    if (n_tok <= 0) return 0;
+    if (!pi_op_moe_rounded_ok(wup, wdown, n_exp, ff, xh_stride, n_tok, top)) { pi_set_error("pi_op_moe_experts_rounded: this shape takes pi_op_moe_experts or pi_op_moe_experts_grouped"); return -1; }
+    if (wup->type != PI_BF16 || wdown->type != PI_BF16 || wup->ne1 != (int64_t) n_exp * ff || wdown->ne0 != ff || wdown->ne1 != (int64_t) n_exp * wup->ne0 || xh_stride % 8 || xh_stride < wup->ne0 || (((uintptr_t) xh | (uintptr_t) up_dev | (uintptr_t) dn_dev) & 15)) {
+        pi_set_error("pi_op_moe_experts_rounded: expert matrices must be bfloat16 [experts * ff][width] and [experts * width][ff], inputs 16-byte aligned rows"); return -1;
+    }
+    hipStream_t s = (hipStream_t) stream;
+    const int64_t width = wup->ne0;
+    const int ns = n_tok * top, mt = moe_max_tiles(ns, n_exp), nta = std::min(n_tok, PI_KT_MAXNT - 1), tl = moe_tile_len(ns, n_exp), est = (ns + tl - 1) / tl + std::min(n_exp, ns) / 2;
+    const double bytes = std::min<double>(ns, n_exp) * 2.0 * ff * width + 2.0 * ns * (width + ff);
+    PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 8.0 * ns, k_moe_group, dim3(1), dim3(256), 0, s, sel_dev, ns, n_exp, mt, tl, idx_dev, pi_abort_word());
+    PI_CHECK_LAUNCH();
+    moe_async_launch<true>((const uint16_t *) wup->p0, width, ff, xh, xh_stride, top, idx_dev, mt, tl, est, nullptr, up_dev, nta, bytes, s);
+    PI_CHECK_LAUNCH();
+    moe_async_launch<false>((const uint16_t *) wdown->p0, ff, (int) width, up_dev, ff, top, idx_dev, mt, tl, est, dn_dev, nullptr, nta, bytes, s);
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 4.0 * n_tok * width * (top + 2), k_moe_combine, dim3((unsigned) ((width + 255) / 256), (unsigned) n_tok), dim3(256), 0, s,
                  dn_dev, width, n_exp, top, x, x_stride, sel_dev, selw_dev, out, out_stride, pi_abort_word());

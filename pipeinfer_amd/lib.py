@@ -176,6 +176,8 @@ def _declare(lib):
     lib.pi_op_moe_experts_grouped_act.argtypes = [vp, vp, i32, i32, i32, vp, i64, vp, vp, i32, i32, vp, vp, vp, vp, i64, vp]
     # blocks with the norm after the sum, recurrences with a decay per key channel, soft-max attention in chunks
     lib.pi_op_dense_segments.argtypes = [vp, vp, i64, i64, i64, i32, i32, vp, i64, i32, i64, i32, i32, vp]
+    lib.pi_op_moe_rounded_ok.argtypes = [vp, vp, i32, i32, i64, i32, i32]
+    lib.pi_op_moe_experts_rounded.argtypes = [vp, vp, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, vp, vp, vp, vp, i64, vp]
     lib.pi_set_rounded_output.argtypes = [vp, i64, i64, i64, i32]
     lib.pi_op_round_bf16.argtypes = [vp, i64, i64, i32, vp, i64, vp]
     lib.pi_op_dense_rounded_ok.argtypes = [vp, i64, i32]

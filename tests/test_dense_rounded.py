@@ -144,3 +144,40 @@ def test_a_products_columns_rounded_for_the_next():
     L.check(lib.pi_op_round_bf16(odd.ptr + 4, 67, 64, T, h.ptr, 64, None))
     assert np.array_equal(h.get(np.uint16, (T, 64)), bf16(odd.get(np.float32, (T, 67))[:, 1:65]))
     lib.pi_weight_free(W)
+
+
+# tiles of 64 and 128 slots by every number of rows; one step of K and fewer than stages; an expert without tokens, identity experts, runs that end inside a tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,I,ff,width,T,top", [(2, 1, 128, 192, 300, 2), (8, 2, 64, 3136, 200, 2), (8, 0, 64, 1536, 210, 2), (70, 3, 64, 64, 40, 6), (1, 0, 64, 64, 33, 1), (3, 0, 64, 128, 700, 2), (2, 0, 64, 8256, 1500, 2), (8, 0, 2048, 256, 3000, 2)])
+def test_experts_of_rounded_inputs(E, I, ff, width, T, top):
+    from tests import gpu_util as U
+    lib = U.init()
+    rng = np.random.default_rng([E, T])
+    x = rng.standard_normal((T, width)).astype(np.float32)
+    ups, downs = bf16(rng.standard_normal((E, ff, width)) * width ** -0.5), bf16(rng.standard_normal((E, width, ff)) * ff ** -0.5)
+    sel = np.stack([rng.permutation(E + I)[:top] for _ in range(T)]).astype(np.int32)
+    sel[sel == 1] = 0 if E > 3 else 1
+    selw = rng.uniform(0.1, 1.0, (T, top)).astype(np.float32)
+    ud = lib.pi_weight_upload(30, width, E * ff, ups.ctypes.data_as(C.c_void_p), None)
+    dd = lib.pi_weight_upload(30, ff, E * width, downs.ctypes.data_as(C.c_void_p), None)
+    xd, xh, sd, wd = U.Dev(x), U.Dev(bf16(x)), U.Dev(sel), U.Dev(selw)
+    hd, nd, od = U.Dev(nbytes=2 * T * top * ff), U.Dev(nbytes=4 * T * top * width), U.Dev(nbytes=4 * T * width)
+    idx = U.Dev(nbytes=4 * lib.pi_op_moe_grouped_index_ints(T, top, E))
+    assert lib.pi_op_moe_rounded_ok(ud, dd, E, ff, width, T, top) == 1
+    L.check(lib.pi_op_moe_experts_rounded(ud, dd, E, ff, xh.ptr, width, xd.ptr, width, sd.ptr, wd.ptr, T, top, hd.ptr, nd.ptr, idx.ptr, od.ptr, width, None))
+    hidden, got = wide(hd.get(np.uint16, (T, top, ff))).astype(np.float64), od.get(np.float32, (T, width))
+    xr = wide(bf16(x)).astype(np.float64)
+    want = np.zeros((T, width))
+    for e in range(E + I):
+        for k in range(top):
+            at = np.flatnonzero(sel[:, k] == e)
+            if e >= E:
+                want[at] += selw[at, k, None] * x[at]
+                continue
+            h = np.maximum(xr[at] @ wide(ups[e]).astype(np.float64).T, 0) ** 2
+            # a hidden value is the fp32 one rounded to bfloat16: 2^-8 of it, and the fp32 sum's own error (squared)
+            assert (np.abs(hidden[at, k] - h) <= 2.0 ** -8 * h + 1e-5).all()
+            want[at] += selw[at, k, None] * (hidden[at, k] @ wide(downs[e]).astype(np.float64).T)
+    assert np.sqrt(((got - want) ** 2).mean()) < 3e-6 * np.sqrt((want ** 2).mean())      # (fp32 sums of at most 8256 terms)
+    for w in (ud, dd):
+        lib.pi_weight_free(w)
