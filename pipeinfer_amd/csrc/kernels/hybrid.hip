@@ -582,6 +582,13 @@ static __device__ __forceinline__ void la_find_piece(const int * recs, int n_tok
         ord += own[k];
     }
 }
+// whether all tokens of the pass are one sequence's (every thread of the block calls): most prompts, for which nothing has to be searched
+static __device__ __forceinline__ bool la_one_run(const int32_t * __restrict__ rec, int n_tok) {
+    const int own = rec[0];
+    int other = 0;
+    for (int t = threadIdx.x; t < n_tok; t += blockDim.x) other |= (rec[t] ^ own) & ~LA_FRESH;
+    return !__syncthreads_or(other);
+}
 template <int DPT>
 __global__ void __launch_bounds__(256) k_linear_attention(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int dim, int vdim, int vstored, int R,
                                                           const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
@@ -680,71 +687,80 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
         for (int ii = 0; ii < DPT; ii++) { const int i = sp * DPT + ii; if (i < dim) S_to[(int64_t) i * vdim + j] = S[ii]; }
 }
 
-// The pieces of a long pass on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), 64 tokens long, for key widths of 32 DI <= 128.  What bounds the token loop of k_linear_attention is its chain: a token's state
+// Long passes on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), pieces of 64 or 32 tokens, for key widths of 32 DI <= 128.  What bounds the token loop of k_linear_attention is its chain: a token's state
 // value waits for the one before, two products per state value on the vector units.  Per head and piece, with a_t = lambda_1 .. lambda_t and D[t][j] = lambda_{j+1} .. lambda_t (products only, no quotients):
-//   states   L = sum_j (lambda_{j+1} .. lambda_64 s_j k_j) v_j^T                 (as mode 1)
-//   outputs  O = a_t (Q S_in) + (Q K^T o D s) V;  a run's last piece also leaves a_64 S_in + L   (as mode 2)
-// A piece of up to 16 or 32 tokens takes as many tiles (a run of 16 tokens alone: 42 us with all four, 23).
-// 2048 tokens, 32 heads of 128 x 128: 2 x 759 us -> 98 + 124, the scan between them 58 -> 34 (half the pieces, half the memory); 512 tokens, 16 heads: 2 x 93 -> 27 + 48, 11 -> 7.
+//   O = a_t (Q S_in) + (Q K^T o D s) V,   S_out = a_64 S_in + sum_j (lambda_{j+1} .. lambda_64 s_j k_j) v_j^T
+// k_linear_pieces: a pass of up to 64 tokens, every run one piece of up to 16, 32 or 64 tokens (a run of 16 tokens alone: 42 us with all four tiles, 23).  More tokens: k_linear_scores and k_linear_walk.
 #define LM_TB 64
 #define LM_MAX_TOKENS 16384                       // (the pass's slot words in LDS beside the 54 KB of a piece)
 typedef float hy_f32x4 __attribute__((ext_vector_type(4)));
 static __device__ __forceinline__ hy_f32x4 hy_mfma(float a, float b, hy_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 // base[i] with a 32-bit offset from a uniform base (an address per load in flight would not stay in registers)
+typedef float hy_f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 static __device__ __forceinline__ float lm_at(const float * __restrict__ base, uint32_t i) { return *(const float *) ((const char *) base + i * 4u); }
+static __device__ __forceinline__ hy_f32x4 lm_at4(const float * __restrict__ base, uint32_t i) { return *(const hy_f32x4_u *) ((const char *) base + i * 4u); }
 // the value of token j of the piece in column c: the values end at vstored, a further column is ones
 static __device__ __forceinline__ float lm_value(const float * __restrict__ vp, uint32_t j, uint32_t stride, int c, int vstored) { const float x = lm_at(vp, j * stride + (uint32_t) min(c, vstored - 1)); return c < vstored ? x : 1.0f; }
-template <int DI, bool OUTPUTS>
+// the decays of a piece's tokens (a wave, a lane per token): decay, factor on k v^T (0 behind the piece's end), products of a tile of 16 up to this token and from the next one on, products 1 .. t, t + 1 .. 64 times the factor, a tile's
+static __device__ __forceinline__ void lm_factors(int lane, int len, int64_t at, const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int h, float * lam, float * sc, float * pre,
+                                                  float * suf, float * upto, float * from, float * whole) {
+    const int n = lane & 15, g = lane >> 4;
+    const float l = lane >= len ? 1.0f : tdecay ? tdecay[at] : decay[h], s = lane < len ? (tscale ? tscale[at] : 1.0f) : 0.0f;
+    float a = l, b = l;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) { const float x = __shfl_up(a, o, 16), y = __shfl_down(b, o, 16); if (n >= o) a *= x; if (n + o < 16) b *= y; }
+    const float after = __shfl_down(b, 1, 16);
+    float w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = __shfl(a, 16 * i + 15, 64);
+    float before = 1.0f, behind = 1.0f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) { if (i < g) before *= w[i]; if (i > g) behind *= w[i]; }
+    const float s1 = n == 15 ? 1.0f : after;
+    lam[lane] = l; sc[lane] = s;
+    pre[lane] = a; suf[lane] = s1; upto[lane] = before * a; from[lane] = s1 * behind * s;
+    if (n == 15) whole[g] = a;
+}
+// lambda_{j+1} .. lambda_t inside a tile of 16, in that order (a loop over them made a trip to LDS for each)
+static __device__ __forceinline__ float lm_inside(const float * lam, int j, int t) {
+    float d = 1.0f;
+#pragma unroll
+    for (int m = 1; m < 16; m++) { const float l = lam[m]; d *= m > j && m <= t ? l : 1.0f; }
+    return d;
+}
+template <int DI>
 __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim, int vstored,
                                                        const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
-                                                       float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+                                                       float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     if (pi_aborted(abort_w)) return;
     constexpr int DIM = 32 * DI, PITCH = DIM + 4, PP = LM_TB + 4;
-    __shared__ __attribute__((aligned(16))) float qk[LM_TB * PITCH];  // the piece's queries (OUTPUTS), then, where its state is wanted, its keys
-    __shared__ __attribute__((aligned(16))) float pt[OUTPUTS ? LM_TB * PP : 4];
+    __shared__ __attribute__((aligned(16))) float qk[LM_TB * PITCH];  // the queries, then the keys
+    __shared__ __attribute__((aligned(16))) float pt[LM_TB * PP];
     __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
-    __shared__ float lam[LM_TB], sc[LM_TB], upto[LM_TB], from[LM_TB], pre[LM_TB], suf[LM_TB], whole[4];     // decay, factor on k v^T; products: 1 .. t, t + 1 .. 64, and the same inside a tile of 16; a tile's
+    __shared__ __attribute__((aligned(16))) float lam[LM_TB]; __shared__ float sc[LM_TB], upto[LM_TB], from[LM_TB], pre[LM_TB], suf[LM_TB], whole[4];     // decay, factor on k v^T; products: 1 .. t, t + 1 .. 64, and the same inside a tile of 16; a tile's
     extern __shared__ int lm_recs[];              // the slot words of the pass
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
     for (int t = tid; t < n_tok; t += 256) lm_recs[t] = rec[t];
     __syncthreads();
     const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
-    if (tid < 64) la_find_piece(lm_recs, n_tok, bnd, n_runs, LM_TB, blockIdx.y, seg);
+    if (tid < 64) la_find_piece(lm_recs, n_tok, bnd, n_runs, 0, blockIdx.y, seg);
     __syncthreads();
-    const int first = seg[0], len = seg[1], word = seg[2], last = seg[3];
-    if (len == 0 || word < 0 || (!OUTPUTS && last)) return;
+    const int first = seg[0], len = seg[1], word = seg[2];
+    if (len == 0 || word < 0) return;
     const int hq = h / hpg;
     const float * qp = q + (int64_t) first * stride + (int64_t) hq * DIM, * kp = k + (int64_t) first * stride + (int64_t) hq * DIM, * vp = v + (int64_t) first * stride + (int64_t) h * vstored;
     const int tiles = len <= 16 ? 1 : len <= 32 ? 2 : 4;              // of 16 tokens
     auto stage = [&](const float * src) {                             // rows behind the last repeat it: nothing of theirs is used
         for (int i = tid; i < 16 * tiles * DIM; i += 256) { const int t = i / DIM, d = i % DIM; qk[t * PITCH + d] = src[(int64_t) min(t, len - 1) * stride + d]; }
     };
-    stage(OUTPUTS ? qp : kp);
-    if (wave == 0) {
-        const int64_t at = (int64_t) (first + min(lane, len - 1)) * tds + h;
-        const float l = lane >= len ? 1.0f : tdecay ? tdecay[at] : decay[h];
-        float a = l, b = l;                                            // products of the tile up to this token, and from it on
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) { const float x = __shfl_up(a, o, 16), y = __shfl_down(b, o, 16); if (n >= o) a *= x; if (n + o < 16) b *= y; }
-        const float after = __shfl_down(b, 1, 16);
-        float w[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) w[i] = __shfl(a, 16 * i + 15, 64);
-        float before = 1.0f, behind = 1.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) { if (i < g) before *= w[i]; if (i > g) behind *= w[i]; }
-        const float s1 = n == 15 ? 1.0f : after;
-        lam[lane] = l; sc[lane] = lane < len ? (tscale ? tscale[at] : 1.0f) : 0.0f;
-        pre[lane] = a; suf[lane] = s1; upto[lane] = before * a; from[lane] = s1 * behind;
-        if (n == 15) whole[g] = a;
-    }
+    stage(qp);
+    if (wave == 0) lm_factors(lane, len, (int64_t) (first + min(lane, len - 1)) * tds + h, decay, tdecay, tscale, h, lam, sc, pre, suf, upto, from, whole);
     __syncthreads();
     const int64_t per = (int64_t) DIM * vdim;
-    float * S_scr = scratch + ((int64_t) blockIdx.y * heads + h) * per;
-    const float * S_in = OUTPUTS && !scratch ? state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per : S_scr;      // (no scratch: a piece is its sequence's whole run)
-    const bool zero = OUTPUTS && !scratch && (word & LA_FRESH);
+    float * S_hbm = state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per;
+    const bool zero = (word & LA_FRESH) != 0;
     const int n_tiles = (vdim + 15) / 16;
-    if constexpr (OUTPUTS) {
+    {
         // (Q K^T o D s) transposed: tiles (rows j, columns t) on and below the diagonal, shared out among the waves; a lane's four rows are consecutive values of row t of pt
         for (int i = wave; i < tiles * (tiles + 1) / 2; i += 4) {
             const int tt = i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3, jt = i - tt * (tt + 1) / 2, j = 16 * jt + n;
@@ -762,9 +778,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int jr = 16 * jt + 4 * g + r;
-                float d = 1.0f;
-                if (jt < tt) d = suf[jr] * between * pre[t];
-                else for (int m = jr + 1; m <= t; m++) d *= lam[m];
+                const float d = jt < tt ? suf[jr] * between * pre[t] : lm_inside(lam + 16 * tt, 4 * g + r, n);
                 a[r] = jr <= t && jr < len ? a[r] * d * sc[jr] : 0.0f;
             }
             *(hy_f32x4 *) &pt[t * PP + 16 * jt + 4 * g] = a;
@@ -778,7 +792,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
 #pragma unroll
                 for (int s = 0; s < 2 * DI; s++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) { const float x = lm_at(S_in, (uint32_t) (16 * s + 4 * g + i) * (uint32_t) vdim + (uint32_t) cc); sv[4 * s + i] = zero ? 0.0f : x; }
+                    for (int i = 0; i < 4; i++) { const float x = lm_at(S_hbm, (uint32_t) (16 * s + 4 * g + i) * (uint32_t) vdim + (uint32_t) cc); sv[4 * s + i] = zero ? 0.0f : x; }
                 float vv[4 * MT];                                          // values: rows 16 jt + 4 g + r
 #pragma unroll
                 for (int i = 0; i < 4 * MT; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored); }
@@ -838,13 +852,11 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
         if (tiles == 1) outputs(std::integral_constant<int, 1>{});
         else if (tiles == 2) outputs(std::integral_constant<int, 2>{});
         else outputs(std::integral_constant<int, 4>{});
-        if (!last) return;
         __syncthreads();
         stage(kp);
         __syncthreads();
     }
-    // the state of the piece: from zero (scratch), or from S_in (the slot)
-    float * S_to = OUTPUTS ? state + ((int64_t) (word & ~LA_FRESH) * heads + h) * per : S_scr;
+    // the slot's new state
     const float all = upto[LM_TB - 1];
     auto states = [&](auto n_mt) {
         constexpr int MT = decltype(n_mt)::value;
@@ -852,7 +864,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
             const int c = 16 * nt + n, cc = min(c, vdim - 1);
             float vv[4 * MT];
 #pragma unroll
-            for (int i = 0; i < 4 * MT; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = j < len ? lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored) * (from[j] * sc[j]) : 0.0f; }
+            for (int i = 0; i < 4 * MT; i++) { const int j = 16 * (i >> 2) + 4 * g + (i & 3); vv[i] = j < len ? lm_value(vp, min(j, len - 1), (uint32_t) stride, cc, vstored) * from[j] : 0.0f; }
             hy_f32x4 acc[2 * DI];
 #pragma unroll
             for (int m = 0; m < 2 * DI; m++) acc[m] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
@@ -869,14 +881,254 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
                         const uint32_t at = ((uint32_t) (16 * m + 4 * g + r) * (uint32_t) vdim + (uint32_t) c) * 4u;
-                        if (OUTPUTS && r == 0) __builtin_amdgcn_sched_barrier(0);
-                        *(float *) ((char *) S_to + at) = !OUTPUTS || zero ? acc[m][r] : fmaf(all, *(const float *) ((const char *) S_in + at), acc[m][r]);
+                        if (r == 0) __builtin_amdgcn_sched_barrier(0);
+                        *(float *) ((char *) S_hbm + at) = zero ? acc[m][r] : fmaf(all, *(const float *) ((const char *) S_hbm + at), acc[m][r]);
                     }
         }
     };
     if (tiles == 1) states(std::integral_constant<int, 1>{});
     else if (tiles == 2) states(std::integral_constant<int, 2>{});
     else states(std::integral_constant<int, 4>{});
+}
+
+// A pass of more than 64 tokens, in pieces of 32: the scores of every piece side by side, then every run walked piece by piece with its state in registers.  (States of all pieces from zero, a scan that chains them and the outputs
+// from every piece's true state moved 64 KB per piece and head four times: 2048 tokens, 32 heads of 128 x 128: 93 + 31 + 140 us, now 30 + 87; 512 tokens, 16 heads: 27 + 8 + 60, now 9 + 24.)
+// scratch per (piece, head): (Q K^T o D s) [32 t][32 j], nothing in the tile above the diagonal | lambda_1 .. lambda_t [32] | lambda_{j+1} .. lambda_32 s_j [32] (0 behind the piece's end)
+#define LW_TB 32
+#define LW_SCR (LW_TB * LW_TB + 2 * LW_TB)
+#define LW_LDS(DI) (4 * LW_TB * (32 * (DI) + 4) * 4)        /* k_linear_walk: two buffers of queries and of keys */
+// grid (head, piece): queries and keys through LDS (a matrix operand straight from memory is sixteen rows at a time, 59 clocks of the address unit a load), a wave to each of the three tiles
+template <int DI>
+__global__ void __launch_bounds__(256) k_linear_scores(const float * __restrict__ q, const float * __restrict__ k, int64_t stride, int heads, int hpg, const float * __restrict__ decay, const float * __restrict__ tdecay,
+                                                       const float * __restrict__ tscale, int64_t tds, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    constexpr int DIM = 32 * DI, PITCH = DIM + 4;
+    __shared__ __attribute__((aligned(16))) float qs[LW_TB * PITCH], ks[LW_TB * PITCH];
+    __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
+    __shared__ __attribute__((aligned(16))) float lam[64];
+    __shared__ float sc[64], pre[64], suf[64], upto[64], from[64], whole[4];
+    extern __shared__ int lm_recs[];
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
+    if (la_one_run(rec, n_tok)) {
+        if (tid == 0) { seg[0] = (int) blockIdx.y * LW_TB; seg[1] = max(0, min(LW_TB, n_tok - (int) blockIdx.y * LW_TB)); seg[2] = rec[0]; }
+    } else {
+        for (int t = tid; t < n_tok; t += 256) lm_recs[t] = rec[t];
+        __syncthreads();
+        const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
+        if (tid < 64) la_find_piece(lm_recs, n_tok, bnd, n_runs, LW_TB, blockIdx.y, seg);
+    }
+    __syncthreads();
+    const int first = seg[0], len = seg[1], word = seg[2];
+    if (len == 0 || word < 0) return;
+    const float * qp = q + (int64_t) first * stride + (int64_t) (h / hpg) * DIM, * kp = k + (int64_t) first * stride + (int64_t) (h / hpg) * DIM;
+    hy_f32x4 x[2 * DI];
+#pragma unroll
+    for (int i = 0; i < DI; i++) {
+        const int at = tid + 256 * i, t = at / (DIM / 4), d = at % (DIM / 4) * 4;
+        const uint32_t o = (uint32_t) min(t, len - 1) * (uint32_t) stride + d;
+        x[2 * i] = lm_at4(qp, o); x[2 * i + 1] = lm_at4(kp, o);
+    }
+    if (wave == 3) lm_factors(lane, len, (int64_t) (first + min(lane, len - 1)) * tds + h, decay, tdecay, tscale, h, lam, sc, pre, suf, upto, from, whole);
+#pragma unroll
+    for (int i = 0; i < DI; i++) {
+        const int at = tid + 256 * i, t = at / (DIM / 4), d = at % (DIM / 4) * 4;
+        *(hy_f32x4 *) &qs[t * PITCH + d] = x[2 * i]; *(hy_f32x4 *) &ks[t * PITCH + d] = x[2 * i + 1];
+    }
+    __syncthreads();
+    float * own = scratch + ((int64_t) blockIdx.y * heads + h) * LW_SCR;
+    if (wave == 3) { own[LW_TB * LW_TB + lane] = lane < LW_TB ? upto[lane] : from[lane - LW_TB]; return; }
+    const int tt = wave == 0 ? 0 : 1, jt = wave == 2 ? 1 : 0, t = 16 * tt + n;
+    if (16 * tt >= len) return;
+    hy_f32x4 a = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+    for (int s = 0; s < 2 * DI; s++) {
+        const hy_f32x4 kv = *(const hy_f32x4 *) &ks[(16 * jt + n) * PITCH + 16 * s + 4 * g], qv = *(const hy_f32x4 *) &qs[t * PITCH + 16 * s + 4 * g];
+#pragma unroll
+        for (int e = 0; e < 4; e++) a = hy_mfma(kv[e], qv[e], a);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {                                     // transposed: a lane's four rows j are consecutive values of row t
+        const int jr = 16 * jt + 4 * g + r;
+        const float d = jt < tt ? suf[jr] * pre[t] : lm_inside(lam + 16 * tt, 4 * g + r, n);
+        a[r] = jr <= t && jr < len ? a[r] * d * sc[jr] : 0.0f;
+    }
+    *(hy_f32x4 *) (own + t * LW_TB + 16 * jt + 4 * g) = a;
+}
+// grid (head, sixteen columns of values, run): the run's pieces in order.  Wave w keeps 16 MW rows of the state in registers as the matrix cores leave them, which is how they take them for Q S: row 16 MW w + MW (4 g + r) + i in
+// register r of tile i, so that a lane's keys are MW neighbours.  Of a piece it computes Q S over those rows for all tokens, a quarter of P V (value r = w of every four), and its rows' new state; the four waves' shares of an output
+// meet in LDS.  Four more waves bring the pieces' queries, keys, values and scores through LDS in two buffers, two pieces ahead in registers, and add up and write the outputs: one barrier a piece.  Bound by the chain of a piece, whatever the number of heads: 35 products of 32 clocks
+// and two trips through LDS.
+template <int DI>
+__global__ void __launch_bounds__(512, 2) k_linear_walk(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim, int vstored,
+                                                        const float * __restrict__ skip, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, const float * __restrict__ scratch, float * __restrict__ out,
+                                                        int64_t os, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    constexpr int DIM = 32 * DI, MW = (2 * DI + 3) / 4, PITCH = DIM + 4, PP = LW_TB + 4;
+    __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
+    __shared__ __attribute__((aligned(16))) float vs[2][LW_TB * 16], ps[2][LW_TB * PP], fs[2][2 * LW_TB];
+    __shared__ hy_f32x4 part[2][4][2][64];                             // [piece % 2][wave][tile of tokens][lane]
+    extern __shared__ __attribute__((aligned(16))) float lw_lds[];     // queries and keys, two buffers each; ahead of them the slot words of the pass
+    int * const lm_recs = (int *) lw_lds; float * const qs = lw_lds, * const ks = lw_lds + 2 * LW_TB * PITCH;
+    constexpr int BUF = LW_TB * PITCH;
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 15, g = lane >> 4;
+    if (la_one_run(rec, n_tok)) {
+        if (tid == 0) { seg[0] = 0; seg[1] = 0; seg[2] = blockIdx.z == 0 ? n_tok : 0; seg[3] = rec[0]; }
+    } else {
+        for (int t = tid; t < n_tok; t += 512) lm_recs[t] = rec[t];
+        __syncthreads();
+        const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
+        if (tid < 64) {
+            int own[4], ord = la_pieces_before(bnd, n_runs, n_tok, LW_TB, own);
+            if (tid == 0) seg[2] = 0;
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const int r = 4 * tid + x;
+                if (r == (int) blockIdx.z && r < n_runs) { seg[0] = bnd[r]; seg[1] = ord; seg[2] = (r + 1 < n_runs ? bnd[r + 1] : n_tok) - bnd[r]; seg[3] = lm_recs[bnd[r]]; }
+                ord += own[x];
+            }
+        }
+    }
+    __syncthreads();
+    const int run0 = seg[0], run_len = seg[2], word = seg[3], c0 = (int) blockIdx.y * 16, c = c0 + n, cc = min(c, vdim - 1);
+    const int64_t ord0 = seg[1];
+    if (run_len == 0 || word < 0) return;
+    const int pieces = (run_len + LW_TB - 1) / LW_TB;
+    float * S_hbm = state + ((int64_t) (word & ~LA_FRESH) * heads + h) * (int64_t) DIM * vdim;
+    const float skp = skip ? skip[h] : 0.0f;
+    const bool walks = wave < 4;
+    const int st = tid & 255;                                          // of the four waves that bring the pieces
+    auto row_of = [&](int i, int r) { return 16 * MW * wave + MW * (4 * g + r) + i; };
+    hy_f32x4 S[MW];
+    if (walks)
+#pragma unroll
+    for (int i = 0; i < MW; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) { const int row = row_of(i, r); const float x = lm_at(S_hbm, (uint32_t) min(row, DIM - 1) * (uint32_t) vdim + (uint32_t) cc); S[i][r] = (word & LA_FRESH) || row >= DIM ? 0.0f : x; }
+    // what this thread brings of a piece: DI runs of four values of the queries and of the keys, two values, four scores, one factor
+    struct piece_regs { hy_f32x4 q[DI], k[DI], p; float v[2], f; } R[2];
+    const int vt = st >> 4, vc = min(c0 + (st & 15), vstored - 1);
+    auto fetch = [&](piece_regs & F, int p) __attribute__((always_inline)) {
+        const int len = min(LW_TB, run_len - p * LW_TB);
+        const int64_t first = run0 + (int64_t) p * LW_TB;
+        const float * qp = q + first * stride + (int64_t) (h / hpg) * DIM, * kp = k + first * stride + (int64_t) (h / hpg) * DIM, * vp = v + first * stride + (int64_t) h * vstored;
+        const float * own = scratch + ((ord0 + p) * heads + h) * LW_SCR;
+#pragma unroll
+        for (int i = 0; i < DI; i++) {
+            const int at = st + 256 * i, t = at / (DIM / 4), d = at % (DIM / 4) * 4;      // (rows behind the last repeat it)
+            const uint32_t o = (uint32_t) min(t, len - 1) * (uint32_t) stride + d;
+            F.q[i] = lm_at4(qp, o); F.k[i] = lm_at4(kp, o);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) F.v[i] = lm_at(vp, (uint32_t) min(vt + 16 * i, len - 1) * (uint32_t) stride + (uint32_t) vc);
+        F.p = *(const hy_f32x4 *) (own + 4 * st);
+        F.f = own[LW_TB * LW_TB + (st & 63)];
+    };
+    auto stage = [&](piece_regs & F, int p) __attribute__((always_inline)) {
+        const int b = p & 1, len = min(LW_TB, run_len - p * LW_TB);
+#pragma unroll
+        for (int i = 0; i < DI; i++) {
+            const int at = st + 256 * i, t = at / (DIM / 4), d = at % (DIM / 4) * 4;
+            *(hy_f32x4 *) &qs[b * BUF + t * PITCH + d] = F.q[i]; *(hy_f32x4 *) &ks[b * BUF + t * PITCH + d] = F.k[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) vs[b][st + 256 * i] = vt + 16 * i >= len ? 0.0f : c0 + (st & 15) < vstored ? F.v[i] : 1.0f;      // (a column the values do not have: ones)
+        *(hy_f32x4 *) &ps[b][(st >> 3) * PP + (st & 7) * 4] = F.p;
+        if (st < 64) fs[b][st] = F.f;
+    };
+    const int own_rows = 16 * MW * min(wave, 2 * DI / MW - 1);        // (a wave without rows repeats the last ones: its state is zero and stays so)
+    typedef float keys __attribute__((ext_vector_type(MW)));
+    auto compute = [&](int p) __attribute__((always_inline)) {
+        const int b = p & 1, len = min(LW_TB, run_len - p * LW_TB);
+        hy_f32x4 qv[2][MW], o[2], up[2], w[2]; keys kv[8]; float vv[8], pv[2], pw[3];
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+            for (int i = 0; i < MW; i++) qv[tt][i] = *(const hy_f32x4 *) &qs[b * BUF + (16 * tt + n) * PITCH + own_rows + 4 * MW * g + 4 * i];
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) { w[tt] = *(const hy_f32x4 *) &fs[b][LW_TB + 16 * tt + 4 * g]; up[tt] = *(const hy_f32x4 *) &fs[b][16 * tt + 4 * g]; }
+        const float all = fs[b][LW_TB - 1];
+#pragma unroll
+        for (int x = 0; x < 8; x++) { const int t = 16 * (x >> 2) + 4 * g + (x & 3); vv[x] = vs[b][t * 16 + n]; kv[x] = *(const keys *) &ks[b * BUF + t * PITCH + own_rows + MW * n]; }
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++) pv[jt] = vs[b][(16 * jt + 4 * g + wave) * 16 + n];
+        pw[0] = ps[b][n * PP + 4 * g + wave]; pw[1] = ps[b][(16 + n) * PP + 4 * g + wave]; pw[2] = ps[b][(16 + n) * PP + 16 + 4 * g + wave];
+        o[0] = o[1] = hy_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int i = 0; i < MW; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int tt = 0; tt < 2; tt++) o[tt] = hy_mfma(qv[tt][(MW * e + i) >> 2][(MW * e + i) & 3], S[i][e], o[tt]);
+        // the piece's new state: what is left of its keys' products at its end
+#pragma unroll
+        for (int i = 0; i < MW; i++) S[i] *= all;
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+            const float vw = wave * MW < 2 * DI && 16 * (x >> 2) + 4 * g + (x & 3) < len ? vv[x] * w[x >> 2][x & 3] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < MW; i++) S[i] = hy_mfma(kv[x][i], vw, S[i]);
+        }
+        o[0] *= up[0]; o[1] *= up[1];
+        // an infinity or a NaN among the values must not meet the zero weights of the tokens before it: the diagonal's tiles then go value by value, in the first wave
+        const uint32_t big = max(__float_as_uint(pv[0]) & 0x7fffffffu, __float_as_uint(pv[1]) & 0x7fffffffu);
+        const bool odd = __any(big >= 0x7f800000u);
+        hy_f32x4 (* meet)[2][64] = part[b];
+        if (!odd) { o[0] = hy_mfma(pw[0], pv[0], o[0]); o[1] = hy_mfma(pw[2], pv[1], o[1]); }
+        else
+#pragma unroll
+            for (int tt = 0; tt < 2; tt++)
+                for (int gg = 0; gg < 4; gg++) {                       // (the keys 4 gg + w: this wave's share of them)
+                    const int j = 16 * tt + 4 * gg + wave;
+                    const float x = vs[b][j * 16 + n];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) if (j <= 16 * tt + 4 * g + r && j < len) o[tt][r] = fmaf(ps[b][(16 * tt + 4 * g + r) * PP + j], x, o[tt][r]);
+                }
+        o[1] = hy_mfma(pw[1], pv[0], o[1]);
+        meet[wave][0][lane] = o[0]; meet[wave][1][lane] = o[1];
+    };
+    auto finish = [&](int p) __attribute__((always_inline)) {
+        const int b = p & 1, len = min(LW_TB, run_len - p * LW_TB), tt = (wave & 3) >> 1, half = wave & 1;
+        const int64_t first = run0 + (int64_t) p * LW_TB;
+        typedef float two __attribute__((ext_vector_type(2)));
+        two y[4];
+#pragma unroll
+        for (int x = 0; x < 4; x++) y[x] = *(const two *) ((const float *) &part[b][x][tt][lane] + 2 * half);
+        const two sum = (y[0] + y[1]) + (y[2] + y[3]);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int t = 16 * tt + 4 * g + 2 * half + r;
+            if (t >= len || c >= vdim) continue;
+            out[(first + t) * os + (int64_t) h * vdim + c] = skip ? fmaf(skp, lm_value(v + first * stride + (int64_t) h * vstored, t, (uint32_t) stride, c, vstored), sum[r]) : sum[r];
+        }
+    };
+    auto meet_all = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };      // (loads stay on their way)
+    // Between two barriers the walking waves compute piece p while the others sum up piece p - 1, put piece p + 1 into the other buffer and ask for piece p + 3.  (The walkers doing all of it, one thing after another: 120 us, now 87)
+    if (!walks) {
+        // (always two next ones, behind the last piece that again, and no way out between two pieces: where paths with different loads on their way meet, the compiler waits for the younger ones too)
+        fetch(R[0], 0);
+        fetch(R[1], min(1, pieces - 1));
+        stage(R[0], 0);
+        fetch(R[0], min(2, pieces - 1));
+        meet_all();
+        auto step = [&](int p, piece_regs & F) __attribute__((always_inline)) {
+            if (p > 0) finish(p - 1);
+            stage(F, p + 1);                                           // (behind the last piece: of no use)
+            fetch(F, min(p + 3, pieces - 1));
+            meet_all();
+        };
+        int p = 0;
+        for (; p + 2 <= pieces; p += 2) { step(p, R[1]); step(p + 1, R[0]); }
+        if (p < pieces) step(p, R[1]);
+        finish(pieces - 1);
+        return;
+    }
+    meet_all();
+    for (int p = 0; p < pieces; p++) { compute(p); meet_all(); }
+    if (c < vdim)
+#pragma unroll
+        for (int i = 0; i < MW; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) { const int row = row_of(i, r); if (row < DIM) S_hbm[(int64_t) row * vdim + c] = S[i][r]; }
 }
 
 // grid (head, blocks over dim * vdim, run): scratch[piece] holds L_p coming in and S_in(p) going out
@@ -941,18 +1193,17 @@ extern "C" int pi_op_linear_attention_reserve(void) {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<8>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<16>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_attention<32>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
-#define LM_RES(DI) PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_pieces<DI, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS)); \
-                   PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_pieces<DI, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS));
+#define LM_RES(DI) PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_scores<DI>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS)); \
+                   PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_walk<DI>, hipFuncAttributeMaxDynamicSharedMemorySize, std::max(4 * LM_MAX_TOKENS, LW_LDS(DI))));
     LM_RES(1) LM_RES(2) LM_RES(3) LM_RES(4)
 #undef LM_RES
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_state_scan<LA_TB>, hipFuncAttributeMaxDynamicSharedMemorySize, LA_LDS_MAX));
-    PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_linear_state_scan<LM_TB>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * LM_MAX_TOKENS));
     done = true;
     return 0;
 }
 static int la_max_pieces(int n_tok, int max_segments) { return n_tok / LA_TB + std::min(n_tok, std::max(1, max_segments)) + 1; }
 extern "C" size_t pi_op_linear_attention_scratch_floats(int heads, int dim, int vdim, int n_tok, int max_segments) {
-    return n_tok <= LA_TB ? 0 : (size_t) la_max_pieces(n_tok, max_segments) * heads * dim * vdim;
+    return n_tok <= LA_TB ? 0 : (size_t) heads * std::max((size_t) la_max_pieces(n_tok, max_segments) * dim * vdim, dim % 32 == 0 && dim <= 128 ? (size_t) la_max_pieces(n_tok, max_segments) * LW_SCR : (size_t) 0);
 }
 extern "C" int pi_op_linear_attention(const float * q, const float * k, const float * v, int64_t stride, int heads, int dim, int vdim, const float * decay_dev, float * state_dev,
                                       const int32_t * rec_dev, int n_tok, int max_segments, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride, void * stream) {
@@ -999,31 +1250,32 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
 #define LA_ANY(MODE) do { if (dpt == 8) LA_GO(8, MODE); else if (dpt == 16) LA_GO(16, MODE); else LA_GO(32, MODE); } while (0)
     const bool matrix = dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22);       // (32-bit offsets within a piece; pieces twice as long take half of the scratch that was asked for)
     const unsigned gr = (unsigned) std::max(1, std::min(n_tok, max_segments)), gb = (unsigned) (((int64_t) dim * vdim + 255) / 256);
-#define LM_GO(DI, OUT, SCR) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_linear_pieces<DI, OUT>), pg, dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, \
-                                    state_dev, rec_dev, n_tok, SCR, out, out_stride, pi_abort_word())
-#define LM_ANY(OUT, SCR) do { if (dim == 32) LM_GO(1, OUT, SCR); else if (dim == 64) LM_GO(2, OUT, SCR); else if (dim == 96) LM_GO(3, OUT, SCR); else LM_GO(4, OUT, SCR); } while (0)
+#define LM_ANY(GO) do { if (dim == 32) GO(1); else if (dim == 64) GO(2); else if (dim == 96) GO(3); else GO(4); } while (0)
+#define LM_PIECES(DI) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_pieces<DI>, dim3((unsigned) heads, gr), dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, \
+                                   skip_dev, state_dev, rec_dev, n_tok, out, out_stride, pi_abort_word())
+#define LM_SCORES(DI) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 4.0 * n_tok * heads * (2 * dim + LW_TB), k_linear_scores<DI>, dim3((unsigned) heads, (unsigned) la_max_pieces(n_tok, max_segments)), dim3(256), (size_t) 4 * n_tok, s, q, k, stride, heads, hpg, \
+                                   decay_dev, tdecay_dev, tscale_dev, t_stride, rec_dev, n_tok, scratch_dev, pi_abort_word())
+#define LM_WALK(DI) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_walk<DI>, dim3((unsigned) heads, (unsigned) ((vdim + 15) / 16), gr), dim3(512), std::max((size_t) 4 * n_tok, (size_t) LW_LDS(DI)), s, q, k, v, stride, heads, hpg, vdim, value_cols, skip_dev, state_dev, \
+                                 rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word())
     // Up to 64 tokens every run is one piece: one launch from the slots' states to the slots' states.  Beyond LA_TB always (32 heads of 128 x 128, three launches against it: a run of 64 tokens 55 -> 48 us, 64 runs of a
     // token 450 -> 123, for the pieces are walked twice and the scan starts for every run); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
     // (24 tokens 53 -> 29, 9 about even; eight runs of a token or two 14 .. 18, here 25 .. 29)
     if (matrix && n_tok <= LM_TB && (pieces || n_tok > 8 * gr)) {
-        const dim3 pg((unsigned) heads, gr);
-        LM_ANY(true, nullptr);
+        LM_ANY(LM_PIECES);
         PI_CHECK_LAUNCH(); return 0;
     }
     if (!pieces) { LA_ANY(0); PI_CHECK_LAUNCH(); return 0; }
     if (matrix) {
-        if (n_tok > 2048 && pi_op_linear_attention_reserve() != 0) return -1;
-        const dim3 pg((unsigned) heads, (unsigned) (n_tok / LM_TB + std::min(n_tok, std::max(1, max_segments)) + 1));
-        LM_ANY(false, scratch_dev);
+        if (pi_op_linear_attention_reserve() != 0) return -1;
+        LM_ANY(LM_SCORES);
         PI_CHECK_LAUNCH();
-        PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * pg.y * heads * dim * vdim, k_linear_state_scan<LM_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,
-                     heads, dim, vdim, decay_dev, tdecay_dev, t_stride, state_dev, rec_dev, n_tok, scratch_dev, pi_abort_word());
-        PI_CHECK_LAUNCH();
-        LM_ANY(true, scratch_dev);
+        LM_ANY(LM_WALK);
         PI_CHECK_LAUNCH(); return 0;
     }
 #undef LM_ANY
-#undef LM_GO
+#undef LM_PIECES
+#undef LM_SCORES
+#undef LM_WALK
     LA_ANY(1);
     PI_CHECK_LAUNCH();
     PI_KT_LAUNCH(PI_KT_ATT, 0, nta, 12.0 * gz * heads * dim * vdim, k_linear_state_scan<LA_TB>, dim3((unsigned) heads, gb, gr), dim3(256), (size_t) 4 * n_tok, s,
