@@ -34,12 +34,12 @@ class Served:
         return 1
 
 
-@pytest.mark.parametrize("rows", ["many", "few"])
+@pytest.mark.parametrize("rows", ["many", "some", "few"])
 def test_rows_stay_where_a_run_brings_none(rows):
     """rows that are many change hands with the run's buffer, few are copied: either way the rows of the last run that brought some are read until the next one brings its own — past a run that could not be
     started, through the next run's time in flight, and past a cancelled run, shorter or longer"""
     model = LL.Model(MODEL)
-    n = (4 << 20) // (4 * model.n_vocab) + 1 if rows == "many" else 3
+    n = {"many": (4 << 20) // (4 * model.n_vocab) + 1, "some": (3 << 16) // (4 * model.n_vocab) + 1, "few": 3}[rows]
     ctx = LL.Context(model, n_ctx=2 * n + 64, n_batch=2 * n, logits_all=True)
     s = Served(ctx)
 
