@@ -220,11 +220,13 @@ extern "C" int pi_op_token_shift(const float * h, int64_t h_stride, int n, const
 #define CR_MAXRUNS 256
 #define CR_SCAN_MAXDIM 128                        // widest key whose transition matrix the scan keeps in LDS
 // the pass's runs in order (a run: the consecutive tokens of one slot): every thread looks at its own tokens for a run's first one, the few found are ranked by position.  first[r] in `sorted`
-static __device__ __forceinline__ int cr_runs(const int32_t * __restrict__ rec, int n_tok, int * bnd, int * sorted, int * nb) {
+static __device__ __forceinline__ int cr_mark(const int32_t * __restrict__ rec, int t) { return t == 0 || (rec[t] & ~CM_FRESH) != (rec[t - 1] & ~CM_FRESH); }
+// (mark: a caller's own for token threadIdx.x, asked for ahead of loads of its own, which would be waited for with it)
+static __device__ __forceinline__ int cr_runs(const int32_t * __restrict__ rec, int n_tok, int * bnd, int * sorted, int * nb, int mark = -1) {
     if (threadIdx.x == 0) *nb = 0;
     __syncthreads();
     for (int t = threadIdx.x; t < n_tok; t += blockDim.x)
-        if (t == 0 || (rec[t] & ~CM_FRESH) != (rec[t - 1] & ~CM_FRESH)) { const int at = atomicAdd(nb, 1); if (at < CR_MAXRUNS) bnd[at] = t; }
+        if (mark >= 0 && t == (int) threadIdx.x ? mark : cr_mark(rec, t)) { const int at = atomicAdd(nb, 1); if (at < CR_MAXRUNS) bnd[at] = t; }
     __syncthreads();
     const int n = min(*nb, CR_MAXRUNS);
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
@@ -484,13 +486,18 @@ __global__ void __launch_bounds__(256) k_channel_state_scan_diag(int heads, int 
 //   (I + A) U = beta (V - W S_in),  W_t = G_t k_t,  A[t][j] = beta_t sum_i k_t k_j (g_{j+1} .. g_t)_i for j < t      (bonus rule: U = V)
 //   O = Q' S_in + P U,  Q'_t = G_t q_t,  P[t][j] = sum_i q_t k_j (g_{j+1} .. g_t)_i for j <= t                     (bonus rule: products up to t - 1, the bonus on the diagonal)
 //   S_out = G_32 S_in + K' U,  K'_j = k_j (g_{j+1} .. g_32)
-//   k_channel_pieces  per (head, piece), side by side: everything that does not know S_in, T = (I + A)^-1 applied to beta V and beta W.  Decays are products of factors only, never quotients: inside a tile of 16
-//                     tokens they are multiplied up pair by pair, across the two tiles they meet at the border between them (a decay of 1e-30 per token is as good as any other).  Unit keys and beta <= 1
-//                     bound T's entries by 1; keys as they come (qk_unit = 0) of the delta rule stay with the walks
-//   k_channel_walk    per (head, 16 value columns, run): one wave takes the run's pieces in order, the state in registers all the way - a product's result is laid out as the next one's operand.
-//                     An infinity or a NaN in a piece would meet zeros of tokens before it: such a piece is walked token by token
-// 333 tokens of one sequence, delta rule, 16 heads of 128 x 128: 2 x 271 us + scan 331 -> 42 + 48; bonus rule, 32 heads of 64 x 64: 2 x 129 + scan 22 -> 21 + 27.
+//   k_channel_pieces  per (head, piece), side by side: everything that does not know S_in, T = (I + A)^-1 applied to beta V and beta W.  Decays are products of factors only, never quotients: two tokens' decays meet at
+//                     the border between them - of the piece's two tiles of 16, or of two halves of a square inside one, down to single tokens (a decay of 1e-30 per token is as good as any other).  Unit keys and
+//                     beta <= 1 bound T's entries by 1; keys as they come (qk_unit = 0) of the delta rule stay with the walks.  Bound by a workgroup's run through its phases: of 18 us (delta rule, 128 x 128) loads and
+//                     the search for its run take 4, the decays' logarithms 4, the squares 3.5.  A column's walk down the tile with eight threads took 8, the loads one after the other 7: 25 us with both
+//   k_channel_walk    per (head, 16 value columns, run): takes the run's pieces in order, the state in the registers of four waves (a quarter of the rows each) - a product's result is laid out as the next one's
+//                     operand; the waves' parts of T beta (V - W S_in) meet in LDS.  Helping waves bring the pieces through LDS, two ahead in registers, add up and write the outputs: one barrier a piece.  Of a
+//                     piece's 3100 clocks (delta rule, 128 x 128) 1630 are products, the rest the exchange and waits for LDS, and the 54 KB that a workgroup loads per piece take nearly as long.  One wave with the
+//                     whole state, loads and all: 10000.  An infinity or a NaN in a piece would meet zeros of tokens before it: such a piece is walked token by token
+// 333 tokens of one sequence, pieces + walk, us: delta rule, 16 heads of 128 x 128: 82 with those, 39 now (walked token by token: 2 x 271 + scan 331); bonus rule, 32 heads of 64 x 64: 42, 24 (2 x 129 + scan 22).
+// 2048 tokens, delta rule, 32 heads: 466, 200
 #define CP_TB 32
+#define CP_PIECE_THREADS 512
 typedef float cm_f32x4 __attribute__((ext_vector_type(4)));
 static __device__ __forceinline__ cm_f32x4 cm_mfma(float a, float b, cm_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 static __device__ __forceinline__ cm_f32x4 cm_mfma4(cm_f32x4 a, cm_f32x4 b, cm_f32x4 c) {
@@ -498,7 +505,7 @@ static __device__ __forceinline__ cm_f32x4 cm_mfma4(cm_f32x4 a, cm_f32x4 b, cm_f
     for (int i = 0; i < 4; i++) c = cm_mfma(a[i], b[i], c);
     return c;
 }
-// a piece's block in scratch, in floats: operands as the lanes hold them, [tile][lane][4]:  Q' [2][dim / 16], K' [dim / 16][2], -T beta W [2][dim / 16], P [3], G_32 [dim], a flag, T beta V [2][vdim / 16]
+// a piece's block in scratch, in floats: operands as the lanes hold them, [tile][lane][4]:  Q' [2][dim / 16], K' [dim / 16][2], -T beta W [2][dim / 16], P [3], G_32 [dim], a flag, U: T beta V (bonus rule: V) [2][vdim / 16]
 // (flagged: q, k, g as rows [32][dim] in the first three places, beta [32] and the scalar of the token's own write [32] in P's)
 struct cp_layout { int q, k, w, p, g, flag, u, total; };
 static __host__ __device__ __forceinline__ cp_layout cp_of(int dim, int vdim) {
@@ -507,16 +514,39 @@ static __host__ __device__ __forceinline__ cp_layout cp_of(int dim, int vdim) {
     return l;
 }
 template <int DI, int RULE>
-__global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs, const float * __restrict__ draw, int64_t ds,
+__global__ void __launch_bounds__(CP_PIECE_THREADS) k_channel_pieces(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs, const float * __restrict__ draw, int64_t ds,
                                                         int decay_mode, const float * __restrict__ dbias, const float * __restrict__ a_log, const float * __restrict__ braw, int64_t bs, const float * __restrict__ bonus,
                                                         int qk_unit, float q_mult, int heads, int hpg, int vdim, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
-    constexpr int DIM = 16 * DI, PITCH = DIM + 4, SL = 2 * DI;        // SL: the eighth of the channels that a thread of the diagonal tiles takes
-    __shared__ __attribute__((aligned(16))) float qt[CP_TB * PITCH], kt[CP_TB * PITCH], gt[CP_TB * PITCH], Am[CP_TB][36], Pm[CP_TB][36], Tm[CP_TB][36], whole[2][DIM];
+    const int gone = pi_abort_peek(abort_w);
+    constexpr int DIM = 16 * DI, PITCH = DIM + 4, TH = CP_PIECE_THREADS, NW = TH / 64, PER = CP_TB * DIM / TH;
+    __shared__ __attribute__((aligned(16))) float qt[CP_TB * PITCH], kt[CP_TB * PITCH], gt[CP_TB * PITCH], Am[CP_TB][36], Pm[CP_TB][36], Tm[CP_TB][36], whole[2][DIM], ones[DIM];
     __shared__ float beta[CP_TB], dot[CP_TB];
     __shared__ int seg[3], bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;
-    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
-    const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd);
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, nvt = vdim / 16;
+    // every load of the piece on its way before the first is waited for, and ahead of the search for the runs: for the piece that a pass of one run has here (another one's are loaded behind the search)
+    float qv[PER], kv[PER], dv[PER], bv = 0.0f;
+    cm_f32x4 x0[2];                                                   // the values of the wave's first tile, as the product over them takes them
+    auto values = [&](cm_f32x4 * x, int vt, int first, int last) {
+#pragma unroll
+        for (int jt = 0; jt < 2; jt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[jt][r] = v[(int64_t) min(first + 16 * jt + 4 * g + r, last) * vs + (int64_t) h * vdim + 16 * vt + n];
+    };
+    auto fetch = [&](int first, int last) {
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int idx = tid + u * TH, i = idx % DIM;
+            const int64_t tok = min(first + idx / DIM, last);
+            qv[u] = q[tok * qs + (int64_t) (h / hpg) * DIM + i]; kv[u] = k[tok * ks + (int64_t) (h / hpg) * DIM + i]; dv[u] = draw[tok * ds + (int64_t) h * DIM + i];
+        }
+        values(x0, min(wave, nvt - 1), first, last);
+        if (tid < CP_TB && braw) bv = braw[(int64_t) min(first + tid, last) * bs + h];
+    };
+    const int mark = tid < n_tok ? cr_mark(rec, tid) : 0;
+    const int guess = min((int) blockIdx.y * CP_TB, n_tok - 1);
+    fetch(guess, n_tok - 1);
+    const float ah = decay_mode == 2 ? expf(a_log[h]) : 0.0f, db = decay_mode != 0 && dbias ? dbias[h * DIM + tid % DIM] : 0.0f;      // (TH is a multiple of DIM: one channel per thread)
+    const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd, mark);
     if (tid == 0) {
         int ord = 0;
         seg[1] = 0;
@@ -526,70 +556,106 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
             ord += nsub;
         }
     }
+    for (int idx = tid; idx < CP_TB * 36; idx += TH) { (&Am[0][0])[idx] = 0.0f; (&Pm[0][0])[idx] = 0.0f; (&Tm[0][0])[idx] = 0.0f; }
+    if (tid < DIM) ones[tid] = 1.0f;
     __syncthreads();
     const int first = seg[0], len = seg[1];
     if (len == 0 || seg[2] < 0) return;
+    if (pi_abort_late(gone, abort_w)) return;
+    const int last = first + len - 1;
+    if (first != guess) fetch(first, last);
     const cp_layout L = cp_of(DIM, vdim);
     float * blk = scratch + ((int64_t) blockIdx.y * heads + h) * L.total;
-    const float ah = decay_mode == 2 ? expf(a_log[h]) : 0.0f;
     uint32_t big = 0;
-    for (int idx = tid; idx < CP_TB * DIM; idx += 256) {
-        const int t = idx / DIM, i = idx % DIM;
-        const int64_t tok = first + min(t, len - 1);
-        float qv = q[tok * qs + (int64_t) (h / hpg) * DIM + i], kv = k[tok * ks + (int64_t) (h / hpg) * DIM + i], d = draw[tok * ds + (int64_t) h * DIM + i];
-        if (decay_mode == 1) d = expf(-expf(d + (dbias ? dbias[h * DIM + i] : 0.0f)));
-        else if (decay_mode == 2) d = expf(-ah * cm_softplus(d + (dbias ? dbias[h * DIM + i] : 0.0f)));
-        if (t >= len) { qv = 0.0f; kv = 0.0f; d = 1.0f; }
-        qt[t * PITCH + i] = qv; kt[t * PITCH + i] = kv; gt[t * PITCH + i] = d;
-        big = max(big, max(__float_as_uint(d) & 0x7fffffffu, max(__float_as_uint(qv) & 0x7fffffffu, __float_as_uint(kv) & 0x7fffffffu)));
+    auto seen = [&](float x) { big = max(big, __float_as_uint(x) & 0x7fffffffu); };
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const int idx = tid + u * TH, t = idx / DIM, i = idx % DIM;
+        if (t >= len) { qv[u] = 0.0f; kv[u] = 0.0f; }
+        qt[t * PITCH + i] = qv[u]; kt[t * PITCH + i] = kv[u]; gt[t * PITCH + i] = dv[u];
+        seen(qv[u]); seen(kv[u]);
     }
-    if (tid < CP_TB) {
-        const float b = tid >= len ? 0.0f : braw ? cm_sigmoid(braw[(int64_t) (first + tid) * bs + h]) : 1.0f;
-        beta[tid] = b; big = max(big, __float_as_uint(b) & 0x7fffffffu);
+#pragma unroll 1
+    for (int u = 0; u < PER; u++) {                                    // (not unrolled, like the squares below: a workgroup runs through the code once, and what it runs through has to be fetched)
+        const int t = (tid + u * TH) / DIM;
+        float * at = gt + t * PITCH + tid % DIM, d = *at;
+        if (decay_mode == 1) d = expf(-expf(d + db));
+        else if (decay_mode == 2) d = expf(-ah * cm_softplus(d + db));
+        if (t >= len) d = 1.0f;
+        *at = d;
+        seen(d);
     }
-    for (int idx = tid; idx < len * vdim; idx += 256) big = max(big, __float_as_uint(v[(int64_t) (first + idx / vdim) * vs + (int64_t) h * vdim + idx % vdim]) & 0x7fffffffu);
-    for (int idx = tid; idx < CP_TB * 36; idx += 256) { (&Am[0][0])[idx] = 0.0f; (&Pm[0][0])[idx] = 0.0f; (&Tm[0][0])[idx] = 0.0f; }
+    if (tid < CP_TB) { bv = tid >= len ? 0.0f : braw ? cm_sigmoid(bv) : 1.0f; beta[tid] = bv; seen(bv); }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {                                      // (behind the piece's end there may be another run's values: the products take the last one of this)
+        if (first + 16 * (i >> 2) + 4 * g + (i & 3) > last) x0[i >> 2][i & 3] = 0.0f;
+        seen(x0[i >> 2][i & 3]);
+    }
+    for (int vt = wave + NW; vt < nvt; vt += NW) {
+        cm_f32x4 x[2];
+        values(x, vt, first, last);
+#pragma unroll
+        for (int i = 0; i < 8; i++) seen(x[i >> 2][i & 3]);
+    }
     const bool odd = __syncthreads_or(big >= 0x7f800000u);
-    for (int t = wave; t < CP_TB; t += 4) {                           // unit vectors, and the scalar of the token's own write
-        float * qr = qt + t * PITCH, * kr = kt + t * PITCH;
+    {   // unit vectors, and the scalar of the token's own write: sixteen lanes per token
+        const int t = tid >> 4;
+        float * qr = qt + t * PITCH + n, * kr = kt + t * PITCH + n, y[DI], z[DI], iq = q_mult, ik = 1.0f, d = 0.0f;
+#pragma unroll
+        for (int i = 0; i < DI; i++) { y[i] = qr[16 * i]; z[i] = kr[16 * i]; }
         if (qk_unit) {
             float sq = 0.0f, sk = 0.0f;
-            for (int i = lane; i < DIM; i += 64) { sq = fmaf(qr[i], qr[i], sq); sk = fmaf(kr[i], kr[i], sk); }
-            const float iq = q_mult / sqrtf(pi_lanes_sum<64>(sq) + 1e-6f), ik = 1.0f / sqrtf(pi_lanes_sum<64>(sk) + 1e-6f);
-            for (int i = lane; i < DIM; i += 64) { qr[i] *= iq; kr[i] *= ik; }
-        } else if (q_mult != 1.0f) for (int i = lane; i < DIM; i += 64) qr[i] *= q_mult;
-        float d = 0.0f;
-        for (int i = lane; i < DIM; i += 64) d = fmaf(RULE == 1 && bonus ? qr[i] * bonus[h * DIM + i] : qr[i], kr[i], d);
-        d = pi_lanes_sum<64>(d);
-        if (lane == 0) dot[t] = d;
+#pragma unroll
+            for (int i = 0; i < DI; i++) { sq = fmaf(y[i], y[i], sq); sk = fmaf(z[i], z[i], sk); }
+            iq = q_mult / sqrtf(pi_lanes_sum<16>(sq) + 1e-6f); ik = 1.0f / sqrtf(pi_lanes_sum<16>(sk) + 1e-6f);
+        }
+#pragma unroll
+        for (int i = 0; i < DI; i++) {
+            y[i] *= iq; z[i] *= ik;
+            if (qk_unit || q_mult != 1.0f) { qr[16 * i] = y[i]; kr[16 * i] = z[i]; }
+            d = fmaf(RULE == 1 && bonus ? y[i] * bonus[h * DIM + n + 16 * i] : y[i], z[i], d);
+        }
+        d = pi_lanes_sum<16>(d);
+        if (n == 0) dot[t] = d;
     }
     __syncthreads();
     if (tid == 0) *(int *) (blk + L.flag) = odd ? 1 : 0;
     if (odd) {
-        for (int idx = tid; idx < CP_TB * DIM; idx += 256) { const int at = idx / DIM * PITCH + idx % DIM; blk[L.q + idx] = qt[at]; blk[L.k + idx] = kt[at]; blk[L.w + idx] = gt[at]; }
+        for (int idx = tid; idx < CP_TB * DIM; idx += TH) { const int at = idx / DIM * PITCH + idx % DIM; blk[L.q + idx] = qt[at]; blk[L.k + idx] = kt[at]; blk[L.w + idx] = gt[at]; }
         if (tid < CP_TB) { blk[L.p + tid] = beta[tid]; blk[L.p + CP_TB + tid] = dot[tid]; }
         return;
     }
-    {   // the tiles on the diagonal: eight threads share a column j, walk down from it and keep k_j decayed to where they are
-        const int sl = tid & 7, j = tid >> 3 & 15, t0 = tid >> 7 << 4;
-        cm_f32x4 r[SL / 4];
+    {   // the tiles on the diagonal, cut into squares below it whose sides are 8, 4, 2 and 1 (a wave for each size and tile): a square's rows and columns are decayed to the border between them, its rows from there,
+        // its columns up to there - a token is one or the other, so one product of its decays serves both.  Of a 16 x 16 product the squares of its size are kept
+        const int t0 = wave >> 2 << 4, hs = 8 >> (wave & 3), top = (n & -2 * hs) + hs;
+        const bool row = (n & hs) != 0;
+        const int from = row ? top : n + 1, to = row ? (RULE == 1 ? n : n + 1) : top;       // the decays [from, to) of the tile (bonus rule: a row takes the state ahead of its own decay)
+        const float * qr = qt + (t0 + n) * PITCH + 4 * g, * kr = kt + (t0 + n) * PITCH + 4 * g;
+        cm_f32x4 a = { 0.0f, 0.0f, 0.0f, 0.0f }, p = { 0.0f, 0.0f, 0.0f, 0.0f };
+        auto square = [&](auto most) {
+            const float * gr[decltype(most)::value];
 #pragma unroll
-        for (int i = 0; i < SL / 4; i++) r[i] = *(const cm_f32x4 *) &kt[(t0 + j) * PITCH + SL * sl + 4 * i];
-        for (int t = j; t < 16; t++) {
-            const int at = (t0 + t) * PITCH + SL * sl;
-            float a = 0.0f, p = 0.0f;
+            for (int u = 0; u < decltype(most)::value; u++) gr[u] = (from + u < to ? gt + (t0 + from + u) * PITCH : ones) + 4 * g;
+#pragma unroll 1
+            for (int s = 0; s < DI; s++) {
+                cm_f32x4 f = *(const cm_f32x4 *) (gr[0] + 16 * s);
 #pragma unroll
-            for (int i = 0; i < SL / 4; i++) {
-                const cm_f32x4 qv = *(const cm_f32x4 *) &qt[at + 4 * i], kv = *(const cm_f32x4 *) &kt[at + 4 * i], gv = *(const cm_f32x4 *) &gt[at + 4 * i];
-                if (RULE == 0 && t > j) r[i] *= gv;
-#pragma unroll
-                for (int e = 0; e < 4; e++) { if (RULE == 0) a = fmaf(r[i][e], kv[e], a); p = fmaf(r[i][e], qv[e], p); }
-                if (RULE == 1 && t > j) r[i] *= gv;
+                for (int u = 1; u < decltype(most)::value; u++) f *= *(const cm_f32x4 *) (gr[u] + 16 * s);
+                const cm_f32x4 kf = *(const cm_f32x4 *) (kr + 16 * s) * f, qf = *(const cm_f32x4 *) (qr + 16 * s) * f;
+                if (RULE == 0) a = cm_mfma4(kf, kf, a);
+                p = cm_mfma4(qf, kf, p);
             }
+        };
+        if (hs == 8) square(std::integral_constant<int, 8>{});
+        else if (hs == 4) square(std::integral_constant<int, 4>{});
+        else if (hs == 2) square(std::integral_constant<int, 2>{});
+        else square(std::integral_constant<int, 1>{});
 #pragma unroll
-            for (int o = 1; o < 8; o <<= 1) { if (RULE == 0) a += __shfl_xor(a, o, 64); p += __shfl_xor(p, o, 64); }
-            if (sl == 0) { if (t > j) Am[t0 + t][t0 + j] = a; Pm[t0 + t][t0 + j] = t > j ? p : dot[t0 + j]; }
+        for (int r = 0; r < 4; r++) {                                  // (row 4 g + r, column n)
+            const int t = 4 * g + r;
+            if ((t & hs) && !row && (t & -2 * hs) == (n & -2 * hs)) { if (RULE == 0) Am[t0 + t][t0 + n] = a[r]; Pm[t0 + t][t0 + n] = p[r]; }
         }
+        if (hs == 1 && g == 0) Pm[t0 + n][t0 + n] = dot[t0 + n];
     }
     __syncthreads();
     if (tid < 2 * DIM) {                                               // a thread per channel and tile: gt <- k to the tile's start, qt <- q to it (both decayed), kt <- k to the tile's end
@@ -619,8 +685,15 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
         for (int r = 0; r < 4; r++) (wave == 0 ? Am : Pm)[16 + 4 * g + r][n] = a[r];
     }
     __syncthreads();
+    if constexpr (RULE == 1) {
+        for (int vt = wave; vt < nvt; vt += NW) {
+            if (vt != wave) values(x0, vt, first, last);
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++) *(cm_f32x4 *) (blk + L.u + ((mt * nvt + vt) * 64 + lane) * 4) = x0[mt];      // (behind the end: met by keys of zero)
+        }
+    }
     if constexpr (RULE == 0) {
-        for (int idx = tid; idx < CP_TB * CP_TB; idx += 256) Am[idx >> 5][idx & 31] *= beta[idx >> 5];
+        for (int idx = tid; idx < CP_TB * CP_TB; idx += TH) Am[idx >> 5][idx & 31] *= beta[idx >> 5];
         __syncthreads();
         if (tid < 32) {                                                // T on the diagonal: a thread per column, forward substitution
             const int t0 = tid & 16, c = tid & 15;
@@ -635,18 +708,18 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
             }
         }
         __syncthreads();
-        const int t = tid >> 4, c = tid & 15;                          // below it: -T_11 (A_10 T_00)
+        const int t = tid >> 4 & 15, c = tid & 15;                     // below it: -T_11 (A_10 T_00)
         float m = 0.0f;
 #pragma unroll
         for (int j = 0; j < 16; j++) m = fmaf(Am[16 + t][j], Tm[j][c], m);
-        Am[t][16 + c] = m;
+        if (tid < 256) Am[t][16 + c] = m;
         __syncthreads();
         m = 0.0f;
 #pragma unroll
         for (int j = 0; j < 16; j++) m = fmaf(Tm[16 + t][16 + j], Am[j][16 + c], m);
-        Tm[16 + t][c] = -m;
+        if (tid < 256) Tm[16 + t][c] = -m;
         __syncthreads();
-        for (int s = wave; s < DI; s += 4) {                           // -(T beta W), transposed: a lane's four rows are four channels of one token
+        for (int s = wave; s < DI; s += NW) {                           // -(T beta W), transposed: a lane's four rows are four channels of one token
             const int i = 16 * s + n;
             const float w0 = whole[0][i];
             cm_f32x4 a[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
@@ -661,14 +734,14 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
 #pragma unroll
             for (int mt = 0; mt < 2; mt++) *(cm_f32x4 *) (blk + L.w + ((mt * DI + s) * 64 + lane) * 4) = a[mt];
         }
-        const int nvt = vdim / 16;
-        for (int vt = wave; vt < nvt; vt += 4) {
+        for (int vt = wave; vt < nvt; vt += NW) {
+            if (vt != wave) values(x0, vt, first, last);
             cm_f32x4 a[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
 #pragma unroll
             for (int jt = 0; jt < 2; jt++) {
                 cm_f32x4 x;
 #pragma unroll
-                for (int r = 0; r < 4; r++) { const int j = 16 * jt + 4 * g + r; x[r] = beta[j] * v[(int64_t) (first + min(j, len - 1)) * vs + (int64_t) h * vdim + 16 * vt + n]; }       // (beta = 0 behind the end)
+                for (int r = 0; r < 4; r++) { const int j = 16 * jt + 4 * g + r; x[r] = beta[j] * x0[jt][r]; }       // (beta = 0 behind the end)
 #pragma unroll
                 for (int mt = jt; mt < 2; mt++) a[mt] = cm_mfma4(*(const cm_f32x4 *) &Tm[16 * mt + n][16 * jt + 4 * g], x, a[mt]);
             }
@@ -676,7 +749,7 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
             for (int mt = 0; mt < 2; mt++) *(cm_f32x4 *) (blk + L.u + ((mt * nvt + vt) * 64 + lane) * 4) = a[mt];
         }
     }
-    for (int idx = tid; idx < 2 * DI * 64; idx += 256) {
+    for (int idx = tid; idx < 2 * DI * 64; idx += TH) {
         const int tile = idx >> 6, ln = idx & 15, lg = idx >> 4 & 3;
         const int t = 16 * (tile / DI) + ln, i = 16 * (tile % DI) + 4 * lg;
         cm_f32x4 x = *(const cm_f32x4 *) &qt[t * PITCH + i];
@@ -689,128 +762,247 @@ __global__ void __launch_bounds__(256) k_channel_pieces(const float * __restrict
         *(cm_f32x4 *) (blk + L.k + idx * 4) = y;
     }
     if (wave < 3) *(cm_f32x4 *) (blk + L.p + tid * 4) = *(const cm_f32x4 *) &Pm[(wave ? 16 : 0) + n][(wave == 2 ? 16 : 0) + 4 * g];
-    for (int i = tid; i < DIM; i += 256) blk[L.g + i] = whole[0][i] * whole[1][i];
+    for (int i = tid; i < DIM; i += TH) blk[L.g + i] = whole[0][i] * whole[1][i];
 }
 
+// the walk's waves: CP_WAVES walk, each with DI / CP_WAVES sixteens of the state's rows, and CP_HELP help.  Helpers of the delta rule: 8 (its pieces are half as large again; 4: 40.1 us for pieces and walk of 16 heads of
+// 128 x 128, 333 tokens; 8: 39.3); of the bonus rule 4 (one sequence of 333 tokens, 32 heads of 64 x 64: 24.1, with 8 22.4; eight of 42: 27.4, with 8 32.9, where workgroups come and go)
+#define CP_WAVES(DI) ((DI) < 4 ? (DI) : 4)
+#define CP_HELP(RULE) ((RULE) == 0 ? 8 : 4)
+// memory accesses stay on their side (loads of two pieces mixed would have the wait for the first wait for both)
+static __device__ __forceinline__ void cp_keep_order() { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+template <int DI, int RULE> struct cp_stage {                          // a piece in LDS, tiles of 256 floats: Q', K', -T beta W (delta rule), P and what follows it, U of the value columns
+    static constexpr int NT = (RULE == 0 ? 6 : 4) * DI, P = NT * 256, G = P + 768, FLAG = G + 16 * DI, U = P + 1024, TILES = NT + 6, FLOATS = TILES * 256;
+    static constexpr int NW = CP_WAVES(DI), PARTS = NW * 512, OUT = NW * 512, LDS = 4 * (2 * FLOATS + (RULE == 0 ? 2 * PARTS : 0) + 2 * OUT);
+};
 template <int DI, int RULE>
-__global__ void __launch_bounds__(64, 1) k_channel_walk(const float * __restrict__ v, int64_t vs, int heads, int vdim, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, const float * __restrict__ scratch,
-                                                        float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
-    constexpr int DIM = 16 * DI;
+__global__ void __launch_bounds__(64 * (CP_WAVES(DI) + CP_HELP(RULE)), 1) k_channel_walk(const float * __restrict__ v, int64_t vs, int heads, int vdim, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok,
+                                                                                   const float * __restrict__ scratch, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    typedef cp_stage<DI, RULE> ST;
+    constexpr int DIM = 16 * DI, NW = ST::NW, MT = DI / NW, HELP = CP_HELP(RULE);
+    extern __shared__ __attribute__((aligned(16))) float walk_lds[];
     __shared__ int bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;
-    const int h = blockIdx.x, vt = blockIdx.y, lane = threadIdx.x, n = lane & 15, g = lane >> 4, c = 16 * vt + n;
+    __shared__ float one[2][NW][2][16];
+    float * const stage = walk_lds, * const op = stage + 2 * ST::FLOATS, * const us = op + 2 * ST::OUT;      // two buffers of each
+    const int h = blockIdx.x, vt = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4, c = 16 * vt + n, m0 = wave * MT;
     const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd);
     if ((int) blockIdx.z >= n_runs) return;
     int ord = 0;
     for (int r = 0; r < (int) blockIdx.z; r++) ord += ((r + 1 < n_runs ? sorted[r + 1] : n_tok) - sorted[r] + CP_TB - 1) / CP_TB;
     const int start = sorted[blockIdx.z], end = (int) blockIdx.z + 1 < n_runs ? sorted[blockIdx.z + 1] : n_tok, word = rec[start], np = (end - start + CP_TB - 1) / CP_TB;
     if (word < 0) return;
+    if (pi_abort_late(gone, abort_w)) return;
     const cp_layout L = cp_of(DIM, vdim);
     const int nvt = vdim / 16;
-    const float * blk = scratch + ((int64_t) ord * heads + h) * L.total;
+    const float * blk0 = scratch + ((int64_t) ord * heads + h) * L.total;
     const int64_t step = (int64_t) heads * L.total;
-    float * S_hbm = state + ((int64_t) (word & ~CM_FRESH) * heads + h) * DIM * vdim + c;
-    cm_f32x4 S[DI];                                                   // rows 16 m + 4 g + r of column c: as a product leaves them, and as the next one takes them
+    if (wave >= NW) {                                                  // a helper: pieces through LDS, two ahead in registers, and the outputs of the piece before
+        const int hw = wave - NW, ht = tid - 64 * NW;
+        constexpr int CH = (ST::TILES + HELP - 1) / HELP;
+        int from[CH];                                                  // (the tail repeats the last tile)
 #pragma unroll
-    for (int m = 0; m < DI; m++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) S[m][r] = word & CM_FRESH ? 0.0f : S_hbm[(int64_t) (16 * m + 4 * g + r) * vdim];
-    cm_f32x4 W[RULE == 0 ? 2 * DI : 1], U[2];
-    int flag;
-    auto ahead = [&](const float * b, int at) {                       // what the piece's first product reads
-        flag = *(const int *) (b + L.flag);
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            if constexpr (RULE == 0) U[m] = *(const cm_f32x4 *) (b + L.u + ((m * nvt + vt) * 64 + lane) * 4);
-            else
-#pragma unroll
-                for (int r = 0; r < 4; r++) U[m][r] = v[(int64_t) min(at + 16 * m + 4 * g + r, end - 1) * vs + (int64_t) h * vdim + c];      // (behind the end: met by keys of zero)
+        for (int j = 0; j < CH; j++) {
+            const int t = min(hw + HELP * j, ST::TILES - 1);
+            from[j] = (t < 4 * DI || RULE == 0 && t < 6 * DI ? 256 * t : t < ST::NT + 4 ? L.p + 256 * (t - ST::NT) : L.u + ((t - ST::NT - 4) * nvt + vt) * 256) + 4 * lane;
         }
+        cm_f32x4 A[CH], B[CH];
+        auto load = [&](cm_f32x4 * x, int p) {
+            const float * b = blk0 + min(p, np - 1) * step;
+#pragma unroll
+            for (int j = 0; j < CH; j++) x[j] = *(const cm_f32x4 *) (b + from[j]);
+        };
+        auto pass = [&](const cm_f32x4 * x, int p) {
+            float * to = stage + (p & 1) * ST::FLOATS + 4 * lane;
+#pragma unroll
+            for (int j = 0; j < CH; j++) *(cm_f32x4 *) (to + min(hw + HELP * j, ST::TILES - 1) * 256) = x[j];
+        };
+        bool due = false;                                              // whether the piece before left outputs to be added
+        auto put = [&](int p) {                                        // the waves' parts, added in their order
+#pragma unroll
+            for (int i = 0; i < 8 / HELP; i++) {                    // (row t, column ht & 15 of what the products left: 4 g + r = t & 15)
+                const int t = (ht >> 4) + 4 * HELP * i, at = start + p * CP_TB + t;
+                const float * o = op + (p & 1) * ST::OUT + (t >> 4) * 256 + (t >> 2 & 3) * 64 + (ht & 15) * 4 + (t & 3);
+                float y = *o;
+#pragma unroll
+                for (int w = 1; w < NW; w++) y += o[w * 512];
+                if (at < end) out[(int64_t) at * os + (int64_t) h * vdim + 16 * vt + (ht & 15)] = y;
+            }
+        };
+        auto turn = [&](cm_f32x4 * x, int p) {                         // x: piece p + 1, and then p + 3
+            const bool odd = __float_as_int(stage[(p & 1) * ST::FLOATS + ST::FLAG]) != 0;
+            pass(x, p + 1);
+            cp_keep_order();
+            load(x, p + 3);
+            cp_keep_order();
+            if (odd) for (int t = 0; t < min(CP_TB, end - start - p * CP_TB); t++) __syncthreads();
+            __syncthreads();
+            if (due) put(p - 1);
+            due = !odd;
+        };
+        load(A, 0);
+        pass(A, 0);
+        cp_keep_order();
+        load(B, 1);
+        cp_keep_order();
+        load(A, 2);
+        cp_keep_order();
+        __syncthreads();
+        for (int p = 0; p < np; p += 2) {
+            turn(B, p);
+            if (p + 1 >= np) break;
+            turn(A, p + 1);
+        }
+        __syncthreads();
+        if (due) put(np - 1);
+        return;
+    }
+    float * S_hbm = state + ((int64_t) (word & ~CM_FRESH) * heads + h) * DIM * vdim + c;
+    cm_f32x4 S[MT];                                                   // rows 16 (m0 + m) + 4 g + r of column c: as a product leaves them, and as the next one takes them
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) S[m][r] = word & CM_FRESH ? 0.0f : S_hbm[(int64_t) (16 * (m0 + m) + 4 * g + r) * vdim];
+    __builtin_amdgcn_s_setprio(1);
+    __syncthreads();
+    // a piece's operands are in registers when it begins: what its first products have read is read again behind the barrier, for the next piece, the rest behind its last products
+    cm_f32x4 W[RULE == 0 ? 2 * MT : 1], Q[2 * MT], K[2 * MT], G[MT], V[2];
+    float P[3][4 / NW];
+    int flag;
+    auto first = [&](int p) {
+        const float * x = stage + (p & 1) * ST::FLOATS + 4 * lane;
+        flag = __float_as_int(stage[(p & 1) * ST::FLOATS + ST::FLAG]);
         if constexpr (RULE == 0)
 #pragma unroll
-            for (int i = 0; i < 2 * DI; i++) W[i] = *(const cm_f32x4 *) (b + L.w + (i * 64 + lane) * 4);
+            for (int m = 0; m < 2; m++)
+#pragma unroll
+                for (int i = 0; i < MT; i++) W[m * MT + i] = *(const cm_f32x4 *) (x + (4 * DI + m * DI + m0 + i) * 256);
+#pragma unroll
+        for (int m = 0; m < 2; m++) V[m] = *(const cm_f32x4 *) (x + ST::U + m * 256);
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int i = 0; i < MT; i++) Q[m * MT + i] = *(const cm_f32x4 *) (x + (m * DI + m0 + i) * 256);
     };
-    ahead(blk, start);
-    for (int p = 0; p < np; p++, blk += step) {
-        const int at = start + p * CP_TB, len = min(CP_TB, end - at);
-        if (flag) {
+    auto second = [&](int p) {
+        const float * x = stage + (p & 1) * ST::FLOATS;
+#pragma unroll
+        for (int m = 0; m < MT; m++) G[m] = *(const cm_f32x4 *) (x + ST::G + 16 * (m0 + m) + 4 * g);
+#pragma unroll
+        for (int i = 0; i < 2 * MT; i++) K[i] = *(const cm_f32x4 *) (x + (2 * DI + 2 * m0 + i) * 256 + 4 * lane);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int e = 0; e < 4 / NW; e++) P[i][e] = x[ST::P + i * 256 + 4 * lane + wave + NW * e];
+    };
+    first(0); second(0);
+    for (int p = 0; p < np; p++) {
+        const bool odd = __builtin_amdgcn_readfirstlane(flag) != 0;
+        cm_f32x4 U[2], O[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
+        if (odd) {                                                     // token by token
+            const float * blk = blk0 + p * step;
+            const int at = start + p * CP_TB, len = min(CP_TB, end - at);
             for (int t = 0; t < len; t++) {
-                cm_f32x4 kv[DI];
+                cm_f32x4 kv[MT];
                 float a = 0.0f, o = 0.0f;
 #pragma unroll
-                for (int m = 0; m < DI; m++) {
-                    kv[m] = *(const cm_f32x4 *) (blk + L.k + t * DIM + 16 * m + 4 * g);
-                    const cm_f32x4 qv = *(const cm_f32x4 *) (blk + L.q + t * DIM + 16 * m + 4 * g), gv = *(const cm_f32x4 *) (blk + L.w + t * DIM + 16 * m + 4 * g);
+                for (int m = 0; m < MT; m++) {
+                    const int i = t * DIM + 16 * (m0 + m) + 4 * g;
+                    kv[m] = *(const cm_f32x4 *) (blk + L.k + i);
+                    const cm_f32x4 qv = *(const cm_f32x4 *) (blk + L.q + i), gv = *(const cm_f32x4 *) (blk + L.w + i);
                     if (RULE == 0) S[m] *= gv;
 #pragma unroll
                     for (int r = 0; r < 4; r++) { a = fmaf(S[m][r], kv[m][r], a); o = fmaf(S[m][r], qv[r], o); }
                     if (RULE == 1) S[m] *= gv;
                 }
                 a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64); o += __shfl_xor(o, 16, 64); o += __shfl_xor(o, 32, 64);
-                const float x = v[(int64_t) (at + t) * vs + (int64_t) h * vdim + c], u = RULE == 0 ? blk[L.p + t] * (x - a) : x;
+                if (g == 0) { one[t & 1][wave][0][n] = a; one[t & 1][wave][1][n] = o; }
+                __syncthreads();
+                a = one[t & 1][0][0][n]; o = one[t & 1][0][1][n];
 #pragma unroll
-                for (int m = 0; m < DI; m++)
+                for (int w = 1; w < NW; w++) { a += one[t & 1][w][0][n]; o += one[t & 1][w][1][n]; }
+                const float y = v[(int64_t) (at + t) * vs + (int64_t) h * vdim + c], u = RULE == 0 ? blk[L.p + t] * (y - a) : y;
+#pragma unroll
+                for (int m = 0; m < MT; m++)
 #pragma unroll
                     for (int r = 0; r < 4; r++) S[m][r] = fmaf(kv[m][r], u, S[m][r]);
-                if (g == 0) out[(int64_t) (at + t) * os + (int64_t) h * vdim + c] = fmaf(u, blk[L.p + CP_TB + t], o);
+                if (tid < 16) out[(int64_t) (at + t) * os + (int64_t) h * vdim + c] = fmaf(u, blk[L.p + CP_TB + t], o);
             }
-            const float * nb = p + 1 < np ? blk + step : blk;
-            ahead(nb, p + 1 < np ? at + CP_TB : at);
-            continue;
+        } else {
+            U[0] = V[0]; U[1] = V[1];
+            if constexpr (RULE == 0) {
+                if (wave) U[0] = U[1] = cm_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };       // (T beta V goes in once)
+#pragma unroll
+                for (int s = 0; s < MT; s++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) { U[0] = cm_mfma(W[s][i], S[s][i], U[0]); U[1] = cm_mfma(W[MT + s][i], S[s][i], U[1]); }
+                float * const mine = us + (p & 1) * ST::PARTS + wave * 512 + lane * 4;
+                *(cm_f32x4 *) mine = U[0];
+                *(cm_f32x4 *) (mine + 256) = U[1];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 2 * MT; i++) { O[0] = cm_mfma(Q[i >> 2][i & 3], S[i >> 2][i & 3], O[0]); O[1] = cm_mfma(Q[MT + (i >> 2)][i & 3], S[i >> 2][i & 3], O[1]); }
         }
-        cm_f32x4 Q[2 * DI], K[2 * DI], P[3], G[DI], O[2] = { { 0.0f, 0.0f, 0.0f, 0.0f }, { 0.0f, 0.0f, 0.0f, 0.0f } };
-#pragma unroll
-        for (int i = 0; i < 2 * DI; i++) Q[i] = *(const cm_f32x4 *) (blk + L.q + (i * 64 + lane) * 4);
-#pragma unroll
-        for (int i = 0; i < 3; i++) P[i] = *(const cm_f32x4 *) (blk + L.p + (i * 64 + lane) * 4);
-#pragma unroll
-        for (int i = 0; i < 2 * DI; i++) K[i] = *(const cm_f32x4 *) (blk + L.k + (i * 64 + lane) * 4);
-#pragma unroll
-        for (int m = 0; m < DI; m++) G[m] = *(const cm_f32x4 *) (blk + L.g + 16 * m + 4 * g);
-        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                               // the waves' parts of U are there, and the next piece; this one's buffer is free
+        cm_f32x4 part[RULE == 0 ? 2 * NW : 1];
         if constexpr (RULE == 0)
 #pragma unroll
-            for (int s = 0; s < DI; s++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) { U[0] = cm_mfma(W[s][i], S[s][i], U[0]); U[1] = cm_mfma(W[DI + s][i], S[s][i], U[1]); }
-        const cm_f32x4 U0 = U[0], U1 = U[1];
+            for (int i = 0; i < 2 * NW; i++) part[i] = *(const cm_f32x4 *) (us + (p & 1) * ST::PARTS + i * 256 + lane * 4);
         __builtin_amdgcn_sched_barrier(0);
-        ahead(p + 1 < np ? blk + step : blk, p + 1 < np ? at + CP_TB : at);
+        if (!odd) {                                                    // (the second half of Q' S: the parts arrive meanwhile)
+#pragma unroll
+            for (int i = 2 * MT; i < 4 * MT; i++) { O[0] = cm_mfma(Q[i >> 2][i & 3], S[i >> 2][i & 3], O[0]); O[1] = cm_mfma(Q[MT + (i >> 2)][i & 3], S[i >> 2][i & 3], O[1]); }
+#pragma unroll
+            for (int m = 0; m < MT; m++) S[m] *= G[m];
+        }
         __builtin_amdgcn_sched_barrier(0);
+        first(p + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!odd) {
+            if constexpr (RULE == 0) {
+                U[0] = part[0]; U[1] = part[1];
 #pragma unroll
-        for (int s = 0; s < DI; s++)
+                for (int w = 1; w < NW; w++) { U[0] += part[2 * w]; U[1] += part[2 * w + 1]; }
+            }
 #pragma unroll
-            for (int i = 0; i < 4; i++) { O[0] = cm_mfma(Q[s][i], S[s][i], O[0]); O[1] = cm_mfma(Q[DI + s][i], S[s][i], O[1]); }
+            for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int m = 0; m < DI; m++) S[m] *= G[m];
+                for (int m = 0; m < MT; m++) S[m] = cm_mfma(K[2 * m][i], U[0][i], S[m]);
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+            for (int e = 0; e < 4 / NW; e++) {                        // P U: a part of the inner index per wave
+                const int i = wave + NW * e;
+                const float u0 = i == 0 ? U[0][0] : i == 1 ? U[0][1] : i == 2 ? U[0][2] : U[0][3], u1 = i == 0 ? U[1][0] : i == 1 ? U[1][1] : i == 2 ? U[1][2] : U[1][3];
+                O[0] = cm_mfma(P[0][e], u0, O[0]);
+                O[1] = cm_mfma(P[1][e], u0, O[1]);
+                O[1] = cm_mfma(P[2][e], u1, O[1]);
+            }
 #pragma unroll
-            for (int m = 0; m < DI; m++) S[m] = cm_mfma(K[2 * m][i], U0[i], S[m]);
-        O[0] = cm_mfma4(P[0], U0, O[0]);
-        O[1] = cm_mfma4(P[1], U0, O[1]);
-        O[1] = cm_mfma4(P[2], U1, O[1]);
+            for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int m = 0; m < DI; m++) S[m] = cm_mfma(K[2 * m + 1][i], U1[i], S[m]);
-#pragma unroll
-        for (int m = 0; m < 2; m++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) { const int t = 16 * m + 4 * g + r; if (t < len) out[(int64_t) (at + t) * os + (int64_t) h * vdim + c] = O[m][r]; }
+                for (int m = 0; m < MT; m++) S[m] = cm_mfma(K[2 * m + 1][i], U[1][i], S[m]);
+            __builtin_amdgcn_sched_barrier(0);
+            float * o = op + (p & 1) * ST::OUT + wave * 512 + lane * 4;
+            *(cm_f32x4 *) o = O[0];
+            *(cm_f32x4 *) (o + 256) = O[1];
+        }
+        second(p + 1);
     }
+    __syncthreads();
 #pragma unroll
-    for (int m = 0; m < DI; m++)
+    for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) S_hbm[(int64_t) (16 * m + 4 * g + r) * vdim] = S[m][r];
+        for (int r = 0; r < 4; r++) S_hbm[(int64_t) (16 * (m0 + m) + 4 * g + r) * vdim] = S[m][r];
 }
 
 #define CR_LDS_MAX (150 * 1024)
 template <int DPT, int RULE> static int cr_reserve_one() { PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_recurrence<DPT, RULE>, hipFuncAttributeMaxDynamicSharedMemorySize, CR_LDS_MAX)); return 0; }
+template <int DI, int RULE> static int cp_reserve_one() { PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_walk<DI, RULE>, hipFuncAttributeMaxDynamicSharedMemorySize, cp_stage<DI, RULE>::LDS)); return 0; }
 extern "C" int pi_op_channel_recurrence_reserve(void) {
     static bool done = false;
     if (done) return 0;
     if (cr_reserve_one<8, 0>() || cr_reserve_one<16, 0>() || cr_reserve_one<32, 0>() || cr_reserve_one<8, 1>() || cr_reserve_one<16, 1>() || cr_reserve_one<32, 1>()) return -1;
+    if (cp_reserve_one<2, 0>() || cp_reserve_one<4, 0>() || cp_reserve_one<8, 0>() || cp_reserve_one<2, 1>() || cp_reserve_one<4, 1>() || cp_reserve_one<8, 1>()) return -1;
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_state_scan<8>, hipFuncAttributeMaxDynamicSharedMemorySize, CR_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_state_scan<16>, hipFuncAttributeMaxDynamicSharedMemorySize, CR_LDS_MAX));
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_channel_state_scan<32>, hipFuncAttributeMaxDynamicSharedMemorySize, CR_LDS_MAX));
@@ -870,11 +1062,12 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
     if (!pieces) return launch(0);
     if (cp_takes(dim, vdim) && (rule == PI_RULE_BONUS || qk_unit) && scratch_floats >= cp_floats(heads, dim, vdim, n_tok, max_segments) && ((uintptr_t) scratch_dev & 15) == 0) {
         const dim3 pg((unsigned) heads, (unsigned) cr_max_pieces(n_tok, max_segments, CP_TB)), wg((unsigned) heads, (unsigned) (vdim / 16), (unsigned) runs);
+        if (pi_op_channel_recurrence_reserve() != 0) return -1;
         const double blocks = 4.0 * pg.y * heads * cp_of(dim, vdim).total;
-#define CP_GO(DI, RL) do { PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_pieces<DI, RL>), pg, dim3(256), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
+#define CP_GO(DI, RL) do { PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_pieces<DI, RL>), pg, dim3(CP_PIECE_THREADS), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
                                         beta_raw, beta_stride, bonus_dev, qk_unit, q_mult, heads, heads / qk_heads, vdim, rec_dev, n_tok, scratch_dev, pi_abort_word()); \
                            PI_CHECK_LAUNCH(); \
-                           PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_walk<DI, RL>), wg, dim3(64), 0, s, v, v_stride, heads, vdim, state_dev, rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word()); } while (0)
+                           PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes + blocks, (k_channel_walk<DI, RL>), wg, dim3(64 * (CP_WAVES(DI) + CP_HELP(RL))), (cp_stage<DI, RL>::LDS), s, v, v_stride, heads, vdim, state_dev, rec_dev, n_tok, scratch_dev, out, out_stride, pi_abort_word()); } while (0)
 #define CP_RULE(RL) do { if (dim == 32) CP_GO(2, RL); else if (dim == 64) CP_GO(4, RL); else CP_GO(8, RL); } while (0)
         if (rule == PI_RULE_DELTA) CP_RULE(0); else CP_RULE(1);
 #undef CP_RULE
