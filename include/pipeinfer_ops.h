@@ -210,9 +210,15 @@ PI_API int pi_op_latent_attention(const float * q_dev, int64_t q_stride, const f
 PI_API size_t pi_op_latent_attention_scratch_floats(int heads, int rank, int n_tok, int n_kv);
 PI_API int pi_op_latent_attention_reserve(void);                   /* once per process, outside graph capture: LDS limit of the score kernels */
 PI_API int pi_op_latent_attention_max_cells(int rank);             /* longest context the kernels serve */
+/* pi_op_rms_scale with a residual, and of the result another one, plain, -> out2 (an asked rounding is out2's) */
+PI_API int pi_op_rms_scale_twice(const float * x_dev, int64_t x_stride, const float * w_dev, float w_offset, float eps, int n, int n_tok, const float * residual_dev, int64_t residual_stride, float mult,
+                                 float * out_dev, int64_t out_stride, const float * w2_dev, float w2_offset, float * out2_dev, int64_t out2_stride, void * stream);
 /* Router of a mixture of experts: scores = softmax(W_router x) over all outputs; the `top` outputs with the largest score + correction are chosen (lowest index wins a tie); their
  * weights are the scores themselves.  sel_dev / selw_dev: [n_tok][top] */
 PI_API int pi_op_moe_route(const pi_weight * router, const float * correction_dev, const float * x_dev, int64_t x_stride, int n_tok, int top, int exact, int32_t * sel_dev, float * selw_dev, void * stream);
+/* pi_op_rms_scale with a residual, and pi_op_moe_route of the result */
+PI_API int pi_op_rms_scale_route(const float * y_dev, int64_t y_stride, const float * w_dev, float w_offset, float eps, const float * residual_dev, int64_t residual_stride, float mult, float * out_dev, int64_t out_stride,
+                                 const pi_weight * router, const float * correction_dev, int n_tok, int top, int exact, int32_t * sel_dev, float * selw_dev, void * stream);
 /* out[t] = sum over the chosen outputs e of weight * (e < n_exp ? W_down[e] relu(W_up[e] x[t])^2 : x[t]); w_up: [n_exp * ff][width], w_down: [n_exp * width][ff]; up_dev: scratch [n_tok][top][ff] */
 PI_API int pi_op_moe_experts(const pi_weight * w_up, const pi_weight * w_down, int n_exp, int ff, const float * x_dev, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev, int n_tok, int top,
                              int exact, float * up_dev, float * out_dev, int64_t out_stride, void * stream);
@@ -224,6 +230,11 @@ PI_API int pi_op_moe_rounded_ok(const pi_weight * wup, const pi_weight * wdown, 
 /* the same from inputs in bfloat16 (xh; x: the same in fp32, what identity experts hand on), up_dev [n_tok * top][ff] in bfloat16; pi_op_moe_rounded_ok says for which passes */
 PI_API int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh_dev, int64_t xh_stride, const float * x_dev, int64_t x_stride, const int32_t * sel_dev,
                                      const float * selw_dev, int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out_dev, int64_t out_stride, void * stream);
+/* the same, and pi_op_rms_scale of the result with a residual (w2 not null: pi_op_rms_scale_twice); sum: [n_tok][width], where the result may have to stand in between */
+PI_API int pi_op_moe_experts_rounded_norm(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh_dev, int64_t xh_stride, const float * x_dev, int64_t x_stride, const int32_t * sel_dev,
+                                          const float * selw_dev, int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * sum_dev, int64_t sum_stride, const float * w_dev, float w_offset, float eps,
+                                          const float * residual_dev, int64_t residual_stride, float mult, float * out_dev, int64_t out_stride, const float * w2_dev, float w2_offset, float * out2_dev, int64_t out2_stride,
+                                          void * stream);
 PI_API int pi_op_moe_experts_grouped(const pi_weight * w_up, const pi_weight * w_down, int n_exp, int ff, const float * x_dev, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev, int n_tok, int top,
                                      float * up_dev, float * dn_dev, int32_t * idx_dev, float * out_dev, int64_t out_stride, void * stream);
 

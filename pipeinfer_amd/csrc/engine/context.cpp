@@ -906,7 +906,7 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
     float * x = ctx->x, * P = ctx->h_in, * A = ctx->h_att, * Y = ctx->h_out;
     // the stream in bfloat16 where the next projection reads it so
     auto x_rounded = [&](size_t il) { return il < hp.hybrid.size() ? reads_rounded(ctx, m->hweights[(size_t) hp.hybrid[il].weights].w_in, n_tok, ctx->x_h) : nullptr; };
-    uint16_t * xh = x_rounded(0);
+    uint16_t * xh = x_rounded(0), * nh = reads_rounded(ctx, m->tok_embd, n_tok, ctx->x_h);
     OP_OK(op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_embed(m->tok_embd, ctx->tokens_dev, n_tok, hp.embed_scale, x, s); }));
     for (size_t il = 0; il < hp.hybrid.size(); il++) {
         const pi_hybrid_layer & H = hp.hybrid[il];
@@ -930,21 +930,32 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         xh = x_rounded(il + 1);
         // experts without a gate, a prompt: by expert on the matrix cores, from the stream in bfloat16
         const bool moe_h = H.has_mlp && !ex && pi_op_moe_rounded_ok(W.e_up, W.e_down, H.n_expert, H.ff, width, n_tok, H.top);
-        OP_OK(op_rounded(ctx, H.has_mlp ? (moe_h ? ctx->x_h : nullptr) : xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm1, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
-        if (H.has_mlp) {
-            OP_OK(pi_op_moe_route(W.router, W.correction, x, width, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s));
+        // the layer's last norm: a row of the stream, and behind the last layer the head's input with it
+        const float * w2 = il + 1 == hp.hybrid.size() ? m->output_norm : nullptr;
+        auto stream_norm = [&](const float * w) {
+            return w2 ? op_rounded(ctx, nh, ctx->nx, width, 0, width, n_tok, true, s, [&] { return pi_op_rms_scale_twice(Y, width, w, 1.0f, eps, width, n_tok, x, width, rm, x, width, w2, 1.0f, ctx->nx, width, s); })
+                      : op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, w, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); });
+        };
+        if (!H.has_mlp) OP_OK(stream_norm(W.norm1));
+        else {
+            OP_OK(op_rounded(ctx, moe_h ? ctx->x_h : nullptr, x, width, 0, width, n_tok, false, s, [&] {
+                return pi_op_rms_scale_route(Y, width, W.norm1, 1.0f, eps, x, width, rm, x, width, W.router, W.correction, n_tok, H.top, ex, ctx->moe_sel, ctx->moe_w, s);
+            }));
             if (moe_h)
-                OP_OK(pi_op_moe_experts_rounded(W.e_up, W.e_down, H.n_expert, H.ff, ctx->x_h, width, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, (uint16_t *) ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
-            else if (pi_op_moe_grouped_ok(W.e_up, W.e_down, H.n_expert, H.ff, 0, n_tok, H.top, ex))
-                OP_OK(pi_op_moe_experts_grouped(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
-            else
-                OP_OK(pi_op_moe_experts(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ex, ctx->moe_up, Y, width, s));
-            OP_OK(op_rounded(ctx, xh, x, width, 0, width, n_tok, false, s, [&] { return pi_op_rms_scale(Y, width, W.norm2, 1.0f, eps, width, n_tok, nullptr, 0, x, width, rm, x, width, nullptr, 0, s); }));
+                OP_OK(op_rounded(ctx, w2 ? nh : xh, w2 ? ctx->nx : x, width, 0, width, n_tok, w2 != nullptr, s, [&] {
+                    return pi_op_moe_experts_rounded_norm(W.e_up, W.e_down, H.n_expert, H.ff, ctx->x_h, width, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, (uint16_t *) ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width,
+                                                          W.norm2, 1.0f, eps, x, width, rm, x, width, w2, 1.0f, ctx->nx, width, s);
+                }));
+            else {
+                if (pi_op_moe_grouped_ok(W.e_up, W.e_down, H.n_expert, H.ff, 0, n_tok, H.top, ex))
+                    OP_OK(pi_op_moe_experts_grouped(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ctx->moe_up, ctx->moe_dn, ctx->moe_idx, Y, width, s));
+                else
+                    OP_OK(pi_op_moe_experts(W.e_up, W.e_down, H.n_expert, H.ff, x, width, ctx->moe_sel, ctx->moe_w, n_tok, H.top, ex, ctx->moe_up, Y, width, s));
+                OP_OK(stream_norm(W.norm2));
+            }
         }
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
-    uint16_t * nh = reads_rounded(ctx, m->tok_embd, n_tok, ctx->x_h);
-    OP_OK(op_rounded(ctx, nh, ctx->nx, width, 0, width, n_tok, true, s, [&] { return pi_op_rms_scale(x, width, m->output_norm, 1.0f, eps, width, n_tok, nullptr, 0, nullptr, 0, 1.0f, ctx->nx, width, nullptr, 0, s); }));
     OP_OK(dense(ctx, m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, nh, width));
     OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
     return true;

@@ -19,7 +19,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <type_traits>
+#include <utility>
 
 static __device__ __forceinline__ float hy_widen(uint16_t b) { return __uint_as_float((uint32_t) b << 16); }
 static __device__ __forceinline__ float hy_round(float f) { const uint32_t u = __float_as_uint(f); return __uint_as_float(((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) << 16); }
@@ -64,10 +66,55 @@ static __device__ __forceinline__ float hy_block_max(float v, float * red) {
 }
 
 // ---- RMS norm with its usual companions ---------------------------------------------------------------------------------------------------------
+// A row of up to 1024 NV values in the registers of 256 threads (thread i: values 4 i .. of every 1024): its norm, gate, multiplier and residual, in place.  Further threads of the workgroup only take part in the sum
+// (as zeros: a row's bits do not depend on their number).  red: a float for each wave
+template <int NV>
+static __device__ __forceinline__ void hy_rms_row(float4 (&xv)[NV], const float4 (&wv)[NV], float w_off, float eps, int n, const float4 * gv, const float4 * rv, float mult, float * red) {
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) if (threadIdx.x < 256 && (int) threadIdx.x * 4 + 1024 * j < n) { ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss); ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss); }
+    ss = hy_block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float) n + eps);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        float y[4] = { xv[j].x * inv * (wv[j].x + w_off), xv[j].y * inv * (wv[j].y + w_off), xv[j].z * inv * (wv[j].z + w_off), xv[j].w * inv * (wv[j].w + w_off) };
+        if (gv) { y[0] *= gv[j].x; y[1] *= gv[j].y; y[2] *= gv[j].z; y[3] *= gv[j].w; }
+#pragma unroll
+        for (int k = 0; k < 4; k++) y[k] *= mult;
+        if (rv) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
+        xv[j] = make_float4(y[0], y[1], y[2], y[3]);
+    }
+}
+// the row's results: a second norm's where w2 is given (the one ahead of the output head: its input is this row), beside the row itself
+struct hy_second { const float * w; float w_off; float * out; int64_t os; };
+struct hy_norm { const float * w; float w_off, eps; const float * res; int64_t rs; float mult; float * out; int64_t os; hy_second two; };
+template <int NV>
+static __device__ __forceinline__ void hy_rms_store(float4 (&xv)[NV], int t, int64_t orow, int n, float eps, float * out, int64_t os, const hy_second & two, const pi_round_dst & rd, float * red) {
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = (int) threadIdx.x * 4 + 1024 * j;
+        if (i >= n || threadIdx.x >= 256) break;
+        if (two.w || !rd.only) *(float4 *) (out + orow * os + i) = xv[j];
+        if (!two.w && rd.h) pi_round_store4(rd, t, i, xv[j].x, xv[j].y, xv[j].z, xv[j].w);
+    }
+    if (!two.w) return;
+    float4 wv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) wv[j] = *(const float4 *) (two.w + min((int) threadIdx.x * 4 + 1024 * j, n - 4));
+    hy_rms_row<NV>(xv, wv, two.w_off, eps, n, nullptr, nullptr, 1.0f, red);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = (int) threadIdx.x * 4 + 1024 * j;
+        if (i >= n || threadIdx.x >= 256) break;
+        if (!rd.only) *(float4 *) (two.out + (int64_t) t * two.os + i) = xv[j];
+        if (rd.h) pi_round_store4(rd, t, i, xv[j].x, xv[j].y, xv[j].z, xv[j].w);
+    }
+}
 // rows of up to 1024 NV aligned values: everything the row needs is on its way before its sum (a row that was read again behind the sum: one more trip to memory, 3.4 us a launch instead of 3.1)
 template <int NV>
 __global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n, const float * __restrict__ gate, int64_t gs,
-                                                        const float * __restrict__ res, int64_t rs, float mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
+                                                        const float * __restrict__ res, int64_t rs, float mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ dyn, int to_cells, const hy_second two,
+                                                        const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     __shared__ float red[4];
     const int t = blockIdx.x;
@@ -80,24 +127,9 @@ __global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict
         if (gate) gv[j] = *(const float4 *) (gate + (int64_t) t * gs + i);
         if (res) rv[j] = *(const float4 *) (res + (int64_t) t * rs + i);
     }
-    float ss = 0.0f;
-#pragma unroll
-    for (int j = 0; j < NV; j++) if ((int) threadIdx.x * 4 + 1024 * j < n) { ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss); ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss); }
-    ss = hy_block_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float) n + eps);
+    hy_rms_row<NV>(xv, wv, w_off, eps, n, gate ? gv : nullptr, res ? rv : nullptr, mult, red);
     if (pi_abort_late(gone, abort_w)) return;
-#pragma unroll
-    for (int j = 0; j < NV; j++) {
-        const int i = (int) threadIdx.x * 4 + 1024 * j;
-        if (i >= n) break;
-        float y[4] = { xv[j].x * inv * (wv[j].x + w_off), xv[j].y * inv * (wv[j].y + w_off), xv[j].z * inv * (wv[j].z + w_off), xv[j].w * inv * (wv[j].w + w_off) };
-        if (gate) { y[0] *= gv[j].x; y[1] *= gv[j].y; y[2] *= gv[j].z; y[3] *= gv[j].w; }
-#pragma unroll
-        for (int k = 0; k < 4; k++) y[k] *= mult;
-        if (res) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
-        if (!rd.only) *(float4 *) (out + orow * os + i) = make_float4(y[0], y[1], y[2], y[3]);
-        if (rd.h) pi_round_store4(rd, t, i, y[0], y[1], y[2], y[3]);
-    }
+    hy_rms_store<NV>(xv, t, orow, n, eps, out, os, two, rd, red);
 }
 __global__ void __launch_bounds__(256) k_rms_scale(const float * __restrict__ x, int64_t xs, const float * __restrict__ w, float w_off, float eps, int n,
                                                    const float * __restrict__ gate, int64_t gs, const float * __restrict__ res, int64_t rs, float mult,
@@ -133,21 +165,41 @@ __global__ void __launch_bounds__(256) k_rms_scale(const float * __restrict__ x,
     }
 }
 
+static bool rms_vec(int n, std::initializer_list<std::pair<const void *, int64_t>> rows) {
+    bool ok = n % 4 == 0;
+    for (const auto & r : rows) ok = ok && (!r.first || (((uintptr_t) r.first % 16) == 0 && r.second % 4 == 0));
+    return ok;
+}
 extern "C" int pi_op_rms_scale(const float * x, int64_t x_stride, const float * w, float w_offset, float eps, int n, int n_tok, const float * gate, int64_t gate_stride,
                                const float * residual, int64_t residual_stride, float mult, float * out, int64_t out_stride, const int32_t * dyn_dev, int to_cells, void * stream) {
     if (n_tok <= 0 || n <= 0) return 0;
     if (to_cells && !dyn_dev) { pi_set_error("pi_op_rms_scale: rows go to cache cells but no cell table was given"); return -1; }
-    auto al = [](const void * p, int64_t stride) { return !p || (((uintptr_t) p % 16) == 0 && stride % 4 == 0); };
-    const int vec = n % 4 == 0 && al(x, x_stride) && al(w, 0) && al(gate, gate_stride) && al(residual, residual_stride) && al(out, out_stride);
-#define RS_GO(NV) do { PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale_once<NV>, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride, residual, \
-                                    residual_stride, mult, out, out_stride, dyn_dev, to_cells, to_cells ? pi_round_dst{} : pi_round_asked(0, n), pi_abort_word()); PI_CHECK_LAUNCH(); return 0; } while (0)
-    if (vec && n <= 1024) RS_GO(1);
-    if (vec && n <= 2048) RS_GO(2);
-    if (vec && n <= 4096) RS_GO(4);
-#undef RS_GO
+    const int vec = rms_vec(n, { { x, x_stride }, { w, 0 }, { gate, gate_stride }, { residual, residual_stride }, { out, out_stride } });
+#define RS_GO(NV, TWO) do { PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale_once<NV>, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride, residual, \
+                                    residual_stride, mult, out, out_stride, dyn_dev, to_cells, TWO, to_cells ? pi_round_dst{} : pi_round_asked(0, n), pi_abort_word()); PI_CHECK_LAUNCH(); return 0; } while (0)
+    if (vec && n <= 1024) RS_GO(1, hy_second{});
+    if (vec && n <= 2048) RS_GO(2, hy_second{});
+    if (vec && n <= 4096) RS_GO(4, hy_second{});
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 12.0 * n * n_tok, k_rms_scale, dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, x, x_stride, w, w_offset, eps, n, gate, gate_stride,
                  residual, residual_stride, mult, out, out_stride, dyn_dev, to_cells, vec, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
+}
+// pi_op_rms_scale of a row and, of the result, a second one (plain) -> out2, in one launch where the row's values stay in registers; an asked rounding is the second's.  us of the two launches / of this: one token of
+// 2048 8.6 / 4.6; 512 of 2048 9.4 / 6.3; 2048 of 4096 36 / 30
+extern "C" int pi_op_rms_scale_twice(const float * x, int64_t x_stride, const float * w, float w_offset, float eps, int n, int n_tok, const float * residual, int64_t residual_stride, float mult, float * out, int64_t out_stride,
+                                     const float * w2, float w2_offset, float * out2, int64_t out2_stride, void * stream) {
+    if (n_tok <= 0 || n <= 0) return 0;
+    const bool vec = rms_vec(n, { { x, x_stride }, { w, 0 }, { residual, residual_stride }, { out, out_stride }, { w2, 0 }, { out2, out2_stride } });
+    const float * gate = nullptr; const int64_t gate_stride = 0; const int32_t * dyn_dev = nullptr; const int to_cells = 0;
+    const hy_second two = { w2, w2_offset, out2, out2_stride };
+    if (vec && n <= 1024) RS_GO(1, two);
+    if (vec && n <= 2048) RS_GO(2, two);
+    if (vec && n <= 4096) RS_GO(4, two);
+#undef RS_GO
+    const pi_round_dst asked = pi_round_take();
+    if (pi_op_rms_scale(x, x_stride, w, w_offset, eps, n, n_tok, gate, gate_stride, residual, residual_stride, mult, out, out_stride, nullptr, 0, stream) != 0) return -1;
+    pi_set_rounded_output(asked.h, asked.stride, asked.from, asked.n, asked.only);
+    return pi_op_rms_scale(out, out_stride, w2, w2_offset, eps, n, n_tok, nullptr, 0, nullptr, 0, 1.0f, out2, out2_stride, nullptr, 0, stream);
 }
 
 // ---- layer norm (weight and bias) over one or the weighted sum of two inputs, optional residual; the row operations at the end of a block -----------------------------
@@ -2015,20 +2067,9 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
 // one workgroup per token: logits of all router outputs (a wave per output; few tokens: up to sixteen waves, so that ten outputs are one trip to memory: 7.2 us on four, 5.4 so), soft-max, choice = score + correction, `top` rounds of arg-max (lowest index wins a tie)
 // n_groups > 0: the scores are sigmoid(logit), consecutive outputs are bundled into n_groups groups of equal size, a group is ranked by top1 + top2 of its members' scores, and the
 // choice is restricted to members of the `keep` highest-ranked groups (then by their own score; lowest index wins a tie, among groups as among outputs)
-__global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict__ router, int64_t width, int n_out, const float * __restrict__ corr, const float * __restrict__ x, int64_t xs,
-                                                   int top, int exact, int vec, int n_groups, int keep, int32_t * __restrict__ sel, float * __restrict__ selw, const int32_t * __restrict__ abort_w) {
-    const int gone = pi_abort_peek(abort_w);
-    extern __shared__ float z[];                  // [n_out] logits -> scores | [n_out] choice | [n_groups] group scores
-    float * ch = z + n_out, * gsc = ch + n_out;
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const float * xr = x + (int64_t) t * xs;
-    for (int e = wave; e < n_out; e += (int) (blockDim.x >> 6)) {
-        const float a = pi_lanes_sum<64>(hy_dot_lane(router + (int64_t) e * width, xr, width, lane, exact != 0, vec != 0));
-        if (gone & 1) break;                                           // (no further outputs for a cancelled run)
-        if (lane == 0) z[e] = a;
-    }
-    __syncthreads();
-    if (wave != 0 || pi_abort_late(gone, abort_w)) return;
+// (moe_choose: one wave, from the logits in z)
+static __device__ __forceinline__ void moe_choose(float * z, int n_out, const float * __restrict__ corr, int top, int n_groups, int keep, int t, int lane, int32_t * __restrict__ sel, float * __restrict__ selw) {
+    float * ch = z + n_out, * gsc = ch + n_out;   // [n_out] logits -> scores | [n_out] choice | [n_groups] group scores
     if (n_groups < 0) {                           // by logit (+ bias); the weights are worked out over the chosen ones below
         for (int e = lane; e < n_out; e += 64) { z[e] += corr ? corr[e] : 0.0f; ch[e] = z[e]; }
     } else if (n_groups > 0) {
@@ -2076,6 +2117,73 @@ __global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict_
         for (int kk = 0; kk < top; kk++) { wt[kk] = expf(wt[kk] - m); l += wt[kk]; }
         for (int kk = 0; kk < top; kk++) wt[kk] = wt[kk] / l;
     }
+}
+__global__ void __launch_bounds__(1024) k_moe_route(const uint16_t * __restrict__ router, int64_t width, int n_out, const float * __restrict__ corr, const float * __restrict__ x, int64_t xs,
+                                                   int top, int exact, int vec, int n_groups, int keep, int32_t * __restrict__ sel, float * __restrict__ selw, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    extern __shared__ float z[];
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const float * xr = x + (int64_t) t * xs;
+    for (int e = wave; e < n_out; e += (int) (blockDim.x >> 6)) {
+        const float a = pi_lanes_sum<64>(hy_dot_lane(router + (int64_t) e * width, xr, width, lane, exact != 0, vec != 0));
+        if (gone & 1) break;                                           // (no further outputs for a cancelled run)
+        if (lane == 0) z[e] = a;
+    }
+    __syncthreads();
+    if (wave != 0 || pi_abort_late(gone, abort_w)) return;
+    moe_choose(z, n_out, corr, top, n_groups, keep, t, lane, sel, selw);
+}
+// The norm ahead of the router and the router, a workgroup per token: the row goes from the norm's registers to LDS as the products read it (exact: as it is; else rounded once, not once per output), and a wave's first
+// output's weights leave ahead of the norm.  us of the two launches / of this, 10 outputs: 1 token of
+// 2048 7.9 / 5.5, of 4096 10.0 / 6.7; 512 tokens of 2048 12.4 / 7.5, 2048 of 4096 50 / 23; 64 outputs, 2048 tokens of 4096 143 / 57
+template <int NV>
+__global__ void __launch_bounds__(1024) k_rms_route(const float * __restrict__ y, int64_t ys, const hy_norm p, const uint16_t * __restrict__ router, int width, int n_out, const float * __restrict__ corr, int top, int exact,
+                                                    int32_t * __restrict__ sel, float * __restrict__ selw, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    extern __shared__ __attribute__((aligned(16))) float row[];        // [width] | z
+    __shared__ float red[16];
+    float * const z = row + width;
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (int) (blockDim.x >> 6);
+    hy_u16x8v rw[2 * NV];
+#pragma unroll
+    for (int j = 0; j < 2 * NV; j++) rw[j] = *(const hy_u16x8v *) (router + (int64_t) min(wave, n_out - 1) * width + min(lane * 8 + 512 * j, width - 8));
+    float4 xv[NV], wv[NV], rv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = min(((int) threadIdx.x & 255) * 4 + 1024 * j, width - 4);
+        xv[j] = *(const float4 *) (y + (int64_t) t * ys + i); wv[j] = *(const float4 *) (p.w + i); rv[j] = *(const float4 *) (p.res + (int64_t) t * p.rs + i);
+    }
+    hy_rms_row<NV>(xv, wv, p.w_off, p.eps, width, nullptr, rv, p.mult, red);
+    if (pi_abort_late(gone, abort_w)) return;
+    if (threadIdx.x < 256) {
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int i = (int) threadIdx.x * 4 + 1024 * j;
+            if (i < width) *(float4 *) (row + i) = exact ? xv[j] : make_float4(hy_round(xv[j].x), hy_round(xv[j].y), hy_round(xv[j].z), hy_round(xv[j].w));
+        }
+    }
+    hy_rms_store<NV>(xv, t, t, width, p.eps, p.out, p.os, hy_second{}, rd, red);
+    __syncthreads();
+    for (int e = wave; e < n_out; e += nw) {
+        float a = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2 * NV; j++) {
+            const int i = lane * 8 + 512 * j;
+            if (i >= width) break;
+            const float4 x0 = *(const float4 *) (row + i), x1 = *(const float4 *) (row + i + 4);
+            const float xf[8] = { x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w };
+#pragma unroll
+            for (int k = 0; k < 8; k++) a = fmaf(hy_widen(rw[j][k]), xf[k], a);
+        }
+        if (e + nw < n_out) {
+#pragma unroll
+            for (int j = 0; j < 2 * NV; j++) rw[j] = *(const hy_u16x8v *) (router + (int64_t) (e + nw) * width + min(lane * 8 + 512 * j, width - 8));
+        }
+        a = pi_lanes_sum<64>(a);
+        if (lane == 0) z[e] = a;
+    }
+    __syncthreads();
+    if (wave == 0) moe_choose(z, n_out, corr, top, 0, 0, t, lane, sel, selw);
 }
 
 // up[t][kk][f] = relu(W_up[e] x_t)^2 for the kk-th chosen expert e of token t (nothing for identity experts); a wave per row f.
@@ -2128,6 +2236,27 @@ static int moe_route_launch(const pi_weight * router, const float * correction_d
     PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 2.0 * router->ne0 * router->ne1 + 4.0 * n_tok * router->ne0, k_moe_route, dim3((unsigned) n_tok), dim3((unsigned) (64 * (n_tok <= 64 ? std::min<int64_t>(16, router->ne1) : 4))), (size_t) 8 * router->ne1 + (size_t) 4 * std::max(n_groups, 1), (hipStream_t) stream,
                  (const uint16_t *) router->p0, router->ne0, (int) router->ne1, correction_dev, x, x_stride, top, exact,
                  (int) (router->ne0 % 8 == 0 && ((uintptr_t) router->p0 % 16) == 0 && ((uintptr_t) x % 16) == 0 && x_stride % 4 == 0), n_groups, keep, sel_dev, selw_dev, pi_abort_word());
+    PI_CHECK_LAUNCH(); return 0;
+}
+// pi_op_rms_scale with a residual, and pi_op_moe_route of the result
+extern "C" int pi_op_rms_scale_route(const float * y, int64_t y_stride, const float * w, float w_offset, float eps, const float * residual, int64_t residual_stride, float mult, float * out, int64_t out_stride,
+                                     const pi_weight * router, const float * correction_dev, int n_tok, int top, int exact, int32_t * sel_dev, float * selw_dev, void * stream) {
+    if (n_tok <= 0) return 0;
+    if (!router || router->type != PI_BF16 || top < 1 || top > router->ne1 || router->ne1 > 8192) { pi_set_error("pi_op_rms_scale_route: a bfloat16 router of at most 8192 outputs and 1 <= top <= outputs are required"); return -1; }
+    const int n = (int) router->ne0, n_out = (int) router->ne1;
+    const size_t lds = 4 * ((size_t) n + 2 * n_out + 1);
+    const bool one = residual && n <= 4096 && n % 8 == 0 && n_out <= 4096 && rms_vec(n, { { y, y_stride }, { w, 0 }, { residual, residual_stride }, { out, out_stride }, { router->p0, 0 } });
+    if (!one) {
+        if (pi_op_rms_scale(y, y_stride, w, w_offset, eps, n, n_tok, nullptr, 0, residual, residual_stride, mult, out, out_stride, nullptr, 0, stream) != 0) return -1;
+        return moe_route_launch(router, correction_dev, out, out_stride, n_tok, top, exact, 0, 0, sel_dev, selw_dev, stream);
+    }
+    const hy_norm p = { w, w_offset, eps, residual, residual_stride, mult, out, out_stride, {} };
+    const int waves = n_tok <= 64 ? std::max(4, std::min(16, n_out)) : 4;
+    const pi_round_dst rd = pi_round_asked(0, n);
+#define RR_GO(NV) PI_KT_LAUNCH(PI_KT_OTHER, PI_BF16, 1, 2.0 * n * n_out + 16.0 * n_tok * n, k_rms_route<NV>, dim3((unsigned) n_tok), dim3(64 * waves), lds, (hipStream_t) stream, y, y_stride, p, (const uint16_t *) router->p0, \
+                               n, n_out, correction_dev, top, exact, sel_dev, selw_dev, rd, pi_abort_word())
+    if (n <= 1024) RR_GO(1); else if (n <= 2048) RR_GO(2); else RR_GO(4);
+#undef RR_GO
     PI_CHECK_LAUNCH(); return 0;
 }
 extern "C" int pi_op_moe_route(const pi_weight * router, const float * correction_dev, const float * x, int64_t x_stride, int n_tok, int top, int exact, int32_t * sel_dev, float * selw_dev, void * stream) {
@@ -2290,6 +2419,34 @@ __global__ void __launch_bounds__(256) k_moe_combine(const float * __restrict__ 
     out[(int64_t) t * os + n] = acc;
 }
 
+// The same and the norm behind it, a workgroup per token (the sum stays in registers: 2048 tokens' top-2 rows of 4096 35 us and the norm 17, 27 so; 512 tokens of 2048 6 and 5, 6 so).  What a combination does not
+// need to know - the norm's weights, the residual - leaves ahead of it
+template <int NV>
+__global__ void __launch_bounds__(256) k_moe_combine_norm(const float * __restrict__ dn, int64_t width, int n_exp, int top, const float * x, int64_t xs, const int32_t * __restrict__ sel,
+                                                          const float * __restrict__ selw, const hy_norm p, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    __shared__ float red[4];
+    const int t = blockIdx.x, n = (int) width;
+    float4 acc[NV], wv[NV], rv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        const int i = min((int) threadIdx.x * 4 + 1024 * j, n - 4);
+        wv[j] = *(const float4 *) (p.w + i); rv[j] = *(const float4 *) (p.res + (int64_t) t * p.rs + i);
+        acc[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    for (int kk = 0; kk < top; kk++) {
+        const float g = selw[(int64_t) t * top + kk];
+        const float * from = sel[(int64_t) t * top + kk] >= n_exp ? x + (int64_t) t * xs : dn + ((int64_t) t * top + kk) * width;
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const float4 v = *(const float4 *) (from + min((int) threadIdx.x * 4 + 1024 * j, n - 4));
+            acc[j].x = fmaf(g, v.x, acc[j].x); acc[j].y = fmaf(g, v.y, acc[j].y); acc[j].z = fmaf(g, v.z, acc[j].z); acc[j].w = fmaf(g, v.w, acc[j].w);
+        }
+    }
+    hy_rms_row<NV>(acc, wv, p.w_off, p.eps, n, nullptr, rv, p.mult, red);
+    hy_rms_store<NV>(acc, t, t, n, p.eps, p.out, p.os, p.two, rd, red);
+}
+
 // slots of a tile
 static int moe_tile_len(int n_slots, int n_exp) { return n_slots / n_exp >= 256 ? 128 : 64; }
 // rows of a tile: as for k_dense_tile, the largest that gives every compute unit a workgroup; where none does, two groups of waves share K.  Of 128 slots 256 rows as soon as tiles of 128 rows would be more than a round
@@ -2370,12 +2527,12 @@ extern "C" int pi_op_moe_rounded_ok(const pi_weight * wup, const pi_weight * wdo
     return pi_op_moe_grouped_ok(wup, wdown, n_exp, ff, PI_GLU_OFF, n_tok, top, 0) && wup->ne0 % 64 == 0 && ff % 64 == 0 && wup->ne0 < (1 << 22) && ff < (1 << 22) && (int64_t) n_tok * x_stride < (1ll << 31) && (int64_t) n_tok * top * ff < (1ll << 31);
 }
 // pi_op_moe_experts_grouped from inputs in bfloat16 (xh); x: the same in fp32, what identity experts hand on.  up_dev holds the hidden layer, bfloat16 [n_tok * top][ff]
-extern "C" int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh, int64_t xh_stride, const float * x, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev,
-                                         int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out, int64_t out_stride, void * stream) {
+static int moe_experts_rounded(const char * name, const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh, int64_t xh_stride, const float * x, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev,
+                                         int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out, int64_t out_stride, const hy_norm * norm, void * stream) {
     if (n_tok <= 0) return 0;
-    if (!pi_op_moe_rounded_ok(wup, wdown, n_exp, ff, xh_stride, n_tok, top)) { pi_set_error("pi_op_moe_experts_rounded: this shape takes pi_op_moe_experts or pi_op_moe_experts_grouped"); return -1; }
+    if (!pi_op_moe_rounded_ok(wup, wdown, n_exp, ff, xh_stride, n_tok, top)) { pi_set_error("%s: this shape takes pi_op_moe_experts or pi_op_moe_experts_grouped", name); return -1; }
     if (wup->type != PI_BF16 || wdown->type != PI_BF16 || wup->ne1 != (int64_t) n_exp * ff || wdown->ne0 != ff || wdown->ne1 != (int64_t) n_exp * wup->ne0 || xh_stride % 8 || xh_stride < wup->ne0 || (((uintptr_t) xh | (uintptr_t) up_dev | (uintptr_t) dn_dev) & 15)) {
-        pi_set_error("pi_op_moe_experts_rounded: expert matrices must be bfloat16 [experts * ff][width] and [experts * width][ff], inputs 16-byte aligned rows"); return -1;
+        pi_set_error("%s: expert matrices must be bfloat16 [experts * ff][width] and [experts * width][ff], inputs 16-byte aligned rows", name); return -1;
     }
     hipStream_t s = (hipStream_t) stream;
     const int64_t width = wup->ne0;
@@ -2387,7 +2544,30 @@ extern "C" int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight 
     PI_CHECK_LAUNCH();
     moe_async_launch<false>((const uint16_t *) wdown->p0, ff, (int) width, up_dev, ff, top, idx_dev, mt, tl, est, dn_dev, nullptr, nta, bytes, s);
     PI_CHECK_LAUNCH();
+    if (norm) {
+#define CN_GO(NV) PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 4.0 * n_tok * width * (top + 3), k_moe_combine_norm<NV>, dim3((unsigned) n_tok), dim3(256), 0, s, dn_dev, width, n_exp, top, x, x_stride, sel_dev, selw_dev, *norm, pi_round_asked(0, (int) width), pi_abort_word())
+        if (width <= 1024) CN_GO(1); else if (width <= 2048) CN_GO(2); else CN_GO(4);
+#undef CN_GO
+        PI_CHECK_LAUNCH(); return 0;
+    }
     PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, 4.0 * n_tok * width * (top + 2), k_moe_combine, dim3((unsigned) ((width + 255) / 256), (unsigned) n_tok), dim3(256), 0, s,
                  dn_dev, width, n_exp, top, x, x_stride, sel_dev, selw_dev, out, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
+}
+extern "C" int pi_op_moe_experts_rounded(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh, int64_t xh_stride, const float * x, int64_t x_stride, const int32_t * sel_dev, const float * selw_dev,
+                                         int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * out, int64_t out_stride, void * stream) {
+    return moe_experts_rounded("pi_op_moe_experts_rounded", wup, wdown, n_exp, ff, xh, xh_stride, x, x_stride, sel_dev, selw_dev, n_tok, top, up_dev, dn_dev, idx_dev, out, out_stride, nullptr, stream);
+}
+// the same and pi_op_rms_scale of the result with a residual (w2: pi_op_rms_scale_twice); sum: where the result stands in between, if it has to
+extern "C" int pi_op_moe_experts_rounded_norm(const pi_weight * wup, const pi_weight * wdown, int n_exp, int ff, const uint16_t * xh, int64_t xh_stride, const float * x, int64_t x_stride, const int32_t * sel_dev,
+                                              const float * selw_dev, int n_tok, int top, uint16_t * up_dev, float * dn_dev, int32_t * idx_dev, float * sum, int64_t sum_stride, const float * w, float w_offset, float eps,
+                                              const float * residual, int64_t residual_stride, float mult, float * out, int64_t out_stride, const float * w2, float w2_offset, float * out2, int64_t out2_stride, void * stream) {
+    if (n_tok <= 0 || !wup) return 0;
+    const int n = (int) wup->ne0;
+    const hy_norm norm = { w, w_offset, eps, residual, residual_stride, mult, out, out_stride, { w2, w2_offset, out2, out2_stride } };
+    const bool one = residual && n <= 4096 && rms_vec(n, { { x, x_stride }, { w, 0 }, { residual, residual_stride }, { out, out_stride }, { w2, 0 }, { w2 ? out2 : nullptr, out2_stride } });
+    if (one) return moe_experts_rounded("pi_op_moe_experts_rounded_norm", wup, wdown, n_exp, ff, xh, xh_stride, x, x_stride, sel_dev, selw_dev, n_tok, top, up_dev, dn_dev, idx_dev, nullptr, 0, &norm, stream);
+    if (moe_experts_rounded("pi_op_moe_experts_rounded_norm", wup, wdown, n_exp, ff, xh, xh_stride, x, x_stride, sel_dev, selw_dev, n_tok, top, up_dev, dn_dev, idx_dev, sum, sum_stride, nullptr, stream) != 0) return -1;
+    if (w2) return pi_op_rms_scale_twice(sum, sum_stride, w, w_offset, eps, n, n_tok, residual, residual_stride, mult, out, out_stride, w2, w2_offset, out2, out2_stride, stream);
+    return pi_op_rms_scale(sum, sum_stride, w, w_offset, eps, n, n_tok, nullptr, 0, residual, residual_stride, mult, out, out_stride, nullptr, 0, stream);
 }

@@ -149,6 +149,9 @@ def _declare(lib):
     lib.pi_op_latent_attention.argtypes = [vp, i64, vp, vp, vp, vp, vp, f32, i32, i32, i32, i32, i32, i32, vp, sz, vp, i64, vp, vp]
     lib.pi_op_latent_attention_scratch_floats.argtypes = [i32, i32, i32, i32]; lib.pi_op_latent_attention_scratch_floats.restype = sz
     lib.pi_op_latent_attention_max_cells.argtypes = [i32]
+    lib.pi_op_rms_scale_twice.argtypes = [vp, i64, vp, f32, f32, i32, i32, vp, i64, f32, vp, i64, vp, f32, vp, i64, vp]
+    lib.pi_op_rms_scale_route.argtypes = [vp, i64, vp, f32, f32, vp, i64, f32, vp, i64, vp, vp, i32, i32, i32, vp, vp, vp]
+    lib.pi_op_moe_experts_rounded_norm.argtypes = [vp, vp, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, vp, vp, vp, vp, i64, vp, f32, f32, vp, i64, f32, vp, i64, vp, f32, vp, i64, vp]
     lib.pi_op_moe_route.argtypes = [vp, vp, vp, i64, i32, i32, i32, vp, vp, vp]
     lib.pi_op_moe_experts.argtypes = [vp, vp, i32, i32, vp, i64, vp, vp, i32, i32, i32, vp, vp, i64, vp]
     lib.pi_op_moe_grouped_ok.argtypes = [vp, vp, i32, i32, i32, i32, i32, i32]
