@@ -1,8 +1,11 @@
 // Attention of a prompt: 32 tokens x one head per workgroup, scores and sums on the fp32 matrix cores.
 //
-// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; about 75 reached at 2048 tokens x 32 heads of 128).  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
-// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  Whole calls: 2048 tokens, 32 heads of 128, rank 512: 6.9 ms -> 0.46; 1000 tokens, 16 heads of 192: 1.11 ms -> 0.13;
-// 1000 tokens of 16 differential heads over a window of 256: 526 us -> 74; 333 tokens of 16 heads of 64: 382 us -> 21.
+// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; about 94 reached at 2048 tokens x 32 heads of 128) and the vector instructions, one after the other: while such a
+// product runs, nothing else goes to its SIMD's vector unit, of whichever wave (2048 tokens: 830000 clocks, 530000 of products, 125000 of 240 vector instructions per tile of 16 cells x 32 tokens; with 460 of them 930000;
+// tiles through LDS instead of registers, or the weights between the next tile's products: no less).  So a tile's vector work is kept small: weights relative to a maximum that may lag (below), cells that a token does
+// not see as scores of minus infinity and only where there are some, an exponential for this range alone, no look at single values.  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
+// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  Whole calls: 2048 tokens, 32 heads of 128, rank 512: 6.9 ms -> 0.44; 1000 tokens, 16 heads of 192: 1.11 ms -> 0.12;
+// 1000 tokens of 16 differential heads over a window of 256: 526 us -> 70; 333 tokens of 16 heads of 64: 382 us -> 19.
 //   k_latent_expand   the keys and values of the pass's cells written out once: an fp32 latent in three bfloat16 parts times the bfloat16 matrix on the matrix cores, exact products (dense_tile.h)
 //   k_prompt_attention  a wave owns 32 queries (two operand tiles, so a key is read for both) and every fourth run of 32 cells; no barrier until the four waves' sums meet at the end.  The scores are
 //                     computed transposed (rows = cells): what a lane then holds - four cells of one query - is already the operand of the product with the values, nothing crosses lanes but the maximum.
@@ -62,6 +65,12 @@ static __device__ __forceinline__ uint32_t pa_near(const int32_t * __restrict__ 
     return near;
 }
 
+// e^x of a score below the maximum (or up to e^8): x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
+// errors of expf (rms 2.6e-8, at most 8.3e-8) without its two ends of the range.  Minus infinity: 0 (what the fused part gives below the bound), no number: no number
+static __device__ __forceinline__ float pa_exp(float x) {
+    const float t = fmaxf(x * 1.44269502f, -300.0f), r = rintf(t);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - r) + fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -t))), (int) r);
+}
 static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
@@ -123,6 +132,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         for (int o = 1; o < 16; o <<= 1) first_min = min(first_min, __shfl_xor(first_min, o, 64));
         first_min = __builtin_amdgcn_readfirstlane(first_min);
     }
+    // (a lane's rows from the tile's first on: the first that a tile reads is the scalar unit's)
+    const uint32_t row1 = (uint32_t) A.k1_row * 4u, row2 = (uint32_t) A.k2_row * 4u, rowv = (uint32_t) A.v_row * 4u, lane1 = n * row1 + 16u * g, lane2 = n * row2 + 16u * g, lanev = 4u * g * rowv + 4u * (uint32_t) (NJ * n);
+    // Values that are no numbers are looked for in the sums, behind the walk: where one is not finite, the wave walks again with a look at every value
+    for (int careful = 0; ; careful = 1) {
     unsigned long long todo = 0;
     for (int c0 = start; c0 < c_end; c0 += 32 * PARTS) {
         if (far) {
@@ -159,10 +172,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
             for (int u = 0; u < 2; u++) { near[u] |= __shfl_xor(near[u], 16, 64); near[u] |= __shfl_xor(near[u], 32, 64); vis[u] &= near[u]; }
         }
-        uint32_t some = vis[0] | vis[1];                              // the cells that any of the tokens sees; what the others hold is not read
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) some |= __shfl_xor(some, o, 64);
-        some = (uint32_t) __builtin_amdgcn_readfirstlane((int) some);
+        int any = (int) (vis[0] | vis[1]);                            // the cells that any of the tokens sees; what the others hold is not read
+        pi_butterfly<8>([&](auto o) { any |= pi_partner<decltype(o)::value>(any); });
+        const uint32_t some = (uint32_t) __builtin_amdgcn_readfirstlane(any);
+        const bool whole0 = __all(((vis[0] & vis[1]) & 0xffffu) == 0xffffu), whole1 = __all((vis[0] & vis[1]) >> 16 == 0xffffu);
 #pragma unroll 1
         for (int half = 0; half < 2; half++) {
             const uint32_t here = (some >> (16 * half)) & 0xffffu;
@@ -171,7 +184,8 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             const int ck = cb + (here >> n & 1u ? n : spare);
             pa_f32x4 kf[NK], vf[4][NV];
             if constexpr (N1 > 0) {
-                const uint32_t o1 = ((uint32_t) (ck - A.cell0) * (uint32_t) A.k1_row + 4u * g) * 4u, o2 = ((uint32_t) ck * (uint32_t) A.k2_row + 4u * g) * 4u;
+                const bool own = here >> n & 1u;
+                const uint32_t o1 = (uint32_t) (cb - A.cell0) * row1 + (own ? lane1 : spare * row1 + 16u * g), o2 = N1 < NK ? (uint32_t) cb * row2 + (own ? lane2 : spare * row2 + 16u * g) : 0u;
 #pragma unroll
                 for (int i = 0; i < NK; i++) kf[i] = i < N1 ? *(const pa_f32x4 *) ((const char *) k1 + o1 + 64 * i) : *(const pa_f32x4 *) ((const char *) A.k2 + o2 + 64 * (i - N1));
             } else {
@@ -185,13 +199,12 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             auto values = [&]() {
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    const int cell = cb + (here >> (4 * g + c) & 1u ? 4 * g + c : spare) - A.cell0;
                     if constexpr (N1 > 0) {
-                        const uint32_t o = ((uint32_t) cell * (uint32_t) A.v_row + (uint32_t) (NJ * n)) * 4u;
+                        const uint32_t o = (uint32_t) (cb - A.cell0) * rowv + (here >> (4 * g) & (1u << c) ? lanev + c * rowv : spare * rowv + 4u * (uint32_t) (NJ * n));
 #pragma unroll
                         for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) ((const char *) vb + o + 16 * j);
                     } else {
-                        const float * vr = vb + (int64_t) cell * A.v_row;
+                        const float * vr = vb + (int64_t) (cb + (here >> (4 * g + c) & 1u ? 4 * g + c : spare) - A.cell0) * A.v_row;
 #pragma unroll
                         for (int j = 0; j < NV; j++) vf[c][j] = *(const pa_f32x4 *) (vr + min(NJ * n + 4 * j, vdim - 4));
                     }
@@ -206,50 +219,75 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
                 for (int c = 0; c < 4; c++) { s[0] = pa_mfma(kf[i][c], q[0][i][c], s[0]); s[1] = pa_mfma(kf[i][c], q[1][i][c], s[1]); }
             if constexpr (LATE) { __builtin_amdgcn_sched_barrier(0); values(); }
+            // Scores to weights (whole: every token sees every cell; else a cell that a token does not see scores minus infinity).  The maximum that a query's weights are relative to follows the scores' only when these pass
+            // it by 8 (weights up to e^8 are as good in fp32): of 128 tiles of a wave some 75 hold a new maximum of one of its 32 queries, and each of them cost all the sums their factor
 #pragma unroll
             for (int u = 0; u < 2; u++) {
-                const uint32_t mine = vis[u] >> (16 * half + 4 * g);
-                float top = -INFINITY;
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    float x = s[u][c] * A.scale + bias;
-                    if (soft && A.softcap > 0.0f) x = A.softcap * tanhf(x / A.softcap);
-                    s[u][c] = x;
-                    if (mine >> c & 1u) top = fmaxf(top, x);
+                for (int c = 0; c < 4; c++) s[u][c] = fmaf(s[u][c], A.scale, bias);
+                if (soft && A.softcap > 0.0f) {
+#pragma unroll
+                    for (int c = 0; c < 4; c++) s[u][c] = A.softcap * tanhf(s[u][c] / A.softcap);
+                }
+                if (!(half ? whole1 : whole0)) {
+                    const uint32_t mine = vis[u] >> (16 * half + 4 * g);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) s[u][c] = mine >> c & 1u ? s[u][c] : -INFINITY;
                 }
                 if (soft) {
-                    top = fmaxf(top, __shfl_xor(top, 16, 64)); top = fmaxf(top, __shfl_xor(top, 32, 64));
-                    const float m_new = fmaxf(m_run[u], top);
-                    const float f = m_run[u] == m_new ? 1.0f : expf(m_run[u] - m_new);            // (nothing seen yet: expf(-inf) = 0, or both -inf)
-                    const float from = m_new == -INFINITY ? 0.0f : m_new;                         // (scores of minus infinity alone: no weight, not a NaN)
-                    float sum = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < 4; c++) { const float e = mine >> c & 1u ? expf(s[u][c] - from) : 0.0f; s[u][c] = e; sum += e; }
-                    l_run[u] = fmaf(l_run[u], f, sum); m_run[u] = m_new;                          // (a lane's own cells; the four of a query meet at the end)
-                    if (__any(f != 1.0f))
+                    float top = fmaxf(fmaxf(s[u][0], s[u][1]), fmaxf(s[u][2], s[u][3]));
+                    top = fmaxf(top, pi_partner<16>(top)); top = fmaxf(top, pi_partner<32>(top));
+                    if (__any(top > m_run[u] + 8.0f)) {
+                        const float m_new = top > m_run[u] + 8.0f ? top : m_run[u];
+                        const float f = m_run[u] == m_new ? 1.0f : expf(m_run[u] - m_new);    // (nothing seen yet: expf(-inf) = 0)
+                        l_run[u] *= f; m_run[u] = m_new;
 #pragma unroll
                         for (int j = 0; j < NJ; j++) acc[u][j] *= f;
+                    }
+                    const float from = m_run[u] == -INFINITY ? 0.0f : m_run[u];               // (scores of minus infinity alone: no weight, not a NaN)
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) { const float e = pa_exp(s[u][c] - from); s[u][c] = e; sum += e; }
+                    l_run[u] += sum;                                                          // (a lane's own cells; the four of a query meet at the end)
                 } else
 #pragma unroll
-                    for (int c = 0; c < 4; c++) s[u][c] = mine >> c & 1u ? 1.0f / (1.0f + expf(-s[u][c])) : 0.0f;
+                    for (int c = 0; c < 4; c++) s[u][c] = 1.0f / (1.0f + expf(-s[u][c]));
             }
-            uint32_t big = 0;                                         // an infinity or a NaN among the values must not meet the zero weight of a token that does not see it: it joins at the end
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int j = 0; j < NJ; j++) big = max(big, __float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu);
-            if (__any(big >= 0x7f800000u)) {
-                odd = 1;
+            if (careful) {                                            // an infinity or a NaN among the values must not meet the zero weight of a token that does not see it: it joins at the end
+                uint32_t big = 0;
 #pragma unroll
                 for (int c = 0; c < 4; c++)
 #pragma unroll
-                    for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[c][j >> 2][j & 3] = 0.0f;
+                    for (int j = 0; j < NJ; j++) big = max(big, __float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu);
+                if (__any(big >= 0x7f800000u)) {
+                    odd = 1;
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) if ((__float_as_uint(vf[c][j >> 2][j & 3]) & 0x7fffffffu) >= 0x7f800000u) vf[c][j >> 2][j & 3] = 0.0f;
+                }
             }
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
                 for (int j = 0; j < NJ; j++) { acc[0][j] = pa_mfma(vf[c][j >> 2][j & 3], s[0][c], acc[0][j]); acc[1][j] = pa_mfma(vf[c][j >> 2][j & 3], s[1][c], acc[1][j]); }
         }
+    }
+    if (careful) break;
+    uint32_t big = 0;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) big = max(big, __float_as_uint(acc[u][j][c]) & 0x7fffffffu);
+    if (!__any(big >= 0x7f800000u)) break;
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        m_run[u] = -INFINITY; l_run[u] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[u][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
+    }
     }
 #pragma unroll
     for (int u = 0; u < 2; u++) {

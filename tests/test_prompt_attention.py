@@ -282,3 +282,28 @@ def test_scores_of_minus_infinity(T, n_kv, maps):
     args[1] = pos[:T - 1]
     want = diff_attention_ref(q[:T - 1], kc[near], vc[near], cpos[near], *args)
     assert rel_rms(got[:T - 1], want) < 1e-5 and np.all(got[T - 1] == 0.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("step", [0.4, 3.0, -3.0, 30.0])
+@pytest.mark.parametrize("D,V,maps", [(64, 64, 1), (64, 128, 2), (36, 68, 1)])
+def test_scores_that_climb_and_fall(step, D, V, maps):
+    """scores that rise or fall from cell to cell, by less and by more than the maximum may lag, in tiles that all tokens see and tiles that some see; a value that is no number where nobody sees it and where two tokens do"""
+    U, lib = gpu()
+    H, G, T, n_kv = 4, 2, 70, 400
+    rng = np.random.default_rng(D + V)
+    q = np.zeros((T, H, maps, D), np.float32)
+    q[..., 0], q[..., 1:] = 1.0, rng.standard_normal((T, H, maps, D - 1)) * 0.1
+    kc, vc = rng.standard_normal((n_kv, G, maps, D)).astype(np.float32), rng.standard_normal((n_kv, G, V)).astype(np.float32)
+    kc[..., 0] = (step * np.arange(n_kv) / 16)[:, None, None]
+    vis = np.arange(n_kv)[None, :] <= np.arange(n_kv - T, n_kv)[:, None]
+    vis[:, 100] = False
+    vis[40:, 200] = False
+    args = [np.arange(n_kv, dtype=np.int32), vis, np.arange(n_kv - T, n_kv, dtype=np.int32), 1.0, 0, 0, maps, 0.45, 0.7, 1e-3, H, G]
+    want = diff_attention_ref(q, kc, vc, *args)
+    # a score of size s is a sum of D fp32 terms, each rounded to s 2^-24 at worst: the exponent of its weight is off by some s 2^-24 sqrt(D)
+    bound = max(1e-5, abs(step) * n_kv / 16 * 2.0 ** -24 * D ** 0.5)
+    assert rel_rms(run_diff(U, lib, q, kc, vc, *args, True), want) < bound
+    vc[100], vc[200, 0, 5] = np.nan, np.inf                               # (seen by none; seen by the first forty, in one value of the first key head)
+    got = run_diff(U, lib, q, kc, vc, *args, True)
+    assert rel_rms(got[40:], want[40:]) < bound and np.isfinite(got[:, H // G:]).all() and not np.isfinite(got[:40, :H // G]).all()
