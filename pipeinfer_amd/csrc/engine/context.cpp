@@ -213,7 +213,12 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
         if (hipStreamCreateWithFlags(&ctx->ctl_stream, hipStreamNonBlocking) != hipSuccess) { err = "hipStreamCreate(control) failed"; return false; }
     }
     ctx->use_graphs = ctx->use_graphs && getenv("PI_NO_GRAPHS") == nullptr;
-    if (pi_op_latent_attention_reserve() != 0 || (hp.n_recurrent() > 0 && (pi_op_linear_attention_reserve() != 0 || pi_op_channel_recurrence_reserve() != 0))) { err = pi_last_error(); return false; }
+    bool linear = false, channels = false;                                     // (an attribute of every instance of a kernel: not of those that no layer launches)
+    for (const pi_hybrid_layer & H : hp.hybrid) {
+        linear |= H.mixer == PI_MIXER_LIGHTNING || H.mixer == PI_MIXER_MEMORY || H.mixer == PI_MIXER_PARALLEL;
+        channels |= H.mixer == PI_MIXER_CHANNEL_DELTA || H.mixer == PI_MIXER_PARALLEL_SHIFT;
+    }
+    if (pi_op_latent_attention_reserve() != 0 || (linear && pi_op_linear_attention_reserve() != 0) || (channels && pi_op_channel_recurrence_reserve() != 0)) { err = pi_last_error(); return false; }
     ctx->mask_cap_words = (size_t) nb * ((ctx->n_ctx + 31) / 32);
     if (!(ctx->mask_dev = (uint32_t *) dev(ctx->mask_cap_words * 4))) return false;
     for (auto & kv : ctx->window_masks) if (!(kv.second = (uint32_t *) dev(ctx->mask_cap_words * 4))) return false;

@@ -376,6 +376,34 @@ def test_causal_conv_over_sequences_and_passes(taps, channels, fused):
         assert np.array_equal(st[2], state[2])                      # a slot nobody named is untouched
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_causal_conv_of_long_passes(taps):
+    """runs of tokens: sequences that start, go on and end anywhere in a run of sixteen, shorter than the taps and longer than a run, one that starts from nothing and one with a state, a last run that is not full"""
+    U, lib = gpu()
+    channels, slots, T = 5000, 6, 187
+    rng = np.random.default_rng(taps)
+    w, state = rng.standard_normal((channels, taps)).astype(np.float32), rng.standard_normal((slots, taps - 1, channels)).astype(np.float32)
+    rec = [0] * 15 + [1 | F] + [2] * 2 + [3 | F] + [3] * 60 + [4] * 47
+    rec += [5 | F] + [5] * (T - len(rec) - 1)
+    x = rng.standard_normal((T, channels)).astype(np.float32)
+    outs = []
+    for cut in (T, 100):                                                     # in one pass, and in two with the state between them
+        wd, sd, got = U.Dev(w), U.Dev(state), []
+        for a, b in ((0, cut), (cut, T)):
+            if a < b:
+                xd, rd, od = U.Dev(x[a:b]), U.Dev(np.array(rec[a:b], np.int32)), U.Dev(nbytes=4 * (b - a) * channels)
+                L.check(lib.pi_op_causal_conv(xd.ptr, channels, channels, taps, wd.ptr, None, sd.ptr, rd.ptr, b - a, SILU, od.ptr, channels, None))
+                got.append(od.get(np.float32, (b - a, channels)))
+        outs.append((np.concatenate(got), sd.get(np.float32, state.shape)))
+    tails = {s: [state[s, i].astype(np.float64) for i in range(taps - 1)] for s in range(slots)}
+    want = conv_ref(x.astype(np.float64), w.astype(np.float64), np.zeros(channels), tails, rec, taps)
+    for got, left in outs:
+        assert rel_rms(got, want) < 2e-6
+        for s in range(slots):
+            assert rel_rms(left[s], np.stack(tails[s])) < 1e-6
+
+
 def ssd_ref(C_, B, x, dt, decay, D, S, heads, groups):
     out = np.zeros_like(x)
     for t in range(x.shape[0]):
