@@ -207,6 +207,10 @@ PI_API int pi_op_copy_f32(const float * src_dev, float * dst_dev, int64_t n, voi
 PI_API int pi_op_latent_attention(const float * q_dev, int64_t q_stride, const float * cache_dev, const uint32_t * mask_dev, const pi_weight * w_uk, const pi_weight * w_uv, const float * sink_dev,
                                   float scale, int heads, int dim, int vdim, int rank, int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out_dev, int64_t out_stride,
                                   const int32_t * dyn_dev, void * stream);
+/* the tokens' own latents kv (rows of `rank` values), normed (pi_op_rms_scale, eps) into their cells of the cache first */
+PI_API int pi_op_latent_attention_tokens(const float * kv_dev, int64_t kv_stride, const float * kv_norm_dev, float eps, const float * q_dev, int64_t q_stride, float * cache_dev, const uint32_t * mask_dev, const pi_weight * w_uk,
+                                         const pi_weight * w_uv, const float * sink_dev, float scale, int heads, int dim, int vdim, int rank, int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out_dev,
+                                         int64_t out_stride, const int32_t * dyn_dev, void * stream);
 PI_API size_t pi_op_latent_attention_scratch_floats(int heads, int rank, int n_tok, int n_kv);
 PI_API int pi_op_latent_attention_reserve(void);                   /* once per process, outside graph capture: LDS limit of the score kernels */
 PI_API int pi_op_latent_attention_max_cells(int rank);             /* longest context the kernels serve */

@@ -921,9 +921,10 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         if (H.mixer == PI_MIXER_LATENT_ATTENTION) {
             float * cache = ctx->lat_cache + ctx->lat_off[il];
             OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_NONE, pw, PI_ACT_NONE, s, xh, width));                                    // q | W_dkv h
-            OP_OK(pi_op_rms_scale(P + hd, pw, W.mix_norm, 0.0f, eps, H.kv_rank, n_tok, nullptr, 0, nullptr, 0, 1.0f, cache, H.kv_rank, ctx->dyn_dev, 1, s));   // the latent, into its cell
-            OP_OK(op_rounded(ctx, ah, A, hv, 0, hv, n_tok, true, s, [&] { return pi_op_latent_attention(P, pw, cache, ctx->mask_dev, W.w_uk, W.w_uv, W.sink, H.scale, H.heads, H.dim, H.vdim, H.kv_rank, n_tok, n_kv, ctx->lat_scratch,
-                                                                                                        ctx->lat_scratch_floats, A, hv, ctx->dyn_dev, s); }));
+            OP_OK(op_rounded(ctx, ah, A, hv, 0, hv, n_tok, true, s, [&] {                                                                       // (the latent into its cell, then the attention)
+                return pi_op_latent_attention_tokens(P + hd, pw, W.mix_norm, eps, P, pw, cache, ctx->mask_dev, W.w_uk, W.w_uv, W.sink, H.scale, H.heads, H.dim, H.vdim, H.kv_rank, n_tok, n_kv, ctx->lat_scratch,
+                                                     ctx->lat_scratch_floats, A, hv, ctx->dyn_dev, s);
+            }));
         } else {
             float * state = ctx->rec_state + ctx->rec_off[il];
             OP_OK(dense(ctx, W.w_in, x, width, n_tok, P, pw, PI_ACT_SILU, 2 * hd + hv, PI_ACT_SIGMOID, s, xh, width));                        // silu(q | k | v) | sigmoid(g)

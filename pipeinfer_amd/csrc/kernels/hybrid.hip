@@ -1389,12 +1389,39 @@ static bool lat_rows_takes(int heads, int rank, int rot, int n_tok, int n_ctx) {
                                                                                                  (n_ctx >= 64 || (int64_t) n_tok * heads * rank <= 384 * 512)));
 }
 
-// grid (token tile of 4, head, 64 values of the rank, then 64 values of the rotated part): lane = one rank value, the four waves take a quarter of the head's dim each and meet in LDS.  A query head is
+// the tokens' own latents on their way to their cells: a norm of rows of `rank` values (256 or 512), of no rows where w is null
+struct lat_kv { const float * x; int64_t xs; const float * w; float eps; float * cache; };
+// grid (token tile of 4, head, 64 values of the rank, then 64 values of the rotated part, then the tokens' latents): lane = one rank value, the four waves take a quarter of the head's dim each and meet in LDS.  A query head is
 // [dim values | rot values]; the last are turned in pairs by the token's position (cs: the rotation table) and go behind the rank values
 __global__ void __launch_bounds__(256) k_latent_absorb(const float * __restrict__ q, int64_t qs, const uint16_t * __restrict__ wuk, float scale, int heads, int dim, int rank, int rot, const float2 * __restrict__ cs, int n_pos,
-                                                       int pairing, const int32_t * __restrict__ pos, int n_tok, float * __restrict__ qa, const int32_t * __restrict__ dyn, int live_min, const int32_t * __restrict__ abort_w) {
+                                                       int pairing, const int32_t * __restrict__ pos, int n_tok, float * __restrict__ qa, const int32_t * __restrict__ dyn, int live_min, const lat_kv kv, const int32_t * __restrict__ abort_w) {
     if (live_min > 0 && dyn[1] <= live_min) return;                    // (a pass that prompt_attention.hip takes: latent_tiles_to)
     const int gone = pi_abort_peek(abort_w);
+    if (kv.w && blockIdx.z == gridDim.z - 1) {                         // wave = token; the bits of k_rms_scale_once, whose waves sum 256 values each
+        const int t = blockIdx.x * 4 + (threadIdx.x >> 6), i = (threadIdx.x & 63) * 4;
+        if (blockIdx.y != 0 || t >= n_tok) return;
+        const float * x = kv.x + (int64_t) t * kv.xs;
+        const int64_t cell = pi_cell_of(dyn, 0, t);
+        float4 v[2], w[2];
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2; j++) { const int at = min(i + 256 * j, rank - 4); v[j] = *(const float4 *) (x + at); w[j] = *(const float4 *) (kv.w + at); }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if (256 * j >= rank) break;
+            float a = fmaf(v[j].x, v[j].x, 0.0f);
+            a = fmaf(v[j].y, v[j].y, a); a = fmaf(v[j].z, v[j].z, a); a = fmaf(v[j].w, v[j].w, a);
+            ss += pi_lanes_sum<64>(a);
+        }
+        const float inv = 1.0f / sqrtf(ss / (float) rank + kv.eps);
+        if (pi_abort_late(gone, abort_w, 5)) return;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            if (256 * j >= rank) break;
+            *(float4 *) (kv.cache + cell * rank + i + 256 * j) = make_float4(v[j].x * inv * (w[j].x + 0.0f), v[j].y * inv * (w[j].y + 0.0f), v[j].z * inv * (w[j].z + 0.0f), v[j].w * inv * (w[j].w + 0.0f));
+        }
+        return;
+    }
     __shared__ float part[4][4][64];
     extern __shared__ float4 qsh[];                                    // [dim]: the head's query values of the four tokens, side by side
     const int t0 = blockIdx.x * 4, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.z * 64 + lane;
@@ -1980,9 +2007,9 @@ static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int
     }
     return to;
 }
-extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev, const float * gate_dev,
+static int latent_attention(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev, const float * gate_dev,
                                             int64_t gate_stride, int gate_act, int gate_width, float scale, int heads, int dim, int rot, int vdim, int rank, const void * rotary_table, int pairing, const int32_t * pos_dev,
-                                            int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride, const int32_t * dyn_dev, void * stream) {
+                                            int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride, const int32_t * dyn_dev, const lat_kv & tokens, void * stream) {
     if (n_tok <= 0) return 0;
     const float2 * cs = nullptr; int n_pos = 0, half = 0;
     if (rot < 0 || (rot & 1)) { pi_set_error("pi_op_latent_attention: %d rotated dimensions (an even number)", rot); return -1; }
@@ -2016,12 +2043,18 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     const bool whole = lat_rows_takes(heads, rank, rot, n_tok, n_kv) && (n_tok * heads >= 8 || n_kv < 4096) && lat_rows_floats(heads, rank, rot, n_tok, n_kv) <= scratch_floats &&
                        (((uintptr_t) cache | (uintptr_t) scratch_dev) & 15) == 0 && (int64_t) n_kv * (rank + rot) < (1ll << 30);
     int live_min = 0;                                                  // the launches below are for passes of more live cells
+    // the tokens' latents, normed on their way: beside the queries where those kernels follow, which read nothing of the cells' (us a step's layer less: 5), else ahead of everything
+    lat_kv kv = tokens;
+    if (kv.w && (!whole || rot > 0 || ((uintptr_t) kv.x & 15) || kv.xs % 4 || ((uintptr_t) kv.w & 15))) {
+        if (pi_op_rms_scale(kv.x, kv.xs, kv.w, 0.0f, kv.eps, rank, n_tok, nullptr, 0, nullptr, 0, 1.0f, kv.cache, rank + rot, dyn_dev, 1, stream) != 0) return -1;
+        kv.w = nullptr;
+    }
     if (!whole && (live_min = latent_prompt(a, p, cache, rank, wuk, wuv, scratch_dev, scratch_floats, 4.0 * acct * heads * (double) (dim + vdim) + 4.0 * n_tok * heads * (double) (dim + rot + vdim), s)) > 0) {
         PI_CHECK_LAUNCH();
         if (live_min >= n_kv) return 0;
     }
-    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * dim + 4.0 * n_tok * heads * (dim + rank + 2.0 * rot), k_latent_absorb, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((rank + 63) / 64 + (rot + 63) / 64)), dim3(256), (size_t) 16 * dim, s,
-                 q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, dyn_dev, live_min, pi_abort_word());
+    PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * dim + 4.0 * n_tok * heads * (dim + rank + 2.0 * rot), k_latent_absorb, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((rank + 63) / 64 + (rot + 63) / 64 + (kv.w ? 1 : 0))), dim3(256), (size_t) 16 * dim, s,
+                 q, q_stride, (const uint16_t *) wuk->p0, scale, heads, dim, rank, rot, cs, n_pos, pairing, pos_dev, n_tok, qa, dyn_dev, live_min, kv, pi_abort_word());
     PI_CHECK_LAUNCH();
     const double bytes = 4.0 * acct * (rank + rot) + 4.0 * n_tok * heads * (rank + rot + (double) rank * p.S);
     // most rows and more shares of the splits than the 256 MB of the last cache: the kernels per token (32 tokens of 16 heads, rank 512 + 64, us here / per token: 6000 cells 327 / 482, 9000 611 / 510, 16000 1029 / 968; of
@@ -2061,6 +2094,20 @@ extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, c
     return combine(p.S, false);
 #undef LAT_COMBINE
     PI_CHECK_LAUNCH(); return 0;
+}
+extern "C" int pi_op_latent_attention_gated(const float * q, int64_t q_stride, const float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv, const float * sink_dev, const float * gate_dev,
+                                            int64_t gate_stride, int gate_act, int gate_width, float scale, int heads, int dim, int rot, int vdim, int rank, const void * rotary_table, int pairing, const int32_t * pos_dev,
+                                            int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride, const int32_t * dyn_dev, void * stream) {
+    return latent_attention(q, q_stride, cache, mask, wuk, wuv, sink_dev, gate_dev, gate_stride, gate_act, gate_width, scale, heads, dim, rot, vdim, rank, rotary_table, pairing, pos_dev, n_tok, n_kv, scratch_dev, scratch_floats, out,
+                            out_stride, dyn_dev, {}, stream);
+}
+// pi_op_rms_scale of the tokens' latents into their cells, and pi_op_latent_attention
+extern "C" int pi_op_latent_attention_tokens(const float * kv, int64_t kv_stride, const float * kv_norm, float eps, const float * q, int64_t q_stride, float * cache, const uint32_t * mask, const pi_weight * wuk, const pi_weight * wuv,
+                                             const float * sink_dev, float scale, int heads, int dim, int vdim, int rank, int n_tok, int n_kv, float * scratch_dev, size_t scratch_floats, float * out, int64_t out_stride,
+                                             const int32_t * dyn_dev, void * stream) {
+    if (!sink_dev || !kv || !kv_norm || !dyn_dev) { pi_set_error("pi_op_latent_attention_tokens: the latents, their norm, the sink and the cell table are required"); return -1; }
+    return latent_attention(q, q_stride, cache, mask, wuk, wuv, sink_dev, nullptr, 0, PI_ACT_NONE, 1, scale, heads, dim, 0, vdim, rank, nullptr, PI_PAIR_HALVES, nullptr, n_tok, n_kv, scratch_dev, scratch_floats, out, out_stride, dyn_dev,
+                            { kv, kv_stride, kv_norm, eps, cache }, stream);
 }
 
 // ---- routed feed-forward ------------------------------------------------------------------------------------------------------------------------------

@@ -152,6 +152,7 @@ def _declare(lib):
     lib.pi_op_rms_scale_twice.argtypes = [vp, i64, vp, f32, f32, i32, i32, vp, i64, f32, vp, i64, vp, f32, vp, i64, vp]
     lib.pi_op_rms_scale_route.argtypes = [vp, i64, vp, f32, f32, vp, i64, f32, vp, i64, vp, vp, i32, i32, i32, vp, vp, vp]
     lib.pi_op_moe_experts_rounded_norm.argtypes = [vp, vp, i32, i32, vp, i64, vp, i64, vp, vp, i32, i32, vp, vp, vp, vp, i64, vp, f32, f32, vp, i64, f32, vp, i64, vp, f32, vp, i64, vp]
+    lib.pi_op_latent_attention_tokens.argtypes = [vp, i64, vp, f32, vp, i64, vp, vp, vp, vp, vp, f32, i32, i32, i32, i32, i32, i32, vp, C.c_size_t, vp, i64, vp, vp]
     lib.pi_op_moe_route.argtypes = [vp, vp, vp, i64, i32, i32, i32, vp, vp, vp]
     lib.pi_op_moe_experts.argtypes = [vp, vp, i32, i32, vp, i64, vp, vp, i32, i32, i32, vp, vp, i64, vp]
     lib.pi_op_moe_grouped_ok.argtypes = [vp, vp, i32, i32, i32, i32, i32, i32]

@@ -96,3 +96,29 @@ def test_experts_of_a_prompt_and_the_norms_behind_them(lib, width, T, second, pa
         got.append([xs.get()] + ([o2.get()] if second else []))
     for one, other in zip(*got):
         assert np.array_equal(one, other)
+
+
+@pytest.mark.parametrize("rank,T,n_kv,pad", [(256, 1, 40, 0), (512, 1, 700, 4), (512, 7, 96, 0), (256, 30, 100, 0), (256, 5, 64, 1), (64, 3, 50, 0), (512, 200, 200, 0), (1024, 2, 33, 0)])
+def test_latents_into_their_cells_and_the_attention_over_them(lib, rank, T, n_kv, pad):
+    rng = np.random.default_rng(rank + T)
+    H, D, V = 4, 32, 64
+    w_uk, w_uv = upload(lib, rng.standard_normal((H * D, rank)) * rank ** -0.5), upload(lib, rng.standard_normal((H * V, rank)) * rank ** -0.5)
+    row = H * D + rank + pad
+    p, w, sink = U.Dev(rng.standard_normal((T, row)).astype(np.float32)), Rows(rng.standard_normal((1, rank))), U.Dev(rng.standard_normal(H).astype(np.float32))
+    old, vis = rng.standard_normal((n_kv, rank)).astype(np.float32), np.arange(n_kv)[None, :] <= np.arange(n_kv - T, n_kv)[:, None]
+    mask = U.Dev(np.packbits(np.pad(vis, ((0, 0), (0, -n_kv % 32))), axis=1, bitorder="little").view(np.uint32))
+    dyn = U.Dev(np.array([n_kv - T, n_kv, T, 0], np.int32))
+    n_scr = lib.pi_op_latent_attention_scratch_floats(H, rank, T, n_kv)
+    got = []
+    for fused in (False, True):
+        cache, scr, out = U.Dev(old), U.Dev(nbytes=4 * n_scr), U.Dev(nbytes=4 * T * H * V)
+        latents = p.ptr + 4 * H * D
+        tail = (mask.ptr, w_uk, w_uv, sink.ptr, D ** -0.5, H, D, V, rank, T, n_kv, scr.ptr, n_scr, out.ptr, H * V, dyn.ptr, None)
+        if fused:
+            L.check(lib.pi_op_latent_attention_tokens(latents, row, w.ptr, 1e-6, p.ptr, row, cache.ptr, *tail))
+        else:
+            L.check(lib.pi_op_rms_scale(latents, row, w.ptr, 0.0, 1e-6, rank, T, None, 0, None, 0, 1.0, cache.ptr, rank, dyn.ptr, 1, None))
+            L.check(lib.pi_op_latent_attention(p.ptr, row, cache.ptr, *tail))
+        got.append([cache.get(np.uint32, old.shape), out.get(np.uint32, (T, H * V))])
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert np.array_equal(got[1][0][:n_kv - T], old.view(np.uint32)[:n_kv - T])
