@@ -67,9 +67,10 @@ static __device__ __forceinline__ float hy_block_max(float v, float * red) {
 
 // ---- RMS norm with its usual companions ---------------------------------------------------------------------------------------------------------
 // A row of up to 1024 NV values in the registers of 256 threads (thread i: values 4 i .. of every 1024): its norm, gate, multiplier and residual, in place.  Further threads of the workgroup only take part in the sum
-// (as zeros: a row's bits do not depend on their number).  red: a float for each wave
+// (as zeros: a row's bits do not depend on their number).  red: a float for each wave.  gv, rv: looked at where gated and added say so (arrays and not pointers that may be null: behind a choice between a pointer and null
+// the arrays went to scratch memory, 48 / 80 / 144 bytes a lane)
 template <int NV>
-static __device__ __forceinline__ void hy_rms_row(float4 (&xv)[NV], const float4 (&wv)[NV], float w_off, float eps, int n, const float4 * gv, const float4 * rv, float mult, float * red) {
+static __device__ __forceinline__ void hy_rms_row(float4 (&xv)[NV], const float4 (&wv)[NV], float w_off, float eps, int n, bool gated, const float4 (&gv)[NV], bool added, const float4 (&rv)[NV], float mult, float * red) {
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < NV; j++) if (threadIdx.x < 256 && (int) threadIdx.x * 4 + 1024 * j < n) { ss = fmaf(xv[j].x, xv[j].x, ss); ss = fmaf(xv[j].y, xv[j].y, ss); ss = fmaf(xv[j].z, xv[j].z, ss); ss = fmaf(xv[j].w, xv[j].w, ss); }
@@ -78,10 +79,10 @@ static __device__ __forceinline__ void hy_rms_row(float4 (&xv)[NV], const float4
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         float y[4] = { xv[j].x * inv * (wv[j].x + w_off), xv[j].y * inv * (wv[j].y + w_off), xv[j].z * inv * (wv[j].z + w_off), xv[j].w * inv * (wv[j].w + w_off) };
-        if (gv) { y[0] *= gv[j].x; y[1] *= gv[j].y; y[2] *= gv[j].z; y[3] *= gv[j].w; }
+        if (gated) { y[0] *= gv[j].x; y[1] *= gv[j].y; y[2] *= gv[j].z; y[3] *= gv[j].w; }
 #pragma unroll
         for (int k = 0; k < 4; k++) y[k] *= mult;
-        if (rv) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
+        if (added) { y[0] = rv[j].x + y[0]; y[1] = rv[j].y + y[1]; y[2] = rv[j].z + y[2]; y[3] = rv[j].w + y[3]; }
         xv[j] = make_float4(y[0], y[1], y[2], y[3]);
     }
 }
@@ -101,7 +102,7 @@ static __device__ __forceinline__ void hy_rms_store(float4 (&xv)[NV], int t, int
     float4 wv[NV];
 #pragma unroll
     for (int j = 0; j < NV; j++) wv[j] = *(const float4 *) (two.w + min((int) threadIdx.x * 4 + 1024 * j, n - 4));
-    hy_rms_row<NV>(xv, wv, two.w_off, eps, n, nullptr, nullptr, 1.0f, red);
+    hy_rms_row<NV>(xv, wv, two.w_off, eps, n, false, wv, false, wv, 1.0f, red);
 #pragma unroll
     for (int j = 0; j < NV; j++) {
         const int i = (int) threadIdx.x * 4 + 1024 * j;
@@ -127,7 +128,7 @@ __global__ void __launch_bounds__(256) k_rms_scale_once(const float * __restrict
         if (gate) gv[j] = *(const float4 *) (gate + (int64_t) t * gs + i);
         if (res) rv[j] = *(const float4 *) (res + (int64_t) t * rs + i);
     }
-    hy_rms_row<NV>(xv, wv, w_off, eps, n, gate ? gv : nullptr, res ? rv : nullptr, mult, red);
+    hy_rms_row<NV>(xv, wv, w_off, eps, n, gate != nullptr, gv, res != nullptr, rv, mult, red);
     if (pi_abort_late(gone, abort_w)) return;
     hy_rms_store<NV>(xv, t, orow, n, eps, out, os, two, rd, red);
 }
@@ -2200,7 +2201,7 @@ __global__ void __launch_bounds__(1024) k_rms_route(const float * __restrict__ y
         const int i = min(((int) threadIdx.x & 255) * 4 + 1024 * j, width - 4);
         xv[j] = *(const float4 *) (y + (int64_t) t * ys + i); wv[j] = *(const float4 *) (p.w + i); rv[j] = *(const float4 *) (p.res + (int64_t) t * p.rs + i);
     }
-    hy_rms_row<NV>(xv, wv, p.w_off, p.eps, width, nullptr, rv, p.mult, red);
+    hy_rms_row<NV>(xv, wv, p.w_off, p.eps, width, false, wv, true, rv, p.mult, red);
     if (pi_abort_late(gone, abort_w)) return;
     if (threadIdx.x < 256) {
 #pragma unroll
@@ -2501,7 +2502,7 @@ __global__ void __launch_bounds__(256) k_moe_combine_norm(const float * __restri
             acc[j].x = fmaf(g, v.x, acc[j].x); acc[j].y = fmaf(g, v.y, acc[j].y); acc[j].z = fmaf(g, v.z, acc[j].z); acc[j].w = fmaf(g, v.w, acc[j].w);
         }
     }
-    hy_rms_row<NV>(acc, wv, p.w_off, p.eps, n, nullptr, rv, p.mult, red);
+    hy_rms_row<NV>(acc, wv, p.w_off, p.eps, n, false, wv, true, rv, p.mult, red);
     hy_rms_store<NV>(acc, t, t, n, p.eps, p.out, p.os, p.two, rd, red);
 }
 
