@@ -90,7 +90,8 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     if (A.live_max > 0 && n_kv > A.live_max) return;
     const int dim1 = N1 > 0 ? 16 * N1 : A.dim1, dim2 = N1 > 0 ? 16 * (NK - N1) : A.dim2, vdim = N1 > 0 ? VW : A.vdim, n1 = (dim1 + 15) / 16;
     const float * k1 = A.k1 + (int64_t) (h / A.per_kv) * A.k1_head + map * dim1, * vb = A.v + (int64_t) (h / A.per_kv) * A.v_head;
-    const bool soft = A.weights != PI_WEIGHTS_SIGMOID;
+    constexpr bool SHARED = N1 > 0 && N1 < NK;                         // keys of a latent: soft-max, the mask alone, no soft cap (pa_launch); the branches for the rest cost <12, 8, 2> 24 bytes of scratch a lane, 112.6 us instead of 109.7 for 1000 tokens
+    const bool soft = SHARED || A.weights != PI_WEIGHTS_SIGMOID;
     pa_f32x4 q[2][NK], acc[2][NJ];
     float m_run[2] = { -INFINITY, -INFINITY }, l_run[2] = { 0.0f, 0.0f };
     int first_pos[2], odd = 0;
@@ -147,7 +148,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll 8
                     for (int t = 0; t < 32; t++) any |= A.mask[(int64_t) min(t0 + t, A.n_tok - 1) * words + (c >> 5)];
                 }
-                if (A.cell_pos) any &= pa_near(A.cell_pos, c0, 32 * PARTS, c_end, first_min, A.keep_first, lane);
+                if (!SHARED && A.cell_pos) any &= pa_near(A.cell_pos, c0, 32 * PARTS, c_end, first_min, A.keep_first, lane);
                 todo = __ballot(any != 0);
             }
             if (~todo) {
@@ -161,7 +162,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         const uint32_t in = (c_end - c0 >= 32 ? 0xffffffffu : (1u << (c_end - c0)) - 1u) & (c0 < A.cell0 ? 0xffffffffu << (A.cell0 - c0) : 0xffffffffu);
 #pragma unroll
         for (int u = 0; u < 2; u++) vis[u] = mrow[u][c0 >> 5] & in;
-        if (A.cell_pos) {                              // a lane looks at eight cells, the four of a query put them together
+        if (!SHARED && A.cell_pos) {                   // a lane looks at eight cells, the four of a query put them together
             uint32_t near[2] = { 0u, 0u };
 #pragma unroll
             for (int b = 0; b < 8; b++) {
@@ -225,7 +226,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             for (int u = 0; u < 2; u++) {
 #pragma unroll
                 for (int c = 0; c < 4; c++) s[u][c] = fmaf(s[u][c], A.scale, bias);
-                if (soft && A.softcap > 0.0f) {
+                if (!SHARED && soft && A.softcap > 0.0f) {
 #pragma unroll
                     for (int c = 0; c < 4; c++) s[u][c] = A.softcap * tanhf(s[u][c] / A.softcap);
                 }
@@ -429,9 +430,10 @@ static void pa_go(const pa_args & a, int maps, double bytes, hipStream_t s) {
 void pa_launch(const pa_args & a, int maps, double bytes, hipStream_t s) {
     const int nk = pa_steps(a), n1 = a.dim1 / 16;
     const int64_t most = (int64_t) 1 << 30;                            // floats within 32-bit byte offsets
+    const bool latent = !a.cell_pos && a.softcap <= 0.0f && a.weights != PI_WEIGHTS_SIGMOID;
     const bool whole = a.dim1 % 16 == 0 && a.dim2 % 16 == 0 && (a.vdim == 64 || a.vdim == 128) && (a.cell1 - a.cell0) * a.k1_row < most && (a.cell1 - a.cell0) * a.v_row < most && a.cell1 * a.k2_row < most;
 #define PA_NK(NV) do { if (whole && nk == 4 && n1 == 4) pa_go<4, 4, NV>(a, maps, bytes, s); else if (whole && nk == 8 && n1 == 8) pa_go<8, 8, NV>(a, maps, bytes, s); \
-                       else if (whole && nk == 6 && n1 == 4) pa_go<6, 4, NV>(a, maps, bytes, s); else if (whole && nk == 12 && n1 == 8) pa_go<12, 8, NV>(a, maps, bytes, s); \
+                       else if (whole && latent && nk == 6 && n1 == 4) pa_go<6, 4, NV>(a, maps, bytes, s); else if (whole && latent && nk == 12 && n1 == 8) pa_go<12, 8, NV>(a, maps, bytes, s); \
                        else if (nk <= 4) pa_go<4, 0, NV>(a, maps, bytes, s); else if (nk <= 8) pa_go<8, 0, NV>(a, maps, bytes, s); else pa_go<12, 0, NV>(a, maps, bytes, s); } while (0)
     if (a.vdim <= 64) PA_NK(1); else PA_NK(2);
 #undef PA_NK

@@ -34,7 +34,7 @@ def scratch_of_kernels():
     return found
 
 
-@pytest.mark.parametrize("kernel", ["k_rms_scale_once"])
+@pytest.mark.parametrize("kernel", ["k_rms_scale_once", "k_prompt_attention"])
 def test_kernels_without_scratch_memory(kernel):
     mine = {n: s for n, s in scratch_of_kernels().items() if kernel in n}
     assert mine and not any(mine.values()), mine
