@@ -95,11 +95,11 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     pa_f32x4 q[2][NK], acc[2][NJ];
     float m_run[2] = { -INFINITY, -INFINITY }, l_run[2] = { 0.0f, 0.0f };
     int first_pos[2], odd = 0;
-    const uint32_t * mrow[2];
+    uint32_t mrow[2];                                                  // (where its mask begins: pa_takes)
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         const int t = min(t0 + 16 * u + n, A.n_tok - 1), p = A.pos ? A.pos[t] : 0;
-        mrow[u] = A.mask + (int64_t) t * words;
+        mrow[u] = (uint32_t) t * (uint32_t) words;
         first_pos[u] = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
         const float * qr = A.q + (int64_t) t * A.qs + (int64_t) (h * MAPS + map) * (dim1 + dim2);
 #pragma unroll
@@ -135,8 +135,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     }
     // (a lane's rows from the tile's first on: the first that a tile reads is the scalar unit's)
     const uint32_t row1 = (uint32_t) A.k1_row * 4u, row2 = (uint32_t) A.k2_row * 4u, rowv = (uint32_t) A.v_row * 4u, lane1 = n * row1 + 16u * g, lane2 = n * row2 + 16u * g, lanev = 4u * g * rowv + 4u * (uint32_t) (NJ * n);
-    // Values that are no numbers are looked for in the sums, behind the walk: where one is not finite, the wave walks again with a look at every value
+    // Values that are no numbers are looked for in the sums, behind the walk: where one is not finite, or so large (2^100) that a maximum which lags could have made it so, or the waves' sums together, the workgroup walks again with
+    // a look at every value and weights of at most 1.  (Sums that the next launch adds to are relative to the maximum from the start)
     for (int careful = 0; ; careful = 1) {
+    const float lag = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(careful || A.state ? 0.0f : 8.0f)));
     unsigned long long todo = 0;
     for (int c0 = start; c0 < c_end; c0 += 32 * PARTS) {
         if (far) {
@@ -161,7 +163,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         uint32_t vis[2];
         const uint32_t in = (c_end - c0 >= 32 ? 0xffffffffu : (1u << (c_end - c0)) - 1u) & (c0 < A.cell0 ? 0xffffffffu << (A.cell0 - c0) : 0xffffffffu);
 #pragma unroll
-        for (int u = 0; u < 2; u++) vis[u] = mrow[u][c0 >> 5] & in;
+        for (int u = 0; u < 2; u++) vis[u] = A.mask[mrow[u] + (uint32_t) (c0 >> 5)] & in;
         if (!SHARED && A.cell_pos) {                   // a lane looks at eight cells, the four of a query put them together
             uint32_t near[2] = { 0u, 0u };
 #pragma unroll
@@ -221,7 +223,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                 for (int c = 0; c < 4; c++) { s[0] = pa_mfma(kf[i][c], q[0][i][c], s[0]); s[1] = pa_mfma(kf[i][c], q[1][i][c], s[1]); }
             if constexpr (LATE) { __builtin_amdgcn_sched_barrier(0); values(); }
             // Scores to weights (whole: every token sees every cell; else a cell that a token does not see scores minus infinity).  The maximum that a query's weights are relative to follows the scores' only when these pass
-            // it by 8 (weights up to e^8 are as good in fp32): of 128 tiles of a wave some 75 hold a new maximum of one of its 32 queries, and each of them cost all the sums their factor
+            // it by 8 (weights up to e^8 are as good in fp32 as long as no sum nears its range: below): of 128 tiles of a wave some 75 hold a new maximum of one of its 32 queries, and each of them cost all the sums their factor
 #pragma unroll
             for (int u = 0; u < 2; u++) {
 #pragma unroll
@@ -238,8 +240,8 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                 if (soft) {
                     float top = fmaxf(fmaxf(s[u][0], s[u][1]), fmaxf(s[u][2], s[u][3]));
                     top = fmaxf(top, pi_partner<16>(top)); top = fmaxf(top, pi_partner<32>(top));
-                    if (__any(top > m_run[u] + 8.0f)) {
-                        const float m_new = top > m_run[u] + 8.0f ? top : m_run[u];
+                    if (__any(top > m_run[u] + lag)) {
+                        const float m_new = top > m_run[u] + lag ? top : m_run[u];
                         const float f = m_run[u] == m_new ? 1.0f : expf(m_run[u] - m_new);    // (nothing seen yet: expf(-inf) = 0)
                         l_run[u] *= f; m_run[u] = m_new;
 #pragma unroll
@@ -282,7 +284,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int c = 0; c < 4; c++) big = max(big, __float_as_uint(acc[u][j][c]) & 0x7fffffffu);
-    if (!__any(big >= 0x7f800000u)) break;
+    if (!__syncthreads_or(big >= 0x71800000u)) break;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         m_run[u] = -INFINITY; l_run[u] = 0.0f;
@@ -417,7 +419,7 @@ static int pa_steps(const pa_args & a) { return (a.dim1 + 15) / 16 + (a.dim2 + 1
 bool pa_takes(const pa_args & a, int maps, int min_tokens) {
     auto four = [](int64_t n) { return (n & 3) == 0; };
     return a.n_tok >= min_tokens && pa_steps(a) <= 12 && a.vdim <= 128 && a.dim1 >= 4 && a.vdim >= 4 && four(a.dim1) && four(a.dim2) && four(a.vdim) && four(a.k1_row) && four(a.k1_head) && four(a.k2_row) && four(a.v_row) &&
-           four(a.v_head) && ((uintptr_t) a.k1 & 15) == 0 && ((uintptr_t) a.k2 & 15) == 0 && ((uintptr_t) a.v & 15) == 0 && (maps == 1 || a.dim2 == 0);
+           four(a.v_head) && ((uintptr_t) a.k1 & 15) == 0 && ((uintptr_t) a.k2 & 15) == 0 && ((uintptr_t) a.v & 15) == 0 && (maps == 1 || a.dim2 == 0) && (int64_t) a.n_tok * ((a.n_kv + 31) / 32) < (1ll << 32);
 }
 template <int NK, int N1, int NV>
 static void pa_go(const pa_args & a, int maps, double bytes, hipStream_t s) {

@@ -307,3 +307,23 @@ def test_scores_that_climb_and_fall(step, D, V, maps):
     vc[100], vc[200, 0, 5] = np.nan, np.inf                               # (seen by none; seen by the first forty, in one value of the first key head)
     got = run_diff(U, lib, q, kc, vc, *args, True)
     assert rel_rms(got[40:], want[40:]) < bound and np.isfinite(got[:, H // G:]).all() and not np.isfinite(got[:40, :H // G]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [33, 70])
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (36, 68)])
+def test_large_values_under_a_climbing_score(D, V, T):
+    """scores that climb by less than the maximum may lag, values near the top of fp32's range: weights of at most 1 keep their sums finite, as do the waves' sums together"""
+    U, lib = gpu()
+    H, G, n_kv = 4, 2, 400
+    rng = np.random.default_rng(D + T)
+    q = np.zeros((T, H, 1, D), np.float32)
+    q[..., 0] = 1.0
+    kc, vc = np.zeros((n_kv, G, 1, D), np.float32), (1.0 + rng.random((n_kv, G, V))).astype(np.float32)
+    kc[..., 0] = (7.5 * np.arange(n_kv) / n_kv)[:, None, None]
+    vis = np.arange(n_kv)[None, :] <= np.arange(n_kv - T, n_kv)[:, None]
+    args = [np.arange(n_kv, dtype=np.int32), vis, np.arange(n_kv - T, n_kv, dtype=np.int32), 1.0, 0, 0, 1, 0.0, 1.0, 1e-3, H, G]
+    want = diff_attention_ref(q, kc, vc, *args)
+    big = np.float32(2.0 ** 119)                                          # (a token's sum at weights of at most 1: 54 effective cells of up to 2 big; at weights of up to e^7.5: past the range)
+    got = run_diff(U, lib, q, kc, vc * big, *args, True)
+    assert np.isfinite(got).all() and rel_rms(got.astype(np.float64) / float(big), want) < 1e-5
