@@ -378,7 +378,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 template <int CR_SCAN_COLS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))) k_channel_state_scan(int heads, int dim, int vdim, int piece, const float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok,
                                                                                                      float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    if (pi_aborted_together(pi_abort_peek(abort_w), abort_w)) return;
     extern __shared__ float lds[];                // T^T [dim][tp] | S [2][dim][CR_SCAN_COLS]
     __shared__ int seg[3], bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;      // slot word, first piece ordinal, pieces of the run (0: no such run)
     const int tid = threadIdx.x, h = blockIdx.x, j0 = blockIdx.y * CR_SCAN_COLS;
@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4))
 // the same chain where T_p is diagonal (bonus rule): scratch[p] holds [L_p | diag T_p] ([dim][vdim + 1]).  grid (head, blocks over dim * vdim, run): eight pieces' loads in flight, the chain in registers
 __global__ void __launch_bounds__(256) k_channel_state_scan_diag(int heads, int dim, int vdim, int piece, const float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch,
                                                                  const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    if (pi_aborted_together(pi_abort_peek(abort_w), abort_w)) return;
     __shared__ int seg[3], bnd[CR_MAXRUNS], sorted[CR_MAXRUNS], nbnd;
     const int tid = threadIdx.x, h = blockIdx.x;
     const int n_runs = cr_runs(rec, n_tok, bnd, sorted, &nbnd);

@@ -785,7 +785,7 @@ template <int DI>
 __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim, int vstored,
                                                        const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
                                                        float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     constexpr int DIM = 32 * DI, PITCH = DIM + 4, PP = LM_TB + 4;
     __shared__ __attribute__((aligned(16))) float qk[LM_TB * PITCH];  // the queries, then the keys
     __shared__ __attribute__((aligned(16))) float pt[LM_TB * PP];
@@ -794,7 +794,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
     extern __shared__ int lm_recs[];              // the slot words of the pass
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, g = lane >> 4;
     for (int t = tid; t < n_tok; t += 256) lm_recs[t] = rec[t];
-    __syncthreads();
+    if (pi_aborted_together(gone, abort_w)) return;
     const int n_runs = la_runs(lm_recs, n_tok, bnd, &nbnd);
     if (tid < 64) la_find_piece(lm_recs, n_tok, bnd, n_runs, 0, blockIdx.y, seg);
     __syncthreads();
@@ -954,7 +954,7 @@ __global__ void __launch_bounds__(256, 2) k_linear_pieces(const float * __restri
 template <int DI>
 __global__ void __launch_bounds__(256) k_linear_scores(const float * __restrict__ q, const float * __restrict__ k, int64_t stride, int heads, int hpg, const float * __restrict__ decay, const float * __restrict__ tdecay,
                                                        const float * __restrict__ tscale, int64_t tds, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    if (pi_aborted_together(pi_abort_peek(abort_w), abort_w)) return;
     constexpr int DIM = 32 * DI, PITCH = DIM + 4;
     __shared__ __attribute__((aligned(16))) float qs[LW_TB * PITCH], ks[LW_TB * PITCH];
     __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
@@ -1015,7 +1015,7 @@ template <int DI>
 __global__ void __launch_bounds__(512, 2) k_linear_walk(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim, int vstored,
                                                         const float * __restrict__ skip, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, const float * __restrict__ scratch, float * __restrict__ out,
                                                         int64_t os, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    if (pi_aborted_together(pi_abort_peek(abort_w), abort_w)) return;
     constexpr int DIM = 32 * DI, MW = (2 * DI + 3) / 4, PITCH = DIM + 4, PP = LW_TB + 4;
     __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd;
     __shared__ __attribute__((aligned(16))) float vs[2][LW_TB * 16], ps[2][LW_TB * PP], fs[2][2 * LW_TB];
@@ -1188,11 +1188,11 @@ __global__ void __launch_bounds__(512, 2) k_linear_walk(const float * __restrict
 template <int TB>
 __global__ void __launch_bounds__(256) k_linear_state_scan(int heads, int dim, int vdim, const float * __restrict__ decay, const float * __restrict__ tdecay, int64_t tds, const float * __restrict__ state,
                                                            const int32_t * __restrict__ rec, int n_tok, float * __restrict__ scratch, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    const int gone = pi_abort_peek(abort_w);
     __shared__ int seg[4], bnd[LA_MAXRUNS], nbnd; // seg: slot word, first piece ordinal, pieces of the run (0: no such run), the run's first token
     extern __shared__ int recs[];                 // the slot words of the pass
     for (int t = threadIdx.x; t < n_tok; t += 256) recs[t] = rec[t];
-    __syncthreads();
+    if (pi_aborted_together(gone, abort_w)) return;
     const int n_runs = la_runs(recs, n_tok, bnd, &nbnd);
     if (threadIdx.x < 64) {
         int own[4], ord = la_pieces_before(bnd, n_runs, n_tok, TB, own);
@@ -1807,9 +1807,9 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         for (int s = lane + 64; s < n_s; s += 64) { const float ms = pml_t[s * 2]; if (ms != -INFINITY) d += pml_t[s * 2 + 1] * expf(ms - mstar); }
         den = pi_lanes_sum<64>(d) + (sink ? expf(sk - mstar) : 0.0f);
     }
-    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the splits' maxima, requested after it)
+    if (pi_aborted_together(gone, abort_w, 5)) return;                 // (behind the splits' maxima, requested after it)
     for (int sb = 0; sb < n_s; sb += 64) {
-        __syncthreads();
+        if (sb) __syncthreads();
         if (wave < nt) {
             const int s = sb + lane;
             const float ms = s >= n_s ? -INFINITY : sb == 0 ? m_own : pml_t[s * 2];
@@ -2370,8 +2370,7 @@ __global__ void __launch_bounds__(1024) k_moe_group(const int32_t * __restrict__
 #pragma unroll
     for (int u = 0; u < MOE_GROUP_KEEP; u++) { const int i = (int) threadIdx.x + 1024 * u; own[u] = i < n_slots ? sel[i] : -1; }
     for (int e = threadIdx.x; e < n_exp; e += 1024) cnt[e] = 0;
-    if (pi_abort_late(gone, abort_w)) return;
-    __syncthreads();
+    if (pi_aborted_together(gone, abort_w)) return;
 #pragma unroll
     for (int u = 0; u < MOE_GROUP_KEEP; u++) if (own[u] >= 0 && own[u] < n_exp) atomicAdd(&cnt[own[u]], 1);
     for (int i = threadIdx.x + 1024 * MOE_GROUP_KEEP; i < n_slots; i += 1024) { const int e = sel[i]; if (e >= 0 && e < n_exp) atomicAdd(&cnt[e], 1); }

@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
     extern __shared__ float lds[];                // q [hpg][D] | key tile [tile][D + 1], then the value tile [tile][V] in the same place | weights [tile][hpg]
     if (pool_z > 0 && (int) blockIdx.z == pool_z) {                   // the extra slice of workgroups: the pooled rows of the blocks this pass's tokens close (no token of the pass reads them: the host checked n_tok <= window)
         const int p = pos[blockIdx.x];
-        if (pi_abort_late(gone, abort_w, 5) || (p + 1) % pool != 0) return;
+        if (pi_aborted_together(gone, abort_w, 5) || (p + 1) % pool != 0) return;
         pm_pool_block((float *) kc, (float *) vc, cell_pos, mask + (int64_t) blockIdx.x * ((n_kv_arg + 31) / 32), p, pool, pool_off, G, blockIdx.y, D, V, min(dyn ? dyn[1] : n_kv_arg, n_kv_arg), pi_cell_of(dyn, 0, blockIdx.x), (int *) lds);
         return;
     }
@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
     // the first position the token sees as itself: the start of its block of `chunk` positions, or of the window of `chunk` positions that ends with the token
     const int first_pos = chunk <= 0 ? 0 : mask_kind == PI_MASK_WINDOW ? p - chunk + 1 : p / chunk * chunk;
     for (int i = tid; i < nr * D; i += 256) qsh[i] = q[(int64_t) t * qs + (int64_t) h0 * KD + i];
-    if (pi_abort_late(gone, abort_w, 5)) return;                       // (behind the queries, requested after it)
+    if (pi_aborted_together(gone, abort_w, 5)) return;                 // (behind the queries, requested after it)
     float acc[CA_MAXOUT];
 #pragma unroll
     for (int i = 0; i < CA_MAXOUT; i++) acc[i] = 0.0f;
@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(256) k_chunk_attention(const float * __restric
         }
 #pragma unroll
         for (int u = 0; u < CA_SB; u++) bal[u] = __ballot(vis[u]);
-        __syncthreads();                          // (the previous round's list and tiles are no longer read)
+        if (c0 != c_first) __syncthreads();       // (the previous round's list and tiles are no longer read)
         if (lane == 0)
 #pragma unroll
             for (int u = 0; u < CA_SB; u++) wcnt[u * 4 + wave] = __popcll(bal[u]);
@@ -626,7 +626,7 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
 // included: call this behind the launch that stores the pass's keys and values), sums their rows in position order and leaves the means in row pool_off + its own cell of both caches.
 __global__ void __launch_bounds__(256) k_pool_blocks(float * __restrict__ kc, float * __restrict__ vc, const int32_t * __restrict__ cell_pos, const uint32_t * __restrict__ mask, const int32_t * __restrict__ pos,
                                                      int pool, int64_t pool_off, int G, int D, int V, int n_kv_arg, const int32_t * __restrict__ dyn, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
+    if (pi_aborted_together(pi_abort_peek(abort_w), abort_w)) return;
     extern __shared__ int members[];              // [pool] the cell of every position of the block (-1: none)
     const int t = blockIdx.x, g = blockIdx.y;
     const int p = pos[t];

@@ -99,6 +99,15 @@ static __device__ __forceinline__ bool pi_abort_late(int peek, const int32_t * w
     return true;
 }
 
+// The same, decided for the whole workgroup by its first thread's look: for kernels whose threads take an index from what other waves have left in LDS.  Every wave asks for the word by itself, and a cancel may come in between:
+// behind waves that left, the others would take a token, a slot or a cell from where nobody wrote one, and read or write there.  A barrier (place it where the kernel needs one anyway); once per kernel
+static __device__ __forceinline__ bool pi_aborted_together(int peek, const int32_t * w, int fam = 6) {
+    __shared__ int gone;
+    if ((threadIdx.x | threadIdx.y | threadIdx.z) == 0) gone = peek;
+    __syncthreads();
+    return pi_abort_late(gone, w, fam);
+}
+
 // KV cell of token i of a pass.  dyn (device memory, refreshed per call so that one captured graph serves every call): {kv_head, n_kv, n_tokens, has_table, cell[0..n_tokens)}.
 // A run's tokens sit in consecutive cells from kv_head (find_slot, llama.cpp:1593-1644); a pass that carries several runs at once (context.cpp: coalescing) brings a table.
 static __device__ __forceinline__ int pi_cell_of(const int32_t * dyn, int kv_head, int i) { return dyn ? (dyn[3] ? dyn[4 + i] : dyn[0] + i) : kv_head + i; }
