@@ -1956,9 +1956,9 @@ int context_finish(llama_context * ctx, pi_run * run) {
     if (ctx->is_last) {
         size_t wanted = run->last_only ? 1 : 0;
         if (!run->last_only) for (int i = 0; i < n; i++) wanted += run->want_logits[i] != 0;
-        // more than a row or so (a verify batch, a step of several sequences, a scored text): the run's buffer itself goes to the caller.  What the GPU wrote is in no cache: copied, 333 rows of 32000 took 2 ms of a 4 ms pass,
-        // seven rows 28 us of a pass of 517.  A single row is copied (10 us), to where the last one was
-        const bool take = run->launched && !run->last_only && wanted * nv * 4 >= ((size_t) 3 << 16) && (!run->compact || wanted == (size_t) n);
+        // many rows (a scored text): the run's buffer itself goes to the caller (333 rows of 32000 copied: 2 ms of a 4 ms pass).  Fewer are copied to where the last ones were: a program may have kept the address, and what the GPU wrote
+        // is in no cache until somebody has read it - here (seven rows of 32000: 28 us), not in the caller's first pass over its rows
+        const bool take = run->launched && !run->last_only && wanted * nv * 4 >= ((size_t) 4 << 20) && (!run->compact || wanted == (size_t) n);
         if (take) { std::swap(ctx->logits_own, run->logits_host); std::swap(ctx->logits_own_cap, run->logits_cap); ctx->logits_out = ctx->logits_own; }
         else {                                                                 // llama.cpp:5734-5743
             const size_t size = run->last_only ? nv : (size_t) n * nv;

@@ -68,3 +68,34 @@ def test_rows_stay_where_a_run_brings_none(rows):
     assert np.all(ctx.decode(*batch(2)) == 4.0)
     ctx.free()
     model.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [2, 97, 400])
+def test_rows_of_a_next_run_are_where_the_last_ones_were(rows):
+    """a program that asked for the buffer once reads every later run's rows there, whether they are as many or fewer and whether or not the next run started before this one's rows were fetched - as long as they are below the 4 MB from
+    which rows change hands with the run's buffer"""
+    model = LL.Model(MODEL)
+    assert 4 * rows * model.n_vocab < 4 << 20
+    ctx = LL.Context(model, n_ctx=4 * rows + 64, n_batch=2 * rows, logits_all=True)
+
+    def batch(token, n, seq=0):
+        return [token] * n, list(range(n)), [[seq]] * n
+
+    def shown():
+        return np.ctypeslib.as_array(C.cast(ctx.lib.llama_get_logits(ctx.h), C.POINTER(C.c_float)), shape=(rows, model.n_vocab))
+
+    own = ctx.decode(*batch(5, rows))
+    kept = shown()
+    assert np.array_equal(kept, own)
+    for token, n in ((6, rows), (7, 1), (8, rows), (9, rows - 1)):
+        ctx.kv_clear()
+        own = ctx.decode(*batch(token, n))
+        assert shown().ctypes.data == kept.ctypes.data and np.array_equal(kept[:n], own), (token, n)
+    ctx.kv_clear()
+    tickets = [ctx.start(*batch(10 + i, rows, i)) for i in range(2)]
+    for t in tickets:
+        own = ctx.finish(t)
+        assert shown().ctypes.data == kept.ctypes.data and np.array_equal(kept, own)
+    ctx.free()
+    model.free()
