@@ -722,18 +722,18 @@ __global__ void __launch_bounds__(256) k_conv_state_update(const float * __restr
     unsigned long long ends = __ballot((threadIdx.x & 63) < CV_RUN && mine < n_tok && (mine + 1 == n_tok || ((rec[min(mine + 1, n_tok - 1)] ^ word) & ~PM_FRESH) != 0));
     if (c >= channels) return;
     for (; ends; ends &= ends - 1) {
-    const int t = blockIdx.x * CV_RUN + __ffsll(ends) - 1, slot = __builtin_amdgcn_readlane(word, __ffsll(ends) - 1) & ~PM_FRESH;
-    int len = 1, fresh = 0;                                           // tokens of the sequence in this pass, counted up to taps - 1
-    while (len < taps - 1 && t - len >= 0 && (rec[t - len] & ~PM_FRESH) == slot) len++;
-    if (len < taps - 1) fresh = (rec[t - len + 1] & PM_FRESH) != 0;
-    float * st = state + (int64_t) slot * (taps - 1) * channels + c;
-    for (int i = 0; i < taps - 1; i++) {
-        const int from = i + len;                                     // row of (old state, then the pass's tokens) that becomes row i
-        float v;
-        if (from < taps - 1) v = fresh ? 0.0f : st[(int64_t) from * channels];
-        else v = x[(int64_t) (t - len + 1 + from - (taps - 1)) * xs + c];
-        st[(int64_t) i * channels] = v;
-    }
+        const int t = blockIdx.x * CV_RUN + __ffsll(ends) - 1, slot = rec[t] & ~PM_FRESH;       // (asked for again: the lane that looked at it may have left)
+        int len = 1, fresh = 0;                                       // tokens of the sequence in this pass, counted up to taps - 1
+        while (len < taps - 1 && t - len >= 0 && (rec[t - len] & ~PM_FRESH) == slot) len++;
+        if (len < taps - 1) fresh = (rec[t - len + 1] & PM_FRESH) != 0;
+        float * st = state + (int64_t) slot * (taps - 1) * channels + c;
+        for (int i = 0; i < taps - 1; i++) {
+            const int from = i + len;                                 // row of (old state, then the pass's tokens) that becomes row i
+            float v;
+            if (from < taps - 1) v = fresh ? 0.0f : st[(int64_t) from * channels];
+            else v = x[(int64_t) (t - len + 1 + from - (taps - 1)) * xs + c];
+            st[(int64_t) i * channels] = v;
+        }
     }
 }
 

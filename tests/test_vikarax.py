@@ -377,11 +377,12 @@ def test_causal_conv_over_sequences_and_passes(taps, channels, fused):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("taps", [2, 3, 4])
-def test_causal_conv_of_long_passes(taps):
-    """runs of tokens: sequences that start, go on and end anywhere in a run of sixteen, shorter than the taps and longer than a run, one that starts from nothing and one with a state, a last run that is not full"""
+@pytest.mark.parametrize("taps,channels", [(2, 5000), (3, 5000), (4, 5000), (2, 3841), (4, 3841)])
+def test_causal_conv_of_long_passes(taps, channels):
+    """runs of tokens: sequences that start, go on and end anywhere in a run of sixteen, shorter than the taps and longer than a run, one that starts from nothing and one with a state, a last run that is not full; a last wave of eight channels and
+    of one, fewer than the sixteen lanes that look at a run's tokens"""
     U, lib = gpu()
-    channels, slots, T = 5000, 6, 187
+    slots, T = 6, 187
     rng = np.random.default_rng(taps)
     w, state = rng.standard_normal((channels, taps)).astype(np.float32), rng.standard_normal((slots, taps - 1, channels)).astype(np.float32)
     rec = [0] * 15 + [1 | F] + [2] * 2 + [3 | F] + [3] * 60 + [4] * 47
