@@ -387,7 +387,10 @@ static bool mul_mat_grouped(int n, const pi_weight * const * ws, const void * co
 }
 
 // A product of the serving precision in a pass of many tokens reads activations that are bfloat16 already: xh, where a kernel ahead wrote them, or rounded here, into the context's scratch (products of a context follow each other on
-// its stream).  Everything else goes to the operators that take fp32
+// its stream).  Everything else goes to the operators that take fp32.
+// Rounded by a launch of its own (1.8 .. 3 us) a product of K below 1024, or of many rows and few tokens, is slower on cold weights than the tile that rounds by itself (us, tile / both launches: 4096 x 512 at 48 tokens 6.1 / 6.6,
+// 32000 x 2048 30.3 / 34.7; 4096 x 2048 15.8 / 13.2), but no call is: the designs that round so (Vikarax with experts and dense, Rarevik, Rerizen; widths 1024, 2048, 4096; 33 .. 256 tokens) take 0.64 .. 1.006 times what they
+// took with the tile.  A line at K 1024, 12288 rows and 64 tokens made calls of width 1024 up to 4 % slower (their weights stay in the last cache) and none of the others quicker by more than 1 %
 static int dense_segments(llama_context * ctx, const pi_weight * w, const float * x, int64_t xs, int64_t seg_rows, int64_t seg_off, int n_seg, int n_tok, float * out, int64_t os, int act_a, int64_t rows_a, int act_b, hipStream_t s,
                           const uint16_t * xh = nullptr, int64_t xhs = 0, const float * bias = nullptr) {
     const int64_t n = (n_seg - 1) * seg_off + pi_weight_columns(w), hs = xh ? xhs : n;

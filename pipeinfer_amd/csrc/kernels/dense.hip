@@ -12,7 +12,8 @@
 //   k_dense_tile   serving precision, more tokens: tiles of 64 .. 256 rows x 64 .. 128 tokens through LDS (dense_tile.h).  Small grids are bound by what one compute unit can have on its way from memory and by the
 //                  latency of a step, large ones by the shared levels of memory: 850 TFLOP/s at 16384 x 4096 x 2048 tokens (128 x 128 tiles with a step's parts one after another: 710), 14 us for
 //                  2048 x 2048 x 512 (17)
-//   k_dense_async  the same from activations that are bfloat16 in memory (dense_async.h): what the engine's passes of more than 32 tokens take; k_round_bf16 makes such activations where no kernel ahead writes them
+//   k_dense_async  the same from activations that are bfloat16 in memory (dense_async.h): what the engine's passes of more than 32 tokens take (matrices of 16384 rows and more: of more than 8); k_round_bf16 makes such activations where no kernel
+//                  ahead writes them
 //   k_embed        rows of the table gathered, widened and scaled
 #include "ops_common.h"
 #include "dense_tile.h"

@@ -574,10 +574,11 @@ extern "C" int pi_op_sum_tanh_norm_shift(const float * x, int64_t x_stride, cons
 // rec[t] = state slot of token t (| 1 << 30 on the first token of a sequence whose state starts from zero), tokens of one slot are consecutive.  Workgroup (head, column block,
 // piece): thread (column j, part sp of R) keeps S[i][j] for its DPT rows i in registers and walks the piece's tokens in order.
 // A pass of up to LA_TB tokens is one launch: a piece is a sequence's whole run, S comes from and goes back to HBM.  Longer passes cut every sequence's run into pieces of LA_TB
-// tokens and take three launches (on the matrix cores: pieces of LM_TB, see there; a pass of as many tokens one launch), so that the serial depth is two pieces instead of the whole prompt (the recurrence is linear in S):
+// tokens and take three launches, so that the serial depth is two pieces instead of the whole prompt (the recurrence is linear in S):
 //   mode 1  every piece but a run's last: the state it would build from ZERO, L_p = sum_j lambda^(len-1-j) k_j v_j^T, into scratch
 //   k_linear_state_scan  per run, piece by piece: S_in(p + 1) = lambda^len_p * S_in(p) + L_p, S_in(0) = the slot's state (or zero); scratch[p] <- S_in(p)
 //   mode 2  every piece from its true S_in(p): outputs; a run's last piece leaves the slot's new state
+// Key widths of 32, 64, 96 and 128 take the fp32 matrix cores instead: up to LM_TB tokens one launch (k_linear_pieces), more of them two over pieces of LW_TB (k_linear_scores, k_linear_walk).
 #define LA_TB 32                                  // tokens of a piece; q, k and v of a piece are staged in LDS
 #define LA_FRESH (1 << 30)
 #define LA_MAXRUNS 256                            // sequences a pass may carry (the host checks)
@@ -1301,7 +1302,7 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
     const int nta = std::min(n_tok, PI_KT_MAXNT - 1);
 #define LA_GO(D, MODE) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_attention<D>, grid, dim3(threads), lds, s, q, k, v, stride, heads, hpg, dim, vdim, value_cols, R, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, state_dev, rec_dev, n_tok, MODE, scratch_dev, out, out_stride, pi_abort_word())
 #define LA_ANY(MODE) do { if (dpt == 8) LA_GO(8, MODE); else if (dpt == 16) LA_GO(16, MODE); else LA_GO(32, MODE); } while (0)
-    const bool matrix = dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22);       // (32-bit offsets within a piece; pieces twice as long take half of the scratch that was asked for)
+    const bool matrix = dim % 32 == 0 && dim <= 128 && n_tok <= LM_MAX_TOKENS && stride < (1 << 24) && vdim <= (1 << 22);       // (32-bit offsets within a piece)
     const unsigned gr = (unsigned) std::max(1, std::min(n_tok, max_segments)), gb = (unsigned) (((int64_t) dim * vdim + 255) / 256);
 #define LM_ANY(GO) do { if (dim == 32) GO(1); else if (dim == 64) GO(2); else if (dim == 96) GO(3); else GO(4); } while (0)
 #define LM_PIECES(DI) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_pieces<DI>, dim3((unsigned) heads, gr), dim3(256), (size_t) 4 * n_tok, s, q, k, v, stride, heads, hpg, vdim, value_cols, decay_dev, tdecay_dev, tscale_dev, t_stride, \

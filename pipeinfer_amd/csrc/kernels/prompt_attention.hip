@@ -1,10 +1,10 @@
 // Attention of a prompt: 32 tokens x one head per workgroup, scores and sums on the fp32 matrix cores.
 //
-// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; about 94 reached at 2048 tokens x 32 heads of 128) and the vector instructions, one after the other: while such a
+// What bounds it: the fp32 matrix products (v_mfma_f32_16x16x4_f32: 157 TFLOP/s on the whole chip; 79 reached at 2048 tokens x 32 heads of 128) and the vector instructions, one after the other: while such a
 // product runs, nothing else goes to its SIMD's vector unit, of whichever wave (2048 tokens: 830000 clocks, 530000 of products, 125000 of 240 vector instructions per tile of 16 cells x 32 tokens; with 460 of them 930000;
 // tiles through LDS instead of registers, or the weights between the next tile's products: no less).  So a tile's vector work is kept small: weights relative to a maximum that may lag (below), cells that a token does
 // not see as scores of minus infinity and only where there are some, an exponential for this range alone, no look at single values.  The kernels that give every token a workgroup (k_latent_scores, k_chunk_attention) are right for single
-// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  Whole calls: 2048 tokens, 32 heads of 128, rank 512: 6.9 ms -> 0.44; 1000 tokens, 16 heads of 192: 1.11 ms -> 0.12;
+// tokens; with a prompt they read every key and value once per token and pay 2 rank instead of dim + vdim multiply-adds per pair of token and cell where the keys are up-projections of a latent.  Whole calls: 2048 tokens, 32 heads of 128, rank 512: 6.9 ms -> 0.44; 1000 tokens, 16 heads of 192: 1.11 ms -> 0.11;
 // 1000 tokens of 16 differential heads over a window of 256: 526 us -> 70; 333 tokens of 16 heads of 64: 382 us -> 19.
 //   k_latent_expand   the keys and values of the pass's cells written out once: an fp32 latent in three bfloat16 parts times the bfloat16 matrix on the matrix cores, exact products (dense_tile.h)
 //   k_prompt_attention  a wave owns 32 queries (two operand tiles, so a key is read for both) and every fourth run of 32 cells; no barrier until the four waves' sums meet at the end.  The scores are
@@ -65,7 +65,7 @@ static __device__ __forceinline__ uint32_t pa_near(const int32_t * __restrict__ 
     return near;
 }
 
-// e^x of a score below the maximum (or up to e^8): x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
+// e^x of a score below the maximum (or up to e^8), by Cody and Waite's reduction in two parts: x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
 // errors of expf (rms 2.6e-8, at most 8.3e-8) without its two ends of the range.  Minus infinity: 0 (what the fused part gives below the bound), no number: no number
 static __device__ __forceinline__ float pa_exp(float x) {
     const float t = fmaxf(x * 1.44269502f, -300.0f), r = rintf(t);
