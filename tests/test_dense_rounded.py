@@ -90,7 +90,7 @@ def _asked(lib, U, op, out, from_, n, rows, only):
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,n", [(33, 64), (40, 1000), (35, 2048), (33, 4096)])
 def test_rounded_outputs_are_the_fp32_ones_rounded(T, n):
-    """norms, gates, shifts and embeddings: the rounded rows against the rounded fp32 result of the same call; asked for alone they leave the fp32 rows as they were"""
+    """norms, gates, shifts and embeddings: the rounded rows against the rounded fp32 result of the same call; asked for alone they leave the fp32 rows as they were, but for the operators whose fp32 rows something else reads as well"""
     from tests import gpu_util as U
     lib = U.init()
     rng = np.random.default_rng([T, n])
@@ -120,8 +120,12 @@ def test_rounded_outputs_are_the_fp32_ones_rounded(T, n):
         full = out.get(np.float32, (T, width), 0, T * width)
         assert met == 1, name
         assert np.array_equal(got, bf16(full)), name
+        before = np.full(T * 3 * n, 777.0, np.float32)
+        L.check(lib.pi_memcpy_h2d(out.ptr, before.ctypes.data_as(C.c_void_p), before.nbytes, None))
+        L.check(lib.pi_stream_sync(None))
         alone, met = _asked(lib, U, op, out, 0, width, T, 1)
         assert met == 1 and np.array_equal(alone, got), name
+        assert np.array_equal(out.get(np.float32, (T, width), 0, T * width), full if name in ("rms_post", "embed", "embed_pair") else before[:T * width].reshape(T, width)), name
         _, met = _asked(lib, U, op, out, 0, width - 8, T, 0)      # not the operator's rows: not met, and not left behind for the next one
         assert met == 0 and lib.pi_rounded_output_written() == 1, name
         assert np.array_equal(out.get(np.float32, (T, width), 0, T * width), full), name

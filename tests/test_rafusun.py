@@ -378,7 +378,7 @@ def test_channel_recurrence_rules_decays_and_passes(H, G, D, V, rule, pieces):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 16), (3, 3, 64, 64), (4, 2, 128, 48), (1, 1, 128, 128)])
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 16), (3, 3, 64, 64), (4, 2, 128, 48), (1, 1, 128, 128), (1, 1, 64, 144), (2, 1, 32, 272)])
 @pytest.mark.parametrize("rule", [DELTA, BONUS])
 def test_channel_recurrence_pieces_on_the_matrix_cores(H, G, D, V, rule):
     """the sizes that long passes take the matrix cores for: the same plan of passes"""
@@ -386,12 +386,12 @@ def test_channel_recurrence_pieces_on_the_matrix_cores(H, G, D, V, rule):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rule,qk_unit", [(DELTA, 1), (BONUS, 0), (DELTA, 0)])
-def test_channel_recurrence_pieces_against_the_walk(rule, qk_unit):
+@pytest.mark.parametrize("rule,qk_unit,V", [(DELTA, 1, 32), (BONUS, 0, 32), (DELTA, 0, 32), (DELTA, 1, 144), (BONUS, 0, 144), (DELTA, 1, 272), (BONUS, 0, 272)])
+def test_channel_recurrence_pieces_against_the_walk(rule, qk_unit, V):
     """against the walk token by token: decays of nothing and of one, equal keys (every entry of the piece's triangle as large as it gets), a state that was there; values, keys and decays that are no numbers
-    reach their own token's outputs and later ones, and no others"""
+    reach their own token's outputs and later ones, and no others (a value's among the first sixteen columns, and among the last, which of many columns a wave looks at second)"""
     U, lib = gpu()
-    H, D, V, T, slots = 2, 64, 32, 150, 2
+    H, D, T, slots = 2, 64, 150, 2
     rng = np.random.default_rng(rule + qk_unit)
     q, k, v = (rng.standard_normal((T, H * n)).astype(np.float32) * 0.3 for n in (D, D, V))
     k[40:60] = k[40]
@@ -400,10 +400,10 @@ def test_channel_recurrence_pieces_against_the_walk(rule, qk_unit):
     state = rng.standard_normal((slots, H, D, V)).astype(np.float32)
     rec = np.array([0] * 113 + [1 | F] + [1] * 36, np.int32)
     n = int(lib.pi_op_channel_recurrence_scratch_floats(H, D, V, T, slots))
-    for where in (None, "v", "k", "g"):
+    for where, column in ((None, 0), ("v", 3), ("k", 3), ("g", 3), ("v", V - 5)):
         a = {"q": q.copy(), "k": k.copy(), "v": v.copy(), "g": raw.copy()}
         if where:
-            a[where][50, 3] = np.inf if where != "g" else np.nan
+            a[where][50, column] = np.inf if where != "g" else np.nan
         outs, states = [], []
         for pieces in (True, False):
             ds = [U.Dev(x) for x in (a["q"], a["k"], a["v"], a["g"], braw, bonus, rec)]
@@ -587,11 +587,13 @@ def test_prompt_portions_and_decoding_agree_with_the_oracle(tmp_path, variant, e
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("decay_rank,gate_rank", [(8, 8), (64, 64), (64, 128)])
 @pytest.mark.parametrize("exact", [True, False])
-def test_a_wider_model_with_long_passes(tmp_path, exact):
-    """widths and passes that reach the matrix-core products and the tiles of the recurrences: 300 tokens in passes of 128, then single tokens"""
-    layers = [O.delta_layer(heads=4, kv_heads=2, dim=32, vdim=48, conv=4, decay_rank=8, gate_rank=8, mlp=None),
-              O.parallel_layer(heads=4, kv_heads=2, dim=64, vdim=32, chunk=100, rot_dims=16, scale=0.2, r_heads=4, r_dim=32, decay_rank=8, mlp=O.dense_mlp(256))]
+def test_a_wider_model_with_long_passes(tmp_path, exact, decay_rank, gate_rank):
+    """widths and passes that reach the matrix-core products and the tiles of the recurrences, ranks below a step of those products and of whole ones (equal ranks: one matrix in two segments; two matrices): 300 tokens in passes of 128,
+    then single tokens"""
+    layers = [O.delta_layer(heads=4, kv_heads=2, dim=32, vdim=48, conv=4, decay_rank=decay_rank, gate_rank=gate_rank, mlp=None),
+              O.parallel_layer(heads=4, kv_heads=2, dim=64, vdim=32, chunk=100, rot_dims=16, scale=0.2, r_heads=4, r_dim=32, decay_rank=decay_rank, mlp=O.dense_mlp(256))]
     m = small_model(seed=13, layers=layers, width=128, vocab=200)
     rng = np.random.default_rng(6)
     toks = [int(t) for t in rng.integers(0, 200, 320)]
