@@ -135,9 +135,10 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
     }
     // (a lane's rows from the tile's first on: the first that a tile reads is the scalar unit's)
     const uint32_t row1 = (uint32_t) A.k1_row * 4u, row2 = (uint32_t) A.k2_row * 4u, rowv = (uint32_t) A.v_row * 4u, lane1 = n * row1 + 16u * g, lane2 = n * row2 + 16u * g, lanev = 4u * g * rowv + 4u * (uint32_t) (NJ * n);
-    // Values that are no numbers are looked for in the sums, behind the walk: where one is not finite, or so large (2^100) that a maximum which lags could have made it so, or the waves' sums together, the workgroup walks again with
-    // a look at every value and weights of at most 1.  (Sums that the next launch adds to are relative to the maximum from the start)
-    for (int careful = 0; ; careful = 1) {
+    // Values that are no numbers are looked for in the sums, behind the walk: where one is not finite, or so large (2^100) that a maximum which lags could have made it so, or the waves' sums together, the wave walks again with a look at
+    // every value and weights of at most 1.  (Sums that the next launch adds to are relative to the maximum from the start)
+    int careful = 0;
+    for (; ; careful = 1) {
     const float lag = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(careful || A.state ? 0.0f : 8.0f)));
     unsigned long long todo = 0;
     for (int c0 = start; c0 < c_end; c0 += 32 * PARTS) {
@@ -284,7 +285,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
         for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int c = 0; c < 4; c++) big = max(big, __float_as_uint(acc[u][j][c]) & 0x7fffffffu);
-    if (!__syncthreads_or(big >= 0x71800000u)) break;
+    if (!__any(big >= 0x71800000u)) break;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         m_run[u] = -INFINITY; l_run[u] = 0.0f;
@@ -295,7 +296,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         l_run[u] += __shfl_xor(l_run[u], 16, 64); l_run[u] += __shfl_xor(l_run[u], 32, 64);
-        if (lane == 0) meet_odd[wave] = odd;
+        if (lane == 0) meet_odd[wave] = odd | careful << 1;
         if (g == 0) { meet_m[wave][16 * u + n] = m_run[u]; meet_l[wave][16 * u + n] = l_run[u]; }
     }
     // the waves meet, 16 tokens at a time: sixteen threads per token, four outputs of every 64 each
@@ -307,7 +308,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
 #pragma unroll
             for (int j = 0; j < NV; j++) *(pa_f32x4 *) &meet[wave][n][NJ * (4 * g + c) + 4 * j] = pa_f32x4{ acc[u][4 * j][c], acc[u][4 * j + 1][c], acc[u][4 * j + 2][c], acc[u][4 * j + 3][c] };
         __syncthreads();
-        const int r = tid >> 4, t = t0 + 16 * u + r, v0 = (tid & 15) * 4;
+        const int r = tid >> 4, t = t0 + 16 * u + r, v0 = (tid & 15) * 4, again = (meet_odd[0] | meet_odd[1] | meet_odd[2] | meet_odd[3]) & 2;
         pa_f32x4 o[MAPS][NV]; float M[MAPS], L[MAPS];
         float * st = A.state ? A.state + ((int64_t) min(t, A.n_tok - 1) * A.heads + h) * (vdim + 2) : nullptr;
 #pragma unroll
@@ -317,6 +318,9 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             if (soft) {
 #pragma unroll
                 for (int w = 0; w < PARTS; w++) M[mp] = fmaxf(M[mp], meet_m[w * MAPS + mp][16 * u + r]);
+                if (again && !st)                                     // beside sums that weights of at most 1 are to keep in range: what the others' scores may have reached
+#pragma unroll
+                    for (int w = 0; w < PARTS; w++) M[mp] = fmaxf(M[mp], meet_m[w * MAPS + mp][16 * u + r] + (meet_odd[w * MAPS + mp] & 2 ? 0.0f : 8.0f));
             }
 #pragma unroll
             for (int j = 0; j < NV; j++) o[mp][j] = pa_f32x4{ 0.0f, 0.0f, 0.0f, 0.0f };
@@ -340,7 +344,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
             }
         }
         if (t >= A.n_tok) continue;
-        if (meet_odd[0] | meet_odd[1] | meet_odd[2] | meet_odd[3]) {  // the infinities and NaNs of the cells that this token sees
+        if ((meet_odd[0] | meet_odd[1] | meet_odd[2] | meet_odd[3]) & 1) {  // the infinities and NaNs of the cells that this token sees
             const int p = A.pos ? A.pos[t] : 0, fp = A.chunk <= 0 ? 0 : A.mask_kind == PI_MASK_WINDOW ? p - A.chunk + 1 : p / A.chunk * A.chunk;
             for (int cell = A.cell0; cell < c_end; cell++) {
                 if (!(A.mask[(int64_t) t * words + (cell >> 5)] >> (cell & 31) & 1u)) continue;

@@ -327,3 +327,22 @@ def test_large_values_under_a_climbing_score(D, V, T):
     big = np.float32(2.0 ** 119)                                          # (a token's sum at weights of at most 1: 54 effective cells of up to 2 big; at weights of up to e^7.5: past the range)
     got = run_diff(U, lib, q, kc, vc * big, *args, True)
     assert np.isfinite(got).all() and rel_rms(got.astype(np.float64) / float(big), want) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (36, 68)])
+def test_large_values_beside_a_lagging_maximum(D, V):
+    """three waves that each see one value near the top of fp32's range, the fourth scores that climb within its run of cells by less than its maximum may lag: what the three weigh beside them keeps their sum finite"""
+    U, lib = gpu()
+    H, G, T, n_kv = 2, 1, 40, 128
+    q = np.zeros((T, H, 1, D), np.float32)
+    q[..., 0] = 1.0
+    kc, vc = np.zeros((n_kv, G, 1, D), np.float32), np.ones((n_kv, G, V), np.float32)
+    kc[112:, ..., 0] = 7.5
+    vc[[0, 32, 64]] = 2.5e38
+    vis = np.zeros((T, n_kv), bool)
+    vis[:, [0, 32, 64]] = vis[:, 96:] = True
+    args = [np.arange(n_kv, dtype=np.int32), vis, np.full(T, n_kv, np.int32), 1.0, 0, 0, 1, 0.0, 1.0, 1e-3, H, G]
+    want = diff_attention_ref(q, kc, vc, *args)
+    got = run_diff(U, lib, q, kc, vc, *args, True)
+    assert np.isfinite(got).all() and rel_rms(got / 1e38, want / 1e38) < 1e-5
