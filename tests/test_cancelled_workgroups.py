@@ -10,7 +10,7 @@ import pytest
 KERNELS = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pipeinfer_amd", "csrc", "kernels")
 # the look behind the barrier that follows the last write of an index: nobody who stays lacks one
 LOOKS_BEHIND = {"k_linear_attention", "k_channel_recurrence", "k_channel_pieces", "k_channel_walk", "k_attention_tiles"}
-# what is in LDS only narrows a range that the arguments bound (k_latent_scores), picks between two walks over the same cells (k_prompt_attention) or is a result (k_topk1)
+# what is in LDS only narrows a range that the arguments bound (k_latent_scores), says whether cells that the arguments bound are looked at again (k_prompt_attention) or is a result (k_topk1)
 BOUNDED = {"k_latent_scores", "k_prompt_attention", "k_topk1"}
 
 
