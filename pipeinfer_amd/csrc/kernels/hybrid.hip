@@ -1975,35 +1975,44 @@ extern "C" int pi_op_latent_attention_rot(const float * q, int64_t q_stride, con
 // tiles / workgroups per token 33 tokens of 16000 cells, 8 heads of rank 256 610 / 455, 16 of 512 + 64 1205 / 1060, 16 of 128 + 32 (in several launches) 1576 / 360, 9 tokens of them 1587 / 199; 128 heads, 9 tokens of
 // 4000 cells 751 / 480, of 300 100 / 184; 33 tokens of 512 of 65536, rank 512 114 / 202.
 // 0: none; n_kv: all.  The line between is looked at on the device, where the number of live cells is known: both sets of launches go out and one returns at once
-static int latent_tiles_to(const lat_plan & p, const pa_args & a, int rank, int launches) {
+// split: keys and values in three parts (split_attention.hip): a round of 256 workgroups and 128 cells 1.2 + 0.085 per step, the parts written out at 800 TFLOP/s, 20 for every pair of launches (tiles / workgroups per token there: 33 tokens
+// of 1033 cells, 16 heads of 128, rank 512 60 / 362, of 12033 465 / 899, 32 heads of 4033 238 / 468; 8 heads of 128 + 64, 33 tokens of 12033 338 / 554)
+static int latent_tiles_to(const lat_plan & p, const pa_args & a, int rank, int launches, bool split) {
     const double steps = (a.dim1 + 15) / 16 + (a.dim2 + 15) / 16 + 4 * ((a.vdim + 63) / 64);
-    const int64_t rounds = ((int64_t) a.heads * ((a.n_tok + 31) / 32) + 511) / 512, heads = (a.heads + p.M - 1) / p.M;
-    auto tiles = [&](int64_t live) { return (double) ((live + 127) / 128 * rounds) * (2.0 + 0.385 * steps) + 6e-9 * (double) live * a.heads * (a.dim1 + a.vdim) * rank + 8.0 * launches; };
+    const int64_t slots = split ? 256 : 512, rounds = ((int64_t) a.heads * ((a.n_tok + 31) / 32) + slots - 1) / slots, heads = (a.heads + p.M - 1) / p.M;
+    auto tiles = [&](int64_t live) {
+        return (double) ((live + 127) / 128 * rounds) * (split ? 1.2 + 0.085 * steps : 2.0 + 0.385 * steps) + (split ? 7.8e-9 : 6e-9) * (double) live * a.heads * (a.dim1 + a.vdim) * rank + (split ? 20.0 : 8.0) * launches;
+    };
     auto tokens = [&](int64_t live) { return std::ceil((double) (a.n_tok * heads) * live / p.cap / 256) * (double) std::min<int64_t>(live, p.cap) * (rank + a.dim2) * (1.9e-4 + 2.9e-5 * p.M) + 25.0; };
     int64_t to = a.n_kv, live = a.n_kv;                                // down from all cells as long as the tiles lose
     while (live >= 64 && 0.72 * tiles(live) > tokens(live)) { to = live = live * 5 / 7; }
-    return live < 64 ? 0 : (int) to;
+    return to == a.n_kv ? a.n_kv : live < 64 ? 0 : (int) to;          // (33 tokens alone in a context of 33 cells: 20 us, a workgroup per token 80)
 }
 // A prompt with its keys and values written out (prompt_attention.hip), in as few launches over the cells as the scratch memory allows.  How many live cells it took the pass for: 0 none, a.n_kv any
 static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, size_t scratch_floats, double bytes, hipStream_t s) {
     if ((rank & 7) || (a.k2_row & 3) || ((uintptr_t) cache & 15) || ((uintptr_t) scratch & 15)) return 0;
-    const size_t per_cell = (size_t) a.heads * (a.dim1 + a.vdim), state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3;
-    size_t cells = ((size_t) a.n_kv + 63) / 64 * 64;
-    if (cells * per_cell > scratch_floats) {
+    const size_t state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3;
+    size_t cells = 0;
+    auto fits = [&](size_t per_cell) {                                 // the cells of a launch, 0: too few
+        cells = ((size_t) a.n_kv + 63) / 64 * 64; a.state = nullptr;
+        if (cells * per_cell <= scratch_floats) return true;
         cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
-        if (cells < 1024) return 0;
         a.state = scratch + cells * per_cell;
-    }
+        return cells >= 1024;
+    };
+    const bool split = sa_takes(a, rank) && fits(sa_cell_floats(a.heads, a.dim1, a.dim2, a.vdim));
+    if (!split && !fits((size_t) a.heads * (a.dim1 + a.vdim))) return 0;
     a.k1 = scratch; a.k1_row = (int64_t) a.heads * a.dim1; a.k1_head = a.dim1;
     a.v = scratch + cells * (size_t) a.k1_row; a.v_row = (int64_t) a.heads * a.vdim; a.v_head = a.vdim;
     a.k2 = cache + rank;
     if (!pa_takes(a, 1, PA_LATENT_TOKENS)) return 0;
-    const int to = latent_tiles_to(p, a, rank, (int) (((size_t) a.n_kv + cells - 1) / cells));
+    const int to = latent_tiles_to(p, a, rank, (int) (((size_t) a.n_kv + cells - 1) / cells), split);
     if (to == 0 || (to < a.n_kv && !a.dyn)) return 0;
     a.live_max = to < a.n_kv ? to : 0;
     if (to == a.n_kv) a.rd = pi_round_asked(0, (int64_t) a.heads * a.vdim);      // (else other launches may be the ones that write)
     for (size_t c = 0; c < (size_t) to; c += cells) {
         a.cell0 = (int) c; a.cell1 = (int) std::min((size_t) to, c + cells); a.first = c == 0; a.last = c + cells >= (size_t) to;
+        if (split) { sa_launch(a, cache, rank, wuk, wuv, scratch, bytes, s); continue; }
         pa_expand(cache, a.k2_row, rank, wuk, wuv, a.cell0, a.cell1, a.n_kv, a.live_max, a.dyn, scratch, scratch + cells * (size_t) a.k1_row, s);
         pa_launch(a, 1, bytes, s);
     }

@@ -15,7 +15,6 @@
 
 #include <algorithm>
 
-typedef float pa_f32x4 __attribute__((ext_vector_type(4)));
 typedef int pa_i32x4 __attribute__((ext_vector_type(4)));
 
 // tiles of 128 rows of the two matrices x 64 cells; an XCD takes a contiguous run of tiles, eight blocks of rows wide and then along the cells (k_dense_tile)
@@ -64,14 +63,6 @@ static __device__ __forceinline__ uint32_t pa_near(const int32_t * __restrict__ 
     }
     return near;
 }
-
-// e^x of a score below the maximum (or up to e^8), by Cody and Waite's reduction in two parts: x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
-// errors of expf (rms 2.6e-8, at most 8.3e-8) without its two ends of the range.  Minus infinity: 0 (what the fused part gives below the bound), no number: no number
-static __device__ __forceinline__ float pa_exp(float x) {
-    const float t = fmaxf(x * 1.44269502f, -300.0f), r = rintf(t);
-    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - r) + fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -t))), (int) r);
-}
-static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // NK: steps of 16 key values (dim1 and dim2 rounded up each), NV: steps of 64 outputs.  Lane l of a wave holds, with n = l % 16 and g = l / 16: query 16 u + n (u = 0, 1), its key values 16 i + 4 g + c, the scores and
 // weights of the cells 4 g + c of a tile of 16, and of the sums the outputs 4 NV (4 g + c) + j.  N1 > 0: whole steps only (dim1 = 16 N1, dim2 = 16 (NK - N1), vdim = 64 NV) and 32-bit offsets, so that a row's
