@@ -431,14 +431,14 @@ extern "C" int pi_op_round_bf16(const float * x, int64_t x_stride, int64_t n, in
                      out + (int64_t) t * out_stride, out_stride, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
-// The tile that needs the least time, by rounds of 256 workgroups: 2.5 us + K / 2048 * rounds * the cost of one (us at K 2048 on weights from memory, measured over 1024 .. 32000 rows x 64 .. 2048 tokens):
-// 32 x 64 4.6, 64 x 64 6.3, 64 x 96 8.5, 128 x 128 19.5, 128 x 192 26, 128 x 256 31, 256 x 256 58.  Both sides of the crossings: 2048 x 2048 at 200 tokens 32 x 64 7.1, 64 x 64 8.2, at 333 9.0 / 8.7; at 700 64 x 64 13.2,
-// 64 x 96 10.5; 4096 x 4096 at 512 64 x 96 30.8, 128 x 128 34.6, at 1000 49.1 / 36.3; 12288 x 4096 at 200 64 x 64 46.6, 128 x 128 37.2, at 700 128 x 128 92, 128 x 192 77; 32000 x 1024 at 200 128 x 128 27.6, 128 x 256 21.2;
-// 32000 x 2048 at 512 128 x 192 79, 256 x 256 61
+// The tile that needs the least time, by rounds of 256 workgroups: 2.5 us + K / 2048 * rounds * the cost of one, in us at K 2048: 32 x 64 4.6, 64 x 64 7.2, 64 x 96 10, 64 x 128 10.5, 128 x 128 19.5, 128 x 192 26, 128 x 256 31,
+// 256 x 256 58.  The numbers are those that choose best among all tiles at 300 sizes (512 .. 32000 rows, K 1024 .. 4096, 40 .. 2048 tokens, weights from memory): 0.2 % above the quickest tile of each on the mean, 3.8 % with 6.3 and 8.5
+// for the two smaller ones and without 64 x 128.  Both sides of the crossings, us: 2048 x 2048 at 512 tokens 64 x 64 12.0, 64 x 128 15.3, at 1000 18.4 and 15.4; 2560 x 2048 at 512 64 x 96 12.6, 64 x 64 15.2; 3072 x 2048 at 1000
+// 64 x 64 24.8, 128 x 128 21.7; 12288 x 4096 at 700 64 x 96 106, 128 x 192 83; 32000 x 2048 at 512 128 x 192 79, 256 x 256 61
 static int async_tile_of(int64_t rows, int64_t K, int n_tok, int64_t seg_rows, int n_seg, int & row_blocks, int & tok_blocks, int & blocks_of) {
-    static const struct { int bn, bt; double us; } shape[] = { { 32, 64, 4.6 }, { 64, 64, 6.3 }, { 64, 96, 8.5 }, { 128, 128, 19.5 }, { 128, 192, 26.0 }, { 128, 256, 31.0 }, { 256, 256, 58.0 } };
+    static const struct { int bn, bt; double us; } shape[] = { { 32, 64, 4.6 }, { 64, 64, 7.2 }, { 64, 96, 10.0 }, { 64, 128, 10.5 }, { 128, 128, 19.5 }, { 128, 192, 26.0 }, { 128, 256, 31.0 }, { 256, 256, 58.0 } };
     int best = 0; double least = 1e30;
-    for (int i = 0; i < 7; i++) {
+    for (int i = 0; i < 8; i++) {
         const int64_t seg_blocks = seg_rows > 0 ? (seg_rows + shape[i].bn - 1) / shape[i].bn : 0, blocks = seg_rows > 0 ? (n_seg - 1) * seg_blocks + (rows - (n_seg - 1) * seg_rows + shape[i].bn - 1) / shape[i].bn : (rows + shape[i].bn - 1) / shape[i].bn;
         const int64_t toks = (n_tok + shape[i].bt - 1) / shape[i].bt, tiles = blocks * toks;
         if (tiles > INT32_MAX / 2) continue;
@@ -472,11 +472,12 @@ extern "C" int pi_op_dense_rounded(const pi_weight * w, const float * bias, cons
                      (const uint16_t *) w->p0, w->ne0, w->ne1, x, x_stride, n_tok, out, out_stride, act_a, rows_a, act_b, bias, blocks_of, seg_rows, seg_off, n_seg - 1, tok_blocks, tiles, rd, pi_abort_word())
     switch (which) {
         case 0:  DN_ASYNC(32, 64, 2, 2, 4); break;
-        case 1:  DN_ASYNC(64, 64, 4, 2, 4); break;
+        case 1:  DN_ASYNC(64, 64, 2, 2, 4); break;                       // (eight waves of 16 x 32: 1 .. 13 % more, 5 on the mean)
         case 2:  DN_ASYNC(64, 96, 2, 2, 4); break;
-        case 3:  DN_ASYNC(128, 128, 4, 2, 4); break;
-        case 4:  DN_ASYNC(128, 192, 2, 4, 3); break;
-        case 5:  DN_ASYNC(128, 256, 2, 4, 3); break;
+        case 3:  DN_ASYNC(64, 128, 2, 4, 4); break;
+        case 4:  DN_ASYNC(128, 128, 4, 2, 4); break;
+        case 5:  DN_ASYNC(128, 192, 2, 4, 3); break;
+        case 6:  DN_ASYNC(128, 256, 2, 4, 3); break;
         default: DN_ASYNC(256, 256, 4, 2, 2);
     }
 #undef DN_ASYNC
