@@ -7,12 +7,15 @@
 // v_mfma_f32_16x16x4_4b_f16 where a wave has all of them: block c of the instruction is K-slice c.
 //
 // What bounds it.  A tile of 16 rows x 16 tokens and one 256-block is 48 fma that may not be merged (32 for Q3_K, Q6_K), 4 - 16 products of the scales and its share of the weights' operands (9 instructions per lane k and
-// row group in Q4_K, 27 in Q6_K): VALU issue.  So a wave keeps CH chunks of 16 tokens (every operand it builds serves CH tiles) and, where the registers do not do for all eight lanes k of CH chunks, two waves share them
+// row group in Q4_K, 21 in Q6_K): VALU issue.  So a wave keeps CH chunks of 16 tokens (every operand it builds serves CH tiles) and, where the registers do not do for all eight lanes k of CH chunks, two waves share them
 // out (S = 2).  The steps go on across blocks without a gap: the next MFMA, the fragments AR products ahead, a part of the next operand, then the four fma of the MFMA before; loads are a block ahead (activations) and more
 // (weights), a block has one barrier, and loads take a scalar offset (buffer loads: no address arithmetic).  The kernel before walked 32 tokens in two chunks or 64 in four per launch and drained every load in flight at
 // the barrier of every block.  Measured (us for 128 tokens, before / now): Q4_K 8192 x 8192 91 / 45, 57344 x 8192 424 / 320, 8192 x 28672 279 / 162; Q6_K 8192 x 28672 303 / 212, 32000 x 8192 310 / 242; Q5_K 8192 x 8192
 // 88 / 56; Q3_K 80 / 48.  Of 45 us 5 are the launch; in the others the VALU issues in 75 % of the cycles.  Taking out the global loads, the barrier or the fragments' reads one at a time changes nothing of the 45 and 2 - 8 % of
 // the 320.
+// Q6_K's K-slices pair halves of two fragment lanes.  They are put together where the image is written: read as two halves 256 bytes apart they met in the LDS banks (41 % of the LDS' cycles, which was busy for 66 % of the launch), and
+// of the weights' operands 27 instructions were needed where the upper bits come in place and one fma takes the offset along (21).  Measured together (us, before / now): 8192 x 28672 columns 181 / 166, 32000 x 8192 205 / 196,
+// 8192 x 8192 at 64 tokens 37.4 / 35.4.  Its two products of a tile apart by a step (the second takes the first as its sum): 163, 194 and 36.7: not kept.
 #include "mmvq_args.h"
 #include <hip/hip_ext.h>
 
@@ -110,9 +113,16 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
         }
         sa = mp_load8(ax_r, a_off, bb * 1024);
     };
+    const uint32_t q6_at = (tid >> 6) * 1024 + (r + 32 * (gq >> 1)) * 16 + 8 * (gq & 1);
     auto stage_store = [&](uint8_t * img) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NL; i++) *(mp_u32x4 *) (img + (i * NTHR + tid) * 16) = st[i];
+        for (int i = 0; i < NL; i++) {
+            if constexpr (Q6) {                        // K-slice (n, hh) pairs 32-groups hh and hh + 2 of half n: the halves of two fragment lanes change places, and read_a reads 16 bytes like the others
+                uint8_t * at = img + i * NTHR * 16 + q6_at;
+                *(mp_u32x2 *) at = mp_u32x2{ st[i][0], st[i][1] };
+                *(mp_u32x2 *) (at + 256) = mp_u32x2{ st[i][2], st[i][3] };
+            } else *(mp_u32x4 *) (img + (i * NTHR + tid) * 16) = st[i];
+        }
         *(mp_u32x2 *) (img + CH * 8192 + tid * 8) = sa;
     };
     float acc[CH][KS][4], accm[CH][CS][4];
@@ -138,14 +148,12 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
     float4 dy[CH];
     float d[CH][4], nd[CH][4];
     uint32_t sc[4];                                    // the block's scales as pairs of f16: Q4_K / Q5_K S1, S2, C1, C2; Q6_K SLa, SHa, SLb, SHb; Q3_K SA, SB
+    uint32_t c6[2];                                    // Q6_K: -1536 times the second sub-block's scales
+    const uint32_t q6_sh = 4 + 2 * (gq & 1);
     float dx, dminx;
     auto read_a = [&](int m, uint32_t img) __attribute__((always_inline)) {              // fragment m = kk * CH + chunk of an image
         const uint8_t * fr = lds + img + m % CH * 8192 + (s * KS + m / CH) * 1024;
-        if constexpr (Q6) {                            // K-slice (n, hh) pairs 32-groups hh and hh + 2 of half n: one half of two fragment lanes
-            const uint32_t at = (r + 32 * (gq >> 1)) * 16 + 8 * (gq & 1);
-            const uint2 lo = *(const uint2 *) (fr + at), hi = *(const uint2 *) (fr + at + 256);
-            af[m % AR] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-        } else af[m % AR] = *(const uint4 *) (fr + lane * 16);
+        af[m % AR] = *(const uint4 *) (fr + lane * 16);
     };
     auto read_aux = [&](int ch, uint32_t img) __attribute__((always_inline)) {
         const uint8_t * aux = lds + img + CH * 8192 + ch * 1024;
@@ -162,6 +170,7 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
             if constexpr (Q6) {
                 sc[0] = mp_add(__builtin_amdgcn_perm(0x64646464u, W.rec, selA), 0xE400E400u); sc[1] = mp_fma(__builtin_amdgcn_perm(0x64646464u, W.rec2, selA), 0x4C004C00u, 0xF408F408u);
                 sc[2] = mp_fma(__builtin_amdgcn_perm(0x64646464u, W.rec, selB), 0x2C002C00u, 0xD400D400u); sc[3] = mp_add(__builtin_amdgcn_perm(0x64646464u, W.rec2, selB), 0xE408E408u);
+                c6[0] = mp_mul(sc[2], 0xE600E600u); c6[1] = mp_mul(sc[3], 0xE600E600u);
             } else {
                 sc[0] = mp_add(__builtin_amdgcn_perm(0x64646464u, W.rec, selA), 0xE420E420u); sc[1] = mp_add(__builtin_amdgcn_perm(0x64646464u, W.rec, selB), 0xE420E420u);
             }
@@ -177,9 +186,14 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
             if constexpr (Q5) { const uint32_t u = W.h[kk] >> (2 * gq + sh); f = hi ? (u & 0x00020002u) << 7 : (u & 0x00010001u) << 4; }
             o = mp_fma((q & (hi ? 0x00F000F0u : 0x000F000Fu)) | magic | f, sc[hi], sc[2 + hi]);
         } else if constexpr (Q6) {
-            const uint32_t h = W.h[kk] >> (2 * (gq & 1) + sh);
-            const uint32_t w = hi ? mp_add((q & 0x00F000F0u) | magic | ((h & 0x00300030u) << 4), 0xE600E600u) : mp_add((q & 0x000F000Fu) | magic | ((h & 0x00030003u) << 4), 0xE420E420u);
-            o = mp_mul(w, sc[2 * hi + 1]); o2 = mp_mul(w, sc[2 * hi]);
+            const uint32_t h = sh ? W.h[kk] >> q6_sh : W.h[kk] << (8 - q6_sh);         // (the two upper bits where they belong)
+            if (hi) {                                  // 16 times the weight plus 1536: one fma a part
+                const uint32_t w = (q & 0x00F000F0u) | magic | (h & 0x03000300u);
+                o = mp_fma(w, sc[3], c6[1]); o2 = mp_fma(w, sc[2], c6[0]);
+            } else {                                   // (1056 times the larger part would pass 65504)
+                const uint32_t w = mp_add((q & 0x000F000Fu) | magic | (h & 0x00300030u), 0xE420E420u);
+                o = mp_mul(w, sc[1]); o2 = mp_mul(w, sc[0]);
+            }
         } else {
             const uint32_t lo2 = W.q[kk] >> (4 * (gq & 1)), hm = W.h[kk] >> (2 * gq);      // (shared by the four dwords)
             const uint32_t u = hi ? ((lo2 >> 2) & 0x03030303u) | ((hm & 0x02020202u) << 1) : (lo2 & 0x03030303u) | ((hm & 0x01010101u) << 2);
