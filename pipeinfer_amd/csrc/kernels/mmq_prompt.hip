@@ -16,6 +16,9 @@
 // Q6_K's K-slices pair halves of two fragment lanes.  They are put together where the image is written: read as two halves 256 bytes apart they met in the LDS banks (41 % of the LDS' cycles, which was busy for 66 % of the launch), and
 // of the weights' operands 27 instructions were needed where the upper bits come in place and one fma takes the offset along (21).  Measured together (us, before / now): 8192 x 28672 columns 181 / 166, 32000 x 8192 205 / 196,
 // 8192 x 8192 at 64 tokens 37.4 / 35.4.  Its two products of a tile apart by a step (the second takes the first as its sum): 163, 194 and 36.7: not kept.
+// Where one wave has all of Q4_K's lanes k (S = 1) a launch is many rounds of workgroups that read their weights from HBM: a block is 1.2 us there, no longer than such a load takes, so the loads run two blocks ahead, with a
+// third set of registers for the weights and the image written a block earlier, from the same registers.  Measured (us, 57344 x 8192, one block / two blocks ahead): 128 tokens 289 / 272, 64 tokens 170 / 162; launches of a
+// round or two are as they were (8192 x 8192 43.7 / 43.6).  The other types and S = 2 lose (registers, steps of half the length): Q3_K 276 / 294, Q5_K 333 / 336, Q6_K 32000 x 8192 192 / 197.
 #include "mmvq_args.h"
 #include <hip/hip_ext.h>
 
@@ -65,6 +68,7 @@ template <int TYPE, int S, int RG, int CH>
 static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, const int group_end, const int group0, const int tb) {
     constexpr bool Q5 = TYPE == PI_Q5_K, Q6 = TYPE == PI_Q6_K, Q3 = TYPE == PI_Q3_K, Q4 = TYPE == PI_Q4_K;
     constexpr uint32_t TILE = Q6 ? PI_MQ_TILE_Q6 : Q5 ? PI_MQ_TILE_Q5 : Q3 ? PI_MQ_TILE_Q3 : PI_MQ_TILE, QOFF = Q6 ? 1600 : (Q5 || Q3) ? 832 : 320, QPART = Q3 ? 512 : 1024;
+    constexpr bool FAR = Q4 && S == 1;                 // loads run two blocks ahead
     constexpr int KS = 8 / S, CS = Q4 ? 4 / S : 1, NTHR = 64 * S * RG, NL = CH * 512 / NTHR, IMG = CH * 8192 + NTHR * 8;      // IMG: LDS image of one block: fragments of CH chunks, then their aux (and what the threads past it write)
     static_assert(S == 1 || S == 2, "one or two waves a row group");
     static_assert((512 % NTHR == 0) && CH * 128 <= NTHR, "whole strips of 16-byte units; eight bytes of aux a thread");
@@ -104,7 +108,7 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
     const int chunks = nch - ch0 < CH ? nch - ch0 : CH;
     const __amdgpu_buffer_rsrc_t fr_r = mp_rsrc(g.frag + (size_t) ch0 * nb * 8192, (uint32_t) chunks * nb * 8192), ax_r = mp_rsrc(g.aux + (size_t) ch0 * nb * 1024, (uint32_t) chunks * nb * 1024);
     const uint32_t a_off = ((tid >> 7) < chunks ? tid >> 7 : chunks - 1) * (nb * 1024) + (tid & 127) * 8;
-    auto stage_load = [&](int b) __attribute__((always_inline)) {
+    auto stage_load = [&](int b, mp_u32x4 * st, mp_u32x2 & sa) __attribute__((always_inline)) {
         const int bb = b < nb ? b : nb - 1;
 #pragma unroll
         for (int i = 0; i < NL; i++) {
@@ -114,7 +118,7 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
         sa = mp_load8(ax_r, a_off, bb * 1024);
     };
     const uint32_t q6_at = (tid >> 6) * 1024 + (r + 32 * (gq >> 1)) * 16 + 8 * (gq & 1);
-    auto stage_store = [&](uint8_t * img) __attribute__((always_inline)) {
+    auto stage_store = [&](uint8_t * img, const mp_u32x4 * st, mp_u32x2 sa) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < NL; i++) {
             if constexpr (Q6) {                        // K-slice (n, hh) pairs 32-groups hh and hh + 2 of half n: the halves of two fragment lanes change places, and read_a reads 16 bytes like the others
@@ -217,14 +221,14 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
         else c.v = mp_mfma(a, bw[p & 1], z);
         return c;
     };
-    mp_w<TYPE, KS> W0, W1;
+    mp_w<TYPE, KS> W0, W1, W2;
     result c;
     // block b: image `img`, weights W; the next block's: img1, Wn.  Its one barrier is in its middle: image img1, written ahead of it, may then be read.
-    // Three images: waves on either side of a barrier read images b - 1 and b, and write b + 1 (b - 2's readers left it before the barrier of b - 1)
+    // Three images: waves on either side of a barrier read images b - 1 and b, and write b + 1 (b - 2's readers left it before the barrier of b - 1).
+    // Two blocks ahead, block b writes image b + 2 at its end: the readers of b - 1, which was there, left it before the barrier of b
     uint32_t img = 0, img1 = IMG, img2 = 2 * IMG;
     auto block = [&](int b, mp_w<TYPE, KS> & W, mp_w<TYPE, KS> & Wn) __attribute__((always_inline)) {
-        stage_store(lds + img1);
-        stage_load(b + 2);
+        if constexpr (!FAR) { stage_store(lds + img1, st, sa); stage_load(b + 2, st, sa); }
 #pragma unroll
         for (int n = 0; n < PS * CH; n++) {
             const int p = n / CH, ch = n % CH;
@@ -250,7 +254,10 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
                     if (p + 1 < KS) build(W, p + 1 < KS ? p + 1 : 0, i);
                     else if (p + 1 == PS) build(Wn, 0, i);
                 }
-            if (n == (PS - 1) * CH) load_w(b + 2, W);                                   // (its last use is behind us)
+            if (n == (PS - 1) * CH) {                                                   // (W's last use is behind us)
+                if constexpr (FAR) { stage_store(lds + img2, st, sa); stage_load(b + 3, st, sa); }
+                load_w(b + (FAR ? 3 : 2), W);
+            }
             const result o = c;
             const mp_f32x4 v = o.v;
             c = n + 1 < PS * CH ? product((n + 1) / CH, (n + 1) % CH) : product(0, 0);
@@ -276,11 +283,24 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
         }
         const uint32_t t = img; img = img1; img1 = img2; img2 = t;
     };
-    stage_load(0);
-    load_w(0, W0);
-    stage_store(lds);
-    stage_load(1);
-    load_w(1, W1);
+    if constexpr (FAR) {
+        mp_u32x4 st0[NL], st1[NL];
+        mp_u32x2 sa0, sa1;
+        stage_load(0, st0, sa0);
+        load_w(0, W0);
+        stage_load(1, st1, sa1);
+        load_w(1, W1);
+        stage_load(2, st, sa);
+        load_w(2, W2);
+        stage_store(lds, st0, sa0);
+        stage_store(lds + IMG, st1, sa1);
+    } else {
+        stage_load(0, st, sa);
+        load_w(0, W0);
+        stage_store(lds, st, sa);
+        stage_load(1, st, sa);
+        load_w(1, W1);
+    }
     mp_barrier<0>();
 #pragma unroll
     for (int m = 0; m < AR; m++) read_a(m, 0);
@@ -292,8 +312,14 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
     for (int i = 0; i < 4; i++) build(W0, 0, i);
     c = product(0, 0);
     int b = 0;
-    for (; b + 1 < nb; b += 2) { block(b, W0, W1); block(b + 1, W1, W0); }
-    if (b < nb) block(b, W0, W1);
+    if constexpr (FAR) {
+        __builtin_amdgcn_s_waitcnt(0x0f70);            // vmcnt(0): the loop's waits count the loads of its own order alone
+        for (; b + 2 < nb; b += 3) { block(b, W0, W1); block(b + 1, W1, W2); block(b + 2, W2, W0); }
+        if (b < nb) { block(b, W0, W1); if (b + 1 < nb) block(b + 1, W1, W2); }
+    } else {
+        for (; b + 1 < nb; b += 2) { block(b, W0, W1); block(b + 1, W1, W0); }
+        if (b < nb) block(b, W0, W1);
+    }
     // ---- fold: hsum_float_8 = ((a0 + a4) + (a2 + a6)) + ((a1 + a5) + (a3 + a7)), mins ((m0 + m2) + (m1 + m3)) ----
     constexpr int XN = KS + CS;                                                        // S = 2: a wave's chains of the chunks that the other one finishes (ch % 2 == its s), [chunk / 2][i][XN][64]
     float * X = (float *) lds + (size_t) wave * ((CH + 1) / 2 * 4 * XN * 64);
@@ -314,18 +340,19 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
     }
     if (!active) return;
     const float * Y = (const float *) lds + (size_t) (wave ^ 1) * ((CH + 1) / 2 * 4 * XN * 64);
-    const int64_t row = row0 + r;
+    const int el = (int) __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), er = el & 15;      // (the lane, asked for again: its registers are the loop's)
+    const int64_t row = row0 + er;
     const bool mine = row < sg.M;
 #pragma unroll
     for (int ch = 0; ch < CH; ch++) {
         if (S == 2 && (ch & 1) != s) continue;
-        const int t0 = (ch0 + ch) * 16 + 4 * gq;
+        const int t0 = (ch0 + ch) * 16 + 4 * (el >> 4);
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             float a[8], m[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
             if constexpr (S == 2) {
-                const float * y = Y + ((ch >> 1) * 4 + i) * XN * 64 + lane;
+                const float * y = Y + ((ch >> 1) * 4 + i) * XN * 64 + el;
 #pragma unroll
                 for (int kk = 0; kk < KS; kk++) { const float o = y[kk * 64]; a[kk] = s == 0 ? acc[ch][kk][i] : o; a[KS + kk] = s == 0 ? o : acc[ch][kk][i]; }
                 if constexpr (Q4) for (int cc = 0; cc < CS; cc++) { const float o = y[(KS + cc) * 64]; m[cc] = s == 0 ? accm[ch][cc][i] : o; m[CS + cc] = s == 0 ? o : accm[ch][cc][i]; }
@@ -357,7 +384,7 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
                 if (mine && t0 + i < nt) {
                     const int tok = g.tok0 + t0 + i;
                     const float2 cs = *(const float2 *) (g.rope_cs + ((int64_t) g.pos[tok] * (g.hd / 2) + j) * 2);
-                    const float y = (r & 1) ? mate * cs.y + v[i] * cs.x : v[i] * cs.x - mate * cs.y;
+                    const float y = (er & 1) ? mate * cs.y + v[i] * cs.x : v[i] * cs.x - mate * cs.y;
                     sg.dst16[(int64_t) (sg.store == 2 ? pi_cell_of(g.dyn, g.kv_head, tok) : tok) * sg.stride16 + row] = pi_f2h(y);
                 }
             }

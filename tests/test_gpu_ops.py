@@ -206,6 +206,18 @@ def test_mul_mat_k_quants_prompt(gpu, t, k, rows, n_tok):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("blocks_a_row", [1, 2, 3, 4, 5, 6, 7])
+def test_mul_mat_q4_k_prompt_two_blocks_ahead(gpu, blocks_a_row):
+    """k_mmq_prompt's tiles of one wave a row group of Q4_K (8190 rows x 125 tokens), whose loop takes three blocks a turn and loads two ahead: every remainder, fewer blocks than it loads - the reference's bits"""
+    lib, U = gpu
+    k, rows, n_tok = 256 * blocks_a_row, 8190, 125
+    blocks = synth.random_blocks(O.Q4_K, rows * k, np.random.default_rng(k), 0.05).reshape(rows, -1)
+    act = np.stack([signal(k, s) for s in range(n_tok)])
+    w = upload_weight(lib, O.Q4_K, rows, k, blocks)
+    assert np.array_equal(gpu_mul_mat(lib, U, O.Q4_K, w, k, rows, act).view(np.uint32), O.Impl("oracle").mul_mat(O.Q4_K, blocks, k, rows, act).view(np.uint32))
+    lib.pi_weight_free(w)
+
+
 @pytest.mark.parametrize("k,rows", [(4096, 40), (4096, 2048), (4096, 2049), (4064, 40)])
 def test_mul_mat_q4_0_nine_tokens(gpu, k, rows):
     """nine tokens, where the mat-vec would take a second pass over the weights (k_mmq_q0 takes them, as it does all from seven), around 2048 rows of 4096 values and a row of whole groups less one block: the reference's bits"""
