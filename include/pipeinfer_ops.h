@@ -179,6 +179,11 @@ PI_API int pi_op_clamp(float * x_dev, float lo, float hi, int64_t n, void * stre
 /* per token: ids/logits of the k largest (logit desc, id asc), max logit and sum_i expf(l_i - max) over the full vocab */
 PI_API size_t pi_op_topk_scratch_bytes(int n_tok);                  /* caller-owned scratch, one per stream */
 PI_API int pi_op_topk(const float * logits_dev, int n_vocab, int n_tok, int k, int32_t * ids_dev, float * vals_dev, float * sumexp_dev, void * scratch_dev, void * stream);
+/* its two launches apart: the bests of every row's slices into the scratch; rows of them merged (scratch_dev + pi_op_topk_scratch_bytes(row0): from row0 on, k = 8) */
+PI_API int pi_op_topk_parts(const float * logits_dev, int n_vocab, int n_tok, int k, void * scratch_dev, void * stream);
+PI_API int pi_op_topk_merge(const void * scratch_dev, int n_tok, int k, int32_t * ids_dev, float * vals_dev, float * sumexp_dev, void * stream);
+/* the merge (k = 8) of rows [row0, row0 + n_tok) and n_logits values of the logits in one launch, into the caller's PAGE-LOCKED host buffers (as pi_op_copy_out writes them) */
+PI_API int pi_op_topk_out(const void * scratch_dev, int row0, int n_tok, int32_t * ids_host, float * vals_host, float * sum_host, const float * logits_dev, float * logits_host, int64_t n_logits, void * stream);
 
 /* ---- dense bfloat16 matrices and the operators of hybrid blocks (recurrent / low-rank-attention mixers, routed feed-forwards) --------------------------------------
  * Weights are PI_BF16 pi_weights ([rows][K] as stored, pi_weight_upload(PI_BF16, K, rows, ...)); activations, norms, scores, states and outputs are fp32.

@@ -514,7 +514,7 @@ static bool forward_pre_post_blocks(llama_context * ctx, int n_tok, int n_kv) {
     }
     OP_OK(dense(ctx, hp.own_head ? m->output : m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
     if (hp.logit_softcap > 0.0f) OP_OK(pi_op_softcap(ctx->logits_dev, (int64_t) n_tok * hp.n_vocab, hp.logit_softcap, s));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -619,7 +619,7 @@ static bool forward_post_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
     OP_OK(dense(ctx, m->output, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, xh, width));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -709,7 +709,7 @@ static bool forward_shared_norm_blocks(llama_context * ctx, int n_tok, int n_kv)
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
     OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -818,7 +818,7 @@ static bool forward_stream_blocks(llama_context * ctx, int n_tok, int n_kv) {
         trace(ctx, "lout", (int) il, X, (int64_t) ns * width, n_tok);
     }
     OP_OK(dense(ctx, m->output, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -896,7 +896,7 @@ static bool forward_pre_norm_blocks(llama_context * ctx, int n_tok, int n_kv) {
         OP_OK(step_to(il + 1, Y));
     }
     OP_OK(dense(ctx, m->tok_embd, N, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, nh, width));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -966,7 +966,7 @@ static bool forward_hybrid(llama_context * ctx, int n_tok, int n_kv) {
         trace(ctx, "lout", (int) il, x, width, n_tok);
     }
     OP_OK(dense(ctx, m->tok_embd, ctx->nx, width, n_tok, ctx->logits_dev, hp.n_vocab, PI_ACT_NONE, hp.n_vocab, PI_ACT_NONE, s, nh, width));
-    OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+    OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     return true;
 }
 
@@ -1116,7 +1116,7 @@ static bool forward(llama_context * ctx, int n_tok, int kv_head, int n_kv, int l
         if (hp.arch == PI_ARCH_LLAMA || (hp.generic() && hp.block.rms)) { if (!norm_for(ctx, x, m->output_norm, nullptr, n_embd, n_tok, hp.f_norm_rms_eps, 1, vo, ctx->q8a)) return false; }
         else                                                              { if (!norm_for(ctx, x, m->output_norm, m->output_norm_b, n_embd, n_tok, hp.f_norm_eps, 0, vo, ctx->q8a)) return false; }
         OP_OK(pi_op_mul_mat(m->output, ctx->q8a, n_tok, ctx->logits_dev, nullptr, s));
-        OP_OK(pi_op_topk(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_ids_dev, ctx->topk_vals_dev, ctx->topk_sum_dev, ctx->topk_scratch_dev, s));
+        OP_OK(pi_op_topk_parts(ctx->logits_dev, hp.n_vocab, n_tok, 8, ctx->topk_scratch_dev, s));
     }
     return true;
 }
@@ -1219,11 +1219,15 @@ static bool launch_segment(llama_context * ctx, int n_tokens, int kv_head, int s
     return fwd;
 }
 static bool outputs_by_memcpy() { static const bool on = getenv("PIPEINFER_COPY_OUT") && !strcmp(getenv("PIPEINFER_COPY_OUT"), "memcpy"); return on; }
+// the top 8 of rows [row0, row0 + n) where copies take them from (launch_outputs' kernel merges into the run's buffers by itself)
+static bool topk_to_device(llama_context * ctx, int row0, int n) {
+    return pi_op_topk_merge((const char *) ctx->topk_scratch_dev + pi_op_topk_scratch_bytes(row0), n, 8, ctx->topk_ids_dev + (size_t) row0 * 8, ctx->topk_vals_dev + (size_t) row0 * 8, ctx->topk_sum_dev + row0, ctx->stream) == 0;
+}
 static bool launch_outputs(llama_context * ctx, pi_run * run) {
     if (!ctx->is_last) return true;
     hipStream_t s = ctx->stream;
     const size_t nv = ctx->model->hparams.n_vocab, r0 = (size_t) run->row0; const int n_tokens = run->n_tokens;
-    // by a kernel that writes the run's page-locked buffers (pi_op_copy_out: a copy-engine transfer waits for the OTHER context's kernels); PIPEINFER_COPY_OUT=memcpy: plain copies of all rows
+    // by a kernel that writes the run's page-locked buffers (pi_op_topk_out: a copy-engine transfer waits for the OTHER context's kernels); PIPEINFER_COPY_OUT=memcpy: plain copies of all rows
     if (!outputs_by_memcpy() && !run->host_plain) {
         // the rows that phase 1 hands back (all of them for a tap): consecutive ones in one launch, the first launch brings the top-8 of every row.  A 512-token prompt that wants its last row brings
         // 128 KB over the bus instead of 65 MB (1.2 ms at the bus's 56 GB/s, a fifth of such a pass)
@@ -1238,17 +1242,16 @@ static bool launch_outputs(llama_context * ctx, pi_run * run) {
             first = false;
             float * to = run->logits_host + (size_t) (run->compact ? at : a) * nv;
             at += b - a;
-            return pi_op_copy_out(ctx->logits_dev + (r0 + (size_t) a) * nv, to, (int64_t) (b - a) * (int64_t) nv, ctx->topk_ids_dev + r0 * 8, run->topk_ids, ctx->topk_vals_dev + r0 * 8,
-                                  run->topk_vals, ctx->topk_sum_dev + r0, run->topk_sum, tops, s) == 0;
+            return pi_op_topk_out(ctx->topk_scratch_dev, run->row0, tops, run->topk_ids, run->topk_vals, run->topk_sum, ctx->logits_dev + (r0 + (size_t) a) * nv, to, (int64_t) (b - a) * (int64_t) nv, s) == 0;
         };
         bool ok = true;
         if (ranges == 0) ok = copy(0, 0);
         else if (whole) ok = copy(low, high);
         else for (int a = low; a < high && ok; a++) if (wanted(a)) { int b = a + 1; while (b < high && wanted(b)) b++; ok = copy(a, b); a = b; }
-        if (!ok) { ctx->last_error = std::string("pi_op_copy_out: ") + pi_last_error(); return false; }
+        if (!ok) { ctx->last_error = std::string("pi_op_topk_out: ") + pi_last_error(); return false; }
         return true;
     }
-    const bool ok = hipMemcpyAsync(run->logits_host, ctx->logits_dev + r0 * nv, (size_t) 4 * n_tokens * nv, hipMemcpyDeviceToHost, s) == hipSuccess &&
+    const bool ok = topk_to_device(ctx, run->row0, n_tokens) && hipMemcpyAsync(run->logits_host, ctx->logits_dev + r0 * nv, (size_t) 4 * n_tokens * nv, hipMemcpyDeviceToHost, s) == hipSuccess &&
                     hipMemcpyAsync(run->topk_ids, ctx->topk_ids_dev + r0 * 8, (size_t) 4 * n_tokens * 8, hipMemcpyDeviceToHost, s) == hipSuccess &&
                     hipMemcpyAsync(run->topk_vals, ctx->topk_vals_dev + r0 * 8, (size_t) 4 * n_tokens * 8, hipMemcpyDeviceToHost, s) == hipSuccess &&
                     hipMemcpyAsync(run->topk_sum, ctx->topk_sum_dev + r0, (size_t) 4 * n_tokens, hipMemcpyDeviceToHost, s) == hipSuccess;
@@ -1788,7 +1791,7 @@ int stage_run(llama_context * ctx, int n_tokens, const void * meta, size_t meta_
     // ... and the consumer's arrival flag right behind them (with the abort this run ended with: a run cut short here must not be computed downstream either)
     if (ok && flag_out && pi_op_flag_publish(hop->out_flag, hop->out_ticket, ctx->abort_dev, cut ? 1 : 0, s) != 0) { ctx->last_error = std::string("pi_op_flag_publish: ") + pi_last_error(); ok = false; }
     if (ok && !cut && ctx->is_last)
-        ok = hipMemcpyAsync(logits_host, ctx->logits_dev, (size_t) 4 * n_tokens * nv, hipMemcpyDeviceToHost, s) == hipSuccess &&
+        ok = topk_to_device(ctx, 0, n_tokens) && hipMemcpyAsync(logits_host, ctx->logits_dev, (size_t) 4 * n_tokens * nv, hipMemcpyDeviceToHost, s) == hipSuccess &&
              hipMemcpyAsync(topk_ids, ctx->topk_ids_dev, (size_t) 4 * n_tokens * 8, hipMemcpyDeviceToHost, s) == hipSuccess &&
              hipMemcpyAsync(topk_vals, ctx->topk_vals_dev, (size_t) 4 * n_tokens * 8, hipMemcpyDeviceToHost, s) == hipSuccess &&
              hipMemcpyAsync(topk_sum, ctx->topk_sum_dev, (size_t) 4 * n_tokens, hipMemcpyDeviceToHost, s) == hipSuccess;
@@ -1878,6 +1881,7 @@ int stage_run_pass(llama_context * ctx, int n_members, const void * const * meta
     const size_t nv = ctx->model->hparams.n_vocab;
     if (ok && !cut) {
         size_t r0 = 0;
+        ok = topk_to_device(ctx, 0, n);
         for (int i = 0; ok && i < n_members; i++) {                            // every member's rows into its own result slot
             const size_t m = (size_t) n_tokens[i];
             ok = hipMemcpyAsync(logits_host[i], ctx->logits_dev + r0 * nv, 4 * m * nv, hipMemcpyDeviceToHost, s) == hipSuccess &&

@@ -683,7 +683,7 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // plus max and sum_i expf(l_i - max) so p_j = expf(l_j - max) / sum on the host.
 // =================================================================================================================
 // stage 1: grid (n_tok, NCH) — each workgroup finds the k best of its slice of the vocabulary and its partial max / sum-exp
-// stage 2: one workgroup per token merges NCH*k candidates (same ordering) and the partial sums.
+// stage 2: one wave per token merges NCH*k candidates (same ordering) and the partial sums; at the end of a pass beside the rows' way out (k_topk_out).
 #define TOPK_NCH 32
 // What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One way
 // to go on is a round for each of the k, two wave reductions and one rescan of the lane that lost its best.  The other, for one wave to a slice and many rounds (the rule is at the launch): the least of eight lane groups' bests
@@ -704,8 +704,10 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
     pi_butterfly<32>([&](auto o) { i = min(i, pi_partner<decltype(o)::value>(i)); });
     key = m; id = i;
 }
+// a row's share of the scratch: the k best of every slice (ids, values), the slices' maxima and sums
+static __host__ __device__ __forceinline__ int topk_words(int k) { return TOPK_NCH * (2 * k + 2); }
 template <int VPT, int WS>
-__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int candidates, int32_t * __restrict__ cid, float * __restrict__ cval, float * __restrict__ cmax, float * __restrict__ csum, const int32_t * __restrict__ abort_w) {
+__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int candidates, int32_t * __restrict__ part, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
     constexpr int MET = WS > 1 ? 32 : 256;                              // the four waves' bests; a wave's own candidates
@@ -713,6 +715,7 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per), own0 = lo + lane + (WS > 1 ? 64 * wave : 0);
     const float * l = logits + (int64_t) t * n_vocab;
+    int32_t * cid = part + (int64_t) t * topk_words(k); float * cval = (float *) (cid + TOPK_NCH * k), * cmax = cval + TOPK_NCH * k, * csum = cmax + TOPK_NCH;
     uint32_t key[VPT > 0 ? VPT : 1]; float rv[VPT > 0 ? VPT : 1];
     uint32_t bk = 0; int bm = 0;                                        // this lane's best among the ones not taken: key, number
     if constexpr (VPT > 0) {
@@ -746,9 +749,9 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     if constexpr (WS == 1) {
 #pragma unroll
         for (int w = 0; w < 4; w++) s[w] = pi_lanes_sum<64>(s[w]);
-        if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (s[0] + s[1]) + (s[2] + s[3]); }
+        if (lane == 0) { cmax[ch] = first; csum[ch] = (s[0] + s[1]) + (s[2] + s[3]); }
     } else { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; }
-    const int64_t out = ((int64_t) t * TOPK_NCH + ch) * k;
+    const int out = ch * k;
     if constexpr (WS == 1) if (candidates) {
         // what is not below `low` goes to a lane each, which counts those ahead of it
         const uint32_t least = max(low, 1u);
@@ -775,7 +778,7 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
                 const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(ci, j);
                 ahead += kj > ck || (kj == ck && ij < ci);
             }
-            if (lane < n ? ahead < k : lane < k) { const int64_t at = out + (lane < n ? ahead : lane); cid[at] = ci; cval[at] = cv; }
+            if (lane < n ? ahead < k : lane < k) { const int at = out + (lane < n ? ahead : lane); cid[at] = ci; cval[at] = cv; }
             return;
         }
         topk_best(wk, wi);
@@ -812,27 +815,59 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
             if (lane == r) own = wi;
             if (mi == wi) mk = 0;
         }
-        if (lane == 0) { cmax[t * TOPK_NCH + ch] = first; csum[t * TOPK_NCH + ch] = (met_sum[0] + met_sum[1]) + (met_sum[2] + met_sum[3]); }
+        if (lane == 0) { cmax[ch] = first; csum[ch] = (met_sum[0] + met_sum[1]) + (met_sum[2] + met_sum[3]); }
     }
     if (lane < k) { cid[out + lane] = own; cval[out + lane] = own != 0x7fffffff ? l[own] : -INFINITY; }
 }
-__global__ void __launch_bounds__(64) k_topk2(int k, const int32_t * __restrict__ cid, const float * __restrict__ cval, const float * __restrict__ cmax, const float * __restrict__ csum,
-                                               int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int32_t * __restrict__ abort_w) {
-    const int gone = pi_abort_peek(abort_w);
-    const int t = blockIdx.x, lane = threadIdx.x;
-    const int n = TOPK_NCH * k;                                        // <= 256: four candidates per lane
+// one wave merges a row's slices: ids[k], vals[k] and the sum (device or page-locked memory).  A serial chain: rounds of two reductions each (0.25 us) it was, now the floor, ballot and count of k_topk1 - lane groups that hold
+// whole slices, so that the floor is the least of eight groups' bests and few reach it; a crowd of equal values takes the rounds
+struct topk_merge_lds { uint32_t key[64], id[64]; float val[64]; };
+static __device__ __forceinline__ void topk_merge(int k, const int32_t * __restrict__ cid, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int lane, topk_merge_lds & M) {
+    const float * cval = (const float *) (cid + TOPK_NCH * k), * cmax = cval + TOPK_NCH * k, * csum = cmax + TOPK_NCH;
+    const int n = TOPK_NCH * k;                                         // <= 256: four candidates per lane
     float cv[4]; int ci[4]; uint32_t key[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) { const int i = lane + 64 * j; cv[j] = i < n ? cval[(int64_t) t * n + i] : -INFINITY; ci[j] = i < n ? cid[(int64_t) t * n + i] : 0x7fffffff; key[j] = ci[j] != 0x7fffffff ? topk_key(cv[j]) : 0u; }
-    const float pm = lane < TOPK_NCH ? cmax[t * TOPK_NCH + lane] : -INFINITY, ps = lane < TOPK_NCH ? csum[t * TOPK_NCH + lane] : 0.0f;
-    if (pi_abort_late(gone, abort_w)) return;
-    for (int r = 0; r < k; r++) {
+    for (int j = 0; j < 4; j++) { const int i = 4 * lane + j; cv[j] = i < n ? cval[i] : -INFINITY; ci[j] = i < n ? cid[i] : 0x7fffffff; }
+    const float pm = lane < TOPK_NCH ? cmax[lane] : -INFINITY, ps = lane < TOPK_NCH ? csum[lane] : 0.0f;
+    uint32_t top = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) { key[j] = ci[j] != 0x7fffffff ? topk_key(cv[j]) : 0u; top = max(top, key[j]); }
+    // eight groups of eight lanes: lanes of the same bits 1 .. 3 (a slice of eight candidates is two lanes)
+    top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<1>((int) top));
+    uint32_t least = top;
+    least = min(least, (uint32_t) pi_partner<8>((int) least)); least = min(least, (uint32_t) pi_partner<4>((int) least)); least = min(least, (uint32_t) pi_partner<2>((int) least));
+    least = max(least, 1u);
+    uint64_t who[4]; int m = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) { who[j] = __ballot(key[j] >= least); m += __popcll(who[j]); }
+    if (m <= 64) {
+        int base = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (key[j] >= least) {
+                const int at = base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[j], 0));
+                M.key[at] = key[j]; M.id[at] = (uint32_t) ci[j]; M.val[at] = cv[j];
+            }
+            base += __popcll(who[j]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t ck = lane < m ? M.key[lane] : 0u; const int id = lane < m ? (int) M.id[lane] : 0x7fffffff;
+        const float val = lane < m ? M.val[lane] : -INFINITY;
+        int ahead = 0;
+#pragma unroll 4
+        for (int j = 0; j < m; j++) {
+            const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(id, j);
+            ahead += kj > ck || (kj == ck && ij < id);
+        }
+        if (lane < m ? ahead < k : lane < k) { const int at = lane < m ? ahead : lane; ids[at] = id; vals[at] = val; }
+    } else for (int r = 0; r < k; r++) {
         uint32_t bk = 0; int bi = 0x7fffffff; float bv = -INFINITY;     // this lane's best
 #pragma unroll
         for (int j = 0; j < 4; j++) if (key[j] > bk || (key[j] == bk && bk != 0 && ci[j] < bi)) { bk = key[j]; bi = ci[j]; bv = cv[j]; }
         uint32_t wk = bk; int wi = bi;
         topk_best(wk, wi);
-        if (wk == 0 ? lane == 0 : wi == bi) { ids[t * k + r] = wi; vals[t * k + r] = bv; }      // (an id is in one lane only)
+        if (wk == 0 ? lane == 0 : wi == bi) { ids[r] = wi; vals[r] = bv; }      // (an id is in one lane only)
 #pragma unroll
         for (int j = 0; j < 4; j++) if (ci[j] == wi) key[j] = 0;
     }
@@ -840,27 +875,60 @@ __global__ void __launch_bounds__(64) k_topk2(int k, const int32_t * __restrict_
     float mx = pi_wave_max(pm);
     float s = (lane < TOPK_NCH && pm != -INFINITY) ? ps * expf(pm - mx) : 0.0f;
     s = pi_lanes_sum<64>(s);
-    if (lane == 0) sumexp[t] = s;
+    if (lane == 0) *sumexp = s;
+}
+__global__ void __launch_bounds__(256) k_topk2(int k, int n_tok, const int32_t * __restrict__ part, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int32_t * __restrict__ abort_w) {
+    if (pi_aborted(abort_w)) return;
+    __shared__ topk_merge_lds M[4];
+    const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+    if (t < n_tok) topk_merge(k, part + (int64_t) t * topk_words(k), ids + (int64_t) t * k, vals + (int64_t) t * k, sumexp + t, threadIdx.x & 63, M[wave]);
+}
+// The end of a pass: rows of logits to the run's page-locked buffer and, beside them, the merge of its rows' slices, which writes the run's buffers itself.  The first workgroups merge (four rows each), the others copy.
+// One launch for what was k_topk2 in front of k_copy_out: the merge is a chain, the copy the bus (a row of 32000: 128 KB).  Measured (us, vocabulary 32000, apart / together): one row 5.8 + 4.6 / 5.6, eight rows 6.7 + 19.1 / 19.4.
+// What it writes for a cancelled run is dropped, so it does not look at the abort word (k_copy_out does not either)
+__global__ void __launch_bounds__(256) k_topk_out(const int32_t * __restrict__ part, int n_tok, int merges, int32_t * __restrict__ ids_h, float * __restrict__ vals_h, float * __restrict__ sum_h, const float * __restrict__ logits, float * __restrict__ logits_h, size_t n_logits) {
+    __shared__ topk_merge_lds M[4];
+    if ((int) blockIdx.x < merges) {
+        const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+        if (t < n_tok) topk_merge(8, part + (int64_t) t * topk_words(8), ids_h + (int64_t) t * 8, vals_h + (int64_t) t * 8, sum_h + t, threadIdx.x & 63, M[wave]);
+        return;
+    }
+    pi_rows_out(logits, logits_h, n_logits, (size_t) (blockIdx.x - merges) * 256 + threadIdx.x, (size_t) (gridDim.x - merges) * 256);
 }
 
 // bytes of caller-owned scratch pi_op_topk needs for n_tok rows (one buffer per stream: contexts decode concurrently)
 extern "C" size_t pi_op_topk_scratch_bytes(int n_tok) { return (size_t) n_tok * TOPK_NCH * (2 * 8 + 2) * 4; }
-extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * scratch, void * stream) {
+// the slices' bests of every row, left in the scratch for pi_op_topk_merge or pi_op_topk_out
+extern "C" int pi_op_topk_parts(const float * logits, int n_vocab, int n_tok, int k, void * scratch, void * stream) {
     if (n_tok <= 0) return 0;
     if (k > 8) { pi_set_error("pi_op_topk: k=%d > 8", k); return -1; }
     if (!scratch) { pi_set_error("pi_op_topk: scratch is NULL (needs pi_op_topk_scratch_bytes(n_tok) bytes)"); return -1; }
-    int32_t * cid = (int32_t *) scratch; float * cval = (float *) (cid + (size_t) n_tok * TOPK_NCH * k);
-    float * cmax = cval + (size_t) n_tok * TOPK_NCH * k, * csum = cmax + (size_t) n_tok * TOPK_NCH;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
     // One wave to a slice: candidates cost the same for every k, rounds some 0.8 us each of them, and 1 / 3 us less at the start of 64 / 256 rows.  us by rounds / candidates, vocabulary 32000: 512 rows k = 1 20.1 / 28.7,
     // 4 30.6 / 30.2, 5 34.3 / 30.8, 8 44.5 / 32.5; 256 rows k = 5 21.0 / 20.6; 128 rows k = 6 15.0 / 15.0, 7 16.3 / 15.5; 64 rows k = 7 12.6 / 13.2; k = 8 of one row 12.7 / 11.4, 6 rows 13.4 / 13.1, 16 11.7 / 12.7,
     // 32 11.9 / 12.8, 48 13.5 / 13.6; of 65536 8 rows 15.6 / 14.7, 16 14.8 / 15.0
     const int candidates = n_tok >= 256 ? k >= 5 : n_tok >= 128 ? k >= 7 : k == 8 && (n_tok <= (per > 1024 ? 12 : 7) || n_tok > 32);
-#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, candidates, cid, cval, cmax, csum, pi_abort_word())
+#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, candidates, (int32_t *) scratch, pi_abort_word())
     if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4);
     else if (per <= 64 * 8) TOPK_GO(8, 1); else if (per <= 64 * 16) TOPK_GO(16, 1); else if (per <= 64 * 32) TOPK_GO(32, 1);
     else if (per <= 256 * 16) TOPK_GO(16, 4); else if (per <= 256 * 32) TOPK_GO(32, 4); else TOPK_GO(0, 4);
 #undef TOPK_GO
-    PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2, dim3(n_tok), dim3(64), 0, (hipStream_t) stream, k, cid, cval, cmax, csum, ids, vals, sumexp, pi_abort_word());
+    PI_CHECK_LAUNCH(); return 0;
+}
+extern "C" int pi_op_topk_merge(const void * scratch, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * stream) {
+    if (n_tok <= 0) return 0;
+    PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2, dim3((n_tok + 3) / 4), dim3(256), 0, (hipStream_t) stream, k, n_tok, (const int32_t *) scratch, ids, vals, sumexp, pi_abort_word());
+    PI_CHECK_LAUNCH(); return 0;
+}
+extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * scratch, void * stream) {
+    const int rc = pi_op_topk_parts(logits, n_vocab, n_tok, k, scratch, stream);
+    return rc != 0 ? rc : pi_op_topk_merge(scratch, n_tok, k, ids, vals, sumexp, stream);
+}
+// rows [row0, row0 + n_tok) of a pass whose pi_op_topk_parts took k = 8
+extern "C" int pi_op_topk_out(const void * scratch, int row0, int n_tok, int32_t * ids_host, float * vals_host, float * sum_host, const float * logits_dev, float * logits_host, int64_t n_logits, void * stream) {
+    const int merges = (n_tok + 3) / 4;
+    const unsigned copies = (unsigned) std::min<int64_t>(256, (n_logits + 4095) / 4096);                       // four 16-byte stores per thread
+    if (merges + copies == 0) return 0;
+    hipLaunchKernelGGL(k_topk_out, dim3(merges + copies), dim3(256), 0, (hipStream_t) stream, (const int32_t *) scratch + (size_t) row0 * topk_words(8), n_tok, merges, ids_host, vals_host, sum_host, logits_dev, logits_host, (size_t) n_logits);
     PI_CHECK_LAUNCH(); return 0;
 }

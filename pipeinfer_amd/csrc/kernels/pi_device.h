@@ -112,6 +112,16 @@ static __device__ __forceinline__ bool pi_aborted_together(int peek, const int32
 // A run's tokens sit in consecutive cells from kv_head (find_slot, llama.cpp:1593-1644); a pass that carries several runs at once (context.cpp: coalescing) brings a table.
 static __device__ __forceinline__ int pi_cell_of(const int32_t * dyn, int kv_head, int i) { return dyn ? (dyn[3] ? dyn[4 + i] : dyn[0] + i) : kv_head + i; }
 
+// rows to page-locked host memory, thread `tid` of `nthr`
+static __device__ __forceinline__ void pi_rows_out(const float * __restrict__ rows, float * __restrict__ rows_h, size_t n, size_t tid, size_t nthr) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    if ((((uintptr_t) rows | (uintptr_t) rows_h) & 15) == 0) {
+        const size_t n4 = n / 4;
+        for (size_t i = tid; i < n4; i += nthr) __builtin_nontemporal_store(((const u32x4 *) rows)[i], (u32x4 *) rows_h + i);
+        for (size_t i = n4 * 4 + tid; i < n; i += nthr) rows_h[i] = rows[i];
+    } else for (size_t i = tid; i < n; i += nthr) rows_h[i] = rows[i];
+}
+
 // signed 4 x int8 dot product accumulate: v_dot4c_i32_i8
 static __device__ __forceinline__ int pi_dot4(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 

@@ -192,15 +192,10 @@ extern "C" int pi_op_abort_cancel(int32_t * word_dev, int32_t run_id, void * str
 // keep the device busy: a draft step of 1.2 ms waited for the whole 11 ms target run beside it (tools_dev/wrap_beside.py, profiles/r04_d2h_copy_stall.log; the same step
 // with its results written by a kernel: 1.3 ms beside the target).  Page-locked host memory is device-addressable, so the last kernel of a run writes the caller's
 // buffers itself; the event recorded behind it releases them to the host.
-typedef uint32_t rt_u32x4 __attribute__((ext_vector_type(4)));
 __global__ void __launch_bounds__(256) k_copy_out(const float * __restrict__ logits, float * __restrict__ logits_h, size_t n_logits, const int32_t * __restrict__ ids, int32_t * __restrict__ ids_h,
                                                   const float * __restrict__ vals, float * __restrict__ vals_h, const float * __restrict__ sum, float * __restrict__ sum_h, int n_tok) {
     const size_t tid = (size_t) blockIdx.x * 256 + threadIdx.x, nthr = (size_t) gridDim.x * 256;
-    if ((((uintptr_t) logits | (uintptr_t) logits_h) & 15) == 0) {
-        const size_t n4 = n_logits / 4;
-        for (size_t i = tid; i < n4; i += nthr) __builtin_nontemporal_store(((const rt_u32x4 *) logits)[i], (rt_u32x4 *) logits_h + i);
-        for (size_t i = n4 * 4 + tid; i < n_logits; i += nthr) logits_h[i] = logits[i];
-    } else for (size_t i = tid; i < n_logits; i += nthr) logits_h[i] = logits[i];
+    pi_rows_out(logits, logits_h, n_logits, tid, nthr);
     // (spread over the grid like the rows: the top 8 of 2048 rows and a row of logits by one workgroup: 13.5 us, now 6.5)
     for (size_t i = tid; i < 8 * (size_t) n_tok; i += nthr) { ids_h[i] = ids[i]; vals_h[i] = vals[i]; }
     for (size_t i = tid; i < (size_t) n_tok; i += nthr) sum_h[i] = sum[i];

@@ -139,6 +139,7 @@ def _declare(lib):
     lib.pi_op_add.argtypes = [vp, vp, vp, i64, vp]
     lib.pi_op_topk_scratch_bytes.argtypes = [i32]; lib.pi_op_topk_scratch_bytes.restype = C.c_size_t
     lib.pi_op_topk.argtypes = [vp, i32, i32, i32, vp, vp, vp, vp, vp]
+    lib.pi_op_topk_parts.argtypes = [vp, i32, i32, i32, vp, vp]; lib.pi_op_topk_merge.argtypes = [vp, i32, i32, vp, vp, vp, vp]; lib.pi_op_topk_out.argtypes = [vp, i32, i32, vp, vp, vp, vp, vp, C.c_int64, vp]
     # dense bfloat16 matrices and the operators of hybrid blocks
     lib.pi_op_embed.argtypes = [vp, vp, i32, f32, vp, vp]
     lib.pi_op_dense.argtypes = [vp, vp, i64, i32, vp, i64, i32, i64, i32, i32, vp]

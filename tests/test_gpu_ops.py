@@ -1117,6 +1117,36 @@ def test_copy_out_writes_the_page_locked_buffers(gpu, n_tok, nv, skew):
         hip.hipHostFree(host)
 
 
+@pytest.mark.parametrize("n_tok,nv,row0,tops,rows", [(1, 32000, 0, 1, 1), (9, 1001, 2, 5, 3), (8, 259, 3, 5, 0), (6, 4096, 1, 0, 2), (40, 33000, 7, 33, 33)])
+def test_topk_out_merges_and_copies(gpu, n_tok, nv, row0, tops, rows):
+    """pi_op_topk_out (elementwise.hip): some rows' top 8 and soft-max sums, merged straight into page-locked memory, and their logits beside them: what pi_op_topk and a copy give, rows that end inside a workgroup, logits off
+    the 16-byte path, neither rows nor a merge, nothing past the buffers"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]; hip.hipHostFree.argtypes = [C.c_void_p]
+    x = np.round(np.random.default_rng(nv + n_tok).standard_normal((n_tok, nv)) * 30).astype(np.float32)
+    x[row0 + tops // 2] = 1.5                                        # (a crowd of equal values)
+    d, scr, ids, vals, se = U.Dev(x), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(n_tok)), U.Dev(nbytes=32 * n_tok), U.Dev(nbytes=32 * n_tok), U.Dev(nbytes=4 * n_tok)
+    L.check(lib.pi_op_topk(d.ptr, nv, n_tok, 8, ids.ptr, vals.ptr, se.ptr, scr.ptr, None))
+    top = slice(row0, row0 + tops)
+    parts = [x[row0:row0 + rows], ids.get(np.uint32, (n_tok, 8))[top], vals.get(np.uint32, (n_tok, 8))[top], se.get(np.uint32)[top]]
+    at = np.cumsum([0] + [(p.nbytes + 79) // 16 * 16 for p in parts])
+    host = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(host), int(at[-1]) + 64, 0) == 0
+    try:
+        C.memset(host, 0xA5, int(at[-1]) + 64)
+        h = [host.value + int(a) for a in at]
+        L.check(lib.pi_op_topk_parts(d.ptr, nv, n_tok, 8, scr.ptr, None))
+        L.check(lib.pi_op_topk_out(scr.ptr, row0, tops, h[1], h[2], h[3], d.ptr + 4 * row0 * nv, h[0], rows * nv, None))
+        L.check(lib.pi_stream_sync(None))
+        raw = np.frombuffer((C.c_char * (int(at[-1]) + 64)).from_address(host.value), dtype=np.uint8)
+        for p, a, b in zip(parts, at, at[1:]):
+            assert raw[a:a + p.nbytes].tobytes() == p.tobytes() and (raw[a + p.nbytes:b] == 0xA5).all()
+    finally:
+        hip.hipHostFree(host)
+
+
 @pytest.mark.parametrize("counts", [(1, 1, 4, 8), (7, 7, 18, 35, 7, 7), (513, 513, 4, 300001, 513, 0), (0, 0, 0, 0), (5,)])
 def test_copy_in_reads_the_page_locked_block(gpu, counts):
     """pi_op_copy_in (runtime.hip): the parts of a page-locked block at their places, none of them past its end, a part without a place skipped; the abort word armed as pi_op_abort_begin arms it"""

@@ -18,11 +18,11 @@ if len(sys.argv) > 2 and sys.argv[1] == "--analyse":
     tq, dq = qs[0], qs[1]                                   # most launches: the target; next: the draft
     T = sorted(by_q[tq]); D = sorted(by_q[dq])
     t_end = T[-1][1]
-    # split the draft's kernels into calls: a gap of more than 300 us between consecutive kernels' starts... (calls are back to back: use the top-k kernel as the end marker)
+    # split the draft's kernels into calls: a gap of more than 300 us between consecutive kernels' starts... (calls are back to back: use the kernel that brings the results out as the end marker)
     calls, cur = [], []
     for k in D:
         cur.append(k)
-        if "k_topk2" in k[2]:
+        if "k_topk_out" in k[2]:
             calls.append(cur); cur = []
     print(f"target kernels {len(T)}, draft kernels {len(D)}, draft calls {len(calls)}")
     for ci, c in enumerate(calls[-12:]):
