@@ -687,7 +687,9 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 #define TOPK_NCH 32
 // What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One way
 // to go on is a round for each of the k, two wave reductions and one rescan of the lane that lost its best.  The other, for one wave to a slice and many rounds (the rule is at the launch): the least of eight lane groups' bests
-// is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
+// is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  The vector unit's instructions bounded many rows: the candidates' way
+// looks at its values as floats (two instructions each for the best, one for the floor), makes no keys, takes eight for an exponential, and adds the four sums across the lanes together.  us, vocabulary 32000, before / now: 2048
+// rows that a product has just written 127 / 88 (read again and again 86 / 59: 4.4 TB/s), 1000 47 / 34, 512 33 / 26, 333 19.7 / 15.3.  (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
 // (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
 // One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
@@ -704,84 +706,116 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
     pi_butterfly<32>([&](auto o) { i = min(i, pi_partner<decltype(o)::value>(i)); });
     key = m; id = i;
 }
+// e^x of a value below the largest: 2^(x log2(e)) by the hardware, times what that product's rounding and log2(e)'s second part left out (expf's errors without its reduction and its ends of the range: 8 instructions, not 14).
+// Minus infinity: 0 (the correction is bounded), no number: no number; below 2^-126 0
+static __device__ __forceinline__ float topk_exp(float x) {
+    const float hi = x * 1.44269502f, c = fmaxf(x, -150.0f), lo = fminf(fmaf(c, 1.92596303e-8f, fmaf(c, 1.44269502f, -hi)), 1.0f), e = __builtin_amdgcn_exp2f(hi);
+    return fmaf(e * 0.693147182f, lo, e);
+}
+// the larger of what an exchange of a register with itself brings together
+template <typename T> static __device__ __forceinline__ uint32_t topk_across(T both) { return max((uint32_t) both[0], (uint32_t) both[1]); }
 // a row's share of the scratch: the k best of every slice (ids, values), the slices' maxima and sums
 static __host__ __device__ __forceinline__ int topk_words(int k) { return TOPK_NCH * (2 * k + 2); }
 template <int VPT, int WS>
 __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int candidates, int32_t * __restrict__ part, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
-    constexpr int MET = WS > 1 ? 32 : 256;                              // the four waves' bests; a wave's own candidates
-    __shared__ uint32_t met_key[MET]; __shared__ int met_id[MET]; __shared__ float met_sum[4], met_val[WS > 1 ? 1 : MET];
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
+    __shared__ uint32_t met_key[WS > 1 ? 32 : 1]; __shared__ int met_id[WS > 1 ? 32 : 1]; __shared__ float met_sum[4];      // the four waves' bests
+    __shared__ float2 met[WS > 1 ? 1 : 256];                            // a wave's own candidates: value, number in the slice
+    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per), own0 = lo + lane + (WS > 1 ? 64 * wave : 0);
     const float * l = logits + (int64_t) t * n_vocab;
     int32_t * cid = part + (int64_t) t * topk_words(k); float * cval = (float *) (cid + TOPK_NCH * k), * cmax = cval + TOPK_NCH * k, * csum = cmax + TOPK_NCH;
+    static_assert(VPT > 0 || WS > 1, "values that are read again: four waves");
     uint32_t key[VPT > 0 ? VPT : 1]; float rv[VPT > 0 ? VPT : 1];
-    uint32_t bk = 0; int bm = 0;                                        // this lane's best among the ones not taken: key, number
-    if constexpr (VPT > 0) {
-#pragma unroll
-        for (int m = 0; m < VPT; m++) rv[m] = l[min(own0 + STEP * m, n_vocab - 1)];
-#pragma unroll
+    uint32_t bk = 0, wk; int bm = 0, wi;                                // this lane's best among the ones not taken: key, number; the wave's
+    float first, s[4] = { 0.0f, 0.0f, 0.0f, 0.0f };                     // the slice's largest, its sum of exponentials in the order of 256 threads of four waves
+    const int out = ch * k;
+    auto keys = [&]() __attribute__((always_inline)) {
+        if constexpr (VPT > 0)
+#pragma unroll VPT
         for (int m = 0; m < VPT; m++) { key[m] = own0 + STEP * m < hi ? topk_key(rv[m]) : 0u; if (key[m] > bk) { bk = key[m]; bm = m; } }
-    } else for (int i = own0, m = 0; i < hi; i += STEP, m++) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = m; } }
-    if (pi_abort_late(gone, abort_w)) return;
-    uint32_t wk = bk; int wi = bk ? own0 + STEP * bm : 0x7fffffff;
-    uint32_t top = bk, low = 0;                                         // low: at least eight values are not below it — the least of the bests of eight lanes each (lanes of the same number mod 8)
-    if (WS == 1 && candidates) {
-        top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<8>((int) top));
-        low = top;
-        pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); low = min(low, (uint32_t) pi_partner<O>((int) low)); });
-    } else { topk_best(wk, wi); top = wk; }
-    if constexpr (WS > 1) {
+    };
+    if constexpr (WS == 1) {
+        // (what is past the slice's end adds nothing to the sum, and is no candidate)
+        const float * at = l + min(lo, n_vocab - 1);
+#pragma unroll
+        for (int m = 0; m < VPT; m++) { rv[m] = -INFINITY; if (lane < hi - lo - 64 * m) rv[m] = at[lane + 64 * m]; }
+        if (pi_abort_late(gone, abort_w)) return;
+        auto sum_up = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int m = 0; m < VPT; m++) s[m & 3] += topk_exp(rv[m] - first);
+            // the four sums share the way across the lanes: behind two exchanges rows 0 .. 3 of sixteen lanes hold s[0], s[2], s[1] and s[3]
+            const auto s01 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[0]), __float_as_int(s[1]), false, false), s23 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[2]), __float_as_int(s[3]), false, false);
+            const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(__int_as_float(s01[0]) + __int_as_float(s01[1])), __float_as_int(__int_as_float(s23[0]) + __int_as_float(s23[1])), false, false);
+            float sum = __int_as_float(rows[0]) + __int_as_float(rows[1]);
+            pi_butterfly<8>([&](auto o) { sum += pi_partner<decltype(o)::value>(sum); });
+            sum += pi_partner<32>(sum); sum += pi_partner<16>(sum);
+            if (lane == 0) { cmax[ch] = first; csum[ch] = sum; }
+        };
+        if (candidates) {
+            float best = -INFINITY;                                         // (what is no number is never above it)
+#pragma unroll
+            for (int m = 0; m < VPT; m++) best = rv[m] > best ? rv[m] : best;
+            uint32_t top = topk_key(best);
+            top = topk_across(__builtin_amdgcn_permlane32_swap(top, top, false, false)); top = topk_across(__builtin_amdgcn_permlane16_swap(top, top, false, false)); top = max(top, (uint32_t) pi_partner<8>((int) top));
+            uint32_t least = top;                                           // at least eight values are not below it: the least of the bests of eight lanes each (lanes of the same number mod 8)
+            pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); least = min(least, (uint32_t) pi_partner<O>((int) least)); });
+            first = topk_value(top);
+            const float low = topk_value(least);
+            sum_up();
+            if (low > -INFINITY) {
+                // what is not below `low` goes to a lane each, which counts those ahead of it
+                uint64_t who[VPT]; int n = 0;
+#pragma unroll
+                for (int m = 0; m < VPT; m++) { who[m] = __ballot(rv[m] >= low); n += __popcll(who[m]); }
+                if (n <= 64) {                                              // (else, a crowd of equal values: the rounds below)
+                    int base = 0;
+#pragma unroll
+                    for (int m = 0; m < VPT; m++) {
+                        if (rv[m] >= low) met[WS == 1 ? 64 * wave + base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[m], 0)) : 0] = make_float2(rv[m], __int_as_float(lane + 64 * m));
+                        base += __popcll(who[m]);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    const float2 mine = lane < n ? met[WS == 1 ? 64 * wave + lane : 0] : make_float2(-INFINITY, 0.0f);
+                    const float cv = mine.x + 0.0f; const int ci = __float_as_int(mine.y);      // (-0 ties with +0)
+                    int ahead = 0;                                          // (a lower lane has a lower id)
+#pragma unroll 4
+                    for (int j = 0; j < n; j++) {
+                        const float vj = __uint_as_float((uint32_t) __builtin_amdgcn_readlane(__float_as_int(cv), j));
+                        const uint64_t is = __ballot(vj > cv) | (__ballot(vj == cv) & (~1ull << j));
+                        asm("v_addc_co_u32_e64 %0, vcc, %1, 0, %2" : "=v"(ahead) : "v"(ahead), "s"(is) : "vcc");
+                    }
+                    if (lane < n ? ahead < k : lane < k) { const int to = out + (lane < n ? ahead : lane); cid[to] = lane < n ? lo + ci : 0x7fffffff; cval[to] = mine.x; }
+                    return;
+                }
+            }
+        }
+        keys();
+        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
+        topk_best(wk, wi);
+        if (!candidates) { first = topk_value(wk); sum_up(); }
+    } else {
+        if constexpr (VPT > 0) {
+#pragma unroll
+            for (int m = 0; m < VPT; m++) rv[m] = l[min(own0 + STEP * m, n_vocab - 1)];
+            keys();
+        } else for (int i = own0, m = 0; i < hi; i += STEP, m++) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = m; } }
+        if (pi_abort_late(gone, abort_w)) return;
+        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
+        topk_best(wk, wi);
         if (lane == 0) met_key[wave] = wk;
         __syncthreads();
-        top = max(max(met_key[0], met_key[1]), max(met_key[2], met_key[3]));
+        const uint32_t top = max(max(met_key[0], met_key[1]), max(met_key[2], met_key[3]));
         __syncthreads();
-    }
-    const float first = topk_value(top);
-    // the slice's sum of exponentials, in the order of 256 threads of four waves
-    float s[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-    if constexpr (VPT > 0) {
+        first = topk_value(top);
+        if constexpr (VPT > 0) {
 #pragma unroll
-        for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[WS > 1 ? 0 : m & 3] += expf(rv[m] - first);
-    } else for (int i = own0; i < hi; i += STEP) s[0] += expf(l[i] - first);
-    static_assert(VPT > 0 || WS > 1, "values that are read again: four waves");
-    if constexpr (WS == 1) {
-#pragma unroll
-        for (int w = 0; w < 4; w++) s[w] = pi_lanes_sum<64>(s[w]);
-        if (lane == 0) { cmax[ch] = first; csum[ch] = (s[0] + s[1]) + (s[2] + s[3]); }
-    } else { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; }
-    const int out = ch * k;
-    if constexpr (WS == 1) if (candidates) {
-        // what is not below `low` goes to a lane each, which counts those ahead of it
-        const uint32_t least = max(low, 1u);
-        uint64_t who[VPT]; int n = 0;
-#pragma unroll
-        for (int m = 0; m < VPT; m++) { who[m] = __ballot(key[m] >= least); n += __popcll(who[m]); }
-        if (n <= 64) {                                                  // (else, a crowd of equal values: the rounds below)
-            int base = 0;
-#pragma unroll
-            for (int m = 0; m < VPT; m++) {
-                if (key[m] >= least) {
-                    const int at = base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[m], 0));
-                    met_key[64 * wave + at] = key[m]; met_id[64 * wave + at] = lo + lane + 64 * m; met_val[64 * wave + at] = rv[m];
-                }
-                base += __popcll(who[m]);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            const uint32_t ck = lane < n ? met_key[64 * wave + lane] : 0u; const int ci = lane < n ? met_id[64 * wave + lane] : 0x7fffffff;
-            const float cv = lane < n ? met_val[64 * wave + lane] : -INFINITY;
-            int ahead = 0;
-#pragma unroll 4
-            for (int j = 0; j < n; j++) {
-                const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(ci, j);
-                ahead += kj > ck || (kj == ck && ij < ci);
-            }
-            if (lane < n ? ahead < k : lane < k) { const int at = out + (lane < n ? ahead : lane); cid[at] = ci; cval[at] = cv; }
-            return;
-        }
-        topk_best(wk, wi);
+            for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[0] += topk_exp(rv[m] - first);
+        } else for (int i = own0; i < hi; i += STEP) s[0] += topk_exp(l[i] - first);
+        const float sum = pi_lanes_sum<64>(s[0]);
+        if (lane == 0) met_sum[wave] = sum;
     }
     int own = 0x7fffffff; uint32_t own_key = 0;                       // lane r keeps the r-th: their values are read back together, not one by one between the rounds
     for (int r = 0; ; r++) {
@@ -904,10 +938,9 @@ extern "C" int pi_op_topk_parts(const float * logits, int n_vocab, int n_tok, in
     if (k > 8) { pi_set_error("pi_op_topk: k=%d > 8", k); return -1; }
     if (!scratch) { pi_set_error("pi_op_topk: scratch is NULL (needs pi_op_topk_scratch_bytes(n_tok) bytes)"); return -1; }
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
-    // One wave to a slice: candidates cost the same for every k, rounds some 0.8 us each of them, and 1 / 3 us less at the start of 64 / 256 rows.  us by rounds / candidates, vocabulary 32000: 512 rows k = 1 20.1 / 28.7,
-    // 4 30.6 / 30.2, 5 34.3 / 30.8, 8 44.5 / 32.5; 256 rows k = 5 21.0 / 20.6; 128 rows k = 6 15.0 / 15.0, 7 16.3 / 15.5; 64 rows k = 7 12.6 / 13.2; k = 8 of one row 12.7 / 11.4, 6 rows 13.4 / 13.1, 16 11.7 / 12.7,
-    // 32 11.9 / 12.8, 48 13.5 / 13.6; of 65536 8 rows 15.6 / 14.7, 16 14.8 / 15.0
-    const int candidates = n_tok >= 256 ? k >= 5 : n_tok >= 128 ? k >= 7 : k == 8 && (n_tok <= (per > 1024 ? 12 : 7) || n_tok > 32);
+    // One wave to a slice: candidates cost the same for every k, rounds some 0.4 us each of them.  us by rounds / candidates, vocabulary 32000: one row k = 8 6.5 / 5.7, 4 5.6 / 5.6, 2 4.8 / 5.5; 8 rows k = 8 6.6 / 6.0, 4 5.3 / 5.9;
+    // 24 rows k = 8 6.3 / 6.4; 64 rows 8.0 / 7.3, k = 4 6.4 / 7.1; 256 rows k = 4 14.2 / 12.1, 2 11.5 / 12.4.  Slices of 32 values a lane: 8 rows of 50257 k = 8 9.4 / 8.3, 4 8.0 / 8.6; 16 of 65536 k = 8 9.4 / 10.2
+    const int candidates = per <= 1024 ? k >= (n_tok >= 128 ? 3 : 6) : n_tok >= 256 ? k >= 5 : n_tok >= 128 ? k >= 7 : k == 8 && (n_tok <= 12 || n_tok > 32);
 #define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, candidates, (int32_t *) scratch, pi_abort_word())
     if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4);
     else if (per <= 64 * 8) TOPK_GO(8, 1); else if (per <= 64 * 16) TOPK_GO(16, 1); else if (per <= 64 * 32) TOPK_GO(32, 1);

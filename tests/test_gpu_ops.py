@@ -617,6 +617,27 @@ def test_topk_rounds_and_candidates(gpu, n_vocab):
         assert np.array_equal(got[:7], sums[:7]), (n_tok, k)
 
 
+@pytest.mark.parametrize("n_tok,k", [(1, 5), (1, 6), (9, 8), (127, 5), (127, 6), (128, 2), (128, 3)])
+@pytest.mark.parametrize("n_vocab", [63, 64 * 32, 32001])
+def test_topk_candidates_of_few_and_many_rows(gpu, n_tok, k, n_vocab):
+    """both sides of the lines for slices of up to 1024 values: slices of one or two values, ones that end inside a wave's step, rows of many equal values, with infinities, with fewer numbers than a floor needs"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rng = np.random.default_rng(n_tok * 10 + k)
+    x = (rng.standard_normal((n_tok, n_vocab)) * 4).astype(np.float32)
+    x[::3] = np.round(x[::3])                                        # ties at every rank
+    x[-1, ::2], x[-1, 1::4] = -np.inf, np.nan
+    x[n_tok // 2, n_vocab // 3] = np.inf
+    order = np.lexsort((np.broadcast_to(np.arange(n_vocab), x.shape), -np.nan_to_num(x, nan=-np.inf, posinf=np.inf, neginf=-1e38)), axis=1)[:, :k].astype(np.int32)
+    top = np.take_along_axis(x, order, 1)
+    ld, ids, vals, se, scr = U.Dev(x), U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(n_tok))
+    L.check(lib.pi_op_topk(ld.ptr, n_vocab, n_tok, k, ids.ptr, vals.ptr, se.ptr, scr.ptr, None))
+    assert np.array_equal(ids.get(np.int32, (n_tok, k)), order) and np.array_equal(vals.get(np.float32, (n_tok, k)), top)
+    want = np.exp(x[0].astype(np.float64) - x[0].max().astype(np.float64)).sum()
+    if np.isfinite(want) and n_tok > 1:
+        assert abs(se.get(np.float32)[0] - want) / want < 1e-5      # (as test_topk_edges: fp32 sum of up to 32001 terms in pairs per slice)
+
+
 @pytest.mark.parametrize("n_vocab", [512, 32000, 65024])
 def test_topk(gpu, n_vocab):
     lib, U = gpu
