@@ -1756,8 +1756,8 @@ __global__ void __launch_bounds__(256, NJ == 4 ? 3 : EX == 0 ? 2 : 1) k_latent_r
 // grid (token tile of 4, head, 16 output values): merges the splits (with the sink if there is one), normalises, applies its rows of W_uv[h], then the gate if there is one: one value per head, or (gate_width = vdim)
 // one per output value
 // MANY: more than eight splits (the code for them costs the launches of fewer 0.3 us of 9.5)
-template <bool MANY>
-__global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
+template <bool MANY, int NT>
+__global__ void __launch_bounds__(NT) k_latent_combine(const float * __restrict__ pol, const float * __restrict__ pml, const uint16_t * __restrict__ wuv, const float * __restrict__ sink,
                                                         const float * __restrict__ gate, int64_t gs, int gate_act, int gate_width, int heads, int vdim, int rank, int S, int n_tok, int n_kv, int cap, const int32_t * __restrict__ dyn, int live_min, int live_max, int vec, float * __restrict__ out, int64_t os,
                                                         const int32_t * __restrict__ abort_w) {
     if ((live_min > 0 && dyn[1] <= live_min) || (live_max > 0 && dyn[1] > live_max)) return;
@@ -1768,28 +1768,29 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     __shared__ float gsh[4];                                          // per token: the head's gate (one value per head)
     const int t0 = blockIdx.x * 4, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nt = min(4, n_tok - t0), n_s = min(S, (min(dyn ? dyn[1] : n_kv, n_kv) + cap - 1) / cap);      // (splits of cap cells: the ones behind the live cells hold nothing)
-    hy_u16x8v wrow[4]; float gv[4] = { 1.0f, 1.0f, 1.0f, 1.0f };      // (wide: eight weights of the rank per lane; the wave's four rows and their gates are on their way while the splits are merged)
+    constexpr int NW = NT / 64, RW = 16 / NW;                         // waves, rows of W_uv of a wave
+    hy_u16x8v wrow[RW]; float gv[RW];      // (wide: eight weights of the rank per lane; the wave's rows and their gates are on their way while the splits are merged)
     const bool wide = vec && rank > 64;                             // (of fewer values a lane per value is quicker: rank 64, 6.0 us against 6.9; calls of rank 96 with one split, 4 tokens, 17.1 that way, 16.3 so)
     if (wide) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)) * rank + min(lane * 8, rank - 8));
+        for (int k = 0; k < RW; k++) wrow[k] = *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + NW * k, vdim - 1)) * rank + min(lane * 8, rank - 8));
         if (gate && gate_width > 1)
 #pragma unroll
-            for (int k = 0; k < 4; k++) gv[k] = gate[(int64_t) (t0 + min(lane, nt - 1)) * gs + (int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + 4 * k, vdim - 1)];
+            for (int k = 0; k < RW; k++) gv[k] = gate[(int64_t) (t0 + min(lane, nt - 1)) * gs + (int64_t) h * vdim + min((int) blockIdx.z * 16 + wave + NW * k, vdim - 1)];
     }
     // many splits: a thread per four values of the rank, for all tokens at a time or, where that leaves some threads idle but no second group of them and the splits are many, for one token after the other; the groups take eight splits
     // in turn (1 token of 8 heads, rank 256, over 16384 cells: 83 us with one group, now 43)
-    __shared__ __attribute__((aligned(16))) float4 shares[MANY ? 4 : 1][MANY ? 256 : 1];
+    __shared__ __attribute__((aligned(16))) float4 shares[MANY && NT == 256 ? 4 : 1][MANY ? NT : 1];
     int groups = 1, per = 1, at_once = 1, grp = 0, mine = 0, col = 0;
-    float4 share[4];
+    float4 share[NT == 256 ? 4 : 1];
     if (MANY && vec) {
         const int cols = rank >> 2;
-        at_once = nt * cols <= 128 ? nt : 1; per = at_once * cols;
-        if (n_s > 16 && (at_once == nt || (n_s > 64 && (nt * cols & 255))) && per <= 128) { groups = 256 / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
+        at_once = nt * cols <= NT / 2 ? nt : 1; per = at_once * cols;
+        if (n_s > (NT == 256 ? 16 : 8) && (at_once == nt || (NT == 256 && n_s > 64 && (nt * cols & 255))) && per <= NT / 2) { groups = NT / per; grp = tid / per; mine = tid % per / cols; col = tid % cols; }
 #pragma unroll
-        for (int i = 0; i < 4; i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int i = 0; i < (NT == 256 ? 4 : 1); i++) share[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
-    for (int idx = tid; idx < 4 * rank; idx += 256) ol[idx] = 0.0f;
+    for (int idx = tid; idx < 4 * rank; idx += NT) ol[idx] = 0.0f;
     if (tid < 4) {
         float g = 1.0f;
         if (gate && gate_width == 1 && tid < nt) { g = gate[(int64_t) (t0 + tid) * gs + h]; if (gate_act == PI_ACT_SIGMOID) g = 1.0f / (1.0f + expf(-g)); }
@@ -1821,7 +1822,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         __syncthreads();
         if (MANY && groups > 1) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < (NT == 256 ? 4 : 1); i++) {
                 const int tt = min(i * at_once + mine, nt - 1), n = i * at_once < nt && grp < groups ? cnt[tt] : 0;
                 const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + col * 4;
                 for (int s0 = 8 * grp; s0 < n; s0 += 8 * groups) {
@@ -1836,7 +1837,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             continue;
         }
         if (vec) {                                                     // four values of the rank per thread, eight splits on their way at a time (one by one, every split was a trip to memory: 23 us for 11 of 4 tokens)
-            for (int idx = tid; idx < nt * (rank >> 2); idx += 256) {
+            for (int idx = tid; idx < nt * (rank >> 2); idx += NT) {
                 const int tt = idx / (rank >> 2), r = idx % (rank >> 2) * 4, n = cnt[tt];
                 if (n == 0) continue;
                 const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + r;
@@ -1853,7 +1854,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             }
             continue;
         }
-        for (int idx = tid; idx < nt * rank; idx += 256) {
+        for (int idx = tid; idx < nt * rank; idx += NT) {
             const int tt = idx / rank, r = idx % rank;
             const float * p = pol + (((int64_t) (t0 + tt) * heads + h) * S) * rank + r;
             float v = ol[idx];
@@ -1865,10 +1866,10 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     }
     if (MANY && groups > 1) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) if (i * at_once < nt) shares[i][tid] = share[i];
+        for (int i = 0; i < (NT == 256 ? 4 : 1); i++) if (i * at_once < nt) shares[i][tid] = share[i];
         __syncthreads();
         const int cols = rank >> 2;
-        for (int idx = tid; idx < nt * cols; idx += 256) {
+        for (int idx = tid; idx < nt * cols; idx += NT) {
             const float4 * from = shares[idx / per];
             float4 v = from[idx % per];
             for (int g = 1; g < groups; g++) { const float4 x = from[g * per + idx % per]; v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w; }
@@ -1878,17 +1879,17 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
     __syncthreads();
     if (wide) {
         const int v0 = blockIdx.z * 16 + wave;
-        float a[4][4];
+        float a[RW][4];
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < RW; k++)
 #pragma unroll
             for (int tt = 0; tt < 4; tt++) a[k][tt] = 0.0f;
         for (int rb = 0; rb < rank; rb += 512) {
             const int r = rb + lane * 8;
             if (r >= rank) break;
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const hy_u16x8v w = rb == 0 ? wrow[k] : *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min(v0 + 4 * k, vdim - 1)) * rank + r);
+            for (int k = 0; k < RW; k++) {
+                const hy_u16x8v w = rb == 0 ? wrow[k] : *(const hy_u16x8v *) (wuv + ((int64_t) h * vdim + min(v0 + NW * k, vdim - 1)) * rank + r);
 #pragma unroll
                 for (int tt = 0; tt < 4; tt++)
 #pragma unroll
@@ -1896,8 +1897,8 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
             }
         }
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int vv = v0 + 4 * k;
+        for (int k = 0; k < RW; k++) {
+            const int vv = v0 + NW * k;
             if (vv >= vdim) break;
             float v = 0.0f;
 #pragma unroll
@@ -1909,7 +1910,7 @@ __global__ void __launch_bounds__(256) k_latent_combine(const float * __restrict
         }
         return;
     }
-    for (int vv = blockIdx.z * 16 + wave; vv < min(vdim, (int) blockIdx.z * 16 + 16); vv += 4) {
+    for (int vv = blockIdx.z * 16 + wave; vv < min(vdim, (int) blockIdx.z * 16 + 16); vv += NW) {
         const uint16_t * wv = wuv + ((int64_t) h * vdim + vv) * rank;
         float a[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
         const bool mine = lane < nt;                                   // lane tt writes token t0 + tt; its gate is on the way while the row is summed
@@ -2072,12 +2073,15 @@ static int latent_attention(const float * q, int64_t q_stride, const float * cac
     // 24 tokens, 384 rows, 16000 cells still 695 / 973)
     const int64_t rows_to = n_tok > 8 && dyn_dev && (int64_t) n_tok * heads * rank > 448 * 512 ? ((int64_t) 1 << 31) / ((int64_t) n_tok * heads * rank) : n_kv;
     const int live_max = whole && rows_to < n_kv ? (int) rows_to : 0;
-#define LAT_COMBINE(MANY) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * S + vdim), k_latent_combine<MANY>, dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
-                 dim3(256), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, S, n_tok, n_kv, rows ? 32 : p.cap, dyn_dev, rows ? 0 : live_min, rows ? live_max : 0, \
+#define LAT_COMBINE(MANY, NT) PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, nta, 2.0 * rank * heads * vdim + 4.0 * n_tok * heads * (rank * S + vdim), (k_latent_combine<MANY, NT>), dim3((unsigned) ((n_tok + 3) / 4), (unsigned) heads, (unsigned) ((vdim + 15) / 16)), \
+                 dim3(NT), (size_t) 16 * rank, s, pol, pml, (const uint16_t *) wuv->p0, sink_dev, gate_dev, gate_stride, gate_act, gate_width, heads, vdim, rank, S, n_tok, n_kv, rows ? 32 : p.cap, dyn_dev, rows ? 0 : live_min, rows ? live_max : 0, \
                  vec, out, out_stride, pi_abort_word())
     auto combine = [&](int S, bool rows) -> int {
         const int vec = (rank & 7) == 0 && (rank > 64 || S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
-        if (S > 8) LAT_COMBINE(true); else LAT_COMBINE(false);
+        // Many splits of whole rows: eight waves, as a thread's trips to memory one behind the other are what is waited for; up to two workgroups a compute unit.  us of 256 / 512 threads, rank 512: 4 tokens x 16 heads, 23 splits
+        // 12.7 / 10.6, 10 splits 10.9 / 8.3, 1 token 23 splits 9.1 / 7.4, 250 splits 27.6 / 19.6, 8 tokens x 32 heads (512 workgroups), 32 splits 17.7 / 14.8, x 64 heads 22.5 / 26.8
+        const int64_t wgs = (int64_t) ((n_tok + 3) / 4) * heads * ((vdim + 15) / 16);
+        if (S > 8 && vec && rank > 64 && wgs <= 2 * pi_cu_count()) LAT_COMBINE(true, 512); else if (S > 8) LAT_COMBINE(true, 256); else LAT_COMBINE(false, 256);
         PI_CHECK_LAUNCH(); return 0;
     };
     if (whole) {
