@@ -372,6 +372,119 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
+// The same for a step: a few tokens, most of them a run of their own.  What bounds it: a state is read and written once (16.8 MB of eight sequences, 6.7 us at a copy's rate), and the trips to memory in front of that.  So nothing goes
+// through LDS but the sums over the rows, which the four waves share: a wave finds its run by a ballot, every operand of its first token leaves beside the state, the unit vectors' lengths and the token's scalar are added up by
+// every wave for itself.  Workgroup (head, 32 columns of values, run); thread (four columns, rows rg + 32 m), states in runs of 128 bytes; a token is one barrier.
+// Measured, us (k_channel_recurrence / this), 32 heads of 128 x 128 under the delta rule: one token 14.5 / 4.8, eight of a sequence each 19.8 / 8.3, eight of one 35.6 / 13.7, 32 of one 109 / 46; 64 heads of 64 x 64 under the bonus rule
+// 11.8 / 3.7, 15.6 / 6.1, 24.5 / 8.6, 67.8 / 23.5.  (There a token's operands were staged for 32, with four barriers and a search by one thread ahead of them, and a state came in runs of 64 bytes.)
+#define CS_TOKENS CR_TB                           // (a run's first tokens are found among a wave's lanes; longer passes go in pieces)
+template <int NR, int RULE>
+__global__ void __launch_bounds__(256) k_channel_step(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs,
+                                                      const float * __restrict__ draw, int64_t ds, int decay_mode, const float * __restrict__ dbias, const float * __restrict__ a_log,
+                                                      const float * __restrict__ braw, int64_t bs, const float * __restrict__ bonus, int qk_unit, float q_mult,
+                                                      int heads, int hpg, int vdim, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok,
+                                                      float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    constexpr int DIM = 32 * NR, NL = (DIM + 63) / 64;
+    __shared__ __attribute__((aligned(16))) float meet[2][4][2][32];    // [token % 2][wave][with the keys, with the queries][column]
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = tid & 7, rg = tid >> 3, col = blockIdx.y * 32 + quad * 4, hq = h / hpg;
+    // run number blockIdx.z
+    const int own = rec[min(lane, n_tok - 1)], before = rec[max(min(lane, n_tok - 1) - 1, 0)];
+    const float ah = decay_mode == 2 ? expf(a_log[h]) : 0.0f;
+    uint64_t starts = __ballot(lane < n_tok && (lane == 0 || (own & ~CM_FRESH) != (before & ~CM_FRESH)));
+    for (int r = 0; r < (int) blockIdx.z; r++) starts &= starts - 1;
+    if (!starts) return;
+    const int first = __ffsll((unsigned long long) starts) - 1, rest = __ffsll((unsigned long long) (starts & (starts - 1))), end = rest ? rest - 1 : n_tok, word = __builtin_amdgcn_readlane(own, first);
+    if (word < 0) return;
+    float * const S_hbm = state + ((int64_t) (word & ~CM_FRESH) * heads + h) * DIM * vdim + (int64_t) rg * vdim + col;
+    float4 S[NR];
+    if (word & CM_FRESH) {
+#pragma unroll
+        for (int m = 0; m < NR; m++) S[m] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else {
+#pragma unroll
+        for (int m = 0; m < NR; m++) S[m] = *(const float4 *) (S_hbm + (int64_t) 32 * m * vdim);
+    }
+    struct token { float q[NR], k[NR], d[NR], lq[NL], lk[NL], lb[NL], beta; float4 v; };
+    float bias[NR];
+#pragma unroll
+    for (int m = 0; m < NR; m++) bias[m] = dbias ? dbias[h * DIM + rg + 32 * m] : 0.0f;
+    auto ask = [&](token & T, int t) __attribute__((always_inline)) {
+        const float * qr = q + (int64_t) t * qs + (int64_t) hq * DIM, * kr = k + (int64_t) t * ks + (int64_t) hq * DIM, * dr = draw + (int64_t) t * ds + (int64_t) h * DIM;
+#pragma unroll
+        for (int m = 0; m < NR; m++) { T.q[m] = qr[rg + 32 * m]; T.k[m] = kr[rg + 32 * m]; T.d[m] = dr[rg + 32 * m]; }
+#pragma unroll
+        for (int x = 0; x < NL; x++) {
+            const int i = min(lane + 64 * x, DIM - 1);
+            T.lq[x] = qr[i]; T.lk[x] = kr[i]; T.lb[x] = RULE == 1 && bonus ? bonus[h * DIM + i] : 1.0f;
+        }
+        T.beta = braw ? braw[(int64_t) t * bs + h] : 0.0f;
+        T.v = *(const float4 *) (v + (int64_t) t * vs + (int64_t) h * vdim + col);
+    };
+    token T;
+    ask(T, first);
+    if (pi_abort_late(gone, abort_w)) return;
+    for (int t = first; t < end; t++) {
+        // lengths, then the token's scalar (k . q, or sum q b k)
+        float iq = q_mult, ik = 1.0f, dot = 0.0f;
+        if (qk_unit) {
+            float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+            for (int x = 0; x < NL; x++) if (DIM % 64 == 0 || lane < DIM) { sq = fmaf(T.lq[x], T.lq[x], sq); sk = fmaf(T.lk[x], T.lk[x], sk); }
+            pi_butterfly<32>([&](auto o) { constexpr int O = decltype(o)::value; sq += pi_partner<O>(sq); sk += pi_partner<O>(sk); });
+            iq = q_mult / sqrtf(sq + 1e-6f); ik = 1.0f / sqrtf(sk + 1e-6f);
+        }
+#pragma unroll
+        for (int x = 0; x < NL; x++) if (DIM % 64 == 0 || lane < DIM) dot = fmaf(T.lq[x] * iq * T.lb[x], T.lk[x] * ik, dot);
+        dot = pi_lanes_sum<64>(dot);
+        float kk[NR], a[4] = { 0.0f, 0.0f, 0.0f, 0.0f }, c[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+        const float beta = braw ? cm_sigmoid(T.beta) : 1.0f;
+        const float4 vv = T.v;
+#pragma unroll
+        for (int m = 0; m < NR; m++) {
+            float g = T.d[m];
+            if (decay_mode == 1) g = expf(-expf(g + bias[m]));
+            else if (decay_mode == 2) g = expf(-ah * cm_softplus(g + bias[m]));
+            const float qq = T.q[m] * iq;
+            kk[m] = T.k[m] * ik;
+            if (RULE == 0) {
+                S[m].x *= g; S[m].y *= g; S[m].z *= g; S[m].w *= g;
+                a[0] = fmaf(S[m].x, kk[m], a[0]); a[1] = fmaf(S[m].y, kk[m], a[1]); a[2] = fmaf(S[m].z, kk[m], a[2]); a[3] = fmaf(S[m].w, kk[m], a[3]);
+            }
+            c[0] = fmaf(S[m].x, qq, c[0]); c[1] = fmaf(S[m].y, qq, c[1]); c[2] = fmaf(S[m].z, qq, c[2]); c[3] = fmaf(S[m].w, qq, c[3]);
+            if (RULE == 1) { S[m].x *= g; S[m].y *= g; S[m].z *= g; S[m].w *= g; }
+        }
+        if (t + 1 < end) ask(T, t + 1);
+        // over the wave's eight rows: lanes 8 apart
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            if (RULE == 0) { a[x] += pi_partner<8>(a[x]); a[x] += pi_partner<16>(a[x]); a[x] += pi_partner<32>(a[x]); }
+            c[x] += pi_partner<8>(c[x]); c[x] += pi_partner<16>(c[x]); c[x] += pi_partner<32>(c[x]);
+        }
+        float (* const M)[2][32] = meet[t & 1];
+        if (lane < 8) {
+            if (RULE == 0) *(float4 *) &M[wave][0][quad * 4] = make_float4(a[0], a[1], a[2], a[3]);
+            *(float4 *) &M[wave][1][quad * 4] = make_float4(c[0], c[1], c[2], c[3]);
+        }
+        __syncthreads();
+        float4 u = vv;                                                  // what the token writes under its key
+        if (RULE == 0) {
+            const float4 w0 = *(const float4 *) &M[0][0][quad * 4], w1 = *(const float4 *) &M[1][0][quad * 4], w2 = *(const float4 *) &M[2][0][quad * 4], w3 = *(const float4 *) &M[3][0][quad * 4];
+            u.x = beta * (vv.x - ((w0.x + w1.x) + (w2.x + w3.x))); u.y = beta * (vv.y - ((w0.y + w1.y) + (w2.y + w3.y)));
+            u.z = beta * (vv.z - ((w0.z + w1.z) + (w2.z + w3.z))); u.w = beta * (vv.w - ((w0.w + w1.w) + (w2.w + w3.w)));
+        }
+#pragma unroll
+        for (int m = 0; m < NR; m++) { S[m].x = fmaf(kk[m], u.x, S[m].x); S[m].y = fmaf(kk[m], u.y, S[m].y); S[m].z = fmaf(kk[m], u.z, S[m].z); S[m].w = fmaf(kk[m], u.w, S[m].w); }
+        if (tid < 8) {
+            const float4 w0 = *(const float4 *) &M[0][1][quad * 4], w1 = *(const float4 *) &M[1][1][quad * 4], w2 = *(const float4 *) &M[2][1][quad * 4], w3 = *(const float4 *) &M[3][1][quad * 4];
+            *(float4 *) (out + (int64_t) t * os + (int64_t) h * vdim + col) = make_float4(fmaf(u.x, dot, (w0.x + w1.x) + (w2.x + w3.x)), fmaf(u.y, dot, (w0.y + w1.y) + (w2.y + w3.y)),
+                                                                                       fmaf(u.z, dot, (w0.z + w1.z) + (w2.z + w3.z)), fmaf(u.w, dot, (w0.w + w1.w) + (w2.w + w3.w)));
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < NR; m++) *(float4 *) (S_hbm + (int64_t) 32 * m * vdim) = S[m];
+}
+
 // grid (head, blocks of CR_SCAN_COLS value columns, run): per piece p of the run, in order: scratch[p] holds [L_p | T_p] coming in and S_in(p) (in L_p's place) going out.
 // A workgroup keeps its columns of S in LDS (two buffers) and T_p transposed ([c][i], so that a thread's rows are neighbours); a thread owns a tile of 8 rows x 4 columns: per column c of T_p
 // three 16-byte LDS reads feed 32 multiply-adds.
@@ -1059,6 +1172,16 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
 #undef CR_GO
         PI_CHECK_LAUNCH(); return 0;
     };
+    // every pass that is not cut into pieces, of key widths and columns that the step kernel's threads share out whole (its figures: both kernels at every number of tokens)
+    if (n_tok <= CS_TOKENS && (dim == 32 || dim == 64 || dim == 128) && vdim % 32 == 0 && v_stride % 4 == 0 && out_stride % 4 == 0 && (((uintptr_t) v | (uintptr_t) out | (uintptr_t) state_dev) & 15) == 0) {
+        const dim3 grid((unsigned) heads, (unsigned) (vdim / 32), (unsigned) runs);
+#define CS_GO(NR, RL) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_channel_step<NR, RL>), grid, dim3(256), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
+                                   beta_raw, beta_stride, bonus_dev, qk_unit, q_mult, heads, heads / qk_heads, vdim, state_dev, rec_dev, n_tok, out, out_stride, pi_abort_word())
+        if (rule == PI_RULE_DELTA) { if (dim == 32) CS_GO(1, 0); else if (dim == 64) CS_GO(2, 0); else CS_GO(4, 0); }
+        else                       { if (dim == 32) CS_GO(1, 1); else if (dim == 64) CS_GO(2, 1); else CS_GO(4, 1); }
+#undef CS_GO
+        PI_CHECK_LAUNCH(); return 0;
+    }
     if (!pieces) return launch(0);
     if (cp_takes(dim, vdim) && (rule == PI_RULE_BONUS || qk_unit) && scratch_floats >= cp_floats(heads, dim, vdim, n_tok, max_segments) && ((uintptr_t) scratch_dev & 15) == 0) {
         const dim3 pg((unsigned) heads, (unsigned) cr_max_pieces(n_tok, max_segments, CP_TB)), wg((unsigned) heads, (unsigned) (vdim / 16), (unsigned) runs);

@@ -378,6 +378,49 @@ def test_channel_recurrence_rules_decays_and_passes(H, G, D, V, rule, pieces):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 32), (3, 3, 64, 96), (4, 2, 128, 64)])
+@pytest.mark.parametrize("rule", [DELTA, BONUS])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_channel_recurrence_steps(H, G, D, V, rule, mode):
+    """passes of up to 32 tokens of whole key widths: a token or some to a sequence, sequences in any order, carried and fresh states, every decay, the 33rd token that goes another way; a sequence that is not in the pass keeps its state"""
+    U, lib = gpu()
+    rng = np.random.default_rng(D + V + rule + mode)
+    slots, unit = 9, rule == DELTA
+    start = (rng.standard_normal((slots, H, D, V)) * 2).astype(np.float32)
+    states, sd = start.astype(np.float64), U.Dev(start)
+    dbias, a_log, bonus = (rng.standard_normal(H * D) - 1).astype(np.float32), (rng.standard_normal(H) * 0.5).astype(np.float32), rng.standard_normal((H, D)).astype(np.float32)
+    dbd, ald, bod = U.Dev(dbias), U.Dev(a_log), U.Dev(bonus)
+    for step in ([(4, 1, False)], [(7, 1, True), (0, 1, False), (3, 1, False)], [(0, 2, False), (6, 5, True), (1, 1, False)], [(s, 1, False) for s in (5, 1, 0, 7, 2, 4, 6)], [(2, 31, True), (1, 1, False)], [(2, 33, False)]):
+        T = sum(c for _, c, _ in step)
+        q, k = (rng.standard_normal((T, G * D + 1)).astype(np.float32) * (1.0 if unit else 0.3) for _ in range(2))
+        v, raw, braw = rng.standard_normal((T, H * V + 4)).astype(np.float32), rng.standard_normal((T, H * D + 3)).astype(np.float32), rng.standard_normal((T, H + 1)).astype(np.float32)
+        if mode == 0:
+            raw = rng.uniform(0.3, 1.0, raw.shape).astype(np.float32)
+        rec, want, at = [], np.zeros((T, H, V)), 0
+        for slot, count, fresh in step:
+            if fresh:
+                states[slot] = 0.0
+            for i in range(count):
+                rec.append(slot | (F if fresh and i == 0 else 0))
+                for h in range(H):
+                    j = h // (H // G)
+                    qh, kh = q[at, j * D:(j + 1) * D].astype(np.float64), k[at, j * D:(j + 1) * D].astype(np.float64)
+                    if unit:
+                        qh, kh = O.unit_length(qh) * 0.7, O.unit_length(kh)
+                    r = raw[at, h * D:(h + 1) * D].astype(np.float64)
+                    g = r if mode == 0 else np.exp(-np.exp(r + dbias[h * D:(h + 1) * D])) if mode == 1 else np.exp(-np.exp(a_log[h]) * O.softplus(r + dbias[h * D:(h + 1) * D]))
+                    want[at, h], states[slot][h] = recurrence_ref(rule, qh, kh, v[at, h * V:(h + 1) * V].astype(np.float64), g, O.sigmoid(braw[at, h]), bonus[h].astype(np.float64), states[slot][h])
+                at += 1
+        qd, kd, vd, rd, bd, rc, od = U.Dev(q), U.Dev(k), U.Dev(v), U.Dev(raw), U.Dev(braw), U.Dev(np.array(rec, np.int32)), U.Dev(nbytes=4 * T * H * V)
+        L.check(lib.pi_op_channel_recurrence(rule, qd.ptr, G * D + 1, kd.ptr, G * D + 1, vd.ptr, H * V + 4, rd.ptr, H * D + 3, mode, dbd.ptr, ald.ptr, bd.ptr if rule == DELTA else None, H + 1,
+                                             bod.ptr if rule == BONUS else None, int(unit), 0.7 if unit else 1.0, H, G, D, V, sd.ptr, rc.ptr, T, slots, None, 0, od.ptr, H * V, None))
+        assert rel_rms(od.get(np.float32, (T, H, V)), want) < 2e-5, step
+    st = sd.get(np.float32, (slots, H, D, V))
+    assert np.array_equal(st[8], start[8])
+    assert rel_rms(st, states) < 2e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 16), (3, 3, 64, 64), (4, 2, 128, 48), (1, 1, 128, 128), (1, 1, 64, 144), (2, 1, 32, 272)])
 @pytest.mark.parametrize("rule", [DELTA, BONUS])
 def test_channel_recurrence_pieces_on_the_matrix_cores(H, G, D, V, rule):
