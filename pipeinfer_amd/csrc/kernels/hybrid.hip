@@ -741,6 +741,73 @@ __global__ void __launch_bounds__(256) k_linear_attention(const float * __restri
         for (int ii = 0; ii < DPT; ii++) { const int i = sp * DPT + ii; if (i < dim) S_to[(int64_t) i * vdim + j] = S[ii]; }
 }
 
+// The same for a step: a few tokens, most of them a run of their own, whole key widths and columns.  What bounds it: the trips to memory in front of a state's one.  Nothing goes through LDS but the sums over the rows: a wave finds its
+// run by a ballot, its first token's operands leave beside the state, the next one's ahead of the sums.  Workgroup (head, 32 columns of values, run); thread (four columns, rows rg + 32 m), states in runs of 128 bytes.
+// Measured, us (k_linear_attention or k_linear_pieces, whichever it was / this): 16 heads of 128 x 128, one token 7.7 / 3.1, eight of a sequence each 10.5 / 4.4, eight of one 22.2 / 7.2, 16 of one 23.0 / 12.2; 16 heads of 64 x 64 7.4 / 2.9,
+// 9.6 / 3.1, 16.9 / 6.4, 11.4 / 10.4.  (There a token's operands were staged for 32, behind a search through LDS, and a state came in runs of 64 bytes.)
+template <int NR>
+__global__ void __launch_bounds__(256) k_linear_step(const float * __restrict__ q, const float * __restrict__ k, const float * __restrict__ v, int64_t stride, int heads, int hpg, int vdim,
+                                                     const float * __restrict__ decay, const float * __restrict__ tdecay, const float * __restrict__ tscale, int64_t tds, const float * __restrict__ skip,
+                                                     float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    constexpr int DIM = 32 * NR;
+    __shared__ __attribute__((aligned(16))) float meet[2][4][32];       // [token % 2][wave][column]
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = tid & 7, rg = tid >> 3, col = blockIdx.y * 32 + quad * 4, hq = h / hpg;
+    const int own = rec[min(lane, n_tok - 1)], before = rec[max(min(lane, n_tok - 1) - 1, 0)];
+    const float lam0 = decay ? decay[h] : 1.0f, skp = skip ? skip[h] : 0.0f;
+    uint64_t starts = __ballot(lane < n_tok && (lane == 0 || (own & ~LA_FRESH) != (before & ~LA_FRESH)));
+    for (int r = 0; r < (int) blockIdx.z; r++) starts &= starts - 1;
+    if (!starts) return;
+    const int first = __ffsll((unsigned long long) starts) - 1, rest = __ffsll((unsigned long long) (starts & (starts - 1))), end = rest ? rest - 1 : n_tok, word = __builtin_amdgcn_readlane(own, first);
+    if (word < 0) return;
+    float * const S_hbm = state + ((int64_t) (word & ~LA_FRESH) * heads + h) * DIM * vdim + (int64_t) rg * vdim + col;
+    float4 S[NR];
+    if (word & LA_FRESH) {
+#pragma unroll
+        for (int m = 0; m < NR; m++) S[m] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else {
+#pragma unroll
+        for (int m = 0; m < NR; m++) S[m] = *(const float4 *) (S_hbm + (int64_t) 32 * m * vdim);
+    }
+    struct token { float q[NR], k[NR], lam, sc; float4 v; };
+    auto ask = [&](token & T, int t) __attribute__((always_inline)) {
+        const float * qr = q + (int64_t) t * stride + (int64_t) hq * DIM, * kr = k + (int64_t) t * stride + (int64_t) hq * DIM;
+#pragma unroll
+        for (int m = 0; m < NR; m++) { T.q[m] = qr[rg + 32 * m]; T.k[m] = kr[rg + 32 * m]; }
+        T.lam = tdecay ? tdecay[(int64_t) t * tds + h] : lam0;
+        T.sc = tscale ? tscale[(int64_t) t * tds + h] : 1.0f;
+        T.v = *(const float4 *) (v + (int64_t) t * stride + (int64_t) h * vdim + col);
+    };
+    token T;
+    ask(T, first);
+    if (pi_abort_late(gone, abort_w)) return;
+    for (int t = first; t < end; t++) {
+        const float4 vv = T.v;
+        const float vx = vv.x * T.sc, vy = vv.y * T.sc, vz = vv.z * T.sc, vw = vv.w * T.sc, lam = T.lam;
+        float o[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int m = 0; m < NR; m++) {
+            const float kk = T.k[m], qq = T.q[m];
+            S[m].x = fmaf(kk, vx, lam * S[m].x); S[m].y = fmaf(kk, vy, lam * S[m].y); S[m].z = fmaf(kk, vz, lam * S[m].z); S[m].w = fmaf(kk, vw, lam * S[m].w);
+            o[0] = fmaf(S[m].x, qq, o[0]); o[1] = fmaf(S[m].y, qq, o[1]); o[2] = fmaf(S[m].z, qq, o[2]); o[3] = fmaf(S[m].w, qq, o[3]);
+        }
+        if (t + 1 < end) ask(T, t + 1);
+        // over the wave's eight rows: lanes 8 apart
+#pragma unroll
+        for (int x = 0; x < 4; x++) { o[x] += pi_partner<8>(o[x]); o[x] += pi_partner<16>(o[x]); o[x] += pi_partner<32>(o[x]); }
+        float (* const M)[32] = meet[t & 1];
+        if (lane < 8) *(float4 *) &M[wave][quad * 4] = make_float4(o[0], o[1], o[2], o[3]);
+        __syncthreads();
+        if (tid < 8) {
+            const float4 w0 = *(const float4 *) &M[0][quad * 4], w1 = *(const float4 *) &M[1][quad * 4], w2 = *(const float4 *) &M[2][quad * 4], w3 = *(const float4 *) &M[3][quad * 4];
+            *(float4 *) (out + (int64_t) t * os + (int64_t) h * vdim + col) = make_float4(fmaf(skp, vv.x, (w0.x + w1.x) + (w2.x + w3.x)), fmaf(skp, vv.y, (w0.y + w1.y) + (w2.y + w3.y)),
+                                                                                       fmaf(skp, vv.z, (w0.z + w1.z) + (w2.z + w3.z)), fmaf(skp, vv.w, (w0.w + w1.w) + (w2.w + w3.w)));
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < NR; m++) *(float4 *) (S_hbm + (int64_t) 32 * m * vdim) = S[m];
+}
+
 // Long passes on the fp32 matrix cores (v_mfma_f32_16x16x4_f32), pieces of 64 or 32 tokens, for key widths of 32 DI <= 128.  What bounds the token loop of k_linear_attention is its chain: a token's state
 // value waits for the one before, two products per state value on the vector units.  Per head and piece, with a_t = lambda_1 .. lambda_t and D[t][j] = lambda_{j+1} .. lambda_t (products only, no quotients):
 //   O = a_t (Q S_in) + (Q K^T o D s) V,   S_out = a_64 S_in + sum_j (lambda_{j+1} .. lambda_64 s_j k_j) v_j^T
@@ -1314,6 +1381,15 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
     // Up to 64 tokens every run is one piece: one launch from the slots' states to the slots' states.  Beyond LA_TB always (32 heads of 128 x 128, three launches against it: a run of 64 tokens 55 -> 48 us, 64 runs of a
     // token 450 -> 123, for the pieces are walked twice and the scan starts for every run); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
     // (24 tokens 53 -> 29, 9 about even; eight runs of a token or two 14 .. 18, here 25 .. 29)
+    // The step's kernel walks a run at 0.6 us a token, the pieces below take 9 .. 29 us for up to 32: us of one run, step / pieces, 16 heads: key width 32 12 tokens 8.0 / 9.5, 16 10.1 / 9.4; 64 20 tokens 13.0 / 13.9, 24 14.3 / 14.0; 96 32
+    // tokens 19.5 / 25.8; 128 32 tokens 20.9 / 29.1
+    if (n_tok <= LA_TB && matrix && n_tok <= (int) gr * (dim == 32 ? 12 : dim == 64 ? 20 : LA_TB) && !key_sum && vdim % 32 == 0 && stride % 4 == 0 && out_stride % 4 == 0 && (((uintptr_t) v | (uintptr_t) out | (uintptr_t) state_dev) & 15) == 0) {
+#define LS_GO(NR) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_step<NR>, dim3((unsigned) heads, (unsigned) (vdim / 32), gr), dim3(256), 0, s, q, k, v, stride, heads, hpg, vdim, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, state_dev, \
+                               rec_dev, n_tok, out, out_stride, pi_abort_word())
+        LM_ANY(LS_GO);
+#undef LS_GO
+        PI_CHECK_LAUNCH(); return 0;
+    }
     if (matrix && n_tok <= LM_TB && (pieces || n_tok > 8 * gr)) {
         LM_ANY(LM_PIECES);
         PI_CHECK_LAUNCH(); return 0;

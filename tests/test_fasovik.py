@@ -434,6 +434,46 @@ def test_linear_attention_pieces_on_the_matrix_cores(H, G, D, V, per_token, key_
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V", [(3, 3, 32, 64), (2, 1, 64, 32), (2, 2, 96, 96), (4, 2, 128, 64)])
+@pytest.mark.parametrize("per_token", [False, True])
+def test_linear_attention_steps(H, G, D, V, per_token):
+    """passes of up to 32 tokens of whole key widths and columns: a token or some to a sequence, in any order, carried and fresh states, decays per head and per token, factors and a skip; both sides of the lines to the pieces; a value that is
+    no number stays in its column; a sequence that is not in the pass keeps its state"""
+    U, lib = gpu()
+    rng = np.random.default_rng(H * D + V)
+    slots, F = 9, 1 << 30
+    stride = 2 * G * D + H * V + 4
+    start = rng.standard_normal((slots, H, D, V)).astype(np.float32)
+    ref, sd, lam, skip = start.astype(np.float64), U.Dev(start), np.linspace(0.4, 0.999, H).astype(np.float32), rng.standard_normal(H).astype(np.float32)
+    for rec, most in (([4], 1), ([7 | F, 0, 3], 9), ([0, 0, 6 | F, 6, 6, 1], 9), ([5, 1, 0, 7, 2, 4, 6], 9), ([2] * 12, 1), ([2] * 13, 1), ([3] * 20, 1), ([3] * 21, 1), ([1] * 31 + [5 | F], 2), ([6] * 33, 1)):
+        T = len(rec)
+        buf = (rng.standard_normal((T, stride)) * 0.5).astype(np.float32)
+        dec, fac = np.exp(-np.exp(rng.standard_normal((T, H)) * 3 - 4)).astype(np.float32), rng.uniform(0.1, 2.0, (T, H)).astype(np.float32)
+        q, k, v = (buf[:, a:b].reshape(T, n, -1).astype(np.float64) for a, b, n in ((0, G * D, G), (G * D, 2 * G * D, G), (2 * G * D, 2 * G * D + H * V, H)))
+        ds = [U.Dev(a) for a in (buf, np.array(rec, np.int32), lam, dec, fac, skip)]
+        od, n = U.Dev(nbytes=4 * T * H * V), lib.pi_op_linear_attention_scratch_floats(H, D, V, T, most)
+        scr = U.Dev(np.full(max(n, 1), np.nan, np.float32))
+        L.check(lib.pi_op_linear_attention_keysum(ds[0].ptr, ds[0].ptr + 4 * G * D, ds[0].ptr + 8 * G * D, stride, H, G, D, V, 0, None if per_token else ds[2].ptr, ds[3].ptr if per_token else None,
+                                                  ds[4].ptr if per_token else None, H, ds[5].ptr if per_token else None, sd.ptr, ds[1].ptr, T, most, scr.ptr, n, od.ptr, H * V, None))
+        want, g = np.zeros((T, H, V)), np.arange(H) // (H // G)
+        for t in range(T):
+            s = rec[t] & ~F
+            if rec[t] & F:
+                ref[s] = 0.0
+            a, f = (dec[t], fac[t]) if per_token else (lam, np.ones(H))
+            ref[s] = ref[s] * a.astype(np.float64)[:, None, None] + k[t][g][:, :, None] * (v[t] * f.astype(np.float64)[:, None])[:, None, :]
+            want[t] = np.einsum("hd,hdv->hv", q[t][g], ref[s]) + (skip.astype(np.float64)[:, None] * v[t] if per_token else 0.0)
+        assert rel_rms(od.get(np.float32, (T, H, V)), want) < 2e-5, (rec, most)
+    got = sd.get(np.float32, start.shape)
+    assert np.array_equal(got[8], start[8]) and rel_rms(got, ref) < 2e-5
+    buf[:, 2 * G * D + 5] = np.inf                                   # (one column of the first head's values)
+    bd, rc, od = U.Dev(buf[:3]), U.Dev(np.array([8, 8, 8], np.int32)), U.Dev(nbytes=4 * 3 * H * V)
+    L.check(lib.pi_op_linear_attention_keysum(bd.ptr, bd.ptr + 4 * G * D, bd.ptr + 8 * G * D, stride, H, G, D, V, 0, ds[2].ptr, None, None, H, None, sd.ptr, rc.ptr, 3, 1, None, 0, od.ptr, H * V, None))
+    odd = ~np.isfinite(od.get(np.float32, (3, H, V)))
+    assert odd[:, 0, 5].all() and odd.sum() == 3
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [32, 24])
 @pytest.mark.parametrize("lengths", [[1] * 5, [1] * 30, [2, 1, 3] * 40, [1] * 255 + [70], [1] * 3 + [130] + [1, 2] * 35 + [64, 65]])
 def test_linear_attention_of_many_sequences(D, lengths):
