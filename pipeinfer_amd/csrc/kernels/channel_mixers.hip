@@ -126,6 +126,75 @@ __global__ void __launch_bounds__(256) k_rms_post(const float * __restrict__ a, 
         if (rd.h) rd.h[t * rd.stride + i] = pi_round_one(y);
     } }
 }
+// The same in loads of 16 bytes, for rows whose places and lengths allow them: a thread has NV times four values.  A row of a step is bound by its one trip to memory and by how many loads a thread has on it, many rows by memory.
+// Every sum has a place of its own in LDS: a barrier each.  us of one norm / with two inputs and a second norm, before -> now: one row of 2048 3.6 / 5.7 -> 2.2 / 3.2, eight rows of 4096 5.5 / 8.5 -> 3.2 / 4.8, 333 of 2048 4.4 / 7.0 ->
+// 3.1 / 5.1, 2048 of 4096 19.6 / 34 -> 15.6 / 26, one of 8192 11.4 / 20.0 -> 2.6 / 5.2, 2048 of 8192 50 / 112 -> 31 / 75
+template <int NV, int NT>
+__global__ void __launch_bounds__(NT) k_rms_post4(const float * __restrict__ a, int64_t as, const float * __restrict__ wa, const float * __restrict__ b, int64_t bs, const float * __restrict__ wb, float mb,
+                                                  const float * __restrict__ ls, const float * __restrict__ x, int64_t xs, float alpha, const float * __restrict__ w, float eps, int n,
+                                                  float * __restrict__ out, int64_t os, const float * __restrict__ w_next, float * __restrict__ out_next, int64_t ons, const pi_round_dst rd, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w);
+    __shared__ float red[4][16];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = (int) (blockDim.x >> 6);
+    float4 m[NV], v[NV], pwa[NV], pwb[NV], pls[NV], px[NV], pw[NV], pwn[NV];
+    const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f), one = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+#pragma unroll
+    for (int j = 0; j < NV; j++) {                                     // (behind the row's end: its last values, which count for nothing)
+        const int i = min(4 * (j * (int) blockDim.x + tid), n - 4);
+        m[j] = *(const float4 *) (a + (int64_t) t * as + i); px[j] = *(const float4 *) (x + (int64_t) t * xs + i); pw[j] = *(const float4 *) (w + i);
+        v[j] = none; pwa[j] = none; pwb[j] = none; pwn[j] = none; pls[j] = one;
+        if (b) { v[j] = *(const float4 *) (b + (int64_t) t * bs + i); pwa[j] = *(const float4 *) (wa + i); pwb[j] = *(const float4 *) (wb + i); }
+        if (ls) pls[j] = *(const float4 *) (ls + i);
+        if (w_next) pwn[j] = *(const float4 *) (w_next + i);
+    }
+    auto in = [&](int j) { return 4 * (j * (int) blockDim.x + tid) < n; };
+    auto square = [&](const float4 & y, float s) { return fmaf(y.w, y.w, fmaf(y.z, y.z, fmaf(y.y, y.y, fmaf(y.x, y.x, s)))); };
+    auto leave = [&](int k, float s) __attribute__((always_inline)) { s = pi_lanes_sum<64>(s); if (lane == 0) red[k][wave] = s; };
+    auto whole = [&](int k) __attribute__((always_inline)) { float s = (lane & 15) < nw ? red[k][lane & 15] : 0.0f; pi_butterfly<8>([&](auto o) { s += pi_partner<decltype(o)::value>(s); }); return 1.0f / sqrtf(s / (float) n + eps); };
+    if (b) {
+        float sa = 0.0f, sb = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; j++) if (in(j)) { sa = square(m[j], sa); sb = square(v[j], sb); }
+        leave(0, sa); leave(1, sb);
+        __syncthreads();
+        const float ia = whole(0), ib = whole(1);
+#pragma unroll
+        for (int j = 0; j < NV; j++)
+            m[j] = make_float4(mb * (m[j].x * ia * pwa[j].x + v[j].x * ib * pwb[j].x), mb * (m[j].y * ia * pwa[j].y + v[j].y * ib * pwb[j].y), mb * (m[j].z * ia * pwa[j].z + v[j].z * ib * pwb[j].z), mb * (m[j].w * ia * pwa[j].w + v[j].w * ib * pwb[j].w));
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        v[j] = make_float4(fmaf(alpha, px[j].x, pls[j].x * m[j].x), fmaf(alpha, px[j].y, pls[j].y * m[j].y), fmaf(alpha, px[j].z, pls[j].z * m[j].z), fmaf(alpha, px[j].w, pls[j].w * m[j].w));
+        if (in(j)) ss = square(v[j], ss);
+    }
+    leave(2, ss);
+    __syncthreads();
+    const float inv = whole(2);
+    if (pi_abort_late(gone, abort_w)) return;
+    float s2 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; j++) {
+        v[j] = make_float4(v[j].x * inv * pw[j].x, v[j].y * inv * pw[j].y, v[j].z * inv * pw[j].z, v[j].w * inv * pw[j].w);
+        if (in(j)) { *(float4 *) (out + (int64_t) t * os + 4 * (j * (int) blockDim.x + tid)) = v[j]; s2 = square(v[j], s2); }
+    }
+    if (!w_next) {
+        if (rd.h)
+#pragma unroll
+            for (int j = 0; j < NV; j++) if (in(j)) pi_round_store4(rd, t, 4 * (j * (int) blockDim.x + tid), v[j].x, v[j].y, v[j].z, v[j].w);
+        return;
+    }
+    leave(3, s2);
+    __syncthreads();
+    const float inv2 = whole(3);
+#pragma unroll
+    for (int j = 0; j < NV; j++) if (in(j)) {
+        const int i = 4 * (j * (int) blockDim.x + tid);
+        const float4 y = make_float4(v[j].x * inv2 * pwn[j].x, v[j].y * inv2 * pwn[j].y, v[j].z * inv2 * pwn[j].z, v[j].w * inv2 * pwn[j].w);
+        if (!rd.only) *(float4 *) (out_next + (int64_t) t * ons + i) = y;
+        if (rd.h) pi_round_store4(rd, t, i, y.x, y.y, y.z, y.w);
+    }
+}
 extern "C" int pi_op_rms_post(const float * a, int64_t a_stride, const float * wa, const float * b, int64_t b_stride, const float * wb, float mean_mult, const float * layer_scale, const float * x, int64_t x_stride,
                               float alpha, const float * w, float eps, int n, int n_tok, float * out, int64_t out_stride, const float * w_next, float * out_next, int64_t out_next_stride, void * stream) {
     if (n_tok <= 0 || n <= 0) return 0;
@@ -134,6 +203,17 @@ extern "C" int pi_op_rms_post(const float * a, int64_t a_stride, const float * w
     if (w_next && !out_next) { pi_set_error("pi_op_rms_post: a second norm needs a place for its result"); return -1; }
     const double bytes = 4.0 * n * n_tok * (3.0 + (b ? 1 : 0) + (w_next ? 1 : 0));
     const pi_round_dst rd = pi_round_asked(0, n);                      // (of the second norm where there is one)
+    const uintptr_t at = (uintptr_t) a | (uintptr_t) wa | (uintptr_t) b | (uintptr_t) wb | (uintptr_t) layer_scale | (uintptr_t) x | (uintptr_t) w | (uintptr_t) out | (uintptr_t) w_next | (uintptr_t) out_next;
+    const int64_t apart = a_stride | (b ? b_stride : 0) | x_stride | out_stride | (w_next ? out_next_stride : 0) | (rd.h ? rd.stride : 0) | n;
+    // workgroups of 256 up to what a thread's registers hold, beyond of 1024 (of 1024 from the start: eight rows of 4096 and two norms 5.0 us, 4.8 so, 2048 rows 28.6 and 26.4)
+    if ((at & 15) == 0 && ((uintptr_t) rd.h & 7) == 0 && (apart & 3) == 0) {
+        const int threads = std::min(n > 4096 ? 1024 : 256, (n / 4 + 63) / 64 * 64);
+#define RP_GO4(N, T) PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, (k_rms_post4<N, T>), dim3((unsigned) n_tok), dim3((unsigned) threads), 0, (hipStream_t) stream, a, a_stride, wa, b, b_stride, wb, mean_mult, layer_scale, x, x_stride, alpha, w, eps, n, \
+                                  out, out_stride, w_next, out_next, out_next_stride, rd, pi_abort_word())
+        if (n <= 1024) RP_GO4(1, 256); else if (n <= 2048) RP_GO4(2, 256); else if (n <= 4096) RP_GO4(4, 256); else RP_GO4(2, 1024);
+#undef RP_GO4
+        PI_CHECK_LAUNCH(); return 0;
+    }
 #define RP_GO(N, P) PI_KT_LAUNCH(PI_KT_OTHER, 0, 1, bytes, (k_rms_post<N, P>), dim3((unsigned) n_tok), dim3(256), 0, (hipStream_t) stream, a, a_stride, wa, b, b_stride, wb, mean_mult, layer_scale, x, x_stride, alpha, w, eps, n, \
                               out, out_stride, w_next, out_next, out_next_stride, rd, pi_abort_word())
     if (n <= 256 * 2) RP_GO(2, true); else if (n <= 256 * 4) RP_GO(4, true); else if (n <= 256 * 8) RP_GO(8, true); else if (n <= 256 * 16) RP_GO(16, true); else RP_GO(32, false);

@@ -281,6 +281,27 @@ def test_sublayer_end_with_one_and_two_inputs(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [4, 252, 260, 1024, 1028, 2048, 2052, 4096, 4100, 8192])
+@pytest.mark.parametrize("T", [1, 70])
+def test_sublayer_end_in_loads_of_16_bytes(n, T):
+    """rows whose places and lengths are multiples of four values, around what each instance holds: one and two inputs, with and without layer scale and second norm, in place; what stands behind a row stays"""
+    U, lib = gpu()
+    rng = np.random.default_rng(n + T)
+    a, b, x = ((rng.standard_normal((T, n + 4)) * 3).astype(np.float32) for _ in range(3))
+    wa, wb, ls, w, wn = (rng.standard_normal(n).astype(np.float32) for _ in range(5))
+    ad, bd, xd, od, nd = U.Dev(a), U.Dev(b), U.Dev(x), U.Dev(nbytes=4 * T * n), U.Dev(nbytes=4 * T * n)
+    ws = [U.Dev(v) for v in (wa, wb, ls, w, wn)]
+    a64, b64, x64 = (y[:, :n].astype(np.float64) for y in (a, b, x))
+    unit = lambda y: y / np.sqrt((y * y).mean(1, keepdims=True) + 1e-3)
+    L.check(lib.pi_op_rms_post(ad.ptr, n + 4, None, None, 0, None, 1.0, None, xd.ptr, n + 4, -0.5, ws[3].ptr, 1e-3, n, T, od.ptr, n, None, None, 0, None))
+    assert rel_rms(od.get(np.float32, (T, n)), unit(-0.5 * x64 + a64) * w) < 2e-6
+    two = unit(1.7 * x64 + ls * 0.5 * (unit(a64) * wa + unit(b64) * wb)) * w
+    L.check(lib.pi_op_rms_post(ad.ptr, n + 4, ws[0].ptr, bd.ptr, n + 4, ws[1].ptr, 0.5, ws[2].ptr, xd.ptr, n + 4, 1.7, ws[3].ptr, 1e-3, n, T, xd.ptr, n + 4, ws[4].ptr, nd.ptr, n, None))
+    assert rel_rms(xd.get(np.float32, (T, n + 4))[:, :n], two) < 3e-6 and rel_rms(nd.get(np.float32, (T, n)), unit(two) * wn) < 4e-6
+    assert np.array_equal(xd.get(np.float32, (T, n + 4))[:, n:], x[:, n:])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n,n_mix", [(7, 1), (300, 5), (64, 3)])
 def test_token_shift_over_sequences_and_passes(n, n_mix):
     """three sequences, passes of 1..40 tokens (both entries of the operator), a slot handed to a new owner over the old owner's row"""
