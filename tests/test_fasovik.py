@@ -583,6 +583,32 @@ def test_latent_attention_sink_takes_its_share():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_out,top", [(1, 1), (2, 2), (10, 2), (63, 8), (64, 16), (64, 17), (64, 64), (65, 3)])
+@pytest.mark.parametrize("by_logit", [False, True])
+def test_choice_of_outputs_around_a_wave(n_out, top, by_logit):
+    """soft-max over all outputs and a correction, or over the chosen logits: as many outputs as a wave has lanes, one less, one more; equal outputs, of which the first is chosen"""
+    U, lib = gpu()
+    rng = np.random.default_rng(n_out + top)
+    T, width = 5, 64
+    x, router = bf(rng, T, width), bf(rng, n_out, width, s=0.3)
+    router[n_out // 2:] = router[:n_out - n_out // 2]                  # (pairs of equal outputs)
+    corr = np.repeat(bf(rng, (n_out + 1) // 2, s=0.2), 2)[:n_out].copy()
+    corr[n_out // 2:] = corr[:n_out - n_out // 2]
+    rd, cd, xd, sel, selw = upload_bf16(lib, router), U.Dev(corr), U.Dev(x), U.Dev(nbytes=4 * T * top), U.Dev(nbytes=4 * T * top)
+    L.check((lib.pi_op_moe_route_top_logits if by_logit else lib.pi_op_moe_route)(rd, cd.ptr, xd.ptr, width, T, top, 1, sel.ptr, selw.ptr, None))
+    gs, gw = sel.get(np.int32, (T, top)), selw.get(np.float32, (T, top))
+    z = x.astype(np.float64) @ router.T.astype(np.float64)
+    p = np.exp(z - z.max(1, keepdims=True)); p /= p.sum(1, keepdims=True)
+    choice = z + corr if by_logit else p + corr
+    for t in range(T):
+        order = np.lexsort((np.arange(n_out), -np.round(choice[t], 9)))[:top]      # (equal outputs differ in the last bit of this sum)
+        assert list(gs[t]) == list(order)
+        want = np.exp(choice[t][order] - choice[t][order[0]]) / np.exp(choice[t][order] - choice[t][order[0]]).sum() if by_logit else p[t][order]
+        assert np.allclose(gw[t], want, rtol=2e-5)
+    lib.pi_weight_free(rd)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,I,top,ff,width", [(5, 2, 3, 24, 48), (1, 0, 1, 7, 33), (4, 4, 2, 64, 96), (0, 3, 2, 0, 40), (70, 3, 6, 16, 64)])
 @pytest.mark.parametrize("exact", [True, False])
 def test_router_and_experts(E, I, top, ff, width, exact):
