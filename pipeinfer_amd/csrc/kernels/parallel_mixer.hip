@@ -493,26 +493,33 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
     extern __shared__ float maps_lds[];                               // [2][V]
     const int t = blockIdx.x, h = blockIdx.y, map = threadIdx.x >> 6, lane = threadIdx.x & 63;        // a wave per map
     const float * pr = part + (((int64_t) t * H + h) * 2 + map) * n_cs * (V + 2);
-    // (the splits' maxima and denominators are read side by side, a lane per split: n_cs <= CA_SPLIT_MAX <= 64)
-    const float ms_l = lane < n_cs ? pr[(int64_t) lane * (V + 2) + V] : -INFINITY;
+    // sixteen splits of 128 values on their way at a time, the first of them beside the splits' maxima and denominators, of which a lane has one each (n_cs <= CA_SPLIT_MAX <= 64).  Eight splits of 64 values,
+    // behind those, and weights through LDS: 4 tokens of 16 heads of 128 values, 26 splits 5.7 us, 5.2 so, 32 splits 5.5 and 4.4; in a model's step 6.6 and 5.8.  (One map, 128 values to two waves: no less)
+    float x[2][16];
+    auto ask = [&](int v0, int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int u = 0; u < 16; u++) x[c][u] = pr[(int64_t) min(s0 + u, n_cs - 1) * (V + 2) + min(v0 + 64 * c + lane, V - 1)];
+    };
+    const float ms_l = lane < n_cs ? pr[(int64_t) lane * (V + 2) + V] : -INFINITY, ls_l = lane < n_cs ? pr[(int64_t) lane * (V + 2) + V + 1] : 0.0f;
+    ask(0, 0);
     const float M = pi_wave_max(ms_l);
     const float f_l = ms_l != -INFINITY ? expf(ms_l - M) : 0.0f;
-    const float den = pi_lanes_sum<64>(f_l > 0.0f ? pr[(int64_t) lane * (V + 2) + V + 1] * f_l : 0.0f);
+    const float den = pi_lanes_sum<64>(f_l > 0.0f ? ls_l * f_l : 0.0f);
     if (pi_abort_late(gone, abort_w)) return;
-    for (int v0 = 0; v0 < V; v0 += 64) {
-        const int v = v0 + lane;
-        float a = 0.0f;
-        for (int s0 = 0; s0 < n_cs; s0 += 8) {                         // eight splits on their way at a time
-            float x[8];
+    for (int v0 = 0; v0 < V; v0 += 128) {
+        float a[2] = { 0.0f, 0.0f };
+        for (int s0 = 0; s0 < n_cs; s0 += 16) {
+            if (v0 + s0 > 0) ask(v0, s0);
 #pragma unroll
-            for (int u = 0; u < 8; u++) x[u] = pr[(int64_t) min(s0 + u, n_cs - 1) * (V + 2) + min(v, V - 1)];
-#pragma unroll
-            for (int u = 0; u < 8; u++) {
-                const float f = s0 + u < n_cs ? __shfl(f_l, s0 + u, 64) : 0.0f;
-                if (f > 0.0f) a = fmaf(x[u], f, a);
+            for (int u = 0; u < 16; u++) {
+                const float f = s0 + u < n_cs ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f_l), (s0 + u) & 63)) : 0.0f;
+                if (f > 0.0f) { a[0] = fmaf(x[0][u], f, a[0]); a[1] = fmaf(x[1][u], f, a[1]); }
             }
         }
-        if (v < V) maps_lds[map * V + v] = den > 0.0f ? a / den : 0.0f;
+#pragma unroll
+        for (int c = 0; c < 2; c++) if (v0 + 64 * c + lane < V) maps_lds[map * V + v0 + 64 * c + lane] = den > 0.0f ? a[c] / den : 0.0f;
     }
     __syncthreads();
     if (map == 0) ca_join_maps(maps_lds, maps_lds + V, V, mp, out_mult, out + (int64_t) t * os + (int64_t) h * V, lane);

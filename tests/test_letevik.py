@@ -313,6 +313,23 @@ def run_diff(U, lib, q, kc, vc, cpos, vis, pos, scale, size, keep, maps, lam, mu
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_kv", [15 * 64, 16 * 64, 16 * 64 + 1, 2048])
+@pytest.mark.parametrize("V", [64, 100, 128, 200])
+@pytest.mark.parametrize("maps", [2, 1])
+def test_merge_of_splits_around_sixteen(n_kv, V, maps):
+    """15, 16, 17 and 32 splits, most of them outside the window (what they hold is no number), value widths around what a merging wave asks for at a time"""
+    U, lib = gpu()
+    rng = np.random.default_rng(n_kv + V)
+    H, G, D, T = 4, 2, 64, 2
+    q, kc, vc = rng.standard_normal((T, H, maps, D)).astype(np.float32), rng.standard_normal((n_kv, G, maps, D)).astype(np.float32), rng.standard_normal((n_kv, G, V)).astype(np.float32)
+    cpos, pos = np.arange(n_kv, dtype=np.int32), np.array([n_kv - 3, n_kv - 1])
+    vis = cpos[None, :] <= pos[:, None]
+    for size in (n_kv, 200):
+        a = (q, kc, vc, cpos, vis, pos, 0.3, size, 3, maps, 0.4, 1.3, 1e-5, H, G)
+        assert rel_rms(run_diff(U, lib, *a, True), diff_attention_ref(*a)) < 2e-5, size
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,D,V,size,keep,n_kv,T", [(1, 1, 4, 6, 3, 2, 20, 2), (3, 1, 8, 6, 7, 0, 70, 5), (8, 2, 40, 72, 48, 6, 700, 9), (4, 4, 33, 130, 100, 300, 320, 4), (12, 2, 16, 24, 0, 0, 520, 3),
                                                        (2, 2, 64, 64, 300, 1, 1100, 2), (4, 2, 96, 64, 9, 33, 400, 70), (32, 1, 64, 128, 60, 4, 300, 3), (2, 1, 1, 1, 1, 1, 40, 1)])
 @pytest.mark.parametrize("maps", [2, 1])
