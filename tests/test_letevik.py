@@ -460,6 +460,16 @@ def latent_case(U, lib, rng, H, D, R, V, rank, n_kv, pos, base, pairing, gate_wi
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,H,V,rank,n_kv", [(1, 3, 40, 256, 8 * 32 + 1), (4, 3, 64, 512, 16 * 32), (3, 2, 128, 512, 16 * 32 + 1), (2, 4, 64, 256, 64 * 32 + 1), (5, 2, 64, 1024, 700), (4, 64, 128, 256, 300), (5, 64, 128, 256, 300)])
+def test_merge_of_many_latent_splits(T, H, V, rank, n_kv):
+    """9, 16, 17 and 65 splits of 32 cells, one to four tokens of a workgroup and a token more, ranks of one and of two rounds of a wave's weights; both sides of two workgroups a compute unit; a gate per value, with and without a sink"""
+    U, lib = gpu()
+    for sink in (None, np.linspace(-1.0, 2.0, H)):
+        got, want = latent_case(U, lib, np.random.default_rng(T + n_kv), H, 32, 0, V, rank, n_kv, np.arange(n_kv - T, n_kv), 10000.0, NEIGHBOURS, V, sink, 0.1)
+        assert rel_rms(got, want) < 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,D,R,V,rank", [(3, 7, 6, 5, 12), (1, 1, 2, 1, 2), (16, 32, 16, 24, 64), (5, 70, 66, 40, 136), (4, 8, 64, 8, 512), (2, 6, 0, 7, 20), (20, 16, 8, 18, 300)])
 @pytest.mark.parametrize("T,n_kv", [(1, 33), (1, 700), (5, 90), (70, 70), (33, 400)])
 def test_latent_attention_with_a_sink_and_a_gate_per_value(H, D, R, V, rank, T, n_kv):
