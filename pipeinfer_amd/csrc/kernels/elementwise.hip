@@ -932,11 +932,16 @@ __global__ void __launch_bounds__(256) k_topk_out(const int32_t * __restrict__ p
 
 // bytes of caller-owned scratch pi_op_topk needs for n_tok rows (one buffer per stream: contexts decode concurrently)
 extern "C" size_t pi_op_topk_scratch_bytes(int n_tok) { return (size_t) n_tok * TOPK_NCH * (2 * 8 + 2) * 4; }
+// (the scratch is sized for k = 8, and the merge has room for its candidates alone)
+static int topk_refuses(int k, const void * scratch) {
+    if (k < 0 || k > 8) { pi_set_error(k > 8 ? "pi_op_topk: k=%d > 8" : "pi_op_topk: k=%d < 0", k); return -1; }
+    if (!scratch) { pi_set_error("pi_op_topk: scratch is NULL (needs pi_op_topk_scratch_bytes(n_tok) bytes)"); return -1; }
+    return 0;
+}
 // the slices' bests of every row, left in the scratch for pi_op_topk_merge or pi_op_topk_out
 extern "C" int pi_op_topk_parts(const float * logits, int n_vocab, int n_tok, int k, void * scratch, void * stream) {
     if (n_tok <= 0) return 0;
-    if (k > 8) { pi_set_error("pi_op_topk: k=%d > 8", k); return -1; }
-    if (!scratch) { pi_set_error("pi_op_topk: scratch is NULL (needs pi_op_topk_scratch_bytes(n_tok) bytes)"); return -1; }
+    if (topk_refuses(k, scratch) != 0) return -1;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
     // One wave to a slice: candidates cost the same for every k, rounds some 0.4 us each of them.  us by rounds / candidates, vocabulary 32000: one row k = 8 6.5 / 5.7, 4 5.6 / 5.6, 2 4.8 / 5.5; 8 rows k = 8 6.6 / 6.0, 4 5.3 / 5.9;
     // 24 rows k = 8 6.3 / 6.4; 64 rows 8.0 / 7.3, k = 4 6.4 / 7.1; 256 rows k = 4 14.2 / 12.1, 2 11.5 / 12.4.  Slices of 32 values a lane: 8 rows of 50257 k = 8 9.4 / 8.3, 4 8.0 / 8.6; 16 of 65536 k = 8 9.4 / 10.2
@@ -950,6 +955,7 @@ extern "C" int pi_op_topk_parts(const float * logits, int n_vocab, int n_tok, in
 }
 extern "C" int pi_op_topk_merge(const void * scratch, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * stream) {
     if (n_tok <= 0) return 0;
+    if (topk_refuses(k, scratch) != 0) return -1;
     PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2, dim3((n_tok + 3) / 4), dim3(256), 0, (hipStream_t) stream, k, n_tok, (const int32_t *) scratch, ids, vals, sumexp, pi_abort_word());
     PI_CHECK_LAUNCH(); return 0;
 }
@@ -959,6 +965,9 @@ extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, i
 }
 // rows [row0, row0 + n_tok) of a pass whose pi_op_topk_parts took k = 8
 extern "C" int pi_op_topk_out(const void * scratch, int row0, int n_tok, int32_t * ids_host, float * vals_host, float * sum_host, const float * logits_dev, float * logits_host, int64_t n_logits, void * stream) {
+    if (row0 < 0 || n_tok < 0 || n_logits < 0) { pi_set_error("pi_op_topk_out: rows [%d, + %d), %lld logits", row0, n_tok, (long long) n_logits); return -1; }
+    if (n_tok > 0 && topk_refuses(8, scratch) != 0) return -1;
+    if ((n_tok > 0 && (!ids_host || !vals_host || !sum_host)) || (n_logits > 0 && (!logits_dev || !logits_host))) { pi_set_error("pi_op_topk_out: a place to write to or the logits are NULL"); return -1; }
     const int merges = (n_tok + 3) / 4;
     const unsigned copies = (unsigned) std::min<int64_t>(256, (n_logits + 4095) / 4096);                       // four 16-byte stores per thread
     if (merges + copies == 0) return 0;
