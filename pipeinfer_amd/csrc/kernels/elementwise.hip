@@ -688,8 +688,9 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // What bounds it: picking the k best (8 MB of logits a millisecond of reading is nothing beside it).  A wave holds its values in registers as order-preserving integers; a lane keeps its own best.  One way
 // to go on is a round for each of the k, two wave reductions and one rescan of the lane that lost its best.  The other, for one wave to a slice and many rounds (the rule is at the launch): the least of eight lane groups' bests
 // is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  The vector unit's instructions bounded many rows: the candidates' way
-// looks at its values as floats (two instructions each for the best, one for the floor), makes no keys, takes eight for an exponential, and adds the four sums across the lanes together.  us, vocabulary 32000, before / now: 2048
-// rows that a product has just written 127 / 88 (read again and again 86 / 59: 4.4 TB/s), 1000 47 / 34, 512 33 / 26, 333 19.7 / 15.3.  (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
+// looks at its values as floats (two instructions each for the best, one for the floor), makes no keys, takes ten for an exponential (pi_exp_below), and adds the four sums across the lanes together.  us of both launches, vocabulary 32000,
+// before / now: 2048 rows 86 / 63, 1000 49 / 37.6, 512 31 / 25.5, 333 25 / 21, 64 13.7 / 12.8.  (2^(x log2(e)) without a reduction, eight instructions, takes 2 us less of 2048 rows, but its errors are 1.4 times expf's.)
+// (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
 // (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
 // One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
@@ -705,12 +706,6 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
     int i = key == m && m != 0 ? id : 0x7fffffff;
     pi_butterfly<32>([&](auto o) { i = min(i, pi_partner<decltype(o)::value>(i)); });
     key = m; id = i;
-}
-// e^x of a value below the largest: 2^(x log2(e)) by the hardware, times what that product's rounding and log2(e)'s second part left out (expf's errors without its reduction and its ends of the range: 8 instructions, not 14).
-// Minus infinity: 0 (the correction is bounded), no number: no number; below 2^-126 0
-static __device__ __forceinline__ float topk_exp(float x) {
-    const float hi = x * 1.44269502f, c = fmaxf(x, -150.0f), lo = fminf(fmaf(c, 1.92596303e-8f, fmaf(c, 1.44269502f, -hi)), 1.0f), e = __builtin_amdgcn_exp2f(hi);
-    return fmaf(e * 0.693147182f, lo, e);
 }
 // the larger of what an exchange of a register with itself brings together
 template <typename T> static __device__ __forceinline__ uint32_t topk_across(T both) { return max((uint32_t) both[0], (uint32_t) both[1]); }
@@ -744,7 +739,7 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         if (pi_abort_late(gone, abort_w)) return;
         auto sum_up = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int m = 0; m < VPT; m++) s[m & 3] += topk_exp(rv[m] - first);
+            for (int m = 0; m < VPT; m++) s[m & 3] += pi_exp_below(rv[m] - first);
             // the four sums share the way across the lanes: behind two exchanges rows 0 .. 3 of sixteen lanes hold s[0], s[2], s[1] and s[3]
             const auto s01 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[0]), __float_as_int(s[1]), false, false), s23 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[2]), __float_as_int(s[3]), false, false);
             const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(__int_as_float(s01[0]) + __int_as_float(s01[1])), __float_as_int(__int_as_float(s23[0]) + __int_as_float(s23[1])), false, false);
@@ -812,8 +807,8 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         first = topk_value(top);
         if constexpr (VPT > 0) {
 #pragma unroll
-            for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[0] += topk_exp(rv[m] - first);
-        } else for (int i = own0; i < hi; i += STEP) s[0] += topk_exp(l[i] - first);
+            for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[0] += pi_exp_below(rv[m] - first);
+        } else for (int i = own0; i < hi; i += STEP) s[0] += pi_exp_below(l[i] - first);
         const float sum = pi_lanes_sum<64>(s[0]);
         if (lane == 0) met_sum[wave] = sum;
     }

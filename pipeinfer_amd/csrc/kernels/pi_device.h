@@ -112,6 +112,13 @@ static __device__ __forceinline__ bool pi_aborted_together(int peek, const int32
 // A run's tokens sit in consecutive cells from kv_head (find_slot, llama.cpp:1593-1644); a pass that carries several runs at once (context.cpp: coalescing) brings a table.
 static __device__ __forceinline__ int pi_cell_of(const int32_t * dyn, int kv_head, int i) { return dyn ? (dyn[3] ? dyn[4 + i] : dyn[0] + i) : kv_head + i; }
 
+// e^x of a value below a maximum (or up to e^8), by Cody and Waite's reduction in two parts: x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
+// errors of expf (rms 2.6e-8, at most 8.3e-8) without its two ends of the range.  Minus infinity: 0 (what the fused part gives below the bound), no number: no number
+static __device__ __forceinline__ float pi_exp_below(float x) {
+    const float t = fmaxf(x * 1.44269502f, -300.0f), r = rintf(t);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - r) + fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -t))), (int) r);
+}
+
 // rows to page-locked host memory, thread `tid` of `nthr`
 static __device__ __forceinline__ void pi_rows_out(const float * __restrict__ rows, float * __restrict__ rows_h, size_t n, size_t tid, size_t nthr) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -21,12 +21,6 @@ struct pa_args {
     float * state; int first, last;                                    // the cells in several launches: [token][head][vdim sums | maximum | denominator] between them
 };
 typedef float pa_f32x4 __attribute__((ext_vector_type(4)));
-// e^x of a score below the maximum (or up to e^8), by Cody and Waite's reduction in two parts: x log2(e) = r + f, 2^f by the hardware for |f| <= 1/2, f with what the product's rounding left out and log2(e)'s second part: the
-// errors of expf (rms 2.6e-8, at most 8.3e-8) without its two ends of the range.  Minus infinity: 0 (what the fused part gives below the bound), no number: no number
-static __device__ __forceinline__ float pa_exp(float x) {
-    const float t = fmaxf(x * 1.44269502f, -300.0f), r = rintf(t);
-    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - r) + fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -t))), (int) r);
-}
 static __device__ __forceinline__ pa_f32x4 pa_mfma(float a, float b, pa_f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 // a launch over the cells [cell0, cell1); maps = 2: see ca_join_maps.  false: sizes or alignment that the kernel does not take (pa_takes)

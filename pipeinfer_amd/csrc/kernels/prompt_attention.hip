@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(256, N1 == 0 && NK + 4 * NV > 16 ? 1 : 2) k_pr
                     const float from = m_run[u] == -INFINITY ? 0.0f : m_run[u];               // (scores of minus infinity alone: no weight, not a NaN)
                     float sum = 0.0f;
 #pragma unroll
-                    for (int c = 0; c < 4; c++) { const float e = pa_exp(s[u][c] - from); s[u][c] = e; sum += e; }
+                    for (int c = 0; c < 4; c++) { const float e = pi_exp_below(s[u][c] - from); s[u][c] = e; sum += e; }
                     l_run[u] += sum;                                                          // (a lane's own cells; the four of a query meet at the end)
                 } else
 #pragma unroll

@@ -420,7 +420,7 @@ __global__ void __launch_bounds__(256, 1) k_split_attention(const pa_args A, con
             float sum = 0.0f;
             auto task = [&](int i) __attribute__((always_inline)) {
                 const int d = i / 3;
-                if (i % 3 < 2) { const float e = pa_exp(s[2 * d + i % 3] - from); s[2 * d + i % 3] = e; sum += e; }
+                if (i % 3 < 2) { const float e = pi_exp_below(s[2 * d + i % 3] - from); s[2 * d + i % 3] = e; sum += e; }
                 else { uint32_t hi, mid, lo; sa_split(s[2 * d], s[2 * d + 1], hi, mid, lo); w[d >> 2][0][d & 3] = hi; w[d >> 2][1][d & 3] = mid; w[d >> 2][2][d & 3] = lo; }
             };
             if constexpr (MORE) scores(cn, then, std::integral_constant<int, (300 + 6 * KS - 1) / (6 * KS)>{}, [&](int i) __attribute__((always_inline)) {
@@ -493,7 +493,7 @@ __global__ void __launch_bounds__(256, 1) k_split_attention(const pa_args A, con
             raise(0.0f);
             const float from = m_run == -INFINITY ? 0.0f : m_run;
 #pragma unroll
-            for (int i = 0; i < 16; i++) { s[i] = pa_exp(s[i] - from); l_run += s[i]; }
+            for (int i = 0; i < 16; i++) { s[i] = pi_exp_below(s[i] - from); l_run += s[i]; }
 #pragma unroll
             for (int j = 0; j < NJ; j++)
 #pragma unroll

@@ -638,6 +638,30 @@ def test_topk_candidates_of_few_and_many_rows(gpu, n_tok, k, n_vocab):
         assert abs(se.get(np.float32)[0] - want) / want < 1e-5      # (as test_topk_edges: fp32 sum of up to 32001 terms in pairs per slice)
 
 
+@pytest.mark.parametrize("n_vocab,k", [(2048, 8), (2048, 1), (32 * 2100, 8), (32 * 8200, 8)])
+def test_topk_exponentials(gpu, n_vocab, k):
+    """the exponentials behind the soft-max sums are as exact as expf's: a slice of one maximum and 63 equal values, a lane each, whose sum in pairs rounds six times and no more, so that an exponential's own error shows in
+    it.  On the candidates' way, on the rounds', by four waves with values in registers and with values read again"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    rows, per = 256, n_vocab // 32
+    x = -np.random.default_rng(k).uniform(1.0, 3.0, (rows, 32)).astype(np.float32)
+    l = np.full((rows, 32, per), -np.inf, np.float32)
+    l[:, :, :64] = x[:, :, None]
+    l[:, :, 5] = 0.0
+    ld, scr = U.Dev(l), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(rows))
+    L.check(lib.pi_op_topk_parts(ld.ptr, n_vocab, rows, k, scr.ptr, None))
+    got = scr.get(np.float32)[:rows * 32 * (2 * k + 2)].reshape(rows, -1)[:, 32 * (2 * k + 1):].astype(np.float64)
+    e = np.exp(x.astype(np.float64))
+    want, tree = 1.0 + 63.0 * e, np.repeat(e[:, :, None], 64, 2)
+    tree[:, :, 5] = 1.0
+    while tree.shape[2] > 1:                                           # what the sums alone do: exponentials in 64 bits, sums of pairs in 32 (rms 4.7e-8)
+        tree = (tree[:, :, :tree.shape[2] // 2] + tree[:, :, tree.shape[2] // 2:]).astype(np.float32).astype(np.float64)
+    rms = lambda d: np.sqrt(((d / want) ** 2).mean())
+    # beside that: 0.9e-8 with exponentials of at most expf's error (rms 2.6e-8, of which the first sum's rounding takes some along), 2.1e-8 .. 2.5e-8 where 2^(x log2(e)) is taken without a reduction (3.6e-8); 8192 sums: known to 0.8 %
+    assert rms(got - want) < np.hypot(rms(tree[:, :, 0] - want), 1.6e-8)
+
+
 @pytest.mark.parametrize("n_vocab", [512, 32000, 65024])
 def test_topk(gpu, n_vocab):
     lib, U = gpu
