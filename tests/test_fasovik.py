@@ -474,6 +474,24 @@ def test_linear_attention_steps(H, G, D, V, per_token):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,T,most", [(32, 17, 2), (32, 24, 2), (32, 32, 3), (64, 21, 2), (64, 32, 3), (64, 32, 1)])
+def test_one_sequence_of_a_pass_that_may_have_several(D, T, most):
+    """one run of more tokens than a step's kernel is the quicker for goes to the pieces of the matrix cores, however many runs there might have been (up to eight tokens for each of them): the same bits as with room for one run"""
+    U, lib = gpu()
+    rng = np.random.default_rng(D + T)
+    H, V, F = 3, 64, 1 << 30
+    stride = 2 * H * D + H * V
+    buf, start, lam = rng.standard_normal((T, stride)).astype(np.float32), rng.standard_normal((4, H, D, V)).astype(np.float32), np.linspace(0.4, 0.999, H).astype(np.float32)
+    bd, rc, ld = U.Dev(buf), U.Dev(np.full(T, 2, np.int32)), U.Dev(lam)
+    got = []
+    for segments in (1, most):
+        sd, od = U.Dev(start), U.Dev(nbytes=4 * T * H * V)
+        L.check(lib.pi_op_linear_attention(bd.ptr, bd.ptr + 4 * H * D, bd.ptr + 8 * H * D, stride, H, D, V, ld.ptr, sd.ptr, rc.ptr, T, segments, None, 0, od.ptr, H * V, None))
+        got.append((od.get(np.uint32), sd.get(np.uint32)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [32, 24])
 @pytest.mark.parametrize("lengths", [[1] * 5, [1] * 30, [2, 1, 3] * 40, [1] * 255 + [70], [1] * 3 + [130] + [1, 2] * 35 + [64, 65]])
 def test_linear_attention_of_many_sequences(D, lengths):
