@@ -450,6 +450,9 @@ PI_API int pi_op_latent_attention_rot(const float * q_dev, int64_t q_stride, con
                                       int64_t gate_stride, int gate_act, float scale, int heads, int dim, int rot_dim, int vdim, int rank, const void * rotary_table, const int32_t * pos_dev, int n_tok, int n_kv,
                                       float * scratch_dev, size_t scratch_floats, float * out_dev, int64_t out_stride, const int32_t * dyn_dev, void * stream);
 PI_API size_t pi_op_latent_attention_rot_scratch_floats(int heads, int rank, int rot_dim, int n_tok, int n_kv);
+/* Prompts over a latent write out the keys and values of all n_kv cells where the scratch holds them: as they are, or, quicker, in three bfloat16 parts of 1.5 times the memory (ranks of 128 .. 512 in steps of 128, heads of 64 or 128 values
+ * with no rotated part or half as many, values of 64 or 128).  The floats that the parts of all cells need, beside the two functions above (0: other sizes, fewer than nine tokens); with less a pass takes the form of fewer launches */
+PI_API size_t pi_op_latent_attention_prompt_scratch_floats(int heads, int dim, int rot_dim, int vdim, int rank, int n_tok, int n_kv);
 
 /* ---- operators of plain pre-norm blocks, of latent attention in other pairs with a gate per value, and of differential attention ------------------------------------------------- */
 /* the residual between two sublayers of a pre-norm block: x <- x + y [+ shift] (y, shift [n] nullable) -> x_out (may be x_in), h = x / sqrt(mean(x^2) + eps) * w; rows of x are n floats apart */

@@ -110,6 +110,11 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) { err = "hipStreamCreate failed"; return false; }
     auto dev = [&](size_t bytes) -> void * { void * p = pi_malloc(std::max<size_t>(bytes, 16)); if (!p) err = pi_last_error(); return p; };
     const int nb = ctx->n_batch, width = hp.n_embd;
+    // the keys and values of a prompt's latents in parts: for all cells or not at all, up to 1 GB (16384 cells of 32 heads of 128 take 0.8)
+    auto prompt_floats = [&](const pi_hybrid_layer & H, int rot) {
+        const size_t n = pi_op_latent_attention_prompt_scratch_floats(H.heads, H.dim, rot, H.vdim, H.kv_rank, nb, ctx->n_ctx);
+        return n <= ((size_t) 1 << 28) ? n : 0;
+    };
     size_t lat = 0, rec = 0, in_w = 1, att_w = 1, up_w = 1, sel_w = 1, idx_n = 1, step_w = 0, mid_w = 0; bool positions = false;
     ctx->lat_off.assign(hp.hybrid.size(), 0); ctx->rec_off.assign(hp.hybrid.size(), 0);
     if (hp.n_recurrent() > 0 || hp.pair_buckets > 0) ctx->slots.reset(new state_slots(std::max(1, ctx->n_state_slots)));      // (the previous token of a pair embedding is per-sequence state as well)
@@ -129,7 +134,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
                 ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_window_attention_scratch_floats(H.left.heads * H.left.maps, H.left.vdim, nb));
             } else {
                 att_w = std::max(att_w, (size_t) row_of_4(H.latent.q_rank) + (size_t) H.heads * (H.dim + H.latent.rot_dim) + (size_t) H.heads * H.vdim + 4);
-                ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_latent_attention_rot_scratch_floats(H.heads, H.kv_rank, H.latent.rot_dim, nb, ctx->n_ctx));
+                ctx->lat_scratch_floats = std::max({ ctx->lat_scratch_floats, pi_op_latent_attention_rot_scratch_floats(H.heads, H.kv_rank, H.latent.rot_dim, nb, ctx->n_ctx), prompt_floats(H, H.latent.rot_dim) });
                 if (H.latent.window > 0) ctx->window_masks[H.latent.window] = nullptr;
             }
             positions = true;
@@ -180,7 +185,7 @@ static bool context_prepare_hybrid(llama_context * ctx, std::string & err) {
         if (H.cache_index >= 0) {
             if (ctx->n_ctx > pi_op_latent_attention_max_cells(H.kv_rank)) { err = "n_ctx = " + std::to_string(ctx->n_ctx) + " is beyond the latent-attention kernel at kv_rank " + std::to_string(H.kv_rank) + " (one score row per workgroup in LDS: n_ctx <= " + std::to_string(pi_op_latent_attention_max_cells(H.kv_rank)) + ")"; return false; }
             ctx->lat_off[i] = lat; lat += (size_t) ctx->n_ctx * H.kv_rank;
-            ctx->lat_scratch_floats = std::max(ctx->lat_scratch_floats, pi_op_latent_attention_scratch_floats(H.heads, H.kv_rank, nb, ctx->n_ctx));
+            ctx->lat_scratch_floats = std::max({ ctx->lat_scratch_floats, pi_op_latent_attention_scratch_floats(H.heads, H.kv_rank, nb, ctx->n_ctx), prompt_floats(H, 0) });
         }
         if (H.state_index >= 0) { ctx->rec_off[i] = rec; rec += (size_t) ctx->slots->size() * H.heads * H.dim * H.vdim; ctx->rec_scratch_floats = std::max(ctx->rec_scratch_floats, pi_op_linear_attention_scratch_floats(H.heads, H.dim, H.vdim, nb, ctx->slots->size())); }
         in_w = std::max(in_w, (size_t) H.in_rows()); att_w = std::max(att_w, (size_t) H.heads * H.vdim);

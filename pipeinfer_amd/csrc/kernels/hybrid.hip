@@ -2018,6 +2018,9 @@ extern "C" size_t pi_op_latent_attention_rot_scratch_floats(int heads, int rank,
     for (int few = 1; few <= std::min(n_tok, 32); few++) if (lat_rows_takes(heads, rank, rot_dim, few, n_ctx)) need = std::max(need, lat_rows_floats(heads, rank, rot_dim, few, n_ctx));
     return need;
 }
+extern "C" size_t pi_op_latent_attention_prompt_scratch_floats(int heads, int dim, int rot_dim, int vdim, int rank, int n_tok, int n_ctx) {
+    return n_tok >= PA_LATENT_TOKENS && sa_sizes(dim, rot_dim, vdim, rank) ? ((size_t) n_ctx + 63) / 64 * 64 * sa_cell_floats(heads, dim, rot_dim, vdim) : 0;
+}
 template <int M, int RPT> static int latent_reserve_one() {
     PI_CHECK_HIP(hipFuncSetAttribute((const void *) k_latent_scores<M, RPT>, hipFuncAttributeMaxDynamicSharedMemorySize, LAT_LDS_BUDGET + 4096));
     return 0;
@@ -2070,22 +2073,27 @@ static int latent_tiles_to(const lat_plan & p, const pa_args & a, int rank, int 
 // A prompt with its keys and values written out (prompt_attention.hip), in as few launches over the cells as the scratch memory allows.  How many live cells it took the pass for: 0 none, a.n_kv any
 static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, size_t scratch_floats, double bytes, hipStream_t s) {
     if ((rank & 7) || (a.k2_row & 3) || ((uintptr_t) cache & 15) || ((uintptr_t) scratch & 15)) return 0;
-    const size_t state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3;
-    size_t cells = 0;
-    auto fits = [&](size_t per_cell) {                                 // the cells of a launch, 0: too few
-        cells = ((size_t) a.n_kv + 63) / 64 * 64; a.state = nullptr;
-        if (cells * per_cell <= scratch_floats) return true;
-        cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
-        a.state = scratch + cells * per_cell;
-        return cells >= 1024;
+    const size_t state = (size_t) a.n_tok * a.heads * (a.vdim + 2) + 3, whole = ((size_t) a.n_kv + 63) / 64 * 64;
+    auto fits = [&](size_t per_cell) -> size_t {                       // the cells of a launch, 0: too few
+        if (whole * per_cell <= scratch_floats) return whole;
+        const size_t cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
+        return cells >= 1024 ? cells : 0;
     };
-    const bool split = sa_takes(a, rank) && fits(sa_cell_floats(a.heads, a.dim1, a.dim2, a.vdim));
-    if (!split && !fits((size_t) a.heads * (a.dim1 + a.vdim))) return 0;
+    // In three parts where that takes no more launches than keys and values as they are: of one launch each the parts are quicker at all sizes, but behind one that holds all live cells another one still costs two idle launches and
+    // the sums' way to memory and back.  us as they are in one / in parts in one / in parts in two, cells 3072: 32 heads of 128, rank 512, 512 tokens alone 66 / 53 / 70, 64 alone 27 / 24 / 33; 64 heads of 64 + 32, rank 256, 512 alone
+    // 87 / 74 / 98 (all 3072 cells 311 / 237 / 262 and 355 / 273 / 312: how many are live is not known here)
+    const size_t plain_cell = (size_t) a.heads * (a.dim1 + a.vdim), part_cell = sa_cell_floats(a.heads, a.dim1, a.dim2, a.vdim), plain = fits(plain_cell), parts = sa_takes(a, rank) ? fits(part_cell) : 0;
+    if (plain == 0) return 0;
+    auto launches = [](int to, size_t cells) { return (int) ((to + cells - 1) / cells); };
+    const int to_plain = latent_tiles_to(p, a, rank, launches(a.n_kv, plain), false), to_parts = parts > 0 ? latent_tiles_to(p, a, rank, launches(a.n_kv, parts), true) : 0;
+    const bool split = to_parts > 0 && launches(to_parts, parts) <= std::max(1, launches(to_plain, plain));
+    const size_t cells = split ? parts : plain;
+    const int to = split ? to_parts : to_plain;
+    a.state = cells < whole ? scratch + cells * (split ? part_cell : plain_cell) : nullptr;
     a.k1 = scratch; a.k1_row = (int64_t) a.heads * a.dim1; a.k1_head = a.dim1;
     a.v = scratch + cells * (size_t) a.k1_row; a.v_row = (int64_t) a.heads * a.vdim; a.v_head = a.vdim;
     a.k2 = cache + rank;
     if (!pa_takes(a, 1, PA_LATENT_TOKENS)) return 0;
-    const int to = latent_tiles_to(p, a, rank, (int) (((size_t) a.n_kv + cells - 1) / cells), split);
     if (to == 0 || (to < a.n_kv && !a.dyn)) return 0;
     a.live_max = to < a.n_kv ? to : 0;
     if (to == a.n_kv) a.rd = pi_round_asked(0, (int64_t) a.heads * a.vdim);      // (else other launches may be the ones that write)

@@ -616,8 +616,9 @@ __global__ void __launch_bounds__(256, 1) k_split_attention(const pa_args A, con
 }
 
 size_t sa_cell_floats(int heads, int dim, int rot, int vdim) { return (size_t) 3 * ((size_t) heads * (dim + vdim) + rot) / 2; }
+bool sa_sizes(int dim, int rot, int vdim, int rank) { return rank > 0 && rank % 128 == 0 && rank <= SA_MAX_RANK && (dim == 64 || dim == 128) && (rot == 0 || rot == dim / 2) && (vdim == 64 || vdim == 128); }
 bool sa_takes(const pa_args & a, int rank) {
-    return rank % 128 == 0 && rank <= SA_MAX_RANK && a.n_tok >= PA_LATENT_TOKENS && (a.dim1 == 64 || a.dim1 == 128) && (a.dim2 == 0 || a.dim2 == a.dim1 / 2) && (a.vdim == 64 || a.vdim == 128) && a.qs % 4 == 0 && ((uintptr_t) a.q & 15) == 0 && (int64_t) a.n_tok * ((a.n_kv + 31) / 32) < (1ll << 32);
+    return sa_sizes(a.dim1, a.dim2, a.vdim, rank) && a.n_tok >= PA_LATENT_TOKENS && a.qs % 4 == 0 && ((uintptr_t) a.q & 15) == 0 && (int64_t) a.n_tok * ((a.n_kv + 31) / 32) < (1ll << 32);
 }
 // scratch: 1.5 floats for every value of the cells [cell0, cell1) (sa_cell_floats), 16-byte aligned; cell0 a multiple of 64
 void sa_launch(const pa_args & a, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, double bytes, hipStream_t s) {

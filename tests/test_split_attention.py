@@ -2,7 +2,8 @@
 import numpy as np
 import pytest
 
-from tests.test_letevik import HALVES, NEIGHBOURS, O, gpu, latent_case, rel_rms
+from pipeinfer_amd import lib as L
+from tests.test_letevik import HALVES, NEIGHBOURS, SIGMOID, O, gpu, latent_case, rel_rms, upload_bf16
 
 BOUND = 2e-6        # fp32 sums of up to 512 + 192 + 1000 terms in tiles; rounding the products' inputs to bfloat16 would be 2e-3
 
@@ -72,3 +73,95 @@ def test_split_attention_of_small_and_large_values(scale):
     cache = (rng.standard_normal((n_kv, rank)) * scale).astype(np.float32)
     got, want = latent_case(U, lib, rng, H, D, 0, V, rank, n_kv, np.arange(n_kv - T, n_kv), 500.0, HALVES, 0, None, float(D ** -0.5 / scale), cache=cache)
     assert rel_rms(got, want) < BOUND
+
+
+def floats_of(cells, H, D, R, V):
+    return (cells + 63) // 64 * 64 * 3 * (H * (D + V) + R) // 2
+
+
+def state_of(T, H, V):
+    """sums, maximum and denominator between two launches over the cells"""
+    return T * H * (V + 2) + 3
+
+
+class Call:
+    """one call of the operator: tokens at `pos`, each of which sees the cells up to its own; `live` cells of n_kv are in use (the rest hold NaN), `floats` of scratch memory (none given: the parts of all cells in one launch).
+    out: its output; parts(cell0): whether the scratch holds the keys of the first head's cells from cell0 on as the first operand of three parts"""
+    def __init__(self, U, lib, rng, H, D, R, V, rank, n_kv, pos, pairing=HALVES, gate_width=0, sink=None, scale=None, cache=None, live=None, floats=None):
+        T, live, self.base, self.pairing, self.H, self.V = len(pos), n_kv if live is None else live, 500.0, pairing, H, V
+        self.D, self.R, self.rank, self.live, self.pos, self.gate_width, self.sink, self.scale = D, R, rank, live, np.asarray(pos), gate_width, sink, (D + R) ** -0.5 if scale is None else scale
+        self.Wk, self.Wv = (O.bf16_round((rng.standard_normal((H * s, rank)) / np.sqrt(rank)).astype(np.float32)) for s in (D, V))
+        self.q = rng.standard_normal((T, H, D + R)).astype(np.float32)
+        self.cache = np.full((n_kv, rank + R), np.nan, np.float32)
+        self.cache[:live] = rng.standard_normal((live, rank + R)) if cache is None else cache
+        self.g = rng.standard_normal((T, H * max(gate_width, 1) + 1)).astype(np.float32)
+        words = (n_kv + 31) // 32
+        self.vis = np.arange(words * 32)[None, :] <= self.pos[:, None]
+        mask = np.packbits(self.vis, axis=1, bitorder="little").view(np.uint32)
+        t = lib.pi_rotary_table_create(int(max(pos)) + 2, R, self.base) if R else None
+        uk, uv = upload_bf16(lib, self.Wk), upload_bf16(lib, self.Wv)
+        s = np.zeros(H, np.float32) if sink is None else np.asarray(sink, np.float32)
+        qd, cd, md, gd, sd, pd, dd = (U.Dev(a) for a in (self.q, self.cache, mask, self.g, s, self.pos.astype(np.int32), np.array([0, live, T, 0], np.int32)))
+        n = max(floats_of(n_kv, H, D, R, V) if floats is None else floats, lib.pi_op_latent_attention_rot_scratch_floats(H, rank, R, T, n_kv))
+        if floats is not None:
+            assert n == floats, "the per-token kernels' memory is more: not what the test is about"
+        scr, od = U.Dev(np.full(n, np.nan, np.float32)), U.Dev(nbytes=4 * T * H * V)
+        L.check(lib.pi_op_latent_attention_gated(qd.ptr, H * (D + R), cd.ptr, md.ptr, uk, uv, sd.ptr if sink is not None else None, gd.ptr if gate_width else None, self.g.shape[1], SIGMOID, max(gate_width, 1), self.scale, H, D, R, V,
+                                                 rank, t, pairing, pd.ptr, T, n_kv, scr.ptr, n, od.ptr, H * V, dd.ptr, None))
+        self.out, self.first = od.get(np.float32, (T, H, V)), scr.get(np.uint32, count=512 * 4)
+        lib.pi_weight_free(uk)
+        lib.pi_weight_free(uv)
+        if t:
+            lib.pi_rotary_table_free(t)
+
+    def keys(self, h, cell0=0, cells=None):
+        return self.cache[cell0:self.live if cells is None else min(cell0 + cells, self.live), :self.rank].astype(np.float64) @ self.Wk[h * self.D:(h + 1) * self.D].T.astype(np.float64)
+
+    def parts(self, cell0=0):
+        k = self.keys(0, cell0, 32)[:, :16]
+        got = (self.first.view(np.uint16)[:512].astype(np.uint32) << 16).view(np.float32).reshape(2, 32, 8).transpose(1, 0, 2).reshape(32, 16)[:len(k)]      # lane l: cell l % 32, values 8 (l / 32) .. + 7
+        return bool((np.abs(got - k) <= np.abs(k) * 2.0 ** -8 + np.abs(k).max() * 1e-5).all())
+
+    def want(self, h):
+        """head h of all tokens; a token's sums hold the cells that it sees and no others"""
+        rot, T = {"dims": self.R, "base": self.base}, len(self.pos)
+        k, v = self.keys(h), self.cache[:self.live, :self.rank].astype(np.float64) @ self.Wv[h * self.V:(h + 1) * self.V].T.astype(np.float64)
+        q = self.q[:, h].astype(np.float64)
+        if self.R:
+            k = np.concatenate([k, self.cache[:self.live, self.rank:].astype(np.float64)], 1)
+            q = np.concatenate([q[:, :self.D], np.stack([O.turn(q[t, self.D:], int(self.pos[t]), rot, self.pairing == NEIGHBOURS) for t in range(T)])], 1)
+        s, vis = (q @ k.T) * self.scale, self.vis[:, :self.live]
+        out = np.zeros((T, self.V))
+        if np.isfinite(v).all() and np.isfinite(s).all():
+            s = np.where(vis, s, -np.inf)
+            m = np.maximum(s.max(1), -np.inf if self.sink is None else self.sink[h])
+            e = np.exp(s - m[:, None])
+            out = e @ v / (e.sum(1) + (0.0 if self.sink is None else np.exp(self.sink[h] - m)))[:, None]
+        else:
+            for t in range(T):
+                out[t] = O.softmax(s[t][vis[t]], None if self.sink is None else self.sink[h]) @ v[vis[t]]
+        if self.gate_width:
+            out = out * O.sigmoid(self.g[:, h * self.gate_width:(h + 1) * self.gate_width])
+        return out
+
+    def error(self, heads=None):
+        heads = list(range(self.H) if heads is None else heads)
+        return rel_rms(self.out[:, heads], np.stack([self.want(h) for h in heads], 1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("live", [600, 3072])
+def test_parts_that_would_take_more_launches(live):
+    """scratch memory for the keys and values of all 3072 cells as they are, or for the parts of 1920: they are written as they are, in one launch"""
+    U, lib = gpu()
+    H, D, V, rank, n_kv, T = 32, 128, 128, 128, 3072, 256
+    c = Call(U, lib, np.random.default_rng(4), H, D, 0, V, rank, n_kv, np.arange(live - T, live), live=live, floats=n_kv * H * (D + V))
+    assert not c.parts(0) and not (live > 1920 and c.parts(1920)) and c.error(range(0, H, 7)) < BOUND
+    assert rel_rms(c.first.view(np.float32)[:16], c.keys(0, 0, 1)[0, :16]) < 1e-6
+
+
+def test_scratch_memory_of_the_parts():
+    """six bytes for every key and value of all cells, in whole blocks of 64; nothing where a pass does not take them"""
+    of = L.load().pi_op_latent_attention_prompt_scratch_floats
+    assert of(32, 128, 0, 128, 512, 512, 3000) == 3008 * 12288 and of(3, 64, 32, 128, 128, 9, 64) == 64 * 912
+    assert [of(3, 64, 0, 64, 128, 8, 64), of(3, 64, 16, 64, 128, 9, 64), of(3, 96, 0, 64, 128, 9, 64), of(3, 64, 0, 96, 128, 9, 64), of(3, 64, 0, 64, 64, 9, 64), of(3, 64, 0, 64, 640, 9, 64), of(3, 64, 0, 64, 0, 9, 64)] == [0] * 7
