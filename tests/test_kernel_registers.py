@@ -34,7 +34,7 @@ def scratch_of_kernels():
     return found
 
 
-@pytest.mark.parametrize("kernel", ["k_rms_scale_once", "k_prompt_attention"])
+@pytest.mark.parametrize("kernel", ["k_rms_scale_once", "k_prompt_attention", "k_split_attention", "k_latent_split", "k_linear_step", "k_channel_step", "k_rms_post4"])
 def test_kernels_without_scratch_memory(kernel):
     mine = {n: s for n, s in scratch_of_kernels().items() if kernel in n}
     assert mine and not any(mine.values()), mine
