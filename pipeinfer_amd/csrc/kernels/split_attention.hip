@@ -627,6 +627,9 @@ void sa_launch(const pa_args & a, const float * cache, int rank, const pi_weight
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, PI_KT_MAXNT - 1, 2.0 * rank * (wuk->ne1 + wuv->ne1) + 4.0 * std::min(a.cell1 - a.cell0, a.n_kv) * (double) (a.k2_row + 1.5 * (wuk->ne1 + wuv->ne1)), k_latent_split, dim3((unsigned) std::min(tiles, 256)), dim3(256), 0, s,
                  cache, a.k2_row, rank, (const uint16_t *) wuk->p0, (int) wuk->ne1, (const uint16_t *) wuv->p0, (int) wuv->ne1, a.dim1 == 64 ? 6 : 7, a.dim2, a.vdim == 64 ? 6 : 7, a.cell0, a.cell1, a.live_max, a.dyn, kf, rf, vf, runs, pi_abort_word());
     const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
+    // A wave for every 32 queries (a workgroup 128) reads keys and values once for 128 queries and has no sums to join; four waves that share the cells of 32 have four times the workgroups.  Measured over 120 sizes (16 .. 512 heads of
+    // 64 and 128, 64 .. 4096 tokens, their own cells and 4096), time of one wave / of four, by workgroups of 128 queries: 64 1.75 .. 2.37, 128 1.06 .. 1.65, 256 0.65 .. 1.2 (heads of 128, rank 512: 32 of them, 1024 tokens alone 116 / 113 us,
+    // 16, 2048 180 / 154, 128, 256 66 / 83), 384 0.8 .. 1.03, 512 0.73 .. 1.04 (32, 2048 251 / 301, 128, 512 138 / 180, 512, 64 79.4 / 78.8)
     const bool many = (int64_t) a.heads * ((a.n_tok + 127) / 128) >= 512;
 #define SA_GO(KO, KR, NJ, P) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_split_attention<KO, KR, NJ, P>), dim3((unsigned) a.heads, (unsigned) ((a.n_tok + 128 / P - 1) / (128 / P))), dim3(256), 0, s, a, kf, rf, vf, runs, pi_abort_word())
 #define SA_NJ(KO, KR) do { if (a.vdim == 64) { if (many) SA_GO(KO, KR, 2, 1); else SA_GO(KO, KR, 2, 4); } else if (many) SA_GO(KO, KR, 4, 1); else SA_GO(KO, KR, 4, 4); } while (0)
