@@ -690,7 +690,7 @@ extern "C" int pi_op_add(const float * a, const float * b, float * o, int64_t n,
 // is a floor that some 20 of 1000 values reach, each gets a lane and counts those ahead of it.  The vector unit's instructions bounded many rows: the candidates' way
 // looks at its values as floats (two instructions each for the best, one for the floor), makes no keys, takes ten for an exponential (pi_exp_below), and adds the four sums across the lanes together.  us of both launches, vocabulary 32000,
 // before / now: 2048 rows 86 / 63, 1000 49 / 37.6, 512 31 / 25.5, 333 25 / 21, 64 13.7 / 12.8.  (2^(x log2(e)) without a reduction, eight instructions, takes 2 us less of 2048 rows, but its errors are 1.4 times expf's.)
-// (k = 8, both kernels together, rounds / candidates: one row of 32000 12.7 / 11.4, 512 44.5 / 32.5, 2048 142 / 91; a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
+// (a workgroup per slice that looked at all its values in every round and met at a barrier: 607 for 2048 rows.)  WS waves share a slice.  One up to a vocabulary of 65536
 // (there one row 19.5 us for k = 8, 64 rows 18; four waves at 65537 14.5 and 28).  Beyond that, and for k = 1 of few rows (50257: 7.9 and 6.2), four, whose bests meet in LDS: a wave's registers would not hold its share.
 // One row of 128256 took 37 us on that workgroup, 117 on one wave that read its slice again in every round, now 15; of 256000 67, 224 and 20.  VPT = 0: values that no registers hold are read again in every round.
 // order-preserving integer of a value: -inf 0x007fffff .. +inf; 0 = not a number, or taken
@@ -711,17 +711,17 @@ static __device__ __forceinline__ void topk_best(uint32_t & key, int & id) {
 template <typename T> static __device__ __forceinline__ uint32_t topk_across(T both) { return max((uint32_t) both[0], (uint32_t) both[1]); }
 // a row's share of the scratch: the k best of every slice (ids, values), the slices' maxima and sums
 static __host__ __device__ __forceinline__ int topk_words(int k) { return TOPK_NCH * (2 * k + 2); }
-template <int VPT, int WS>
-__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int candidates, int32_t * __restrict__ part, const int32_t * __restrict__ abort_w) {
+template <int VPT, int WS, bool CANDIDATES>
+__global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits, int n_vocab, int k, int32_t * __restrict__ part, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     constexpr int STEP = 64 * WS;                                       // a slice's values from one of a lane's to its next
     __shared__ uint32_t met_key[WS > 1 ? 32 : 1]; __shared__ int met_id[WS > 1 ? 32 : 1]; __shared__ float met_sum[4];      // the four waves' bests
-    __shared__ float2 met[WS > 1 ? 1 : 256];                            // a wave's own candidates: value, number in the slice
+    __shared__ float2 met[CANDIDATES ? 256 : 1];                          // a wave's own candidates: value, number in the slice
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ch = WS > 1 ? blockIdx.y : blockIdx.y * 4 + wave;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH, lo = ch * per, hi = min(n_vocab, lo + per), own0 = lo + lane + (WS > 1 ? 64 * wave : 0);
     const float * l = logits + (int64_t) t * n_vocab;
     int32_t * cid = part + (int64_t) t * topk_words(k); float * cval = (float *) (cid + TOPK_NCH * k), * cmax = cval + TOPK_NCH * k, * csum = cmax + TOPK_NCH;
-    static_assert(VPT > 0 || WS > 1, "values that are read again: four waves");
+    static_assert(WS > 1 ? !CANDIDATES : VPT > 0, "candidates: a wave to a slice; values that are read again: four waves");
     uint32_t key[VPT > 0 ? VPT : 1]; float rv[VPT > 0 ? VPT : 1];
     uint32_t bk = 0, wk; int bm = 0, wi;                                // this lane's best among the ones not taken: key, number; the wave's
     float first, s[4] = { 0.0f, 0.0f, 0.0f, 0.0f };                     // the slice's largest, its sum of exponentials in the order of 256 threads of four waves
@@ -730,87 +730,87 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
         if constexpr (VPT > 0)
 #pragma unroll VPT
         for (int m = 0; m < VPT; m++) { key[m] = own0 + STEP * m < hi ? topk_key(rv[m]) : 0u; if (key[m] > bk) { bk = key[m]; bm = m; } }
+        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
+        topk_best(wk, wi);
     };
-    if constexpr (WS == 1) {
+    // a wave's four sums share the way across the lanes: behind two exchanges rows 0 .. 3 of sixteen lanes hold s[0], s[2], s[1] and s[3]
+    auto sums_out = [&]() __attribute__((always_inline)) {
+        const auto s01 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[0]), __float_as_int(s[1]), false, false), s23 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[2]), __float_as_int(s[3]), false, false);
+        const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(__int_as_float(s01[0]) + __int_as_float(s01[1])), __float_as_int(__int_as_float(s23[0]) + __int_as_float(s23[1])), false, false);
+        float sum = __int_as_float(rows[0]) + __int_as_float(rows[1]);
+        pi_butterfly<8>([&](auto o) { sum += pi_partner<decltype(o)::value>(sum); });
+        sum += pi_partner<32>(sum); sum += pi_partner<16>(sum);
+        if (lane == 0) { cmax[ch] = first; csum[ch] = sum; }
+    };
+    if constexpr (CANDIDATES) {
         // (what is past the slice's end adds nothing to the sum, and is no candidate)
         const float * at = l + min(lo, n_vocab - 1);
 #pragma unroll
         for (int m = 0; m < VPT; m++) { rv[m] = -INFINITY; if (lane < hi - lo - 64 * m) rv[m] = at[lane + 64 * m]; }
         if (pi_abort_late(gone, abort_w)) return;
-        auto sum_up = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int m = 0; m < VPT; m++) s[m & 3] += pi_exp_below(rv[m] - first);
-            // the four sums share the way across the lanes: behind two exchanges rows 0 .. 3 of sixteen lanes hold s[0], s[2], s[1] and s[3]
-            const auto s01 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[0]), __float_as_int(s[1]), false, false), s23 = __builtin_amdgcn_permlane32_swap(__float_as_int(s[2]), __float_as_int(s[3]), false, false);
-            const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(__int_as_float(s01[0]) + __int_as_float(s01[1])), __float_as_int(__int_as_float(s23[0]) + __int_as_float(s23[1])), false, false);
-            float sum = __int_as_float(rows[0]) + __int_as_float(rows[1]);
-            pi_butterfly<8>([&](auto o) { sum += pi_partner<decltype(o)::value>(sum); });
-            sum += pi_partner<32>(sum); sum += pi_partner<16>(sum);
-            if (lane == 0) { cmax[ch] = first; csum[ch] = sum; }
-        };
-        if (candidates) {
-            float best = -INFINITY;                                         // (what is no number is never above it)
+        for (int m = 0; m < VPT; m++) asm volatile("" : "+v"(rv[m]));   // (all loads on their way: what the compiler drew of a value's use into its load's branch waited there, value by value)
+        float best = -INFINITY;                                         // (what is no number is never above it)
 #pragma unroll
-            for (int m = 0; m < VPT; m++) best = rv[m] > best ? rv[m] : best;
-            uint32_t top = topk_key(best);
-            top = topk_across(__builtin_amdgcn_permlane32_swap(top, top, false, false)); top = topk_across(__builtin_amdgcn_permlane16_swap(top, top, false, false)); top = max(top, (uint32_t) pi_partner<8>((int) top));
-            uint32_t least = top;                                           // at least eight values are not below it: the least of the bests of eight lanes each (lanes of the same number mod 8)
-            pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); least = min(least, (uint32_t) pi_partner<O>((int) least)); });
-            first = topk_value(top);
-            const float low = topk_value(least);
-            sum_up();
-            if (low > -INFINITY) {
-                // what is not below `low` goes to a lane each, which counts those ahead of it
-                uint64_t who[VPT]; int n = 0;
+        for (int m = 0; m < VPT; m++) best = rv[m] > best ? rv[m] : best;
+        uint32_t top = topk_key(best);
+        top = topk_across(__builtin_amdgcn_permlane32_swap(top, top, false, false)); top = topk_across(__builtin_amdgcn_permlane16_swap(top, top, false, false)); top = max(top, (uint32_t) pi_partner<8>((int) top));
+        uint32_t least = top;                                           // at least eight values are not below it: the least of the bests of eight lanes each (lanes of the same number mod 8)
+        pi_butterfly<4>([&](auto o) { constexpr int O = decltype(o)::value; top = max(top, (uint32_t) pi_partner<O>((int) top)); least = min(least, (uint32_t) pi_partner<O>((int) least)); });
+        first = topk_value(top);
+        const float low = topk_value(least);
 #pragma unroll
-                for (int m = 0; m < VPT; m++) { who[m] = __ballot(rv[m] >= low); n += __popcll(who[m]); }
-                if (n <= 64) {                                              // (else, a crowd of equal values: the rounds below)
-                    int base = 0;
+        for (int m = 0; m < VPT; m++) s[m & 3] += pi_exp_below(rv[m] - first);
+        sums_out();
+        if (!(low > -INFINITY))                                         // (fewer than eight numbers above -inf in as many lanes: all numbers are picked)
 #pragma unroll
-                    for (int m = 0; m < VPT; m++) {
-                        if (rv[m] >= low) met[WS == 1 ? 64 * wave + base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[m], 0)) : 0] = make_float2(rv[m], __int_as_float(lane + 64 * m));
-                        base += __popcll(who[m]);
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    const float2 mine = lane < n ? met[WS == 1 ? 64 * wave + lane : 0] : make_float2(-INFINITY, 0.0f);
-                    const float cv = mine.x + 0.0f; const int ci = __float_as_int(mine.y);      // (-0 ties with +0)
-                    int ahead = 0;                                          // (a lower lane has a lower id)
-#pragma unroll 4
-                    for (int j = 0; j < n; j++) {
-                        const float vj = __uint_as_float((uint32_t) __builtin_amdgcn_readlane(__float_as_int(cv), j));
-                        const uint64_t is = __ballot(vj > cv) | (__ballot(vj == cv) & (~1ull << j));
-                        asm("v_addc_co_u32_e64 %0, vcc, %1, 0, %2" : "=v"(ahead) : "v"(ahead), "s"(is) : "vcc");
-                    }
-                    if (lane < n ? ahead < k : lane < k) { const int to = out + (lane < n ? ahead : lane); cid[to] = lane < n ? lo + ci : 0x7fffffff; cval[to] = mine.x; }
-                    return;
-                }
+            for (int m = 0; m < VPT; m++) if (lane >= hi - lo - 64 * m) rv[m] = __uint_as_float(0x7fc00000u);
+        // what is not below `low` goes to a lane each, which counts those ahead of it
+        uint64_t who[VPT]; int n = 0;
+#pragma unroll
+        for (int m = 0; m < VPT; m++) { who[m] = __ballot(rv[m] >= low); n += __popcll(who[m]); }
+        if (n <= 64) {                                                  // (else, a crowd of equal values: the rounds below)
+            int base = 0;
+#pragma unroll
+            for (int m = 0; m < VPT; m++) {
+                if (rv[m] >= low) met[CANDIDATES ? 64 * wave + base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[m], 0)) : 0] = make_float2(rv[m], __int_as_float(lane + 64 * m));
+                base += __popcll(who[m]);
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const float2 mine = lane < n ? met[CANDIDATES ? 64 * wave + lane : 0] : make_float2(-INFINITY, 0.0f);
+            const float cv = mine.x + 0.0f; const int ci = __float_as_int(mine.y);      // (-0 ties with +0)
+            int ahead = 0;                                              // (a lower lane has a lower id)
+#pragma unroll 4
+            for (int j = 0; j < n; j++) {
+                const float vj = __uint_as_float((uint32_t) __builtin_amdgcn_readlane(__float_as_int(cv), j));
+                const uint64_t is = __ballot(vj > cv) | (__ballot(vj == cv) & (~1ull << j));
+                asm("v_addc_co_u32_e64 %0, vcc, %1, 0, %2" : "=v"(ahead) : "v"(ahead), "s"(is) : "vcc");
+            }
+            if (lane < n ? ahead < k : lane < k) { const int to = out + (lane < n ? ahead : lane); cid[to] = lane < n ? lo + ci : 0x7fffffff; cval[to] = mine.x; }
+            return;
         }
         keys();
-        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
-        topk_best(wk, wi);
-        if (!candidates) { first = topk_value(wk); sum_up(); }
     } else {
         if constexpr (VPT > 0) {
 #pragma unroll
             for (int m = 0; m < VPT; m++) rv[m] = l[min(own0 + STEP * m, n_vocab - 1)];
-            keys();
         } else for (int i = own0, m = 0; i < hi; i += STEP, m++) { const uint32_t q = topk_key(l[i]); if (q > bk) { bk = q; bm = m; } }
         if (pi_abort_late(gone, abort_w)) return;
-        wk = bk; wi = bk ? own0 + STEP * bm : 0x7fffffff;
-        topk_best(wk, wi);
-        if (lane == 0) met_key[wave] = wk;
-        __syncthreads();
-        const uint32_t top = max(max(met_key[0], met_key[1]), max(met_key[2], met_key[3]));
-        __syncthreads();
+        keys();
+        uint32_t top = wk;
+        if constexpr (WS > 1) {
+            if (lane == 0) met_key[wave] = wk;
+            __syncthreads();
+            top = max(max(met_key[0], met_key[1]), max(met_key[2], met_key[3]));
+            __syncthreads();
+        }
         first = topk_value(top);
         if constexpr (VPT > 0) {
 #pragma unroll
-            for (int m = 0; m < VPT; m++) if (own0 + STEP * m < hi) s[0] += pi_exp_below(rv[m] - first);
+            for (int m = 0; m < VPT; m++) s[WS > 1 ? 0 : m & 3] += pi_exp_below((own0 + STEP * m < hi ? rv[m] : -INFINITY) - first);
         } else for (int i = own0; i < hi; i += STEP) s[0] += pi_exp_below(l[i] - first);
-        const float sum = pi_lanes_sum<64>(s[0]);
-        if (lane == 0) met_sum[wave] = sum;
+        if constexpr (WS > 1) { const float sum = pi_lanes_sum<64>(s[0]); if (lane == 0) met_sum[wave] = sum; } else sums_out();
     }
     int own = 0x7fffffff; uint32_t own_key = 0;                       // lane r keeps the r-th: their values are read back together, not one by one between the rounds
     for (int r = 0; ; r++) {
@@ -848,49 +848,57 @@ __global__ void __launch_bounds__(256) k_topk1(const float * __restrict__ logits
     }
     if (lane < k) { cid[out + lane] = own; cval[out + lane] = own != 0x7fffffff ? l[own] : -INFINITY; }
 }
-// one wave merges a row's slices: ids[k], vals[k] and the sum (device or page-locked memory).  A serial chain: rounds of two reductions each (0.25 us) it was, now the floor, ballot and count of k_topk1 - lane groups that hold
-// whole slices, so that the floor is the least of eight groups' bests and few reach it; a crowd of equal values takes the rounds
+// One wave merges a row's slices: ids[k], vals[k] and the sum (device or page-locked memory).  A serial chain: rounds of two reductions each (0.35 us a round), or (FLOOR) the floor, ballot and count of k_topk1 - lane groups that hold
+// whole slices of eight candidates, so that the floor is the least of eight groups' bests and few reach it; a crowd of equal values takes the rounds
 struct topk_merge_lds { uint32_t key[64], id[64]; float val[64]; };
-static __device__ __forceinline__ void topk_merge(int k, const int32_t * __restrict__ cid, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int lane, topk_merge_lds & M) {
+template <bool FLOOR>
+static __device__ __forceinline__ void topk_merge(int k, const int32_t * __restrict__ cid, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int lane, topk_merge_lds & M, const int gone,
+                                                  const int32_t * __restrict__ abort_w) {
     const float * cval = (const float *) (cid + TOPK_NCH * k), * cmax = cval + TOPK_NCH * k, * csum = cmax + TOPK_NCH;
     const int n = TOPK_NCH * k;                                         // <= 256: four candidates per lane
     float cv[4]; int ci[4]; uint32_t key[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) { const int i = 4 * lane + j; cv[j] = i < n ? cval[i] : -INFINITY; ci[j] = i < n ? cid[i] : 0x7fffffff; }
+    for (int j = 0; j < 4; j++) { const int i = FLOOR ? 4 * lane + j : lane + 64 * j; cv[j] = i < n ? cval[i] : -INFINITY; ci[j] = i < n ? cid[i] : 0x7fffffff; }
     const float pm = lane < TOPK_NCH ? cmax[lane] : -INFINITY, ps = lane < TOPK_NCH ? csum[lane] : 0.0f;
+    if (pi_abort_late(gone, abort_w)) return;
     uint32_t top = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) { key[j] = ci[j] != 0x7fffffff ? topk_key(cv[j]) : 0u; top = max(top, key[j]); }
-    // eight groups of eight lanes: lanes of the same bits 1 .. 3 (a slice of eight candidates is two lanes)
-    top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<1>((int) top));
-    uint32_t least = top;
-    least = min(least, (uint32_t) pi_partner<8>((int) least)); least = min(least, (uint32_t) pi_partner<4>((int) least)); least = min(least, (uint32_t) pi_partner<2>((int) least));
-    least = max(least, 1u);
-    uint64_t who[4]; int m = 0;
+    bool rounds = true;
+    if constexpr (FLOOR) {
+        // eight groups of eight lanes: lanes of the same bits 1 .. 3 (a slice of eight candidates is two lanes)
+        top = max(top, (uint32_t) pi_partner<32>((int) top)); top = max(top, (uint32_t) pi_partner<16>((int) top)); top = max(top, (uint32_t) pi_partner<1>((int) top));
+        uint32_t least = top;
+        least = min(least, (uint32_t) pi_partner<8>((int) least)); least = min(least, (uint32_t) pi_partner<4>((int) least)); least = min(least, (uint32_t) pi_partner<2>((int) least));
+        least = max(least, 1u);
+        uint64_t who[4]; int m = 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++) { who[j] = __ballot(key[j] >= least); m += __popcll(who[j]); }
-    if (m <= 64) {
-        int base = 0;
+        for (int j = 0; j < 4; j++) { who[j] = __ballot(key[j] >= least); m += __popcll(who[j]); }
+        if (m <= 64) {
+            rounds = false;
+            int base = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (key[j] >= least) {
-                const int at = base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[j], 0));
-                M.key[at] = key[j]; M.id[at] = (uint32_t) ci[j]; M.val[at] = cv[j];
+            for (int j = 0; j < 4; j++) {
+                if (key[j] >= least) {
+                    const int at = base + (int) __builtin_amdgcn_mbcnt_hi((uint32_t) (who[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t) who[j], 0));
+                    M.key[at] = key[j]; M.id[at] = (uint32_t) ci[j]; M.val[at] = cv[j];
+                }
+                base += __popcll(who[j]);
             }
-            base += __popcll(who[j]);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t ck = lane < m ? M.key[lane] : 0u; const int id = lane < m ? (int) M.id[lane] : 0x7fffffff;
-        const float val = lane < m ? M.val[lane] : -INFINITY;
-        int ahead = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t ck = lane < m ? M.key[lane] : 0u; const int id = lane < m ? (int) M.id[lane] : 0x7fffffff;
+            const float val = lane < m ? M.val[lane] : -INFINITY;
+            int ahead = 0;
 #pragma unroll 4
-        for (int j = 0; j < m; j++) {
-            const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(id, j);
-            ahead += kj > ck || (kj == ck && ij < id);
+            for (int j = 0; j < m; j++) {
+                const uint32_t kj = (uint32_t) __builtin_amdgcn_readlane((int) ck, j); const int ij = __builtin_amdgcn_readlane(id, j);
+                ahead += kj > ck || (kj == ck && ij < id);
+            }
+            if (lane < m ? ahead < k : lane < k) { const int at = lane < m ? ahead : lane; ids[at] = id; vals[at] = val; }
         }
-        if (lane < m ? ahead < k : lane < k) { const int at = lane < m ? ahead : lane; ids[at] = id; vals[at] = val; }
-    } else for (int r = 0; r < k; r++) {
+    }
+    if (rounds) for (int r = 0; r < k; r++) {
         uint32_t bk = 0; int bi = 0x7fffffff; float bv = -INFINITY;     // this lane's best
 #pragma unroll
         for (int j = 0; j < 4; j++) if (key[j] > bk || (key[j] == bk && bk != 0 && ci[j] < bi)) { bk = key[j]; bi = ci[j]; bv = cv[j]; }
@@ -906,11 +914,11 @@ static __device__ __forceinline__ void topk_merge(int k, const int32_t * __restr
     s = pi_lanes_sum<64>(s);
     if (lane == 0) *sumexp = s;
 }
-__global__ void __launch_bounds__(256) k_topk2(int k, int n_tok, const int32_t * __restrict__ part, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int32_t * __restrict__ abort_w) {
-    if (pi_aborted(abort_w)) return;
-    __shared__ topk_merge_lds M[4];
-    const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
-    if (t < n_tok) topk_merge(k, part + (int64_t) t * topk_words(k), ids + (int64_t) t * k, vals + (int64_t) t * k, sumexp + t, threadIdx.x & 63, M[wave]);
+template <bool FLOOR>
+__global__ void __launch_bounds__(64) k_topk2(int k, const int32_t * __restrict__ part, int32_t * __restrict__ ids, float * __restrict__ vals, float * __restrict__ sumexp, const int32_t * __restrict__ abort_w) {
+    const int gone = pi_abort_peek(abort_w), t = blockIdx.x;
+    __shared__ topk_merge_lds M;
+    topk_merge<FLOOR>(k, part + (int64_t) t * topk_words(k), ids + (int64_t) t * k, vals + (int64_t) t * k, sumexp + t, threadIdx.x, M, gone, abort_w);
 }
 // The end of a pass: rows of logits to the run's page-locked buffer and, beside them, the merge of its rows' slices, which writes the run's buffers itself.  The first workgroups merge (four rows each), the others copy.
 // One launch for what was k_topk2 in front of k_copy_out: the merge is a chain, the copy the bus (a row of 32000: 128 KB).  Measured (us, vocabulary 32000, apart / together): one row 5.8 + 4.6 / 5.6, eight rows 6.7 + 19.1 / 19.4.
@@ -919,7 +927,7 @@ __global__ void __launch_bounds__(256) k_topk_out(const int32_t * __restrict__ p
     __shared__ topk_merge_lds M[4];
     if ((int) blockIdx.x < merges) {
         const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
-        if (t < n_tok) topk_merge(8, part + (int64_t) t * topk_words(8), ids_h + (int64_t) t * 8, vals_h + (int64_t) t * 8, sum_h + t, threadIdx.x & 63, M[wave]);
+        if (t < n_tok) topk_merge<true>(8, part + (int64_t) t * topk_words(8), ids_h + (int64_t) t * 8, vals_h + (int64_t) t * 8, sum_h + t, threadIdx.x & 63, M[wave], 0, nullptr);
         return;
     }
     pi_rows_out(logits, logits_h, n_logits, (size_t) (blockIdx.x - merges) * 256 + threadIdx.x, (size_t) (gridDim.x - merges) * 256);
@@ -938,20 +946,24 @@ extern "C" int pi_op_topk_parts(const float * logits, int n_vocab, int n_tok, in
     if (n_tok <= 0) return 0;
     if (topk_refuses(k, scratch) != 0) return -1;
     const int per = (n_vocab + TOPK_NCH - 1) / TOPK_NCH;
-    // One wave to a slice: candidates cost the same for every k, rounds some 0.4 us each of them.  us by rounds / candidates, vocabulary 32000: one row k = 8 6.5 / 5.7, 4 5.6 / 5.6, 2 4.8 / 5.5; 8 rows k = 8 6.6 / 6.0, 4 5.3 / 5.9;
-    // 24 rows k = 8 6.3 / 6.4; 64 rows 8.0 / 7.3, k = 4 6.4 / 7.1; 256 rows k = 4 14.2 / 12.1, 2 11.5 / 12.4.  Slices of 32 values a lane: 8 rows of 50257 k = 8 9.4 / 8.3, 4 8.0 / 8.6; 16 of 65536 k = 8 9.4 / 10.2
-    const int candidates = per <= 1024 ? k >= (n_tok >= 128 ? 3 : 6) : n_tok >= 256 ? k >= 5 : n_tok >= 128 ? k >= 7 : k == 8 && (n_tok <= 12 || n_tok > 32);
-#define TOPK_GO(VPT, WS) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, candidates, (int32_t *) scratch, pi_abort_word())
-    if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4);
-    else if (per <= 64 * 8) TOPK_GO(8, 1); else if (per <= 64 * 16) TOPK_GO(16, 1); else if (per <= 64 * 32) TOPK_GO(32, 1);
-    else if (per <= 256 * 16) TOPK_GO(16, 4); else if (per <= 256 * 32) TOPK_GO(32, 4); else TOPK_GO(0, 4);
+    // One wave to a slice: candidates cost the same for every k, a round 0.3 .. 0.6 us of few rows (slices of 32 values a lane: 0.7 .. 1.3) and more of many.  us of this launch by rounds / candidates, vocabulary 32000: one row k = 4 5.5 / 5.5,
+    // 8 7.9 / 5.5; 24 rows k = 6 5.8 / 6.4, 8 6.6 / 6.7; 64 k = 7 7.3 / 7.0; 128 k = 5 8.5 / 8.3, 6 9.3 / 8.4; 256 k = 4 12.2 / 11.9; 512 k = 4 21.9 / 19.6; of 12000 4 rows k = 5 4.4 / 4.9, 32 rows k = 6 4.5 / 5.6.
+    // Slices of 32 values a lane, 65536: one row k = 3 7.6 / 8.1, 4 8.8 / 8.1, 24 k = 5 8.0 / 8.4, 6 8.7 / 8.4, 32 k = 8 9.8 / 10.2, 128 k = 4 12.2 / 12.0, 512 k = 3 34.3 / 31.4
+    const bool candidates = per <= 1024 ? k >= (n_tok <= 4 ? 6 : n_tok < 96 ? 7 : n_tok < 192 ? 6 : n_tok < 512 ? 5 : 4) : k >= (n_tok <= 4 ? 4 : n_tok < 96 ? 6 : n_tok < 512 ? 4 : 3);
+#define TOPK_GO(VPT, WS, C) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 4.0 * n_tok * n_vocab, (k_topk1<VPT, WS, C>), dim3(n_tok, TOPK_NCH * WS / 4), dim3(256), 0, (hipStream_t) stream, logits, n_vocab, k, (int32_t *) scratch, pi_abort_word())
+    if (k == 1 && n_tok <= 16 && per > 256 && per <= 256 * 8) TOPK_GO(8, 4, false);
+    else if (per <= 64 * 32 && candidates) { if (per <= 64 * 8) TOPK_GO(8, 1, true); else if (per <= 64 * 16) TOPK_GO(16, 1, true); else TOPK_GO(32, 1, true); }
+    else if (per <= 64 * 8) TOPK_GO(8, 1, false); else if (per <= 64 * 16) TOPK_GO(16, 1, false); else if (per <= 64 * 32) TOPK_GO(32, 1, false);
+    else if (per <= 256 * 16) TOPK_GO(16, 4, false); else if (per <= 256 * 32) TOPK_GO(32, 4, false); else TOPK_GO(0, 4, false);
 #undef TOPK_GO
     PI_CHECK_LAUNCH(); return 0;
 }
 extern "C" int pi_op_topk_merge(const void * scratch, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * stream) {
     if (n_tok <= 0) return 0;
     if (topk_refuses(k, scratch) != 0) return -1;
-    PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2, dim3((n_tok + 3) / 4), dim3(256), 0, (hipStream_t) stream, k, n_tok, (const int32_t *) scratch, ids, vals, sumexp, pi_abort_word());
+#define TOPK_MERGE(F) PI_KT_LAUNCH(PI_KT_OTHER, 0, n_tok, 0.0, k_topk2<F>, dim3(n_tok), dim3(64), 0, (hipStream_t) stream, k, (const int32_t *) scratch, ids, vals, sumexp, pi_abort_word())
+    if (k >= 6) TOPK_MERGE(true); else TOPK_MERGE(false);             // (us by the floor / by rounds, 8 rows of 32000: k = 1 4.3 / 3.0, 4 4.3 / 4.1, 5 4.2 / 4.4, 6 4.3 / 4.8, 8 4.4 / 5.5; one row 4.0 / 2.7, 3.5 / 3.7, 3.5 / 4.1, 3.6 / 4.5, 4.0 / 5.2)
+#undef TOPK_MERGE
     PI_CHECK_LAUNCH(); return 0;
 }
 extern "C" int pi_op_topk(const float * logits, int n_vocab, int n_tok, int k, int32_t * ids, float * vals, float * sumexp, void * scratch, void * stream) {

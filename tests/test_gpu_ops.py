@@ -638,6 +638,28 @@ def test_topk_candidates_of_few_and_many_rows(gpu, n_tok, k, n_vocab):
         assert abs(se.get(np.float32)[0] - want) / want < 1e-5      # (as test_topk_edges: fp32 sum of up to 32001 terms in pairs per slice)
 
 
+@pytest.mark.parametrize("n_tok", [4, 5, 95, 96, 192, 512])
+@pytest.mark.parametrize("n_vocab", [100, 32 * 9, 32 * 1025])
+def test_topk_around_its_lines(gpu, n_tok, n_vocab):
+    """every k on both sides of the lines between rounds and candidates, slices of four, nine and 1025 values; rows of one value over and over, of one number among -infinities or NaNs, of fewer numbers than k, of none"""
+    lib, U = gpu
+    from pipeinfer_amd import lib as L
+    x = (np.random.default_rng(n_tok).standard_normal((n_tok, n_vocab)) * 4).astype(np.float32)
+    x[0] = 2.5
+    x[1] = -np.inf; x[1, 77] = 1.0
+    x[2] = np.nan; x[2, 99] = -3.0; x[2, 3] = -np.inf
+    x[3] = np.nan
+    order = np.lexsort((np.broadcast_to(np.arange(n_vocab), x.shape), -np.nan_to_num(x, nan=-np.inf, neginf=-1e38)), axis=1)
+    best = np.take_along_axis(x, order, 1)
+    ids, vals = np.where(np.isnan(best), 0x7fffffff, order).astype(np.int32), np.where(np.isnan(best), -np.inf, best)
+    ld, scr = U.Dev(x), U.Dev(nbytes=lib.pi_op_topk_scratch_bytes(n_tok))
+    for k in range(1, 9):
+        idd, vd, se = U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok * k), U.Dev(nbytes=4 * n_tok)
+        L.check(lib.pi_op_topk(ld.ptr, n_vocab, n_tok, k, idd.ptr, vd.ptr, se.ptr, scr.ptr, None))
+        assert np.array_equal(idd.get(np.int32, (n_tok, k)), ids[:, :k]) and np.array_equal(vd.get(np.float32, (n_tok, k)), vals[:, :k]), k
+        assert se.get(np.float32)[0] == n_vocab and se.get(np.float32)[1] == 1.0
+
+
 @pytest.mark.parametrize("n_vocab,k", [(2048, 8), (2048, 1), (32 * 2100, 8), (32 * 8200, 8)])
 def test_topk_exponentials(gpu, n_vocab, k):
     """the exponentials behind the soft-max sums are as exact as expf's: a slice of one maximum and 63 equal values, a lane each, whose sum in pairs rounds six times and no more, so that an exponential's own error shows in
