@@ -83,7 +83,11 @@ __global__ void __launch_bounds__(256, 1) k_latent_split(const float * __restric
     if (dyn) { if (live_max > 0 && dyn[1] > live_max) return; cell1 = min(cell1, dyn[1]); }
     if (pi_abort_late(gone, abort_w, 5)) return;
     const int live = (max(cell1 - cell0, 0) + 31) / 32, k_blocks = (nk + 255) / 256, blocks = k_blocks + (nv + 255) / 256, steps = rank / 64;
-    const int first = (int) ((int64_t) live * blocks * blockIdx.x / gridDim.x), last = (int) ((int64_t) live * blocks * (blockIdx.x + 1) / gridDim.x);
+    // From three tiles a workgroup on the same whole number to each but the last: the 32 of an XCD then stand at a few blocks of the matrices, whose rows they share in its L2.  In equal fractions they drift apart by a tile each at odd numbers
+    // of runs (us, fractions / whole: 32 heads of 128, rank 512, 63 runs 96.6 / 68.2, 125 runs 172.9 / 110.5, even numbers alike); below, whole numbers leave compute units idle (1.5 tiles: up to 1.2 times as long)
+    const int64_t all = (int64_t) live * blocks, wgs = gridDim.x, share = (all + wgs - 1) / wgs;
+    const bool whole = all >= 3 * wgs;
+    const int first = (int) (whole ? min(all, share * blockIdx.x) : all * blockIdx.x / wgs), last = (int) (whole ? min(all, share * (blockIdx.x + 1)) : all * (blockIdx.x + 1) / wgs);
     if (first >= last) return;
     sa_u32x4 * const xs = (sa_u32x4 *) lds;                            // [step of 16][part][64]
     uint8_t * const mine = lds + rank * 192 + wave * (2 * SL_STAGE);
