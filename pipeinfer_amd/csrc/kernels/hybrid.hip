@@ -2079,14 +2079,14 @@ static int latent_prompt(pa_args a, const lat_plan & p, const float * cache, int
         const size_t cells = scratch_floats > state ? (scratch_floats - state) / per_cell / 64 * 64 : 0;
         return cells >= 1024 ? cells : 0;
     };
-    // In three parts where that takes no more launches than keys and values as they are: of one launch each the parts are quicker at all sizes, but behind one that holds all live cells another one still costs two idle launches and
+    // In three parts where they are the quicker (sa_pays: of one launch each) and take no more launches than keys and values as they are: behind a launch that holds all live cells another one still costs two idle launches and
     // the sums' way to memory and back.  us as they are in one / in parts in one / in parts in two, cells 3072: 32 heads of 128, rank 512, 512 tokens alone 66 / 53 / 70, 64 alone 27 / 24 / 33; 64 heads of 64 + 32, rank 256, 512 alone
     // 87 / 74 / 98 (all 3072 cells 311 / 237 / 262 and 355 / 273 / 312: how many are live is not known here)
     const size_t plain_cell = (size_t) a.heads * (a.dim1 + a.vdim), part_cell = sa_cell_floats(a.heads, a.dim1, a.dim2, a.vdim), plain = fits(plain_cell), parts = sa_takes(a, rank) ? fits(part_cell) : 0;
     if (plain == 0) return 0;
     auto launches = [](int to, size_t cells) { return (int) ((to + cells - 1) / cells); };
     const int to_plain = latent_tiles_to(p, a, rank, launches(a.n_kv, plain), false), to_parts = parts > 0 ? latent_tiles_to(p, a, rank, launches(a.n_kv, parts), true) : 0;
-    const bool split = to_parts > 0 && launches(to_parts, parts) <= std::max(1, launches(to_plain, plain));
+    const bool split = to_parts > 0 && launches(to_parts, parts) <= std::max(1, launches(to_plain, plain)) && sa_pays(a, rank, to_parts);
     const size_t cells = split ? parts : plain;
     const int to = split ? to_parts : to_plain;
     a.state = cells < whole ? scratch + cells * (split ? part_cell : plain_cell) : nullptr;

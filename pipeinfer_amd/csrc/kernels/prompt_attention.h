@@ -40,8 +40,9 @@ void pa_expand(const float * cache, int64_t width, int rank, const pi_weight * w
 int pa_few_split(const pa_args & a, int maps, size_t scratch_floats, int * split_cells);
 void pa_few_launch(const pa_args & a, int maps, int n_cs, int split_cells, double bytes, hipStream_t s);
 #define PA_FEW_SPLITS 32
-// Keys and values of a latent in three bfloat16 parts and the attention over them (split_attention.hip).  sa_sizes: heads and ranks that the kernels take, sa_takes: passes; sa_cell_floats: scratch memory for a cell
+// Keys and values of a latent in three bfloat16 parts and the attention over them (split_attention.hip).  sa_sizes: heads and ranks that the kernels take, sa_takes: passes, sa_pays: which of them are the quicker that way; sa_cell_floats: scratch memory for a cell
 bool sa_sizes(int dim, int rot, int vdim, int rank);
 bool sa_takes(const pa_args & a, int rank);
+bool sa_pays(const pa_args & a, int rank, int live_max);
 size_t sa_cell_floats(int heads, int dim, int rot, int vdim);
 void sa_launch(const pa_args & a, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, double bytes, hipStream_t s);

@@ -15,6 +15,7 @@
 #include "kernel_timing.h"
 
 #include <algorithm>
+#include <cmath>
 
 #define SA_MAX_RANK 512                                                /* a run's latents fill 96 KB of LDS */
 
@@ -624,6 +625,30 @@ bool sa_sizes(int dim, int rot, int vdim, int rank) { return rank > 0 && rank % 
 bool sa_takes(const pa_args & a, int rank) {
     return sa_sizes(a.dim1, a.dim2, a.vdim, rank) && a.n_tok >= PA_LATENT_TOKENS && a.qs % 4 == 0 && ((uintptr_t) a.q & 15) == 0 && (int64_t) a.n_tok * ((a.n_kv + 31) / 32) < (1ll << 32);
 }
+// What a prompt takes, us: keys and values as they are (k_latent_expand + k_prompt_attention: two workgroups of 32 queries to a compute unit), in parts by four waves that share the cells of 32 queries, in parts by a wave for
+// every 32 queries (a workgroup 128).  The last reads keys and values once for 128 queries and has no sums to join; the others have four times the workgroups.  The start, the latents' products, keys and values written and read, rounds of
+// workgroups, and the walk: runs of cells x steps of a run, of all workgroups over the chip or of one over all cells, the longer one and a share of the other.  The constants are those that are nearest to 3500 sizes (six shapes of heads, 4 .. 192
+// of them, 12 .. 2048 tokens, 12 .. 16000 cells): 14 .. 19 % off on the mean
+enum { SA_PLAIN, SA_FOUR, SA_ONE };
+static double sa_us(int form, const pa_args & a, int rank, int live) {
+    static const struct { double start, latents, values, round, longer, shorter; int queries, cells, slots; } F[3] = {
+        { 0.908, 5.74, 772, 18.2, 0.334, 0.353, 32, 128, 512 }, { 7.7, 5.02, 1520, 9.41, 0.153, 0.0183, 32, 128, 256 }, { 6.04, 3.87, 1520, 16.3, 0.133, 0.0434, 128, 32, 256 } };
+    const auto & f = F[form];
+    live = std::max(live, a.n_tok);
+    const double values = 1e-9 * live * a.heads * (a.dim1 + a.vdim), groups = (double) a.heads * ((a.n_tok + f.queries - 1) / f.queries), seen = live - a.n_tok + 0.5 * (a.n_tok + f.queries);
+    const double steps = form == SA_PLAIN ? (a.dim1 + 15) / 16 + (a.dim2 + 15) / 16 + 4 * ((a.vdim + 63) / 64) : (a.dim1 + a.dim2 + a.vdim) / 16;
+    const double all = groups * seen / f.slots / f.cells * steps, one = (double) live / f.cells * steps;
+    return f.start + f.latents * values * rank + f.values * values + f.round * std::ceil(groups / f.slots) + f.longer * std::max(all, one) + f.shorter * std::min(all, one);
+}
+// Four waves or one to 32 queries: by what they take with the pass's own cells alone and with all that there may be (how many are live is not known here).  us, four / one: 32 heads of 128, rank 512, 512 tokens alone 55 / 75, 1024 113 / 117, 2048
+// 301 / 251; 128 heads, 128 tokens alone 44 / 47, 256 83 / 66, 512 180 / 138
+static bool sa_many(const pa_args & a, int rank) { return sa_us(SA_ONE, a, rank, a.n_tok) / sa_us(SA_FOUR, a, rank, a.n_tok) + sa_us(SA_ONE, a, rank, a.n_kv) / sa_us(SA_FOUR, a, rank, a.n_kv) < 2; }
+// In parts where that takes clearly less by the estimates, at both ends.  Few cells of more heads than a round of workgroups holds lose (us, as they are / in parts: 128 heads of 128, rank 512, 136 tokens alone 61 / 69; 64 heads of 64,
+// rank 128, 300 tokens alone 34 / 40).  Of 8896 triples of a pass, cells live and cells there may be, times of the choice over those as they are: mean 0.80 (0.77 the quickest form each time), 1.00 at the 99th percent, at most 1.21
+bool sa_pays(const pa_args & a, int rank, int live_max) {
+    const int form = sa_many(a, rank) ? SA_ONE : SA_FOUR;
+    return sa_us(form, a, rank, a.n_tok) <= 0.89 * sa_us(SA_PLAIN, a, rank, a.n_tok) && sa_us(form, a, rank, live_max) <= 0.89 * sa_us(SA_PLAIN, a, rank, live_max);
+}
 // scratch: 1.5 floats for every value of the cells [cell0, cell1) (sa_cell_floats), 16-byte aligned; cell0 a multiple of 64
 void sa_launch(const pa_args & a, const float * cache, int rank, const pi_weight * wuk, const pi_weight * wuv, float * scratch, double bytes, hipStream_t s) {
     const int runs = (a.cell1 - a.cell0 + 63) / 64 * 2, tiles = (a.cell1 - a.cell0 + 31) / 32 * (int) ((wuk->ne1 + 255) / 256 + (wuv->ne1 + 255) / 256);
@@ -631,10 +656,7 @@ void sa_launch(const pa_args & a, const float * cache, int rank, const pi_weight
     PI_KT_LAUNCH(PI_KT_ATT, PI_BF16, PI_KT_MAXNT - 1, 2.0 * rank * (wuk->ne1 + wuv->ne1) + 4.0 * std::min(a.cell1 - a.cell0, a.n_kv) * (double) (a.k2_row + 1.5 * (wuk->ne1 + wuv->ne1)), k_latent_split, dim3((unsigned) std::min(tiles, 256)), dim3(256), 0, s,
                  cache, a.k2_row, rank, (const uint16_t *) wuk->p0, (int) wuk->ne1, (const uint16_t *) wuv->p0, (int) wuv->ne1, a.dim1 == 64 ? 6 : 7, a.dim2, a.vdim == 64 ? 6 : 7, a.cell0, a.cell1, a.live_max, a.dyn, kf, rf, vf, runs, pi_abort_word());
     const int nta = std::min(a.n_tok, PI_KT_MAXNT - 1);
-    // A wave for every 32 queries (a workgroup 128) reads keys and values once for 128 queries and has no sums to join; four waves that share the cells of 32 have four times the workgroups.  Measured over 120 sizes (16 .. 512 heads of
-    // 64 and 128, 64 .. 4096 tokens, their own cells and 4096), time of one wave / of four, by workgroups of 128 queries: 64 1.75 .. 2.37, 128 1.06 .. 1.65, 256 0.65 .. 1.2 (heads of 128, rank 512: 32 of them, 1024 tokens alone 116 / 113 us,
-    // 16, 2048 180 / 154, 128, 256 66 / 83), 384 0.8 .. 1.03, 512 0.73 .. 1.04 (32, 2048 251 / 301, 128, 512 138 / 180, 512, 64 79.4 / 78.8)
-    const bool many = (int64_t) a.heads * ((a.n_tok + 127) / 128) >= 512;
+    const bool many = sa_many(a, rank);
 #define SA_GO(KO, KR, NJ, P) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_split_attention<KO, KR, NJ, P>), dim3((unsigned) a.heads, (unsigned) ((a.n_tok + 128 / P - 1) / (128 / P))), dim3(256), 0, s, a, kf, rf, vf, runs, pi_abort_word())
 #define SA_NJ(KO, KR) do { if (a.vdim == 64) { if (many) SA_GO(KO, KR, 2, 1); else SA_GO(KO, KR, 2, 4); } else if (many) SA_GO(KO, KR, 4, 1); else SA_GO(KO, KR, 4, 4); } while (0)
     if (a.dim1 == 64) { if (a.dim2) SA_NJ(4, 2); else SA_NJ(4, 0); }
