@@ -66,11 +66,12 @@ PI_API int     pi_op_abort_cancel(int32_t * word_dev, int32_t run_id, void * str
  *                           aborted and *timeout_flag_dev = 1), then arms the abort word like pi_op_abort_begin, with the producer's abort bit or-ed in;
  *                           hop_ticks_dev (nullable) accumulates {flag written -> seen, time waited, runs} in 10 ns ticks */
 /* A run's results (logits rows, top-8 ids / values, soft-max sums) written into the caller's PAGE-LOCKED host buffers by a kernel on the run's stream, instead of
- * hipMemcpyAsync: on this runtime a device -> host copy of the logits' size does not complete while another stream's kernels keep the device busy (runtime.hip). */
+ * hipMemcpyAsync: on this runtime a device -> host copy of the logits' size does not complete while another stream's kernels keep the device busy (runtime.hip).
+ * For results that are merged already (pi_op_topk); the engine's passes end in pi_op_topk_out, which merges them on the way. */
 PI_API int     pi_op_copy_out(const float * logits_dev, float * logits_host, int64_t n_logits, const int32_t * ids_dev, int32_t * ids_host, const float * vals_dev, float * vals_host,
                               const float * sum_dev, float * sum_host, int n_tok, void * stream);
 /* A pass's inputs read out of its PAGE-LOCKED block by one launch on the run's stream: consecutive parts of n[i] 32-bit words each go to dst[i] (null: skipped), at most PI_COPY_IN_PARTS.
- * abort_word_dev (nullable): armed first, as pi_op_abort_begin arms it. */
+ * abort_word_dev (nullable): armed by the same launch, as pi_op_abort_begin arms it. */
 #define PI_COPY_IN_PARTS 6
 PI_API int     pi_op_copy_in(const void * block_host, int parts, void * const * dst_dev, const int64_t * n, int32_t * abort_word_dev, int32_t run_id, const int32_t * host_flag, void * stream);
 PI_API int     pi_op_flag_publish(void * flag_dev, uint32_t ticket, const int32_t * abort_word_dev, int force_abort, void * stream);

@@ -921,8 +921,8 @@ __global__ void __launch_bounds__(64) k_topk2(int k, const int32_t * __restrict_
     topk_merge<FLOOR>(k, part + (int64_t) t * topk_words(k), ids + (int64_t) t * k, vals + (int64_t) t * k, sumexp + t, threadIdx.x, M, gone, abort_w);
 }
 // The end of a pass: rows of logits to the run's page-locked buffer and, beside them, the merge of its rows' slices, which writes the run's buffers itself.  The first workgroups merge (four rows each), the others copy.
-// One launch for what was k_topk2 in front of k_copy_out: the merge is a chain, the copy the bus (a row of 32000: 128 KB).  Measured (us, vocabulary 32000, apart / together): one row 5.8 + 4.6 / 5.6, eight rows 6.7 + 19.1 / 19.4.
-// What it writes for a cancelled run is dropped, so it does not look at the abort word (k_copy_out does not either)
+// One launch for what was k_topk2 and a copy behind it: the merge is a chain, the copy the bus (a row of 32000: 128 KB).  Measured (us, vocabulary 32000, apart / together): one row 5.8 + 4.6 / 5.6, eight rows 6.7 + 19.1 / 19.4.
+// What it writes for a cancelled run is dropped, so it does not look at the abort word
 __global__ void __launch_bounds__(256) k_topk_out(const int32_t * __restrict__ part, int n_tok, int merges, int32_t * __restrict__ ids_h, float * __restrict__ vals_h, float * __restrict__ sum_h, const float * __restrict__ logits, float * __restrict__ logits_h, size_t n_logits) {
     __shared__ topk_merge_lds M[4];
     if ((int) blockIdx.x < merges) {

@@ -191,7 +191,8 @@ extern "C" int pi_op_abort_cancel(int32_t * word_dev, int32_t run_id, void * str
 // hipMemcpyAsync(device -> page-locked host) of a run's logits goes through a copy engine on this runtime, and that copy does not complete while ANOTHER stream's kernels
 // keep the device busy: a draft step of 1.2 ms waited for the whole 11 ms target run beside it (tools_dev/wrap_beside.py, profiles/r04_d2h_copy_stall.log; the same step
 // with its results written by a kernel: 1.3 ms beside the target).  Page-locked host memory is device-addressable, so the last kernel of a run writes the caller's
-// buffers itself; the event recorded behind it releases them to the host.
+// buffers itself; the event recorded behind it releases them to the host.  In the engine that is k_topk_out (elementwise.hip), which merges the top 8 as well; this one, an operator for programs of their own,
+// is for results that are merged already.
 __global__ void __launch_bounds__(256) k_copy_out(const float * __restrict__ logits, float * __restrict__ logits_h, size_t n_logits, const int32_t * __restrict__ ids, int32_t * __restrict__ ids_h,
                                                   const float * __restrict__ vals, float * __restrict__ vals_h, const float * __restrict__ sum, float * __restrict__ sum_h, int n_tok) {
     const size_t tid = (size_t) blockIdx.x * 256 + threadIdx.x, nthr = (size_t) gridDim.x * 256;
