@@ -454,19 +454,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
 
 // The same for a step: a few tokens, most of them a run of their own.  What bounds it: a state is read and written once (16.8 MB of eight sequences, 6.7 us at a copy's rate), and the trips to memory in front of that.  So nothing goes
 // through LDS but the sums over the rows, which the four waves share: a wave finds its run by a ballot, every operand of its first token leaves beside the state, the unit vectors' lengths and the token's scalar are added up by
-// every wave for itself.  Workgroup (head, 32 columns of values, run); thread (four columns, rows rg + 32 m), states in runs of 128 bytes; a token is one barrier.
+// every wave for itself.  Workgroup (head, 32 columns of values, run); thread (four columns, rows rg + 8 NW m), states in runs of 128 bytes; a token is one barrier.
+// Keys of 32 values: one wave (NW = 1), no LDS and no barrier.  What every wave repeats is most of such a token, and where workgroups fill the chip four waves paid for it four times: 64 heads of 32 x 256 under the delta rule, eight runs
+// of four tokens, 35.3 by k_channel_recurrence, 49.2 by four waves, 15.7 by one; 32 tokens of one run, 128 heads of 32 x 128, 74 / 60 / 37; one token of 32 heads of 32 x 64 11.5 / 3.8 / 3.5.
 // Measured, us (k_channel_recurrence / this), 32 heads of 128 x 128 under the delta rule: one token 14.5 / 4.8, eight of a sequence each 19.8 / 8.3, eight of one 35.6 / 13.7, 32 of one 109 / 46; 64 heads of 64 x 64 under the bonus rule
 // 11.8 / 3.7, 15.6 / 6.1, 24.5 / 8.6, 67.8 / 23.5.  (There a token's operands were staged for 32, with four barriers and a search by one thread ahead of them, and a state came in runs of 64 bytes.)
 #define CS_TOKENS CR_TB                           // (a run's first tokens are found among a wave's lanes; longer passes go in pieces)
-template <int NR, int RULE>
-__global__ void __launch_bounds__(256) k_channel_step(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs,
+template <int NR, int RULE, int NW>
+__global__ void __launch_bounds__(64 * NW) k_channel_step(const float * __restrict__ q, int64_t qs, const float * __restrict__ k, int64_t ks, const float * __restrict__ v, int64_t vs,
                                                       const float * __restrict__ draw, int64_t ds, int decay_mode, const float * __restrict__ dbias, const float * __restrict__ a_log,
                                                       const float * __restrict__ braw, int64_t bs, const float * __restrict__ bonus, int qk_unit, float q_mult,
                                                       int heads, int hpg, int vdim, float * __restrict__ state, const int32_t * __restrict__ rec, int n_tok,
                                                       float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
-    constexpr int DIM = 32 * NR, NL = (DIM + 63) / 64;
-    __shared__ __attribute__((aligned(16))) float meet[2][4][2][32];    // [token % 2][wave][with the keys, with the queries][column]
+    constexpr int STEP = 8 * NW, DIM = STEP * NR, NL = (DIM + 63) / 64;
+    __shared__ __attribute__((aligned(16))) float meet[2][NW][2][NW > 1 ? 32 : 1];    // [token % 2][wave][with the keys, with the queries][column]
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), quad = tid & 7, rg = tid >> 3, col = blockIdx.y * 32 + quad * 4, hq = h / hpg;
     // run number blockIdx.z
     const int own = rec[min(lane, n_tok - 1)], before = rec[max(min(lane, n_tok - 1) - 1, 0)];
@@ -483,16 +485,16 @@ __global__ void __launch_bounds__(256) k_channel_step(const float * __restrict__
         for (int m = 0; m < NR; m++) S[m] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     } else {
 #pragma unroll
-        for (int m = 0; m < NR; m++) S[m] = *(const float4 *) (S_hbm + (int64_t) 32 * m * vdim);
+        for (int m = 0; m < NR; m++) S[m] = *(const float4 *) (S_hbm + (int64_t) STEP * m * vdim);
     }
     struct token { float q[NR], k[NR], d[NR], lq[NL], lk[NL], lb[NL], beta; float4 v; };
     float bias[NR];
 #pragma unroll
-    for (int m = 0; m < NR; m++) bias[m] = dbias ? dbias[h * DIM + rg + 32 * m] : 0.0f;
+    for (int m = 0; m < NR; m++) bias[m] = dbias ? dbias[h * DIM + rg + STEP * m] : 0.0f;
     auto ask = [&](token & T, int t) __attribute__((always_inline)) {
         const float * qr = q + (int64_t) t * qs + (int64_t) hq * DIM, * kr = k + (int64_t) t * ks + (int64_t) hq * DIM, * dr = draw + (int64_t) t * ds + (int64_t) h * DIM;
 #pragma unroll
-        for (int m = 0; m < NR; m++) { T.q[m] = qr[rg + 32 * m]; T.k[m] = kr[rg + 32 * m]; T.d[m] = dr[rg + 32 * m]; }
+        for (int m = 0; m < NR; m++) { T.q[m] = qr[rg + STEP * m]; T.k[m] = kr[rg + STEP * m]; T.d[m] = dr[rg + STEP * m]; }
 #pragma unroll
         for (int x = 0; x < NL; x++) {
             const int i = min(lane + 64 * x, DIM - 1);
@@ -541,28 +543,32 @@ __global__ void __launch_bounds__(256) k_channel_step(const float * __restrict__
             if (RULE == 0) { a[x] += pi_partner<8>(a[x]); a[x] += pi_partner<16>(a[x]); a[x] += pi_partner<32>(a[x]); }
             c[x] += pi_partner<8>(c[x]); c[x] += pi_partner<16>(c[x]); c[x] += pi_partner<32>(c[x]);
         }
-        float (* const M)[2][32] = meet[t & 1];
-        if (lane < 8) {
-            if (RULE == 0) *(float4 *) &M[wave][0][quad * 4] = make_float4(a[0], a[1], a[2], a[3]);
-            *(float4 *) &M[wave][1][quad * 4] = make_float4(c[0], c[1], c[2], c[3]);
+        // of all rows: what the four waves left (a wave alone has it in every lane)
+        float (* const M)[2][NW > 1 ? 32 : 1] = meet[t & 1];
+        if constexpr (NW > 1) {
+            if (lane < 8) {
+                if (RULE == 0) *(float4 *) &M[wave][0][quad * 4] = make_float4(a[0], a[1], a[2], a[3]);
+                *(float4 *) &M[wave][1][quad * 4] = make_float4(c[0], c[1], c[2], c[3]);
+            }
+            __syncthreads();
         }
-        __syncthreads();
+        auto met = [&](int which, const float * own) __attribute__((always_inline)) {
+            if constexpr (NW > 1) {
+                const float4 w0 = *(const float4 *) &M[0][which][quad * 4], w1 = *(const float4 *) &M[1][which][quad * 4], w2 = *(const float4 *) &M[2][which][quad * 4], w3 = *(const float4 *) &M[3][which][quad * 4];
+                return make_float4((w0.x + w1.x) + (w2.x + w3.x), (w0.y + w1.y) + (w2.y + w3.y), (w0.z + w1.z) + (w2.z + w3.z), (w0.w + w1.w) + (w2.w + w3.w));
+            } else return make_float4(own[0], own[1], own[2], own[3]);
+        };
         float4 u = vv;                                                  // what the token writes under its key
-        if (RULE == 0) {
-            const float4 w0 = *(const float4 *) &M[0][0][quad * 4], w1 = *(const float4 *) &M[1][0][quad * 4], w2 = *(const float4 *) &M[2][0][quad * 4], w3 = *(const float4 *) &M[3][0][quad * 4];
-            u.x = beta * (vv.x - ((w0.x + w1.x) + (w2.x + w3.x))); u.y = beta * (vv.y - ((w0.y + w1.y) + (w2.y + w3.y)));
-            u.z = beta * (vv.z - ((w0.z + w1.z) + (w2.z + w3.z))); u.w = beta * (vv.w - ((w0.w + w1.w) + (w2.w + w3.w)));
-        }
+        if (RULE == 0) { const float4 wa = met(0, a); u.x = beta * (vv.x - wa.x); u.y = beta * (vv.y - wa.y); u.z = beta * (vv.z - wa.z); u.w = beta * (vv.w - wa.w); }
 #pragma unroll
         for (int m = 0; m < NR; m++) { S[m].x = fmaf(kk[m], u.x, S[m].x); S[m].y = fmaf(kk[m], u.y, S[m].y); S[m].z = fmaf(kk[m], u.z, S[m].z); S[m].w = fmaf(kk[m], u.w, S[m].w); }
         if (tid < 8) {
-            const float4 w0 = *(const float4 *) &M[0][1][quad * 4], w1 = *(const float4 *) &M[1][1][quad * 4], w2 = *(const float4 *) &M[2][1][quad * 4], w3 = *(const float4 *) &M[3][1][quad * 4];
-            *(float4 *) (out + (int64_t) t * os + (int64_t) h * vdim + col) = make_float4(fmaf(u.x, dot, (w0.x + w1.x) + (w2.x + w3.x)), fmaf(u.y, dot, (w0.y + w1.y) + (w2.y + w3.y)),
-                                                                                       fmaf(u.z, dot, (w0.z + w1.z) + (w2.z + w3.z)), fmaf(u.w, dot, (w0.w + w1.w) + (w2.w + w3.w)));
+            const float4 wc = met(1, c);
+            *(float4 *) (out + (int64_t) t * os + (int64_t) h * vdim + col) = make_float4(fmaf(u.x, dot, wc.x), fmaf(u.y, dot, wc.y), fmaf(u.z, dot, wc.z), fmaf(u.w, dot, wc.w));
         }
     }
 #pragma unroll
-    for (int m = 0; m < NR; m++) *(float4 *) (S_hbm + (int64_t) 32 * m * vdim) = S[m];
+    for (int m = 0; m < NR; m++) *(float4 *) (S_hbm + (int64_t) STEP * m * vdim) = S[m];
 }
 
 // grid (head, blocks of CR_SCAN_COLS value columns, run): per piece p of the run, in order: scratch[p] holds [L_p | T_p] coming in and S_in(p) (in L_p's place) going out.
@@ -1255,10 +1261,10 @@ extern "C" int pi_op_channel_recurrence(int rule, const float * q, int64_t q_str
     // every pass that is not cut into pieces, of key widths and columns that the step kernel's threads share out whole (its figures: both kernels at every number of tokens)
     if (n_tok <= CS_TOKENS && (dim == 32 || dim == 64 || dim == 128) && vdim % 32 == 0 && v_stride % 4 == 0 && out_stride % 4 == 0 && (((uintptr_t) v | (uintptr_t) out | (uintptr_t) state_dev) & 15) == 0) {
         const dim3 grid((unsigned) heads, (unsigned) (vdim / 32), (unsigned) runs);
-#define CS_GO(NR, RL) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_channel_step<NR, RL>), grid, dim3(256), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
+#define CS_GO(NR, RL, NW) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, (k_channel_step<NR, RL, NW>), grid, dim3(64 * NW), 0, s, q, q_stride, k, k_stride, v, v_stride, decay_raw, decay_stride, decay_mode, decay_bias_dev, a_log_dev, \
                                    beta_raw, beta_stride, bonus_dev, qk_unit, q_mult, heads, heads / qk_heads, vdim, state_dev, rec_dev, n_tok, out, out_stride, pi_abort_word())
-        if (rule == PI_RULE_DELTA) { if (dim == 32) CS_GO(1, 0); else if (dim == 64) CS_GO(2, 0); else CS_GO(4, 0); }
-        else                       { if (dim == 32) CS_GO(1, 1); else if (dim == 64) CS_GO(2, 1); else CS_GO(4, 1); }
+        if (rule == PI_RULE_DELTA) { if (dim == 32) CS_GO(4, 0, 1); else if (dim == 64) CS_GO(2, 0, 4); else CS_GO(4, 0, 4); }
+        else                       { if (dim == 32) CS_GO(4, 1, 1); else if (dim == 64) CS_GO(2, 1, 4); else CS_GO(4, 1, 4); }
 #undef CS_GO
         PI_CHECK_LAUNCH(); return 0;
     }

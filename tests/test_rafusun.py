@@ -442,6 +442,15 @@ def test_channel_recurrence_steps(H, G, D, V, rule, mode):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V", [(5, 5, 32, 128), (6, 2, 32, 64)])
+@pytest.mark.parametrize("rule", [DELTA, BONUS])
+def test_channel_recurrence_steps_by_one_wave(H, G, D, V, rule):
+    """keys of 32 values, whose rows one wave holds: several blocks of columns, a head for every query and three of them to one"""
+    for mode in (0, 1, 2):
+        test_channel_recurrence_steps(H, G, D, V, rule, mode)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 32, 16), (3, 3, 64, 64), (4, 2, 128, 48), (1, 1, 128, 128), (1, 1, 64, 144), (2, 1, 32, 272)])
 @pytest.mark.parametrize("rule", [DELTA, BONUS])
 def test_channel_recurrence_pieces_on_the_matrix_cores(H, G, D, V, rule):
