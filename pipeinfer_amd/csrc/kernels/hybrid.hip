@@ -1382,9 +1382,10 @@ extern "C" int pi_op_linear_attention_keysum(const float * q, const float * k, c
     // token 450 -> 123, for the pieces are walked twice and the scan starts for every run); up to there where the walk, whose time is its longest run's (7 us and 1.9 a token), has more than eight tokens in one whatever the runs are
     // (24 tokens 53 -> 29, 9 about even; eight runs of a token or two 14 .. 18, here 25 .. 29)
     // The step's kernel walks a run at 0.6 us a token, the pieces below take 9 .. 29 us for up to 32: us of one run, step / pieces, 16 heads: key width 32 12 tokens 8.0 / 9.5, 16 10.1 / 9.4; 64 20 tokens 13.0 / 13.9, 24 14.3 / 14.0; 96 32
-    // tokens 19.5 / 25.8; 128 32 tokens 20.9 / 29.1.  The host knows how many runs there may be, not how many there are: one may have all tokens, so the line is a single run's; and no fewer tokens than those that k_linear_attention's
-    // walk would take otherwise (24 tokens of width 32 as one run: where there may be two 13.4 by the step and 10.5 by the pieces, where there may be three 13.3 by the step and 38 by that walk; 32 of width 64, two 18.7 and 14.3)
-    const int alone = dim == 32 ? 12 : dim == 64 ? 20 : LA_TB;
+    // tokens 19.5 / 25.8; 128 32 tokens 20.9 / 29.1; of values of 64 and less, whose states are the fewer loads, 96 28 tokens 17.6 / 18.8, 32 19.9 / 19.0, 128 32
+    // tokens 21.0 / 20.1.  The host knows how many runs there may be, not how many there are: one may have all tokens, so the line is a single run's; and no fewer tokens than those that k_linear_attention's walk would take otherwise
+    // (24 tokens of width 32 as one run: where there may be two 13.4 by the step and 10.5 by the pieces, where there may be three 13.3 by the step and 38 by that walk; 32 of width 64, two 18.7 and 14.3)
+    const int alone = dim == 32 ? 12 : dim == 64 ? 20 : vdim <= 64 ? 28 : LA_TB;
     if (n_tok <= LA_TB && matrix && n_tok <= std::max(alone, 8 * (int) gr) && !key_sum && vdim % 32 == 0 && stride % 4 == 0 && out_stride % 4 == 0 && (((uintptr_t) v | (uintptr_t) out | (uintptr_t) state_dev) & 15) == 0) {
 #define LS_GO(NR) PI_KT_LAUNCH(PI_KT_ATT, 0, nta, bytes, k_linear_step<NR>, dim3((unsigned) heads, (unsigned) (vdim / 32), gr), dim3(256), 0, s, q, k, v, stride, heads, hpg, vdim, decay_dev, tdecay_dev, tscale_dev, t_stride, skip_dev, state_dev, \
                                rec_dev, n_tok, out, out_stride, pi_abort_word())

@@ -492,6 +492,23 @@ def test_one_sequence_of_a_pass_that_may_have_several(D, T, most):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,V,T", [(96, 64, 29), (128, 64, 32), (128, 32, 30), (96, 32, 32)])
+def test_one_long_sequence_of_few_values_goes_to_the_pieces(D, V, T):
+    """the same bits as with output rows that the step's kernel does not take"""
+    U, lib = gpu()
+    rng = np.random.default_rng(D + V + T)
+    H, stride = 3, 3 * (2 * D + V)
+    buf, start, lam = rng.standard_normal((T, stride)).astype(np.float32), rng.standard_normal((3, H, D, V)).astype(np.float32), np.linspace(0.4, 0.999, H).astype(np.float32)
+    bd, rc, ld = U.Dev(buf), U.Dev(np.full(T, 1, np.int32)), U.Dev(lam)
+    got = []
+    for segments, row in ((1, H * V + 1), (1, H * V), (2, H * V)):
+        sd, od = U.Dev(start), U.Dev(nbytes=4 * T * row)
+        L.check(lib.pi_op_linear_attention(bd.ptr, bd.ptr + 4 * H * D, bd.ptr + 8 * H * D, stride, H, D, V, ld.ptr, sd.ptr, rc.ptr, T, segments, None, 0, od.ptr, row, None))
+        got.append((od.get(np.uint32, (T, row))[:, :H * V], sd.get(np.uint32)))
+    assert all(np.array_equal(o, got[0][0]) and np.array_equal(s, got[0][1]) for o, s in got[1:])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [32, 24])
 @pytest.mark.parametrize("lengths", [[1] * 5, [1] * 30, [2, 1, 3] * 40, [1] * 255 + [70], [1] * 3 + [130] + [1, 2] * 35 + [64, 65]])
 def test_linear_attention_of_many_sequences(D, lengths):
