@@ -488,6 +488,7 @@ __global__ void __launch_bounds__(128) k_attention_combine(const float * __restr
     }
 }
 // the same where a head is two maps: grid (token, head), both maps' splits merged into LDS, then joined by one wave
+template <int NC>
 __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __restrict__ part, int n_cs, int H, int V, ca_maps mp, float out_mult, float * __restrict__ out, int64_t os, const int32_t * __restrict__ abort_w) {
     const int gone = pi_abort_peek(abort_w);
     extern __shared__ float maps_lds[];                               // [2][V]
@@ -495,10 +496,11 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
     const float * pr = part + (((int64_t) t * H + h) * 2 + map) * n_cs * (V + 2);
     // sixteen splits of 128 values on their way at a time, the first of them beside the splits' maxima and denominators, of which a lane has one each (n_cs <= CA_SPLIT_MAX <= 64).  Eight splits of 64 values,
     // behind those, and weights through LDS: 4 tokens of 16 heads of 128 values, 26 splits 5.7 us, 5.2 so, 32 splits 5.5 and 4.4; in a model's step 6.6 and 5.8.  (One map, 128 values to two waves: no less)
-    float x[2][16];
+    // Heads of up to 64 values: one of them a lane (NC = 1).  With loads for 128 that were the same twice attention and merge of 4 tokens of 16 heads, 409 of 4096 cells, took 17.0 us where the eight splits of 64 took 16.4; 16.4 so
+    float x[NC][16];
     auto ask = [&](int v0, int s0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int c = 0; c < NC; c++)
 #pragma unroll
             for (int u = 0; u < 16; u++) x[c][u] = pr[(int64_t) min(s0 + u, n_cs - 1) * (V + 2) + min(v0 + 64 * c + lane, V - 1)];
     };
@@ -508,18 +510,22 @@ __global__ void __launch_bounds__(128) k_attention_combine_maps(const float * __
     const float f_l = ms_l != -INFINITY ? expf(ms_l - M) : 0.0f;
     const float den = pi_lanes_sum<64>(f_l > 0.0f ? ls_l * f_l : 0.0f);
     if (pi_abort_late(gone, abort_w)) return;
-    for (int v0 = 0; v0 < V; v0 += 128) {
-        float a[2] = { 0.0f, 0.0f };
+    for (int v0 = 0; v0 < V; v0 += 64 * NC) {
+        float a[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) a[c] = 0.0f;
         for (int s0 = 0; s0 < n_cs; s0 += 16) {
             if (v0 + s0 > 0) ask(v0, s0);
 #pragma unroll
             for (int u = 0; u < 16; u++) {
                 const float f = s0 + u < n_cs ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f_l), (s0 + u) & 63)) : 0.0f;
-                if (f > 0.0f) { a[0] = fmaf(x[0][u], f, a[0]); a[1] = fmaf(x[1][u], f, a[1]); }
+                if (f > 0.0f)
+#pragma unroll
+                    for (int c = 0; c < NC; c++) a[c] = fmaf(x[c][u], f, a[c]);
             }
         }
 #pragma unroll
-        for (int c = 0; c < 2; c++) if (v0 + 64 * c + lane < V) maps_lds[map * V + v0 + 64 * c + lane] = den > 0.0f ? a[c] / den : 0.0f;
+        for (int c = 0; c < NC; c++) if (v0 + 64 * c + lane < V) maps_lds[map * V + v0 + 64 * c + lane] = den > 0.0f ? a[c] / den : 0.0f;
     }
     __syncthreads();
     if (map == 0) ca_join_maps(maps_lds, maps_lds + V, V, mp, out_mult, out + (int64_t) t * os + (int64_t) h * V, lane);
@@ -592,8 +598,10 @@ static int window_attention(const float * q, int64_t q_stride, float * k_cache, 
     const double visible = chunk > 0 ? std::min(acct, chunk) + (pool > 0 ? std::max(acct - chunk, 0) / pool : std::min(std::max(acct - chunk, 0), keep_first)) : acct;
     auto merge = [&]() -> int {                                        // the splits' shares, where there are any
         if (maps == 2) {
-            PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * (2.0 * n_cs * (vdim + 2) + vdim), k_attention_combine_maps, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), (size_t) 2 * vdim * sizeof(float),
-                         (hipStream_t) stream, scratch, n_cs, heads, vdim, mp, out_mult, out, out_stride, pi_abort_word());
+#define CM_GO(NC) PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * (2.0 * n_cs * (vdim + 2) + vdim), k_attention_combine_maps<NC>, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), \
+                               (size_t) 2 * vdim * sizeof(float), (hipStream_t) stream, scratch, n_cs, heads, vdim, mp, out_mult, out, out_stride, pi_abort_word())
+            if (vdim <= 64) CM_GO(1); else CM_GO(2);
+#undef CM_GO
             PI_CHECK_LAUNCH();
         } else {
             PI_KT_LAUNCH(PI_KT_ATT, 0, std::min(n_tok, PI_KT_MAXNT - 1), 4.0 * n_tok * heads * ((double) n_cs * (vdim + 2) + vdim), k_attention_combine, dim3((unsigned) n_tok, (unsigned) heads), dim3(128), 0, (hipStream_t) stream,
