@@ -17,8 +17,8 @@
 // of the weights' operands 27 instructions were needed where the upper bits come in place and one fma takes the offset along (21).  Measured together (us, before / now): 8192 x 28672 columns 181 / 166, 32000 x 8192 205 / 196,
 // 8192 x 8192 at 64 tokens 37.4 / 35.4.  Its two products of a tile apart by a step (the second takes the first as its sum): 163, 194 and 36.7: not kept.
 // Where one wave has all of Q4_K's lanes k (S = 1) a launch is many rounds of workgroups that read their weights from HBM: a block is 1.2 us there, no longer than such a load takes, so the loads run two blocks ahead, with a
-// third set of registers for the weights and the image written a block earlier, from the same registers.  Measured (us, 57344 x 8192, one block / two blocks ahead): 128 tokens 289 / 272, 64 tokens 170 / 162; launches of a
-// round or two are as they were (8192 x 8192 43.7 / 43.6).  The other types and S = 2 lose (registers, steps of half the length): Q3_K 276 / 294, Q5_K 333 / 336, Q6_K 32000 x 8192 192 / 197.
+// third set of registers for the weights and the image written a block earlier, from the same registers.  Measured (us, 57344 x 8192, one block / two blocks ahead): 128 tokens 289 / 272, 64 tokens 170 / 162; short rows
+// lose (MP_FAR_BLOCKS).  The other types and S = 2 lose (registers, steps of half the length): Q3_K 276 / 294, Q5_K 333 / 336, Q6_K 32000 x 8192 192 / 197.
 #include "mmvq_args.h"
 #include <hip/hip_ext.h>
 
@@ -64,11 +64,11 @@ static __device__ __forceinline__ uint32_t mp_load4(__amdgpu_buffer_rsrc_t r, ui
 // S waves share a row group's accumulator lanes: lane kk of wave s is lane k = s * 8 / S + kk of the reference
 template <int TYPE, int KS> struct mp_w { uint32_t dd, rec, rec2, q[KS], h[TYPE == PI_Q4_K ? 1 : KS]; };       // a lane's share of one block
 
-template <int TYPE, int S, int RG, int CH>
+template <int TYPE, int S, int RG, int CH, bool NEAR>
 static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, const int group_end, const int group0, const int tb) {
     constexpr bool Q5 = TYPE == PI_Q5_K, Q6 = TYPE == PI_Q6_K, Q3 = TYPE == PI_Q3_K, Q4 = TYPE == PI_Q4_K;
     constexpr uint32_t TILE = Q6 ? PI_MQ_TILE_Q6 : Q5 ? PI_MQ_TILE_Q5 : Q3 ? PI_MQ_TILE_Q3 : PI_MQ_TILE, QOFF = Q6 ? 1600 : (Q5 || Q3) ? 832 : 320, QPART = Q3 ? 512 : 1024;
-    constexpr bool FAR = Q4 && S == 1;                 // loads run two blocks ahead
+    constexpr bool FAR = Q4 && S == 1 && !NEAR;        // loads run two blocks ahead
     constexpr int KS = 8 / S, CS = Q4 ? 4 / S : 1, NTHR = 64 * S * RG, NL = CH * 512 / NTHR, IMG = CH * 8192 + NTHR * 8;      // IMG: LDS image of one block: fragments of CH chunks, then their aux (and what the threads past it write)
     static_assert(S == 1 || S == 2, "one or two waves a row group");
     static_assert((512 % NTHR == 0) && CH * 128 <= NTHR, "whole strips of 16-byte units; eight bytes of aux a thread");
@@ -395,22 +395,22 @@ static __device__ __forceinline__ void mmq_prompt_body(const mmvq_args & g, cons
 // workgroup n runs on XCD n % 8: the token blocks of a row block go to one XCD one behind the other, so that its weights come from HBM once.
 // SB, RGB: waves per row group and row groups of the second type's workgroups.  They are few and come last, so the launch ends with one of them: where the first type keeps one wave to a row group the second takes two
 // (a Q6_K tile costs a wave 1.6 times a Q4_K one; 8192 + 1024 rows of Q4_K with 1024 of Q6_K, 8192 columns, 64 tokens: 57.6 us with one wave to all row groups, now 41.4; Q5_K 50 and 41.1)
-template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG>
+template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG, bool NEAR = false>
 __global__ void __launch_bounds__(64 * S * RG) k_mmq_prompt(const mmvq_args g, const int groups_a, const int groups_all, const int blocks_a, const int row_blocks, const int tok_blocks) {
     static_assert(S * RG == SB * RGB, "workgroups of one size");
     if (pi_aborted(g.abort_w, 1)) return;
     const int slot = blockIdx.x >> 3, rb = (blockIdx.x & 7) + 8 * (slot / tok_blocks), tb = slot % tok_blocks;
     if (rb >= row_blocks) return;
     if constexpr (TA != TB) {
-        if (rb >= blocks_a) { mmq_prompt_body<TB, SB, RGB, CH>(g, groups_all, groups_a + (rb - blocks_a) * RGB, tb); return; }
+        if (rb >= blocks_a) { mmq_prompt_body<TB, SB, RGB, CH, NEAR>(g, groups_all, groups_a + (rb - blocks_a) * RGB, tb); return; }
     }
-    mmq_prompt_body<TA, S, RG, CH>(g, groups_a, rb * RG, tb);
+    mmq_prompt_body<TA, S, RG, CH, NEAR>(g, groups_a, rb * RG, tb);
 }
 
-template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG>
+template <int TA, int TB, int S, int RG, int CH, int SB = S, int RGB = RG, bool NEAR = false>
 static int prompt_go(const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     constexpr size_t image = 3 * ((size_t) CH * 8192 + 64 * S * RG * 8), fold = S == 2 || SB == 2 ? (size_t) S * RG * ((CH + 1) / 2) * 4 * 6 * 256 : 0, lds = image > fold ? image : fold;
-    const auto kernel = k_mmq_prompt<TA, TB, S, RG, CH, SB, RGB>;
+    const auto kernel = k_mmq_prompt<TA, TB, S, RG, CH, SB, RGB, NEAR>;
     if (!g.frag) { PI_CHECK_HIP(hipFuncSetAttribute((const void *) kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds)); return 0; }       // pi_op_mul_mat_reserve
     const int blocks_a = (groups_a + RG - 1) / RG, row_blocks = blocks_a + (groups_all - groups_a + RGB - 1) / RGB, tok_blocks = (g.nt + CH * 16 - 1) / (CH * 16);
     const unsigned grid = (unsigned) ((row_blocks + 7) / 8 * 8) * (unsigned) tok_blocks;
@@ -419,6 +419,14 @@ static int prompt_go(const mmvq_args & g, int groups_a, int groups_all, hipStrea
     PI_CHECK_LAUNCH();
     return 0;
 }
+// Loads two blocks ahead from rows of eight blocks on: a row asks for three blocks behind its end instead of two, and three have to be there before its first product.  us one block / two blocks ahead, weights
+// from memory: 28672 rows x 64 tokens K 512 13.6 / 14.0, 768 15.8 / 17.1, 1536 24.1 / 24.3, 2048 29.3 / 28.6, 4096 50.0 / 48.6, 8192 88.4 / 83.1; x 128 tokens 768 27.3 / 29.6, 1536 41.8 / 42.3, 2048 51.6 / 50.0, 8192 161 / 152; 57344 x 300
+// 768 105 / 114, 2048 198 / 200, 8192 679 / 673
+#define MP_FAR_BLOCKS 8
+template <int TA, int TB, bool NEAR>
+static int prompt_182(const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
+    if constexpr (TA != TB) return prompt_go<TA, TB, 1, 8, 2, 2, 4, NEAR>(g, groups_a, groups_all, stream, ea, eb); else return prompt_go<TA, TB, 1, 8, 2, 1, 8, NEAR>(g, groups_a, groups_all, stream, ea, eb);
+}
 template <int TA, int TB>
 static int prompt_cfg(int cfg, const mmvq_args & g, int groups_a, int groups_all, hipStream_t stream, hipEvent_t ea, hipEvent_t eb) {
     switch (cfg) {                                             // S, RG, CH
@@ -426,7 +434,9 @@ static int prompt_cfg(int cfg, const mmvq_args & g, int groups_a, int groups_all
         case 243: return prompt_go<TA, TB, 2, 4, 3>(g, groups_a, groups_all, stream, ea, eb);
         case 244: return prompt_go<TA, TB, 2, 4, 4>(g, groups_a, groups_all, stream, ea, eb);
         case 222: return prompt_go<TA, TB, 2, 2, 2>(g, groups_a, groups_all, stream, ea, eb);
-        case 182: if constexpr (TA != TB) return prompt_go<TA, TB, 1, 8, 2, 2, 4>(g, groups_a, groups_all, stream, ea, eb); else return prompt_go<TA, TB, 1, 8, 2>(g, groups_a, groups_all, stream, ea, eb);
+        case 182:
+            if constexpr (TA == PI_Q4_K) if (g.nb < MP_FAR_BLOCKS) { const int rc = prompt_182<TA, TB, true>(g, groups_a, groups_all, stream, ea, eb); if (g.frag || rc != 0) return rc; }      // (reserving: both)
+            return prompt_182<TA, TB, false>(g, groups_a, groups_all, stream, ea, eb);
     }
     pi_set_error("mmq_prompt: configuration %d", cfg);
     return -1;

@@ -218,6 +218,19 @@ def test_mul_mat_q4_k_prompt_two_blocks_ahead(gpu, blocks_a_row):
     lib.pi_weight_free(w)
 
 
+@pytest.mark.parametrize("blocks_a_row", [8, 9, 10])
+def test_mul_mat_q4_k_prompt_around_the_line_to_two_blocks_ahead(gpu, blocks_a_row):
+    """shorter rows load one block ahead: the first that load two, with every remainder"""
+    test_mul_mat_q4_k_prompt_two_blocks_ahead(gpu, blocks_a_row)
+
+
+@pytest.mark.parametrize("types", [(O.Q4_K, O.Q4_K, O.Q5_K), (O.Q4_K, O.Q4_K, O.Q6_K)])
+@pytest.mark.parametrize("k", [1792, 2048, 2304])
+def test_two_weight_types_around_the_line_to_two_blocks_ahead(gpu, types, k):
+    """the same where the second type's workgroups, of two waves a row group, load one block ahead in any case"""
+    test_two_weight_types_prompt_tiles(gpu, types, k, (8176, 9, 33), 63, 255)
+
+
 @pytest.mark.parametrize("k,rows", [(4096, 40), (4096, 2048), (4096, 2049), (4064, 40)])
 def test_mul_mat_q4_0_nine_tokens(gpu, k, rows):
     """nine tokens, where the mat-vec would take a second pass over the weights (k_mmq_q0 takes them, as it does all from seven), around 2048 rows of 4096 values and a row of whole groups less one block: the reference's bits"""
