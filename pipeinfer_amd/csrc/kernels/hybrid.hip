@@ -2166,7 +2166,8 @@ static int latent_attention(const float * q, int64_t q_stride, const float * cac
     auto combine = [&](int S, bool rows) -> int {
         const int vec = (rank & 7) == 0 && (rank > 64 || S > 32) && (((uintptr_t) wuv->p0 | (uintptr_t) pol) & 15) == 0;      // (rank 64: one split 16.3 us, 17.1 so; 64 splits 18.9 and 18.3)
         // Many splits of whole rows: eight waves, as a thread's trips to memory one behind the other are what is waited for; up to two workgroups a compute unit.  us of 256 / 512 threads, rank 512: 4 tokens x 16 heads, 23 splits
-        // 12.7 / 10.6, 10 splits 10.9 / 8.3, 1 token 23 splits 9.1 / 7.4, 250 splits 27.6 / 19.6, 8 tokens x 32 heads (512 workgroups), 32 splits 17.7 / 14.8, x 64 heads 22.5 / 26.8
+        // 12.7 / 10.6, 10 splits 10.9 / 8.3, 1 token 23 splits 9.1 / 7.4, 250 splits 27.6 / 19.6, 8 tokens x 32 heads (512 workgroups), 32 splits 17.7 / 14.8, x 64 heads 22.5 / 26.8.  (How many splits are live is not known here: 2 tokens x 64 heads
+        // with the launches ahead, over 204 of 4096 cells 22.3 / 23.5, over 4096 65 / 59)
         const int64_t wgs = (int64_t) ((n_tok + 3) / 4) * heads * ((vdim + 15) / 16);
         if (S > 8 && vec && rank > 64 && wgs <= 2 * pi_cu_count()) LAT_COMBINE(true, 512); else if (S > 8) LAT_COMBINE(true, 256); else LAT_COMBINE(false, 256);
         PI_CHECK_LAUNCH(); return 0;
